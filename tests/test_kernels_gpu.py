@@ -126,6 +126,22 @@ def test_gemm_f32(M, N, K):
     assert rel_err(out_nb, x.double() @ w.double().T) < F32_TOL
 
 
+@pytest.mark.parametrize("N,K", [(48, 1000), (1024, 1024), (1028, 130), (3072, 256), (2048, 2052), (20480, 128)])
+def test_gemm_f32_order_of_sums(N, K):
+    """Each kernel that a 32-bit product may take, by its rows (16 x 16 with eight or sixteen
+    waves, tiles of 32 x 32 to 64 x 64 with K over one to four groups), with edges of rows,
+    outputs and chains of K: right, and the same bits for a row whatever else is in the step."""
+    x, w = rand((1100, K), torch.float32, 60).to(dev()), rand((N, K), torch.float32, 61).to(dev())
+    whole = ops().linear(x, w)
+    # (sums of K products of unit normal values: 32-bit rounding along 128 products and K / 128
+    # sums stays below 1e-6 of the largest)
+    assert rel_err(whole, x.double() @ w.double().T) < 1e-6
+    for M in (1, 16, 17, 63, 130, 200, 400, 513, 1099):
+        assert torch.equal(ops().linear(x[:M].contiguous(), w), whole[:M]), M
+    bias = rand((N,), torch.float32, 62).to(dev())
+    assert torch.equal(ops().linear(x[:33].contiguous(), w, bias), whole[:33] + bias)
+
+
 def test_gemm_f32_weight_with_bf16_activations():
     """A weight stored in 32-bit stays 32-bit in a bfloat16 run."""
     x, w = rand((9, 40), torch.bfloat16, 11), rand((23, 40), torch.float32, 12)

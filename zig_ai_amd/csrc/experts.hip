@@ -34,8 +34,9 @@
 //      64 of K at a time with the next step's pieces on their way into registers, four
 //      waves of 64 x 64 each: every element of either operand is then read from memory
 //      once a tile and used 128 times.
-//      32-bit: LDS-tiled FMA, 64 x 64 tiles (no matrix-core rounding mode).
+//      32-bit: tiles of 32 x 64 on the matrix cores' 32-bit instruction (gemm_f32.h).
 #include "common.h"
+#include "gemm_f32.h"
 
 #define EX_MAX_EXPERTS 1024
 
@@ -348,75 +349,47 @@ grouped_gemm_bf16_tiled_kernel(GroupedArgs g) {
     }
 }
 
-// 32-bit weights (src of either type): 64 x 64 tiles through LDS, plain FMA.  GATED: a tile is 32
-// outputs, a thread's four weight rows are two gate rows and the two up rows that go with them.
-template <typename TA, typename TO, bool GATED>
-__global__ void __launch_bounds__(256)
+// 32-bit weights (src of either type): tiles of 32 assignments x 64 weight rows, the sums in the
+// order of gemm_f32.h.  GATED: a tile is 32 outputs, its weight rows gate and up rows in turn, 16
+// each, so that a lane holds both columns.
+#define GF_BM 32
+#define GF_BN 64
+
+template <typename TA, typename TO, bool GATED, bool VEC>
+__global__ void __launch_bounds__(512)
 grouped_gemm_f32_kernel(GroupedArgs g) {
-  __shared__ float As[16][64 + 4];
-  __shared__ float Ws[16][64 + 4];
   int e, tile, count;
-  if (!find_tile<64>(g.counts, g.E, blockIdx.x, &e, &tile, &count)) return;
-  const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
-  const int n0 = blockIdx.y * (GATED ? 32 : 64);
+  if (!find_tile<GF_BM>(g.counts, g.E, blockIdx.x, &e, &tile, &count)) return;
+  const int n0 = blockIdx.y * (GATED ? GF_BN / 2 : GF_BN), m0 = tile * GF_BM;
   const int* mine = g.lists + (size_t)e * g.A;
   const int K = g.K, N = g.N;
   const float* W = (const float*)g.W + (size_t)e * (GATED ? 2 * N : N) * K;
-  const int lrow = tid / 4, lk = (tid % 4) * 4;
-  const int arow_idx = tile * 64 + lrow;
-  const bool a_ok = arow_idx < count;
-  const TA* arow = (const TA*)g.src + (size_t)(a_ok ? mine[arow_idx] / g.src_div : 0) * K;
-  const int wn = n0 + (GATED ? (lrow / 4) * 2 + (lrow & 1) : lrow);
-  const bool w_ok = wn < N;
-  const float* wrow = W + (size_t)(w_ok ? wn + (GATED && (lrow & 2) ? N : 0) : 0) * K;
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-  for (int k0 = 0; k0 < K; k0 += 16) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = k0 + lk + j;
-      As[lk + j][lrow] = (a_ok && k < K) ? to_f32<TA>(arow[k]) : 0.f;
-      Ws[lk + j][lrow] = (w_ok && k < K) ? wrow[k] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[4], w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = Ws[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
   TO* out = (TO*)g.out;
+  f32_tile<TA, GF_BM, GF_BN, 2, VEC>(
+      K, [&](int r) { return (const TA*)g.src + (size_t)(mine[min(m0 + r, count - 1)] / g.src_div) * K; },
+      [&](int r) {
+        const int n = min(n0 + (GATED ? (r >> 5) * 16 + (r & 15) : r), N - 1);
+        return W + (size_t)(n + (GATED && (r & 16) ? N : 0)) * K;
+      },
+      [&](int r, int n, const f32x4_t(&v)[GF_BN / 32]) {
+        if (m0 + r >= count) return;
+        const int a = mine[m0 + r];
+        TO* at = out + dst_row(g, a) * N;
+        const float w = g.row_weight ? g.row_weight[a] : 1.0f;
+        if constexpr (GATED) {
+          const int first = n0 + (n >> 5) * 16 + (n & 15);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = tile * 64 + ty * 4 + i;
-    if (r >= count) continue;
-    const size_t d = dst_row(g, mine[r]);
-    const float w = g.row_weight ? g.row_weight[mine[r]] : 1.0f;
-    if constexpr (GATED) {
+          for (int i = 0; i < 4; ++i)
+            if (first + i < N) at[first + i] = from_f32<TO>(expert_unit(g, v[0][i], v[1][i], w));
+        } else {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int n = n0 + tx * 2 + j;
-        if (n < N) out[d * N + n] = from_f32<TO>(expert_unit(g, acc[i][j], acc[i][j + 2], w));
-      }
-    } else {
+          for (int j = 0; j < GF_BN / 32; ++j)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = n0 + tx * 4 + j;
-        if (n < N) out[d * N + n] = from_f32<TO>(expert_act(acc[i][j], g.act) * g.out_scale * w);
-      }
-    }
-  }
+            for (int i = 0; i < 4; ++i)
+              if (n0 + n + j * 16 + i < N)
+                at[n0 + n + j * 16 + i] = from_f32<TO>(expert_act(v[j][i], g.act) * g.out_scale * w);
+        }
+      });
 }
 
 // dtype codes: 0 = float32, 1 = bfloat16.  `src` has `src_rows` rows of K elements; the
@@ -470,12 +443,18 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     return za_launch_status();
   }
   if (w_dtype != 0) return ZA_ERR_UNSUPPORTED;
-  const int columns = gate ? 32 : 64;
-  dim3 grid((unsigned)((A + 63) / 64 + experts), (unsigned)((N + columns - 1) / columns)), block(256);
-#define ZA_GF(TA, TO)                                                                             \
-  {                                                                                               \
-    if (gate) hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, true>), grid, block, 0, stream, g); \
-    else hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, false>), grid, block, 0, stream, g);     \
+  const int columns = gate ? GF_BN / 2 : GF_BN;
+  dim3 grid((unsigned)((A + GF_BM - 1) / GF_BM + experts), (unsigned)((N + columns - 1) / columns)), block(512);
+  const bool vec = K % 4 == 0 && (uintptr_t)src % (src_dtype == 1 ? 8 : 16) == 0 && (uintptr_t)W % 16 == 0;
+#define ZA_GFV(TA, TO, GATED)                                                                              \
+  {                                                                                                        \
+    if (vec) hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, GATED, true>), grid, block, 0, stream, g); \
+    else hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, GATED, false>), grid, block, 0, stream, g);    \
+  }
+#define ZA_GF(TA, TO)                 \
+  {                                   \
+    if (gate) ZA_GFV(TA, TO, true)    \
+    else ZA_GFV(TA, TO, false)        \
   }
   if (src_dtype == 0 && out_dtype == 0) ZA_GF(float, float)
   else if (src_dtype == 1 && out_dtype == 0) ZA_GF(bf16_t, float)
@@ -483,6 +462,7 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
   else if (src_dtype == 0 && out_dtype == 1) ZA_GF(float, bf16_t)
   else return ZA_ERR_UNSUPPORTED;
 #undef ZA_GF
+#undef ZA_GFV
   return za_launch_status();
 }
 

@@ -1609,3 +1609,44 @@ def test_repetition_penalty():
     work = logits.clone().to(dev())
     ops().repetition_penalty_(work, rows.to(dev()), toks.to(dev()), fac.to(dev()))
     assert torch.allclose(work.cpu(), torch.tensor([[1.0, -4.0, 0.0, 4.0], [1.0 / 1.5, 1.0, -1.0, -4.0]]))
+
+
+# ------------------------------------------------------------------- experts
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("E,top,N,K,T", [(8, 2, 72, 64, 1), (8, 3, 130, 200, 40), (3, 1, 256, 192, 200),
+                                         (6, 2, 66, 136, 330), (70, 4, 64, 40, 600), (1, 1, 20, 8, 5)])
+def test_grouped_products_at_the_edges_of_their_tiles(dtype, E, top, N, K, T):
+    """Every height of tile (32, 64 and 128 assignments, by the rows an expert has on average), K
+    below, at and off multiples of a step of 64, outputs off multiples of a tile and of four,
+    experts without rows and more experts than lanes; the lists from the same tokens."""
+    o = ops()
+    gen = torch.Generator().manual_seed(E * 1000 + T)
+    chosen = torch.stack([torch.randperm(E, generator=gen)[:top] for _ in range(T)]).int()
+    if E > 2:
+        chosen[chosen == 1] = 0                      # (an expert without rows, one twice as long)
+    lists, counts = o.expert_lists(None, chosen.to(dev()), T, E)
+    for e in range(E):
+        want = (chosen.view(-1) == e).nonzero().view(-1).int()
+        assert int(counts[e]) == want.numel()
+        assert torch.equal(lists[e, :want.numel()].cpu(), want), e
+    x, w = rand((T, K), dtype, 70), rand((E, N, K), dtype, 71, K ** -0.5)
+    gate_up, weight = rand((E, 2 * N, K), dtype, 72, K ** -0.5), rand((T, top), torch.float32, 73)
+    which, rows = chosen.view(-1).long(), x.double().repeat_interleave(top, 0)
+    full = torch.einsum("ank,ak->an", w.double()[which], rows)
+    got = o.grouped_linear(x.to(dev()), w.to(dev()), lists, counts, T, per_token=True, out_dtype=torch.float32)
+    assert rel_err(got, full) < F32_TOL
+    planes = o.grouped_linear(rows.to(dtype).to(dev()), w.to(dev()), lists, counts, T, per_token=False,
+                              stacked=True, row_weight=weight.to(dev()))
+    want = (full * weight.double().view(-1, 1)).view(T, top, N).transpose(0, 1)
+    assert rel_err(planes, want) < F32_TOL
+    both = torch.einsum("ank,ak->an", gate_up.double()[which], rows)
+    unit = torch.nn.functional.silu(both[:, :N]) * both[:, N:]
+    got = o.grouped_linear(x.to(dev()), gate_up.to(dev()), lists, counts, T, per_token=True, out_dtype=dtype,
+                           gate="silu")
+    assert rel_err(got, unit) < tol_of(dtype)
+    # (a row's bits do not depend on the other tokens of its step)
+    l1, c1 = o.expert_lists(None, chosen[:1].contiguous().to(dev()), 1, E)
+    alone = o.grouped_linear(x[:1].contiguous().to(dev()), w.to(dev()), l1, c1, 1, per_token=True,
+                             out_dtype=torch.float32)
+    whole = o.grouped_linear(x.to(dev()), w.to(dev()), lists, counts, T, per_token=True, out_dtype=torch.float32)
+    assert torch.equal(alone, whole[:top])

@@ -521,6 +521,106 @@ def test_ssd_recurrence_kernel(H, G, N, P):
     assert float(state[1].abs().max()) == 0.0
 
 
+def _chunk_items(lengths, size, dev):
+    seq, row0, cnt, r = [], [], [], 0
+    for i, n in enumerate(lengths):
+        for at in range(0, n, size):
+            seq.append(i), row0.append(r + at), cnt.append(min(size, n - at))
+        r += n
+    return tuple(torch.tensor(v, dtype=torch.int32, device=dev) for v in (seq, row0, cnt)) + (len(seq),)
+
+
+@pytest.mark.parametrize("H,G,d,dv,strong", [(2, 1, 16, 8, False), (3, 3, 40, 72, True), (2, 2, 128, 128, False),
+                                             (4, 2, 64, 200, True), (1, 1, 31, 17, False)])
+def test_delta_recurrence_in_chunks(H, G, d, dv, strong):
+    """Portions taken in chunks of 32 as matrix products: against float64, in two steps so that
+    the second starts from carried states, with portions of exactly a chunk, one token more and
+    fewer, half a chunk and one token; with decays down to zero.  (Bound as for the walk.)"""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator().manual_seed(d + dv)
+    C = ops.DELTA_CHUNK
+    steps = [[C + 1, 1, 2 * C, C - 1, 16], [C // 2 + 1, 70, 1, 5, C]]
+    slots = [3, 0, 4, 5, 1]
+    mem, state = _slots(7, 12 + H * d * dv, dev)
+    A_log = torch.rand(H, generator=gen) * 4 - (1 if strong else 4)
+    dt_bias = torch.randn(H * d, generator=gen)
+    S64 = [torch.zeros(H, d, dv, dtype=torch.float64) for _ in slots]
+    for lengths in steps:
+        T = sum(lengths)
+        conv = torch.randn(T, 2 * G * d + H * dv + 3, generator=gen)
+        proj = torch.randn(T, H + 5, generator=gen)
+        raw = torch.randn(T, H * d + 9, generator=gen) * (8.0 if strong else 1.0)
+        _, start, slot_id = _step_arrays(lengths, slots, dev)
+        out = ops.delta_recurrence_chunked(conv.to(dev), 3, 3 + G * d, 3 + 2 * G * d, proj.to(dev), 5, raw.to(dev),
+                                           dt_bias.to(dev), A_log.to(dev), state, 12, slot_id,
+                                           _chunk_items(lengths, C, dev), H, G, d, dv).cpu().double()
+        c, r = conv.double(), 0
+        for i, n in enumerate(lengths):
+            rows = slice(r, r + n)
+            q, k = c[rows, 3:3 + G * d].view(n, G, d), c[rows, 3 + G * d:3 + 2 * G * d].view(n, G, d)
+            v = c[rows, 3 + 2 * G * d:].view(n, H, dv)
+            q = (q / torch.sqrt((q * q).sum(-1, keepdim=True) + 1e-6) * d ** -0.5).repeat_interleave(H // G, 1)
+            k = (k / torch.sqrt((k * k).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(H // G, 1)
+            beta = torch.sigmoid(proj[rows, 5:5 + H].double())
+            decay = torch.exp(-torch.exp(A_log.double())[None, :, None] * plain.softplus(
+                (raw[rows, :H * d].double() + dt_bias.double()).view(n, H, d)))
+            want = torch.zeros(n, H, dv, dtype=torch.float64)
+            for t in range(n):
+                S64[i] = decay[t][:, :, None] * S64[i]
+                u = beta[t][:, None] * (v[t] - torch.einsum("hkv,hk->hv", S64[i], k[t]))
+                S64[i] = S64[i] + k[t][:, :, None] * u[:, None, :]
+                want[t] = torch.einsum("hkv,hk->hv", S64[i], q[t])
+            assert float((out[rows] - want.reshape(n, -1)).abs().max()) < 2e-5 * max(1.0, float(want.abs().max()))
+            r += n
+        for i, slot in enumerate(slots):
+            kept = state[slot, 12:].double().cpu().view(H, dv, d).transpose(1, 2)
+            assert float((kept - S64[i]).abs().max()) < 2e-5 * max(1.0, float(S64[i].abs().max()))
+    assert float(mem[:, 12 + H * d * dv:].abs().max()) == 0.0
+    assert float(state[:, :12].abs().max()) == 0.0 and float(state[2].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("H,G,N,P,strong", [(4, 2, 24, 16, True), (3, 1, 128, 64, False), (2, 2, 33, 130, False)])
+def test_ssd_recurrence_in_chunks(H, G, N, P, strong):
+    """As above for a decay a head and token, in chunks of 128."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator().manual_seed(N + P)
+    C = ops.RETENTION_CHUNK
+    steps = [[C + 1, 1, 2 * C + 16, C - 1], [40, C, 1, 17]]
+    slots = [2, 3, 0, 4]
+    mem, state = _slots(6, H * N * P, dev)
+    dt_bias, D = torch.randn(H, generator=gen), torch.randn(H, generator=gen)
+    A_log = torch.rand(H, generator=gen) * 3 - (0 if strong else 3)
+    S64 = [torch.zeros(H, N, P, dtype=torch.float64) for _ in slots]
+    for lengths in steps:
+        T = sum(lengths)
+        conv = torch.randn(T, H * P + 2 * G * N, generator=gen)
+        proj = (torch.randn(T, 4 + H, generator=gen) * (6.0 if strong else 1.0)).to(torch.bfloat16)
+        _, start, slot_id = _step_arrays(lengths, slots, dev)
+        out = ops.ssd_recurrence_chunked(conv.to(dev), H * P + G * N, H * P, 0, proj.to(dev), 4, dt_bias.to(dev),
+                                         A_log.to(dev), D.to(dev), state, 0, slot_id,
+                                         _chunk_items(lengths, C, dev), H, G, N, P).cpu().double()
+        c, r = conv.double(), 0
+        for i, n in enumerate(lengths):
+            rows = slice(r, r + n)
+            x = c[rows, :H * P].view(n, H, P)
+            B = c[rows, H * P:H * P + G * N].view(n, G, N).repeat_interleave(H // G, 1)
+            Cq = c[rows, H * P + G * N:].view(n, G, N).repeat_interleave(H // G, 1)
+            dt = plain.softplus(proj[rows, 4:].double() + dt_bias.double())
+            decay = torch.exp(-torch.exp(A_log.double()) * dt)
+            want = torch.zeros(n, H, P, dtype=torch.float64)
+            for t in range(n):
+                S64[i] = decay[t][:, None, None] * S64[i] + (dt[t][:, None] * B[t])[:, :, None] * x[t][:, None, :]
+                want[t] = torch.einsum("hnp,hn->hp", S64[i], Cq[t]) + D.double()[:, None] * x[t]
+            assert float((out[rows] - want.reshape(n, -1)).abs().max()) < 2e-5 * max(1.0, float(want.abs().max()))
+            r += n
+        for i, slot in enumerate(slots):
+            kept = state[slot].double().cpu().view(H, P, N).transpose(1, 2)
+            assert float((kept - S64[i]).abs().max()) < 2e-5 * max(1.0, float(S64[i].abs().max()))
+    assert float(mem[:, H * N * P:].abs().max()) == 0.0 and float(state[1].abs().max()) == 0.0
+
+
 def test_small_kernels():
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")

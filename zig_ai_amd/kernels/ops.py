@@ -161,10 +161,16 @@ _SIGNATURES = {
         c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
         c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int,
         c_float, c_void_p, c_float, c_int, c_int, c_void_p],
-    ("recurrent", "za_retention_chunked"): [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
-                                            c_longlong, c_void_p, c_void_p, c_void_p, c_void_p,
-                                            c_void_p, c_int, c_int, c_int, c_void_p, c_void_p,
-                                            c_int, c_int, c_int, c_int, c_int, c_void_p],
+    ("recurrent_chunks", "za_decay_chunked"): [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int,
+                                               c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_longlong,
+                                               c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
+                                               c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
+                                               c_void_p],
+    ("recurrent_chunks", "za_delta_chunked"): [c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int,
+                                               c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_longlong,
+                                               c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p,
+                                               c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
+                                               c_int, c_int, c_int, c_int, c_void_p],
     ("experts", "za_expert_lists"): [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p,
                                      c_void_p, c_void_p],
     ("experts", "za_grouped_gemm"): [c_void_p, c_int, c_longlong, c_void_p, c_int, c_void_p,
@@ -2191,8 +2197,66 @@ def _fixed_decay_recurrence(vectors: torch.Tensor, q_col: int, k_col: int, x_col
     return out
 
 
-RETENTION_CHUNK = 256          # rows of a work item of the chunked fixed-decay walk
-RETENTION_CHUNK_MAX_DK = 128   # state rows the correction keeps in registers
+RETENTION_CHUNK = 128          # rows of a work item where a head has one decay a token
+DELTA_CHUNK = 32               # and where every key channel has one beside a delta rule
+CHUNKED_MAX_DK = 128           # state rows of a head that the chunks' kernels take
+
+
+def in_chunks(seq_lens) -> bool:
+    """Whether a step's portions (``seq_lens``: the tokens of every request) are taken as chunks
+    rather than walked token by token (a function of the step's shape alone): from 192 tokens in a
+    portion on.  The walk's time is its longest portion's, 0.34 us a token (delta rule 0.4), more
+    when there are many; chunks start at some 30 us.  Measured (us, walked and in chunks; 64 heads
+    of 128 x 64 with one decay a token; 16 of 128 x 128 with a delta rule): one portion of 64 tokens
+    25 and 32; 36 and 37; of 128 46 and 45; 65 and 43; eight of 256 330 and 156; 285 and 144; one of
+    2,048 698 and 155; 878 and 206.  Between 112 and 192 chunks would win 10 to 30 us a layer;
+    portions that short are walked all the same, so that a prompt cut into small portions gives
+    the same bits as whole."""
+    return max(seq_lens, default=0) >= 192
+
+
+def _chunk_items(items, n_seqs: int, what: str):
+    item_seq, item_row0, item_count, n_items = items
+    for name, t in (("item_seq", item_seq), ("item_row0", item_row0), ("item_count", item_count)):
+        _need(t, name, torch.int32)
+        if t.numel() < n_items:
+            raise KernelError(f"{name} holds {t.numel()} entries, fewer than {n_items} items")
+    if n_items < n_seqs:
+        raise KernelError(f"{what}: {n_items} items for {n_seqs} requests")
+
+
+def _columns(width: int, *blocks) -> None:
+    for name, col, n in blocks:
+        if col < 0 or col + n > width:
+            raise KernelError(f"{name}: columns {col}..{col + n} of {width}")
+
+
+def _decay_chunked(vectors, q_col, k_col, x_col, proj, gate_col, dt_bias, A_log, D, fixed, state, state_offset,
+                   slot_id, items, heads, groups, dk, dv):
+    T, width = vectors.shape
+    S = slot_id.numel()
+    _need(vectors, "vectors", torch.float32)
+    _need(slot_id, "slot_id", torch.int32, (S,))
+    _chunk_items(items, S, "recurrence in chunks")
+    if dk > CHUNKED_MAX_DK:
+        raise KernelError(f"dk={dk}: chunks take up to {CHUNKED_MAX_DK} state rows")
+    if heads % groups:
+        raise KernelError(f"{heads} heads do not divide into {groups} groups")
+    _columns(width, ("q_col", q_col, groups * dk), ("k_col", k_col, groups * dk), ("x_col", x_col, heads * dv))
+    base, slot_stride = _state_window(state, state_offset, heads * dk * dv, "state")
+    item_seq, item_row0, item_count, n_items = items
+    dev = vectors.device
+    out = torch.empty((T, heads * dv), dtype=torch.float32, device=dev)
+    sums = torch.empty((T, heads, 3), dtype=torch.float32, device=dev)
+    chunk_state = torch.empty((n_items, heads * dv * dk), dtype=torch.float32, device=dev)
+    total = torch.empty((n_items, heads), dtype=torch.float32, device=dev)
+    rc = _fn("recurrent_chunks", "za_decay_chunked")(
+        _ptr(vectors), width, int(q_col), int(k_col), int(x_col), _ptr(proj), _code(proj.dtype) if proj is not None else 0,
+        proj.shape[1] if proj is not None else 0, int(gate_col), _ptr(dt_bias), _ptr(A_log), _ptr(D), _ptr(fixed),
+        base, slot_stride, _ptr(slot_id), _ptr(item_seq), _ptr(item_row0), _ptr(item_count), n_items, S,
+        _ptr(sums), _ptr(chunk_state), _ptr(total), _ptr(out), T, heads, groups, dk, dv, _stream())
+    _check(rc, "recurrence in chunks", f"heads={heads} dk={dk} dv={dv} items={n_items}")
+    return out
 
 
 def fixed_decay_recurrence_chunked(vectors: torch.Tensor, q_col: int, k_col: int, x_col: int,
@@ -2201,36 +2265,71 @@ def fixed_decay_recurrence_chunked(vectors: torch.Tensor, q_col: int, k_col: int
                                    dv: int) -> torch.Tensor:
     """The fixed-decay walk of ``matrix_recurrence`` for steps with long portions: ``items``
     (``StepContext.attention_items(RETENTION_CHUNK)``: request, first row, rows, number) cut
-    every request's rows into chunks that are walked side by side from empty states; the
-    states before each chunk follow from a short pass over the chunks, and what they add to
-    each token's read-out is added afterwards (csrc/recurrent.hip).  Same result as the plain
-    walk up to the order of 32-bit additions."""
-    item_seq, item_row0, item_count, n_items = items
-    T, width = vectors.shape
-    S = slot_id.numel()
-    _need(vectors, "vectors", torch.float32)
+    every request's rows into chunks that are taken side by side as matrix products
+    (csrc/recurrent_chunks.hip).  Decays must not be negative.  Same result as the plain walk up
+    to the order of 32-bit additions."""
     _need(decay, "decay", torch.float32, (heads,))
+    return _decay_chunked(vectors, q_col, k_col, x_col, None, 0, None, None, None, decay, state, state_offset,
+                          slot_id, items, heads, heads, dk, dv)
+
+
+def ssd_recurrence_chunked(conv: torch.Tensor, q_col: int, k_col: int, x_col: int, proj: torch.Tensor,
+                           gate_col: int, dt_bias: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor,
+                           state: torch.Tensor, state_offset: int, slot_id: torch.Tensor, items, heads: int,
+                           groups: int, dk: int, dv: int) -> torch.Tensor:
+    """``matrix_recurrence``'s form ``"ssd"`` in chunks, as ``fixed_decay_recurrence_chunked``."""
+    _need(proj, "proj", (torch.float32, torch.bfloat16))
+    if proj.dim() != 2 or proj.shape[0] != conv.shape[0]:
+        raise KernelError(f"proj has shape {tuple(proj.shape)}, expected [{conv.shape[0]}, columns]")
+    _columns(proj.shape[1], ("gate_col", gate_col, heads))
+    for name, t in (("dt_bias", dt_bias), ("A_log", A_log), ("D", D)):
+        _need(t, name, torch.float32, (heads,))
+    return _decay_chunked(conv, q_col, k_col, x_col, proj, gate_col, dt_bias, A_log, D, None, state,
+                          state_offset, slot_id, items, heads, groups, dk, dv)
+
+
+def delta_recurrence_chunked(conv: torch.Tensor, q_col: int, k_col: int, x_col: int, proj: torch.Tensor,
+                             gate_col: int, decay: torch.Tensor, dt_bias: torch.Tensor, A_log: torch.Tensor,
+                             state: torch.Tensor, state_offset: int, slot_id: torch.Tensor, items,
+                             heads: int, groups: int, dk: int, dv: int) -> torch.Tensor:
+    """``matrix_recurrence``'s form ``"delta"`` for steps with long portions, in chunks of
+    ``DELTA_CHUNK`` tokens (``items``: ``StepContext.attention_items(DELTA_CHUNK)``) as matrix
+    products (csrc/recurrent_chunks.hip).  Same result up to the order of 32-bit operations."""
+    T, conv_width = conv.shape
+    _need(conv, "conv", torch.float32)
+    _need(proj, "proj", (torch.float32, torch.bfloat16))
+    if proj.dim() != 2 or proj.shape[0] != T:
+        raise KernelError(f"proj has shape {tuple(proj.shape)}, expected [{T}, columns]")
+    if heads % groups:
+        raise KernelError(f"{heads} heads do not divide into {groups} groups")
+    _columns(conv_width, ("q_col", q_col, groups * dk), ("k_col", k_col, groups * dk), ("x_col", x_col, heads * dv))
+    _columns(proj.shape[1], ("gate_col", gate_col, heads))
+    _need(A_log, "A_log", torch.float32, (heads,))
+    _need(decay, "decay", proj.dtype)
+    if decay.dim() != 2 or decay.shape[0] != T or decay.shape[1] < heads * dk:
+        raise KernelError(f"decay has shape {tuple(decay.shape)}, expected [{T}, >= {heads * dk}]")
+    _need(dt_bias, "dt_bias", torch.float32, (heads * dk,))
+    S = slot_id.numel()
     _need(slot_id, "slot_id", torch.int32, (S,))
-    for name, t in (("item_seq", item_seq), ("item_row0", item_row0), ("item_count", item_count)):
-        _need(t, name, torch.int32)
-        if t.numel() < n_items:
-            raise KernelError(f"{name} holds {t.numel()} entries, fewer than {n_items} items")
-    if n_items < S or dk > RETENTION_CHUNK_MAX_DK:
-        raise KernelError(f"{n_items} items for {S} requests, dk={dk}")
-    for name, col, n in (("q_col", q_col, heads * dk), ("k_col", k_col, heads * dk),
-                         ("x_col", x_col, heads * dv)):
-        if col < 0 or col + n > width:
-            raise KernelError(f"{name}: columns {col}..{col + n} of {width}")
+    _chunk_items(items, S, "delta rule in chunks")
+    if dk > CHUNKED_MAX_DK:
+        raise KernelError(f"dk={dk}: chunks take up to {CHUNKED_MAX_DK} state rows")
     base, slot_stride = _state_window(state, state_offset, heads * dk * dv, "state")
-    lanes, _, _ = recurrence_plan(dk, dv)
-    out = torch.empty((T, heads * dv), dtype=torch.float32, device=vectors.device)
-    chunk_state = torch.zeros((n_items, heads * dv * dk), dtype=torch.float32, device=vectors.device)
-    iota = torch.arange(n_items, dtype=torch.int32, device=vectors.device)
-    rc = _fn("recurrent", "za_retention_chunked")(
-        _ptr(vectors), width, int(q_col), int(k_col), int(x_col), _ptr(decay), base, slot_stride,
-        _ptr(slot_id), _ptr(item_seq), _ptr(item_row0), _ptr(item_count), _ptr(iota), n_items, S,
-        RETENTION_CHUNK, _ptr(chunk_state), _ptr(out), T, heads, dk, dv, lanes, _stream())
-    _check(rc, "fixed_decay_recurrence_chunked", f"heads={heads} dk={dk} dv={dv} items={n_items}")
+    item_seq, item_row0, item_count, n_items = items
+    dev = conv.device
+
+    def scratch(*shape):
+        return torch.empty(shape, dtype=torch.float32, device=dev)
+
+    out = scratch(T, heads * dv)
+    qp, W, kp, U, Q = (scratch(n_items, heads, DELTA_CHUNK, n) for n in (dk, dk, dk, dv, DELTA_CHUNK))
+    grow = scratch(n_items, heads, dk)
+    rc = _fn("recurrent_chunks", "za_delta_chunked")(
+        _code(proj.dtype), _ptr(conv), conv_width, int(q_col), int(k_col), int(x_col), _ptr(proj), proj.shape[1],
+        int(gate_col), _ptr(decay), decay.shape[1], _ptr(dt_bias), _ptr(A_log), base, slot_stride, _ptr(slot_id),
+        _ptr(item_seq), _ptr(item_row0), _ptr(item_count), n_items, S, _ptr(qp), _ptr(W), _ptr(U), _ptr(Q),
+        _ptr(kp), _ptr(grow), _ptr(out), T, heads, groups, dk, dv, _stream())
+    _check(rc, "delta rule in chunks", f"heads={heads} dk={dk} dv={dv} items={n_items}")
     return out
 
 

@@ -43,9 +43,9 @@ side by side are normed together, times a weight ``norm.weight`` of ``num_heads 
 and ``gate`` (``"silu"`` or ``"sigmoid"`` of the gate's projection, applied behind the norm).
 Lightning attention is ``activation="silu"``, ``key_scale=1``, ``output_norm="all"``,
 ``gate="sigmoid"`` and no position encoding.
-A step in which some request brings more than ``ops.RETENTION_CHUNK`` tokens walks its
-portions as chunks side by side (``ops.fixed_decay_recurrence_chunked``): with a constant
-decay the state is linear in what the tokens bring.
+A step with long portions takes them in chunks, as matrix products
+(``ops.fixed_decay_recurrence_chunked``; ``ssd`` and ``gated_delta`` have such forms too): the
+state is linear in what it was before a chunk.
 
 ``gated_linear`` (gated linear attention: a decay of its own for every key channel, made from
 the token).  Projections q, k (``num_heads x head_dim``), v and a gate g (``num_heads x
@@ -77,7 +77,7 @@ class StateSpaceDuality(Mixer):
     kind = "ssd"
     graph_safe = True
     takes_normed_rows = True      # ``x`` is only ever handed to ``ops.linear``
-    kernel_sources = ("gemm", "recurrent")
+    kernel_sources = ("gemm", "recurrent", "recurrent_chunks")
 
     @staticmethod
     def _sizes(params):
@@ -125,6 +125,9 @@ class StateSpaceDuality(Mixer):
         self.dt_bias, self.A_log, self.D = tensors["dt_bias"], tensors["A_log"], tensors["D"]
         self.norm_w = tensors["norm.weight"]
         self.conv_state = (self.inner + 2 * G * N) * (L - 1)      # floats before S in a slot
+        # long portions are taken in chunks (the step's work items of that size)
+        self.chunked = N <= ops.CHUNKED_MAX_DK
+        self.item_granularities = [ops.RETENTION_CHUNK] if self.chunked else []
         ops.check_projection_weight(self.w_in, "ssd in_proj")
         ops.check_projection_weight(self.w_out, "ssd out_proj")
 
@@ -133,10 +136,16 @@ class StateSpaceDuality(Mixer):
         z = ops.linear(x, self.w_in, tune=self.runtime.tune)
         conv = ops.causal_conv_silu(z, inner, self.conv_w, self.conv_b, cache.state, 0,
                                     step.token_seq, step.seq_start, step.slot_id)
-        y = ops.matrix_recurrence("ssd", conv, inner + G * N, inner, 0, z, 2 * inner + 2 * G * N,
-                                  None, self.dt_bias, self.A_log, self.D, cache.state,
-                                  self.conv_state, step.seq_start, step.slot_id, self.heads, G, N,
-                                  self.head_dim)
+        if self.chunked and ops.in_chunks(step.seq_lens_host):
+            items = step.attention_items(ops.RETENTION_CHUNK)
+            y = ops.ssd_recurrence_chunked(conv, inner + G * N, inner, 0, z, 2 * inner + 2 * G * N, self.dt_bias,
+                                           self.A_log, self.D, cache.state, self.conv_state, step.slot_id,
+                                           items, self.heads, G, N, self.head_dim)
+        else:
+            y = ops.matrix_recurrence("ssd", conv, inner + G * N, inner, 0, z, 2 * inner + 2 * G * N,
+                                      None, self.dt_bias, self.A_log, self.D, cache.state,
+                                      self.conv_state, step.seq_start, step.slot_id, self.heads, G, N,
+                                      self.head_dim)
         h = ops.gated_group_norm(y, z, 0, self.norm_w, inner // self.norm_groups, self.eps,
                                  "silu", gate_first=True)
         return ops.linear(h, self.w_out, tune=self.runtime.tune)
@@ -146,7 +155,7 @@ class GatedDeltaRule(Mixer):
     kind = "gated_delta"
     graph_safe = True
     takes_normed_rows = True      # ``x`` is only ever handed to ``ops.linear``
-    kernel_sources = ("gemm", "recurrent", "activation")
+    kernel_sources = ("gemm", "recurrent", "recurrent_chunks", "activation")
 
     @staticmethod
     def _sizes(params):
@@ -210,6 +219,9 @@ class GatedDeltaRule(Mixer):
         self.norm_w = tensors["norm.weight"]
         self.w_out = ops.projection_weight(tensors["out_proj.weight"])
         self.conv_state = (2 * G * d + H * dv) * (L - 1)
+        # long portions are taken in chunks (the step's work items of that size)
+        self.chunked = d <= ops.CHUNKED_MAX_DK
+        self.item_granularities = [ops.DELTA_CHUNK] if self.chunked else []
         for w, what in ((self.w_in, "in"), (self.w_up, "low-rank up"), (self.w_out, "out")):
             ops.check_projection_weight(w, f"gated_delta {what} projection")
 
@@ -220,9 +232,15 @@ class GatedDeltaRule(Mixer):
                                     step.seq_start, step.slot_id)
         low = ops.copy_columns(z, self.low_col, self.low_width)
         up = ops.linear(low, self.w_up, tune=self.runtime.tune)      # decay: H*d | gate: H*dv
-        o = ops.matrix_recurrence("delta", conv, 0, G * d, 2 * G * d, z, self.beta_col, up,
-                                  self.dt_bias, self.A_log, None, cache.state, self.conv_state,
-                                  step.seq_start, step.slot_id, H, G, d, dv)
+        if self.chunked and ops.in_chunks(step.seq_lens_host):
+            items = step.attention_items(ops.DELTA_CHUNK)
+            o = ops.delta_recurrence_chunked(conv, 0, G * d, 2 * G * d, z, self.beta_col, up, self.dt_bias,
+                                             self.A_log, cache.state, self.conv_state, step.slot_id, items, H,
+                                             G, d, dv)
+        else:
+            o = ops.matrix_recurrence("delta", conv, 0, G * d, 2 * G * d, z, self.beta_col, up,
+                                      self.dt_bias, self.A_log, None, cache.state, self.conv_state,
+                                      step.seq_start, step.slot_id, H, G, d, dv)
         h = ops.gated_group_norm(o, up, H * d, self.norm_w, dv, self.eps, "sigmoid",
                                  gate_first=False)
         return ops.linear(h, self.w_out, tune=self.runtime.tune)
@@ -233,7 +251,7 @@ class Retention(Mixer):
     graph_safe = True
     takes_normed_rows = True      # ``x`` is only ever handed to ``ops.linear``
     accepts_stream = True         # ``forward`` takes ``stream`` and may add its result there
-    kernel_sources = ("gemm", "recurrent")
+    kernel_sources = ("gemm", "recurrent", "recurrent_chunks")
 
     @staticmethod
     def _sizes(params):
@@ -293,8 +311,8 @@ class Retention(Mixer):
         else:
             self.norm_w = torch.ones((1,), dtype=torch.float32, device=runtime.device)
             self.norm_group = dv
-        # long portions are walked in chunks side by side (the step's work items of that size)
-        self.chunked = d <= ops.RETENTION_CHUNK_MAX_DK
+        # long portions are taken in chunks (the step's work items of that size)
+        self.chunked = d <= ops.CHUNKED_MAX_DK and all(x >= 0.0 for x in decay)
         self.item_granularities = [ops.RETENTION_CHUNK] if self.chunked else []
         ops.check_projection_weight(self.w_in, "retention opening projection")
         ops.check_projection_weight(self.w_out, "retention out_proj")
@@ -306,10 +324,8 @@ class Retention(Mixer):
             z, 0, H * d, 2 * H * d, step.positions,
             self.position.inv_freq if self.rotary_dim else None, H, d, dv, self.rotary_dim,
             self.k_scale, self.activation)
-        items = step.attention_items(ops.RETENTION_CHUNK) if self.chunked else None
-        if items is not None and items[3] > step.n_seqs:
-            # some request brings more than a chunk: chunks side by side (a function of the
-            # step's shape alone)
+        if self.chunked and ops.in_chunks(step.seq_lens_host):
+            items = step.attention_items(ops.RETENTION_CHUNK)
             o = ops.fixed_decay_recurrence_chunked(vectors, 0, H * d, 2 * H * d, self.decay,
                                                    cache.state, 0, step.slot_id, items, H, d, dv)
         else:

@@ -661,6 +661,23 @@ def test_latent_attention_kernels(H, W, R, page_size):
         assert float((got - want).abs().max()) < 2e-2, nsplit
 
 
+@pytest.mark.parametrize("H,R,rotated,page_size", [
+    (16, 512, 64, 16), (16, 512, 32, 64), (3, 512, 0, 16), (70, 256, 64, 8), (5, 256, 32, 16), (64, 256, 0, 4),
+    (1, 128, 64, 16), (9, 128, 32, 32), (40, 128, 0, 16), (2, 512, 64, 12)])
+def test_latent_prefill_on_whole_tiles(H, R, rotated, page_size):
+    """Rows that the tiled kernel takes (the last: a page size that it leaves to the other)."""
+    from zig_ai_amd.kernels import ops
+    requests = [(70, 9), (0, 150), (133, 1), (0, 1), (31, 34), (64, 64), (63, 2), (191, 1)]
+    W, most = R + rotated, ops.LATENT_MFMA_ROWS
+    q, plane, table, pos, iseq, irow, icnt, n, scale, sink, want = _latent_attention_case(
+        torch.bfloat16, H, W, R, requests, page_size, max(1, most // min(H, most)), seed=H + W)
+    for keys, nsplit in ((0, 1), (64, 4), (128, 2)):
+        got = ops.latent_attention(q, plane, R, table, pos, iseq, irow, icnt, n, scale, sink, keys, nsplit,
+                                   4).cpu().double()
+        # (the probabilities and the result in bfloat16: 2^-9 of values up to 4 either time)
+        assert float((got - want).abs().max()) < 2e-2, nsplit
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,N,K,mode", [(3, 24, 16, None), (8, 128, 64, "element"), (5, 40, 32, "head"),
                                         (1, 8, 320, "element"), (40, 72, 8, None)])

@@ -19,8 +19,10 @@
 //   latent_attention   the attention itself: causal, streaming softmax in 32-bit with a sink
 //                      a head, any mix of prompt portions and single tokens in one launch,
 //                      contexts optionally cut into ranges (latent_combine merges them)
-//   latent_attention_mfma   the same on the matrix cores (bfloat16, 16-byte pieces): four waves
-//                      of 16 rows each for prompt portions and mixed steps
+//   latent_prefill_mfma     the same on the matrix cores for prompt portions and mixed steps:
+//                      latents of 128, 256 or 512 with up to 64 rotated elements
+//   latent_attention_mfma   the same for other widths (bfloat16, 16-byte pieces): four waves of
+//                      16 rows each
 //   latent_decode_mfma      steps that only decode: four waves share 16 rows
 // Rotation: adjacent pairs (2i, 2i + 1) or halves (i, i + dims/2) of the first `rot_dims`
 // elements, angle = position * inv_freq[i] in 32-bit, cosine and sine times `magnitude`.
@@ -805,6 +807,396 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ 
   }
 }
 
+// ------------------------------------------------------------ latent_prefill_mfma
+// The same for prompt portions and mixed steps where R is 128, 256 or 512 and the rotated part
+// 0, 32 or 64: eight waves serve one work item and one chunk of heads, at most 64 rows, 64 keys
+// a tile, and every fragment serves all the rows that it can.
+//   tiles    go from memory into one of two places in LDS without passing registers, a wave
+//            eight keys, the next tile while this one is used.  A key's 16-byte pieces lie in
+//            the order piece ^ (key % 8), so that neither kind of read meets a bank twice.
+//   S^T      wave w takes the 16 keys w % 4 and 32 rows (w / 4): a fragment of keys serves two
+//            products, and the rows stay in registers
+//   softmax  the waves' maxima meet in LDS; every wave then holds every row's maximum, and
+//            leaves its probabilities (bfloat16) in LDS
+//   O^T      wave w takes R / 8 of the latent for all 64 rows: the tile's keys are read turned
+//            round (ds_read_b64_tr_b16: of 4 keys x 16 elements a lane gets one element's four
+//            keys), each once a workgroup
+// Reads of LDS and matrix products would bound it in equal parts (35 fragments for 68 products a
+// wave and tile at R = 512 with 64 rotated); what does are the waits between them, three meetings
+// of the waves a tile.  (Four waves that each take 16 rows through the whole tile, as below for
+// other widths, read a fragment for every product and wait for each, one wave a SIMD.)
+// 16 heads, a first portion of 1,777 tokens, R = 512 with 64 rotated: 115 us against 313 of that
+// form, R = 256: 84 against 191, R = 128: 71 against 147; 8 tokens behind 2,048 cached ones beside
+// 256 new ones 68 against 99; 40 tokens of 4 heads 18 against 20.  Its error against 64 bits is the
+// same (1.85e-3 of the result's norm, the rounding of probabilities and result).
+#define LP_KT 64
+#define LP_NT 512
+#define LP_PAIRS 2          // pairs of fragments that a wave takes at once (3: registers run over)
+
+__device__ __forceinline__ unsigned lp_lds(const void* p) {
+  return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)p;
+}
+
+// The waits are written by hand: the compiler would wait for the next tile's requests before
+// any read of LDS.
+__device__ __forceinline__ void lp_meet() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Fragments 2 * PAIRS from two addresses, 128 bytes from pair to pair.
+template <int PAIRS>
+__device__ __forceinline__ void lp_take_keys(bf16x8_t (&f)[6], unsigned even, unsigned odd) {
+  if constexpr (PAIRS == 3)
+    asm volatile(
+        "ds_read_b128 %0, %6 offset:0\n" "ds_read_b128 %1, %7 offset:0\n"
+        "ds_read_b128 %2, %6 offset:128\n" "ds_read_b128 %3, %7 offset:128\n"
+        "ds_read_b128 %4, %6 offset:256\n" "ds_read_b128 %5, %7 offset:256\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5])
+        : "v"(even), "v"(odd)
+        : "memory");
+  if constexpr (PAIRS == 2)
+    asm volatile(
+        "ds_read_b128 %0, %4 offset:0\n" "ds_read_b128 %1, %5 offset:0\n"
+        "ds_read_b128 %2, %4 offset:128\n" "ds_read_b128 %3, %5 offset:128\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
+        : "v"(even), "v"(odd)
+        : "memory");
+  if constexpr (PAIRS == 1)
+    asm volatile(
+        "ds_read_b128 %0, %2 offset:0\n" "ds_read_b128 %1, %3 offset:0\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(f[0]), "=&v"(f[1])
+        : "v"(even), "v"(odd)
+        : "memory");
+}
+
+// Of 32 keys: the probabilities of four times 16 rows and the first one or two tiles of the
+// latent (from two addresses each), or the next two tiles alone.
+template <int TILES, bool P>
+__device__ __forceinline__ void lp_take_values(bf16x8_t (&p)[4], bf16x4_t (&v)[TILES][2], unsigned pa,
+                                               const unsigned (&va)[TILES][2]) {
+  if constexpr (TILES == 2 && P)
+    asm volatile(
+        "ds_read_b128 %0, %8 offset:0\n" "ds_read_b128 %1, %8 offset:2048\n"
+        "ds_read_b128 %2, %8 offset:4096\n" "ds_read_b128 %3, %8 offset:6144\n"
+        "ds_read_b64_tr_b16 %4, %9\n" "ds_read_b64_tr_b16 %5, %10\n"
+        "ds_read_b64_tr_b16 %6, %11\n" "ds_read_b64_tr_b16 %7, %12\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3]), "=&v"(v[0][0]), "=&v"(v[0][1]),
+          "=&v"(v[1][0]), "=&v"(v[1][1])
+        : "v"(pa), "v"(va[0][0]), "v"(va[0][1]), "v"(va[1][0]), "v"(va[1][1])
+        : "memory");
+  if constexpr (TILES == 2 && !P)
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4\n" "ds_read_b64_tr_b16 %1, %5\n"
+        "ds_read_b64_tr_b16 %2, %6\n" "ds_read_b64_tr_b16 %3, %7\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v[0][0]), "=&v"(v[0][1]), "=&v"(v[1][0]), "=&v"(v[1][1])
+        : "v"(va[0][0]), "v"(va[0][1]), "v"(va[1][0]), "v"(va[1][1])
+        : "memory");
+  if constexpr (TILES == 1)
+    asm volatile(
+        "ds_read_b128 %0, %6 offset:0\n" "ds_read_b128 %1, %6 offset:2048\n"
+        "ds_read_b128 %2, %6 offset:4096\n" "ds_read_b128 %3, %6 offset:6144\n"
+        "ds_read_b64_tr_b16 %4, %7\n" "ds_read_b64_tr_b16 %5, %8\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3]), "=&v"(v[0][0]), "=&v"(v[0][1])
+        : "v"(pa), "v"(va[0][0]), "v"(va[0][1])
+        : "memory");
+}
+
+template <int RT, int DT>
+struct LpShape {
+  static constexpr int R = RT * 16, W = R + DT * 32, WS = W / 32;
+  static constexpr int PIECES = (WS * 4 + 7) / 8 * 8;      // of a key in LDS
+  static constexpr int TILE = LP_KT * PIECES * 8;          // elements of a place
+  static constexpr int KEPT = WS < 17 ? WS : 17;           // steps of the rows in registers; the rest in LDS
+  static constexpr size_t LDS = (size_t)2 * TILE * 2 + 64 * LP_KT * 2 + 64 * 4 * 4 + (WS - KEPT) * 64 * 32 * 2;
+};
+
+template <int RT, int DT>
+__global__ void __launch_bounds__(LP_NT)
+latent_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
+                           const bf16_t* __restrict__ plane, long long page_stride,
+                           const int* __restrict__ block_table, int bt_stride,
+                           const int* __restrict__ positions, const int* __restrict__ wi_seq,
+                           const int* __restrict__ wi_row0, const int* __restrict__ wi_count,
+                           float* __restrict__ part_acc, float* __restrict__ part_ml, int H,
+                           int HC, int page_shift, float scale_log2,
+                           int keys_per_split, int nsplit, const float* __restrict__ sink) {
+  using S = LpShape<RT, DT>;
+  constexpr int R = S::R, W = S::W, WS = S::WS, NP = S::PIECES, OT = RT / 8, KEPT = S::KEPT;
+  static_assert(WS - KEPT <= 1, "one step of the rows in LDS at most");
+  extern __shared__ __attribute__((aligned(16))) unsigned char lm_lds[];
+  bf16_t* Ks = reinterpret_cast<bf16_t*>(lm_lds);                 // [2][LP_KT][NP * 8]
+  bf16_t* Ps = Ks + 2 * S::TILE;                                  // [64 rows][LP_KT]
+  float* Xs = reinterpret_cast<float*>(Ps + 64 * LP_KT);          // [64 rows][4]
+  bf16_t* Qs = reinterpret_cast<bf16_t*>(Xs + 64 * 4);            // [4][64 lanes][8]: the rows' last step
+
+  // the last items first: within a request the later an item, the more keys it has, and
+  // workgroups start in the order of their numbers, so the long ones do not start last
+  const int item = gridDim.x - 1 - blockIdx.x, z = blockIdx.z;
+  const int h0 = blockIdx.y * HC;
+  const int G = min(HC, H - h0);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int kt = wave & 3, rh = wave >> 2;
+  const int seq = wi_seq[item];
+  const int row0 = wi_row0[item];
+  int count = wi_count[item];
+  if (count * G > 64) count = 64 / G;               // the host never asks for more
+  const int rows = count * G;
+  const int hi = positions[row0 + count - 1];       // inclusive
+  int range_lo = z * keys_per_split;
+  int range_hi = range_lo + keys_per_split - 1;
+  if (nsplit == 1) { range_lo = 0; range_hi = hi; }
+  if (range_hi > hi) range_hi = hi;
+  const int* table = block_table + (size_t)seq * bt_stride;
+
+  // the page of key wave * 8 + lane % 8 of a tile (a key beyond the range reads the range's last
+  // one, whose scores are then masked)
+  auto page_of = [&](int tile0) -> int {
+    const int kp = min(tile0 + wave * 8 + (lane & 7), range_hi);
+    return table[kp >> page_shift];
+  };
+  auto request = [&](int page, int tile0, int buffer) {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));                  // (worked out again for each tile: registers)
+    const int kp = min(tile0 + wave * 8 + (lane & 7), range_hi);
+    const int off = kp & ((1 << page_shift) - 1);
+    const long long at = (long long)max(page, 0) * page_stride + (long long)off * W;
+    long long base[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      base[j] = (long long)((unsigned)__builtin_amdgcn_readlane((int)at, j)) |
+                ((long long)__builtin_amdgcn_readlane((int)(at >> 32), j) << 32);
+    bf16_t* to = Ks + buffer * S::TILE + wave * 8 * NP * 8;
+#pragma unroll
+    for (int i = 0; i < NP / 8; ++i) {
+      long long from = base[i * 64 / NP];
+      int key = i * 64 / NP;
+#pragma unroll
+      for (int j = i * 64 / NP + 1; j <= (i * 64 + 63) / NP; ++j)
+        if (lane >= j * NP - i * 64) { from = base[j]; key = j; }
+      int piece = (i * 64 + lane - key * NP) ^ key;
+      if (WS % 2 && piece >= W / 8) piece = 0;       // room that no fragment reads
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(plane + from + piece * 8),
+          (__attribute__((address_space(3))) void*)(to + i * 512), 16, 0, 0);
+    }
+  };
+
+  int page = 0;                // of the tile that is requested next
+  if (range_lo <= range_hi) {
+    request(page_of(range_lo), range_lo, 0);
+    page = page_of(range_lo + LP_KT);
+  }
+
+  // this wave's rows of the first product
+  bf16x8_t qf[2][KEPT];
+  int pos_q[2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    const int my = (rh * 2 + a) * 16 + r16;
+    const bool row_ok = my < rows;
+    const int tok = row0 + (row_ok ? my / G : 0), h = h0 + (row_ok ? my % G : 0);
+    pos_q[a] = row_ok ? positions[tok] : -1;
+    const bf16_t* qrow = q + ((size_t)tok * H + h) * W + kq * 8;     // (a row beyond: masked below)
+#pragma unroll
+    for (int ks = 0; ks < KEPT; ++ks) qf[a][ks] = *reinterpret_cast<const bf16x8_t*>(qrow + ks * 32);
+    if (KEPT < WS && kt == 0) {
+      const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(qrow + KEPT * 32);
+      asm volatile("ds_write_b128 %0, %1" ::"v"(lp_lds(Qs) + (rh * 2 + a) * 1024 + lane * 16), "v"(v) : "memory");
+    }
+  }
+  float m[4], l[2] = {0.f, 0.f};
+  f32x4_t o[4][OT];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    m[a] = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < OT; ++t) o[a][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+
+  const unsigned ks_at = lp_lds(Ks), ps_at = lp_lds(Ps), xs_at = lp_lds(Xs);
+  int buffer = 0;
+  for (int tile0 = range_lo; tile0 <= range_hi; tile0 += LP_KT, buffer ^= 1) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lp_meet();            // this tile is here, and nobody reads the other place any more
+    if (tile0 + LP_KT <= range_hi) {
+      request(page, tile0 + LP_KT, buffer ^ 1);
+      page = page_of(tile0 + 2 * LP_KT);
+    }
+    const unsigned in_buffer = buffer * S::TILE * 2;
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int r16 = lane & 15, kq = lane >> 4;
+    const unsigned key_row = ks_at + (kt * 16 + r16) * NP * 16 + in_buffer;
+    const unsigned even = key_row + ((kq ^ (r16 & 7)) << 4), odd = even ^ 64;
+    f32x4_t s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    constexpr int PAIRS = (WS + 1) / 2;
+#pragma unroll
+    for (int b = 0; b < PAIRS; b += LP_PAIRS) {
+      bf16x8_t kf[6];
+      if (b + LP_PAIRS <= PAIRS) lp_take_keys<LP_PAIRS>(kf, even + b * 128, odd + b * 128);
+      else if (PAIRS - b == 2) lp_take_keys<2>(kf, even + b * 128, odd + b * 128);
+      else lp_take_keys<1>(kf, even + b * 128, odd + b * 128);
+#pragma unroll
+      for (int i = 0; i < 2 * LP_PAIRS; ++i) {
+        const int ks = b * 2 + i;
+        if (KEPT < WS && ks == KEPT) {
+          bf16x8_t qs[2];
+          asm volatile("ds_read_b128 %0, %2\n" "ds_read_b128 %1, %2 offset:1024\n" "s_waitcnt lgkmcnt(0)"
+                       : "=&v"(qs[0]), "=&v"(qs[1])
+                       : "v"(lp_lds(Qs) + rh * 2048 + lane * 16)
+                       : "memory");
+          s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i], qs[0], s[0], 0, 0, 0);
+          s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i], qs[1], s[1], 0, 0, 0);
+        } else if (ks < KEPT) {
+          s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i], qf[0][ks], s[0], 0, 0, 0);
+          s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i], qf[1][ks], s[1], 0, 0, 0);
+        }
+      }
+    }
+    float top[2];
+    const int kp0 = tile0 + kt * 16 + kq * 4;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      top[a] = -INFINITY;
+      const int last = min(pos_q[a], range_hi);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[a][i] = kp0 + i <= last ? s[a][i] * scale_log2 : -INFINITY;
+        top[a] = fmaxf(top[a], s[a][i]);
+      }
+      top[a] = fmaxf(top[a], __shfl_xor(top[a], 16, 64));
+      top[a] = fmaxf(top[a], __shfl_xor(top[a], 32, 64));
+    }
+    if (kq < 2)
+      asm volatile("ds_write_b32 %0, %1" ::"v"(xs_at + (((rh * 2 + kq) * 16 + r16) * 4 + kt) * 4),
+                   "v"(kq ? top[1] : top[0]) : "memory");
+    lp_meet();
+    float alpha[4];
+#pragma unroll
+    for (int b = 0; b < 4; b += 2) {
+      f32x4_t seen[2];
+      asm volatile("ds_read_b128 %0, %2\n" "ds_read_b128 %1, %2 offset:256\n" "s_waitcnt lgkmcnt(0)"
+                   : "=&v"(seen[0]), "=&v"(seen[1])
+                   : "v"(xs_at + r16 * 16 + b * 256)
+                   : "memory");
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int a = b + i;
+        const float m_new = fmaxf(fmaxf(fmaxf(seen[i][0], seen[i][1]), fmaxf(seen[i][2], seen[i][3])), m[a]);
+        alpha[a] = m[a] == m_new ? 1.0f : exp2f(m[a] - m_new);
+        m[a] = m_new;
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const float mx = rh ? m[2 + a] : m[a];
+      const float m_use = mx > -INFINITY ? mx : 0.f;
+      bf16x4_t pb;
+      float psum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        pb[i] = (bf16_t)exp2f(s[a][i] - m_use);
+        psum += (float)pb[i];
+      }
+      l[a] = l[a] * (rh ? alpha[2 + a] : alpha[a]) + psum;
+      asm volatile("ds_write_b64 %0, %1" ::"v"(ps_at + ((rh * 2 + a) * 16 + r16) * (LP_KT * 2) +
+                                               (((kt * 2 + (kq >> 1)) ^ (r16 & 7)) << 4) + (kq & 1) * 8),
+                   "v"(pb) : "memory");
+    }
+    lp_meet();
+    if (!__all(alpha[0] == 1.0f && alpha[1] == 1.0f && alpha[2] == 1.0f && alpha[3] == 1.0f)) {
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int t = 0; t < OT; ++t) {
+          o[a][t][0] *= alpha[a]; o[a][t][1] *= alpha[a];
+          o[a][t][2] *= alpha[a]; o[a][t][3] *= alpha[a];
+        }
+    }
+#pragma unroll
+    for (int step = 0; step < LP_KT / 32; ++step) {
+      int lane = threadIdx.x & 63;
+      asm volatile("" : "+v"(lane));
+      const int r16 = lane & 15, kq = lane >> 4;
+      constexpr int TILES = OT < 2 ? OT : 2;
+      bf16x8_t pf[4];
+#pragma unroll
+      for (int t0 = 0; t0 < OT; t0 += TILES) {
+        unsigned va[TILES][2];
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {
+            const int low = hf * 4 + (r16 >> 2);         // of the key that this lane points at
+            const int piece = (wave * OT + t0 + t) * 2 + ((r16 >> 1) & 1);
+            va[t][hf] = ks_at + in_buffer + (step * 32 + kq * 8 + low) * NP * 16 + ((piece ^ low) << 4) +
+                        (r16 & 1) * 8;
+          }
+        bf16x4_t vh[TILES][2];
+        const unsigned pa = ps_at + r16 * (LP_KT * 2) + (((step * 4 + kq) ^ (r16 & 7)) << 4);
+        if (t0 == 0) lp_take_values<TILES, true>(pf, vh, pa, va);
+        else lp_take_values<TILES, false>(pf, vh, pa, va);
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+          const bf16x8_t vf = __builtin_shufflevector(vh[t][0], vh[t][1], 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+          for (int a = 0; a < 4; ++a)
+            o[a][t0 + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[a], o[a][t0 + t], 0, 0, 0);
+        }
+      }
+    }
+  }
+
+  // the rows' sums meet like their maxima
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    l[a] += __shfl_xor(l[a], 16, 64);
+    l[a] += __shfl_xor(l[a], 32, 64);
+  }
+  __syncthreads();
+  if (kq < 2) Xs[((rh * 2 + kq) * 16 + r16) * 4 + kt] = kq ? l[1] : l[0];
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int my = a * 16 + r16;
+    if (my >= rows) continue;
+    const int tok = row0 + my / G, h = h0 + my % G;
+    const f32x4_t part = *reinterpret_cast<const f32x4_t*>(Xs + my * 4);
+    float lt = (part[0] + part[1]) + (part[2] + part[3]);
+    const int e = wave * OT * 16 + kq * 4;
+    if (nsplit == 1) {
+      if (sink) lt += exp2f(sink[h] * LM_LOG2E - m[a]);
+      const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+      bf16_t* orow = out + ((size_t)tok * H + h) * R + e;
+#pragma unroll
+      for (int t = 0; t < OT; ++t) {
+        bf16x4_t v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (bf16_t)(o[a][t][i] * inv);
+        *reinterpret_cast<bf16x4_t*>(orow + t * 16) = v;
+      }
+    } else {
+      const size_t pidx = ((size_t)tok * H + h) * nsplit + z;
+      float* pa = part_acc + pidx * R + e;
+#pragma unroll
+      for (int t = 0; t < OT; ++t) *reinterpret_cast<f32x4_t*>(pa + t * 16) = o[a][t];
+      if (wave == 0 && kq == 0) {
+        part_ml[pidx * 2] = m[a] * LM_LN2;
+        part_ml[pidx * 2 + 1] = lt;
+      }
+    }
+  }
+}
+
 template <int WS, int RT>
 __global__ void __launch_bounds__(LM_NT)
 latent_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
@@ -1086,6 +1478,33 @@ static int launch_latent_mfma(const void* q, void* out, const void* plane, long 
   return za_launch_status();
 }
 
+template <int RT, int DT>
+static int launch_latent_prefill(const void* q, void* out, const void* plane, long long page_stride,
+                                 const int* block_table, int bt_stride, const int* positions,
+                                 const int* wi_seq, const int* wi_row0, const int* wi_count,
+                                 int n_items, float* part_acc, float* part_ml, int H, int W, int R,
+                                 int page_size, float scale, int keys_per_split, int nsplit,
+                                 const float* sink, hipStream_t stream) {
+  using S = LpShape<RT, DT>;
+  auto kernel = latent_prefill_mfma_kernel<RT, DT>;
+  static bool allowed = false;
+  if (!allowed) {
+    hipError_t e = hipFuncSetAttribute((const void*)kernel,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::LDS);
+    if (e != hipSuccess) return (int)e;
+    allowed = true;
+  }
+  int shift = 0;
+  while ((1 << shift) < page_size) ++shift;
+  const int HC = H < 64 ? H : 64;
+  dim3 grid(n_items, (H + HC - 1) / HC, nsplit), block(LP_NT);
+  hipLaunchKernelGGL(kernel, grid, block, S::LDS, stream, (const bf16_t*)q, (bf16_t*)out,
+                     (const bf16_t*)plane, page_stride, block_table, bt_stride, positions, wi_seq,
+                     wi_row0, wi_count, part_acc, part_ml, H, HC, shift,
+                     scale * LM_LOG2E, keys_per_split, nsplit, sink);
+  return za_launch_status();
+}
+
 // The matrix-core form: bfloat16, `width` and `kv_rank` multiples of 8.  `waves`: 4 (work
 // items of at most 64 / min(heads, 64) tokens, 16 rows a wave) or 1 (single tokens, as a
 // step that only decodes has: heads in chunks of 16 whose rows the four waves share).
@@ -1114,7 +1533,18 @@ extern "C" int za_latent_attention_mfma(const void* q, void* out, const void* pl
   q, out, plane, page_stride, block_table, bt_stride, positions, wi_seq, wi_row0, wi_count,     \
       n_items, part_acc, part_ml, heads, width, kv_rank, page_size, scale, keys_per_split,      \
       nsplit, sink, stream
-  if (ws <= 6 && rt <= 8)
+  const int rotated = width - kv_rank;
+  const bool whole = (kv_rank == 128 || kv_rank == 256 || kv_rank == 512) && rotated % 32 == 0 && rotated <= 64 &&
+                     (page_size & (page_size - 1)) == 0;
+#define ZA_LP(RT)                                                                               \
+  rc = rotated == 0    ? launch_latent_prefill<RT, 0>(ZA_LM_ARGS)                               \
+       : rotated == 32 ? launch_latent_prefill<RT, 1>(ZA_LM_ARGS)                               \
+                       : launch_latent_prefill<RT, 2>(ZA_LM_ARGS)
+  if (waves == 4 && whole) {
+    if (kv_rank == 128) ZA_LP(8);
+    else if (kv_rank == 256) ZA_LP(16);
+    else ZA_LP(32);
+  } else if (ws <= 6 && rt <= 8)
     rc = waves == 4 ? launch_latent_mfma<6, 8, false>(ZA_LM_ARGS)
                     : launch_latent_mfma<6, 8, true>(ZA_LM_ARGS);
   else if (ws <= 10 && rt <= 16)
@@ -1123,6 +1553,7 @@ extern "C" int za_latent_attention_mfma(const void* q, void* out, const void* pl
   else
     rc = waves == 4 ? launch_latent_mfma<18, 32, false>(ZA_LM_ARGS)
                     : launch_latent_mfma<18, 32, true>(ZA_LM_ARGS);
+#undef ZA_LP
 #undef ZA_LM_ARGS
   if (rc != 0 || nsplit == 1) return rc;
   dim3 grid((unsigned)((size_t)n_tokens * heads));

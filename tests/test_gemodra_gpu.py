@@ -700,6 +700,34 @@ def test_head_linear_kernel(dtype, H, N, K, mode):
     assert float((got - want).abs().max()) < tol * max(1.0, float(want.abs().max()))
 
 
+@pytest.mark.parametrize("T", [1, 16, 17, 64, 65, 200])
+@pytest.mark.parametrize("H,N,K,mode", [(3, 140, 264, "element"), (2, 128, 512, "head"), (5, 70, 128, "element"),
+                                        (1, 512, 136, None), (4, 16, 8, None)])
+def test_head_linear_at_the_edges_of_its_tiles(T, H, N, K, mode):
+    """Rows of decode batches and of tiles, K split or not and off the tiles' 64, columns that do
+    and do not fill 16-byte stores, into rows wider than the result."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(T + N + K)
+    x = torch.randn(T, H, K + 16, generator=g).bfloat16()
+    w = (torch.randn(H, N, K, generator=g) * K ** -0.5).bfloat16()
+    gate = torch.randn(T, 4 + (H if mode == "head" else H * N), generator=g).bfloat16()
+    for dtype in (torch.bfloat16, torch.float32):
+        out = torch.full((T, H, N + 8), 7.0, dtype=dtype, device=dev)
+        ops.head_linear(x.to(dev), 8, w.to(dev), out=out, out_col=4, gate=gate.to(dev) if mode else None,
+                        gate_col=4, gate_mode=mode)
+        want = torch.einsum("thk,hnk->thn", x[:, :, 8:8 + K].double(), w.double())
+        if mode == "head":
+            want = want * torch.sigmoid(gate[:, 4:].double())[:, :, None]
+        elif mode == "element":
+            want = want * torch.sigmoid(gate[:, 4:].double()).view(T, H, N)
+        got = out.cpu().double()
+        # (32-bit sums of K products; one rounding to bfloat16 on the way out)
+        bound = (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -20) * max(1.0, float(want.abs().max()))
+        assert float((got[:, :, 4:-4] - want).abs().max()) < bound
+        assert bool((got[:, :, :4] == 7).all()) and bool((got[:, :, -4:] == 7).all())
+
+
 def test_token_side_kernels():
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")

@@ -29,6 +29,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "tiles_bf16.h"
 
 // ------------------------------------------------------------------ latent_prepare
 // down: [T][ld], columns [q_col, q_col + Rq) the query latent, [c_col, c_col + R) the
@@ -196,67 +197,138 @@ __device__ __forceinline__ float head_gate_of(const HeadLinearArgs& a, int t, in
   return 1.0f / (1.0f + expf(-z));
 }
 
-// bfloat16 on the matrix cores, operands straight from memory into the fragments
-// (v_mfma_f32_16x16x32_bf16: lane l supplies row (l % 16), k-slots (l / 16) * 8 .. + 7 of
-// either operand and receives rows (l / 16) * 4 .. + 3, column (l % 16) of the product).
-// TM = 64: four waves of 16 rows x 64 columns; TM = 16 (decode batches): four waves of 16
-// columns each.
-template <int TM, typename TO>
+// A decode batch (at most 16 rows), bfloat16 on the matrix cores, operands straight from memory into
+// the fragments (layout: tiles_bf16.h), 128 elements of K under way at once a wave.  SPLIT: a
+// workgroup has 16 columns of one head, its four waves a quarter of K each, which meet in LDS;
+// otherwise 64 columns, 16 a wave.  What bounds it is the way to memory and back, once with K up to
+// 512: 8 rows of 16 heads, [128 x 512] with a gate an element 2.9 us (64 columns a workgroup, a
+// wave the whole of K in steps of 64: 5.8); [512 x 128] 3.1 (SPLIT 3.6: so from K = 256 on).
+#define HL_SPLIT_MIN_K 256
+template <typename TO, bool SPLIT>
 __global__ void __launch_bounds__(256)
-head_linear_bf16_kernel(HeadLinearArgs a) {
-  constexpr int WM = TM / 16;          // waves along the rows
-  constexpr int WN = 4 / WM;           // waves along the columns
-  constexpr int NT = 4 / WN;           // 16-column tiles a wave
-  const int h = blockIdx.z;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave % WM, wn = wave / WM;
+head_linear_rows16_kernel(HeadLinearArgs a) {
+  __shared__ __attribute__((aligned(16))) float part[SPLIT ? 4 : 1][16][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int h = blockIdx.z, n0 = SPLIT ? blockIdx.y * 16 : blockIdx.y * 64 + wave * 16;
   const int r16 = lane & 15, kq = lane >> 4;
-  const int n0 = blockIdx.y * 64 + wn * NT * 16;
   const int K = a.K, N = a.N;
-  const int row = blockIdx.x * TM + wm * 16 + r16;
-  const bool row_ok = row < a.T;
-  const bf16_t* arow = (const bf16_t*)a.x + ((size_t)(row_ok ? row : 0) * a.H + h) * a.x_ld + a.x_col;
-  const bf16_t* wbase = (const bf16_t*)a.W + (size_t)h * N * K;
-  const bf16_t* wrow[NT];
-  bool col_ok[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int n = n0 + j * 16 + r16;
-    col_ok[j] = n < N;
-    wrow[j] = wbase + (size_t)(col_ok[j] ? n : 0) * K;
-  }
-  f32x4_t acc[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int range = SPLIT ? (K + 127) / 128 * 32 : K, k_lo = SPLIT ? wave * range : 0;
+  const int k_end = min(K, k_lo + range);
+  const bf16_t* arow = (const bf16_t*)a.x + ((size_t)min(r16, a.T - 1) * a.H + h) * a.x_ld + a.x_col;
+  const bf16_t* wrow = (const bf16_t*)a.W + ((size_t)h * N + min(n0 + r16, N - 1)) * K;
+  // SPLIT: the element that this thread stores; its gate on its way with the operands
+  const int st = tid >> 4, sn = n0 + (tid & 15);
+  const bool mine = SPLIT && st < a.T && sn < N;
+  const float gate = mine ? head_gate_of<bf16_t>(a, st, h, sn) : 0.f;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   const bf16x8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  constexpr int U = 2;
-  for (int k0 = 0; k0 < K; k0 += 32 * U) {
-    bf16x8_t fa[U], fw[U][NT];
+  constexpr int U = 4;
+  for (int k0 = k_lo; k0 < k_end; k0 += 32 * U) {
+    bf16x8_t fa[U], fw[U];
 #pragma unroll
-    for (int s = 0; s < U; ++s) {
-      const int k = k0 + s * 32 + kq * 8;
-      const bool k_ok = k < K;           // K is a multiple of 8: a piece is inside or outside
-      fa[s] = (row_ok && k_ok) ? *reinterpret_cast<const bf16x8_t*>(arow + k) : zero;
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-        fw[s][j] = (col_ok[j] && k_ok) ? *reinterpret_cast<const bf16x8_t*>(wrow[j] + k) : zero;
+    for (int s = 0; s < U; ++s) {          // K is a multiple of 8: a piece is inside or outside
+      const int k = min(k0 + s * 32 + kq * 8, K - 8);
+      fa[s] = *reinterpret_cast<const bf16x8_t*>(arow + k);
+      fw[s] = *reinterpret_cast<const bf16x8_t*>(wrow + k);
     }
 #pragma unroll
-    for (int s = 0; s < U; ++s)
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[s], fw[s][j], acc[j], 0, 0, 0);
+    for (int s = 0; s < U; ++s) {
+      if (k0 + s * 32 + kq * 8 >= k_end) fa[s] = fw[s] = zero;
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[s], fw[s], acc, 0, 0, 0);
+    }
   }
+  TO* out = (TO*)a.out + a.o_col;
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part[wave][kq * 4 + i][r16] = acc[i];
+    __syncthreads();
+    if (!mine) return;
+    const int c = tid & 15;
+    const float v = (part[0][st][c] + part[1][st][c]) + (part[2][st][c] + part[3][st][c]);
+    out[((size_t)st * a.H + h) * a.o_ld + sn] = from_f32<TO>(v * gate);
+  } else {
+    const int n = n0 + r16;
+    if (n >= N) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = kq * 4 + i;
+      if (t < a.T)
+        out[((size_t)t * a.H + h) * a.o_ld + n] = from_f32<TO>(acc[i] * head_gate_of<bf16_t>(a, t, h, n));
+    }
+  }
+}
+
+// The same for more rows than a decode batch has, in tiles of BM tokens x 128 columns of one head
+// through LDS (tiles_bf16.h); a lane has four consecutive columns of a token's row.  With many
+// tokens the result's way to memory bounds it ([1777, 16 heads, 512], rows of 576, from 128: 17 us
+// against 37 of fragments straight from memory; [1777, 16, 128] with gates from 512: 15 against
+// 44), with few the steps of K, one after the other (64 tokens: 4.0 against 5.3, 9.0 against 14.7).
+// Tiles of 128 tokens: 21 and 27 us.
+#define HL_BN 128
+template <int BM, int NS, typename TO>
+__global__ void __launch_bounds__(256, 2)
+head_linear_tiled_kernel(HeadLinearArgs a) {
+  using Tiles = TilesBf16<BM, HL_BN, NS>;
+  __shared__ __attribute__((aligned(16))) bf16_t As[NS][BM * GG_BK];
+  __shared__ __attribute__((aligned(16))) bf16_t Ws[NS][HL_BN * GG_BK];
+  const int h = blockIdx.z, t0 = blockIdx.x * BM, n0 = blockIdx.y * HL_BN;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int K = a.K, N = a.N;
+  const int lrow = wave * 8 + (lane >> 3), piece = (lane & 7) ^ (lane >> 3);
+  const bf16_t* arow[Tiles::LA];
+  const bf16_t* wrow[Tiles::LW];
+#pragma unroll
+  for (int i = 0; i < Tiles::LA; ++i)
+    arow[i] = (const bf16_t*)a.x + ((size_t)min(t0 + lrow + 32 * i, a.T - 1) * a.H + h) * a.x_ld + a.x_col + piece * 8;
+#pragma unroll
+  for (int i = 0; i < Tiles::LW; ++i)
+    wrow[i] = (const bf16_t*)a.W + ((size_t)h * N + min(n0 + lrow + 32 * i, N - 1)) * K + piece * 8;
+  const int wm = (wave % Tiles::WM) * (BM / Tiles::WM), wn = (wave / Tiles::WM) * (HL_BN / Tiles::WN);
+  const int r16 = lane & 15, kq = lane >> 4;
+  // a gate an element, four at a time and all at once, before the products
+  const bool gates = a.gate_mode == 2 && ((a.gate_ld | a.gate_col | N) & 3) == 0 &&
+                     (reinterpret_cast<uintptr_t>(a.gate) & 7) == 0;
+  bf16x4_t gate[Tiles::TM][Tiles::TN];
+  if (gates)
+#pragma unroll
+    for (int i = 0; i < Tiles::TM; ++i)
+#pragma unroll
+      for (int j = 0; j < Tiles::TN; ++j)
+        gate[i][j] = *reinterpret_cast<const bf16x4_t*>(
+            (const bf16_t*)a.gate + (size_t)min(t0 + wm + i * 16 + r16, a.T - 1) * a.gate_ld + a.gate_col +
+            (size_t)h * N + min(n0 + wn + j * 16 + kq * 4, N - 4));
+  f32x4_t acc[Tiles::TM][Tiles::TN];
+  Tiles::run(As, Ws, wave, lane, K, arow, wrow, acc);
   TO* out = (TO*)a.out;
+  const bool wide = ((a.o_ld | a.o_col | N) & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & (4 * sizeof(TO) - 1)) == 0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = blockIdx.x * TM + wm * 16 + kq * 4 + i;
-    if (r >= a.T) continue;
-    TO* orow = out + ((size_t)r * a.H + h) * a.o_ld + a.o_col;
+  for (int i = 0; i < Tiles::TM; ++i) {
+    const int t = t0 + wm + i * 16 + r16;
+    if (t >= a.T) continue;
+    TO* to = out + ((size_t)t * a.H + h) * a.o_ld + a.o_col;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int n = n0 + j * 16 + r16;
-      if (n < N) orow[n] = from_f32<TO>(acc[j][i] * head_gate_of<bf16_t>(a, r, h, n));
+    for (int j = 0; j < Tiles::TN; ++j) {
+      const int n = n0 + wn + j * 16 + kq * 4;
+      if (n >= N) continue;
+      f32x4_t v = acc[i][j];
+      if (a.gate_mode == 2 && gates) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] *= 1.0f / (1.0f + expf(-(float)gate[i][j][r]));
+      } else if (a.gate_mode) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] *= head_gate_of<bf16_t>(a, t, h, min(n + r, N - 1));
+      }
+      if (wide) {
+        if constexpr (sizeof(TO) == 4)
+          *reinterpret_cast<f32x4_t*>(to + n) = v;
+        else
+          *reinterpret_cast<bf16x4_t*>(to + n) = bf16x4_t{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n + r < N) to[n + r] = from_f32<TO>(v[r]);
+      }
     }
   }
 }
@@ -332,21 +404,27 @@ extern "C" int za_head_linear(const void* x, int x_dtype, int x_ld, int x_col, c
     return ZA_ERR_ARG;
   HeadLinearArgs a{x, W, out, gate, n_tokens, heads, N, K, x_ld, x_col, o_ld, o_col,
                    gate_ld, gate_col, gate_mode};
-  const unsigned ntiles = (unsigned)((N + 63) / 64);
   if (w_dtype == 1) {
     if (x_dtype != 1 || K % 8 != 0 || x_ld % 8 != 0 || x_col % 8 != 0) return ZA_ERR_UNSUPPORTED;
-    const bool small = n_tokens <= 16;
-    dim3 grid((unsigned)((n_tokens + (small ? 15 : 63)) / (small ? 16 : 64)), ntiles, heads);
-#define ZA_HL(TMM, TO) \
-  hipLaunchKernelGGL((head_linear_bf16_kernel<TMM, TO>), grid, dim3(256), 0, stream, a)
-    if (out_dtype == 0) { if (small) ZA_HL(16, float); else ZA_HL(64, float); }
-    else if (out_dtype == 1) { if (small) ZA_HL(16, bf16_t); else ZA_HL(64, bf16_t); }
-    else return ZA_ERR_UNSUPPORTED;
+    if (out_dtype != 0 && out_dtype != 1) return ZA_ERR_UNSUPPORTED;
+    if (n_tokens <= 16) {
+      const bool split = K >= HL_SPLIT_MIN_K;
+      dim3 grid(1, (unsigned)(split ? (N + 15) / 16 : (N + 63) / 64), heads);
+#define ZA_HL(TO, SPLIT) hipLaunchKernelGGL((head_linear_rows16_kernel<TO, SPLIT>), grid, dim3(256), 0, stream, a)
+      if (out_dtype == 0) { if (split) ZA_HL(float, true); else ZA_HL(float, false); }
+      else { if (split) ZA_HL(bf16_t, true); else ZA_HL(bf16_t, false); }
 #undef ZA_HL
+      return za_launch_status();
+    }
+    dim3 grid((unsigned)((n_tokens + 63) / 64), (unsigned)((N + HL_BN - 1) / HL_BN), heads);
+    if (out_dtype == 0)
+      hipLaunchKernelGGL((head_linear_tiled_kernel<64, 2, float>), grid, dim3(256), 0, stream, a);
+    else
+      hipLaunchKernelGGL((head_linear_tiled_kernel<64, 2, bf16_t>), grid, dim3(256), 0, stream, a);
     return za_launch_status();
   }
   if (w_dtype != 0) return ZA_ERR_UNSUPPORTED;
-  dim3 grid((unsigned)((n_tokens + 63) / 64), ntiles, heads);
+  dim3 grid((unsigned)((n_tokens + 63) / 64), (unsigned)((N + 63) / 64), heads);
 #define ZA_HF(TA, TO) \
   hipLaunchKernelGGL((head_linear_f32_kernel<TA, TO>), grid, dim3(256), 0, stream, a)
   if (x_dtype == 0 && out_dtype == 0) ZA_HF(float, float);

@@ -111,3 +111,19 @@ def test_the_batch_sizes_that_recordings_are_kept_for():
     assert sizes[:17] == [1, 2, 4, 4, 8, 8, 8, 8, 16, 16, 16, 16, 16, 16, 16, 16, 24]
     assert all(0 <= s - n <= 7 for n, s in zip(range(1, 70), sizes))
     assert all(s % 8 == 0 for s in sizes[16:]) and sizes[63] == 64 and sizes[64] == 72
+
+
+def test_where_the_tiles_for_17_to_64_rows_are_taken():
+    """Products whose K comes in ranges, products with enough outputs to occupy the chip, and
+    gated ones with half as many."""
+    from zig_ai_amd.kernels import ops
+    for M in (17, 64):
+        assert ops.tiles_take(M, 2048, 8192, 8) and ops.tiles_take(M, 512, 4096, 8)
+        assert not ops.tiles_take(M, 200, 4096, 8)          # 32 workgroups
+        assert ops.tiles_take(M, 65536, 2048, 1) and not ops.tiles_take(M, 6144, 2048, 1)
+        assert not ops.tiles_take(M, 2048, 1000, 4)         # ranges that are no steps of 64
+        assert ops.tiles_take_gated(M, 8192, 2048) and ops.tiles_take_gated(M, 4608, 1024)
+        assert not ops.tiles_take_gated(M, 2048, 2048) and not ops.tiles_take_gated(M, 8192, 2044)
+    for M in (16, 65):
+        assert not ops.tiles_take(M, 2048, 8192, 8) and not ops.tiles_take(M, 65536, 2048, 1)
+        assert not ops.tiles_take_gated(M, 8192, 2048)

@@ -533,6 +533,33 @@ def test_rows64_products(M, N, K):
         assert rel_err(on_device, base.double() + 2 * exact) < F32_TOL
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+@pytest.mark.parametrize("N,K,ranges", [(2048, 2048, 4), (70, 4096, 8), (1022, 1152, 2), (64, 192, 3), (24, 72, 1),
+                                        (130, 2056, 1)])
+def test_products_of_17_to_64_rows_in_tiles(M, N, K, ranges):
+    """Rows, outputs and K at the edges of the tiles: ranges, plain results of either type, the
+    gated form with either unit."""
+    o = ops()
+    x, w = rand((M, K), torch.bfloat16, 60), rand((N, K), torch.bfloat16, 61)
+    expect = x.double() @ w.double().T
+    stack = torch.full((ranges + 1, M, N), 5.0, dtype=torch.float32, device=dev())
+    assert o._tiles_product(x.to(dev()), w.to(dev()), stack[:ranges], ranges)
+    assert rel_err(stack[:ranges].sum(0), expect) < F32_TOL and bool((stack[ranges] == 5).all())
+    part = x[:, :K // ranges].double() @ w[:, :K // ranges].double().T
+    assert rel_err(stack[0], part) < F32_TOL
+    for dtype, tol in ((torch.float32, F32_TOL), (torch.bfloat16, BF16_TOL)):
+        out = torch.empty((M, N), dtype=dtype, device=dev())
+        assert o._tiles_product(x.to(dev()), w.to(dev()), out)
+        assert rel_err(out, expect) < tol
+    g, u = expect[:, :N // 2], expect[:, N // 2:]
+    units = (g * torch.sigmoid(g) * u,
+             0.5 * g * (1 + torch.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3))) * u)
+    for act, want in enumerate(units):
+        out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=dev())
+        assert o._tiles_product(x.to(dev()), w.to(dev()), out, gated=True, activation=act)
+        assert rel_err(out, want) < BF16_TOL
+
+
 def test_rows64_rows_do_not_depend_on_the_batch():
     """A row's result is a function of that row: the same bits whichever rows stand beside
     it and wherever it stands (the sums over K run in one order for every row)."""

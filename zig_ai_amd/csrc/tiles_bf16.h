@@ -37,7 +37,7 @@ template <int BM, int BN, int NS>
 struct TilesBf16 {
   static constexpr int WM = BM >= 64 || BN == 64 ? 2 : 1, WN = 4 / WM;   // waves along the rows of A and of W
   static constexpr int TM = BM / (16 * WM), TN = BN / (16 * WN);
-  static_assert((TM == 4 && TN == 4) || (TM == 2 && TN == 4) || (TM == 1 && TN == 2), "see take");
+  static_assert((TM == 4 && TN == 4) || (TM == 2 && TN == 4) || (TM == 2 && TN == 2) || (TM == 1 && TN == 2), "see take");
   static constexpr int LA = BM / 32, LW = BN / 32;      // instructions a wave and tile (8 rows each)
 
   // `arow`, `wrow`: a lane's rows of the tile, 32 i + 8 wave + lane / 8, each at its piece
@@ -97,6 +97,18 @@ struct TilesBf16 {
             : "=&v"(fw[0][0]), "=&v"(fw[0][1]), "=&v"(fw[0][2]), "=&v"(fw[0][3]),
               "=&v"(fa[0][0]), "=&v"(fa[0][1]), "=&v"(fw[1][0]), "=&v"(fw[1][1]),
               "=&v"(fw[1][2]), "=&v"(fw[1][3]), "=&v"(fa[1][0]), "=&v"(fa[1][1])
+            : "v"(w0), "v"(w1), "v"(a0), "v"(a1)
+            : "memory");
+      }
+      if constexpr (TM == 2 && TN == 2) {
+        asm volatile(
+            "ds_read_b128 %0, %8 offset:0\n" "ds_read_b128 %1, %8 offset:2048\n"
+            "ds_read_b128 %2, %10 offset:0\n" "ds_read_b128 %3, %10 offset:2048\n"
+            "ds_read_b128 %4, %9 offset:0\n" "ds_read_b128 %5, %9 offset:2048\n"
+            "ds_read_b128 %6, %11 offset:0\n" "ds_read_b128 %7, %11 offset:2048\n"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(fw[0][0]), "=&v"(fw[0][1]), "=&v"(fa[0][0]), "=&v"(fa[0][1]),
+              "=&v"(fw[1][0]), "=&v"(fw[1][1]), "=&v"(fa[1][0]), "=&v"(fa[1][1])
             : "v"(w0), "v"(w1), "v"(a0), "v"(a1)
             : "memory");
       }

@@ -163,7 +163,7 @@ class DecoderModel:
         if self.kernel_sources:
             wanted = list(self.kernel_sources) + ["host"]
             if "gemm" in self.kernel_sources and runtime.dtype == torch.bfloat16:
-                wanted.append("blaslt")     # products of many rows go to the GEMM library
+                wanted += ["blaslt", "gemm_tiles"]     # the products of more than 16 rows
             kernel_build.build_all(wanted, jobs=len(wanted))
 
     # ------------------------------------------------------------- construction

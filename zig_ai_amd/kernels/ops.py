@@ -81,6 +81,8 @@ _SIGNATURES = {
     ("gemm_rows64", "za_gemm_bf16_rows64"): [c_void_p, c_void_p, c_void_p, c_void_p, c_float,
                                              c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                              c_void_p],
+    ("gemm_tiles", "za_gemm_bf16_tiles"): [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                           c_int, c_int, c_int, c_void_p],
     ("sampling", "za_sample"): [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
                                 c_void_p, c_int, c_void_p],
     ("sampling", "za_repetition_penalty"): [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
@@ -776,6 +778,73 @@ def accumulate_plan(M: int, N: int, K: int, normed: bool) -> int:
     return _accumulate_splits(N, K)
 
 
+# Where a step of 17 to 64 rows takes the kernel of csrc/gemm_tiles.hip, by measurement (one MI355X,
+# replayed from graphs, weights from memory, against the library's product): where K comes in
+# ranges (2048 x 8192 at 64 rows 9.8 us against 13.8, 512 x 2048 3.9 against 4.6; products with
+# still fewer outputs, of which no step is made, stay with the library), and without ranges from as
+# many workgroups on as the chip has compute units (65536 x 2048 in 32-bit at 64 rows 64 us against
+# 71); with fewer the library stays (6144 x 2048, 96 workgroups, 11.5 us at 32 rows against 10.2).
+# With the unit of a gated feed-forward from half as many on, since the unit's own kernel goes with
+# it (2 x 8192 x 2048 at 20 and 64 rows 17.2 and 18.9 us against 20.2 and 21.1, 2 x 4608 x 1024,
+# 144 workgroups, 7.7 and 8.4 against 12.4 and 15.5, 2 x 4096 x 2048 12.1 and 14.9 against 17.2 and
+# 14.9; 2 x 2048 x 2048, 64 workgroups, 10.0 and 12.7 against 11.4 and 12.6).
+TILES_MAX_ROWS = 64
+TILES_COLUMNS = 64
+TILES_MIN_WORKGROUPS = 256
+TILES_MIN_RANGED_WORKGROUPS = 64
+TILES_MIN_GATED_WORKGROUPS = 128
+
+
+def tiles_take(M: int, N: int, K: int, ranges: int) -> bool:
+    """Whether a product of 17 to 64 rows (``ranges`` > 1: as that many partial sums) takes the
+    kernel of csrc/gemm_tiles.hip."""
+    return (LIBRARY_GEMM_ROWS < M <= TILES_MAX_ROWS
+            and (ranges > 1 and K % (ranges * 64) == 0
+                 and -(-N // TILES_COLUMNS) * ranges >= TILES_MIN_RANGED_WORKGROUPS
+                 or ranges == 1 and -(-N // TILES_COLUMNS) >= TILES_MIN_WORKGROUPS))
+
+
+def tiles_take_gated(M: int, I: int, K: int) -> bool:
+    """The same for ``linear_gated_tiles`` with ``I`` outputs."""
+    return (LIBRARY_GEMM_ROWS < M <= TILES_MAX_ROWS and K % 8 == 0
+            and -(-I // (TILES_COLUMNS // 2)) >= TILES_MIN_GATED_WORKGROUPS)
+
+
+def _tiles_product(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, ranges: int = 1,
+                   gated: bool = False, activation: int = 0) -> bool:
+    """``False``: operands that do not start on 16 bytes, which the kernel does not take."""
+    if (x.data_ptr() | weight.data_ptr() | out.data_ptr()) % 16:
+        return False
+    M, K = x.shape
+    N = weight.shape[0] // 2 if gated else weight.shape[0]
+    rc = _fn("gemm_tiles", "za_gemm_bf16_tiles")(
+        _ptr(x), _ptr(weight), _ptr(out), _code(out.dtype), M, N, K, ranges, 1 if gated else 0,
+        activation, _stream())
+    _check(rc, "gemm_bf16_tiles", f"M={M} N={N} K={K} ranges={ranges} gated={gated}")
+    return True
+
+
+def linear_gated_tiles(x: torch.Tensor, gate_up_weight: torch.Tensor,
+                       activation: str = "silu") -> Optional[torch.Tensor]:
+    """``act(x Wg^T) * (x Wu^T)`` of a step of 17 to 64 rows of bfloat16 ``x`` (for which
+    ``tiles_take_gated`` says so) in one kernel, the unit on the product's 32-bit sums;
+    ``None``: operands that do not start on 16 bytes."""
+    M, K = x.shape
+    _need(x, "x", torch.bfloat16)
+    _need(gate_up_weight, "gate_up_weight", torch.bfloat16, (gate_up_weight.shape[0], K))
+    if gate_up_weight.shape[0] % 2:
+        raise KernelError("a fused gate|up weight has an even number of rows")
+    I = gate_up_weight.shape[0] // 2
+    if not tiles_take_gated(M, I, K):
+        raise KernelError(f"linear_gated_tiles takes 17 to {TILES_MAX_ROWS} rows and enough outputs, "
+                          f"got M={M} I={I} K={K}")
+    out = torch.empty((M, I), dtype=torch.bfloat16, device=x.device)
+    if not _tiles_product(x, gate_up_weight, out, gated=True, activation=GATE_ACTIVATIONS[activation]):
+        return None
+    _note("linear_swiglu", M=M, N=2 * I, K=K, norm_in_product=False, kernel="tiles")
+    return out
+
+
 def linear(x, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out_dtype: Optional[torch.dtype] = None, force_tiled: bool = False,
            partial_ok: bool = False,
@@ -942,6 +1011,14 @@ def linear(x, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
         _note("linear", M=M, N=N, K=K, norm_in_product=False, added_to_stream=False,
               partial_sums=splits, out=stack.dtype)
         return stack
+    if library and bias is None and tiles_take(M, N, K, splits):
+        out = into if into is not None else \
+            torch.empty((splits, M, N) if splits > 1 else (M, N),
+                        dtype=torch.float32 if splits > 1 else out_dtype, device=x.device)
+        if _tiles_product(x, weight, out, splits):
+            _note("linear", M=M, N=N, K=K, norm_in_product=False, added_to_stream=False,
+                  partial_sums=splits, out=out.dtype, kernel="tiles")
+            return out
     if library:
         # (with ranges of K: one batched product, [P, M, K/P] x [P, K/P, N])
         out = _library_matmul(x, weight, out_dtype, splits, tune,

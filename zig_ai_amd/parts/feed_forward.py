@@ -70,6 +70,14 @@ class SwiGLU(FeedForward):
         ops.check_projection_weight(self.gate_up, "feed_forward gate_up")
         ops.check_projection_weight(self.down, "feed_forward down")
 
+    def gated_by_tiles(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """The gated product of a step of 17 to 64 normalised rows in one kernel; ``None``: not
+        taken."""
+        if x.dtype == torch.bfloat16 and self.gate_up.dtype == torch.bfloat16 \
+                and ops.tiles_take_gated(x.shape[0], self.gate_up.shape[0] // 2, x.shape[1]):
+            return ops.linear_gated_tiles(x, self.gate_up, self.activation)
+        return None
+
     def forward(self, x, step=None, stream: Optional[torch.Tensor] = None):
         if self.activation != "silu":
             if isinstance(x, ops.NormedRows):
@@ -79,8 +87,10 @@ class SwiGLU(FeedForward):
                 # a decode batch: the gate is applied to the projection's accumulators
                 a = ops.linear_swiglu(x, self.gate_up, self.activation)
             else:
-                a = ops.gated_unit(ops.linear(x, self.gate_up, tune=self.runtime.tune),
-                                   self.activation)
+                a = self.gated_by_tiles(x)
+                if a is None:
+                    a = ops.gated_unit(ops.linear(x, self.gate_up, tune=self.runtime.tune),
+                                       self.activation)
             return ops.linear(a, self.down, partial_ok=True, accumulate=stream,
                               tune=self.runtime.tune)
         bf16 = x.dtype == torch.bfloat16 and self.gate_up.dtype == torch.bfloat16
@@ -93,7 +103,9 @@ class SwiGLU(FeedForward):
         else:
             if isinstance(x, ops.NormedRows):
                 x = x.materialise()
-            a = ops.swiglu(ops.linear(x, self.gate_up, tune=self.runtime.tune))
+            a = self.gated_by_tiles(x)
+            if a is None:
+                a = ops.swiglu(ops.linear(x, self.gate_up, tune=self.runtime.tune))
         return ops.linear(a, self.down, partial_ok=True, accumulate=stream, tune=self.runtime.tune)
 
 

@@ -660,3 +660,31 @@ def test_small_kernels():
     assert ops.scaled_add_rmsnorm(res, a.to(torch.bfloat16).to(dev), 2.0) is None
     s = s + 2.0 * a.to(torch.bfloat16).double()
     assert float((res.cpu().double() - s).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("width", [4, 252, 1020, 1024, 1028, 2052, 3076, 4096, 4100, 33])
+def test_rows_in_registers_at_the_edges_of_a_workgroup(width):
+    """The three norms that keep a row in registers, at rows that do and do not fill a
+    workgroup's vectors, and rows beyond them; a stack of partial sums with every count."""
+    from zig_ai_amd.kernels import ops
+    dev, T = torch.device("cuda"), 3
+    g = torch.Generator().manual_seed(width)
+    x, a, b = (torch.randn(T, width, generator=g) for _ in range(3))
+    w = torch.randn(width, generator=g)
+    res = x.to(dev).clone()
+    out = ops.scaled_add_rmsnorm(res, a.to(dev), 0.3, b.to(dev), -1.1, w.to(dev), 1e-6)
+    s = x.double() + 0.3 * a.double() - 1.1 * b.double()
+    assert float((res.cpu().double() - s).abs().max()) < 1e-5
+    assert float((out.cpu().double() - plain.rms(s, 1e-6) * w.double()).abs().max()) < 2e-5
+    # (up to nine 32-bit additions before the norm, which for four elements may divide by little)
+    for n in (1, 2, 8, 9):
+        y = torch.randn(n, T, width, generator=g)
+        res = x.to(dev).clone()
+        out = ops.add_rmsnorm(res, y.to(dev), w.to(dev), 1e-6, torch.float32)
+        s = x.double() + y.double().sum(0)
+        assert float((res.cpu().double() - s).abs().max()) < 2e-5
+        assert float((out.cpu().double() - plain.rms(s, 1e-6) * w.double()).abs().max()) < 4e-5
+        res = x.to(dev).clone()
+        ops.normed_add_(res, y.to(dev), w.to(dev), 1e-6, 0.5)
+        s = x.double() + 0.5 * plain.rms(y.double().sum(0), 1e-6) * w.double()
+        assert float((res.cpu().double() - s).abs().max()) < 4e-5

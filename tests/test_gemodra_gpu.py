@@ -749,3 +749,76 @@ def test_token_side_kernels():
     z = torch.randn(T, width, generator=g) * 20
     got = ops.softcap_(z.to(dev).clone(), 7.0).cpu().double()
     assert float((got - 7.0 * torch.tanh(z.double() / 7.0)).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("mode,renorm", [("softmax", False), ("sigmoid", True)])
+@pytest.mark.parametrize("n,groups,keep,top", [(1, 0, 0, 1), (30, 0, 0, 4), (32, 4, 2, 4), (64, 16, 3, 7),
+                                               (64, 0, 0, 64), (65, 0, 0, 8), (66, 6, 2, 5)])
+def test_router_ties_and_values_that_compare_false(n, groups, keep, top, mode, renorm):
+    """One output a lane or more of them: of equal scores the lower index first, an output whose
+    score is NaN last of all (and output 0 where nothing is left)."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(n + top)
+    T = 24
+    logits = torch.randint(-2, 3, (T, n), generator=g).float()          # ties
+    correction = torch.zeros(n)
+    if n > top + 2 and not groups:
+        correction[1] = float("nan")
+    chosen, weight = ops.route_topk(logits.to(dev), n, top, correction.to(dev), groups, keep, 1.5, mode, renorm)
+    s = torch.softmax(logits.double(), 1) if mode == "softmax" else torch.sigmoid(logits.double())
+    for t in range(T):
+        # (whole numbers stand for the scores, which rise with them: the kernel's ties are exact)
+        c = [float(v) if not math.isnan(float(k)) else None for v, k in zip(logits[t], correction)]
+        usable = [e for e in range(n) if c[e] is not None]
+        if groups and keep < groups:
+            per = n // groups
+            best = sorted(range(groups), key=lambda q: (-max(c[q * per:(q + 1) * per]), q))[:keep]
+            usable = [e for e in usable if e // per in best]
+        want = sorted(usable, key=lambda e: (-c[e], e))[:top]
+        assert chosen[t].tolist() == want
+        w = s[t][want]
+        w = w / w.sum() * 1.5 if renorm else w * 1.5
+        assert float((weight[t].cpu().double() - w).abs().max()) < 1e-6
+    nothing = torch.full((n,), float("nan"))
+    chosen, _ = ops.route_topk(logits.to(dev), n, top, nothing.to(dev), 0, 0, 1.0, mode, renorm)
+    assert not bool(chosen.any())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("Rq,R,Dr,rot,adjacent", [(1536, 512, 64, 64, True), (2048, 512, 32, 16, False), (40, 24, 8, 8, True),
+                                                  (300, 257, 0, 0, False), (2056, 64, 16, 16, True), (64, 520, 8, 0, False)])
+def test_latent_prepare_kernels(dtype, Rq, R, Dr, rot, adjacent):
+    """Latents that a workgroup holds in registers and longer ones."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(Rq + R)
+    T, page, c_col = 5, 4, Rq + 8
+    down = torch.randn(T, c_col + R + Dr, generator=g).to(dtype)
+    qw, cw = torch.randn(Rq, generator=g), torch.randn(R, generator=g)
+    positions, slots = [0, 3, 7, 100, 2000], [2, 9, -1, 0, 7]
+    freq = 1e4 ** (-torch.arange(max(1, rot // 2)).float() / max(1, rot // 2))
+    plane = torch.full((3, 1, page, R + Dr), 9.0, dtype=dtype, device=dev)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    cq = ops.latent_prepare(down.to(dev), 0, Rq, c_col, R, Dr, qw.to(dev), cw.to(dev), 1e-6, i32(positions),
+                            i32(slots), freq.to(dev) if rot else None, rot, adjacent, plane, 1.25)
+    x = down.double()
+    tol = 2e-5 if dtype == torch.float32 else 2e-2      # (32-bit angles up to 2,000; one rounding of values up to 5)
+    norm = lambda v, w: v / torch.sqrt((v * v).mean(1, keepdim=True) + 1e-6) * w.double()
+    want = norm(x[:, :Rq], qw)
+    assert float(((cq.cpu().double() - want) / (1 + want.abs())).abs().max()) < tol
+    c, kr = norm(x[:, c_col:c_col + R], cw), x[:, c_col + R:].clone()
+    if rot:
+        half = rot // 2
+        angle = (torch.tensor(positions).float()[:, None] * freq[None]).double()
+        a = torch.arange(half) * 2 if adjacent else torch.arange(half)
+        b = a + 1 if adjacent else a + half
+        u, v = kr[:, a].clone(), kr[:, b].clone()
+        kr[:, a] = (u * torch.cos(angle) - v * torch.sin(angle)) * 1.25
+        kr[:, b] = (v * torch.cos(angle) + u * torch.sin(angle)) * 1.25
+    got, rows = plane.cpu().double().view(-1, R + Dr), torch.cat([c, kr], 1)
+    for t, s in enumerate(slots):
+        if s >= 0:
+            assert float(((got[s] - rows[t]) / (1 + rows[t].abs())).abs().max()) < tol
+    untouched = [s for s in range(12) if s not in slots]
+    assert bool((got[untouched] == 9).all())

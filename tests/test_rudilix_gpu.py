@@ -688,3 +688,25 @@ def test_rows_in_registers_at_the_edges_of_a_workgroup(width):
         ops.normed_add_(res, y.to(dev), w.to(dev), 1e-6, 0.5)
         s = x.double() + 0.5 * plain.rms(y.double().sum(0), 1e-6) * w.double()
         assert float((res.cpu().double() - s).abs().max()) < 4e-5
+
+
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5])
+def test_causal_conv_at_the_edges_of_its_blocks(taps):
+    """Portions that end before, on and behind a block of 16 tokens, shorter than the taps and of
+    one token; 300 channels behind eight others."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(taps)
+    lengths, slots, C, col0 = [15, 1, 17, 2, 32, 3, 16], [6, 0, 3, 1, 7, 2, 5], 300, 8
+    x = torch.randn(sum(lengths), C + col0 + 4, generator=g).to(torch.bfloat16)
+    w, b = torch.randn(C, taps, generator=g), torch.randn(C, generator=g)
+    _, state = _slots(8, C * (taps - 1) + 4, dev)
+    # (twice: the second time behind the first)
+    got = [ops.causal_conv_silu(x.to(dev), col0, w.to(dev), b.to(dev), state, 4,
+                                *_step_arrays(lengths, slots, dev)).cpu().double() for _ in range(2)]
+    at = 0
+    for n in lengths:
+        rows = x[at:at + n, col0:col0 + C].double()
+        want = plain.silu(plain.causal_conv(torch.cat([rows, rows]), w.double(), b.double()))
+        assert float((torch.cat([y[at:at + n] for y in got]) - want).abs().max()) < 1e-5
+        at += n

@@ -162,8 +162,10 @@ class DecoderModel:
         # the first step.
         if self.kernel_sources:
             wanted = list(self.kernel_sources) + ["host"]
-            if "gemm" in self.kernel_sources and runtime.dtype == torch.bfloat16:
-                wanted += ["blaslt", "gemm_tiles"]     # the products of more than 16 rows
+            if "gemm" in self.kernel_sources:
+                wanted.append("gemm_f32")                    # matrices kept in 32-bit, also in a bfloat16 run
+                if runtime.dtype == torch.bfloat16:
+                    wanted += ["blaslt", "gemm_tiles"]       # the products of more than 16 rows
             kernel_build.build_all(wanted, jobs=len(wanted))
 
     # ------------------------------------------------------------- construction

@@ -26,7 +26,7 @@ _SIGNATURES = {
     ("norm", "za_add_rmsnorm"): [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p,
                                  c_int, c_int, c_float, c_int, c_int, c_longlong, c_void_p],
     ("norm", "za_embed_gather"): [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p],
-    ("gemm", "za_gemm_f32"): [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
+    ("gemm_f32", "za_gemm_f32"): [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                               c_int, c_void_p],
     ("gemm", "za_gemm_bf16"): [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                c_int, c_void_p],
@@ -973,7 +973,7 @@ def linear(x, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
         _need(into, "into", out_dtype, (M, N))
     if weight.dtype == torch.float32:
         out = into if into is not None else torch.empty((M, N), dtype=out_dtype, device=x.device)
-        rc = _fn("gemm", "za_gemm_f32")(_ptr(x), _code(x.dtype), _ptr(weight), _ptr(bias), _ptr(out),
+        rc = _fn("gemm_f32", "za_gemm_f32")(_ptr(x), _code(x.dtype), _ptr(weight), _ptr(bias), _ptr(out),
                                         _code(out_dtype), M, N, K, _stream())
         _check(rc, "gemm_f32", f"M={M} N={N} K={K}")
         _note("linear", M=M, N=N, K=K, norm_in_product=False, added_to_stream=False,

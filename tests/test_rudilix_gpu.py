@@ -621,6 +621,39 @@ def test_ssd_recurrence_in_chunks(H, G, N, P, strong):
     assert float(mem[:, H * N * P:].abs().max()) == 0.0 and float(state[1].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("strength", [1e3, 1e5, 1e7, 1e30])
+def test_ssd_chunks_behind_a_token_that_forgets(strength):
+    """A few tokens whose decay is zero (``exp(A_log) dt`` = ``strength``) among tokens that keep
+    three quarters: what the former leave decays at the latter's pace.  (Bound as above.)"""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator().manual_seed(7)
+    H, G, N, P, C = 2, 1, 32, 48, ops.RETENTION_CHUNK
+    lengths, slots = [C + 70, 33], [1, 0]
+    T = sum(lengths)
+    mem, state = _slots(2, H * N * P, dev)
+    conv = torch.randn(T, H * P + 2 * G * N, generator=gen)
+    proj = math.log(0.3 / (strength / 5)) + 0.1 * torch.randn(T, H, generator=gen)
+    for t in (0, 17, 60, 61, 100, C + 3, C + 90):
+        proj[t, 0], proj[min(t + 1, T - 1), 1] = 5.0, 5.0
+    A_log, bias = torch.full((H,), math.log(strength / 5)), torch.zeros(H)
+    _, start, slot_id = _step_arrays(lengths, slots, dev)
+    out = ops.ssd_recurrence_chunked(conv.to(dev), H * P + G * N, H * P, 0, proj.to(dev), 0, bias.to(dev),
+                                     A_log.to(dev), bias.to(dev), state, 0, slot_id,
+                                     _chunk_items(lengths, C, dev), H, G, N, P).cpu().double()
+    c, dt = conv.double(), plain.softplus(proj.double())
+    decay = torch.exp(-torch.exp(A_log.double()) * dt)
+    for i, slot in enumerate(slots):
+        S = torch.zeros(H, N, P, dtype=torch.float64)
+        for t in range(int(start[i]), int(start[i + 1])):
+            S = decay[t][:, None, None] * S + torch.outer(dt[t], c[t, H * P:H * P + N])[:, :, None] \
+                * c[t, :H * P].view(H, 1, P)
+            want = torch.einsum("hnp,n->hp", S, c[t, H * P + N:]).reshape(-1)
+            assert float((out[t] - want).abs().max()) < 2e-5 * max(1.0, float(want.abs().max())), t
+        kept = state[slot].double().cpu().view(H, P, N).transpose(1, 2)
+        assert float((kept - S).abs().max()) < 2e-5 * max(1.0, float(S.abs().max()))
+
+
 def test_small_kernels():
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")

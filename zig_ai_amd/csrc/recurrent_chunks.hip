@@ -42,7 +42,8 @@ __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + lo
 // State-space duality and fixed decays:  S <- a S + dt k v^T,  o = S^T q (+ D v), with a one
 // number a head, a function of the token or constant.  With c_i = log2 of the product of a chunk's
 // decays up to and including token i (in double, kept as two floats: a difference of two of them
-// is exact where it matters however far the sum has run), n its tokens, B the state before it:
+// is put together before the power is taken, so its error does not grow with the sum), n its
+// tokens, B the state before it:
 //   1. decay_chunk_state:   N = sum_j 2^(c_n - c_j) dt_j k_j v_j^T   of every chunk by itself
 //   2. decay_prefix:        B of every chunk in a request's order, B <- 2^c_n B + N
 //   3. decay_chunk_out:     o_i = 2^c_i B^T q_i + sum_(j <= i) 2^(c_i - c_j) dt_j (q_i . k_j) v_j
@@ -53,9 +54,15 @@ __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + lo
 // 624 us walked, 78 here (92 as chunks of 256 walked side by side and corrected).
 #define DC_CHUNK 128
 
-// 2^(hi + lo), |lo| below the last place of hi.
+// The least log2 of a decay that is told apart from zero.  Any power this small is zero in 32-bit
+// (2^-149 is the last that is not), and a chunk's sum of such numbers still has 37 binary places in
+// double, so the decays behind a token that forgets everything keep theirs.
+#define DC_LEAST_LOG2 -400.0
+
+// 2^(hi + lo), |lo| at most a few last places of the sum that hi came from.
 __device__ __forceinline__ float exp2_of(float hi, float lo) {
-  return exp2f(hi) * fmaf(lo, 0.6931471805599453f, 1.0f);
+  const float e = hi + lo, rest = (hi - e) + lo;      // (rest: below the last place of e)
+  return exp2f(e) * fmaf(rest, 0.6931471805599453f, 1.0f);
 }
 
 struct DecayArgs {
@@ -120,7 +127,7 @@ decay_chunk_state_kernel(DecayArgs a) {
         dt = softplus_f(raw + a.dt_bias[h]);
         l = (double)(-expf(a.A_log[h]) * dt) * 1.4426950408889634;
       }
-      l = l < -1e30 ? -1e30 : l;      // (a decay of zero: differences stay numbers)
+      l = l < DC_LEAST_LOG2 ? DC_LEAST_LOG2 : l;
     }
     c = l;
 #pragma unroll

@@ -654,6 +654,37 @@ def test_ssd_chunks_behind_a_token_that_forgets(strength):
         assert float((kept - S).abs().max()) < 2e-5 * max(1.0, float(S.abs().max()))
 
 
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+@pytest.mark.parametrize("at", [5, 20, 64, 127, 130])
+def test_ssd_chunks_keep_a_bad_value_from_earlier_tokens(bad, at):
+    """A token's value that is infinite or not a number stays in its column, from its token on."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator().manual_seed(at)
+    H, G, N, P, C = 2, 1, 40, 72, ops.RETENTION_CHUNK
+    lengths, slots = [7, C + 20, 9], [1, 0, 2]
+    T, first = sum(lengths), lengths[0]
+    conv = torch.randn(T, H * P + 2 * G * N, generator=gen).to(dev)
+    proj = torch.randn(T, H, generator=gen).to(dev)
+    A_log, bias = torch.full((H,), -2.0, device=dev), torch.zeros(H, device=dev)
+    _, _, slot_id = _step_arrays(lengths, slots, dev)
+
+    def run(x):
+        _, state = _slots(3, H * N * P, dev)
+        out = ops.ssd_recurrence_chunked(x, H * P + G * N, H * P, 0, proj, 0, bias, A_log, bias, state, 0, slot_id,
+                                         _chunk_items(lengths, C, dev), H, G, N, P)
+        return out.view(T, H, P)
+
+    want = run(conv)
+    spoilt = conv.clone()
+    spoilt[first + at, 70] = bad                     # head 0, column 70
+    got = run(spoilt)
+    after = torch.zeros(T, H, P, dtype=torch.bool, device=dev)
+    after[first + at:first + lengths[1], 0, 70] = True
+    assert bool((~torch.isfinite(got[after])).all())
+    assert float((got - want)[~after].abs().max()) < 2e-5 * float(want.abs().max())
+
+
 def test_small_kernels():
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")

@@ -36,6 +36,34 @@ __device__ __forceinline__ f32x4_t load4(const float* p, int n, bool aligned) {
   else return load4_below(p, n, aligned);
 }
 
+// Whether any lane holds a number that is infinite or none (zero times such a number is not zero).
+__device__ __forceinline__ bool any_wild(const f32x4_t& v) {
+  const float z = (v[0] * 0.f + v[1] * 0.f) + (v[2] * 0.f + v[3] * 0.f);
+  return __any(z != 0.f);
+}
+
+__device__ __forceinline__ f32x4_t without_wild(const f32x4_t& v) {
+  f32x4_t x;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = v[j] * 0.f == 0.f ? v[j] : 0.f;
+  return x;
+}
+
+// For a block of sixteen tokens that are their own keys (rows 4 g + j of v, as a second operand):
+// from a wild number's row on every sum of its column in c is no number.  (A later token's weight
+// of zero does not keep such a number out, so the product is taken without.)
+__device__ __forceinline__ void wild_from_its_row(const f32x4_t& v, f32x4_t& c, int g) {
+  int first = 16;
+#pragma unroll
+  for (int j = 3; j >= 0; --j)
+    if (v[j] * 0.f != 0.f) first = 4 * g + j;
+  first = min(first, __shfl_xor(first, 16, ZA_WAVE));
+  first = min(first, __shfl_xor(first, 32, ZA_WAVE));
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (4 * g + r >= first) c[r] = __builtin_nanf("");
+}
+
 __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
 
 // ------------------------------------------------------------- one decay a head and token
@@ -309,6 +337,7 @@ decay_chunk_out_kernel(DecayArgs a) {
       }
     }
   };
+  unsigned wild = 0;                 // of the blocks of own tokens and 16 columns: those with such numbers
   request(0);
   for (int J = 0; J <= last; ++J) {
     f32x4_t k0[NT], v0[4];
@@ -335,9 +364,31 @@ decay_chunk_out_kernel(DecayArgs a) {
         p[r] = key <= tile[i] * 16 + r16 ? s[r] * (exp2_of(d, lost + (q_lo[i] - lo[key])) * step[key]) : 0.f;
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = mfma4(p, v0[j], acc[i][j]);
+      for (int j = 0; j < 4; ++j) {
+        f32x4_t x = v0[j];
+        if (J == tile[i] && any_wild(x)) {
+          wild |= 1u << (i * 4 + j);
+          x = without_wild(x);
+        }
+        acc[i][j] = mfma4(p, x, acc[i][j]);
+      }
     }
   }
+  if (wild)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (wild & (1u << (i * 4 + j))) {
+          f32x4_t x;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int col = n0 + j * 16 + r16;
+            x[r] = FULL || col < dv
+                       ? rows[(size_t)min(tile[i] * 16 + 4 * g + r, n - 1) * a.width + a.x_col + h * dv + col] : 0.f;
+          }
+          wild_from_its_row(x, acc[i][j], g);
+        }
   const float D = a.D ? a.D[h] : 0.f;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {

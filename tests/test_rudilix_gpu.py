@@ -685,6 +685,42 @@ def test_ssd_chunks_keep_a_bad_value_from_earlier_tokens(bad, at):
     assert float((got - want)[~after].abs().max()) < 2e-5 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+@pytest.mark.parametrize("at", [5, 16, 20, 31, 40, 69])
+def test_delta_chunks_keep_a_bad_value_from_earlier_tokens(bad, at):
+    """The same for the delta rule, and for a key and a write strength (which spoil their head)."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator().manual_seed(at)
+    H, G, d, dv = 2, 2, 40, 24
+    lengths, slots = [7, 70, 9], [1, 0, 2]
+    T, first = sum(lengths), lengths[0]
+    conv = torch.randn(T, 2 * G * d + H * dv, generator=gen).to(dev)
+    proj = torch.randn(T, H, generator=gen).to(dev)
+    raw = torch.randn(T, H * d, generator=gen).to(dev)
+    A_log, bias = torch.full((H,), -2.0, device=dev), torch.zeros(H * d, device=dev)
+    _, _, slot_id = _step_arrays(lengths, slots, dev)
+
+    def run(x, strength):
+        _, state = _slots(3, H * d * dv, dev)
+        out = ops.delta_recurrence_chunked(x, 0, G * d, 2 * G * d, strength, 0, raw, bias, A_log, state, 0, slot_id,
+                                           _chunk_items(lengths, ops.DELTA_CHUNK, dev), H, G, d, dv)
+        return out.view(T, H, dv)
+
+    want = run(conv, proj)
+    value, key, strength = conv.clone(), conv.clone(), proj.clone()
+    value[first + at, 2 * G * d + 17] = bad          # head 0, column 17
+    key[first + at, G * d + 3] = bad
+    strength[first + at, 0] = math.nan
+    rows = slice(first + at, first + lengths[1])
+    for got, columns in ((run(value, proj), slice(17, 18)), (run(key, proj), slice(0, dv)),
+                         (run(conv, strength), slice(0, dv))):
+        after = torch.zeros(T, H, dv, dtype=torch.bool, device=dev)
+        after[rows, 0, columns] = True
+        assert bool((~torch.isfinite(got[after])).all())
+        assert float((got - want)[~after].abs().max()) < 2e-5 * float(want.abs().max())
+
+
 def test_small_kernels():
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")

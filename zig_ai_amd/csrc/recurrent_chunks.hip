@@ -864,7 +864,12 @@ delta_chunk_walk_kernel(DeltaArgs a) {
     auto chunk = [&](int item, Operands& x) {
       f32x4_t p = with_state(x.left, zero4());
       lds_barrier();
-      p = mfma4(x.q, u_of(item, half), p);
+      f32x4_t u = u_of(item, half);
+      if (half >= block && any_wild(u)) {
+        if (half == block) wild_from_its_row(u, p, g);      // (block 0 sees none of the second's)
+        u = without_wild(u);
+      }
+      p = mfma4(x.q, u, p);
       if (half == 1) late[block][lane] = p;
       request(min(item + 2, last - 1), x);
       lds_barrier();

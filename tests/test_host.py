@@ -90,6 +90,25 @@ def test_step_buffer_matches_an_independent_layout(window):
     assert again.offsets == ctx.offsets and np.array_equal(again.host, ctx.host)
 
 
+def test_work_items_of_long_portions_alone():
+    """A size with a least portion lists only the requests that bring as much."""
+    m = manager()
+    for r, n in (("a", 7), ("b", 5), ("c", 1), ("d", 6)):
+        m.admit(r)
+        m.reserve(r, n)
+    entries = [StepEntry("a", [1] * 7, []), StepEntry("b", [1] * 5, []), StepEntry("c", [1], [0]),
+               StepEntry("d", [1] * 6, [])]
+    ctx = build_step(entries, m, CPU, 100, ((4, 6), 4, (4, 1), (3, 6), (2, 50)))
+    seq, row0, cnt, n_items = ctx.items[4, 6]
+    assert (seq.tolist(), row0.tolist(), cnt.tolist(), n_items) == ([0, 0, 3, 3], [0, 4, 13, 17], [4, 3, 4, 2], 4)
+    assert ctx.attention_items(3, 6)[0].tolist() == [0, 0, 0, 3, 3] and ctx.items[2, 50][3] == 0
+    assert ctx.attention_items(4)[2].tolist() == [4, 3, 4, 1, 1, 4, 2]
+    for key in list(ctx.items):                      # and as the step itself would list them
+        made = tuple(t.tolist() for t in ctx.items.pop(key)[:3])
+        assert made == tuple(t.tolist() for t in ctx.attention_items(*(key if isinstance(key, tuple) else (key,)))[:3])
+    assert ctx.portions_below(6) == (6, 2, 6, 5) and ctx.portions_below(1) == (1, 0, 0, 0)
+
+
 def test_step_errors_name_the_request():
     m = manager()
     m.admit("a")

@@ -721,6 +721,68 @@ def test_delta_chunks_keep_a_bad_value_from_earlier_tokens(bad, at):
         assert float((got - want)[~after].abs().max()) < 2e-5 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("kind", ["ssd", "delta", "delta wide"])
+def test_a_portion_takes_its_form_by_its_own_length(kind):
+    """Single tokens and short portions of a request give the same bits alone and beside a portion
+    that is taken in chunks, which gives the same bits alone and beside them (32-bit, where every
+    other part sums in an order of its own too)."""
+    from zig_ai_amd.kernels import ops
+    cfg = ALONE[kind]
+    model, _ = build(cfg, seed=5)
+    n = ops.CHUNKED_FROM
+    prompts = [ru.tokens(14, cfg["vocab"], 1), ru.tokens(2 * n + 40, cfg["vocab"], 2)]
+    short = [(0, 0, 3), (0, 3, 4), (0, 4, 5), (0, 5, 13), (0, 13, 14)]
+    long = [(1, 0, n), (1, n, n + 40), (1, n + 40, 2 * n + 40)]
+
+    def run(schedule):
+        return eu.run_schedule(runner_for(model, tokens=2 * n + 80), prompts, schedule)
+
+    alone = run([([e], []) for e in short[:-1]] + [([short[-1]], [0])] + [([e], []) for e in long[:-1]]
+                + [([long[-1]], [1])])
+    beside = run([([short[0]], []), ([short[1], long[0]], []), ([long[1], short[2]], []),
+                  ([short[3], long[2]], [1]), ([short[4]], [0])])
+    for a, b in zip(alone, beside):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("form", ["ssd", "delta", "fixed"])
+def test_the_walk_of_short_portions_alone(form):
+    """With a limit the walk takes the shorter portions, to the bit as in a step of their own, and
+    leaves the others' rows and states alone."""
+    from zig_ai_amd.engine.batch import ShortPortions
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator().manual_seed(3)
+    H, G, d, dv, limit = 4, 2 if form != "fixed" else 4, 24, 40, 192
+    lengths, slots = [3, limit, 1, limit - 1, 250, 17], [3, 0, 5, 1, 6, 2]
+    conv = torch.randn(sum(lengths), 2 * G * d + H * dv, generator=gen).to(dev)
+    proj = torch.randn(sum(lengths), H, generator=gen).to(dev)
+    raw = torch.randn(sum(lengths), H * d, generator=gen).to(dev)
+    heads, channels = torch.rand(H, generator=gen).to(dev), torch.randn(H * d, generator=gen).to(dev)
+    before = torch.randn(7, H * d * dv, generator=gen).to(dev)
+
+    def walk(rows, lens, used, state, **kw):
+        _, start, slot_id = _step_arrays(lens, used, dev)
+        return ops.matrix_recurrence(
+            form, conv[rows].contiguous(), 0, G * d, 2 * G * d, None if form == "fixed" else proj[rows].contiguous(),
+            0, {"ssd": None, "fixed": heads}.get(form, raw[rows].contiguous()),
+            channels if form == "delta" else heads, heads, heads, state, 0, start, slot_id, H, G, d, dv, **kw)
+
+    short = [i for i, n in enumerate(lengths) if n < limit]
+    rows_of = [slice(sum(lengths[:i]), sum(lengths[:i + 1])) for i in range(len(lengths))]
+    lens = [lengths[i] for i in short]
+    out = torch.full((sum(lengths), H * dv), 7.0, device=dev)
+    state = before.clone()
+    walk(slice(None), lengths, slots, state, short=ShortPortions(limit, len(lens), sum(lens), max(lens)), out=out)
+    alone = before.clone()
+    idx = torch.cat([torch.arange(rows_of[i].start, rows_of[i].stop) for i in short]).to(dev)
+    want = walk(idx, lens, [slots[i] for i in short], alone)
+    assert torch.equal(out[idx], want) and torch.equal(state, alone)
+    for i in range(len(lengths)):
+        if i not in short:
+            assert bool((out[rows_of[i]] == 7.0).all()) and torch.equal(state[slots[i]], before[slots[i]])
+
+
 def test_small_kernels():
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")

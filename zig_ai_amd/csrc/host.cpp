@@ -593,8 +593,8 @@ ZA_EXPORT int za_cache_check(void* c) { return static_cast<Cache*>(c)->check(); 
 // ---- the step's integer buffer
 // Sections, in this order, each starting at a multiple of 4 entries: token_ids[T],
 // positions[T], token_seq[T], seq_start[S+1], ctx_len[S], slot_id[S], logit_rows[R];
-// per group slots[T], table[S * width]; per granularity item_seq, item_row0,
-// item_count.  The layout is a function of (tokens per entry, wanted rows per entry,
+// per group slots[T], table[S * width]; per granularity (a pair in `grans`: rows an item,
+// and the tokens from which on a portion is listed at all) item_seq, item_row0, item_count.  The layout is a function of (tokens per entry, wanted rows per entry,
 // table width) only.  `sections` receives (offset, length) pairs in that order,
 // `meta` = {T, S, R, table width, longest context (cached + new), total entries}.
 // With out == null only sections and meta are computed.  Every request must be
@@ -645,11 +645,13 @@ ZA_EXPORT int za_step_build(void* c, int S, const int64_t* reqs, const int* coun
     R += want_counts[s];
   }
   max_pages = std::max(max_pages, min_pages);
-  // work items: at most `gran` consecutive query rows of one request
+  // work items: at most `size` consecutive query rows of one request
   std::vector<long long> item_counts(n_gran, 0);
   for (int k = 0; k < n_gran; ++k) {
-    if (grans[k] <= 0) return fail(ZA_HOST_ARG, "a work-item size must be positive");
-    for (int s = 0; s < S; ++s) item_counts[k] += (counts[s] + grans[k] - 1) / grans[k];
+    const int size = grans[2 * k], from = grans[2 * k + 1];
+    if (size <= 0) return fail(ZA_HOST_ARG, "a work-item size must be positive");
+    for (int s = 0; s < S; ++s)
+      if (counts[s] >= from) item_counts[k] += (counts[s] + size - 1) / size;
   }
   long long total = 0;
   int sec = 0;
@@ -708,12 +710,13 @@ ZA_EXPORT int za_step_build(void* c, int S, const int64_t* reqs, const int* coun
   }
   out[o_start + S] = (int)row;
   for (int k = 0; k < n_gran; ++k) {
+    const int size = grans[2 * k], from = grans[2 * k + 1];
     long long at = 0, first = 0;
     for (int s = 0; s < S; ++s) {
-      for (int done = 0; done < counts[s]; done += grans[k]) {
+      for (int done = 0; counts[s] >= from && done < counts[s]; done += size) {
         out[o_iseq[k] + at] = s;
         out[o_irow[k] + at] = (int)(first + done);
-        out[o_icnt[k] + at] = std::min(grans[k], counts[s] - done);
+        out[o_icnt[k] + at] = std::min(size, counts[s] - done);
         ++at;
       }
       first += counts[s];

@@ -226,6 +226,7 @@ struct RecurrenceArgs {
                               // are given by (start, count) instead of n + 1 starts
   int decay_col;              // channel decay: the decay of head h and key channel i lies in
                               // `conv` at decay_col + h*dk + i
+  int below;                  // 0, or: only portions of fewer tokens are walked
 };
 
 // Forms of the walk: SSD and fixed decay, the delta rule, channel decay.
@@ -237,15 +238,23 @@ struct RecurrenceArgs {
 // vectors, the decays and the write strengths, once per token instead of once per
 // workgroup that walks the token.  grid (tokens, jobs): the first 2*G jobs of a token make
 // one unit vector each, the others take 256 decays each, the last one also the betas; a
-// job is one trip to memory, and the jobs of a token run side by side.
+// job is one trip to memory, and the jobs of a token run side by side.  With `below` (see
+// RecurrenceArgs) the grid is (requests times `longest`, jobs): the tokens of those portions alone.
 template <typename T>
 __global__ void __launch_bounds__(64)
 delta_prepare_kernel(const float* __restrict__ conv, int conv_width, int q_col, int k_col,
                      const T* __restrict__ proj, int proj_stride, int gate_col,
                      const T* __restrict__ decay, int decay_stride,
                      const float* __restrict__ dt_bias, const float* __restrict__ A_log,
-                     float* __restrict__ prep, int prep_width, int H, int G, int dk) {
-  const int t = blockIdx.x, job = blockIdx.y, lane = threadIdx.x;
+                     float* __restrict__ prep, int prep_width, int H, int G, int dk,
+                     const int* __restrict__ seq_start, int below, int longest) {
+  int t = blockIdx.x;
+  const int job = blockIdx.y, lane = threadIdx.x;
+  if (below) {
+    const int s = t / longest, at = t % longest, n = seq_start[s + 1] - seq_start[s];
+    if (n >= below || at >= n) return;
+    t = seq_start[s] + at;
+  }
   float* row = prep + (size_t)t * prep_width;
   if (job < 2 * G) {
     const int is_k = job >= G, g = is_k ? job - G : job;
@@ -339,6 +348,7 @@ matrix_recurrence_kernel(RecurrenceArgs a) {
   const bool owner = col < dv;
   const int start = a.seq_start[s];
   const int n = a.seq_count ? a.seq_count[s] : a.seq_start[s + 1] - start;
+  if (a.below && n >= a.below) return;
 
   // where the token's vectors lie: vector v of token t starts at base[v] + t * stride
   const float* base[NV];
@@ -597,7 +607,9 @@ static int launch_recurrence(const RecurrenceArgs& a, int n_seqs, int P, bool lo
 // `form`: 0 = SSD, 1 = gated delta rule, 2 = fixed decay (`decay` then holds H 32-bit
 // decays, one per head; proj, dt_bias, A_log and D are not read).  `lanes` (P): the power of two, at most 64, with
 // 16 * P >= dk that splits a column's rows.  `prep` (delta): [n_tokens][prep_width]
-// floats of scratch, prep_width >= 2*G*dk + H*dk + H.
+// floats of scratch, prep_width >= 2*G*dk + H*dk + H.  `below`: 0, or only portions of fewer tokens
+// are walked, of which there are short_seqs with short_tokens together and at most short_longest
+// (below `below`) each; the others' rows of `out` and their states are left alone.
 extern "C" int za_matrix_recurrence(int form, int dtype, const float* conv, int conv_width,
                                     int q_col, int k_col, int x_col, const void* proj,
                                     int proj_stride, int gate_col, const void* decay,
@@ -605,10 +617,17 @@ extern "C" int za_matrix_recurrence(int form, int dtype, const float* conv, int 
                                     const float* D, float* prep, int prep_width, float* state,
                                     long long slot_stride, const int* seq_start,
                                     const int* slot_id, float* out, int n_tokens, int n_seqs,
-                                    int H, int G, int dk, int dv, int lanes,
+                                    int H, int G, int dk, int dv, int lanes, int below,
+                                    int short_seqs, int short_tokens, int short_longest,
                                     hipStream_t stream) {
   if (n_seqs == 0 || n_tokens == 0) return 0;
-  if (form < 0 || form > 2) return ZA_ERR_ARG;
+  if (form < 0 || form > 2 || below < 0) return ZA_ERR_ARG;
+  if (below) {
+    if (short_seqs == 0) return 0;
+    if (short_seqs < 0 || short_seqs > n_seqs || short_longest <= 0 || short_longest >= below ||
+        short_tokens < short_seqs || (long long)n_seqs * short_longest > 0x7fffffffLL)
+      return ZA_ERR_ARG;
+  }
   if (n_seqs < 0 || n_tokens < 0 || H <= 0 || G <= 0 || H % G || dk <= 0 || dv <= 0 || !conv ||
       !state || !seq_start || !slot_id || !out)
     return ZA_ERR_ARG;
@@ -625,21 +644,21 @@ extern "C" int za_matrix_recurrence(int form, int dtype, const float* conv, int 
   RecurrenceArgs a{conv, conv_width, q_col, k_col, x_col, proj, proj_stride, gate_col, dtype,
                    prep, prep_width, dt_bias, A_log, form == 2 ? nullptr : D, state, slot_stride,
                    seq_start, slot_id, out, H, G, dk, dv,
-                   form == 2 ? (const float*)decay : nullptr, nullptr, 0};
+                   form == 2 ? (const float*)decay : nullptr, nullptr, 0, below};
   // (a function of the step's shape alone, as a recorded step needs it)
-  const bool long_portions = n_tokens > 4 * n_seqs;
+  const bool long_portions = below ? short_tokens > 4 * short_seqs : n_tokens > 4 * n_seqs;
   if (form != 1) return launch_recurrence<RC_SSD>(a, n_seqs, lanes, long_portions, stream);
-  const dim3 prep_grid(n_tokens, 2 * G + (H * dk + 255) / 256);
+  const dim3 prep_grid(below ? n_seqs * short_longest : n_tokens, 2 * G + (H * dk + 255) / 256);
   if (dtype == 0)
     hipLaunchKernelGGL((delta_prepare_kernel<float>), prep_grid, dim3(64), 0, stream, conv,
                        conv_width, q_col, k_col, (const float*)proj, proj_stride, gate_col,
                        (const float*)decay, decay_stride, dt_bias, A_log, prep, prep_width, H, G,
-                       dk);
+                       dk, seq_start, below, short_longest);
   else
     hipLaunchKernelGGL((delta_prepare_kernel<bf16_t>), prep_grid, dim3(64), 0, stream, conv,
                        conv_width, q_col, k_col, (const bf16_t*)proj, proj_stride, gate_col,
                        (const bf16_t*)decay, decay_stride, dt_bias, A_log, prep, prep_width, H, G,
-                       dk);
+                       dk, seq_start, below, short_longest);
   const int rc = za_launch_status();
   if (rc != 0) return rc;
   return launch_recurrence<RC_DELTA>(a, n_seqs, lanes, long_portions, stream);

@@ -210,8 +210,9 @@ decay_chunk_state_kernel(DecayArgs a) {
   }
 }
 
-// One thread a state element; the chunks of a request are neighbours in the list.  Chunk states
-// become the states before their chunks; the last one goes back to the request's slot.
+// One thread a state element; the chunks of a request are neighbours in the list (a request without
+// one is left alone).  Chunk states become the states before their chunks; the last one goes back
+// to the request's slot.
 __global__ void __launch_bounds__(256)
 decay_prefix_kernel(float* __restrict__ chunk_state, float* __restrict__ state, long long slot_stride,
                     const int* __restrict__ slot_id, const int* __restrict__ item_seq, int n_items,
@@ -226,8 +227,8 @@ decay_prefix_kernel(float* __restrict__ chunk_state, float* __restrict__ state, 
       atomicMax(&bounds[1], i + 1);
     }
   __syncthreads();
-  if (e >= elems) return;
   const int first = bounds[0], last = bounds[1];
+  if (e >= elems || first >= last) return;
   float* slot = state + (size_t)slot_id[s] * slot_stride + e;
   float S = *slot;
   for (int i0 = first; i0 < last; i0 += 8) {
@@ -408,8 +409,8 @@ decay_chunk_out_kernel(DecayArgs a) {
   }
 }
 
-// `items`: the step's work items of at most DC_CHUNK rows, a request's side by side; scratch:
-// `sums` n_tokens*H*3, `chunk_state` n_items*H*dv*dk, `total` n_items*H floats.
+// `items`: work items of at most DC_CHUNK rows, a request's side by side, of the requests that are
+// taken (the others' rows of `out` and their states are left alone); scratch: `sums` n_tokens*H*3, `chunk_state` n_items*H*dv*dk, `total` n_items*H floats.
 extern "C" int za_decay_chunked(const float* vec, int width, int q_col, int k_col, int x_col,
                                 const void* proj, int dtype, int proj_stride, int gate_col,
                                 const float* dt_bias, const float* A_log, const float* D,
@@ -419,7 +420,7 @@ extern "C" int za_decay_chunked(const float* vec, int width, int q_col, int k_co
                                 float* chunk_state, float* total, float* out, int n_tokens, int H,
                                 int G, int dk, int dv, hipStream_t stream) {
   if (n_tokens == 0 || n_items == 0) return 0;
-  if (n_tokens < 0 || n_seqs <= 0 || n_items < n_seqs || H <= 0 || G <= 0 || H % G || dk <= 0 || dv <= 0 ||
+  if (n_tokens < 0 || n_seqs <= 0 || n_items < 0 || H <= 0 || G <= 0 || H % G || dk <= 0 || dv <= 0 ||
       !vec || !state || !slot_id || !item_seq || !item_row0 || !item_count || !sums || !chunk_state ||
       !total || !out || slot_stride < (long long)H * dk * dv)
     return ZA_ERR_ARG;
@@ -907,8 +908,8 @@ delta_chunk_walk_kernel(DeltaArgs a) {
   }
 }
 
-// dtype: 0 = float32, 1 = bfloat16 (proj and decay).  `items`: the step's work items of at most
-// DL_CHUNK rows, a request's side by side and full but for its last; scratch (floats, n_items times
+// dtype: 0 = float32, 1 = bfloat16 (proj and decay).  `items`: work items of at most DL_CHUNK rows, a
+// request's side by side and full but for its last, of the requests that are taken; scratch (floats, n_items times
 // H of them each): qp, W and kp 32*dk, U 32*dv, Q 32*32, grow dk, all on 16 bytes.
 extern "C" int za_delta_chunked(int dtype, const float* conv, int conv_width, int q_col, int k_col, int x_col,
                                 const void* proj, int proj_stride, int gate_col, const void* decay,
@@ -918,7 +919,7 @@ extern "C" int za_delta_chunked(int dtype, const float* conv, int conv_width, in
                                 float* qp, float* W, float* U, float* Q, float* kp, float* grow, float* out,
                                 int n_tokens, int H, int G, int dk, int dv, hipStream_t stream) {
   if (n_tokens == 0 || n_items == 0) return 0;
-  if (n_tokens < 0 || n_seqs <= 0 || n_items < n_seqs || H <= 0 || G <= 0 || H % G || dk <= 0 || dv <= 0 || !conv ||
+  if (n_tokens < 0 || n_seqs <= 0 || n_items < 0 || H <= 0 || G <= 0 || H % G || dk <= 0 || dv <= 0 || !conv ||
       !proj || !decay || !dt_bias || !A_log || !state || !slot_id || !item_seq || !item_row0 || !item_count ||
       !qp || !W || !U || !Q || !kp || !grow || !out || decay_stride < H * dk ||
       slot_stride < (long long)H * dk * dv)

@@ -12,7 +12,7 @@ device in one transfer.
 from __future__ import annotations
 
 from dataclasses import dataclass, field
-from typing import Dict, Hashable, List, Optional, Sequence, Tuple
+from typing import Dict, Hashable, List, NamedTuple, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -33,6 +33,26 @@ class StepEntry:
     want: Sequence[int] = ()      # indices into ``tokens`` whose logits are returned
 
 
+class ShortPortions(NamedTuple):
+    """The portions of a step with fewer than ``limit`` tokens."""
+    limit: int
+    requests: int
+    tokens: int
+    longest: int
+
+
+def item_size(granularity) -> Tuple[int, int]:
+    """A work-item size as (rows an item, tokens from which on a portion is listed at all):
+    given as that pair, or as the rows alone."""
+    rows, start = granularity if isinstance(granularity, tuple) else (granularity, 1)
+    return int(rows), int(start)
+
+
+def item_sizes(granularities) -> np.ndarray:
+    """The sizes as the host library takes them: int32 pairs in ascending order."""
+    return np.asarray(sorted({item_size(g) for g in granularities}), dtype=np.int32).reshape(-1, 2)
+
+
 @dataclass
 class StepContext:
     n_tokens: int
@@ -48,7 +68,8 @@ class StepContext:
     logit_rows: torch.Tensor              # int32 [R]   rows whose logits are wanted
     block_tables: Dict[int, torch.Tensor] = field(default_factory=dict)   # group -> [S, max_pages]
     slot_mapping: Dict[int, torch.Tensor] = field(default_factory=dict)   # group -> [T]
-    items: Dict[int, Tuple[torch.Tensor, torch.Tensor, torch.Tensor, int]] = field(default_factory=dict)
+    items: Dict[Hashable, Tuple[torch.Tensor, torch.Tensor, torch.Tensor, int]] = field(default_factory=dict)
+    short: Dict[int, ShortPortions] = field(default_factory=dict)
     # host copies, for parts written in plain torch and for planning
     seq_lens_host: List[int] = field(default_factory=list)
     ctx_lens_host: List[int] = field(default_factory=list)
@@ -64,24 +85,33 @@ class StepContext:
     # left such a copy; the model drops it as soon as anything else touches the stream
     rounded: Optional[torch.Tensor] = None
 
-    def attention_items(self, rows_per_item: int):
-        """Work items of at most ``rows_per_item`` consecutive query rows of one
-        request: (request index, first row, row count) arrays and their number."""
-        if rows_per_item not in self.items:
-            seq, row0, cnt = _make_items(self.seq_lens_host, rows_per_item)
+    def attention_items(self, rows_per_item: int, from_tokens: int = 1):
+        """Work items of at most ``rows_per_item`` consecutive query rows of one request that
+        brings ``from_tokens`` or more: (request index, first row, row count) arrays and their
+        number."""
+        key = rows_per_item if from_tokens <= 1 else (rows_per_item, from_tokens)
+        if key not in self.items:
+            seq, row0, cnt = _make_items(self.seq_lens_host, rows_per_item, from_tokens)
             dev = self.token_ids.device
-            self.items[rows_per_item] = (
+            self.items[key] = (
                 torch.tensor(seq, dtype=torch.int32, device=dev),
                 torch.tensor(row0, dtype=torch.int32, device=dev),
                 torch.tensor(cnt, dtype=torch.int32, device=dev), len(seq))
-        return self.items[rows_per_item]
+        return self.items[key]
+
+    def portions_below(self, limit: int) -> ShortPortions:
+        """The step's portions of fewer than ``limit`` tokens."""
+        if limit not in self.short:
+            lens = [n for n in self.seq_lens_host if n < limit]
+            self.short[limit] = ShortPortions(limit, len(lens), sum(lens), max(lens, default=0))
+        return self.short[limit]
 
 
-def _make_items(seq_lens: Sequence[int], rows_per_item: int):
+def _make_items(seq_lens: Sequence[int], rows_per_item: int, from_tokens: int = 1):
     seq, row0, cnt = [], [], []
     row = 0
     for s, n in enumerate(seq_lens):
-        done = 0
+        done = 0 if n >= from_tokens else n
         while done < n:
             c = min(rows_per_item, n - done)
             seq.append(s)
@@ -198,7 +228,7 @@ class StagingRing:
 
 
 def build_step(entries: Sequence[StepEntry], cache: CacheManager, device: torch.device,
-               vocab_size: int, item_granularities: Sequence[int] = (),
+               vocab_size: int, item_granularities: Sequence = (),
                max_position: int = 0, min_pages: int = 0, max_keys: int = 0,
                into: Optional[torch.Tensor] = None,
                staging=None,
@@ -219,7 +249,7 @@ def build_step(entries: Sequence[StepEntry], cache: CacheManager, device: torch.
     prep = prepared if prepared is not None else PreparedEntries(entries, cache, vocab_size)
     S = len(entries)
     counts, meta = prep.counts, prep.meta
-    grans = np.asarray(sorted(set(int(g) for g in item_granularities)), dtype=np.int32)
+    grans = item_sizes(item_granularities)
     groups = cache.groups
     n_sections = 7 + 2 * len(groups) + 3 * len(grans)
     sections = np.zeros((2 * n_sections,), dtype=np.int64)
@@ -244,11 +274,12 @@ def build_step(entries: Sequence[StepEntry], cache: CacheManager, device: torch.
     names = ["token_ids", "positions", "token_seq", "seq_start", "ctx_len", "slot_id", "logit_rows"]
     for g in groups:
         names += [f"slots{g.index}", f"table{g.index}"]
-    for gran in grans.tolist():
-        names += [f"iseq{gran}", f"irow{gran}", f"icnt{gran}"]
+    lists = {rows if start <= 1 else (rows, start): str(rows) if start <= 1 else f"{rows}from{start}"
+             for rows, start in grans.tolist()}
+    for name in lists.values():
+        names += [f"iseq{name}", f"irow{name}", f"icnt{name}"]
     offsets = {name: (int(sections[2 * i]), int(sections[2 * i + 1])) for i, name in enumerate(names)}
     seq_lens, ctx_lens, slots = counts.tolist(), ctx_arr.tolist(), slot_arr.tolist()
-    item_lists = {gran: offsets[f"iseq{gran}"][1] for gran in grans.tolist()}
 
     if into is None and ring is not None:
         dev = torch.empty((host.size,), dtype=torch.int32, device=device)
@@ -281,6 +312,7 @@ def build_step(entries: Sequence[StepEntry], cache: CacheManager, device: torch.
     for g in groups:
         ctx.slot_mapping[g.index] = view(f"slots{g.index}")
         ctx.block_tables[g.index] = view(f"table{g.index}").view(S, max_pages)
-    for gran, n_items in item_lists.items():
-        ctx.items[gran] = (view(f"iseq{gran}"), view(f"irow{gran}"), view(f"icnt{gran}"), n_items)
+    for key, name in lists.items():
+        ctx.items[key] = (view(f"iseq{name}"), view(f"irow{name}"), view(f"icnt{name}"),
+                          offsets[f"iseq{name}"][1])
     return ctx

@@ -27,7 +27,7 @@ import torch
 
 from ..cache.pages import raise_for
 from ..kernels import host as hostlib
-from .batch import PreparedEntries, StepEntry, StepError, build_step
+from .batch import PreparedEntries, StepEntry, StepError, build_step, item_sizes
 
 PAGE_BUCKET = 64        # block-table width is rounded up to a multiple of this
 KEYS_BUCKET = 1024      # and the longest context to a multiple of this
@@ -55,7 +55,7 @@ class DecodeGraphs:
     collector, which may run at any allocation, also in the middle of a capture,
     and destroying another graph while a capture is open aborts the process."""
 
-    def __init__(self, vocab_size: int, item_granularities: Sequence[int], max_position: int):
+    def __init__(self, vocab_size: int, item_granularities: Sequence, max_position: int):
         self._vocab = vocab_size
         self._granularities = tuple(item_granularities)
         self._max_position = max_position
@@ -224,7 +224,7 @@ class DecodeGraphs:
                                self._granularities, self._max_position,
                                min_pages=key[1], max_keys=key[2], prepared=prepared)
             words = probe.host.size
-            grans = np.asarray(sorted(set(int(g) for g in self._granularities)), dtype=np.int32)
+            grans = item_sizes(self._granularities)
             slot = {"buffer": torch.full((words,), -1, dtype=torch.int32, device=runner.device),
                     "pinned": torch.empty((words,), dtype=torch.int32, pin_memory=True),
                     "graph": None, "logits": None, "copied": None, "words": words, "seen": 0,
@@ -290,7 +290,7 @@ class DecodeGraphs:
             ctx = build_step(entries, cache, runner.device, self._vocab, self._granularities,
                              self._max_position, prepared=prepared, staging=runner.staging)
             return model.forward(ctx, runner.views)
-        grans = np.asarray(sorted(set(int(g) for g in self._granularities)), dtype=np.int32)
+        grans = item_sizes(self._granularities)
         sections = np.zeros((2 * (7 + 2 * len(cache.groups) + 3 * len(grans)),), dtype=np.int64)
         prepared.build(cache, grans, self._max_position, 0, sections, None, 0)     # sizes only
         widest, longest = int(prepared.meta[3]), int(prepared.meta[4])

@@ -16,7 +16,7 @@ from ..kernels import build as kernel_build
 from ..kernels import ops
 from ..parts import base as parts
 from ..weights.loader import load_tensors
-from .batch import StepContext
+from .batch import StepContext, item_size
 
 EMBEDDING_CACHE = "embedding"      # the embedding's entry among the cache needs
 
@@ -152,8 +152,8 @@ class DecoderModel:
         for b in self.blocks:
             top += list(b.parts.values())
         every = [q for p in top for q in walk_parts(p)]
-        self.item_granularities = sorted({
-            g for p in every for g in getattr(p, "item_granularities", ())})
+        self.item_granularities = sorted(
+            {g for p in every for g in getattr(p, "item_granularities", ())}, key=item_size)
         self.kernel_sources = sorted(sources)
         # A step may be recorded into a HIP graph only if no part looks at the step's
         # numbers on the host while it runs.

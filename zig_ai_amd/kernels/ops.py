@@ -121,7 +121,8 @@ _SIGNATURES = {
                                             c_void_p, c_int, c_int, c_void_p, c_int, c_void_p,
                                             c_void_p, c_void_p, c_void_p, c_int, c_void_p,
                                             c_longlong, c_void_p, c_void_p, c_void_p, c_int, c_int,
-                                            c_int, c_int, c_int, c_int, c_int, c_void_p],
+                                            c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+                                            c_int, c_void_p],
     ("recurrent", "za_gated_group_norm"): [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int,
                                            c_void_p, c_int, c_int, c_int, c_int, c_int, c_float,
                                            c_int, c_int, c_float, c_void_p],
@@ -2168,6 +2169,7 @@ def causal_conv_silu(x: torch.Tensor, col0: int, taps: torch.Tensor, bias: Optio
 
 
 RECURRENCE_ROWS_PER_LANE = 16
+NO_LIMIT = (0, 0, 0, 0)        # in place of a step's short portions: every portion is walked
 
 
 def recurrence_plan(dk: int, dv: int) -> Tuple[int, int, int]:
@@ -2181,11 +2183,19 @@ def recurrence_plan(dk: int, dv: int) -> Tuple[int, int, int]:
     return lanes, RECURRENCE_ROWS_PER_LANE, 64 // lanes
 
 
+def _rows_of(out: Optional[torch.Tensor], T: int, width: int, device) -> torch.Tensor:
+    if out is None:
+        return torch.empty((T, width), dtype=torch.float32, device=device)
+    _need(out, "out", torch.float32, (T, width))
+    return out
+
+
 def matrix_recurrence(form: str, conv: torch.Tensor, q_col: int, k_col: int, x_col: int,
                       proj: torch.Tensor, gate_col: int, decay: Optional[torch.Tensor],
                       dt_bias: torch.Tensor, A_log: torch.Tensor, D: Optional[torch.Tensor],
                       state: torch.Tensor, state_offset: int, seq_start: torch.Tensor,
-                      slot_id: torch.Tensor, heads: int, groups: int, dk: int, dv: int) -> torch.Tensor:
+                      slot_id: torch.Tensor, heads: int, groups: int, dk: int, dv: int,
+                      short=None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The token-by-token walk of csrc/recurrent.hip.  ``form``: ``"ssd"``, ``"delta"`` or
     ``"fixed"`` (one constant decay a head in ``decay``, 32-bit ``[heads]``; ``proj``, ``dt_bias``,
     ``A_log`` and ``D`` are not read and may be None: see ``_fixed_decay_recurrence``).
@@ -2194,12 +2204,14 @@ def matrix_recurrence(form: str, conv: torch.Tensor, q_col: int, k_col: int, x_c
     ``x_col`` (``heads`` of ``dv``); ``proj [T, columns]`` holds one raw number per head at
     ``gate_col`` (ssd: the step size, delta: the write strength); ``decay [T, >= heads*dk]``
     (delta) the raw decays in its first ``heads*dk`` columns.  The state of slot ``s`` lies at ``state[s, state_offset:]`` as
-    ``[heads][dv][dk]``.  Returns 32-bit ``[T, heads*dv]``."""
+    ``[heads][dv][dk]``.  Returns 32-bit ``[T, heads*dv]``.  ``short``
+    (``StepContext.portions_below``): only those portions are walked; the other requests' rows of
+    ``out`` and their states are left alone."""
     if form not in ("ssd", "delta", "fixed"):
         raise KernelError(f"form must be ssd, delta or fixed, got {form!r}")
     if form == "fixed":
         return _fixed_decay_recurrence(conv, q_col, k_col, x_col, decay, state, state_offset,
-                                       seq_start, slot_id, heads, groups, dk, dv)
+                                       seq_start, slot_id, heads, groups, dk, dv, short, out)
     delta = form == "delta"
     T, conv_width = conv.shape
     _need(conv, "conv", torch.float32)
@@ -2228,7 +2240,7 @@ def matrix_recurrence(form: str, conv: torch.Tensor, q_col: int, k_col: int, x_c
     _need(slot_id, "slot_id", torch.int32, (S,))
     base, slot_stride = _state_window(state, state_offset, heads * dk * dv, "state")
     lanes, _, _ = recurrence_plan(dk, dv)
-    out = torch.empty((T, heads * dv), dtype=torch.float32, device=conv.device)
+    out = _rows_of(out, T, heads * dv, conv.device)
     prep, prep_width = None, 0
     if delta:
         # what a token brings that does not depend on the state: unit q and k, decays, betas
@@ -2239,7 +2251,7 @@ def matrix_recurrence(form: str, conv: torch.Tensor, q_col: int, k_col: int, x_c
         int(x_col), _ptr(proj), proj.shape[1], int(gate_col), _ptr(decay) if delta else None,
         decay.shape[1] if delta else 0, _ptr(dt_bias), _ptr(A_log), None if delta else _ptr(D),
         _ptr(prep), prep_width, base, slot_stride, _ptr(seq_start), _ptr(slot_id), _ptr(out), T,
-        S, heads, groups, dk, dv, lanes, _stream())
+        S, heads, groups, dk, dv, lanes, *(short or NO_LIMIT), _stream())
     _check(rc, "matrix_recurrence", f"form={form} heads={heads} dk={dk} dv={dv}")
     return out
 
@@ -2247,7 +2259,8 @@ def matrix_recurrence(form: str, conv: torch.Tensor, q_col: int, k_col: int, x_c
 def _fixed_decay_recurrence(vectors: torch.Tensor, q_col: int, k_col: int, x_col: int,
                             decay: torch.Tensor, state: torch.Tensor, state_offset: int,
                             seq_start: torch.Tensor, slot_id: torch.Tensor, heads: int, groups: int,
-                            dk: int, dv: int) -> torch.Tensor:
+                            dk: int, dv: int, short=None,
+                            out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``matrix_recurrence``'s form ``"fixed"``: ``S <- decay[h] S + k v^T; o = S^T q`` with one
     constant decay a head (32-bit ``[heads]``); ``vectors [T, columns]`` holds q and k
     (``groups`` of ``dk``) and v (``heads`` of ``dv``) at the three columns."""
@@ -2265,11 +2278,11 @@ def _fixed_decay_recurrence(vectors: torch.Tensor, q_col: int, k_col: int, x_col
     _need(slot_id, "slot_id", torch.int32, (S,))
     base, slot_stride = _state_window(state, state_offset, heads * dk * dv, "state")
     lanes, _, _ = recurrence_plan(dk, dv)
-    out = torch.empty((T, heads * dv), dtype=torch.float32, device=vectors.device)
+    out = _rows_of(out, T, heads * dv, vectors.device)
     rc = _fn("recurrent", "za_matrix_recurrence")(
         2, 0, _ptr(vectors), width, int(q_col), int(k_col), int(x_col), None, 0, 0, _ptr(decay),
         0, None, None, None, None, 0, base, slot_stride, _ptr(seq_start), _ptr(slot_id),
-        _ptr(out), T, S, heads, groups, dk, dv, lanes, _stream())
+        _ptr(out), T, S, heads, groups, dk, dv, lanes, *(short or NO_LIMIT), _stream())
     _check(rc, "matrix_recurrence", f"form=fixed heads={heads} dk={dk} dv={dv}")
     return out
 
@@ -2279,27 +2292,32 @@ DELTA_CHUNK = 32               # and where every key channel has one beside a de
 CHUNKED_MAX_DK = 128           # state rows of a head that the chunks' kernels take
 
 
-def in_chunks(seq_lens) -> bool:
-    """Whether a step's portions (``seq_lens``: the tokens of every request) are taken as chunks
-    rather than walked token by token (a function of the step's shape alone): from 192 tokens in a
-    portion on.  The walk's time is its longest portion's, 0.34 us a token (delta rule 0.4), more
-    when there are many; chunks start at some 30 us.  Measured (us, walked and in chunks; 64 heads
-    of 128 x 64 with one decay a token; 16 of 128 x 128 with a delta rule): one portion of 64 tokens
-    25 and 32; 36 and 37; of 128 46 and 45; 65 and 43; eight of 256 330 and 156; 285 and 144; one of
-    2,048 698 and 155; 878 and 206.  Between 112 and 192 chunks would win 10 to 30 us a layer;
-    portions that short are walked all the same, so that a prompt cut into small portions gives
-    the same bits as whole."""
-    return max(seq_lens, default=0) >= 192
+# A portion of this many tokens or more is taken in chunks, a shorter one walked token by token,
+# each by its own length: which form a request meets, and so the order of its sums, does not hang on
+# what else its step brings.  A prompt shorter than this leaves the same bits in one portion as in
+# several; a longer one the same up to the order of its 32-bit sums.
+# The walk's time is its longest portion's, 0.34 us a token (delta rule 0.43), more when there are
+# many, and it comes on top of the chunks of a step that has both; chunks start at some 25 us.
+# Measured (us, walked and in chunks; 64 heads of 128 x 64 and 16 of 64 x 128 with one decay a token,
+# 16 of 128 x 128 with a delta rule):
+#   tokens              64                    96                   128                   160
+#   one portion   25 33, 20 23, 36 37   36 43, 29 31, 50 39   47 47, 38 33, 64 42   58 47, 46 33, 78 44
+#   eight         86 64, 23 26, 86 71 125 80, 32 35, 119 78 164 90, 41 37, 153 88 203 156, 50 54, 186 122
+#   beside 512   102 77, 55 36, 111 74 124 77, 63 36, 124 74 145 78, 71 36, 139 75 167 78, 81 36, 153 75
+# The line is the first of these where chunks are clearly ahead in a portion alone.  Beside a long
+# portion they are from some 32 tokens on, and a lower line would gain 10 to 80 us a layer there; it
+# would also have short prompts, which are walked in any case when they come in pieces, depend on
+# their pieces.  Single tokens beside a long portion: 64 of them beside 2,048 241 us, as chunks of
+# their own 444 (delta rule 248 and 491), 30 beside 512 98 and 167 (102 and 185).
+CHUNKED_FROM = 160
 
 
-def _chunk_items(items, n_seqs: int, what: str):
+def _chunk_items(items):
     item_seq, item_row0, item_count, n_items = items
     for name, t in (("item_seq", item_seq), ("item_row0", item_row0), ("item_count", item_count)):
         _need(t, name, torch.int32)
         if t.numel() < n_items:
             raise KernelError(f"{name} holds {t.numel()} entries, fewer than {n_items} items")
-    if n_items < n_seqs:
-        raise KernelError(f"{what}: {n_items} items for {n_seqs} requests")
 
 
 def _columns(width: int, *blocks) -> None:
@@ -2314,7 +2332,7 @@ def _decay_chunked(vectors, q_col, k_col, x_col, proj, gate_col, dt_bias, A_log,
     S = slot_id.numel()
     _need(vectors, "vectors", torch.float32)
     _need(slot_id, "slot_id", torch.int32, (S,))
-    _chunk_items(items, S, "recurrence in chunks")
+    _chunk_items(items)
     if dk > CHUNKED_MAX_DK:
         raise KernelError(f"dk={dk}: chunks take up to {CHUNKED_MAX_DK} state rows")
     if heads % groups:
@@ -2340,11 +2358,12 @@ def fixed_decay_recurrence_chunked(vectors: torch.Tensor, q_col: int, k_col: int
                                    decay: torch.Tensor, state: torch.Tensor, state_offset: int,
                                    slot_id: torch.Tensor, items, heads: int, dk: int,
                                    dv: int) -> torch.Tensor:
-    """The fixed-decay walk of ``matrix_recurrence`` for steps with long portions: ``items``
-    (``StepContext.attention_items(RETENTION_CHUNK)``: request, first row, rows, number) cut
-    every request's rows into chunks that are taken side by side as matrix products
-    (csrc/recurrent_chunks.hip).  Decays must not be negative.  Same result as the plain walk up
-    to the order of 32-bit additions."""
+    """The fixed-decay walk of ``matrix_recurrence`` for long portions: ``items``
+    (``StepContext.attention_items(RETENTION_CHUNK, CHUNKED_FROM)``: request, first row, rows,
+    number) cut those requests' rows into chunks that are taken side by side as matrix products
+    (csrc/recurrent_chunks.hip); other requests' rows of the result are not written and their
+    states are left alone.  Decays must not be negative.  Same result as the plain walk up to the
+    order of 32-bit additions."""
     _need(decay, "decay", torch.float32, (heads,))
     return _decay_chunked(vectors, q_col, k_col, x_col, None, 0, None, None, None, decay, state, state_offset,
                           slot_id, items, heads, heads, dk, dv)
@@ -2369,9 +2388,10 @@ def delta_recurrence_chunked(conv: torch.Tensor, q_col: int, k_col: int, x_col: 
                              gate_col: int, decay: torch.Tensor, dt_bias: torch.Tensor, A_log: torch.Tensor,
                              state: torch.Tensor, state_offset: int, slot_id: torch.Tensor, items,
                              heads: int, groups: int, dk: int, dv: int) -> torch.Tensor:
-    """``matrix_recurrence``'s form ``"delta"`` for steps with long portions, in chunks of
-    ``DELTA_CHUNK`` tokens (``items``: ``StepContext.attention_items(DELTA_CHUNK)``) as matrix
-    products (csrc/recurrent_chunks.hip).  Same result up to the order of 32-bit operations."""
+    """``matrix_recurrence``'s form ``"delta"`` for long portions, in chunks of ``DELTA_CHUNK``
+    tokens (``items``: ``StepContext.attention_items(DELTA_CHUNK, CHUNKED_FROM)``) as matrix
+    products (csrc/recurrent_chunks.hip); other requests are left alone.  Same result up to the
+    order of 32-bit operations."""
     T, conv_width = conv.shape
     _need(conv, "conv", torch.float32)
     _need(proj, "proj", (torch.float32, torch.bfloat16))
@@ -2388,7 +2408,7 @@ def delta_recurrence_chunked(conv: torch.Tensor, q_col: int, k_col: int, x_col: 
     _need(dt_bias, "dt_bias", torch.float32, (heads * dk,))
     S = slot_id.numel()
     _need(slot_id, "slot_id", torch.int32, (S,))
-    _chunk_items(items, S, "delta rule in chunks")
+    _chunk_items(items)
     if dk > CHUNKED_MAX_DK:
         raise KernelError(f"dk={dk}: chunks take up to {CHUNKED_MAX_DK} state rows")
     base, slot_stride = _state_window(state, state_offset, heads * dk * dv, "state")

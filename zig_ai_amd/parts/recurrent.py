@@ -43,7 +43,7 @@ side by side are normed together, times a weight ``norm.weight`` of ``num_heads 
 and ``gate`` (``"silu"`` or ``"sigmoid"`` of the gate's projection, applied behind the norm).
 Lightning attention is ``activation="silu"``, ``key_scale=1``, ``output_norm="all"``,
 ``gate="sigmoid"`` and no position encoding.
-A step with long portions takes them in chunks, as matrix products
+A portion of ``ops.CHUNKED_FROM`` tokens or more is taken in chunks, as matrix products
 (``ops.fixed_decay_recurrence_chunked``; ``ssd`` and ``gated_delta`` have such forms too): the
 state is linear in what it was before a chunk.
 
@@ -71,6 +71,19 @@ import torch
 from ..kernels import ops
 from .base import Mixer, Runtime, StateNeed, TensorRule, lookup, register_mixer
 from .feed_forward import fuse_rows, pad_columns, pad_rows
+
+
+def by_length(step, walk, chunks, size):
+    """The recurrence of a step: portions of ``ops.CHUNKED_FROM`` tokens or more by
+    ``chunks(items)`` with work items of ``size`` rows, shorter ones by ``walk(short, out)``; ``size``
+    0: all of them walked."""
+    short = step.portions_below(ops.CHUNKED_FROM) if size else None
+    if short is None or short.requests == step.n_seqs:
+        return walk(None, None)
+    out = chunks(step.attention_items(size, ops.CHUNKED_FROM))
+    if short.requests:
+        walk(short, out)
+    return out
 
 
 class StateSpaceDuality(Mixer):
@@ -126,8 +139,8 @@ class StateSpaceDuality(Mixer):
         self.norm_w = tensors["norm.weight"]
         self.conv_state = (self.inner + 2 * G * N) * (L - 1)      # floats before S in a slot
         # long portions are taken in chunks (the step's work items of that size)
-        self.chunked = N <= ops.CHUNKED_MAX_DK
-        self.item_granularities = [ops.RETENTION_CHUNK] if self.chunked else []
+        self.chunk = ops.RETENTION_CHUNK if N <= ops.CHUNKED_MAX_DK else 0
+        self.item_granularities = [(self.chunk, ops.CHUNKED_FROM)] if self.chunk else []
         ops.check_projection_weight(self.w_in, "ssd in_proj")
         ops.check_projection_weight(self.w_out, "ssd out_proj")
 
@@ -136,16 +149,15 @@ class StateSpaceDuality(Mixer):
         z = ops.linear(x, self.w_in, tune=self.runtime.tune)
         conv = ops.causal_conv_silu(z, inner, self.conv_w, self.conv_b, cache.state, 0,
                                     step.token_seq, step.seq_start, step.slot_id)
-        if self.chunked and ops.in_chunks(step.seq_lens_host):
-            items = step.attention_items(ops.RETENTION_CHUNK)
-            y = ops.ssd_recurrence_chunked(conv, inner + G * N, inner, 0, z, 2 * inner + 2 * G * N, self.dt_bias,
-                                           self.A_log, self.D, cache.state, self.conv_state, step.slot_id,
-                                           items, self.heads, G, N, self.head_dim)
-        else:
-            y = ops.matrix_recurrence("ssd", conv, inner + G * N, inner, 0, z, 2 * inner + 2 * G * N,
-                                      None, self.dt_bias, self.A_log, self.D, cache.state,
-                                      self.conv_state, step.seq_start, step.slot_id, self.heads, G, N,
-                                      self.head_dim)
+        y = by_length(
+            step, lambda short, out: ops.matrix_recurrence(
+                "ssd", conv, inner + G * N, inner, 0, z, 2 * inner + 2 * G * N, None, self.dt_bias,
+                self.A_log, self.D, cache.state, self.conv_state, step.seq_start, step.slot_id,
+                self.heads, G, N, self.head_dim, short=short, out=out),
+            lambda items: ops.ssd_recurrence_chunked(
+                conv, inner + G * N, inner, 0, z, 2 * inner + 2 * G * N, self.dt_bias, self.A_log,
+                self.D, cache.state, self.conv_state, step.slot_id, items, self.heads, G, N,
+                self.head_dim), self.chunk)
         h = ops.gated_group_norm(y, z, 0, self.norm_w, inner // self.norm_groups, self.eps,
                                  "silu", gate_first=True)
         return ops.linear(h, self.w_out, tune=self.runtime.tune)
@@ -220,8 +232,8 @@ class GatedDeltaRule(Mixer):
         self.w_out = ops.projection_weight(tensors["out_proj.weight"])
         self.conv_state = (2 * G * d + H * dv) * (L - 1)
         # long portions are taken in chunks (the step's work items of that size)
-        self.chunked = d <= ops.CHUNKED_MAX_DK
-        self.item_granularities = [ops.DELTA_CHUNK] if self.chunked else []
+        self.chunk = ops.DELTA_CHUNK if d <= ops.CHUNKED_MAX_DK else 0
+        self.item_granularities = [(self.chunk, ops.CHUNKED_FROM)] if self.chunk else []
         for w, what in ((self.w_in, "in"), (self.w_up, "low-rank up"), (self.w_out, "out")):
             ops.check_projection_weight(w, f"gated_delta {what} projection")
 
@@ -232,15 +244,14 @@ class GatedDeltaRule(Mixer):
                                     step.seq_start, step.slot_id)
         low = ops.copy_columns(z, self.low_col, self.low_width)
         up = ops.linear(low, self.w_up, tune=self.runtime.tune)      # decay: H*d | gate: H*dv
-        if self.chunked and ops.in_chunks(step.seq_lens_host):
-            items = step.attention_items(ops.DELTA_CHUNK)
-            o = ops.delta_recurrence_chunked(conv, 0, G * d, 2 * G * d, z, self.beta_col, up, self.dt_bias,
-                                             self.A_log, cache.state, self.conv_state, step.slot_id, items, H,
-                                             G, d, dv)
-        else:
-            o = ops.matrix_recurrence("delta", conv, 0, G * d, 2 * G * d, z, self.beta_col, up,
-                                      self.dt_bias, self.A_log, None, cache.state, self.conv_state,
-                                      step.seq_start, step.slot_id, H, G, d, dv)
+        o = by_length(
+            step, lambda short, out: ops.matrix_recurrence(
+                "delta", conv, 0, G * d, 2 * G * d, z, self.beta_col, up, self.dt_bias, self.A_log,
+                None, cache.state, self.conv_state, step.seq_start, step.slot_id, H, G, d, dv,
+                short=short, out=out),
+            lambda items: ops.delta_recurrence_chunked(
+                conv, 0, G * d, 2 * G * d, z, self.beta_col, up, self.dt_bias, self.A_log,
+                cache.state, self.conv_state, step.slot_id, items, H, G, d, dv), self.chunk)
         h = ops.gated_group_norm(o, up, H * d, self.norm_w, dv, self.eps, "sigmoid",
                                  gate_first=False)
         return ops.linear(h, self.w_out, tune=self.runtime.tune)
@@ -312,8 +323,8 @@ class Retention(Mixer):
             self.norm_w = torch.ones((1,), dtype=torch.float32, device=runtime.device)
             self.norm_group = dv
         # long portions are taken in chunks (the step's work items of that size)
-        self.chunked = d <= ops.CHUNKED_MAX_DK and all(x >= 0.0 for x in decay)
-        self.item_granularities = [ops.RETENTION_CHUNK] if self.chunked else []
+        self.chunk = ops.RETENTION_CHUNK if d <= ops.CHUNKED_MAX_DK and all(x >= 0.0 for x in decay) else 0
+        self.item_granularities = [(self.chunk, ops.CHUNKED_FROM)] if self.chunk else []
         ops.check_projection_weight(self.w_in, "retention opening projection")
         ops.check_projection_weight(self.w_out, "retention out_proj")
 
@@ -324,14 +335,13 @@ class Retention(Mixer):
             z, 0, H * d, 2 * H * d, step.positions,
             self.position.inv_freq if self.rotary_dim else None, H, d, dv, self.rotary_dim,
             self.k_scale, self.activation)
-        if self.chunked and ops.in_chunks(step.seq_lens_host):
-            items = step.attention_items(ops.RETENTION_CHUNK)
-            o = ops.fixed_decay_recurrence_chunked(vectors, 0, H * d, 2 * H * d, self.decay,
-                                                   cache.state, 0, step.slot_id, items, H, d, dv)
-        else:
-            o = ops.matrix_recurrence("fixed", vectors, 0, H * d, 2 * H * d, None, 0, self.decay,
-                                      None, None, None, cache.state, 0, step.seq_start,
-                                      step.slot_id, H, H, d, dv)
+        o = by_length(
+            step, lambda short, out: ops.matrix_recurrence(
+                "fixed", vectors, 0, H * d, 2 * H * d, None, 0, self.decay, None, None, None,
+                cache.state, 0, step.seq_start, step.slot_id, H, H, d, dv, short=short, out=out),
+            lambda items: ops.fixed_decay_recurrence_chunked(
+                vectors, 0, H * d, 2 * H * d, self.decay, cache.state, 0, step.slot_id, items, H, d,
+                dv), self.chunk)
         if getattr(step, "taps", None) is not None:
             step.taps["vectors"] = vectors.clone()
             step.taps["o"] = o.clone()

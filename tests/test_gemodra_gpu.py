@@ -678,6 +678,25 @@ def test_latent_prefill_on_whole_tiles(H, R, rotated, page_size):
         assert float((got - want).abs().max()) < 2e-2, nsplit
 
 
+@pytest.mark.parametrize("R,rotated,page_size", [(512, 64, 16), (256, 32, 4), (128, 0, 64), (512, 64, 12)])
+def test_latent_prefill_without_a_page(R, rotated, page_size):
+    """A table entry below zero stands for rows of zeros, never for another request's page."""
+    from zig_ai_amd.kernels import ops
+    H, W, most = 8, R + rotated, ops.LATENT_MFMA_ROWS
+    requests = [(70, 9), (0, 150), (133, 1), (200, 31)]
+    q, plane, table, pos, iseq, irow, icnt, n, scale, sink, _ = _latent_attention_case(
+        torch.bfloat16, H, W, R, requests, page_size, max(1, most // H), seed=W)
+    missing = table.clone()
+    missing[:, ::3] = -1                             # every third page, the first among them
+    plane = torch.cat([plane, torch.zeros_like(plane[:1])])      # a page of zeros at the end
+    zeros = table.clone()
+    zeros[:, ::3] = plane.shape[0] - 1
+    for keys, nsplit in ((0, 1), (64, 4)):
+        got, want = (ops.latent_attention(q, plane, R, t, pos, iseq, irow, icnt, n, scale, sink, keys, nsplit, 4)
+                     for t in (missing, zeros))
+        assert torch.equal(got, want), nsplit
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,N,K,mode", [(3, 24, 16, None), (8, 128, 64, "element"), (5, 40, 32, "head"),
                                         (1, 8, 320, "element"), (40, 72, 8, None)])

@@ -1094,6 +1094,9 @@ struct LpShape {
   static constexpr size_t LDS = (size_t)2 * TILE * 2 + 64 * LP_KT * 2 + 64 * 4 * 4 + (WS - KEPT) * 64 * 32 * 2;
 };
 
+// What a key without a page (an entry below zero) holds; the requests into LDS have no other zeros.
+__device__ __attribute__((aligned(16))) bf16_t lp_no_row[512 + 64];
+
 template <int RT, int DT>
 __global__ void __launch_bounds__(LP_NT)
 latent_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
@@ -1145,7 +1148,8 @@ latent_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
     asm volatile("" : "+v"(lane));                  // (worked out again for each tile: registers)
     const int kp = min(tile0 + wave * 8 + (lane & 7), range_hi);
     const int off = kp & ((1 << page_shift) - 1);
-    const long long at = (long long)max(page, 0) * page_stride + (long long)off * W;
+    const long long at = (long long)(page >= 0 ? plane + (long long)page * page_stride + (long long)off * W
+                                               : (const bf16_t*)lp_no_row);
     long long base[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -1162,7 +1166,7 @@ latent_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
       int piece = (i * 64 + lane - key * NP) ^ key;
       if (WS % 2 && piece >= W / 8) piece = 0;       // room that no fragment reads
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void*)(plane + from + piece * 8),
+          (const __attribute__((address_space(1))) void*)((const bf16_t*)from + piece * 8),
           (__attribute__((address_space(3))) void*)(to + i * 512), 16, 0, 0);
     }
   };

@@ -1010,10 +1010,6 @@ latent_attention_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ 
 #define LP_NT 512
 #define LP_PAIRS 2          // pairs of fragments that a wave takes at once (3: registers run over)
 
-__device__ __forceinline__ unsigned lp_lds(const void* p) {
-  return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) void*)p;
-}
-
 // The waits are written by hand: the compiler would wait for the next tile's requests before
 // any read of LDS.
 __device__ __forceinline__ void lp_meet() {
@@ -1023,16 +1019,8 @@ __device__ __forceinline__ void lp_meet() {
 
 // Fragments 2 * PAIRS from two addresses, 128 bytes from pair to pair.
 template <int PAIRS>
-__device__ __forceinline__ void lp_take_keys(bf16x8_t (&f)[6], unsigned even, unsigned odd) {
-  if constexpr (PAIRS == 3)
-    asm volatile(
-        "ds_read_b128 %0, %6 offset:0\n" "ds_read_b128 %1, %7 offset:0\n"
-        "ds_read_b128 %2, %6 offset:128\n" "ds_read_b128 %3, %7 offset:128\n"
-        "ds_read_b128 %4, %6 offset:256\n" "ds_read_b128 %5, %7 offset:256\n"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5])
-        : "v"(even), "v"(odd)
-        : "memory");
+__device__ __forceinline__ void lp_take_keys(bf16x8_t (&f)[2 * LP_PAIRS], unsigned even, unsigned odd) {
+  static_assert(PAIRS == 1 || PAIRS == LP_PAIRS, "the forms below");
   if constexpr (PAIRS == 2)
     asm volatile(
         "ds_read_b128 %0, %4 offset:0\n" "ds_read_b128 %1, %5 offset:0\n"
@@ -1191,7 +1179,7 @@ latent_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
     for (int ks = 0; ks < KEPT; ++ks) qf[a][ks] = *reinterpret_cast<const bf16x8_t*>(qrow + ks * 32);
     if (KEPT < WS && kt == 0) {
       const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(qrow + KEPT * 32);
-      asm volatile("ds_write_b128 %0, %1" ::"v"(lp_lds(Qs) + (rh * 2 + a) * 1024 + lane * 16), "v"(v) : "memory");
+      asm volatile("ds_write_b128 %0, %1" ::"v"(lds_address(Qs) + (rh * 2 + a) * 1024 + lane * 16), "v"(v) : "memory");
     }
   }
   float m[4], l[2] = {0.f, 0.f};
@@ -1203,7 +1191,7 @@ latent_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
     for (int t = 0; t < OT; ++t) o[a][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  const unsigned ks_at = lp_lds(Ks), ps_at = lp_lds(Ps), xs_at = lp_lds(Xs);
+  const unsigned ks_at = lds_address(Ks), ps_at = lds_address(Ps), xs_at = lds_address(Xs);
   int buffer = 0;
   for (int tile0 = range_lo; tile0 <= range_hi; tile0 += LP_KT, buffer ^= 1) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1222,9 +1210,8 @@ latent_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
     constexpr int PAIRS = (WS + 1) / 2;
 #pragma unroll
     for (int b = 0; b < PAIRS; b += LP_PAIRS) {
-      bf16x8_t kf[6];
+      bf16x8_t kf[2 * LP_PAIRS];
       if (b + LP_PAIRS <= PAIRS) lp_take_keys<LP_PAIRS>(kf, even + b * 128, odd + b * 128);
-      else if (PAIRS - b == 2) lp_take_keys<2>(kf, even + b * 128, odd + b * 128);
       else lp_take_keys<1>(kf, even + b * 128, odd + b * 128);
 #pragma unroll
       for (int i = 0; i < 2 * LP_PAIRS; ++i) {
@@ -1233,7 +1220,7 @@ latent_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
           bf16x8_t qs[2];
           asm volatile("ds_read_b128 %0, %2\n" "ds_read_b128 %1, %2 offset:1024\n" "s_waitcnt lgkmcnt(0)"
                        : "=&v"(qs[0]), "=&v"(qs[1])
-                       : "v"(lp_lds(Qs) + rh * 2048 + lane * 16)
+                       : "v"(lds_address(Qs) + rh * 2048 + lane * 16)
                        : "memory");
           s[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i], qs[0], s[0], 0, 0, 0);
           s[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i], qs[1], s[1], 0, 0, 0);

@@ -21,8 +21,8 @@
 
 #define GG_BK 64
 
-__device__ __forceinline__ unsigned lds_address(const bf16_t* p) {
-  return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) bf16_t*)p;
+__device__ __forceinline__ unsigned lds_address(const void* p) {
+  return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
 // The wait for all but the last n requests to memory.

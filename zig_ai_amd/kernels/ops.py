@@ -2304,12 +2304,15 @@ CHUNKED_MAX_DK = 128           # state rows of a head that the chunks' kernels t
 #   one portion   25 33, 20 23, 36 37   36 43, 29 31, 50 39   47 47, 38 33, 64 42   58 47, 46 33, 78 44
 #   eight         86 64, 23 26, 86 71 125 80, 32 35, 119 78 164 90, 41 37, 153 88 203 156, 50 54, 186 122
 #   beside 512   102 77, 55 36, 111 74 124 77, 63 36, 124 74 145 78, 71 36, 139 75 167 78, 81 36, 153 75
-# The line is the first of these where chunks are clearly ahead in a portion alone.  Beside a long
-# portion they are from some 32 tokens on, and a lower line would gain 10 to 80 us a layer there; it
-# would also have short prompts, which are walked in any case when they come in pieces, depend on
-# their pieces.  Single tokens beside a long portion: 64 of them beside 2,048 241 us, as chunks of
-# their own 444 (delta rule 248 and 491), 30 beside 512 98 and 167 (102 and 185).
+# Constant decays (mostly the second of the three): from 64 on, where a portion alone loses 3 us and
+# one beside a long portion gains 20.  Decays from the token and the delta rule: from 160 on, the first
+# of these lengths at which a portion alone is clearly ahead; beside a long portion they would gain 25
+# to 80 us a layer from 64 on, but in these designs, whose bfloat16 runs magnify a last place most,
+# short prompts come out the same however they are cut.
+# Single tokens beside a long portion: 64 of them beside 2,048 241 us, as chunks of their own 444
+# (delta rule 248 and 491), 30 beside 512 98 and 167 (102 and 185).
 CHUNKED_FROM = 160
+RETENTION_CHUNKED_FROM = 64
 
 
 def _chunk_items(items):
@@ -2359,8 +2362,7 @@ def fixed_decay_recurrence_chunked(vectors: torch.Tensor, q_col: int, k_col: int
                                    slot_id: torch.Tensor, items, heads: int, dk: int,
                                    dv: int) -> torch.Tensor:
     """The fixed-decay walk of ``matrix_recurrence`` for long portions: ``items``
-    (``StepContext.attention_items(RETENTION_CHUNK, CHUNKED_FROM)``: request, first row, rows,
-    number) cut those requests' rows into chunks that are taken side by side as matrix products
+    (``StepContext.attention_items(RETENTION_CHUNK, from)``: request, first row, rows, number) cut those requests' rows into chunks that are taken side by side as matrix products
     (csrc/recurrent_chunks.hip); other requests' rows of the result are not written and their
     states are left alone.  Decays must not be negative.  Same result as the plain walk up to the
     order of 32-bit additions."""

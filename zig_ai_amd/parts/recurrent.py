@@ -43,7 +43,7 @@ side by side are normed together, times a weight ``norm.weight`` of ``num_heads 
 and ``gate`` (``"silu"`` or ``"sigmoid"`` of the gate's projection, applied behind the norm).
 Lightning attention is ``activation="silu"``, ``key_scale=1``, ``output_norm="all"``,
 ``gate="sigmoid"`` and no position encoding.
-A portion of ``ops.CHUNKED_FROM`` tokens or more is taken in chunks, as matrix products
+A portion of ``ops.RETENTION_CHUNKED_FROM`` tokens or more is taken in chunks, as matrix products
 (``ops.fixed_decay_recurrence_chunked``; ``ssd`` and ``gated_delta`` have such forms too): the
 state is linear in what it was before a chunk.
 
@@ -73,14 +73,13 @@ from .base import Mixer, Runtime, StateNeed, TensorRule, lookup, register_mixer
 from .feed_forward import fuse_rows, pad_columns, pad_rows
 
 
-def by_length(step, walk, chunks, size):
-    """The recurrence of a step: portions of ``ops.CHUNKED_FROM`` tokens or more by
-    ``chunks(items)`` with work items of ``size`` rows, shorter ones by ``walk(short, out)``; ``size``
-    0: all of them walked."""
-    short = step.portions_below(ops.CHUNKED_FROM) if size else None
+def by_length(step, walk, chunks, items):
+    """The recurrence of a step.  ``items`` (rows an item, first length): portions of that length or
+    more by ``chunks`` of such work items, shorter ones by ``walk(short, out)``; None: all walked."""
+    short = step.portions_below(items[1]) if items else None
     if short is None or short.requests == step.n_seqs:
         return walk(None, None)
-    out = chunks(step.attention_items(size, ops.CHUNKED_FROM))
+    out = chunks(step.attention_items(*items))
     if short.requests:
         walk(short, out)
     return out
@@ -139,8 +138,8 @@ class StateSpaceDuality(Mixer):
         self.norm_w = tensors["norm.weight"]
         self.conv_state = (self.inner + 2 * G * N) * (L - 1)      # floats before S in a slot
         # long portions are taken in chunks (the step's work items of that size)
-        self.chunk = ops.RETENTION_CHUNK if N <= ops.CHUNKED_MAX_DK else 0
-        self.item_granularities = [(self.chunk, ops.CHUNKED_FROM)] if self.chunk else []
+        self.chunks = (ops.RETENTION_CHUNK, ops.CHUNKED_FROM) if N <= ops.CHUNKED_MAX_DK else None
+        self.item_granularities = [self.chunks] if self.chunks else []
         ops.check_projection_weight(self.w_in, "ssd in_proj")
         ops.check_projection_weight(self.w_out, "ssd out_proj")
 
@@ -157,7 +156,7 @@ class StateSpaceDuality(Mixer):
             lambda items: ops.ssd_recurrence_chunked(
                 conv, inner + G * N, inner, 0, z, 2 * inner + 2 * G * N, self.dt_bias, self.A_log,
                 self.D, cache.state, self.conv_state, step.slot_id, items, self.heads, G, N,
-                self.head_dim), self.chunk)
+                self.head_dim), self.chunks)
         h = ops.gated_group_norm(y, z, 0, self.norm_w, inner // self.norm_groups, self.eps,
                                  "silu", gate_first=True)
         return ops.linear(h, self.w_out, tune=self.runtime.tune)
@@ -232,8 +231,8 @@ class GatedDeltaRule(Mixer):
         self.w_out = ops.projection_weight(tensors["out_proj.weight"])
         self.conv_state = (2 * G * d + H * dv) * (L - 1)
         # long portions are taken in chunks (the step's work items of that size)
-        self.chunk = ops.DELTA_CHUNK if d <= ops.CHUNKED_MAX_DK else 0
-        self.item_granularities = [(self.chunk, ops.CHUNKED_FROM)] if self.chunk else []
+        self.chunks = (ops.DELTA_CHUNK, ops.CHUNKED_FROM) if d <= ops.CHUNKED_MAX_DK else None
+        self.item_granularities = [self.chunks] if self.chunks else []
         for w, what in ((self.w_in, "in"), (self.w_up, "low-rank up"), (self.w_out, "out")):
             ops.check_projection_weight(w, f"gated_delta {what} projection")
 
@@ -251,7 +250,7 @@ class GatedDeltaRule(Mixer):
                 short=short, out=out),
             lambda items: ops.delta_recurrence_chunked(
                 conv, 0, G * d, 2 * G * d, z, self.beta_col, up, self.dt_bias, self.A_log,
-                cache.state, self.conv_state, step.slot_id, items, H, G, d, dv), self.chunk)
+                cache.state, self.conv_state, step.slot_id, items, H, G, d, dv), self.chunks)
         h = ops.gated_group_norm(o, up, H * d, self.norm_w, dv, self.eps, "sigmoid",
                                  gate_first=False)
         return ops.linear(h, self.w_out, tune=self.runtime.tune)
@@ -323,8 +322,9 @@ class Retention(Mixer):
             self.norm_w = torch.ones((1,), dtype=torch.float32, device=runtime.device)
             self.norm_group = dv
         # long portions are taken in chunks (the step's work items of that size)
-        self.chunk = ops.RETENTION_CHUNK if d <= ops.CHUNKED_MAX_DK and all(x >= 0.0 for x in decay) else 0
-        self.item_granularities = [(self.chunk, ops.CHUNKED_FROM)] if self.chunk else []
+        self.chunks = (ops.RETENTION_CHUNK, ops.RETENTION_CHUNKED_FROM) \
+            if d <= ops.CHUNKED_MAX_DK and all(x >= 0.0 for x in decay) else None
+        self.item_granularities = [self.chunks] if self.chunks else []
         ops.check_projection_weight(self.w_in, "retention opening projection")
         ops.check_projection_weight(self.w_out, "retention out_proj")
 
@@ -341,7 +341,7 @@ class Retention(Mixer):
                 cache.state, 0, step.seq_start, step.slot_id, H, H, d, dv, short=short, out=out),
             lambda items: ops.fixed_decay_recurrence_chunked(
                 vectors, 0, H * d, 2 * H * d, self.decay, cache.state, 0, step.slot_id, items, H, d,
-                dv), self.chunk)
+                dv), self.chunks)
         if getattr(step, "taps", None) is not None:
             step.taps["vectors"] = vectors.clone()
             step.taps["o"] = o.clone()

@@ -747,6 +747,32 @@ def test_head_linear_at_the_edges_of_its_tiles(T, H, N, K, mode):
         assert bool((got[:, :, :4] == 7).all()) and bool((got[:, :, -4:] == 7).all())
 
 
+@pytest.mark.parametrize("T", [5, 40])
+def test_products_of_views_that_start_off_16_bytes(T):
+    """Grouped products and heads' own products take views that start anywhere: the same bits."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(T)
+
+    def shifted(t):
+        room = torch.empty(t.numel() + 4, dtype=t.dtype, device=dev)
+        room[4:] = t.reshape(-1)
+        return room[4:].view(t.shape)                # eight bytes behind the allocation's start
+
+    x = torch.randn(T, 3, 72, generator=g).bfloat16().to(dev)
+    w = torch.randn(3, 40, 64, generator=g).bfloat16().to(dev)
+    want = ops.head_linear(x, 8, w)
+    assert torch.equal(ops.head_linear(shifted(x), 8, w), want)
+    assert torch.equal(ops.head_linear(x, 8, shifted(w)), want)
+    rows = torch.randn(T, 72, generator=g).bfloat16().to(dev)
+    experts = torch.randn(4, 48, 72, generator=g).bfloat16().to(dev)
+    chosen = torch.randint(0, 4, (T, 1), generator=g).int().to(dev)
+    lists, counts = ops.expert_lists(None, chosen, T, 4)
+    want = ops.grouped_linear(rows, experts, lists, counts, T, per_token=True)
+    assert torch.equal(ops.grouped_linear(shifted(rows), experts, lists, counts, T, per_token=True), want)
+    assert torch.equal(ops.grouped_linear(rows, shifted(experts), lists, counts, T, per_token=True), want)
+
+
 def test_token_side_kernels():
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")

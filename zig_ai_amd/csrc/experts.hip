@@ -330,7 +330,7 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
   GroupedArgs g{src, W, lists, counts, out, (int)A, n_tokens, top, experts, N, K,
                 src_div, stacked, act, out_scale, row_weight, gate, bound, slope, offset};
   if (w_dtype == 1) {
-    if (src_dtype != 1 || K % 8 != 0) return ZA_ERR_UNSUPPORTED;
+    if (src_dtype != 1 || K % 8 != 0 || ((uintptr_t)src | (uintptr_t)W) % 16 != 0) return ZA_ERR_UNSUPPORTED;
     if (out_dtype != 0 && out_dtype != 1) return ZA_ERR_UNSUPPORTED;
     // Tiles as high as the experts have rows on average, and one step of K under way, or as many
     // as keep memory busy where a launch makes fewer workgroups than the chip has compute units or

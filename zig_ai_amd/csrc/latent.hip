@@ -504,7 +504,8 @@ extern "C" int za_head_linear(const void* x, int x_dtype, int x_ld, int x_col, c
   HeadLinearArgs a{x, W, out, gate, n_tokens, heads, N, K, x_ld, x_col, o_ld, o_col,
                    gate_ld, gate_col, gate_mode};
   if (w_dtype == 1) {
-    if (x_dtype != 1 || K % 8 != 0 || x_ld % 8 != 0 || x_col % 8 != 0) return ZA_ERR_UNSUPPORTED;
+    if (x_dtype != 1 || K % 8 != 0 || x_ld % 8 != 0 || x_col % 8 != 0 || ((uintptr_t)x | (uintptr_t)W) % 16 != 0)
+      return ZA_ERR_UNSUPPORTED;
     if (out_dtype != 0 && out_dtype != 1) return ZA_ERR_UNSUPPORTED;
     if (n_tokens <= 16) {
       const bool split = K >= HL_SPLIT_MIN_K;

@@ -305,6 +305,12 @@ def _need(t: torch.Tensor, name: str, dtype=None, shape: Optional[Tuple[int, ...
         raise KernelError(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
 
 
+def _on_16_bytes(t: torch.Tensor) -> torch.Tensor:
+    """``t``, or a copy of it that starts on 16 bytes, for the kernels that request their operands
+    straight into LDS in pieces of that size (a tensor of its own always does; a view may not)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 # --------------------------------------------------------------------- norms
 def add_rmsnorm(residual: Optional[torch.Tensor], delta: Optional[torch.Tensor],
                 weight: torch.Tensor, eps: float, out_dtype: torch.dtype,
@@ -2668,6 +2674,8 @@ def grouped_linear(src: torch.Tensor, weights: torch.Tensor, lists: torch.Tensor
     _need(src, "src", (torch.float32, torch.bfloat16), (n_tokens if per_token else n_tokens * top, K))
     if weights.dtype == torch.bfloat16 and (src.dtype != torch.bfloat16 or K % 8):
         raise KernelError("bfloat16 expert weights need bfloat16 rows and K a multiple of 8")
+    if weights.dtype == torch.bfloat16:
+        src, weights = _on_16_bytes(src), _on_16_bytes(weights)
     out_dtype = torch.float32 if stacked else (out_dtype or src.dtype)
     shape = (top, n_tokens, N) if stacked else (n_tokens * top, N)
     if row_weight is not None:
@@ -2917,6 +2925,8 @@ def head_linear(x: torch.Tensor, x_col: int, weight: torch.Tensor, out: Optional
     if weight.dtype == torch.bfloat16 and (x.dtype != torch.bfloat16 or K % 8 or x_ld % 8 or x_col % 8):
         raise KernelError("bfloat16 head weights need bfloat16 rows whose pieces start on 16-byte "
                           "boundaries; keep the weight in 32-bit otherwise")
+    if weight.dtype == torch.bfloat16:
+        x, weight = _on_16_bytes(x), _on_16_bytes(weight)
     if gate_mode not in HEAD_GATES:
         raise KernelError(f"gate_mode must be None, head or element, got {gate_mode!r}")
     if out is None:

@@ -120,6 +120,7 @@ def test_where_the_tiles_for_17_to_64_rows_are_taken():
     for M in (17, 64):
         assert ops.tiles_take(M, 2048, 8192, 8) and ops.tiles_take(M, 512, 4096, 8)
         assert not ops.tiles_take(M, 200, 4096, 8)          # 32 workgroups
+        assert not ops.tiles_take(M, 512, 2048, 4)          # as many
         assert ops.tiles_take(M, 65536, 2048, 1) and not ops.tiles_take(M, 6144, 2048, 1)
         assert not ops.tiles_take(M, 2048, 1000, 4)         # ranges that are no steps of 64
         assert ops.tiles_take_gated(M, 8192, 2048) and ops.tiles_take_gated(M, 4608, 1024)

@@ -560,6 +560,34 @@ def test_products_of_17_to_64_rows_in_tiles(M, N, K, ranges):
         assert rel_err(out, want) < BF16_TOL
 
 
+@pytest.mark.parametrize("M", [17, 64])
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+def test_gated_product_of_17_to_64_rows_and_operands_it_leaves(M, activation):
+    """The gated product of a feed-forward; operands that start off 16 bytes are not taken, by it nor
+    by a product in ranges, which then goes its other way."""
+    o = ops()
+    I, K = 4096, 512
+    x, w = rand((M, K), torch.bfloat16, 62), rand((2 * I, K), torch.bfloat16, 63)
+    g, u = (x.double() @ v.double().T for v in (w[:I], w[I:]))
+    want = g * torch.sigmoid(g) * u if activation == "silu" else \
+        0.5 * g * (1 + torch.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3))) * u
+
+    def shifted(t):
+        room = torch.empty(t.numel() + 4, dtype=t.dtype, device=dev())
+        room[4:] = t.reshape(-1)
+        return room[4:].view(t.shape)
+
+    assert rel_err(o.linear_gated_tiles(x.to(dev()), w.to(dev()), activation), want) < BF16_TOL
+    assert o.linear_gated_tiles(shifted(x), w.to(dev()), activation) is None
+    assert o.linear_gated_tiles(x.to(dev()), shifted(w), activation) is None
+    stack = torch.empty((4, M, 2 * I), dtype=torch.float32, device=dev())
+    assert not o._tiles_product(shifted(x), w.to(dev()), stack, 4)
+    for bad in ((16, I, K), (65, I, K), (M, 2048, K)):
+        with pytest.raises(o.KernelError):
+            o.linear_gated_tiles(rand((bad[0], bad[2]), torch.bfloat16, 64).to(dev()),
+                                 rand((2 * bad[1], bad[2]), torch.bfloat16, 65).to(dev()), activation)
+
+
 def test_rows64_rows_do_not_depend_on_the_batch():
     """A row's result is a function of that row: the same bits whichever rows stand beside
     it and wherever it stands (the sums over K run in one order for every row)."""

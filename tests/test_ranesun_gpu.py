@@ -617,17 +617,17 @@ def test_gate_in_the_product_of_a_decode_batch(M, K, I):
         assert float((got - want).abs().max()) < 1e-2 * float(want.abs().max()), act
 
 
-@pytest.mark.parametrize("H,d,dv", [(2, 16, 8), (3, 64, 128), (1, 128, 40)])
+@pytest.mark.parametrize("H,d,dv", [(2, 16, 8), (3, 64, 128), (1, 128, 40), (5, 64, 24)])
 def test_retention_in_chunks_against_the_plain_walk(H, d, dv):
     """Long portions walked as chunks side by side: against float64, in two steps so that the
     second starts from carried states, with portions of exactly one chunk, one more and one
-    fewer, and a decay of one and of a half."""
+    fewer, and a decay of one, of a half, of zero and of nearly zero (in 32-bit)."""
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")
     gen = torch.Generator().manual_seed(d + dv)
     C = ops.RETENTION_CHUNK
     steps = [[2 * C + 70, 1, C, C + 1], [C - 1, 3 * C, 5, 1]]
-    decay = torch.tensor(([1.0, 0.5, 0.99609375] * H)[:H])
+    decay = torch.tensor(([1.0, 0.5, 0.99609375, 0.0, 1e-38] * H)[:H])
     mem, state = _slots(6, 7 + H * d * dv, dev)
     slots = [4, 0, 5, 2]
     S64 = [torch.zeros(H, d, dv, dtype=torch.float64) for _ in slots]

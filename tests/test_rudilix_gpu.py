@@ -531,11 +531,15 @@ def _chunk_items(lengths, size, dev):
 
 
 @pytest.mark.parametrize("H,G,d,dv,strong", [(2, 1, 16, 8, False), (3, 3, 40, 72, True), (2, 2, 128, 128, False),
-                                             (4, 2, 64, 200, True), (1, 1, 31, 17, False)])
-def test_delta_recurrence_in_chunks(H, G, d, dv, strong):
+                                             (4, 2, 64, 200, True), (1, 1, 31, 17, False), (2, 1, 64, 64, True),
+                                             (2, 2, 32, 16, False)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_delta_recurrence_in_chunks(dtype, H, G, d, dv, strong):
     """Portions taken in chunks of 32 as matrix products: against float64, in two steps so that
     the second starts from carried states, with portions of exactly a chunk, one token more and
-    fewer, half a chunk and one token; with decays down to zero.  (Bound as for the walk.)"""
+    fewer, half a chunk and one token; with decays down to zero; raw strengths and decays of either
+    storage type; widths that fill the tiles of 32, 64 and 128 and ones that do not.  (Bound as for
+    the walk.)"""
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")
     gen = torch.Generator().manual_seed(d + dv)
@@ -549,8 +553,8 @@ def test_delta_recurrence_in_chunks(H, G, d, dv, strong):
     for lengths in steps:
         T = sum(lengths)
         conv = torch.randn(T, 2 * G * d + H * dv + 3, generator=gen)
-        proj = torch.randn(T, H + 5, generator=gen)
-        raw = torch.randn(T, H * d + 9, generator=gen) * (8.0 if strong else 1.0)
+        proj = torch.randn(T, H + 5, generator=gen).to(dtype)
+        raw = (torch.randn(T, H * d + 9, generator=gen) * (8.0 if strong else 1.0)).to(dtype)
         _, start, slot_id = _step_arrays(lengths, slots, dev)
         out = ops.delta_recurrence_chunked(conv.to(dev), 3, 3 + G * d, 3 + 2 * G * d, proj.to(dev), 5, raw.to(dev),
                                            dt_bias.to(dev), A_log.to(dev), state, 12, slot_id,
@@ -580,8 +584,10 @@ def test_delta_recurrence_in_chunks(H, G, d, dv, strong):
     assert float(state[:, :12].abs().max()) == 0.0 and float(state[2].abs().max()) == 0.0
 
 
-@pytest.mark.parametrize("H,G,N,P,strong", [(4, 2, 24, 16, True), (3, 1, 128, 64, False), (2, 2, 33, 130, False)])
-def test_ssd_recurrence_in_chunks(H, G, N, P, strong):
+@pytest.mark.parametrize("H,G,N,P,strong", [(4, 2, 24, 16, True), (3, 1, 128, 64, False), (2, 2, 33, 130, False),
+                                            (2, 1, 64, 128, True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_ssd_recurrence_in_chunks(dtype, H, G, N, P, strong):
     """As above for a decay a head and token, in chunks of 128."""
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")
@@ -596,7 +602,7 @@ def test_ssd_recurrence_in_chunks(H, G, N, P, strong):
     for lengths in steps:
         T = sum(lengths)
         conv = torch.randn(T, H * P + 2 * G * N, generator=gen)
-        proj = (torch.randn(T, 4 + H, generator=gen) * (6.0 if strong else 1.0)).to(torch.bfloat16)
+        proj = (torch.randn(T, 4 + H, generator=gen) * (6.0 if strong else 1.0)).to(dtype)
         _, start, slot_id = _step_arrays(lengths, slots, dev)
         out = ops.ssd_recurrence_chunked(conv.to(dev), H * P + G * N, H * P, 0, proj.to(dev), 4, dt_bias.to(dev),
                                          A_log.to(dev), D.to(dev), state, 0, slot_id,

@@ -36,10 +36,10 @@
 
 // lists: int [E][A]; counts: int [E].  `ids` names the table's row for each token (null:
 // the token's own index); an id outside [0, rows) names no expert.
-// A thread looks at neighbouring assignments, twice: once to count its own, and, when the
-// workgroup has added up the counts, to write them where they belong; EL_KEEP of them stay
-// known as bits in between.  (A walk of 256 assignments at a time with a barrier each took
-// 18.4 us for 7,108 assignments of 32 experts, all of it waiting; see the launcher.)
+// A workgroup an expert, which reads all assignments once: a thread takes up to EL_KEEP neighbouring
+// ones, keeps as bits which of them name the expert, and writes those where they belong when the
+// workgroup has added up the counts.  (A walk of 256 assignments at a time with a barrier each took
+// 18.4 us for 7,108 assignments of 32 experts, all of it waiting.)
 #define EL_KEEP 32
 __global__ void __launch_bounds__(1024)
 expert_lists_kernel(const int* __restrict__ ids, const int* __restrict__ table, int rows, int T,
@@ -334,16 +334,19 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     if (out_dtype != 0 && out_dtype != 1) return ZA_ERR_UNSUPPORTED;
     // Tiles as high as the experts have rows on average, and one step of K under way, or as many
     // as keep memory busy where a launch makes fewer workgroups than the chip has compute units or
-    // a decode batch reads little else than weights.  Measured (us, gate|up of 32 experts of 1,024
-    // over 2,048 and their down product, 4 a token; the kernels before these: tiles of 128 through
-    // registers from 128 rows an expert on, 64 and 16 rows straight from memory below):
-    //   tokens        8           64         260         400         517        1777
-    //   before     44 + 25    153 + 79   173 + 90               220 + 115   135 + 93
-    //   32 x 64    31 + 17     40 + 23   (58 + 32 at 32 x 128)
-    //   64 x 128               38 + 21    43 + 24    51 + 29     61 + 35    120 + 61
-    //  128 x 128                          45 + 25    48 + 27     48 + 29    101 + 50 (600 TFLOP/s)
-    // 8 experts of 4,096, 2 a token: down 46 -> 22 at 20 tokens, 212 -> 46 at 500 (two steps under way; 57
-    // with one).
+    // a decode batch reads little else than weights.  Measured with the weights of six layers in
+    // turn, so that they come from memory as in a step (us, gate|up of 32 experts of 1,024 over 2,048
+    // and their down product, 4 a token, evenly spread; the kernels before these: tiles of 128
+    // through registers from 128 rows an expert on, 64 and 16 rows straight from memory below):
+    //   tokens            8          64         260         400         517        1777
+    //   before          51 + 25   167 + 85    184 + 96   226 + 118   229 + 123   140 + 90
+    //    32 x  64       39 + 18    60 + 30     64 + 34    72 + 42     80 + 48    180 + 108
+    //    64 x 128       43 + 20    64 + 26     66 + 28    66 + 30     80 + 43    122 + 78
+    //   128 x 128       46 + 23    67 + 30     71 + 32    73 + 34     74 + 35    105 + 61
+    //   the same, two steps under way                     80 + 37     81 + 38    125 + 76
+    // (1,777 tokens, the fullest expert with 664 instead of 249: 131 + 77.  Weights left in the last
+    // level's cache by the launch before gain a tenth to a third on these.)  8 experts of 4,096, 2 a
+    // token: down 47 -> 32 at 20 tokens, 220 -> 52 at 500 (two steps under way; 73 with one).
     const int BM = A >= 40LL * experts ? 128 : A >= 24LL * experts ? 64 : 32, BN = BM == 32 ? 64 : 128;
     const int columns = gate ? BN / 2 : BN;
     const long long rows = (A + BM - 1) / BM + experts, blocks = (rows + 7) / 8 * 8 * ((N + columns - 1) / columns);

@@ -1,6 +1,5 @@
 // The dense projections of gemm.hip in 32-bit throughout (weights, sums; activations of either
-// type): kernels of gemm_f32.h.  A source of its own: with these kernels before them in one code
-// object the decode batches' kernels, unchanged, took half a percent longer.
+// type): kernels of gemm_f32.h.
 #include "common.h"
 #include "gemm_f32.h"
 

@@ -129,11 +129,12 @@ add_rmsnorm_kernel(float* __restrict__ residual, const TD* __restrict__ delta,
 }
 
 // Rows of at most 256 * 4 * VPT elements with width % 4 == 0: the row stays in
-// registers between the sum of squares and the scaling, one pass over memory, everything (the
-// weight too) requested before the first value is waited for: a thread beyond the row loads the
-// row's last four elements, so no load stands behind a condition (the weight after the sum of
-// squares and a vector after the other: 64 rows of 2,048 with a stack of eight partial sums 5.5 us,
-// now 4.4, with a bfloat16 delta 3.5 and 3.1).
+// registers between the sum of squares and the scaling, one pass over memory, with stream, delta
+// and weight requested before the first value is waited for: a thread beyond the row loads the
+// row's last four elements, so none of these stands behind a condition on the lane (partial sums
+// are counted, the same for all; a LayerNorm's bias is read behind the sums).  (The weight after the
+// sum of squares and a vector after the other: 64 rows of 2,048 with a stack of eight partial sums 5.5 us,
+// now 4.4, with a bfloat16 delta 3.5 and 3.1.)
 template <typename TD, typename TO, int VPT, bool STACK>
 __global__ void __launch_bounds__(256)
 add_rmsnorm_regs_kernel(float* __restrict__ residual, const TD* __restrict__ delta,

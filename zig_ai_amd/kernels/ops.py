@@ -787,9 +787,10 @@ def accumulate_plan(M: int, N: int, K: int, normed: bool) -> int:
 
 # Where a step of 17 to 64 rows takes the kernel of csrc/gemm_tiles.hip, by measurement (one MI355X,
 # replayed from graphs, weights from memory, against the library's product): where K comes in
-# ranges (2048 x 8192 at 64 rows 9.8 us against 13.8, 512 x 2048 3.9 against 4.6; products with
-# still fewer outputs, of which no step is made, stay with the library), and without ranges from as
-# many workgroups on as the chip has compute units (65536 x 2048 in 32-bit at 64 rows 64 us against
+# ranges that make 64 workgroups (2048 x 8192 at 64 rows 9.8 us against 13.8; 512 x 2048, whose 4
+# ranges make 32, would take 3.9 against 4.6, but products that small, of which no step is made, stay
+# with the library and, where it has no algorithm, with the kernels behind it), and without ranges
+# from as many workgroups on as the chip has compute units (65536 x 2048 in 32-bit at 64 rows 64 us against
 # 71); with fewer the library stays (6144 x 2048, 96 workgroups, 11.5 us at 32 rows against 10.2).
 # With the unit of a gated feed-forward from half as many on, since the unit's own kernel goes with
 # it (2 x 8192 x 2048 at 20 and 64 rows 17.2 and 18.9 us against 20.2 and 21.1, 2 x 4608 x 1024,

@@ -751,6 +751,26 @@ def test_a_portion_takes_its_form_by_its_own_length(kind):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("kind", ["ssd", "delta"])
+def test_recorded_steps_with_both_forms(kind):
+    """A step of one token beside a portion in chunks, recorded and replayed with other requests: the
+    bits of the same steps run as they are."""
+    from zig_ai_amd.engine import ModelRunner
+    from zig_ai_amd.kernels import ops
+    cfg = ALONE[kind]
+    model, _ = build(cfg, seed=6)
+    n, rounds = ops.CHUNKED_FROM + 5, 5
+    prompts = [ru.tokens(3 + rounds, cfg["vocab"], 1)] + [ru.tokens(n, cfg["vocab"], 2 + i) for i in range(rounds)]
+    schedule = [([(0, 0, 3)], [])] + [([(0, 3 + i, 4 + i), (1 + i, 0, n)], [1 + i] + ([0] if i == rounds - 1 else []))
+                                      for i in range(rounds)]
+    recorded, plain_run = (ModelRunner(model, page_size=4, num_pages=n, num_slots=3, use_graphs=graphs,
+                                       portion_graphs=graphs) for graphs in (True, False))
+    got, want = (eu.run_schedule(r, prompts, schedule) for r in (recorded, plain_run))
+    assert recorded.graphs.portion_replays >= rounds - 2
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("form", ["ssd", "delta", "fixed"])
 def test_the_walk_of_short_portions_alone(form):
     """With a limit the walk takes the shorter portions, to the bit as in a step of their own, and

@@ -1705,3 +1705,45 @@ def test_grouped_products_at_the_edges_of_their_tiles(dtype, E, top, N, K, T):
                              out_dtype=torch.float32)
     whole = o.grouped_linear(x.to(dev()), w.to(dev()), lists, counts, T, per_token=True, out_dtype=torch.float32)
     assert torch.equal(alone, whole[:top])
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320])
+@pytest.mark.parametrize("columns,top", [(1700, 1), (3300, 1), (3304, 2)])
+def test_grouped_products_in_wide_tiles(K, columns, top):
+    """Steps of many rows, in tiles of 256 or (few outputs) 128 assignments: counts around the tiles'
+    edges and an empty expert, one to five steps of K, outputs off multiples of a tile; the same bits
+    as a token on its own has, which takes the low tiles."""
+    o = ops()
+    want = [1, 127, 128, 129, 255, 256, 257, 0, 384, 385, 513]
+    E = len(want) + 1
+    want.append(top - sum(want) % top)               # (a whole number of tokens)
+    A = sum(want)
+    gen = torch.Generator().manual_seed(K + columns)
+    chosen = torch.cat([torch.full((n,), e) for e, n in enumerate(want)])
+    chosen = chosen[torch.randperm(A, generator=gen)].int().view(-1, top).contiguous()
+    T = chosen.shape[0]
+    lists, counts = o.expert_lists(None, chosen.to(dev()), T, E)
+    assert counts.tolist() == want
+    x, w = rand((T, K), torch.bfloat16, 80), rand((E, columns, K), torch.bfloat16, 81, K ** -0.5)
+    weight = rand((T, top), torch.float32, 82)
+    which, rows = chosen.view(-1).long(), x.double().repeat_interleave(top, 0)
+    full = torch.empty((A, columns), dtype=torch.double)
+    for e in range(E):
+        full[which == e] = rows[which == e] @ w[e].double().T
+    xd, wd = x.to(dev()), w.to(dev())
+    got = o.grouped_linear(xd, wd, lists, counts, T, per_token=True, out_dtype=torch.float32)
+    assert rel_err(got, full) < F32_TOL
+    planes = o.grouped_linear(rows.bfloat16().to(dev()), wd, lists, counts, T, per_token=False, stacked=True,
+                              row_weight=weight.to(dev()))
+    scaled = (full * weight.double().view(-1, 1)).view(T, top, columns).transpose(0, 1)
+    assert rel_err(planes, scaled) < F32_TOL
+    unit = torch.nn.functional.silu(full[:, :columns // 2]) * full[:, columns // 2:]
+    gated = o.grouped_linear(xd, wd, lists, counts, T, per_token=True, out_dtype=torch.bfloat16, gate="silu")
+    assert rel_err(gated, unit) < tol_of(torch.bfloat16)
+    for t in (0, T // 2, T - 1):
+        l1, c1 = o.expert_lists(None, chosen[t:t + 1].contiguous().to(dev()), 1, E)
+        one = dict(lists=l1, counts=c1, n_tokens=1, per_token=True)
+        mine = slice(t * top, (t + 1) * top)
+        assert torch.equal(o.grouped_linear(xd[t:t + 1].contiguous(), wd, out_dtype=torch.float32, **one), got[mine])
+        assert torch.equal(o.grouped_linear(xd[t:t + 1].contiguous(), wd, out_dtype=torch.bfloat16, gate="silu",
+                                            **one), gated[mine])

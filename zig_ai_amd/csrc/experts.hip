@@ -28,9 +28,12 @@
 //    does not depend on which other tokens share its expert or its tile.
 //      bfloat16: matrix cores (v_mfma_f32_16x16x32_bf16), tiles through LDS.
 //      32-bit: tiles of 32 x 64 on the matrix cores' 32-bit instruction (gemm_f32.h).
+#include <type_traits>
+
 #include "common.h"
 #include "gemm_f32.h"
 #include "tiles_bf16.h"
+#include "tiles_wide.h"
 
 #define EX_MAX_EXPERTS 1024
 
@@ -180,6 +183,56 @@ __device__ __forceinline__ size_t dst_row(const GroupedArgs& g, int a) {
   return g.stacked ? (size_t)(a % g.top) * g.T + a / g.top : (size_t)a;
 }
 
+// A wave's sums, acc[i][j][r] of assignment m + 16 i + lane % 16 of the expert's list and weight row
+// wn + 16 j + lane / 16 * 4 + r of the tile that begins at output n0, on their way out.  GATED: the
+// tile's weight rows are gate and up rows in turn, 16 each.
+template <typename TO, bool GATED, int TM, int TN>
+__device__ __forceinline__ void grouped_store(const GroupedArgs& g, const int* __restrict__ mine, int count,
+                                              int m, int n0, int wn, int lane, const f32x4_t (&acc)[TM][TN]) {
+  const int r16 = lane & 15, kq = lane >> 4;
+  TO* out = (TO*)g.out;
+  const int N = g.N;
+  const bool wide = N % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & (4 * sizeof(TO) - 1)) == 0;
+  auto put = [&](TO* to, int n, const f32x4_t& v) {      // outputs n .. n + 3 of one row
+    if (wide) {
+      if (n >= N) return;
+      if constexpr (sizeof(TO) == 4) {
+        *reinterpret_cast<f32x4_t*>(to + n) = v;
+      } else {
+        *reinterpret_cast<bf16x4_t*>(to + n) = bf16x4_t{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (n + r < N) to[n + r] = from_f32<TO>(v[r]);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int row = m + i * 16 + r16;
+    if (row >= count) continue;
+    TO* to = out + dst_row(g, mine[row]) * N;
+    const float w = g.row_weight ? g.row_weight[mine[row]] : 1.0f;
+    if constexpr (GATED) {
+#pragma unroll
+      for (int j = 0; j < TN; j += 2) {
+        f32x4_t v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = expert_unit(g, acc[i][j][r], acc[i][j + 1][r], w);
+        put(to, n0 + (wn >> 1) + (j / 2) * 16 + kq * 4, v);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        f32x4_t v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = expert_act(acc[i][j][r], g.act) * g.out_scale * w;
+        put(to, n0 + wn + j * 16 + kq * 4, v);
+      }
+    }
+  }
+}
+
 // Tiles of BM assignments x BN weight rows (tiles_bf16.h).
 // GATED: a tile is BN / 2 outputs; its weight rows are gate and up rows in turn, 16 each.
 template <typename TO, bool GATED, int BM, int BN, int NS>
@@ -223,47 +276,111 @@ grouped_gemm_bf16_tiled_kernel(GroupedArgs g) {
   }
   f32x4_t acc[TM][TN];
   Tiles::run(As, Ws, wave, lane, K, arow, wrow, acc);
-  const int r16 = lane & 15, kq = lane >> 4;
-  TO* out = (TO*)g.out;
-  const bool wide = N % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & (4 * sizeof(TO) - 1)) == 0;
-  auto put = [&](TO* to, int n, const f32x4_t& v) {      // outputs n .. n + 3 of one row
-    if (wide) {
-      if (n >= N) return;
-      if constexpr (sizeof(TO) == 4) {
-        *reinterpret_cast<f32x4_t*>(to + n) = v;
-      } else {
-        *reinterpret_cast<bf16x4_t*>(to + n) = bf16x4_t{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
-      }
-    } else {
+  grouped_store<TO, GATED>(g, mine, count, tile * BM + wm, n0, wn, lane, acc);
+}
+
+// The tile that workgroup `b` of a list of tiles serves, which holds an expert's full tiles (of more than
+// 128 assignments) or, LAST, the one of what is left of at most 128; HIGH 128: all tiles are such.
+// Returns the number of tiles.
+template <int HIGH, bool LAST>
+__device__ __forceinline__ int wide_tiles(int c) {
+  if (HIGH == 128) return LAST ? (c + 127) / 128 : 0;
+  const int full = (c + 127) / 256;
+  return LAST ? (c > full * 256 ? 1 : 0) : full;
+}
+
+template <int HIGH, bool LAST>
+__device__ __forceinline__ int wide_count(const int* __restrict__ counts, int E) {
+  int tiles = 0;
+  for (int e = threadIdx.x & 63; e < E; e += 64) tiles += wide_tiles<HIGH, LAST>(counts[e]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n + r < N) to[n + r] = from_f32<TO>(v[r]);
+  for (int o = ZA_WAVE / 2; o > 0; o >>= 1) tiles += __shfl_xor(tiles, o, ZA_WAVE);
+  return __builtin_amdgcn_readfirstlane(tiles);
+}
+
+// Tile `b` of those: its expert, the first of its assignments and the expert's count.
+template <int HIGH, bool LAST>
+__device__ __forceinline__ void wide_find(const int* __restrict__ counts, int E, int b, int* e_out, int* m0_out,
+                                          int* count_out) {
+  const int lane = threadIdx.x & 63;
+  int first = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int c = e0 + lane < E ? counts[e0 + lane] : 0;
+    const int tiles = wide_tiles<HIGH, LAST>(c);
+    int end = tiles;
+#pragma unroll
+    for (int o = 1; o < ZA_WAVE; o <<= 1) {
+      const int v = __shfl_up(end, o, ZA_WAVE);
+      if (lane >= o) end += v;
     }
-  };
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int row = tile * BM + wm + i * 16 + r16;
-    if (row >= count) continue;
-    TO* to = out + dst_row(g, mine[row]) * N;
-    const float w = g.row_weight ? g.row_weight[mine[row]] : 1.0f;
-    if constexpr (GATED) {
-#pragma unroll
-      for (int j = 0; j < TN; j += 2) {
-        f32x4_t v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = expert_unit(g, acc[i][j][r], acc[i][j + 1][r], w);
-        put(to, n0 + (wn >> 1) + (j / 2) * 16 + kq * 4, v);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        f32x4_t v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = expert_act(acc[i][j][r], g.act) * g.out_scale * w;
-        put(to, n0 + wn + j * 16 + kq * 4, v);
-      }
+    const unsigned long long past = __ballot(b < first + end);
+    if (past) {
+      const int at = __ffsll(past) - 1, n = __builtin_amdgcn_readlane(c, at);
+      const int tile = b - first - (__builtin_amdgcn_readlane(end, at) - __builtin_amdgcn_readlane(tiles, at));
+      *e_out = __builtin_amdgcn_readfirstlane(e0 + at);
+      *count_out = n;
+      *m0_out = HIGH == 256 && LAST ? (n + 127) / 256 * 256 : tile * HIGH;
+      return;
     }
+    first += __builtin_amdgcn_readlane(end, 63);
   }
+}
+
+// Tiles of 256 x 256 or, for what is left of an expert's rows at its end, 128 x 256 (tiles_wide.h);
+// HIGH 128: of 128 x 256 only.  GATED as above.
+template <typename TO, bool GATED, int HIGH>
+__global__ void __launch_bounds__(512, 2)
+grouped_gemm_bf16_wide_kernel(GroupedArgs g) {
+  __shared__ __attribute__((aligned(16))) bf16_t lds[GW_LDS];
+  // Workgroups are dealt to the eight dies in turn: a die takes an eighth of the full tiles, an expert's
+  // stretches of outputs side by side, and then an eighth of the others, which take half as long and
+  // fill the ends.
+  const int columns = (g.N + (GATED ? 127 : 255)) / (GATED ? 128 : 256), die = blockIdx.x & 7;
+  const int full = HIGH == 256 ? wide_count<HIGH, false>(g.counts, g.E) * columns : 0;
+  const int rest = wide_count<HIGH, true>(g.counts, g.E) * columns;
+  const int full_each = (full + 7) >> 3, rest_each = (rest + 7) >> 3;
+  int at = blockIdx.x >> 3, index;
+  const bool last = at >= full_each;
+  if (last) {
+    at -= full_each;
+    index = die * rest_each + at;
+    if (at >= rest_each || index >= rest) return;
+  } else {
+    index = die * full_each + at;
+    if (index >= full) return;
+  }
+  int e, m0, count;
+  if (last) wide_find<HIGH, true>(g.counts, g.E, index / columns, &e, &m0, &count);
+  else wide_find<HIGH, false>(g.counts, g.E, index / columns, &e, &m0, &count);
+  const int n0 = (index % columns) * (GATED ? 128 : 256);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int* mine = g.lists + (size_t)e * g.A;
+  const int K = g.K, N = g.N;
+  const bf16_t* wbase = (const bf16_t*)g.W + (size_t)e * (GATED ? 2 * N : N) * K;
+  auto serve = [&](auto tm) {
+    constexpr int TM = decltype(tm)::value;
+    using Tiles = TilesWide<TM>;
+    const int lrow = wave * 8 + (lane >> 3), piece = ((lane & 7) ^ (lane >> 3)) * 8;
+    const bf16_t* arow[Tiles::LA];
+    const bf16_t* wrow[Tiles::LW];
+#pragma unroll
+    for (int i = 0; i < Tiles::LA; ++i) {
+      const int r = min(m0 + lrow + 64 * i, count - 1);      // (rows beyond are not stored)
+      arow[i] = (const bf16_t*)g.src + (size_t)(mine[r] / g.src_div) * K + piece;
+    }
+#pragma unroll
+    for (int i = 0; i < Tiles::LW; ++i) {
+      const int tr = lrow + 64 * i;
+      const int n = min(n0 + (GATED ? (tr >> 5) * 16 + (tr & 15) : tr), N - 1);
+      wrow[i] = wbase + (size_t)(n + (GATED && (tr & 16) ? N : 0)) * K + piece;
+    }
+    f32x4_t acc[TM][Tiles::TN];
+    Tiles::run(lds, wave, lane, K, arow, wrow, acc);
+    grouped_store<TO, GATED>(g, mine, count, m0 + (wave >> 2) * 16 * TM, n0, (wave & 3) * 64, lane, acc);
+  };
+  if (last) serve(std::integral_constant<int, 4>{});
+  else if constexpr (HIGH == 256) serve(std::integral_constant<int, 8>{});
 }
 
 // 32-bit weights (src of either type): tiles of 32 assignments x 64 weight rows, the sums in the
@@ -347,6 +464,37 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     // (1,777 tokens, the fullest expert with 664 instead of 249: 131 + 77.  Weights left in the last
     // level's cache by the launch before gain a tenth to a third on these.)  8 experts of 4,096, 2 a
     // token: down 47 -> 32 at 20 tokens, 220 -> 52 at 500 (two steps under way; 73 with one).
+    // Many rows an expert and K in whole steps of 64: the wide tiles, 256 assignments high where some 176
+    // of them or more come about, else 128 where some 150 do (half an expert's tile more than its rows
+    // make on average; below that compute units idle).  Measured as above, up | down (us): 32 experts of
+    // 1,024 over 2,048, 4 a token, unevenly taken as a trained router does it, 1,777 tokens 141 | 78 ->
+    // 110 | 66, 1,029 tokens 102 | 56 -> 83 | 42, 862 tokens 101 | 54 -> 79 | 39, 4,096 tokens 231 | 135
+    // -> 182 | 107; at 517 tokens (65 rows an expert) 73 | 36 against 84 | 38.  8 experts of 4,096, 2 a
+    // token, 1,900 tokens: up 99 -> 64 (128 high 85), down, 128 high for want of tiles, 92 -> 75 (256
+    // high 95); 500 tokens: up, 128 high, 56 -> 43, down stays (54 against 66).  The sums are the same
+    // to the last bit.
+    if (K % GG_BK == 0 && A >= 80LL * experts) {
+      const long long columns = (N + (gate ? 127 : 255)) / (gate ? 128 : 256);
+      const int high = (A / 256 + experts / 2) * columns >= 176 ? 256
+                       : (A / 128 + experts / 2) * columns >= 150 ? 128 : 0;
+      // (an expert's full tiles and its last one, each kind an eighth a die)
+      const long long tiles = (A + high - 1) / max(high, 1) + experts;
+      const long long blocks = (tiles * columns + 7) / 8 * 8 + 8;
+      if (high && blocks > 0x7fffffffLL) return ZA_ERR_ARG;
+#define ZA_GW(TO, GATED)                                                                                   \
+  {                                                                                                        \
+    if (high == 256)                                                                                       \
+      hipLaunchKernelGGL((grouped_gemm_bf16_wide_kernel<TO, GATED, 256>), dim3((unsigned)blocks), dim3(512), 0, stream, g); \
+    else                                                                                                   \
+      hipLaunchKernelGGL((grouped_gemm_bf16_wide_kernel<TO, GATED, 128>), dim3((unsigned)blocks), dim3(512), 0, stream, g); \
+    return za_launch_status();                                                                             \
+  }
+      if (high) {
+        if (out_dtype == 0) { if (gate) ZA_GW(float, true) else ZA_GW(float, false) }
+        else { if (gate) ZA_GW(bf16_t, true) else ZA_GW(bf16_t, false) }
+      }
+#undef ZA_GW
+    }
     const int BM = A >= 40LL * experts ? 128 : A >= 24LL * experts ? 64 : 32, BN = BM == 32 ? 64 : 128;
     const int columns = gate ? BN / 2 : BN;
     const long long rows = (A + BM - 1) / BM + experts, blocks = (rows + 7) / 8 * 8 * ((N + columns - 1) / columns);

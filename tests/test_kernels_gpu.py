@@ -1699,6 +1699,11 @@ def test_grouped_products_at_the_edges_of_their_tiles(dtype, E, top, N, K, T):
     got = o.grouped_linear(x.to(dev()), gate_up.to(dev()), lists, counts, T, per_token=True, out_dtype=dtype,
                            gate="silu")
     assert rel_err(got, unit) < tol_of(dtype)
+    # (with its sums rounded first: the bits that the unit's own kernel gives)
+    got = o.grouped_linear(x.to(dev()), gate_up.to(dev()), lists, counts, T, per_token=True, out_dtype=dtype,
+                           gate="gelu_tanh", rounded=True)
+    both = o.grouped_linear(x.to(dev()), gate_up.to(dev()), lists, counts, T, per_token=True, out_dtype=dtype)
+    assert torch.equal(got, o.gated_unit(both, "gelu_tanh"))
     # (a row's bits do not depend on the other tokens of its step)
     l1, c1 = o.expert_lists(None, chosen[:1].contiguous().to(dev()), 1, E)
     alone = o.grouped_linear(x[:1].contiguous().to(dev()), w.to(dev()), l1, c1, 1, per_token=True,
@@ -1747,3 +1752,49 @@ def test_grouped_products_in_wide_tiles(K, columns, top):
         assert torch.equal(o.grouped_linear(xd[t:t + 1].contiguous(), wd, out_dtype=torch.float32, **one), got[mine])
         assert torch.equal(o.grouped_linear(xd[t:t + 1].contiguous(), wd, out_dtype=torch.bfloat16, gate="silu",
                                             **one), gated[mine])
+
+
+@pytest.mark.parametrize("T", [1, 7, 16, 17, 32, 33, 100])
+@pytest.mark.parametrize("n,extra,top,groups,keep,K,scores", [(8, 0, 2, 0, 0, 2048, "softmax"), (32, 1, 4, 4, 2, 1024, "softmax"),
+                                                              (16, 0, 3, 0, 0, 200, "sigmoid"), (48, 0, 5, 0, 0, 520, "sigmoid"),
+                                                              (64, 16, 7, 16, 3, 8, "softmax"), (3, 0, 1, 0, 0, 4104, "softmax")])
+def test_router_product_and_choice_in_one_kernel(T, n, extra, top, groups, keep, K, scores):
+    """One or two blocks of tokens a workgroup and several workgroups, one to five blocks of outputs, K
+    below and off multiples of what the waves take together: the product against 64 bits, choice and
+    lists as the kernels of their own have them for the same logits."""
+    o = ops()
+    x, w = rand((T, K), torch.bfloat16, 90 + T), rand((n + extra, K), torch.bfloat16, 91, K ** -0.5)
+    bias = rand((n + extra,), torch.float32, 92) if n == 8 else None
+    correction = rand((n,), torch.float32, 93, 0.1).to(dev()) if extra else None
+    xd, wd, bd = x.to(dev()), w.to(dev()), bias.to(dev()) if bias is not None else None
+    assert o.route_linear_takes(xd, wd, n)
+    rule = (correction, groups, keep, 1.5, scores, scores == "sigmoid")
+    chosen, weight, logits, (lists, counts) = o.route_linear(xd, wd, bd, n, top, *rule, want_logits=True, experts=n)
+    want = x.double() @ w.double().T + (bias.double() if bias is not None else 0.0)
+    assert rel_err(logits, want) < F32_TOL
+    c, s = o.route_topk(logits, n, top, *rule)
+    assert torch.equal(chosen, c) and torch.equal(weight, s)
+    l, k = o.expert_lists(None, chosen, T, n)
+    assert torch.equal(counts, k)
+    for e in range(n):
+        assert torch.equal(lists[e, :int(k[e])], l[e, :int(k[e])])
+    # (a token's bits do not depend on the others)
+    one = o.route_linear(xd[T - 1:].contiguous(), wd, bd, n, top, *rule, want_logits=True)
+    assert torch.equal(one[2], logits[T - 1:]) and torch.equal(one[0], chosen[T - 1:])
+
+
+@pytest.mark.parametrize("T,width", [(1, 64), (5, 300), (40, 2048)])
+def test_combined_experts_added_to_the_stream(T, width):
+    """The same numbers as the combined rows added by the stream's own kernel, and their rounding."""
+    o = ops()
+    top, E = 3, 6
+    gen = torch.Generator().manual_seed(T)
+    chosen = torch.stack([torch.randperm(E, generator=gen)[:top] for _ in range(T)]).int().to(dev())
+    out, weight = rand((T * top, width), torch.float32, 95).to(dev()), rand((T, top), torch.float32, 96).to(dev())
+    x, stream = rand((T, width), torch.bfloat16, 97).to(dev()), rand((T, width), torch.float32, 98).to(dev())
+    y = o.experts_combine(out, chosen, weight, x, 4)
+    want = stream.clone()
+    o.scaled_add_rmsnorm(want, y, 0.7)
+    copy = o.experts_combine(out, chosen, weight, x, 4, stream=stream, stream_scale=0.7, copy_dtype=torch.bfloat16)
+    assert torch.equal(stream, want) and torch.equal(copy, want.bfloat16())
+    assert o.experts_combine(out, chosen, weight, x, 4, stream=stream) is None

@@ -21,7 +21,8 @@
 //    2N rows, gate rows ahead of up rows, and out[.., n] = act(v[n]) * v[N + n] from the 32-bit
 //    sums (a wave holds both columns), so the products' 2N columns are never stored.
 //    `row_weight`: one number an assignment, times the result, or with a gate times the sums
-//    ahead of it (a weight on an expert's input; there are no biases).
+//    ahead of it (a weight on an expert's input; there are no biases).  `rounded`: a gate reads its
+//    sums rounded to the result's type, as a kernel of its own would.
 //    How many tiles there are is known on the device only; the grid is the upper bound
 //    ceil(A / TM) + E and a workgroup beyond the last tile leaves at once.
 //    Every output element is a sum over k in an order fixed by K alone: a token's result
@@ -112,6 +113,7 @@ struct GroupedArgs {
   const float* row_weight;   // [A] or null
   int gate;                  // 0: none, 1: silu, 2: the tanh form of gelu, 3: bounded
   float bound, slope, offset;
+  int rounded;               // with a gate: the sums are rounded to the result's type ahead of it
 };
 
 // The expert and the tile within it that workgroup `b` serves; false when there is none.  A wave
@@ -163,7 +165,12 @@ __device__ __forceinline__ float expert_act(float v, int act) {
 }
 
 // The gated unit (gate > 0) of one assignment's sums `v` (gate) and `u` (up).
+template <typename TO>
 __device__ __forceinline__ float expert_unit(const GroupedArgs& g, float v, float u, float w) {
+  if (g.rounded) {
+    v = to_f32<TO>(from_f32<TO>(v));
+    u = to_f32<TO>(from_f32<TO>(u));
+  }
   v *= w;
   u *= w;
   if (g.gate == 3) {
@@ -218,7 +225,7 @@ __device__ __forceinline__ void grouped_store(const GroupedArgs& g, const int* _
       for (int j = 0; j < TN; j += 2) {
         f32x4_t v;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = expert_unit(g, acc[i][j][r], acc[i][j + 1][r], w);
+        for (int r = 0; r < 4; ++r) v[r] = expert_unit<TO>(g, acc[i][j][r], acc[i][j + 1][r], w);
         put(to, n0 + (wn >> 1) + (j / 2) * 16 + kq * 4, v);
       }
     } else {
@@ -414,7 +421,7 @@ grouped_gemm_f32_kernel(GroupedArgs g) {
           const int first = n0 + (n >> 5) * 16 + (n & 15);
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (first + i < N) at[first + i] = from_f32<TO>(expert_unit(g, v[0][i], v[1][i], w));
+            if (first + i < N) at[first + i] = from_f32<TO>(expert_unit<TO>(g, v[0][i], v[1][i], w));
         } else {
 #pragma unroll
           for (int j = 0; j < GF_BN / 32; ++j)
@@ -434,7 +441,7 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
                                int out_dtype, int n_tokens, int top, int experts, int N, int K,
                                int src_div, int stacked, int act, float out_scale,
                                const float* row_weight, int gate, float bound, float slope,
-                               float offset, hipStream_t stream) {
+                               float offset, int rounded, hipStream_t stream) {
   if (n_tokens == 0) return 0;
   if (n_tokens < 0 || top <= 0 || experts <= 0 || N <= 0 || K <= 0 || !src || !W || !lists ||
       !counts || !out || (src_div != 1 && src_div != top) || act < 0 || act > 1 ||
@@ -445,7 +452,7 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
   if (experts > EX_MAX_EXPERTS) return ZA_ERR_UNSUPPORTED;
   if (stacked && out_dtype != 0) return ZA_ERR_UNSUPPORTED;
   GroupedArgs g{src, W, lists, counts, out, (int)A, n_tokens, top, experts, N, K,
-                src_div, stacked, act, out_scale, row_weight, gate, bound, slope, offset};
+                src_div, stacked, act, out_scale, row_weight, gate, bound, slope, offset, rounded};
   if (w_dtype == 1) {
     if (src_dtype != 1 || K % 8 != 0 || ((uintptr_t)src | (uintptr_t)W) % 16 != 0) return ZA_ERR_UNSUPPORTED;
     if (out_dtype != 0 && out_dtype != 1) return ZA_ERR_UNSUPPORTED;
@@ -639,67 +646,246 @@ route_topk_kernel(const float* __restrict__ z, int ld, const float* __restrict__
   for (int j = lane; j < top; j += 64) weight[(size_t)t * top + j] *= f;
 }
 
-// The same for at most 64 outputs: a lane has one, in registers, and counts how many come before
-// its own (a broadcast an output, in place of a maximum over the wave and two meetings a choice).  Eight tokens, 32
-// outputs in 4 groups, 4 of them: 7.0 us in a step, 9.0 with the kernel above.
-__global__ void __launch_bounds__(64)
-route_topk_wave_kernel(const float* __restrict__ z, int ld, const float* __restrict__ correction, int n,
-                       int groups, int keep, int top, float scale, int mode, int renorm,
-                       int* __restrict__ chosen, float* __restrict__ weight) {
-  const int t = blockIdx.x, lane = threadIdx.x;
-  const bool in = lane < n;
-  const float zv = in ? z[(size_t)t * ld + lane] : -INFINITY;
-  const float add = in && correction ? correction[lane] : 0.f;
+// The same for at most 64 outputs: a lane has one, in registers.  Everything over the wave runs on the
+// vector unit's own lane patterns (through LDS, a maximum over the wave waits six times): a choice is a
+// maximum and the first lane that holds it, a group's best a maximum over its lanes.
+// `z`: this lane's output, `give(j, output, weight)`: the lane that has the j-th choice.
+struct RouteRule {
+  int n, groups, keep, top, mode, renorm;
+  float scale;
+};
+
+template <int CTRL>
+__device__ __forceinline__ float lanes_moved(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float lane_value(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+// over 2, 4, 8, 16 neighbouring lanes: their pairs, quads, halves of rows, rows
+#define ZA_OVER_16(v, OP)                     \
+  v = OP(v, lanes_moved<0xB1>(v));            \
+  v = OP(v, lanes_moved<0x4E>(v));            \
+  v = OP(v, lanes_moved<0x141>(v));           \
+  v = OP(v, lanes_moved<0x140>(v))
+__device__ __forceinline__ float add_f32(float a, float b) { return a + b; }
+__device__ __forceinline__ float lanes_max(float v) {
+  ZA_OVER_16(v, fmaxf);
+  return fmaxf(fmaxf(lane_value(v, 0), lane_value(v, 16)), fmaxf(lane_value(v, 32), lane_value(v, 48)));
+}
+__device__ __forceinline__ float lanes_sum(float v) {
+  ZA_OVER_16(v, add_f32);
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+
+template <typename F>
+__device__ __forceinline__ void route_wave(const RouteRule& q, float z, float add, int lane, F&& give) {
+  const bool in = lane < q.n;
+  const float zv = in ? z : -INFINITY;
   float s;
-  if (mode == 0) {
-    const float mx = wave_max(zv);
-    const float p = in ? expf(zv - mx) : 0.f;
-    s = p * (1.0f / wave_sum(p));
+  if (q.mode == 0) {
+    const float p = in ? expf(zv - lanes_max(zv)) : 0.f;
+    s = p * (1.0f / lanes_sum(p));
   } else {
     s = 1.0f / (1.0f + expf(-zv));
   }
-  float c = s + add;
-  auto of = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
-  if (groups > 1 && keep < groups) {
-    const int per = n / groups, g = lane / per;
-    float best = -INFINITY;
-    for (int q = 0; q < groups; ++q)
-#pragma unroll 4
-      for (int k = q * per; k < (q + 1) * per; ++k) {
-        const float v = of(c, k);
-        best = q == g ? fmaxf(best, v) : best;
+  float c = s + (in ? add : 0.f);
+  if (q.groups > 1 && q.keep < q.groups) {
+    const int per = q.n / q.groups, g = lane / per;
+    // (the largest that compares: NaN is nobody's best)
+    float best = in && c == c ? c : -INFINITY;
+    if (per == 2 || per == 4 || per == 8 || per == 16) {
+      best = fmaxf(best, lanes_moved<0xB1>(best));
+      if (per > 2) best = fmaxf(best, lanes_moved<0x4E>(best));
+      if (per > 4) best = fmaxf(best, lanes_moved<0x141>(best));
+      if (per > 8) best = fmaxf(best, lanes_moved<0x140>(best));
+    } else {
+      const float own = best;
+      best = -INFINITY;
+      for (int o = 0; o < q.groups; ++o) {
+        const float v = lanes_max(g == o ? own : -INFINITY);
+        best = o == g ? v : best;
       }
+    }
     // (a group whose best is infinite is open whatever the others are)
     int before = 0;
-    for (int k = 0; k < groups; ++k) {
-      const float v = of(best, k * per);
+    for (int k = 0; k < q.groups; ++k) {
+      const float v = lane_value(best, k * per);
       if (v != INFINITY && (v > best || (v == best && k < g))) ++before;
     }
-    if (best != INFINITY && before >= keep) c = -INFINITY;
+    if (best != INFINITY && before >= q.keep) c = -INFINITY;
   }
-  const bool open = in && c == c;                     // NaN is not chosen
-  int before = 0;
-#pragma unroll 8
-  for (int k = 0; k < n; ++k) {
-    const float v = of(c, k);
-    if (v > c || (v == c && k < lane)) ++before;
-  }
-  const int usable = __popcll(__ballot(open));
-  float total = 0.f;
-  for (int j = 0; j < top; ++j) {
+  bool open = in && c == c;                           // NaN is not chosen
+  float total = 0.f, share = 0.f;
+  int place = -1, output = 0;
+  for (int j = 0; j < q.top; ++j) {
+    const float m = lanes_max(open ? c : -INFINITY);
+    const unsigned long long who = __ballot(open && c == m);
     // (nothing left to choose from: output 0)
-    const unsigned long long who = __ballot(open && before == j);
-    total += of(s, j < usable ? __ffsll((long long)who) - 1 : 0);
+    const int at = who ? __ffsll((long long)who) - 1 : 0;
+    const float v = lane_value(s, at);
+    total += v;
+    if (lane == j) {
+      place = j;
+      output = at;
+      share = v;
+    }
+    if (lane == at) open = false;
   }
-  const float f = renorm ? scale / (total + 1e-20f) : scale;   // (all scores may underflow)
-  if (open && before < top) {
-    chosen[(size_t)t * top + before] = lane;
-    weight[(size_t)t * top + before] = s * f;
+  const float f = q.renorm ? q.scale / (total + 1e-20f) : q.scale;   // (all scores may underflow)
+  if (place >= 0) give(place, output, share * f);
+}
+
+__global__ void __launch_bounds__(64)
+route_topk_wave_kernel(const float* __restrict__ z, int ld, const float* __restrict__ correction, RouteRule q,
+                       int* __restrict__ chosen, float* __restrict__ weight) {
+  const int t = blockIdx.x, lane = threadIdx.x;
+  const bool in = lane < q.n;
+  route_wave(q, in ? z[(size_t)t * ld + lane] : 0.f, in && correction ? correction[lane] : 0.f, lane,
+             [&](int j, int output, float w) {
+               chosen[(size_t)t * q.top + j] = output;
+               weight[(size_t)t * q.top + j] = w;
+             });
+}
+
+// A router from its product to its choice in one kernel, for at most 64 outputs (and a few rows behind
+// them, the shared expert's gate): a workgroup takes MT * 16 tokens and all NT * 16 weight rows, its
+// sixteen waves a sixteenth of K each (64 elements in turn, matrix cores, 32-bit sums added up in the
+// waves' order), then a wave chooses for a token.  Where one workgroup has all tokens it writes the
+// experts' lists, too.  Bound by its chain, way to memory, sums, choice, not by bytes; what it replaces
+// is three or four launches with such a chain each, a product of 8 to 36 outputs that leaves all but a
+// few compute units idle among them.
+struct RouteArgs {
+  const bf16_t *x, *W;       // [T][K], [rows][K]
+  const float *bias, *correction;
+  float* logits;             // [T][rows] or null
+  int* chosen;               // [T][top]
+  float* weight;             // [T][top]
+  int* lists;                // [experts][T * top] or null: no lists
+  int* counts;
+  int T, K, rows, experts;
+  RouteRule q;
+};
+
+#define RL_WAVES 16
+
+template <int NT, int MT>
+__global__ void __launch_bounds__(RL_WAVES * 64)
+route_linear_kernel(RouteArgs a) {
+  constexpr int LD = NT * 16 + 4, UNROLL = NT * MT > 3 ? 2 : 4;
+  __shared__ __attribute__((aligned(16))) float sums[RL_WAVES][MT * 16][LD];
+  __shared__ int picked[MT * 16 * 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int t0 = blockIdx.x * MT * 16, K = a.K;
+  const bf16_t *xr[MT], *wr[NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xr[i] = a.x + (size_t)min(t0 + i * 16 + r16, a.T - 1) * K;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) wr[j] = a.W + (size_t)min(j * 16 + r16, a.rows - 1) * K;
+  // (asked for ahead of the product)
+  const float add = a.correction && lane < a.q.n ? a.correction[lane] : 0.f;
+  const float shift = a.bias ? a.bias[min(tid % (NT * 16), a.rows - 1)] : 0.f;
+  f32x4_t acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  const bf16x8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  // (a wave reads whole lines of 128 bytes, 64 elements)
+  for (int k0 = wave * 64 + kq * 8; k0 - kq * 8 < K; k0 += UNROLL / 2 * RL_WAVES * 64) {
+    bf16x8_t fx[UNROLL][MT], fw[UNROLL][NT];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int k = k0 + (u >> 1) * RL_WAVES * 64 + (u & 1) * 32, at = min(k, K - 8);      // (K is a multiple of 8)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) fx[u][i] = *reinterpret_cast<const bf16x8_t*>(xr[i] + at);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) fw[u][j] = *reinterpret_cast<const bf16x8_t*>(wr[j] + at);
+    }
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const bool in = k0 + (u >> 1) * RL_WAVES * 64 + (u & 1) * 32 < K;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(in ? fw[u][j] : zero8, in ? fx[u][i] : zero8,
+                                                               acc[i][j], 0, 0, 0);
+    }
   }
-  if (lane >= usable && lane < top) {
-    chosen[(size_t)t * top + lane] = 0;
-    weight[(size_t)t * top + lane] = of(s, 0) * f;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      *reinterpret_cast<f32x4_t*>(&sums[wave][i * 16 + r16][j * 16 + kq * 4]) = acc[i][j];
+  __syncthreads();
+  for (int i = tid; i < MT * 16 * NT * 16; i += RL_WAVES * 64) {
+    const int t = i / (NT * 16), o = i % (NT * 16);
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < RL_WAVES; ++w) v += sums[w][t][o];
+    if (a.bias && o < a.rows) v += i < RL_WAVES * 64 ? shift : a.bias[o];
+    sums[0][t][o] = v;                               // (only this thread reads or writes the place)
+    if (a.logits && o < a.rows && t0 + t < a.T) a.logits[(size_t)(t0 + t) * a.rows + o] = v;
   }
+  __syncthreads();
+  for (int i = 0; i < MT; ++i) {
+    const int own = i * RL_WAVES + wave, t = t0 + own;
+    if (t >= a.T) break;
+    route_wave(a.q, lane < a.q.n ? sums[0][own][lane] : 0.f, add, lane, [&](int j, int output, float w) {
+      a.chosen[(size_t)t * a.q.top + j] = output;
+      a.weight[(size_t)t * a.q.top + j] = w;
+      picked[own * a.q.top + j] = output;
+    });
+  }
+  if (!a.lists) return;
+  __syncthreads();
+  const int A = a.T * a.q.top;
+  for (int e = wave; e < a.experts; e += RL_WAVES) {
+    int running = 0;
+    for (int base = 0; base < A; base += 64) {
+      const bool hit = base + lane < A && picked[base + lane] == e;
+      const unsigned long long who = __ballot(hit);
+      if (hit) a.lists[(size_t)e * A + running + __popcll(who & ((1ull << lane) - 1))] = base + lane;
+      running += __popcll(who);
+    }
+    if (lane == 0) a.counts[e] = running;
+  }
+}
+
+// `rows` weight rows, the first `n` of them the router's outputs; lists and counts may be null (they must
+// be beyond ZA_ROUTE_LISTS tokens: no workgroup sees all of them).
+#define ZA_ROUTE_LISTS 32
+extern "C" int za_route_linear(const void* x, const void* W, const float* bias, const float* correction,
+                               int n_tokens, int K, int rows, int n, int groups, int keep, int top, float scale,
+                               int mode, int renorm, float* logits, int* chosen, float* weight, int experts,
+                               int* lists, int* counts, hipStream_t stream) {
+  if (n_tokens == 0) return 0;
+  if (n_tokens < 0 || K <= 0 || n <= 0 || rows < n || top <= 0 || top > n || !x || !W || !chosen || !weight ||
+      groups < 0 || (groups > 0 && (n % groups != 0 || keep <= 0 || keep > groups)) || mode < 0 || mode > 1 ||
+      (lists && (!counts || experts <= 0 || n_tokens > ZA_ROUTE_LISTS)))
+    return ZA_ERR_ARG;
+  if (groups > 0 && (long long)keep * (n / groups) < top) return ZA_ERR_ARG;
+  if (n > 64 || rows > 80 || K % 8 != 0 || ((uintptr_t)x | (uintptr_t)W) % 16 != 0) return ZA_ERR_UNSUPPORTED;
+  const int tiles = (rows + 15) / 16;
+  const bool two = lists && n_tokens > 16;            // (all tokens in one workgroup)
+  if (two && tiles > 3) return ZA_ERR_UNSUPPORTED;
+  RouteArgs a{(const bf16_t*)x, (const bf16_t*)W, bias, correction, logits, chosen, weight, lists, counts,
+              n_tokens, K, rows, experts, RouteRule{n, groups, keep, top, mode, renorm, scale}};
+  const dim3 grid(two ? 1 : (n_tokens + 15) / 16), block(RL_WAVES * 64);
+#define ZA_RL(NT, MT) hipLaunchKernelGGL((route_linear_kernel<NT, MT>), grid, block, 0, stream, a)
+  if (two) {
+    if (tiles == 1) ZA_RL(1, 2);
+    else if (tiles == 2) ZA_RL(2, 2);
+    else ZA_RL(3, 2);
+  } else if (tiles == 1) ZA_RL(1, 1);
+  else if (tiles == 2) ZA_RL(2, 1);
+  else if (tiles == 3) ZA_RL(3, 1);
+  else if (tiles == 4) ZA_RL(4, 1);
+  else ZA_RL(5, 1);
+#undef ZA_RL
+  return za_launch_status();
 }
 
 extern "C" int za_route_topk(const float* z, int ld, const float* correction, int n_tokens, int n,
@@ -713,8 +899,8 @@ extern "C" int za_route_topk(const float* z, int ld, const float* correction, in
   if (groups > 0 && (long long)keep * (n / groups) < top) return ZA_ERR_ARG;
   if (n > RT_MAX) return ZA_ERR_UNSUPPORTED;
   if (n <= 64)
-    hipLaunchKernelGGL(route_topk_wave_kernel, dim3(n_tokens), dim3(64), 0, stream, z, ld, correction, n,
-                       groups, keep, top, scale, mode, renorm, chosen, weight);
+    hipLaunchKernelGGL(route_topk_wave_kernel, dim3(n_tokens), dim3(64), 0, stream, z, ld, correction,
+                       RouteRule{n, groups, keep, top, mode, renorm, scale}, chosen, weight);
   else
     hipLaunchKernelGGL(route_topk_kernel, dim3(n_tokens), dim3(64), 0, stream, z, ld, correction, n,
                        groups, keep, top, scale, mode, renorm, chosen, weight);
@@ -727,21 +913,24 @@ extern "C" int za_route_topk(const float* z, int ld, const float* correction, in
 // An output beyond the n_real experts that have weights hands the token's input x[t] on.
 // gate(t) = sigmoid(gate_logits[t * gate_ld]) when gate_logits is given, else 1; `shared`
 // may be absent.  The sum is taken in the order j = 0 .. top - 1, then the shared expert.
+// With `stream` the row goes there, stream[t] += stream_scale * y[t], and rounded to `copy` (may be
+// null); otherwise to y.
 // `weigh` 0: the experts' outputs hold their weights already (a weight on an expert's input).
 // A thread takes one column of one token (a workgroup 256 of them: with a workgroup a token and its
 // columns one after the other, eight tokens of 2,048 took 14.9 us).
-template <typename TE, typename TX>
+template <typename TE, typename TX, bool ADD>
 __global__ void __launch_bounds__(256)
 experts_combine_kernel(const TE* __restrict__ expert_out, const int* __restrict__ chosen,
                        const float* __restrict__ weight, const TX* __restrict__ x,
                        const TE* __restrict__ shared, const float* __restrict__ gate_logits,
                        int gate_ld, float* __restrict__ y, int top, int n_real, int width,
-                       int weigh) {
+                       int weigh, float stream_scale, bf16_t* __restrict__ copy) {
   const size_t t = blockIdx.x;
   const int i = blockIdx.y * blockDim.x + threadIdx.x;
   if (i >= width) return;
   const float sh = shared ? to_f32<TE>(shared[t * width + i]) : 0.f;
   const float own = to_f32<TX>(x[t * width + i]);
+  const float before = ADD ? y[t * width + i] : 0.f;
   float g = 1.0f;
   if (shared && gate_logits) g = 1.0f / (1.0f + expf(-gate_logits[t * gate_ld]));
   float acc = 0.f;
@@ -753,7 +942,9 @@ experts_combine_kernel(const TE* __restrict__ expert_out, const int* __restrict_
     acc = fmaf(w, v, acc);
   }
   if (shared) acc = fmaf(g, sh, acc);
+  if (ADD) acc = fmaf(stream_scale, acc, before);
   y[t * width + i] = acc;
+  if (ADD && copy) copy[t * width + i] = (bf16_t)acc;
 }
 
 // dtype codes: 0 = float32, 1 = bfloat16; `out_dtype` is that of expert_out and shared.
@@ -761,21 +952,27 @@ extern "C" int za_experts_combine(const void* expert_out, int out_dtype, const i
                                   const float* weight, const void* x, int x_dtype,
                                   const void* shared, const float* gate_logits, int gate_ld,
                                   float* y, int n_tokens, int top, int n_real, int width,
-                                  int weigh, hipStream_t stream) {
+                                  int weigh, int add, float stream_scale, void* copy, hipStream_t stream) {
   if (n_tokens == 0) return 0;
   if (n_tokens < 0 || top <= 0 || width <= 0 || n_real < 0 || !chosen || !weight || !x || !y ||
-      (n_real > 0 && !expert_out))
+      (n_real > 0 && !expert_out) || (copy && !add))
     return ZA_ERR_ARG;
   dim3 block(width <= 256 ? 64 : 256), grid(n_tokens, (width + block.x - 1) / block.x);
-#define ZA_EC(TE, TX)                                                                          \
-  hipLaunchKernelGGL((experts_combine_kernel<TE, TX>), grid, block, 0, stream,                 \
+#define ZA_ECA(TE, TX, ADD)                                                                    \
+  hipLaunchKernelGGL((experts_combine_kernel<TE, TX, ADD>), grid, block, 0, stream,            \
                      (const TE*)expert_out, chosen, weight, (const TX*)x, (const TE*)shared,   \
-                     gate_logits, gate_ld, y, top, n_real, width, weigh)
-  if (out_dtype == 0 && x_dtype == 0) ZA_EC(float, float);
-  else if (out_dtype == 0 && x_dtype == 1) ZA_EC(float, bf16_t);
-  else if (out_dtype == 1 && x_dtype == 1) ZA_EC(bf16_t, bf16_t);
-  else if (out_dtype == 1 && x_dtype == 0) ZA_EC(bf16_t, float);
+                     gate_logits, gate_ld, y, top, n_real, width, weigh, stream_scale, (bf16_t*)copy)
+#define ZA_EC(TE, TX)                   \
+  {                                     \
+    if (add) ZA_ECA(TE, TX, true);      \
+    else ZA_ECA(TE, TX, false);         \
+  }
+  if (out_dtype == 0 && x_dtype == 0) ZA_EC(float, float)
+  else if (out_dtype == 0 && x_dtype == 1) ZA_EC(float, bf16_t)
+  else if (out_dtype == 1 && x_dtype == 1) ZA_EC(bf16_t, bf16_t)
+  else if (out_dtype == 1 && x_dtype == 0) ZA_EC(bf16_t, float)
   else return ZA_ERR_UNSUPPORTED;
 #undef ZA_EC
+#undef ZA_ECA
   return za_launch_status();
 }

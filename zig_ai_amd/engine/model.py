@@ -112,7 +112,10 @@ class DecoderModel:
         if self.embedding_rounds:
             first = spec.schedule[0]
             self.embedding.rounded_wanted = first.before is None and \
-                bool(getattr(self.blocks[first.layer], "leaves_rounded", False))
+                bool(getattr(self.blocks[first.layer], "reads_rounded", False))
+        for call in spec.schedule:
+            if call.after is not None and getattr(self.stream_parts[call.after.part], "reads_rounded", False):
+                self.blocks[call.layer].rounded_wanted = True
         self.final_norm = make("norm", spec.final_norm, ("final_norm",))
         self.head = make("head", spec.lm_head, ("lm_head",))
         note(self.final_norm)
@@ -287,11 +290,14 @@ class DecoderModel:
                     residual, pending, origin, step, **dict(call.before.args))
             block = self.blocks[call.layer]
             residual, pending = block.forward(residual, pending, step, view)
-            if call.after is not None or not getattr(block, "leaves_rounded", False):
+            after = self.stream_parts[call.after.part] if call.after is not None else None
+            if not getattr(block, "leaves_rounded", False) or \
+                    (after is not None and not getattr(after, "reads_rounded", False)):
                 step.rounded = None
-            if call.after is not None:
-                residual, pending = self.stream_parts[call.after.part].forward(
-                    residual, pending, origin, step, **dict(call.after.args))
+            if after is not None:
+                residual, pending = after.forward(residual, pending, origin, step,
+                                                  **dict(call.after.args))
+                step.rounded = None
             if taps is not None:
                 now = residual.clone()
                 if pending is not None:

@@ -179,7 +179,7 @@ _SIGNATURES = {
     ("experts", "za_grouped_gemm"): [c_void_p, c_int, c_longlong, c_void_p, c_int, c_void_p,
                                      c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                                      c_int, c_int, c_int, c_float, c_void_p, c_int, c_float,
-                                     c_float, c_float, c_void_p],
+                                     c_float, c_float, c_int, c_void_p],
     ("activation", "za_softcap"): [c_void_p, c_float, c_longlong, c_void_p],
     ("activation", "za_table_gate"): [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int,
                                       c_int, c_void_p, c_int, c_int, c_int, c_void_p],
@@ -203,9 +203,12 @@ _SIGNATURES = {
                                                      c_int, c_int, c_int, c_int, c_void_p],
     ("experts", "za_route_topk"): [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                    c_float, c_int, c_int, c_void_p, c_void_p, c_void_p],
+    ("experts", "za_route_linear"): [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                     c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p,
+                                     c_void_p, c_int, c_void_p, c_void_p, c_void_p],
     ("experts", "za_experts_combine"): [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                                         c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int,
-                                        c_int, c_int, c_void_p],
+                                        c_int, c_int, c_int, c_float, c_void_p, c_void_p],
     ("latent", "za_latent_prepare"): [c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                       c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
                                       c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_longlong,
@@ -2642,7 +2645,7 @@ def grouped_linear(src: torch.Tensor, weights: torch.Tensor, lists: torch.Tensor
                    out_dtype: Optional[torch.dtype] = None, gate: Optional[str] = None,
                    bounded: Optional[Tuple[float, float, float]] = None,
                    row_weight: Optional[torch.Tensor] = None,
-                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   out: Optional[torch.Tensor] = None, rounded: bool = False) -> torch.Tensor:
     """Every assignment's row times its expert's weight: ``weights [experts, N, K]``,
     ``src [T, K]`` (``per_token``: assignment ``a`` reads row ``a // top``) or ``[T*top, K]``
     (one row an assignment).  Returns ``[T*top, N]`` in assignment order, or with ``stacked``
@@ -2652,7 +2655,8 @@ def grouped_linear(src: torch.Tensor, weights: torch.Tensor, lists: torch.Tensor
     (limit, alpha, up_offset)``: ``weights [experts, 2N, K]`` are gate rows and up rows, and the
     result is the gated unit (``gated_unit`` / ``clamped_glu``) of their 32-bit sums, ``N`` columns.
     ``row_weight`` (32-bit, one an assignment) multiplies the result, or with a gate the sums
-    ahead of it.  ``out``: write there."""
+    ahead of it.  ``rounded``: the gate reads its sums rounded to ``out_dtype``, as a kernel of its
+    own would.  ``out``: write there."""
     if activation not in EXPERT_ACTIVATIONS:
         raise KernelError(f"activation must be None or relu2, got {activation!r}")
     _need(weights, "weights", (torch.float32, torch.bfloat16))
@@ -2691,7 +2695,7 @@ def grouped_linear(src: torch.Tensor, weights: torch.Tensor, lists: torch.Tensor
         _ptr(src), _code(src.dtype), src.shape[0], _ptr(weights), _code(weights.dtype), _ptr(lists),
         _ptr(counts), _ptr(out), _code(out_dtype), n_tokens, top, E, N, K, top if per_token else 1,
         1 if stacked else 0, EXPERT_ACTIVATIONS[activation], float(out_scale), _ptr(row_weight),
-        gate_code, *bounds, _stream())
+        gate_code, *bounds, 1 if rounded else 0, _stream())
     _check(rc, "grouped_linear", f"E={E} N={N} K={K} tokens={n_tokens} top={top}")
     return out
 
@@ -2723,14 +2727,63 @@ def route_topk(logits: torch.Tensor, n: int, top: int, correction: Optional[torc
     return chosen, weight
 
 
+ROUTE_OUTPUTS, ROUTE_ROWS, ROUTE_LISTS = 64, 80, 32     # csrc/experts.hip, ``za_route_linear``
+
+
+def route_linear_takes(x: torch.Tensor, weight: torch.Tensor, n: int) -> bool:
+    """Whether ``route_linear`` can run a router's product and choice."""
+    return x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and n <= ROUTE_OUTPUTS \
+        and weight.shape[0] <= ROUTE_ROWS and x.shape[1] % 8 == 0 \
+        and (x.data_ptr() | weight.data_ptr()) % 16 == 0
+
+
+def route_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], n: int, top: int,
+                 correction: Optional[torch.Tensor] = None, groups: int = 0, keep: int = 0,
+                 scale: float = 1.0, scores: str = "softmax", renormalize: bool = False,
+                 want_logits: bool = False, experts: int = 0):
+    """``route_topk(linear(x, weight, bias), n, ...)`` in one kernel, where ``route_linear_takes``:
+    ``(chosen, weight, logits or None, (lists, counts) or None)``.  ``want_logits``: the product's
+    32-bit ``[T, rows]`` too.  ``experts``: ``expert_lists(None, chosen, T, experts)`` too."""
+    _need(x, "x", torch.bfloat16)
+    _need(weight, "weight", torch.bfloat16)
+    if x.dim() != 2 or weight.dim() != 2 or weight.shape[1] != x.shape[1] or weight.shape[0] < n:
+        raise KernelError(f"a router takes x [T, K] and weight [>= {n}, K], got {tuple(x.shape)} and "
+                          f"{tuple(weight.shape)}")
+    if scores not in ("softmax", "sigmoid"):
+        raise KernelError(f"scores must be softmax or sigmoid, got {scores!r}")
+    (T, K), rows = x.shape, weight.shape[0]
+    if bias is not None:
+        _need(bias, "bias", torch.float32, (rows,))
+    if correction is not None:
+        _need(correction, "correction", torch.float32, (n,))
+    chosen = torch.empty((T, top), dtype=torch.int32, device=x.device)
+    share = torch.empty((T, top), dtype=torch.float32, device=x.device)
+    logits = torch.empty((T, rows), dtype=torch.float32, device=x.device) if want_logits else None
+    lists = counts = None
+    if experts and T <= (16 if rows > 48 else ROUTE_LISTS):
+        lists = torch.empty((experts, T * top), dtype=torch.int32, device=x.device)
+        counts = torch.empty((experts,), dtype=torch.int32, device=x.device)
+    rc = _fn("experts", "za_route_linear")(
+        _ptr(x), _ptr(weight), _ptr(bias), _ptr(correction), T, K, rows, int(n), int(groups), int(keep),
+        int(top), float(scale), 0 if scores == "softmax" else 1, 1 if renormalize else 0, _ptr(logits),
+        _ptr(chosen), _ptr(share), int(experts), _ptr(lists), _ptr(counts), _stream())
+    _check(rc, "route_linear", f"T={T} K={K} rows={rows} n={n} top={top} groups={groups} keep={keep}")
+    if experts and lists is None:
+        lists, counts = expert_lists(None, chosen, T, experts)
+    return chosen, share, logits, (lists, counts) if experts else None
+
+
 def experts_combine(expert_out: Optional[torch.Tensor], chosen: torch.Tensor, weight: torch.Tensor,
                     x: torch.Tensor, n_real: int, shared: Optional[torch.Tensor] = None,
                     gate_logits: Optional[torch.Tensor] = None, gate_col: int = 0,
-                    weigh: bool = True) -> torch.Tensor:
+                    weigh: bool = True, stream: Optional[torch.Tensor] = None, stream_scale: float = 1.0,
+                    copy_dtype: Optional[torch.dtype] = None) -> Optional[torch.Tensor]:
     """``y[t] = sum_j weight[t, j] * (expert_out[t * top + j] if chosen[t, j] < n_real else
     x[t]) + gate(t) * shared[t]`` as 32-bit ``[T, width]``; ``gate(t)`` is
     ``sigmoid(gate_logits[t, gate_col])`` (32-bit logits) or one.  ``weigh`` false: the rows of
-    ``expert_out`` hold their weights already."""
+    ``expert_out`` hold their weights already.  ``stream`` (32-bit ``[T, width]``): the rows are added
+    to it, times ``stream_scale``, and what comes back is the sum rounded to ``copy_dtype``
+    (bfloat16), or None."""
     T, top = chosen.shape
     _need(chosen, "chosen", torch.int32, (T, top))
     _need(weight, "weight", torch.float32, (T, top))
@@ -2754,13 +2807,22 @@ def experts_combine(expert_out: Optional[torch.Tensor], chosen: torch.Tensor, we
                               f"of {T} rows is needed")
         gate_ld = gate_logits.shape[1]
         gate_ptr = gate_logits.data_ptr() + 4 * gate_col
-    y = torch.empty((T, width), dtype=torch.float32, device=x.device)
+    copy = None
+    if stream is not None:
+        _need(stream, "stream", torch.float32, (T, width))
+        if copy_dtype is not None:
+            if copy_dtype != torch.bfloat16:
+                raise KernelError(f"the sum's copy is bfloat16, not {copy_dtype}")
+            copy = torch.empty((T, width), dtype=copy_dtype, device=x.device)
+        y = stream
+    else:
+        y = torch.empty((T, width), dtype=torch.float32, device=x.device)
     rc = _fn("experts", "za_experts_combine")(
         _ptr(expert_out), _code(dtype or torch.float32), _ptr(chosen), _ptr(weight), _ptr(x),
         _code(x.dtype), _ptr(shared), gate_ptr, gate_ld, _ptr(y), T, top, int(n_real), width,
-        1 if weigh else 0, _stream())
+        1 if weigh else 0, 1 if stream is not None else 0, float(stream_scale), _ptr(copy), _stream())
     _check(rc, "experts_combine")
-    return y
+    return copy if stream is not None else y
 
 
 def softcap_(x: torch.Tensor, cap: float) -> torch.Tensor:

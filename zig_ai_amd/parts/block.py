@@ -145,7 +145,7 @@ class NormedOutputBlock:
     kind = "normed_output"
     slots = {"mixer": "mixer", "mixer_norm": "norm", "feed_forward": "feed_forward",
              "feed_forward_norm": "norm"}
-    leaves_rounded = True
+    leaves_rounded = reads_rounded = True
 
     def __init__(self, parts):
         self.parts = dict(parts)
@@ -215,10 +215,14 @@ class ScaledResidualBlock:
 
     ``m`` (``residual_scale``), ``a`` and ``b`` (``mixer_scales``) are the layer's
     ``params``.  The weighted sums are taken in 32-bit by one kernel that also runs the
-    norm that follows inside the block; nothing is left pending."""
+    norm that follows inside the block; nothing is left pending.  A feed-forward that combines
+    its result from several (``adds_scaled``) adds it to the stream in the same kernel, which
+    with ``rounded_wanted`` also leaves the sum rounded for what follows (``step.rounded``)."""
 
     mixers = ("mixer",)
     has_feed_forward = True
+    leaves_rounded = True
+    rounded_wanted = False
 
     def __init__(self, parts, residual_scale: float = 1.0, mixer_scales=None):
         self.parts = dict(parts)
@@ -235,6 +239,7 @@ class ScaledResidualBlock:
     def forward(self, residual: torch.Tensor, pending: Optional[torch.Tensor], step,
                 cache) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
         from ..kernels import ops
+        step.rounded = None
         h = None
         if pending is None and all(getattr(p, "takes_stream", False)
                                    or getattr(p, "takes_normed_rows", False)
@@ -260,6 +265,11 @@ class ScaledResidualBlock:
         else:
             ops.scaled_add_rmsnorm(residual, outs[0], self.mixer_scales[0], *second)
             h = norm.forward(residual)
+        if getattr(self.feed_forward, "adds_scaled", False):
+            copy = h.dtype if self.rounded_wanted and h.dtype == torch.bfloat16 else None
+            step.rounded = self.feed_forward.forward(h, step, stream=residual,
+                                                     stream_scale=self.residual_scale, copy_dtype=copy)
+            return residual, None
         y = self.feed_forward.forward(h, step)
         ops.scaled_add_rmsnorm(residual, y, self.residual_scale)
         return residual, None

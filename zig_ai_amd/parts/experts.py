@@ -195,45 +195,55 @@ class RoutedExperts(FeedForward):
                 torch.cat([tensors["shared.gate.weight"], tensors["shared.up.weight"]], dim=0).contiguous())
             self.shared_down = ops.projection_weight(tensors["shared.down.weight"])
 
-    def forward(self, x, step):
+    def forward(self, x, step, stream=None, stream_scale: float = 1.0, copy_dtype=None):
+        """``stream``: the rows are added to it, times ``stream_scale``, and the sum rounded to
+        ``copy_dtype`` (or None) comes back, where they are combined by a kernel of its own."""
         T = x.shape[0]
         tune = self.runtime.tune
-        logits = ops.linear(x, self.w_router, self.b_router, out_dtype=torch.float32, tune=tune)
-        chosen, weight = ops.route_topk(logits, self.outputs, self.top, self.correction,
-                                        self.groups, self.keep, self.route_scale, self.scores,
-                                        self.renormalize)
+        rule = (self.correction, self.groups, self.keep, self.route_scale, self.scores, self.renormalize)
+        lists = None
+        if ops.route_linear_takes(x, self.w_router, self.outputs):
+            # (an output beyond the experts that have weights is in nobody's list)
+            chosen, weight, logits, lists = ops.route_linear(
+                x, self.w_router, self.b_router, self.outputs, self.top, *rule,
+                want_logits=self.shared_gated, experts=self.experts)
+        else:
+            logits = ops.linear(x, self.w_router, self.b_router, out_dtype=torch.float32, tune=tune)
+            chosen, weight = ops.route_topk(logits, self.outputs, self.top, *rule)
+            if self.experts:
+                lists = ops.expert_lists(None, chosen, T, self.experts)
         out = None
         if self.experts:
-            # an output beyond the experts that have weights is in nobody's list
-            lists, counts = ops.expert_lists(None, chosen, T, self.experts)
             on_input = self.weight_on == "input"
             bounded = (self.bound, self.slope, self.offset) if self.activation == "bounded_glu" else None
-            if self.partial_ok and not self.identity and not self.shared_gated:
-                a = ops.grouped_linear(x, self.gate_up, lists, counts, T, per_token=True,
-                                       out_dtype=x.dtype, bounded=bounded,
-                                       gate=None if bounded else self.activation,
-                                       row_weight=weight if on_input else None)
+            # (where the rows are combined by a kernel of its own the gate reads the product's columns
+            # rounded to the run's type)
+            planes = self.sums_as_planes()
+            a = ops.grouped_linear(x, self.gate_up, *lists, T, per_token=True, out_dtype=x.dtype,
+                                   bounded=bounded, gate=None if bounded else self.activation,
+                                   row_weight=weight if on_input else None, rounded=not planes)
+            if planes:
                 planes = self.top + (self.shared_gate_up is not None)
                 out = torch.empty((planes, T, self.down.shape[1]), dtype=torch.float32, device=x.device)
-                ops.grouped_linear(a, self.down, lists, counts, T, per_token=False, stacked=True,
+                ops.grouped_linear(a, self.down, *lists, T, per_token=False, stacked=True,
                                    out=out[:self.top], row_weight=None if on_input else weight)
                 if self.shared_gate_up is not None:
                     self._shared(x, into=out[self.top])
                 return out
-            # (where the rows are combined by a kernel of its own the gate has one, too: the
-            # product's columns are rounded to the run's type in between)
-            a = ops.grouped_linear(x, self.gate_up, lists, counts, T, per_token=True,
-                                   out_dtype=x.dtype)
-            if bounded:
-                a = ops.clamped_glu(a, *bounded, weight if on_input else None)
-            else:
-                a = ops.gated_unit(a, self.activation)
-            out = ops.grouped_linear(a, self.down, lists, counts, T, per_token=False,
-                                     out_dtype=torch.float32)
+            out = ops.grouped_linear(a, self.down, *lists, T, per_token=False, out_dtype=torch.float32)
         shared = self._shared(x) if self.shared_gate_up is not None else None
         return ops.experts_combine(out, chosen, weight, x, self.experts, shared,
                                    logits if self.shared_gated else None, self.outputs,
-                                   weigh=self.weight_on == "output")
+                                   weigh=self.weight_on == "output", stream=stream,
+                                   stream_scale=stream_scale, copy_dtype=copy_dtype)
+
+    def sums_as_planes(self) -> bool:
+        return bool(self.experts and self.partial_ok and not self.identity and not self.shared_gated)
+
+    @property
+    def adds_scaled(self) -> bool:
+        """Whether ``forward`` takes the stream and a weight and adds its result itself."""
+        return not self.sums_as_planes()
 
     def _shared(self, x, into=None):
         """The shared expert's result, 32-bit."""

@@ -101,6 +101,7 @@ class TokenSide(Part):
     kind = "token_side"
     graph_safe = True
     needs_origin = False
+    reads_rounded = True      # takes the block's rounded copy of the stream where there is one
     kernel_sources = ("norm", "gemm", "gemm_rows64", "activation")
 
     @classmethod
@@ -136,7 +137,10 @@ class TokenSide(Part):
             raise ValueError(f"layer {layer} of {self.layers}")
         if pending is not None:
             ops.stream_add_(residual, pending)
-        x = ops.cast(residual, self.runtime.dtype)
+            step.rounded = None
+        x, step.rounded = step.rounded, None
+        if x is None:
+            x = ops.cast(residual, self.runtime.dtype)
         g = ops.table_gate(ops.linear(x, self.gate[i], tune=self.runtime.tune), step.token_ids,
                            self.table, i * self.dim, self.activation)
         y = ops.linear(g, self.proj[i], out_dtype=torch.float32, tune=self.runtime.tune)

@@ -15,9 +15,7 @@
 //
 // A workgroup serves one work item (up to `count` consecutive query tokens of one
 // request) and one key/value head, so a tile of keys staged in LDS is shared by
-// every query head of the group and every token of the item.  Rows (token, head)
-// are dealt to the four waves; in the score phase a lane owns a key, in the
-// value phase it owns head-dimension elements.  Long contexts may be cut into
+// every query head of the group and every token of the item.  Long contexts may be cut into
 // `nsplit` ranges of `keys_per_split` keys whose partial (m, l, accumulator) are
 // merged by `attention_combine_kernel`; the cut points depend on key positions
 // only.
@@ -64,11 +62,37 @@ __device__ __forceinline__ float shaped_score_log2(const ScoreExtras& ex, float 
   return dot * r.a;
 }
 
-#define AT_WAVES 4
-#define AT_RPW 8                     // rows per wave, at most
-#define AT_MAX_ROWS (AT_WAVES * AT_RPW)
+#define AT_MAX_ROWS 32
+#define AT_KT 64                     // keys of a tile, a quarter a wave
 
-template <typename T, int KT>
+// The general kernel: both storage types, any sizes, both products on the matrix cores' 32-bit
+// instruction (v_mfma_f32_16x16x4_f32; its layout in gemm_f32.h), everything in 32-bit.  A work item has
+// up to 32 rows (token, head), two blocks of 16; a tile's 64 keys are dealt to the four waves, 16 each,
+// and a wave keeps maxima, sums and accumulators of its own for all rows:
+//   S^T = K Q^T    queries in registers, keys from LDS; a lane has four keys of one row
+//   O^T += V^T P^T the probabilities go from the accumulator straight into the second operand
+// The waves' parts meet in LDS at the end, in the waves' order: a row's result depends on the places of
+// its keys only.  The next tile is on its way from memory while one is computed.
+// 448 rows of three prompts up to 150 tokens, 16 heads of 64 over 8, 32-bit: 115 us on the vector unit
+// with two reads of LDS a product, 29 here; three of 1,000 tokens 1,052 and 303; heads of 128 over 500
+// tokens 772 and 151, of 256 1,928 and 400; one row a request at 2,000 keys 216 and 143 (a chain of 32
+// tiles there: pages, keys, scores, weights).
+// NC: blocks of 16 channels of keys and of values, at most (4, 8 or 16).
+template <typename T> __device__ __forceinline__ f32x4_t at_load4(const T* p);
+template <> __device__ __forceinline__ f32x4_t at_load4<float>(const float* p) {
+  return *reinterpret_cast<const f32x4_t*>(p);
+}
+template <> __device__ __forceinline__ f32x4_t at_load4<bf16_t>(const bf16_t* p) {
+  const bf16x4_t v = *reinterpret_cast<const bf16x4_t*>(p);
+  return f32x4_t{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+}
+
+template <int NC>
+constexpr size_t at_lds() {        // floats: a tile's keys and values, then the waves' results
+  return (size_t)AT_KT * (NC * 16 + 4) + (size_t)NC * 16 * (AT_KT + 4);
+}
+
+template <typename T, int NC>
 __global__ void __launch_bounds__(256)
 paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __restrict__ kv,
                        const int* __restrict__ block_table, int bt_stride,
@@ -83,17 +107,19 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
   // `gate`: when given, head h of token t is multiplied by
   // sigmoid(gate[t * gate_stride + gate_col + h]) * out_scale; with `gate_elem` every
   // element dd of it by its own sigmoid(gate[t * gate_stride + gate_col + h * dv + dd]).
-  extern __shared__ float smem[];
-  const int ldk = d + 1, ldv = dv + 1;
+  constexpr int LDK = NC * 16 + 4, LDV = AT_KT + 4;   // (16 rows read together: different banks)
+  constexpr bool AHEAD = NC < 16;         // (256 channels leave no registers for the next tile)
+  static_assert(4 * AT_MAX_ROWS * LDK <= at_lds<NC>(), "the waves' results take the tile's place");
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  __shared__ float wave_m[4][AT_MAX_ROWS], wave_l[4][AT_MAX_ROWS];
   const size_t page_elems = (size_t)nkv * page_size * (d + dv);
   const size_t value_base = (size_t)nkv * page_size * d;
-  float* Ks = smem;                       // [KT][d + 1]
-  float* Vs = Ks + KT * ldk;              // [KT][dv + 1]
-  float* Qs = Vs + KT * ldv;              // [AT_MAX_ROWS][d]
-  float* Ps = Qs + AT_MAX_ROWS * d;       // [AT_WAVES][64]
+  float* Ks = smem;                       // [key][channel]
+  float* Vt = Ks + AT_KT * LDK;           // [channel][key]
 
   const int item = blockIdx.x, g = blockIdx.y, z = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, quarter = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int G = nh / nkv;
   const int seq = wi_seq[item];
   const int row0 = wi_row0[item];
@@ -101,6 +127,8 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
   if (count * G > AT_MAX_ROWS) count = AT_MAX_ROWS / G;  // the host never asks for more
   const int rows = count * G;
   const int* table = block_table + (size_t)seq * bt_stride;
+  const int shift = page_shift_of(page_size);
+  const bool fours = page_size % 4 == 0;  // four neighbouring keys of a tile share a page
 
   const int pos_first = positions[row0];
   const int pos_last = positions[row0 + count - 1];
@@ -111,152 +139,221 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
   int range_hi = range_lo + keys_per_split - 1;
   if (nsplit == 1) { range_lo = 0; range_hi = hi; }
   if (range_hi > hi) range_hi = hi;
-  int tile_first = (lo / KT) * KT;
+  int tile_first = (lo / AT_KT) * AT_KT;
   if (tile_first < range_lo) tile_first = range_lo;
   // kept first keys: their tiles come first, then the walk goes on at the window's
-  const int kept_end = lo > 0 ? (ex.keep + KT - 1) / KT * KT : 0;
-  const int start = kept_end > range_lo ? range_lo : tile_first;
+  const int kept_end = lo > 0 ? (ex.keep + AT_KT - 1) / AT_KT * AT_KT : 0;
+  auto next_tile = [&](int t) { return t >= kept_end && t < tile_first ? tile_first : t; };
+  auto there = [&](int kp) { return (kp >= lo || kp < ex.keep) && kp <= range_hi; };
 
-  // queries of this item, as floats
-  for (int idx = tid; idx < rows * d; idx += 256) {
-    const int r = idx / d, dd = idx % d;
-    const int tok = row0 + r / G, h = g * G + r % G;
-    Qs[r * d + dd] = to_f32<T>(q[((size_t)tok * nh + h) * d + dd]);
-  }
-
-  float m[AT_RPW], l[AT_RPW], acc[AT_RPW][AT_DPL];
+  // this lane's rows: their positions and queries (some row's where there is none)
+  int pos[2];
+  f32x4_t qf[2][NC];
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < AT_RPW; ++i) {
-    m[i] = -INFINITY;
-    l[i] = 0.f;
+  for (int rt = 0; rt < 2; ++rt) {
+    const int r = min(rt * 16 + r16, rows - 1), tok = row0 + r / G;
+    pos[rt] = positions[tok];
+    const T* from = q + ((size_t)tok * nh + g * G + r % G) * d;
 #pragma unroll
-    for (int c = 0; c < AT_DPL; ++c) acc[i][c] = 0.f;
+    for (int c = 0; c < NC; ++c) {
+      const int at = 16 * c + 4 * quarter;
+      qf[rt][c] = at < d ? at_load4<T>(from + at) : zero;
+    }
   }
+  const float temper[2] = {query_temperature(ex, pos[0]), query_temperature(ex, pos[1])};
 
-  const int vec_per_row = d / 8;
-  for (int tile0 = start; tile0 <= range_hi; tile0 += KT) {
-    if (tile0 >= kept_end && tile0 < tile_first) tile0 = tile_first;
-    if (tile0 > range_hi) break;
-    __syncthreads();  // previous tile fully consumed (and Qs written, first time)
-    for (int idx = tid; idx < KT * vec_per_row; idx += 256) {
-      const int j = idx / vec_per_row, c = (idx % vec_per_row) * 8;
-      const int kp = tile0 + j;
-      float kx[8];
-      bool ok = (kp >= lo || kp < ex.keep) && kp <= range_hi;
-      int page = -1;
-      if (ok) {
-        page = table[kp / page_size];
-        ok = page >= 0;
-      }
-      if (ok) {
-        load8<T>(kv + page * page_elems + ((size_t)g * page_size + kp % page_size) * d + c, kx);
+  f32x4_t rk[NC], rv[NC];
+  // (pages first, then what lies on them, every request unconditional, some valid place's where there
+  // is nothing: behind conditions each would wait for its own page; pages a tile further ahead gained
+  // nothing)
+  auto page_of = [&](int kp) { return table[page_entry(min(kp, range_hi), page_size, shift)]; };
+  auto fetch_keys = [&](int tile0) {
+    int page[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) page[i] = page_of(tile0 + (tid + 256 * i) / (4 * NC));
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int v = tid + 256 * i, kp = tile0 + v / (4 * NC), c = v % (4 * NC) * 4;
+      rk[i] = at_load4<T>(kv + max(page[i], 0) * page_elems +
+                          ((size_t)g * page_size + page_offset(kp, page_size, shift)) * d + (c < d ? c : 0));
+      if (!(c < d && there(kp) && page[i] >= 0)) rk[i] = zero;
+    }
+  };
+  auto fetch_values = [&](int tile0) {
+    int page[NC];
+    if (fours) {
+#pragma unroll
+      for (int i = 0; i < NC; ++i) page[i] = page_of(tile0 + ((tid + 256 * i) & 15) * 4);
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int v = tid + 256 * i, dd = v >> 4, kp = tile0 + (v & 15) * 4;
+      if (fours) {
+        rv[i] = at_load4<T>(kv + max(page[i], 0) * page_elems + value_base +
+                            ((size_t)g * dv + (dd < dv ? dd : 0)) * page_size + page_offset(kp, page_size, shift));
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (!(dd < dv && there(kp + e) && page[i] >= 0)) rv[i][e] = 0.f;
       } else {
+        rv[i] = zero;
+        if (dd >= dv) continue;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) kx[i] = 0.f;
+        for (int e = 0; e < 4; ++e)
+          if (there(kp + e)) {
+            const int page = table[(kp + e) / page_size];
+            if (page >= 0)
+              rv[i][e] = to_f32<T>(kv[page * page_elems + value_base + ((size_t)g * dv + dd) * page_size +
+                                      (kp + e) % page_size]);
+          }
       }
+    }
+  };
+
+  auto stash_keys = [&]() {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) Ks[j * ldk + c + i] = kx[i];
+    for (int i = 0; i < NC; ++i) {
+      const int v = tid + 256 * i;
+      *reinterpret_cast<f32x4_t*>(&Ks[v / (4 * NC) * LDK + v % (4 * NC) * 4]) = rk[i];
     }
-    {
-      // values: a thread keeps one key of the tile (256 is a multiple of KT) and walks
-      // the head dimension, so the lanes of a wave read consecutive offsets of a page
-      const int j = tid % KT;
-      const int kp = tile0 + j;
-      const T* vsrc = nullptr;
-      if ((kp >= lo || kp < ex.keep) && kp <= range_hi) {
-        const int page = table[kp / page_size];
-        if (page >= 0)
-          vsrc = kv + page * page_elems + value_base + (size_t)g * dv * page_size + kp % page_size;
-      }
-      for (int dd = tid / KT; dd < dv; dd += 256 / KT)
-        Vs[j * ldv + dd] = vsrc ? to_f32<T>(vsrc[(size_t)dd * page_size]) : 0.f;
+  };
+  auto stash_values = [&]() {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int v = tid + 256 * i;
+      *reinterpret_cast<f32x4_t*>(&Vt[(v >> 4) * LDV + (v & 15) * 4]) = rv[i];
     }
+  };
+
+  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};     // l: of this lane's keys
+  f32x4_t acc[2][NC];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[rt][c] = zero;
+
+  int tile0 = next_tile(kept_end > range_lo ? range_lo : tile_first);
+  if (AHEAD && tile0 <= range_hi) {
+    fetch_keys(tile0);
+    fetch_values(tile0);
+  }
+  while (tile0 <= range_hi) {
+    __syncthreads();  // the tile before has been read
+    if (!AHEAD) fetch_keys(tile0);
+    stash_keys();
+    if (!AHEAD) fetch_values(tile0);
+    stash_values();
     __syncthreads();
-
+    const int key0 = tile0 + wave * 16 + quarter * 4;          // this lane's four keys
+    const int next = next_tile(tile0 + AT_KT);
+    if (AHEAD && next <= range_hi) {
+      fetch_keys(next);
+      fetch_values(next);
+    }
+    if (tile0 + wave * 16 <= range_hi) {
+      f32x4_t s[2] = {zero, zero};
 #pragma unroll
-    for (int lr = 0; lr < AT_RPW; ++lr) {
-      const int r = wave + AT_WAVES * lr;
-      if (r < rows) {
-        const int pos = positions[row0 + r / G];
-        const int kp = tile0 + lane;
-        bool valid = kp >= lo;
-        if (window > 0 && kp <= pos - window) valid = false;
-        if (kp < chunk_start(ex, pos)) valid = false;
-        valid = (valid || kp < ex.keep) && lane < KT && kp <= pos && kp <= range_hi;
-        float s = -INFINITY;
-        if (lane < KT) {
-          const float* qr = Qs + r * d;
-          const float* kr = Ks + lane * ldk;
-          float dot = 0.f;
-          for (int dd = 0; dd < d; ++dd) dot = fmaf(qr[dd], kr[dd], dot);
-          if (valid) s = capped_score(ex, dot * query_temperature(ex, pos) * scale);
+      for (int c = 0; c < NC; ++c) {
+        if (16 * c >= d) break;
+        const f32x4_t k = *reinterpret_cast<const f32x4_t*>(&Ks[(wave * 16 + r16) * LDK + 16 * c + 4 * quarter]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], qf[0][c][e], s[0], 0, 0, 0);
+          if (rows > 16) s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], qf[1][c][e], s[1], 0, 0, 0);
         }
-        const float tmax = wave_max(s);
-        const float m_new = fmaxf(m[lr], tmax);
-        if (m_new > -INFINITY) {
-          const float alpha = expf(m[lr] - m_new);
-          const float p = valid ? expf(s - m_new) : 0.f;
-          l[lr] = l[lr] * alpha + wave_sum(p);
-          m[lr] = m_new;
-          __builtin_amdgcn_wave_barrier();
-          Ps[wave * 64 + lane] = p;
-          __builtin_amdgcn_wave_barrier();
+      }
 #pragma unroll
-          for (int c = 0; c < AT_DPL; ++c) {
-            const int dd = lane + 64 * c;
-            if (64 * c < dv) {
-              float a = acc[lr][c] * alpha;
-              if (dd < dv) {
-#pragma unroll 8
-                for (int j = 0; j < KT; ++j) a = fmaf(Ps[wave * 64 + j], Vs[j * ldv + dd], a);
-              }
-              acc[lr][c] = a;
-            }
-          }
-          __builtin_amdgcn_wave_barrier();
+      for (int rt = 0; rt < 2; ++rt) {
+        if (rt * 16 >= rows) break;
+        bool valid[4];
+        float top = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int kp = key0 + e;
+          valid[e] = kp >= lo;
+          if (window > 0 && kp <= pos[rt] - window) valid[e] = false;
+          if (kp < chunk_start(ex, pos[rt])) valid[e] = false;
+          valid[e] = (valid[e] || kp < ex.keep) && kp <= pos[rt] && kp <= range_hi;
+          s[rt][e] = valid[e] ? capped_score(ex, s[rt][e] * temper[rt] * scale) : -INFINITY;
+          top = fmaxf(top, s[rt][e]);
+        }
+        const float m_new = fmaxf(m[rt], quad_max(top));
+        // (no key yet: nothing to rescale, and no difference of infinities)
+        const float alpha = m_new > -INFINITY ? expf(m[rt] - m_new) : 1.f;
+        float own = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          s[rt][e] = valid[e] ? expf(s[rt][e] - m_new) : 0.f;
+          own += s[rt][e];
+        }
+        l[rt] = l[rt] * alpha + own;
+        m[rt] = m_new;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[rt][c] *= alpha;
+      }
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        if (16 * c >= dv) break;
+        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&Vt[(16 * c + r16) * LDV + wave * 16 + 4 * quarter]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          acc[0][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], s[0][e], acc[0][c], 0, 0, 0);
+          if (rows > 16) acc[1][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], s[1][e], acc[1][c], 0, 0, 0);
         }
       }
     }
+    tile0 = next;
   }
 
+  // ---- the waves' parts together
 #pragma unroll
-  for (int lr = 0; lr < AT_RPW; ++lr) {
-    const int r = wave + AT_WAVES * lr;
-    if (r < rows) {
-      const int tok = row0 + r / G, h = g * G + r % G;
-      if (nsplit == 1) {
-        if (ex.sink) l[lr] += expf(ex.sink[h] - m[lr]);
-        const float inv = l[lr] > 0.f ? 1.0f / l[lr] : 0.f;
-        float mult = 1.0f;
-        if (gate && !gate_elem) {
-          const float gl = to_f32<T>(gate[(size_t)tok * gate_stride + gate_col + h]);
-          mult = out_scale / (1.0f + expf(-gl));
-        }
-        T* o = out + ((size_t)tok * nh + h) * dv;
+  for (int rt = 0; rt < 2; ++rt) {
+    const float sum = quad_sum(l[rt]);
+    if (quarter == 0) {
+      wave_m[wave][rt * 16 + r16] = m[rt];
+      wave_l[wave][rt * 16 + r16] = sum;
+    }
+  }
+  __syncthreads();      // (and the last tile has been read)
 #pragma unroll
-        for (int c = 0; c < AT_DPL; ++c) {
-          const int dd = lane + 64 * c;
-          if (dd < dv) {
-            if (gate && gate_elem) {
-              const float gl =
-                  to_f32<T>(gate[(size_t)tok * gate_stride + gate_col + (size_t)h * dv + dd]);
-              mult = out_scale / (1.0f + expf(-gl));
-            }
-            o[dd] = from_f32<T>(gate ? acc[lr][c] * inv * mult : acc[lr][c] * inv);
-          }
-        }
-      } else {
-        const size_t pidx = ((size_t)tok * nh + h) * nsplit + z;
-        float* pa = part_acc + pidx * dv;
+  for (int rt = 0; rt < 2; ++rt) {
+    if (rt * 16 >= rows) break;
+    const int r = rt * 16 + r16;
+    const float top = fmaxf(fmaxf(wave_m[0][r], wave_m[1][r]), fmaxf(wave_m[2][r], wave_m[3][r]));
+    const float f = m[rt] > -INFINITY ? expf(m[rt] - top) : 0.f;
 #pragma unroll
-        for (int c = 0; c < AT_DPL; ++c) {
-          const int dd = lane + 64 * c;
-          if (dd < dv) pa[dd] = acc[lr][c];
-        }
-        if (lane == 0) {
-          part_ml[pidx * 2] = m[lr];
-          part_ml[pidx * 2 + 1] = l[lr];
-        }
+    for (int c = 0; c < NC; ++c)
+      if (16 * c < dv)
+        *reinterpret_cast<f32x4_t*>(&smem[(wave * AT_MAX_ROWS + r) * LDK + 16 * c + 4 * quarter]) = acc[rt][c] * f;
+  }
+  __syncthreads();
+  for (int idx = tid; idx < rows * dv; idx += 256) {
+    const int r = idx / dv, dd = idx - r * dv;
+    const int tok = row0 + r / G, h = g * G + r % G;
+    float top = wave_m[0][r];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) top = fmaxf(top, wave_m[w][r]);
+    float total = 0.f, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      total += wave_m[w][r] > -INFINITY ? wave_l[w][r] * expf(wave_m[w][r] - top) : 0.f;
+      sum += smem[(w * AT_MAX_ROWS + r) * LDK + dd];
+    }
+    if (nsplit == 1) {
+      if (ex.sink) total += expf(ex.sink[h] - top);
+      sum *= total > 0.f ? 1.0f / total : 0.f;
+      if (gate) {
+        const size_t col = gate_elem ? (size_t)h * dv + dd : (size_t)h;
+        const float gl = to_f32<T>(gate[(size_t)tok * gate_stride + gate_col + col]);
+        sum *= out_scale / (1.0f + expf(-gl));
+      }
+      out[((size_t)tok * nh + h) * dv + dd] = from_f32<T>(sum);
+    } else {
+      const size_t pidx = ((size_t)tok * nh + h) * nsplit + z;
+      part_acc[pidx * dv + dd] = sum;
+      if (dd == 0) {
+        part_ml[pidx * 2] = top;
+        part_ml[pidx * 2 + 1] = total;
       }
     }
   }
@@ -1071,7 +1168,7 @@ paged_attention_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restr
   }
 }
 
-template <typename T, int KT>
+template <typename T, int NC>
 static int launch_attention(const void* q, void* out, const void* kv, const int* block_table,
                             int bt_stride, const int* positions, const int* wi_seq,
                             const int* wi_row0, const int* wi_count, int n_items, float* part_acc,
@@ -1079,16 +1176,11 @@ static int launch_attention(const void* q, void* out, const void* kv, const int*
                             int window, int keys_per_split, int nsplit, int dv, const void* gate,
                             int gate_stride, int gate_col, float out_scale, ScoreExtras ex,
                             int gate_elem, hipStream_t stream) {
-  const size_t shmem = ((size_t)KT * (d + 1) + (size_t)KT * (dv + 1) + (size_t)AT_MAX_ROWS * d +
-                        AT_WAVES * 64) * sizeof(float);
-  auto kernel = paged_attention_kernel<T, KT>;
-  static size_t allowed = 0;
-  if (shmem > allowed) {
-    hipError_t e = hipFuncSetAttribute((const void*)kernel,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
-    if (e != hipSuccess) return (int)e;
-    allowed = shmem;
-  }
+  constexpr size_t shmem = at_lds<NC>() * sizeof(float);
+  auto kernel = paged_attention_kernel<T, NC>;
+  static const hipError_t allowed = hipFuncSetAttribute(
+      (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+  if (allowed != hipSuccess) return (int)allowed;
   dim3 grid(n_items, nkv, nsplit), block(256);
   hipLaunchKernelGGL(kernel, grid, block, shmem, stream, (const T*)q, (T*)out, (const T*)kv,
                      block_table, bt_stride, positions, wi_seq, wi_row0, wi_count, part_acc,
@@ -1234,12 +1326,13 @@ static int paged_attention_any(const void* q, void* out, const void* kv, const i
   q, out, kv, block_table, bt_stride, positions, wi_seq, wi_row0, wi_count, n_items, part_acc, \
       part_ml, nh, nkv, d, page_size, scale, window, keys_per_split, nsplit, dv, gate,         \
       gate_stride, gate_col, out_scale, ex, gate_elem, stream
-  const bool small = d <= 128 && dv <= 128;
+  const int wide = d > dv ? d : dv;
   if (dtype == 0) {
-    rc = small ? launch_attention<float, 64>(ZA_AT_ARGS) : launch_attention<float, 32>(ZA_AT_ARGS);
+    rc = wide <= 64 ? launch_attention<float, 4>(ZA_AT_ARGS)
+         : wide <= 128 ? launch_attention<float, 8>(ZA_AT_ARGS) : launch_attention<float, 16>(ZA_AT_ARGS);
   } else if (dtype == 1) {
-    rc = small ? launch_attention<bf16_t, 64>(ZA_AT_ARGS)
-                  : launch_attention<bf16_t, 32>(ZA_AT_ARGS);
+    rc = wide <= 64 ? launch_attention<bf16_t, 4>(ZA_AT_ARGS)
+         : wide <= 128 ? launch_attention<bf16_t, 8>(ZA_AT_ARGS) : launch_attention<bf16_t, 16>(ZA_AT_ARGS);
   } else {
     return ZA_ERR_UNSUPPORTED;
   }

@@ -81,6 +81,7 @@ from .feed_forward import fuse_rows, pad_rows
 # eight waves a compute unit) are best or within a few percent of it, all of the same length.
 BUSY_WORKGROUPS = 512
 SPLIT_TARGET = 256
+PLANES_PORTION_TARGET = 400
 SPLIT_KEYS_MIN = 512
 SPLIT_MAX = 64
 
@@ -521,7 +522,7 @@ class GroupedQueryAttention(Mixer):
                 items = step.attention_items(self.planes_rows_per_item)
             # (an item's list of tiles is cut, not the context: behind a window it stays short)
             tiles, nsplit = self._plan_tiles(items[3] if items else step.n_seqs,
-                                             self._reach(step.max_keys))
+                                             self._reach(step.max_keys), items is not None)
             o = ops.planes_attention(q, key_plane, value_plane, table, step.positions, items,
                                      self.scale, self.window, tiles, nsplit, shape=self.shape)
         else:
@@ -544,11 +545,15 @@ class GroupedQueryAttention(Mixer):
                 max_keys = min(max_keys, limit + self.keep_first)
         return max_keys
 
-    def _plan_tiles(self, n_items: int, keys: int):
-        """``plan_split`` in tiles of the kernel.  (Prompt portions too are cut only up to one
-        workgroup a compute unit: 2,048 tokens of 16 heads on 4 key heads behind a window of
-        1,024, 36.7 us whole, 45.1 in two ranges; 512 tokens 35.2 whole, 24.6 in four.)"""
-        per_range, nsplit = plan_split(n_items, self.num_kv_heads, keys)
+    def _plan_tiles(self, n_items: int, keys: int, portions: bool):
+        """``plan_split`` in tiles of the kernel.  (Prompt portions are cut while that stays within
+        400 workgroups, three for two compute units: an item's walk over its tiles is a chain, and two
+        of them on a compute unit hide each other's waits, but the ranges have to be merged.  Steps of 862 to
+        1,029 tokens of 16 heads on 4 key heads behind a window of 1,024, 132 to 148 workgroups whole:
+        a step's time whole 4,239 us, cut for 320 workgroups 4,150, for 400 4,084, for 511 4,097.
+        2,048 tokens, 256 workgroups: 36.7 us whole, 45.1 in two ranges.)"""
+        per_range, nsplit = plan_split(n_items, self.num_kv_heads, keys,
+                                       **({"target": PLANES_PORTION_TARGET} if portions else {}))
         return -(-per_range // ops.PLANES_TILE_KEYS), nsplit
 
     def _leave_taps(self, step, cache, q: torch.Tensor, o: torch.Tensor) -> None:

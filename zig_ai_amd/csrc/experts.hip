@@ -396,7 +396,8 @@ grouped_gemm_bf16_wide_kernel(GroupedArgs g) {
 #define GF_BM 32
 #define GF_BN 64
 
-template <typename TA, typename TO, bool GATED, bool VEC>
+// VEC: 0 an element at a time, 1 four, 2 (32-bit rows, K a multiple of 32) through LDS without registers.
+template <typename TA, typename TO, bool GATED, int VEC>
 __global__ void __launch_bounds__(512)
 grouped_gemm_f32_kernel(GroupedArgs g) {
   int e, tile, count;
@@ -406,31 +407,32 @@ grouped_gemm_f32_kernel(GroupedArgs g) {
   const int K = g.K, N = g.N;
   const float* W = (const float*)g.W + (size_t)e * (GATED ? 2 * N : N) * K;
   TO* out = (TO*)g.out;
-  f32_tile<TA, GF_BM, GF_BN, 2, VEC>(
-      K, [&](int r) { return (const TA*)g.src + (size_t)(mine[min(m0 + r, count - 1)] / g.src_div) * K; },
-      [&](int r) {
-        const int n = min(n0 + (GATED ? (r >> 5) * 16 + (r & 15) : r), N - 1);
-        return W + (size_t)(n + (GATED && (r & 16) ? N : 0)) * K;
-      },
-      [&](int r, int n, const f32x4_t(&v)[GF_BN / 32]) {
-        if (m0 + r >= count) return;
-        const int a = mine[m0 + r];
-        TO* at = out + dst_row(g, a) * N;
-        const float w = g.row_weight ? g.row_weight[a] : 1.0f;
-        if constexpr (GATED) {
-          const int first = n0 + (n >> 5) * 16 + (n & 15);
+  auto a_at = [&](int r) { return (const TA*)g.src + (size_t)(mine[min(m0 + r, count - 1)] / g.src_div) * K; };
+  auto w_at = [&](int r) {
+    const int n = min(n0 + (GATED ? (r >> 5) * 16 + (r & 15) : r), N - 1);
+    return W + (size_t)(n + (GATED && (r & 16) ? N : 0)) * K;
+  };
+  auto store = [&](int r, int n, const f32x4_t(&v)[GF_BN / 32]) {
+    if (m0 + r >= count) return;
+    const int a = mine[m0 + r];
+    TO* at = out + dst_row(g, a) * N;
+    const float w = g.row_weight ? g.row_weight[a] : 1.0f;
+    if constexpr (GATED) {
+      const int first = n0 + (n >> 5) * 16 + (n & 15);
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (first + i < N) at[first + i] = from_f32<TO>(expert_unit<TO>(g, v[0][i], v[1][i], w));
-        } else {
+      for (int i = 0; i < 4; ++i)
+        if (first + i < N) at[first + i] = from_f32<TO>(expert_unit<TO>(g, v[0][i], v[1][i], w));
+    } else {
 #pragma unroll
-          for (int j = 0; j < GF_BN / 32; ++j)
+      for (int j = 0; j < GF_BN / 32; ++j)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (n0 + n + j * 16 + i < N)
-                at[n0 + n + j * 16 + i] = from_f32<TO>(expert_act(v[j][i], g.act) * g.out_scale * w);
-        }
-      });
+        for (int i = 0; i < 4; ++i)
+          if (n0 + n + j * 16 + i < N)
+            at[n0 + n + j * 16 + i] = from_f32<TO>(expert_act(v[j][i], g.act) * g.out_scale * w);
+    }
+  };
+  if constexpr (VEC == 2) f32_tile_async<GF_BM, GF_BN, 2, 3>(K, a_at, w_at, store);
+  else f32_tile<TA, GF_BM, GF_BN, 2, VEC == 1>(K, a_at, w_at, store);
 }
 
 // dtype codes: 0 = float32, 1 = bfloat16.  `src` has `src_rows` rows of K elements; the
@@ -526,10 +528,17 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
   const int columns = gate ? GF_BN / 2 : GF_BN;
   dim3 grid((unsigned)((A + GF_BM - 1) / GF_BM + experts), (unsigned)((N + columns - 1) / columns)), block(512);
   const bool vec = K % 4 == 0 && (uintptr_t)src % (src_dtype == 1 ? 8 : 16) == 0 && (uintptr_t)W % 16 == 0;
+  const bool whole = vec && src_dtype == 0 && K % F32_BK == 0;
 #define ZA_GFV(TA, TO, GATED)                                                                              \
   {                                                                                                        \
-    if (vec) hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, GATED, true>), grid, block, 0, stream, g); \
-    else hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, GATED, false>), grid, block, 0, stream, g);    \
+    if constexpr (std::is_same<TA, float>::value) {                                                        \
+      if (whole) {                                                                                         \
+        hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, GATED, 2>), grid, block, 0, stream, g);        \
+        return za_launch_status();                                                                         \
+      }                                                                                                    \
+    }                                                                                                      \
+    if (vec) hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, GATED, 1>), grid, block, 0, stream, g);   \
+    else hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, GATED, 0>), grid, block, 0, stream, g);       \
   }
 #define ZA_GF(TA, TO)                 \
   {                                   \

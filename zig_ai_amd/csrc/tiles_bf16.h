@@ -21,18 +21,6 @@
 
 #define GG_BK 64
 
-__device__ __forceinline__ unsigned lds_address(const void* p) {
-  return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
-// The wait for all but the last n requests to memory.
-#define ZA_VMCNT(n) (((n) & 15) | (7 << 4) | (15 << 8) | (((n) >> 4) << 14))
-
-__device__ __forceinline__ void lds_request(const bf16_t* from, bf16_t* to) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
-                                   (__attribute__((address_space(3))) void*)to, 16, 0, 0);
-}
-
 template <int BM, int BN, int NS>
 struct TilesBf16 {
   static constexpr int WM = BM >= 64 || BN == 64 ? 2 : 1, WN = 4 / WM;   // waves along the rows of A and of W

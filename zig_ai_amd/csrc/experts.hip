@@ -250,15 +250,15 @@ grouped_gemm_bf16_tiled_kernel(GroupedArgs g) {
   __shared__ __attribute__((aligned(16))) bf16_t As[NS][BM * GG_BK];
   __shared__ __attribute__((aligned(16))) bf16_t Ws[NS][BN * GG_BK];
   int e, tile, count;
-  // workgroups are dealt to the eight dies in turn: a die takes an eighth of the tiles, side by
-  // side, for one stretch of outputs after the other, and finds the rows of its assignments and
-  // the weights that an expert's tiles share in its cache
-  const int per_die = (count_tiles<BM>(g.counts, g.E) + 7) >> 3, at = blockIdx.x >> 3;
-  if (per_die == 0) return;
-  const int n0 = (at / per_die) * (GATED ? BN / 2 : BN);
-  if (n0 >= g.N ||
-      !find_tile<BM>(g.counts, g.E, (blockIdx.x & 7) * per_die + at % per_die, &e, &tile, &count))
-    return;
+  // workgroups are dealt to the eight dies in turn: a die takes an eighth of all tiles and stretches
+  // of outputs, a tile's stretches side by side, so that few tiles (a decode batch's experts) keep
+  // every die busy: with an eighth of the tiles each, nine tiles took five dies twice, two tiles two
+  const int columns = (g.N + (GATED ? BN / 2 : BN) - 1) / (GATED ? BN / 2 : BN);
+  const int total = count_tiles<BM>(g.counts, g.E) * columns, per_die = (total + 7) >> 3;
+  const int at = blockIdx.x >> 3, index = (blockIdx.x & 7) * per_die + at;
+  if (at >= per_die || index >= total) return;
+  const int n0 = (index % columns) * (GATED ? BN / 2 : BN);
+  if (!find_tile<BM>(g.counts, g.E, index / columns, &e, &tile, &count)) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave % WM) * (BM / WM), wn = (wave / WM) * (BN / WN);

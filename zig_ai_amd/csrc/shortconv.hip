@@ -186,6 +186,68 @@ short_conv_kernel(const T* __restrict__ z, const float* __restrict__ w,
   }
 }
 
+// A step of single tokens whose in_proj came as 32-bit sums over `ranges` ranges of K, [ranges][token]
+// [3 width]: added up in order and rounded as in_proj stores them, then the head's operations.  One
+// thread per (token, channel); everything requested before the first wait.
+template <typename T, int R>
+__global__ void __launch_bounds__(256)
+short_conv_ranges_kernel(const float* __restrict__ z, const float* __restrict__ w, const float* __restrict__ bias,
+                         float* __restrict__ state, const int* __restrict__ slot_id, T* __restrict__ y, int width,
+                         int L, long long slot_stride, size_t range_stride) {
+  const int t = blockIdx.y, ch = blockIdx.x * 256 + threadIdx.x;
+  if (ch >= width) return;
+  float part[3][R], wt[SC_MAX_L], hist[SC_MAX_L];
+  const float* zr = z + (size_t)t * 3 * width + ch;
+#pragma unroll
+  for (int b = 0; b < 3; ++b)
+#pragma unroll
+    for (int r = 0; r < R; ++r) part[b][r] = zr[r * range_stride + (size_t)b * width];
+#pragma unroll
+  for (int j = 0; j < SC_MAX_L; ++j) wt[j] = j < L ? w[(size_t)j * width + ch] : 0.f;
+  float* st = state + (size_t)slot_id[t] * (size_t)slot_stride + (size_t)ch * L;
+#pragma unroll
+  for (int j = 0; j < SC_MAX_L; ++j) hist[j] = j < L ? st[j] : 0.f;
+  float c = bias ? bias[ch] : 0.f;
+  float v[3];
+#pragma unroll
+  for (int b = 0; b < 3; ++b) {
+    float sum = part[b][0];
+#pragma unroll
+    for (int r = 1; r < R; ++r) sum += part[b][r];
+    v[b] = to_f32<T>(from_f32<T>(sum));
+  }
+  const float u = v[0] * v[2];
+#pragma unroll
+  for (int j = 0; j < SC_MAX_L; ++j) hist[j] = j == L - 1 ? u : j < L - 1 ? hist[j + 1 < SC_MAX_L ? j + 1 : j] : 0.f;
+#pragma unroll
+  for (int j = 0; j < SC_MAX_L; ++j)
+    if (j < L) {
+      c = fmaf(wt[j], hist[j], c);
+      st[j] = hist[j];
+    }
+  y[(size_t)t * width + ch] = from_f32<T>(v[1] * c);
+}
+
+// `z`: [ranges][n_tokens][3 * width], row i that of the request with slot slot_id[i]; y bfloat16.
+extern "C" int za_short_conv_ranges(const float* z, int ranges, const float* w, const float* bias, float* state,
+                                    const int* slot_id, void* y, int n_tokens, int width, int L,
+                                    long long slot_stride, hipStream_t stream) {
+  if (n_tokens == 0) return 0;
+  if (n_tokens < 0 || width <= 0 || L <= 0 || !z || !w || !state || !slot_id || !y ||
+      slot_stride < (long long)width * L)
+    return ZA_ERR_ARG;
+  if (L > SC_MAX_L || n_tokens > 65535) return ZA_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)((width + 255) / 256), (unsigned)n_tokens), block(256);
+#define ZA_SC_RANGES(R)                                                                                    \
+  hipLaunchKernelGGL((short_conv_ranges_kernel<bf16_t, R>), grid, block, 0, stream, z, w, bias, state,     \
+                     slot_id, (bf16_t*)y, width, L, slot_stride, (size_t)n_tokens * 3 * width)
+  if (ranges == 2) ZA_SC_RANGES(2);
+  else if (ranges == 4) ZA_SC_RANGES(4);
+  else return ZA_ERR_UNSUPPORTED;
+#undef ZA_SC_RANGES
+  return za_launch_status();
+}
+
 extern "C" int za_short_conv(const void* z, const float* w, const float* bias, float* state,
                              const int* token_seq, const int* seq_start, const int* slot_id,
                              void* y, int dtype, int n_tokens, int n_seqs, int width, int L,

@@ -48,13 +48,15 @@ _SIGNATURES = {
                                                       c_int, c_int, c_int, c_int, c_float, c_int,
                                                       c_int, c_int, c_void_p],
     ("attention", "za_paged_attention_decode_mfma_rope"): [
-        c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+        c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
         c_void_p, c_float, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float, c_int,
         c_int, c_int, c_int, c_void_p],
     ("attention", "za_attention_combine"): [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                                             c_void_p],
     ("gemm", "za_gemm_bf16_rows16_merged"): [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p,
                                              c_int, c_int, c_int, c_int, c_int, c_void_p],
+    ("shortconv", "za_short_conv_ranges"): [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+                                            c_void_p, c_int, c_int, c_int, c_longlong, c_void_p],
     ("shortconv", "za_short_conv"): [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                      c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                      c_longlong, c_void_p],
@@ -821,6 +823,46 @@ def tiles_take_gated(M: int, I: int, K: int) -> bool:
             and -(-I // (TILES_COLUMNS // 2)) >= TILES_MIN_GATED_WORKGROUPS)
 
 
+# The opening product of a mixer in a step of 17 to 64 single tokens, whose outputs alone make too few
+# workgroups: ranges of K, which the kernel that reads them adds up and rounds as the product would
+# (``rope_attention_decode``, ``short_conv``).  Measured as above, the library's product and the
+# ranges' at 20, 32 and 64 rows (us): 6144 x 2048 in 2 ranges 12.9, 12.8, 13.4 and 7.6, 8.3, 10.3;
+# 3072 x 2048 in 4 9.8, 9.2, 10.8 and 4.6, 4.7, 5.3.
+OPENING_WORKGROUPS = 256
+OPENING_RANGE_MIN_K = 256
+
+
+def opening_ranges(M: int, N: int, K: int) -> int:
+    """The ranges of K of such a product (0: it comes as usual)."""
+    if not LIBRARY_GEMM_ROWS < M <= TILES_MAX_ROWS:
+        return 0
+    for ranges in (4, 2):
+        if -(-N // TILES_COLUMNS) * ranges <= OPENING_WORKGROUPS and K >= ranges * OPENING_RANGE_MIN_K \
+                and tiles_take(M, N, K, ranges):
+            return ranges
+    return 0
+
+
+def linear_opening(x, weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """``x [M, K] @ weight[N, K]^T`` as 32-bit sums ``[ranges, M, N]``, or ``None`` where
+    ``opening_ranges`` says so or the operands are not the kernel's."""
+    if not isinstance(x, torch.Tensor) or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+        return None
+    M, K = x.shape
+    N = weight.shape[0]
+    ranges = opening_ranges(M, N, K)
+    if not ranges:
+        return None
+    _need(x, "x", torch.bfloat16)
+    _need(weight, "weight", torch.bfloat16, (N, K))
+    out = torch.empty((ranges, M, N), dtype=torch.float32, device=x.device)
+    if not _tiles_product(x, weight, out, ranges):
+        return None
+    _note("linear", M=M, N=N, K=K, norm_in_product=False, added_to_stream=False, partial_sums=ranges,
+          out=out.dtype, kernel="tiles")
+    return out
+
+
 def _tiles_product(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, ranges: int = 1,
                    gated: bool = False, activation: int = 0) -> bool:
     """``False``: operands that do not start on 16 bytes, which the kernel does not take."""
@@ -1512,16 +1554,21 @@ def rope_attention_decode(qkv: torch.Tensor, positions: torch.Tensor, slots: tor
     the workgroup that meets the token's own position stores key and value to the cache).
     The same bits in the result and in the cache, one kernel and one trip through memory
     less.  Returns the attention's output ``[T, heads, head_dim]``, or, with ``nsplit`` > 1 and
-    ``combine=False``, the ranges' partial results unmerged as ``MergedRows``."""
+    ``combine=False``, the ranges' partial results unmerged as ``MergedRows``.  ``qkv`` may be a
+    32-bit stack ``[ranges, T, columns]`` (``linear_opening``)."""
     if kv_cache.dim() != 5 or kv_cache.shape[1] != 2:
         raise KernelError(f"kv_cache has shape {tuple(kv_cache.shape)}, expected "
                           f"[pages, 2, kv_heads, page_size, head_dim]")
     nkv, page_size, d = kv_cache.shape[2], kv_cache.shape[3], kv_cache.shape[4]
-    T = qkv.shape[0]
+    ranges = qkv.shape[0] if qkv.dim() == 3 else 0
+    T = qkv.shape[1] if ranges else qkv.shape[0]
     nh = int(num_heads)
-    _need(qkv, "qkv", torch.bfloat16, (T, (nh + 2 * nkv) * d))
+    if ranges:
+        _need(qkv, "qkv", torch.float32, (ranges, T, (nh + 2 * nkv) * d))
+    else:
+        _need(qkv, "qkv", torch.bfloat16, (T, (nh + 2 * nkv) * d))
     _need(kv_cache, "kv_cache", torch.bfloat16)
-    if nh % nkv or not decode_rope_fusable(qkv, nh, nkv, d, d, False, page_size, scale):
+    if nh % nkv or not decode_rope_fusable(kv_cache, nh, nkv, d, d, False, page_size, scale):
         raise KernelError(f"rope_attention_decode does not take {nh} heads, {nkv} key/value "
                           f"heads, head_dim {d}, page size {page_size}, scale {scale}")
     _need(block_table, "block_table", torch.int32)
@@ -1542,12 +1589,12 @@ def rope_attention_decode(qkv: torch.Tensor, positions: torch.Tensor, slots: tor
         part_acc = torch.empty((T, nh, nsplit, d), dtype=torch.float32, device=qkv.device)
         part_ml = torch.empty((T, nh, nsplit, 2), dtype=torch.float32, device=qkv.device)
     rc = _fn("attention", "za_paged_attention_decode_mfma_rope")(
-        _ptr(qkv), _ptr(out), _ptr(kv_cache), _ptr(block_table), block_table.shape[1],
+        _ptr(qkv), ranges, _ptr(out), _ptr(kv_cache), _ptr(block_table), block_table.shape[1],
         _ptr(positions), _ptr(slots), _ptr(q_norm_w), _ptr(k_norm_w), _ptr(inv_freq), float(eps),
         T, _ptr(part_acc), _ptr(part_ml), nh, nkv, d, page_size, float(scale), int(window),
         int(keys_per_split), int(nsplit), 0 if unmerged else 1, _stream())
     _check(rc, "rope_attention_decode")
-    _note("attention", kernel="decode_mfma_rope", rows=T, dtype=qkv.dtype, nsplit=int(nsplit),
+    _note("attention", kernel="decode_mfma_rope", rows=T, dtype=kv_cache.dtype, nsplit=int(nsplit),
           combine_kernel=nsplit > 1 and not unmerged)
     return MergedRows(part_acc, part_ml) if unmerged else out
 
@@ -1612,12 +1659,19 @@ def short_conv(z: torch.Tensor, taps: torch.Tensor, bias: Optional[torch.Tensor]
     csrc/shortconv.hip.  ``z [T, 3*width]``; ``taps [L, width]``, the filter tap by
     tap (a checkpoint's ``[width, L]`` turned round, so that a thread's channels lie
     side by side); ``state [slots, width, L]`` (updated in place; slots may be spaced
-    further apart than ``width * L`` floats)."""
-    T = z.shape[0]
+    further apart than ``width * L`` floats).  A step of single tokens may bring ``z`` as a 32-bit
+    stack ``[ranges, T, 3*width]`` (``linear_opening``); the result is then bfloat16."""
+    ranges = z.shape[0] if z.dim() == 3 else 0
+    T = z.shape[1] if ranges else z.shape[0]
     if taps.dim() != 2:
         raise KernelError(f"taps must be [L, width], got {tuple(taps.shape)}")
     L, width = taps.shape
-    _need(z, "z", (torch.float32, torch.bfloat16), (T, 3 * width))
+    if ranges:
+        _need(z, "z", torch.float32, (ranges, T, 3 * width))
+        if slot_id.numel() != T:
+            raise KernelError(f"a stack of sums of {T} tokens for {slot_id.numel()} requests")
+    else:
+        _need(z, "z", (torch.float32, torch.bfloat16), (T, 3 * width))
     _need(taps, "taps", torch.float32)
     if L > 8:
         raise KernelError(f"convolution length {L} exceeds the kernel's limit of 8")
@@ -1633,6 +1687,13 @@ def short_conv(z: torch.Tensor, taps: torch.Tensor, bias: Optional[torch.Tensor]
     _need(token_seq, "token_seq", torch.int32, (T,))
     _need(seq_start, "seq_start", torch.int32)
     _need(slot_id, "slot_id", torch.int32)
+    if ranges:
+        y = torch.empty((T, width), dtype=torch.bfloat16, device=z.device)
+        rc = _fn("shortconv", "za_short_conv_ranges")(
+            _ptr(z), ranges, _ptr(taps), _ptr(bias), _ptr(state), _ptr(slot_id), _ptr(y), T, width, L,
+            state.stride(0), _stream())
+        _check(rc, "short_conv", f"ranges={ranges}")
+        return y
     y = torch.empty((T, width), dtype=z.dtype, device=z.device)
     rc = _fn("shortconv", "za_short_conv")(_ptr(z), _ptr(taps), _ptr(bias), _ptr(state),
                                            _ptr(token_seq), _ptr(seq_start), _ptr(slot_id), _ptr(y),

@@ -68,7 +68,11 @@ class ShortConv(Mixer):
             y = ops.in_proj_gated_conv(x, self.w_in, self.w_conv, self.b_conv, cache.state,
                                        step.slot_id)
         else:
-            z = ops.linear(x, self.w_in, self.b_in, tune=self.runtime.tune)
+            # (single tokens beyond those: in_proj in ranges of K, which the convolution adds up)
+            z = ops.linear_opening(x, self.w_in) \
+                if step.n_tokens == step.n_seqs and self.b_in is None else None
+            if z is None:
+                z = ops.linear(x, self.w_in, self.b_in, tune=self.runtime.tune)
             y = ops.short_conv(z, self.w_conv, self.b_conv, cache.state, step.token_seq,
                                step.seq_start, step.slot_id)
         return ops.linear(y, self.w_out, self.b_out, partial_ok=True, accumulate=stream,

@@ -1857,3 +1857,13 @@ def test_short_conv_adds_up_the_projection(width, L, T, biased, ranges):
     want = o.short_conv(total.bfloat16(), taps, bias, two, seq, start, slots)
     got = o.short_conv(parts, taps, bias, one, seq, start, slots)
     assert torch.equal(got, want) and torch.equal(one, two)
+
+
+@pytest.mark.parametrize("ranges,T,N", [(1, 17, 4), (2, 20, 8192), (4, 33, 1100), (3, 64, 256)])
+def test_activation_adds_up_the_product(ranges, T, N):
+    o = ops()
+    parts = rand((ranges, T, N), torch.float32, 110).to(dev())
+    total = parts[0].clone()
+    for r in range(1, ranges):
+        total += parts[r]
+    assert torch.equal(o.activate(parts, "relu2"), o.activate(total.bfloat16(), "relu2"))

@@ -296,6 +296,34 @@ extern "C" int za_activate(const void* in, void* out, int dtype, long long n, in
   return za_launch_status();
 }
 
+// The same of a product that came as 32-bit sums over `ranges` ranges of K, `total` elements each: added
+// up in order and rounded to bfloat16 first, as the product itself would have been.
+__global__ void __launch_bounds__(256)
+activate_ranges_kernel(const float* __restrict__ in, int ranges, bf16_t* __restrict__ out, size_t total) {
+  const size_t idx = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (idx >= total) return;
+  f32x4_t x = *reinterpret_cast<const f32x4_t*>(in + idx);
+#pragma unroll 4
+  for (int r = 1; r < ranges; ++r) x += *reinterpret_cast<const f32x4_t*>(in + r * total + idx);
+  bf16x4_t o;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float v = fmaxf((float)(bf16_t)x[k], 0.f);
+    o[k] = (bf16_t)(v * v);
+  }
+  *reinterpret_cast<bf16x4_t*>(out + idx) = o;
+}
+
+// `n` a multiple of 4; act 0 only.
+extern "C" int za_activate_ranges(const float* in, int ranges, void* out, long long n, int act, hipStream_t stream) {
+  if (n == 0) return 0;
+  if (n < 0 || ranges < 1 || !in || !out || act != 0) return ZA_ERR_ARG;
+  if (n % 4 != 0 || (uintptr_t)in % 16 != 0 || (uintptr_t)out % 8 != 0) return ZA_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(activate_ranges_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, stream, in, ranges,
+                     (bf16_t*)out, (size_t)n);
+  return za_launch_status();
+}
+
 // out[r, c] = in[r, c] + bias[c]: the bias of a product whose 32-bit sums another kernel (or
 // a library) left, rounded once into the result's type.  `out` may be `in` for 32-bit results.
 template <typename TO>

@@ -142,6 +142,7 @@ _SIGNATURES = {
                                                 c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                                                 c_int, c_int, c_float, c_int, c_void_p],
     ("activation", "za_bias_add"): [c_void_p, c_void_p, c_void_p, c_int, c_longlong, c_int, c_void_p],
+    ("activation", "za_activate_ranges"): [c_void_p, c_int, c_void_p, c_longlong, c_int, c_void_p],
     ("activation", "za_activate"): [c_void_p, c_void_p, c_int, c_longlong, c_int, c_void_p],
     ("attention", "za_element_gate"): [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                        c_int, c_float, c_void_p],
@@ -1742,9 +1743,17 @@ UNARY_ACTIVATIONS = {"relu2": 0}
 
 def activate(x: torch.Tensor, activation: str) -> torch.Tensor:
     """A feed-forward's activation on its own, element by element, in 32-bit: ``relu2``, the
-    square of relu."""
+    square of relu.  ``x`` may be a 32-bit stack ``[ranges, T, N]`` (``linear_opening``, ``N`` a
+    multiple of 4), whose sum is rounded to bfloat16 first."""
     if activation not in UNARY_ACTIVATIONS:
         raise KernelError(f"activation must be one of {sorted(UNARY_ACTIVATIONS)}, got {activation!r}")
+    if isinstance(x, torch.Tensor) and x.dim() == 3:
+        _need(x, "x", torch.float32)
+        out = torch.empty(x.shape[1:], dtype=torch.bfloat16, device=x.device)
+        rc = _fn("activation", "za_activate_ranges")(_ptr(x), x.shape[0], _ptr(out), out.numel(),
+                                                     UNARY_ACTIVATIONS[activation], _stream())
+        _check(rc, "activate", f"{tuple(x.shape)}")
+        return out
     _need(x, "x", (torch.float32, torch.bfloat16))
     out = torch.empty_like(x)
     rc = _fn("activation", "za_activate")(_ptr(x), _ptr(out), _code(x.dtype), x.numel(),

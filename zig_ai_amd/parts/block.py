@@ -100,6 +100,9 @@ class ParallelResidualBlock:
         self.norm = parts["norm"]
         self.mixer = parts["mixer"]
         self.feed_forward = parts.get("feed_forward")
+        # (what is left pending may be a stack of partial sums)
+        if self.feed_forward is not None and hasattr(self.feed_forward, "partial_ok"):
+            self.feed_forward.partial_ok = True
 
     def forward(self, residual: torch.Tensor, pending: Optional[torch.Tensor], step,
                 cache) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:

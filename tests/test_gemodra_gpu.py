@@ -661,6 +661,25 @@ def test_latent_attention_kernels(H, W, R, page_size):
         assert float((got - want).abs().max()) < 2e-2, nsplit
 
 
+@pytest.mark.parametrize("H,W,R", [(16, 576, 512), (3, 40, 32)])
+def test_latent_decoding_cut_far_beyond_its_contexts(H, W, R):
+    """Ranges behind every context, as a recorded step has them: they leave no result, and what their
+    places in the workspace held before does not matter (both kernels that merge)."""
+    from zig_ai_amd.kernels import ops
+    requests = [(200, 1), (0, 1), (63, 1), (64, 1)]
+    q, plane, table, pos, iseq, irow, icnt, n, scale, sink, want = _latent_attention_case(
+        torch.bfloat16, H, W, R, requests, 16, 1, seed=8)
+    few = ops.latent_attention(q, plane, R, table, pos, iseq, irow, icnt, n, scale, sink, 64, 4, 1)
+    assert float((few.cpu().double() - want).abs().max()) < 2e-2
+    for nsplit in (16, 64, 70):
+        held = torch.full((4 * H * nsplit * R,), float("nan"), device="cuda")
+        del held                                     # (the next tensors of its size lie there)
+        many = ops.latent_attention(q, plane, R, table, pos, iseq, irow, icnt, n, scale, sink, 64, nsplit, 1)
+        if nsplit <= 64:
+            assert torch.equal(many, few), nsplit
+        assert float((many.cpu().double() - want).abs().max()) < 2e-2, nsplit
+
+
 @pytest.mark.parametrize("H,R,rotated,page_size", [
     (16, 512, 64, 16), (16, 512, 32, 64), (3, 512, 0, 16), (70, 256, 64, 8), (5, 256, 32, 16), (64, 256, 0, 4),
     (1, 128, 64, 16), (9, 128, 32, 32), (40, 128, 0, 16), (2, 512, 64, 12)])

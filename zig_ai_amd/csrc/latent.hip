@@ -1402,15 +1402,29 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out
   if (range_hi > hi) range_hi = hi;
   const LmCache cache = {plane, page_stride, block_table + (size_t)seq * bt_stride, page_size,
                          page_shift, W, R};
-  {
+  const bool row_ok = r16 < rows;
+  const int tok = row0 + (row_ok ? r16 / G : 0);
+  const int h = h0 + (row_ok ? r16 % G : 0);
+  if (nsplit > 1 && range_lo > hi) {
+    // a range behind the context (a recorded step is cut for the longest of its kind): no result, which
+    // a sum of -1 says
+    if (row_ok && wave == 0 && kq == 0) {
+      const size_t pidx = ((size_t)tok * H + h) * nsplit + z;
+      part_ml[pidx * 2] = -INFINITY;
+      part_ml[pidx * 2 + 1] = -1.f;
+    }
+    return;
+  }
+  LmTile regs_a, regs_b;
+  if (range_lo <= range_hi) lm_fetch(regs_a, cache, range_lo, range_hi, tid);
+  if (range_lo + LM_KT <= range_hi) lm_fetch(regs_b, cache, range_lo + LM_KT, range_hi, tid);
+  // (what a row has beyond whole steps and tiles; without such a rest all that is read is stored first)
+  if (W % 32 || R % 16) {
     const int words = (LM_KT * KS + 8 * VP * LM_VS) / 2;
     uint32_t* w = reinterpret_cast<uint32_t*>(lm_lds);
     for (int i = tid; i < words; i += LM_NT) w[i] = 0u;
   }
 
-  const bool row_ok = r16 < rows;
-  const int tok = row0 + (row_ok ? r16 / G : 0);
-  const int h = h0 + (row_ok ? r16 % G : 0);
   const int pos_q = row_ok ? positions[tok] : -1;
   const bf16x8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
   bf16x8_t qf[QW];          // the steps wave, wave + 4, ... of the row
@@ -1471,9 +1485,6 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out
       }
     }
   };
-  LmTile regs_a, regs_b;
-  if (range_lo <= range_hi) lm_fetch(regs_a, cache, range_lo, range_hi, tid);
-  if (range_lo + LM_KT <= range_hi) lm_fetch(regs_b, cache, range_lo + LM_KT, range_hi, tid);
   for (int tile0 = range_lo; tile0 <= range_hi; tile0 += 2 * LM_KT) {
     tile(regs_a, tile0);
     if (tile0 + LM_KT > range_hi) break;
@@ -1588,14 +1599,18 @@ latent_combine_wide_kernel(const float* __restrict__ part_acc, const float* __re
                            int H) {
   __shared__ float wz[64];
   __shared__ float tot;
+  __shared__ int used;            // ranges up to the last that has a result (a sum of -1: it has none)
   const size_t row = blockIdx.x;  // token * H + head
   const int tid = threadIdx.x;
   if (tid < 64) {
-    float mz = -INFINITY, lz = 0.f;
+    float mz = -INFINITY, lz = -1.f;
     if (tid < nsplit) {
       mz = part_ml[(row * nsplit + tid) * 2];
       lz = part_ml[(row * nsplit + tid) * 2 + 1];
     }
+    const unsigned long long there = __ballot(lz != -1.f);
+    if (lz == -1.f) lz = 0.f;
+    if (tid == 0) used = there ? 64 - __clzll((long long)there) : 0;
     const float mx = wave_max(mz);
     const float w = mz > -INFINITY ? expf(mz - mx) : 0.f;
     float total = wave_sum(lz * w);
@@ -1609,7 +1624,7 @@ latent_combine_wide_kernel(const float* __restrict__ part_acc, const float* __re
     const float* pa = part_acc + row * nsplit * R + dd;
     float acc = 0.f;
 #pragma unroll 4
-    for (int z = 0; z < nsplit; ++z) acc = fmaf(pa[(size_t)z * R], wz[z], acc);
+    for (int z = 0; z < used; ++z) acc = fmaf(pa[(size_t)z * R], wz[z], acc);
     out[row * R + dd] = from_f32<T>(acc * inv);
   }
 }

@@ -627,6 +627,31 @@ def test_ssd_recurrence_in_chunks(dtype, H, G, N, P, strong):
     assert float(mem[:, H * N * P:].abs().max()) == 0.0 and float(state[1].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("H,G,N,P", [(8, 1, 128, 64), (8, 2, 64, 128), (12, 3, 24, 16), (4, 1, 33, 130), (5, 1, 128, 70)])
+def test_ssd_chunks_with_scores_worked_out_once(H, G, N, P):
+    """Heads that share keys and queries take their scores from one place: the bits of the same heads with
+    keys and queries of their own, in chunks of one to a hundred and twenty-eight tokens."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator().manual_seed(H + N)
+    C = ops.RETENTION_CHUNK
+    lengths, slots = [C + 1, 1, 2 * C + 16, C - 1, 17], [2, 3, 0, 4, 1]
+    T, per = sum(lengths), H // G
+    assert per >= ops.SHARED_SCORES_HEADS
+    x, B, Q = (torch.randn(T, n, generator=gen) for n in (H * P, G * N, G * N))
+    proj = torch.randn(T, H, generator=gen)
+    dt_bias, D, A_log = (torch.randn(H, generator=gen).to(dev) for _ in range(3))
+    _, start, slot_id = _step_arrays(lengths, slots, dev)
+    results = []
+    for groups, q, k in ((G, Q, B), (H, *(y.view(T, G, N).repeat_interleave(per, 1).reshape(T, H * N) for y in (Q, B)))):
+        _, state = _slots(6, H * N * P, dev)
+        conv = torch.cat([x, k, q], dim=1).to(dev)
+        out = ops.ssd_recurrence_chunked(conv, H * P + groups * N, H * P, 0, proj.to(dev), 0, dt_bias, A_log, D, state, 0,
+                                         slot_id, _chunk_items(lengths, C, dev), H, groups, N, P)
+        results.append((out, state.clone()))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
 @pytest.mark.parametrize("strength", [1e3, 1e5, 1e7, 1e30])
 def test_ssd_chunks_behind_a_token_that_forgets(strength):
     """A few tokens whose decay is zero (``exp(A_log) dt`` = ``strength``) among tokens that keep

@@ -77,7 +77,9 @@ __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + lo
 //   3. decay_chunk_out:     o_i = 2^c_i B^T q_i + sum_(j <= i) 2^(c_i - c_j) dt_j (q_i . k_j) v_j
 // Every factor is a power of at most zero while decays are at most one.  All products are matrix
 // products of 16 x 16 x dk and 16 x 16 x dv blocks; the walk is a chain of tokens instead, 0.34 us
-// each.  2,048 tokens, 64 heads of 128 x 64: 698 us walked; 42 + 16 + 98 us here, where the products'
+// each.  2,048 tokens, 64 heads of 128 x 64: 698 us walked; 42 + 16 + 98 us here, 64 + 7 in place of the
+// 98 where the heads share their scores (a head's own take 15 of the products' 37 us and most of the
+// registers), where the products
 // time is 14 + 37 us and the rest waits for operands that pass registers; 16 heads of 128 x 128:
 // 624 us walked, 78 here (92 as chunks of 256 walked side by side and corrected).
 #define DC_CHUNK 128
@@ -109,6 +111,7 @@ struct DecayArgs {
   float* total;            // [items][H]: 2^c_n
   float* out;              // [T][H*dv]
   int H, G, dk, dv;
+  float* scores;           // [items][G][128][128]: q_i . k_j, j <= i to whole blocks of 16; or null
 };
 
 // One workgroup a chunk, head and 64 columns; a wave takes 16 columns.
@@ -248,10 +251,43 @@ decay_prefix_kernel(float* __restrict__ chunk_state, float* __restrict__ state, 
   *slot = S;
 }
 
+// The scores of a chunk, once for all heads of a group (a head by itself works them out where it needs
+// them): a workgroup a chunk, group and block of 16 tokens, its waves the blocks of keys in turn.
+template <int NT, bool FULL>
+__global__ void __launch_bounds__(256)
+decay_chunk_scores_kernel(DecayArgs a) {
+  const int item = blockIdx.x, grp = blockIdx.y, tile = blockIdx.z, tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+  const int n = a.item_count[item], dk = a.dk;
+  if (tile * 16 >= n) return;
+  const float* rows = a.vec + (size_t)a.item_row0[item] * a.width;
+  const bool aligned = dk % 4 == 0 && a.width % 4 == 0 && ((a.q_col | a.k_col) % 4) == 0 &&
+                       (reinterpret_cast<uintptr_t>(a.vec) & 15) == 0;
+  auto load = [&](int t0, int column, f32x4_t (&f)[NT]) {
+    const float* p = rows + (size_t)min(t0 + r16, n - 1) * a.width + column + grp * dk;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) f[t] = load4<FULL>(p + t * 16 + 4 * g, dk - (t * 16 + 4 * g), aligned);
+  };
+  f32x4_t fq[NT], fk[NT];
+  load(tile * 16, a.q_col, fq);
+  float* to = a.scores + (((size_t)item * a.G + grp) * DC_CHUNK + tile * 16 + r16) * DC_CHUNK + 4 * g;
+  for (int J = wave; J <= tile; J += 4) {
+    load(J * 16, a.k_col, fk);
+    f32x4_t s = zero4(), u = zero4();
+#pragma unroll
+    for (int t = 0; t < NT; t += 2) {
+      s = mfma4(fk[t], fq[t], s);
+      if (t + 1 < NT) u = mfma4(fk[t + 1], fq[t + 1], u);
+    }
+    *reinterpret_cast<f32x4_t*>(to + J * 16) = s + u;
+  }
+}
+
 // One workgroup a chunk, head and 64 columns; a wave takes two blocks of 16 tokens, one early and
 // one late in the chunk, so that all waves meet the same number of earlier blocks.  The scores
 // are taken turned round (keys along the rows), which is how the product with v reads them.
-template <int NT, bool FULL>
+// SHARED: the scores come from decay_chunk_scores_kernel, and with them a key's dk elements stay away.
+template <int NT, bool FULL, bool SHARED>
 __global__ void __launch_bounds__(256, 2)
 decay_chunk_out_kernel(DecayArgs a) {
   __shared__ float hi[DC_CHUNK], lo[DC_CHUNK], step[DC_CHUNK];
@@ -322,11 +358,21 @@ decay_chunk_out_kernel(DecayArgs a) {
   const int last = second ? tile[1] : tile[0];
   const float q_hi[2] = {hi[tile[0] * 16 + r16], hi[tile[1] * 16 + r16]};
   const float q_lo[2] = {lo[tile[0] * 16 + r16], lo[tile[1] * 16 + r16]};
-  f32x4_t fk[NT], v[4];
-  auto request = [&](int J) {
-    const float* k = rows + (size_t)min(J * 16 + r16, n - 1) * a.width + a.k_col + grp * dk;
+  f32x4_t fk[SHARED ? 2 : NT], v[4];      // SHARED: the scores of both blocks of tokens
+  [[maybe_unused]] const float* scored[2];
+  if constexpr (SHARED)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) fk[t] = load4<FULL>(k + t * 16 + 4 * g, dk - (t * 16 + 4 * g), aligned);
+    for (int i = 0; i < 2; ++i)
+      scored[i] = a.scores + (((size_t)item * a.G + grp) * DC_CHUNK + tile[i] * 16 + r16) * DC_CHUNK + 4 * g;
+  auto request = [&](int J) {
+    if constexpr (SHARED) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) fk[i] = *reinterpret_cast<const f32x4_t*>(scored[i] + J * 16);
+    } else {
+      const float* k = rows + (size_t)min(J * 16 + r16, n - 1) * a.width + a.k_col + grp * dk;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) fk[t] = load4<FULL>(k + t * 16 + 4 * g, dk - (t * 16 + 4 * g), aligned);
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       // (no token sees one beyond the chunk)
@@ -341,22 +387,28 @@ decay_chunk_out_kernel(DecayArgs a) {
   unsigned wild = 0;                 // of the blocks of own tokens and 16 columns: those with such numbers
   request(0);
   for (int J = 0; J <= last; ++J) {
-    f32x4_t k0[NT], v0[4];
+    constexpr int KT = SHARED ? 2 : NT;
+    f32x4_t k0[KT], v0[4];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) k0[t] = fk[t];
+    for (int t = 0; t < KT; ++t) k0[t] = fk[t];
 #pragma unroll
     for (int j = 0; j < 4; ++j) v0[j] = v[j];
     if (J < last) request(J + 1);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       if (J > tile[i] || (i == 1 && !second)) continue;
-      f32x4_t s = zero4(), u = zero4();
+      f32x4_t s = zero4();
+      if constexpr (SHARED) {
+        s = k0[i];
+      } else {
+        f32x4_t u = zero4();
 #pragma unroll
-      for (int t = 0; t < NT; t += 2) {
-        s = mfma4(k0[t], fq[i][t], s);
-        if (t + 1 < NT) u = mfma4(k0[t + 1], fq[i][t + 1], u);
+        for (int t = 0; t < NT; t += 2) {
+          s = mfma4(k0[t], fq[i][t], s);
+          if (t + 1 < NT) u = mfma4(k0[t + 1], fq[i][t + 1], u);
+        }
+        s += u;
       }
-      s += u;
       f32x4_t p;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -410,14 +462,15 @@ decay_chunk_out_kernel(DecayArgs a) {
 }
 
 // `items`: work items of at most DC_CHUNK rows, a request's side by side, of the requests that are
-// taken (the others' rows of `out` and their states are left alone); scratch: `sums` n_tokens*H*3, `chunk_state` n_items*H*dv*dk, `total` n_items*H floats.
+// taken (the others' rows of `out` and their states are left alone); scratch: `sums` n_tokens*H*3, `chunk_state` n_items*H*dv*dk, `total` n_items*H floats; `scores`
+// n_items*G*128*128 floats where heads share their keys and queries, or null.
 extern "C" int za_decay_chunked(const float* vec, int width, int q_col, int k_col, int x_col,
                                 const void* proj, int dtype, int proj_stride, int gate_col,
                                 const float* dt_bias, const float* A_log, const float* D,
                                 const float* fixed, float* state, long long slot_stride,
                                 const int* slot_id, const int* item_seq, const int* item_row0,
                                 const int* item_count, int n_items, int n_seqs, float* sums,
-                                float* chunk_state, float* total, float* out, int n_tokens, int H,
+                                float* chunk_state, float* total, float* scores, float* out, int n_tokens, int H,
                                 int G, int dk, int dv, hipStream_t stream) {
   if (n_tokens == 0 || n_items == 0) return 0;
   if (n_tokens < 0 || n_seqs <= 0 || n_items < 0 || H <= 0 || G <= 0 || H % G || dk <= 0 || dv <= 0 ||
@@ -429,8 +482,9 @@ extern "C" int za_decay_chunked(const float* vec, int width, int q_col, int k_co
   const long long elems = (long long)H * dk * dv;
   if (dk > 128 || elems > 0x7fffffffLL || H > 65535) return ZA_ERR_UNSUPPORTED;
   const DecayArgs a{vec, width, q_col, k_col, x_col, proj, proj_stride, gate_col, dtype, dt_bias, A_log, D,
-                    fixed, item_row0, item_count, sums, chunk_state, total, out, H, G, dk, dv};
-  const dim3 grid(n_items, H, (dv + 63) / 64), block(256);
+                    fixed, item_row0, item_count, sums, chunk_state, total, out, H, G, dk, dv, scores};
+  dim3 grid(n_items, H, (dv + 63) / 64);
+  const dim3 block(256);
   const bool full = dv % 64 == 0 && width % 4 == 0 && q_col % 4 == 0 && k_col % 4 == 0 &&
                     ((reinterpret_cast<uintptr_t>(vec) | reinterpret_cast<uintptr_t>(chunk_state)) & 15) == 0;
 #define ZA_DECAY(KERNEL)                                                                       \
@@ -448,9 +502,28 @@ extern "C" int za_decay_chunked(const float* vec, int width, int q_col, int k_co
                      chunk_state, state, slot_stride, slot_id, item_seq, n_items, total, (int)elems, H, dk * dv);
   const int rc = za_launch_status();
   if (rc != 0) return rc;
-  ZA_DECAY(decay_chunk_out_kernel)
+  if (scores) {
+    if ((reinterpret_cast<uintptr_t>(scores) & 15) != 0 || G > 65535) return ZA_ERR_ARG;
+    const dim3 by_heads = grid;
+    grid = dim3(n_items, G, DC_CHUNK / 16);
+    ZA_DECAY(decay_chunk_scores_kernel)
+    grid = by_heads;
+#define ZA_SHARED(NT, FULL) decay_chunk_out_kernel<NT, FULL, true>
+    if (full && dk == 64) hipLaunchKernelGGL((ZA_SHARED(4, true)), grid, block, 0, stream, a);
+    else if (full && dk == 128) hipLaunchKernelGGL((ZA_SHARED(8, true)), grid, block, 0, stream, a);
+    else if (dk <= 32) hipLaunchKernelGGL((ZA_SHARED(2, false)), grid, block, 0, stream, a);
+    else if (dk <= 64) hipLaunchKernelGGL((ZA_SHARED(4, false)), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((ZA_SHARED(8, false)), grid, block, 0, stream, a);
+#undef ZA_SHARED
+    return za_launch_status();
+  }
+  if (full && dk == 64) hipLaunchKernelGGL((decay_chunk_out_kernel<4, true, false>), grid, block, 0, stream, a);
+  else if (full && dk == 128) hipLaunchKernelGGL((decay_chunk_out_kernel<8, true, false>), grid, block, 0, stream, a);
+  else if (dk <= 32) hipLaunchKernelGGL((decay_chunk_out_kernel<2, false, false>), grid, block, 0, stream, a);
+  else if (dk <= 64) hipLaunchKernelGGL((decay_chunk_out_kernel<4, false, false>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((decay_chunk_out_kernel<8, false, false>), grid, block, 0, stream, a);
+  return za_launch_status();
 #undef ZA_DECAY
-  return 0;
 }
 
 // ------------------------------------------------------------------- gated delta rule

@@ -804,12 +804,12 @@ paged_attention_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restr
     // the raw rows, the norms' weights and the frequencies are requested first of all: none
     // of them waits for anything, and the norm is done by the time the position has arrived
     const size_t row_at = (size_t)tok * (nh + 2 * nkv) * D;
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      if (rope.q_norm_w) load8<float>(rope.q_norm_w + ks * 32 + grp * 8, wq[ks]);
-      if (rope.k_norm_w) load8<float>(rope.k_norm_w + ks * 32 + grp * 8, wk[ks]);
-    }
     if constexpr (ROPE == 2) {
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+        if (rope.q_norm_w) load8<float>(rope.q_norm_w + ks * 32 + grp * 8, wq[ks]);
+        if (rope.k_norm_w) load8<float>(rope.k_norm_w + ks * 32 + grp * 8, wk[ks]);
+      }
       float v[DBLK];
 #pragma unroll
       for (int db = 0; db < DBLK; ++db) v[db] = 0.f;
@@ -849,6 +849,8 @@ paged_attention_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restr
       for (int ks = 0; ks < KSTEPS; ++ks) {
         load8<bf16_t>(row + (size_t)head * D + ks * 32 + grp * 8, xq[ks]);
         load8<bf16_t>(row + (size_t)(nh + gkv) * D + ks * 32 + grp * 8, xk[ks]);
+        if (rope.q_norm_w) load8<float>(rope.q_norm_w + ks * 32 + grp * 8, wq[ks]);
+        if (rope.k_norm_w) load8<float>(rope.k_norm_w + ks * 32 + grp * 8, wk[ks]);
       }
 #pragma unroll
       for (int db = 0; db < DBLK; ++db) vnew[db] = row[(size_t)(nh + nkv + gkv) * D + db * 16 + r16];

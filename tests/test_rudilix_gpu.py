@@ -628,16 +628,18 @@ def test_ssd_recurrence_in_chunks(dtype, H, G, N, P, strong):
 
 
 @pytest.mark.parametrize("H,G,N,P", [(8, 1, 128, 64), (8, 2, 64, 128), (12, 3, 24, 16), (4, 1, 33, 130), (5, 1, 128, 70)])
-def test_ssd_chunks_with_scores_worked_out_once(H, G, N, P):
+def test_ssd_chunks_with_scores_worked_out_once(H, G, N, P, monkeypatch):
     """Heads that share keys and queries take their scores from one place: the bits of the same heads with
-    keys and queries of their own, in chunks of one to a hundred and twenty-eight tokens."""
+    keys and queries of their own, in chunks of one to a hundred and twenty-eight tokens (states of few
+    rows too, which only many heads take this way by themselves)."""
     from zig_ai_amd.kernels import ops
     dev = torch.device("cuda")
     gen = torch.Generator().manual_seed(H + N)
     C = ops.RETENTION_CHUNK
     lengths, slots = [C + 1, 1, 2 * C + 16, C - 1, 17], [2, 3, 0, 4, 1]
     T, per = sum(lengths), H // G
-    assert per >= ops.SHARED_SCORES_HEADS
+    assert ops.shares_scores(64, 64 // per, N) and not ops.shares_scores(H, H, N)
+    monkeypatch.setattr(ops, "shares_scores", lambda heads, groups, dk: heads > groups)
     x, B, Q = (torch.randn(T, n, generator=gen) for n in (H * P, G * N, G * N))
     proj = torch.randn(T, H, generator=gen)
     dt_bias, D, A_log = (torch.randn(H, generator=gen).to(dev) for _ in range(3))

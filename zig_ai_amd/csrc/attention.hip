@@ -226,6 +226,9 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
   };
 
   float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};     // l: of this lane's keys
+  // whether the wave has met a key that the row sees: until then what is in acc is no weight times values
+  // of other rows' keys, zeros, or, where such a value is infinite or undefined, to be thrown away
+  bool seen[2] = {false, false};
   f32x4_t acc[2][NC];
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt)
@@ -278,18 +281,28 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
           top = fmaxf(top, s[rt][e]);
         }
         const float m_new = fmaxf(m[rt], quad_max(top));
-        // (no key yet: nothing to rescale, and no difference of infinities)
+        // (no key yet, or scores of minus infinity only: no difference of infinities)
+        const float m_use = m_new > -INFINITY ? m_new : 0.f;
         const float alpha = m_new > -INFINITY ? expf(m[rt] - m_new) : 1.f;
         float own = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          s[rt][e] = valid[e] ? expf(s[rt][e] - m_new) : 0.f;
+          s[rt][e] = valid[e] ? expf(s[rt][e] - m_use) : 0.f;
           own += s[rt][e];
         }
         l[rt] = l[rt] * alpha + own;
         m[rt] = m_new;
+        if (seen[rt]) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) acc[rt][c] *= alpha;
+          for (int c = 0; c < NC; ++c) acc[rt][c] *= alpha;
+        } else {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) acc[rt][c] = zero;
+        }
+        const int wave_first = tile0 + wave * 16, last = min(pos[rt], range_hi);
+        int first = max(lo, chunk_start(ex, pos[rt]));
+        if (window > 0) first = max(first, pos[rt] - window + 1);
+        seen[rt] |= max(first, wave_first) <= min(last, wave_first + 15) || wave_first <= min(last, ex.keep - 1);
       }
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
@@ -324,7 +337,8 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
 #pragma unroll
     for (int c = 0; c < NC; ++c)
       if (16 * c < dv)
-        *reinterpret_cast<f32x4_t*>(&smem[(wave * AT_MAX_ROWS + r) * LDK + 16 * c + 4 * quarter]) = acc[rt][c] * f;
+        *reinterpret_cast<f32x4_t*>(&smem[(wave * AT_MAX_ROWS + r) * LDK + 16 * c + 4 * quarter]) =
+            seen[rt] ? acc[rt][c] * f : zero;
   }
   __syncthreads();
   for (int idx = tid; idx < rows * dv; idx += 256) {

@@ -1258,6 +1258,30 @@ def test_paged_attention_infinities(dtype, d):
     assert rel_err(out[16:], plain.causal_attention(q[16:].double(), k[16:].double(), v[16:].double())) < tol_of(dtype)
 
 
+@pytest.mark.parametrize("nsplit", [1, 3, 8, 9, 16, 17, 64, 65])
+@pytest.mark.parametrize("d", [8, 64, 72, 128, 256])
+def test_ranges_merged(d, nsplit):
+    """Few and many ranges, which two kernels take, against 64 bits; a range without a key, whose
+    accumulator is not looked at; a row without any."""
+    gen = torch.Generator().manual_seed(d + nsplit)
+    acc = torch.randn((3, 5, nsplit, d), generator=gen)
+    ml = torch.stack([torch.randint(-20, 4, (3, 5, nsplit), generator=gen).float(),
+                      torch.rand((3, 5, nsplit), generator=gen) + 0.5], dim=-1)
+    ml[0, 0, :] = torch.tensor([-math.inf, 0.0])
+    ml[0, 1, nsplit // 2] = torch.tensor([-math.inf, 0.0])
+    acc[0, 0], acc[0, 1, nsplit // 2] = math.nan, math.nan
+    got = ops().MergedRows(acc.to(dev()), ml.to(dev())).materialise().float().cpu().view(3, 5, d)
+    m, l = ml[..., 0].double(), ml[..., 1].double()
+    there = m > -math.inf
+    w = torch.where(there, torch.exp2(m - m.amax(-1, keepdim=True)), 0.0)
+    values = torch.where(there[..., None], acc.double(), 0.0)
+    want = (values * w[..., None]).sum(-2) / (l * w).sum(-1, keepdim=True).clamp(min=1e-300)
+    want[~there.any(-1)] = 0.0
+    assert torch.isfinite(got).all() and not got[0, 0].any()
+    sums = 2 * (nsplit + 4) * 2.0 ** -24 * float(values.abs().max())      # 32-bit sums of shares of at most 2
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -8 + sums).all()     # and one rounding to bfloat16
+
+
 def decode_step_case(nh, nkv, d, page_size, positions, seed):
     """A decode step: request i holds positions[i] cached tokens and brings one more.
     Returns qkv [T, (nh + 2 nkv) d], the cache with random contents in the requests' pages

@@ -1399,13 +1399,11 @@ static int paged_attention_any(const void* q, void* out, const void* kv, const i
   }
 #undef ZA_AT_ARGS
   if (rc != 0 || nsplit == 1) return rc;
-  dim3 grid((unsigned)((size_t)n_tokens * nh)), block(64);
+  const size_t merged = (size_t)n_tokens * nh;
   if (dtype == 0)
-    hipLaunchKernelGGL((attention_combine_kernel<float>), grid, block, 0, stream, part_acc,
-                       part_ml, (float*)out, dv, nsplit, 0, ex.sink, nh);
+    attention_combine(part_acc, part_ml, (float*)out, merged, dv, nsplit, 0, ex.sink, nh, stream);
   else
-    hipLaunchKernelGGL((attention_combine_kernel<bf16_t>), grid, block, 0, stream, part_acc,
-                       part_ml, (bf16_t*)out, dv, nsplit, 0, ex.sink, nh);
+    attention_combine(part_acc, part_ml, (bf16_t*)out, merged, dv, nsplit, 0, ex.sink, nh, stream);
   rc = za_launch_status();
   if (rc != 0 || !gate) return rc;
   return head_gate_any(out, gate, dtype, gate_stride, gate_col, n_tokens, nh, dv, out_scale,
@@ -1462,9 +1460,8 @@ static int launch_attention_mfma(const void* q, void* out, const void* kv, const
                      scale * 1.44269504088896341f, window, keys_per_split, nsplit, ex);
   int rc = za_launch_status();
   if (rc != 0 || nsplit == 1) return rc;
-  dim3 cgrid((unsigned)((size_t)n_tokens * nh)), cblock(64);
-  hipLaunchKernelGGL((attention_combine_kernel<bf16_t>), cgrid, cblock, 0, stream, part_acc,
-                     part_ml, (bf16_t*)out, D, nsplit, 1, SHAPED ? ex.sink : nullptr, nh);
+  attention_combine(part_acc, part_ml, (bf16_t*)out, (size_t)n_tokens * nh, D, nsplit, 1,
+                    SHAPED ? ex.sink : nullptr, nh, stream);
   return za_launch_status();
 }
 
@@ -1573,9 +1570,8 @@ static int launch_decode_mfma(const void* q, void* out, const void* kv, const in
   }
   int rc = za_launch_status();
   if (rc != 0 || nsplit == 1 || !combine) return rc;
-  dim3 cgrid((unsigned)((size_t)n_tokens * nh)), cblock(64);
-  hipLaunchKernelGGL((attention_combine_kernel<bf16_t>), cgrid, cblock, 0, stream, part_acc,
-                     part_ml, (bf16_t*)out, d, nsplit, 1, SHAPED ? ex.sink : nullptr, nh);
+  attention_combine(part_acc, part_ml, (bf16_t*)out, (size_t)n_tokens * nh, d, nsplit, 1,
+                    SHAPED ? ex.sink : nullptr, nh, stream);
   return za_launch_status();
 }
 
@@ -1586,8 +1582,7 @@ extern "C" int za_attention_combine(const float* part_acc, const float* part_ml,
   if (rows == 0) return 0;
   if (rows < 0 || d <= 0 || d > AT_MAX_D || nsplit < 1 || !part_acc || !part_ml || !out)
     return ZA_ERR_ARG;
-  hipLaunchKernelGGL((attention_combine_kernel<bf16_t>), dim3((unsigned)rows), dim3(64), 0, stream,
-                     part_acc, part_ml, (bf16_t*)out, d, nsplit, 1, nullptr, 1);
+  attention_combine(part_acc, part_ml, (bf16_t*)out, (size_t)rows, d, nsplit, 1, nullptr, 1, stream);
   return za_launch_status();
 }
 

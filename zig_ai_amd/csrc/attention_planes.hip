@@ -706,7 +706,6 @@ extern "C" int za_planes_attention(const void* q, void* out, const void* kv, con
   AP_FOR_CAPACITIES(AP_CASE)
 #undef AP_CASE
   if (rc != 0 || nsplit == 1) return rc;
-  hipLaunchKernelGGL((attention_combine_kernel<bf16_t>), dim3((unsigned)((size_t)n_tokens * nh)),
-                     dim3(64), 0, stream, part_acc, part_ml, (bf16_t*)out, dv, nsplit, 1, sink, nh);
+  attention_combine(part_acc, part_ml, (bf16_t*)out, (size_t)n_tokens * nh, dv, nsplit, 1, sink, nh, stream);
   return za_launch_status();
 }

@@ -1919,4 +1919,13 @@ def test_activation_adds_up_the_product(ranges, T, N):
     total = parts[0].clone()
     for r in range(1, ranges):
         total += parts[r]
-    assert torch.equal(o.activate(parts, "relu2"), o.activate(total.bfloat16(), "relu2"))
+    assert torch.equal(o.activate_ranges(parts, "relu2"), o.activate(total.bfloat16(), "relu2"))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(2, 5, 12), (1, 3, 7), (4, 2, 3, 5), (6,)])
+def test_activation_is_taken_element_by_element(shape, dtype):
+    """Whatever the tensor's shape: its dimensions are not looked at, and no sum is taken."""
+    x = rand(shape, dtype, 111)
+    got = ops().activate(x.to(dev()), "relu2")
+    assert got.dtype == dtype and torch.equal(got.cpu(), (x.float().clamp(min=0.0) ** 2).to(dtype))

@@ -1743,22 +1743,29 @@ UNARY_ACTIVATIONS = {"relu2": 0}
 
 def activate(x: torch.Tensor, activation: str) -> torch.Tensor:
     """A feed-forward's activation on its own, element by element, in 32-bit: ``relu2``, the
-    square of relu.  ``x`` may be a 32-bit stack ``[ranges, T, N]`` (``linear_opening``, ``N`` a
-    multiple of 4), whose sum is rounded to bfloat16 first."""
+    square of relu."""
     if activation not in UNARY_ACTIVATIONS:
         raise KernelError(f"activation must be one of {sorted(UNARY_ACTIVATIONS)}, got {activation!r}")
-    if isinstance(x, torch.Tensor) and x.dim() == 3:
-        _need(x, "x", torch.float32)
-        out = torch.empty(x.shape[1:], dtype=torch.bfloat16, device=x.device)
-        rc = _fn("activation", "za_activate_ranges")(_ptr(x), x.shape[0], _ptr(out), out.numel(),
-                                                     UNARY_ACTIVATIONS[activation], _stream())
-        _check(rc, "activate", f"{tuple(x.shape)}")
-        return out
     _need(x, "x", (torch.float32, torch.bfloat16))
     out = torch.empty_like(x)
     rc = _fn("activation", "za_activate")(_ptr(x), _ptr(out), _code(x.dtype), x.numel(),
                                           UNARY_ACTIVATIONS[activation], _stream())
     _check(rc, "activate")
+    return out
+
+
+def activate_ranges(parts: torch.Tensor, activation: str) -> torch.Tensor:
+    """``activate`` of a product that came as a 32-bit stack ``[ranges, T, N]`` (``linear_opening``,
+    ``N`` a multiple of 4): its sum rounded to bfloat16, as the product itself would have been."""
+    if activation not in UNARY_ACTIVATIONS:
+        raise KernelError(f"activation must be one of {sorted(UNARY_ACTIVATIONS)}, got {activation!r}")
+    _need(parts, "parts", torch.float32)
+    if parts.dim() != 3:
+        raise KernelError(f"parts must be [ranges, T, N], got {tuple(parts.shape)}")
+    out = torch.empty(parts.shape[1:], dtype=torch.bfloat16, device=parts.device)
+    rc = _fn("activation", "za_activate_ranges")(_ptr(parts), parts.shape[0], _ptr(out), out.numel(),
+                                                 UNARY_ACTIVATIONS[activation], _stream())
+    _check(rc, "activate_ranges", f"{tuple(parts.shape)}")
     return out
 
 

@@ -176,10 +176,9 @@ class ActivatedMLP(FeedForward):
 
     def forward(self, x, step=None, stream: Optional[torch.Tensor] = None):
         # (a step of 17 to 64 tokens: in ranges of K, which the activation adds up)
-        u = ops.linear_opening(x, self.up) if self.up.shape[0] % 4 == 0 else None
-        if u is None:
-            u = ops.linear(x, self.up, tune=self.runtime.tune)
-        a = ops.activate(u, self.activation)
+        parts = ops.linear_opening(x, self.up) if self.up.shape[0] % 4 == 0 else None
+        a = ops.activate_ranges(parts, self.activation) if parts is not None else \
+            ops.activate(ops.linear(x, self.up, tune=self.runtime.tune), self.activation)
         return ops.linear(a, self.down, out_dtype=torch.float32, accumulate=stream,
                           partial_ok=self.partial_ok, tune=self.runtime.tune)
 

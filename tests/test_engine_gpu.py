@@ -726,6 +726,27 @@ def test_graph_replays_with_library_products():
         assert eu.rel_err(recorded[r:r + 1], want) < TOL["bfloat16"], f"request {r}"
 
 
+@pytest.mark.parametrize("B", [8, 24, 48])
+def test_a_diagnostic_step_gives_the_served_step(B):
+    """The step that leaves its layers' values takes the products and kernels that the served step
+    takes: the same logits to the last bit, and the same cache for the step after."""
+    from zig_ai_amd.engine import DecoderModel, ModelRunner, StepEntry
+    model = DecoderModel.from_random(REAL_2L, seed=5, reproducible=True, quick=True)
+    prompts = [eu.random_tokens(5 + r % 7, 65536, 600 + r) for r in range(B)]
+    tails = [eu.random_tokens(3, 65536, 650 + r) for r in range(B)]
+    runners = [ModelRunner(model, page_size=16, num_pages=3 * B, num_slots=B + 1, use_graphs=False)
+               for _ in range(2)]
+    for runner in runners:
+        for r in range(B):
+            runner.admit(r)
+        runner.step([StepEntry(r, prompts[r], []) for r in range(B)])
+    for j in range(3):
+        batch = [StepEntry(r, [tails[r][j]], [0]) for r in range(B)]
+        taps = []
+        served, dumped = runners[0].step(batch), runners[1].step(batch, taps=taps if j < 2 else None)
+        assert torch.equal(served, dumped) and (len(taps) == len(model.schedule) + 1 or j == 2), f"step {j}"
+
+
 def test_widths_that_are_no_multiple_of_eight():
     """Any width runs in 32-bit; bfloat16 projections need rows that start on 16-byte
     boundaries and say so when the model is built, before anything runs."""

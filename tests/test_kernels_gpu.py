@@ -1867,33 +1867,10 @@ def test_combined_experts_added_to_the_stream(T, width):
 
 
 @pytest.mark.parametrize("ranges", [2, 4])
-@pytest.mark.parametrize("nh,nkv,d,keys,nsplit", [(32, 8, 64, 0, 1), (8, 2, 64, 256, 3), (8, 2, 128, 512, 3)])
-def test_rope_attention_decode_adds_up_the_projection(nh, nkv, d, keys, nsplit, ranges):
-    """The projection as 32-bit sums over ranges of K: the bits that its rounded sum gives, in the
-    result and in the cache."""
-    o = ops()
-    positions = [0, 1, 63, 64, 255, 700, 1100]
-    qkv, cache, table, pos, slots = decode_step_case(nh, nkv, d, 16, positions, 1300 + d)
-    gen = torch.Generator().manual_seed(ranges)
-    parts = torch.randn((ranges,) + tuple(qkv.shape), generator=gen).to(dev())
-    parts[0] += qkv.float()
-    total = parts[0].clone()
-    for r in range(1, ranges):
-        total += parts[r]
-    w = (rand((d,), torch.float32, 1301) * 0.3 + 1.0).to(dev())
-    inv = (1.0 / torch.pow(torch.tensor(1e6, dtype=torch.float64),
-                           2.0 * torch.arange(0, d // 2, dtype=torch.float64) / d)).float().to(dev())
-    one, two = cache.clone(), cache.clone()
-    args = (table, nh, 1e-5, 1.0 / math.sqrt(d), 0, keys, nsplit)
-    want = o.rope_attention_decode(total.bfloat16(), pos, slots, w, w, inv, two, *args)
-    got = o.rope_attention_decode(parts, pos, slots, w, w, inv, one, *args)
-    assert torch.equal(got, want) and torch.equal(one, two) and not torch.equal(one, cache)
-
-
-@pytest.mark.parametrize("ranges", [2, 4])
 @pytest.mark.parametrize("width,L,T,biased", [(2048, 3, 64, False), (300, 1, 17, True), (257, 8, 33, True)])
 def test_short_conv_adds_up_the_projection(width, L, T, biased, ranges):
-    """The same for the convolution of a step of single tokens: result and carried state."""
+    """The projection of a step of single tokens as 32-bit sums over ranges of K: the bits that its
+    rounded sum gives the convolution, in the result and in the carried state."""
     o = ops()
     gen = torch.Generator().manual_seed(width + ranges)
     parts = torch.randn((ranges, T, 3 * width), generator=gen).to(dev())

@@ -766,14 +766,9 @@ struct DecodeRope {
   bf16_t* kv_write;         // the cache, to store the token's key and value
   float eps;
   int write_kv;
-  // ROPE 2, in place of qkv: its 32-bit sums over `ranges` ranges of K, [ranges][tokens][nh + 2 nkv][D];
-  // their sum in order, rounded, is what the projection would have stored
-  const float* qkv_parts;
-  size_t part_stride;
-  int ranges;
 };
 
-template <int D, int NWV, int ROPE, bool SHAPED>
+template <int D, int NWV, bool ROPE, bool SHAPED>
 __global__ void __launch_bounds__(NWV * 64)
 paged_attention_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
                                    const bf16_t* kv,
@@ -817,58 +812,16 @@ paged_attention_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restr
   if constexpr (ROPE) {
     // the raw rows, the norms' weights and the frequencies are requested first of all: none
     // of them waits for anything, and the norm is done by the time the position has arrived
-    const size_t row_at = (size_t)tok * (nh + 2 * nkv) * D;
-    if constexpr (ROPE == 2) {
+    const bf16_t* row = rope.qkv + (size_t)tok * (nh + 2 * nkv) * D;
 #pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        if (rope.q_norm_w) load8<float>(rope.q_norm_w + ks * 32 + grp * 8, wq[ks]);
-        if (rope.k_norm_w) load8<float>(rope.k_norm_w + ks * 32 + grp * 8, wk[ks]);
-      }
-      float v[DBLK];
-#pragma unroll
-      for (int db = 0; db < DBLK; ++db) v[db] = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) xq[ks][i] = xk[ks][i] = 0.f;
-#pragma unroll 2
-      for (int z_ = 0; z_ < rope.ranges; ++z_) {
-        const float* row = rope.qkv_parts + z_ * rope.part_stride + row_at;
-        float a[8], b[8];
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-          load8<float>(row + (size_t)head * D + ks * 32 + grp * 8, a);
-          load8<float>(row + (size_t)(nh + gkv) * D + ks * 32 + grp * 8, b);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            xq[ks][i] += a[i];
-            xk[ks][i] += b[i];
-          }
-        }
-#pragma unroll
-        for (int db = 0; db < DBLK; ++db) v[db] += row[(size_t)(nh + nkv + gkv) * D + db * 16 + r16];
-      }
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          xq[ks][i] = (float)(bf16_t)xq[ks][i];
-          xk[ks][i] = (float)(bf16_t)xk[ks][i];
-        }
-#pragma unroll
-      for (int db = 0; db < DBLK; ++db) vnew[db] = (bf16_t)v[db];
-    } else {
-      const bf16_t* row = rope.qkv + row_at;
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        load8<bf16_t>(row + (size_t)head * D + ks * 32 + grp * 8, xq[ks]);
-        load8<bf16_t>(row + (size_t)(nh + gkv) * D + ks * 32 + grp * 8, xk[ks]);
-        if (rope.q_norm_w) load8<float>(rope.q_norm_w + ks * 32 + grp * 8, wq[ks]);
-        if (rope.k_norm_w) load8<float>(rope.k_norm_w + ks * 32 + grp * 8, wk[ks]);
-      }
-#pragma unroll
-      for (int db = 0; db < DBLK; ++db) vnew[db] = row[(size_t)(nh + nkv + gkv) * D + db * 16 + r16];
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      load8<bf16_t>(row + (size_t)head * D + ks * 32 + grp * 8, xq[ks]);
+      load8<bf16_t>(row + (size_t)(nh + gkv) * D + ks * 32 + grp * 8, xk[ks]);
+      if (rope.q_norm_w) load8<float>(rope.q_norm_w + ks * 32 + grp * 8, wq[ks]);
+      if (rope.k_norm_w) load8<float>(rope.k_norm_w + ks * 32 + grp * 8, wk[ks]);
     }
+#pragma unroll
+    for (int db = 0; db < DBLK; ++db) vnew[db] = row[(size_t)(nh + nkv + gkv) * D + db * 16 + r16];
     freq = rope.inv_freq[tid & (D / 2 - 1)];
   } else {
 #pragma unroll
@@ -1537,7 +1490,7 @@ extern "C" int za_paged_attention_mfma_shaped(const void* q, void* out, const vo
                             ScoreExtras{softcap, sink, qt_coef, qt_every, chunk}, stream);
 }
 
-template <int ROPE, bool SHAPED = false>
+template <bool ROPE, bool SHAPED = false>
 static int launch_decode_mfma(const void* q, void* out, const void* kv, const int* block_table,
                               int bt_stride, const int* positions, const int* wi_seq,
                               const int* wi_row0, const int* wi_count, int n_items, int n_tokens,
@@ -1607,13 +1560,13 @@ static int decode_mfma_any(const void* q, void* out, const void* kv, const int* 
     return ZA_ERR_UNSUPPORTED;
   if (nsplit > 1 && (!part_acc || !part_ml || keys_per_split <= 0 || keys_per_split % 64 != 0))
     return ZA_ERR_ARG;
-  const DecodeRope none = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, 0, nullptr, 0, 0};
+  const DecodeRope none = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, 0};
   if (ex.softcap > 0.f || ex.sink || ex.qt_every > 0 || ex.chunk > 0)
-    return launch_decode_mfma<0, true>(q, out, kv, block_table, bt_stride, positions, wi_seq,
+    return launch_decode_mfma<false, true>(q, out, kv, block_table, bt_stride, positions, wi_seq,
                                            wi_row0, wi_count, n_items, n_tokens, part_acc, part_ml,
                                            nh, nkv, d, page_size, scale, window, keys_per_split,
                                            nsplit, none, true, stream, ex);
-  return launch_decode_mfma<0>(q, out, kv, block_table, bt_stride, positions, wi_seq, wi_row0,
+  return launch_decode_mfma<false>(q, out, kv, block_table, bt_stride, positions, wi_seq, wi_row0,
                                    wi_count, n_items, n_tokens, part_acc, part_ml, nh, nkv, d,
                                    page_size, scale, window, keys_per_split, nsplit, none, true,
                                    stream);
@@ -1656,18 +1609,16 @@ extern "C" int za_paged_attention_decode_mfma_shaped(
 // za_qk_norm_rope_kv_write followed by za_paged_attention_decode_mfma leave.  With
 // nsplit > 1 and `combine` 0 the partial results stay as they are in part_acc / part_ml
 // (`out` is not written and may be null): whoever reads them merges them
-// (za_attention_combine, or za_gemm_bf16_rows16_merged on its way in).  `ranges` > 0: `qkv` holds the
-// projection's 32-bit sums over so many ranges of K, [ranges][n_tokens][nh + 2 nkv][d]; the kernel adds
-// them up on their way in and rounds as the projection does.
+// (za_attention_combine, or za_gemm_bf16_rows16_merged on its way in).
 extern "C" int za_paged_attention_decode_mfma_rope(
-    const void* qkv, int ranges, void* out, void* kv, const int* block_table, int bt_stride,
+    const void* qkv, void* out, void* kv, const int* block_table, int bt_stride,
     const int* positions, const int* slots, const float* q_norm_w, const float* k_norm_w,
     const float* inv_freq, float eps, int n_tokens, float* part_acc, float* part_ml, int nh,
     int nkv, int d, int page_size, float scale, int window, int keys_per_split, int nsplit,
     int combine, hipStream_t stream) {
   if (n_tokens == 0) return 0;
   if (n_tokens < 0 || nh <= 0 || nkv <= 0 || nh % nkv != 0 || page_size <= 0 || bt_stride <= 0 ||
-      nsplit < 1 || ranges < 0 || !qkv || !kv || !block_table || !positions || !slots || !inv_freq ||
+      nsplit < 1 || !qkv || !kv || !block_table || !positions || !slots || !inv_freq ||
       (!out && (combine || nsplit == 1)))
     return ZA_ERR_ARG;
   const int G = nh / nkv;
@@ -1676,10 +1627,9 @@ extern "C" int za_paged_attention_decode_mfma_rope(
   if (nsplit > 1 && (!part_acc || !part_ml || keys_per_split <= 0 || keys_per_split % 64 != 0))
     return ZA_ERR_ARG;
   const DecodeRope rope = {(const bf16_t*)qkv, slots, q_norm_w, k_norm_w, inv_freq, (bf16_t*)kv,
-                           eps, 1, (const float*)qkv, (size_t)n_tokens * (nh + 2 * nkv) * d, ranges};
-  auto launch = ranges > 0 ? launch_decode_mfma<2> : launch_decode_mfma<1>;
-  return launch(nullptr, out, kv, block_table, bt_stride, positions, nullptr, nullptr, nullptr,
-                n_tokens, n_tokens, part_acc, part_ml, nh, nkv, d, page_size, scale, window,
-                keys_per_split, nsplit, rope, combine != 0, stream,
-                ScoreExtras{0.f, nullptr, 0.f, 0, 0});
+                           eps, 1};
+  return launch_decode_mfma<true>(nullptr, out, kv, block_table, bt_stride, positions, nullptr,
+                                  nullptr, nullptr, n_tokens, n_tokens, part_acc, part_ml, nh, nkv,
+                                  d, page_size, scale, window, keys_per_split, nsplit, rope,
+                                  combine != 0, stream);
 }

@@ -48,7 +48,7 @@ _SIGNATURES = {
                                                       c_int, c_int, c_int, c_int, c_float, c_int,
                                                       c_int, c_int, c_void_p],
     ("attention", "za_paged_attention_decode_mfma_rope"): [
-        c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+        c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
         c_void_p, c_float, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float, c_int,
         c_int, c_int, c_int, c_void_p],
     ("attention", "za_attention_combine"): [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
@@ -824,11 +824,15 @@ def tiles_take_gated(M: int, I: int, K: int) -> bool:
             and -(-I // (TILES_COLUMNS // 2)) >= TILES_MIN_GATED_WORKGROUPS)
 
 
-# The opening product of a mixer in a step of 17 to 64 single tokens, whose outputs alone make too few
+# The opening product of a part in a step of 17 to 64 rows, whose outputs alone make too few
 # workgroups: ranges of K, which the kernel that reads them adds up and rounds as the product would
-# (``rope_attention_decode``, ``short_conv``).  Measured as above, the library's product and the
+# (``short_conv``, ``activate_ranges``).  Measured as above, the library's product and the
 # ranges' at 20, 32 and 64 rows (us): 6144 x 2048 in 2 ranges 12.9, 12.8, 13.4 and 7.6, 8.3, 10.3;
-# 3072 x 2048 in 4 9.8, 9.2, 10.8 and 4.6, 4.7, 5.3.
+# 3072 x 2048 in 4 9.8, 9.2, 10.8 and 4.6, 4.7, 5.3.  With the kernel that reads them: the
+# convolution 9.9, 9.9, 11.2 and 7.7, 8.0, 9.2 at 3072 x 2048.  Not for the attention that prepares
+# its token: each of a token's workgroups adds up its heads' columns again, and product and attention
+# of 150 keys a request took, whole and in ranges, 32 heads of 64 on 8 at 20, 40 and 64 rows 20, 28,
+# 21 and 19, 31, 21, 16 heads of 128 on 4 22, 23, 24 and 29, 30, 31.
 OPENING_WORKGROUPS = 256
 OPENING_RANGE_MIN_K = 256
 
@@ -1555,21 +1559,16 @@ def rope_attention_decode(qkv: torch.Tensor, positions: torch.Tensor, slots: tor
     the workgroup that meets the token's own position stores key and value to the cache).
     The same bits in the result and in the cache, one kernel and one trip through memory
     less.  Returns the attention's output ``[T, heads, head_dim]``, or, with ``nsplit`` > 1 and
-    ``combine=False``, the ranges' partial results unmerged as ``MergedRows``.  ``qkv`` may be a
-    32-bit stack ``[ranges, T, columns]`` (``linear_opening``)."""
+    ``combine=False``, the ranges' partial results unmerged as ``MergedRows``."""
     if kv_cache.dim() != 5 or kv_cache.shape[1] != 2:
         raise KernelError(f"kv_cache has shape {tuple(kv_cache.shape)}, expected "
                           f"[pages, 2, kv_heads, page_size, head_dim]")
     nkv, page_size, d = kv_cache.shape[2], kv_cache.shape[3], kv_cache.shape[4]
-    ranges = qkv.shape[0] if qkv.dim() == 3 else 0
-    T = qkv.shape[1] if ranges else qkv.shape[0]
+    T = qkv.shape[0]
     nh = int(num_heads)
-    if ranges:
-        _need(qkv, "qkv", torch.float32, (ranges, T, (nh + 2 * nkv) * d))
-    else:
-        _need(qkv, "qkv", torch.bfloat16, (T, (nh + 2 * nkv) * d))
+    _need(qkv, "qkv", torch.bfloat16, (T, (nh + 2 * nkv) * d))
     _need(kv_cache, "kv_cache", torch.bfloat16)
-    if nh % nkv or not decode_rope_fusable(kv_cache, nh, nkv, d, d, False, page_size, scale):
+    if nh % nkv or not decode_rope_fusable(qkv, nh, nkv, d, d, False, page_size, scale):
         raise KernelError(f"rope_attention_decode does not take {nh} heads, {nkv} key/value "
                           f"heads, head_dim {d}, page size {page_size}, scale {scale}")
     _need(block_table, "block_table", torch.int32)
@@ -1590,12 +1589,12 @@ def rope_attention_decode(qkv: torch.Tensor, positions: torch.Tensor, slots: tor
         part_acc = torch.empty((T, nh, nsplit, d), dtype=torch.float32, device=qkv.device)
         part_ml = torch.empty((T, nh, nsplit, 2), dtype=torch.float32, device=qkv.device)
     rc = _fn("attention", "za_paged_attention_decode_mfma_rope")(
-        _ptr(qkv), ranges, _ptr(out), _ptr(kv_cache), _ptr(block_table), block_table.shape[1],
+        _ptr(qkv), _ptr(out), _ptr(kv_cache), _ptr(block_table), block_table.shape[1],
         _ptr(positions), _ptr(slots), _ptr(q_norm_w), _ptr(k_norm_w), _ptr(inv_freq), float(eps),
         T, _ptr(part_acc), _ptr(part_ml), nh, nkv, d, page_size, float(scale), int(window),
         int(keys_per_split), int(nsplit), 0 if unmerged else 1, _stream())
     _check(rc, "rope_attention_decode")
-    _note("attention", kernel="decode_mfma_rope", rows=T, dtype=kv_cache.dtype, nsplit=int(nsplit),
+    _note("attention", kernel="decode_mfma_rope", rows=T, dtype=qkv.dtype, nsplit=int(nsplit),
           combine_kernel=nsplit > 1 and not unmerged)
     return MergedRows(part_acc, part_ml) if unmerged else out
 

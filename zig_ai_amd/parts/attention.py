@@ -388,16 +388,10 @@ class GroupedQueryAttention(Mixer):
         T = x.shape[0]
         if self.wide:
             return self._forward_wide(x, step, cache, stream)
+        qkv = ops.linear(x, self.w_qkv, self.b_qkv, tune=self.runtime.tune)
         slots = step.slot_mapping[cache.group]
-        prepares = self.rotation_in_attention and step.n_tokens == step.n_seqs and cache.writes \
-            and ops.decode_rope_fusable(cache.kv, nh, nkv, d, d, False, cache.kv.shape[3], self.scale)
-        qkv = None
-        if prepares and self.b_qkv is None and getattr(step, "taps", None) is None:
-            # (beyond a decode batch's rows in ranges of K, which that kernel adds up)
-            qkv = ops.linear_opening(x, self.w_qkv)
-        if qkv is None:
-            qkv = ops.linear(x, self.w_qkv, self.b_qkv, tune=self.runtime.tune)
-        if prepares:
+        if self.rotation_in_attention and step.n_tokens == step.n_seqs and cache.writes \
+                and ops.decode_rope_fusable(qkv, nh, nkv, d, d, False, cache.kv.shape[3], self.scale):
             # single tokens only: the attention kernel prepares queries, key and value itself
             keys, nsplit = plan_split(step.n_seqs, nkv, step.max_keys)
             # few rows in few ranges: the output projection merges the ranges on its way in

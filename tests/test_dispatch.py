@@ -128,3 +128,17 @@ def test_where_the_tiles_for_17_to_64_rows_are_taken():
     for M in (16, 65):
         assert not ops.tiles_take(M, 2048, 8192, 8) and not ops.tiles_take(M, 65536, 2048, 1)
         assert not ops.tiles_take_gated(M, 8192, 2048)
+
+
+def test_where_a_router_runs_in_one_kernel():
+    """Few blocks of 16 weight rows and a short K; with more of either the product's own kernel, which
+    many workgroups share, is faster."""
+    pays = ops.route_linear_pays
+    assert pays(8, 8, 2048) and pays(20, 8, 2048) and pays(64, 16, 2048) and pays(16, 16, 8192)
+    assert not pays(17, 16, 2560) and not pays(64, 8, 4096)
+    assert pays(8, 33, 2048) and pays(1, 32, 2048) and pays(64, 80, 512) and pays(1, 64, 512)
+    assert not pays(9, 33, 2048) and not pays(8, 33, 2560) and not pays(64, 32, 1024)
+    assert not pays(1, 64, 1024) and not pays(64, 80, 4096) and not pays(20, 64, 2048)
+    # steps beyond 64 tokens, where a launch costs more
+    assert pays(65, 80, 1024) and pays(1777, 48, 2048) and pays(8192, 16, 4096)
+    assert not pays(65, 64, 2048) and not pays(1777, 32, 2560) and not pays(4096, 16, 5120)

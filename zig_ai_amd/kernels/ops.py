@@ -2829,6 +2829,30 @@ def route_linear_takes(x: torch.Tensor, weight: torch.Tensor, n: int) -> bool:
         and (x.data_ptr() | weight.data_ptr()) % 16 == 0
 
 
+def route_linear_pays(T: int, rows: int, K: int) -> bool:
+    """Whether ``route_linear`` is the faster way for ``T`` tokens.  Its workgroup reads 16 tokens and all
+    weight rows through one chain, which grows with K and the blocks of 16 rows; product, choice and
+    lists as kernels of their own spread the product over more workgroups.  Measured (us, replayed from
+    graphs, apart and in one kernel; beyond 64 tokens a step is launched kernel by kernel, where one
+    launch less is worth some 3 us more: with 32 x 2048 apart a prompt of 1,777 tokens took 3,894
+    instead of 3,845, eight layers):
+      rows x K       1 token     8         16        20        64        512       2,048 tokens
+       8 x 2048       8,  5     9,  6     9,  6    10,  8    10,  9    12, 10    13, 11
+      16 x 4096      10,  7    11,  9    11, 11    11, 12    11, 13    12, 14    14, 15
+      32 x 2048       9,  7     9,  8     9, 10    11, 11    12, 12    12, 13    16, 16
+      33 x  512       8,  7     8,  7     9,  8    11,  8    13, 11    12, 12    16, 15
+      33 x 2048       9,  9    10, 10    10, 11    11, 13    12, 14    13, 14    17, 18
+      64 x 2048       9, 12    10, 13    10, 15    11, 16    11, 16    13, 18    18, 21
+      80 x 1024      10, 10    10, 11    10, 13    11, 15    13, 15    14, 16    21, 22
+      80 x 4096      12, 24    13, 26    13, 29    13, 30    13, 30    15, 32    26, 38"""
+    blocks = -(-rows // 16)
+    if T > 64:
+        return K <= 1024 or (K <= 2048 and blocks <= 3) or (K <= 4096 and blocks == 1)
+    if blocks == 1:
+        return T <= 16 or K <= 2048
+    return K <= 512 or (T <= 8 and blocks <= 3 and K <= 2048)
+
+
 def route_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], n: int, top: int,
                  correction: Optional[torch.Tensor] = None, groups: int = 0, keep: int = 0,
                  scale: float = 1.0, scores: str = "softmax", renormalize: bool = False,

@@ -202,7 +202,8 @@ class RoutedExperts(FeedForward):
         tune = self.runtime.tune
         rule = (self.correction, self.groups, self.keep, self.route_scale, self.scores, self.renormalize)
         lists = None
-        if ops.route_linear_takes(x, self.w_router, self.outputs):
+        if ops.route_linear_takes(x, self.w_router, self.outputs) \
+                and ops.route_linear_pays(T, *self.w_router.shape):
             # (an output beyond the experts that have weights is in nobody's list)
             chosen, weight, logits, lists = ops.route_linear(
                 x, self.w_router, self.b_router, self.outputs, self.top, *rule,

@@ -1849,6 +1849,27 @@ def test_router_product_and_choice_in_one_kernel(T, n, extra, top, groups, keep,
     assert torch.equal(one[2], logits[T - 1:]) and torch.equal(one[0], chosen[T - 1:])
 
 
+@pytest.mark.parametrize("n,top,groups,keep,scores", [(64, 64, 0, 0, "softmax"), (64, 27, 8, 6, "sigmoid"), (17, 9, 0, 0, "softmax"),
+                                                      (32, 16, 4, 2, "softmax"), (8, 7, 2, 2, "sigmoid")])
+def test_router_choices_of_many_tokens(n, top, groups, keep, scores):
+    """Nearly all outputs for many tokens, where a lane counts those before its own: the bits that a few
+    tokens at a time have, in rounds; with ties, infinities and values that compare false."""
+    o = ops()
+    T = -(-98304 // top)
+    gen = torch.Generator().manual_seed(n + top)
+    logits = (torch.randn((T, n), generator=gen) * 4).round() / 2
+    logits[::7, n // 2] = math.nan
+    logits[::11, : n // 3] = -math.inf
+    logits[5] = math.nan
+    logits, correction = logits.to(dev()), (torch.randn((n,), generator=gen).round() / 8).to(dev())
+    rule = (correction, groups, keep, 1.5, scores, True)
+    chosen, weight = o.route_topk(logits, n, top, *rule)
+    for first in range(0, T, 1500):
+        c, w = o.route_topk(logits[first:first + 1500].contiguous(), n, top, *rule)
+        assert torch.equal(chosen[first:first + 1500], c)
+        assert torch.equal(weight[first:first + 1500].view(torch.int32), w.view(torch.int32))
+
+
 @pytest.mark.parametrize("T,width", [(1, 64), (5, 300), (40, 2048)])
 def test_combined_experts_added_to_the_stream(T, width):
     """The same numbers as the combined rows added by the stream's own kernel, and their rounding."""

@@ -658,11 +658,23 @@ route_topk_kernel(const float* __restrict__ z, int ld, const float* __restrict__
 // The same for at most 64 outputs: a lane has one, in registers.  Everything over the wave runs on the
 // vector unit's own lane patterns (through LDS, a maximum over the wave waits six times): a choice is a
 // maximum and the first lane that holds it, a group's best a maximum over its lanes.
-// `z`: this lane's output, `give(j, output, weight)`: the lane that has the j-th choice.
+// Where nearly all outputs are chosen for many tokens a lane counts the outputs before its own instead
+// (`count`): the rounds are as many as the choices, the broadcasts as the outputs, and with enough waves to
+// hide the waits their number decides.  Rounds and counting (us): 16,384 tokens, 32 outputs, 4, 12, 16,
+// 24 and 32 of them 8 and 16, 16 and 17, 20 and 18, 28 and 20, 35 and 22; 64 outputs, 24, 32, 64 28 and 30, 35 and
+// 32, 67 and 40; 2,048 tokens, 64 outputs, 32, 48, 64 8 and 9, 10 and 10, 13 and 11; up to 64 tokens rounds always.
+// `z`: this lane's output, `give(j, output, weight)`: a lane that has the j-th choice.
 struct RouteRule {
   int n, groups, keep, top, mode, renorm;
   float scale;
+  int count;
 };
+
+static inline RouteRule route_rule(int n_tokens, int n, int groups, int keep, int top, int mode, int renorm,
+                                   float scale) {
+  const bool count = 5 * top > 2 * n && (long long)n_tokens * top >= 98304;
+  return RouteRule{n, groups, keep, top, mode, renorm, scale, count ? 1 : 0};
+}
 
 template <int CTRL>
 __device__ __forceinline__ float lanes_moved(float x) {
@@ -726,6 +738,23 @@ __device__ __forceinline__ void route_wave(const RouteRule& q, float z, float ad
   }
   bool open = in && c == c;                           // NaN is not chosen
   float total = 0.f, share = 0.f;
+  if (q.count) {
+    int before = 0;
+#pragma unroll 8
+    for (int k = 0; k < q.n; ++k) {
+      const float v = lane_value(c, k);
+      if (v > c || (v == c && k < lane)) ++before;
+    }
+    const int usable = __popcll(__ballot(open));
+    for (int j = 0; j < q.top; ++j) {
+      const unsigned long long who = __ballot(open && before == j);
+      total += lane_value(s, j < usable ? __ffsll((long long)who) - 1 : 0);
+    }
+    const float f = q.renorm ? q.scale / (total + 1e-20f) : q.scale;
+    if (open && before < q.top) give(before, lane, s * f);
+    if (lane >= usable && lane < q.top) give(lane, 0, lane_value(s, 0) * f);
+    return;
+  }
   int place = -1, output = 0;
   for (int j = 0; j < q.top; ++j) {
     const float m = lanes_max(open ? c : -INFINITY);
@@ -884,7 +913,7 @@ extern "C" int za_route_linear(const void* x, const void* W, const float* bias, 
   const bool two = lists && n_tokens > 16;            // (all tokens in one workgroup)
   if (two && tiles > 3) return ZA_ERR_UNSUPPORTED;
   RouteArgs a{(const bf16_t*)x, (const bf16_t*)W, bias, correction, logits, chosen, weight, lists, counts,
-              n_tokens, K, rows, experts, RouteRule{n, groups, keep, top, mode, renorm, scale}};
+              n_tokens, K, rows, experts, route_rule(n_tokens, n, groups, keep, top, mode, renorm, scale)};
   const dim3 grid(two ? 1 : (n_tokens + 15) / 16), block(RL_WAVES * 64);
 #define ZA_RL(NT, MT) hipLaunchKernelGGL((route_linear_kernel<NT, MT>), grid, block, 0, stream, a)
   if (two) {
@@ -912,7 +941,7 @@ extern "C" int za_route_topk(const float* z, int ld, const float* correction, in
   if (n > RT_MAX) return ZA_ERR_UNSUPPORTED;
   if (n <= 64)
     hipLaunchKernelGGL(route_topk_wave_kernel, dim3(n_tokens), dim3(64), 0, stream, z, ld, correction,
-                       RouteRule{n, groups, keep, top, mode, renorm, scale}, chosen, weight);
+                       route_rule(n_tokens, n, groups, keep, top, mode, renorm, scale), chosen, weight);
   else
     hipLaunchKernelGGL(route_topk_kernel, dim3(n_tokens), dim3(64), 0, stream, z, ld, correction, n,
                        groups, keep, top, scale, mode, renorm, chosen, weight);

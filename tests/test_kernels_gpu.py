@@ -1230,6 +1230,37 @@ def test_paged_attention_window_skips_freed_pages():
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nh,nkv,d,page_size", [(3, 3, 8, 16), (4, 2, 64, 3), (2, 1, 72, 4), (5, 5, 80, 16), (4, 1, 88, 12),
+                                                (2, 2, 128, 5), (8, 2, 136, 16), (3, 1, 192, 8), (2, 2, 200, 1), (16, 1, 248, 16)])
+def test_paged_attention_widths(dtype, nh, nkv, d, page_size):
+    """Heads at the edges of what the kernel's forms are built for, pages of any size; steps of single
+    tokens, which a form of its own takes, with and without ranges, and portions, with a window."""
+    ctx = [0, 1, 15, 16, 37, 63, 64, 130, 300]
+    for new, window, keys, nsplit in (([1] * len(ctx), 0, 0, 1), ([1] * len(ctx), 40, 0, 1), ([1] * len(ctx), 0, 128, 3),
+                                      ([1, 17, 2, 40, 1, 33, 1, 5, 16], 0, 0, 1), ([9, 1, 1, 1, 70, 3, 1, 1, 20], 21, 0, 1)):
+        out, expect = run_attention(dtype, nh, nkv, d, page_size, ctx, new, window=window, keys_per_split=keys, nsplit=nsplit)
+        assert rel_err(out, expect) < tol_of(dtype), (new, window, nsplit)
+
+
+@pytest.mark.parametrize("d", [64, 80, 104])
+def test_paged_attention_items_that_overlap(d):
+    """As many work items as tokens, which a step of single tokens has, but each of several tokens and
+    more than 16 rows: every item's rows are worked out all the same."""
+    nh, nkv, T, c = 8, 2, 7, 90
+    k, v, q = (rand(s, torch.float32, 400 + i) for i, s in enumerate(((c + T, nkv, d), (c + T, nkv, d), (T, nh, d))))
+    cache, table = paged_from_dense([k], [v], 16, torch.float32)
+    pos = torch.arange(c, c + T, dtype=torch.int32, device=dev())
+    mk = lambda x: torch.tensor(x, dtype=torch.int32, device=dev())
+    args = (cache.to(dev()), table.to(dev()), pos)
+    got = ops().paged_attention(q.to(dev()), *args, mk([0] * T), mk([0] * T), mk([T] * T), T, d ** -0.5)
+    want = ops().paged_attention(q.to(dev()), *args, mk([0]), mk([0]), mk([T]), 1, d ** -0.5)
+    assert torch.equal(got, want)
+    full = torch.zeros((c + T, nh, d), dtype=torch.float64)
+    full[c:] = q.double()
+    assert rel_err(got, plain.causal_attention(full, k.double(), v.double())[c:]) < F32_TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("d", [16, 48, 256])
 def test_paged_attention_infinities(dtype, d):
     """An infinite value behind a row's window stays out of rows whose window begins at a later tile, and

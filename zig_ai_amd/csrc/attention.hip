@@ -67,17 +67,21 @@ __device__ __forceinline__ float shaped_score_log2(const ScoreExtras& ex, float 
 
 // The general kernel: both storage types, any sizes, both products on the matrix cores' 32-bit
 // instruction (v_mfma_f32_16x16x4_f32; its layout in gemm_f32.h), everything in 32-bit.  A work item has
-// up to 32 rows (token, head), two blocks of 16; a tile's 64 keys are dealt to the four waves, 16 each,
-// and a wave keeps maxima, sums and accumulators of its own for all rows:
+// up to 32 rows (token, head), two blocks of 16; four waves share a block of rows and a tile's 64 keys,
+// 16 each, and a wave keeps maxima, sums and accumulators of its own:
 //   S^T = K Q^T    queries in registers, keys from LDS; a lane has four keys of one row
 //   O^T += V^T P^T the probabilities go from the accumulator straight into the second operand
 // The waves' parts meet in LDS at the end, in the waves' order: a row's result depends on the places of
 // its keys only.  The next tile is on its way from memory while one is computed.
-// 448 rows of three prompts up to 150 tokens, 16 heads of 64 over 8, 32-bit: 115 us on the vector unit
-// with two reads of LDS a product, 29 here; three of 1,000 tokens 1,052 and 303; heads of 128 over 500
-// tokens 772 and 151, of 256 1,928 and 400; one row a request at 2,000 keys 216 and 143 (a chain of 32
-// tiles there: pages, keys, scores, weights).
-// NC: blocks of 16 channels of keys and of values, at most (4, 8 or 16).
+// RB 2: eight waves for both blocks of rows; RB 1: four, which take one block after the other, for steps of
+// single tokens.  NC: blocks of 16 channels of keys and of values, at most.  What bounds it is the chain of
+// tiles (page, keys, scores, weights) times how few of a compute unit's workgroups hide each other's waits, and
+// that registers decide: with both blocks of rows in four waves' registers, and wide heads in whole
+// 128 or 256 channels, one workgroup a compute unit (some of them spilled) where two or three are now.
+// Measured (us; vector unit, four waves, now), 32-bit: three prompts of 150 tokens, 16 heads of 64 on 8,
+// 105, 28, 17; 600 tokens, 8 heads of 128 587, 121, 64, 8 heads of 256 on 1 1,489, 297, 102; one token a
+// request, 64 at 300 keys with 12 heads of 80 80, 147, 44, 100 at 250 keys with 4 of 192 138, 191, 58, 8 at
+// 4,000 keys with 16 of 64 on 8 161, 85, 71, one at 9 keys with 8 of 256 18, 29, 11.
 template <typename T> __device__ __forceinline__ f32x4_t at_load4(const T* p);
 template <> __device__ __forceinline__ f32x4_t at_load4<float>(const float* p) {
   return *reinterpret_cast<const f32x4_t*>(p);
@@ -87,13 +91,16 @@ template <> __device__ __forceinline__ f32x4_t at_load4<bf16_t>(const bf16_t* p)
   return f32x4_t{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
 }
 
-template <int NC>
-constexpr size_t at_lds() {        // floats: a tile's keys and values, then the waves' results
-  return (size_t)AT_KT * (NC * 16 + 4) + (size_t)NC * 16 * (AT_KT + 4);
+// floats: a tile's keys and values (TURNS below: one place for both), then the waves' results
+template <int NC, int RB>
+constexpr int at_lds() {
+  constexpr int keys = AT_KT * (NC * 16 + 4), values = NC * 16 * (AT_KT + 4), results = 4 * 16 * RB * (NC * 16 + 4);
+  constexpr int tile = NC < 12 ? keys + values : keys > values ? keys : values;
+  return tile > results ? tile : results;
 }
 
-template <typename T, int NC>
-__global__ void __launch_bounds__(256)
+template <typename T, int NC, int RB>
+__global__ void __launch_bounds__(256 * RB, RB == 1 ? (NC <= 5 ? 3 : NC <= 12 ? 2 : 1) : NC <= 5 ? 4 : 2)
 paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __restrict__ kv,
                        const int* __restrict__ block_table, int bt_stride,
                        const int* __restrict__ positions, const int* __restrict__ wi_seq,
@@ -108,18 +115,17 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
   // sigmoid(gate[t * gate_stride + gate_col + h]) * out_scale; with `gate_elem` every
   // element dd of it by its own sigmoid(gate[t * gate_stride + gate_col + h * dv + dd]).
   constexpr int LDK = NC * 16 + 4, LDV = AT_KT + 4;   // (16 rows read together: different banks)
-  constexpr bool AHEAD = NC < 16;         // (256 channels leave no registers for the next tile)
-  static_assert(4 * AT_MAX_ROWS * LDK <= at_lds<NC>(), "the waves' results take the tile's place");
+  constexpr bool TURNS = NC >= 12;        // keys and values of wide heads take turns in LDS
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  __shared__ float wave_m[4][AT_MAX_ROWS], wave_l[4][AT_MAX_ROWS];
+  __shared__ float wave_m[4 * RB][16], wave_l[4 * RB][16];
   const size_t page_elems = (size_t)nkv * page_size * (d + dv);
   const size_t value_base = (size_t)nkv * page_size * d;
   float* Ks = smem;                       // [key][channel]
-  float* Vt = Ks + AT_KT * LDK;           // [channel][key]
+  float* Vt = TURNS ? smem : Ks + AT_KT * LDK;      // [channel][key]
 
   const int item = blockIdx.x, g = blockIdx.y, z = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, quarter = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), part = wave & 3, block = wave >> 2;
   const int G = nh / nkv;
   const int seq = wi_seq[item];
   const int row0 = wi_row0[item];
@@ -146,228 +152,244 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
   auto next_tile = [&](int t) { return t >= kept_end && t < tile_first ? tile_first : t; };
   auto there = [&](int kp) { return (kp >= lo || kp < ex.keep) && kp <= range_hi; };
 
-  // this lane's rows: their positions and queries (some row's where there is none)
-  int pos[2];
-  f32x4_t qf[2][NC];
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const int r = min(rt * 16 + r16, rows - 1), tok = row0 + r / G;
-    pos[rt] = positions[tok];
-    const T* from = q + ((size_t)tok * nh + g * G + r % G) * d;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int at = 16 * c + 4 * quarter;
-      qf[rt][c] = at < d ? at_load4<T>(from + at) : zero;
+  for (int first_row = 0; first_row < AT_MAX_ROWS; first_row += 16 * RB) {
+    if (first_row > 0) {
+      if (first_row >= rows) break;
+      __syncthreads();                // (the rows before are written)
     }
-  }
-  const float temper[2] = {query_temperature(ex, pos[0]), query_temperature(ex, pos[1])};
-
-  f32x4_t rk[NC], rv[NC];
-  // (pages first, then what lies on them, every request unconditional, some valid place's where there
-  // is nothing: behind conditions each would wait for its own page; pages a tile further ahead gained
-  // nothing)
-  auto page_of = [&](int kp) { return table[page_entry(min(kp, range_hi), page_size, shift)]; };
-  auto fetch_keys = [&](int tile0) {
-    int page[NC];
-#pragma unroll
-    for (int i = 0; i < NC; ++i) page[i] = page_of(tile0 + (tid + 256 * i) / (4 * NC));
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-      const int v = tid + 256 * i, kp = tile0 + v / (4 * NC), c = v % (4 * NC) * 4;
-      rk[i] = at_load4<T>(kv + max(page[i], 0) * page_elems +
-                          ((size_t)g * page_size + page_offset(kp, page_size, shift)) * d + (c < d ? c : 0));
-      if (!(c < d && there(kp) && page[i] >= 0)) rk[i] = zero;
-    }
-  };
-  auto fetch_values = [&](int tile0) {
-    int page[NC];
-    if (fours) {
-#pragma unroll
-      for (int i = 0; i < NC; ++i) page[i] = page_of(tile0 + ((tid + 256 * i) & 15) * 4);
-    }
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-      const int v = tid + 256 * i, dd = v >> 4, kp = tile0 + (v & 15) * 4;
-      if (fours) {
-        rv[i] = at_load4<T>(kv + max(page[i], 0) * page_elems + value_base +
-                            ((size_t)g * dv + (dd < dv ? dd : 0)) * page_size + page_offset(kp, page_size, shift));
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (!(dd < dv && there(kp + e) && page[i] >= 0)) rv[i][e] = 0.f;
-      } else {
-        rv[i] = zero;
-        if (dd >= dv) continue;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (there(kp + e)) {
-            const int page = table[(kp + e) / page_size];
-            if (page >= 0)
-              rv[i][e] = to_f32<T>(kv[page * page_elems + value_base + ((size_t)g * dv + dd) * page_size +
-                                      (kp + e) % page_size]);
-          }
-      }
-    }
-  };
-
-  auto stash_keys = [&]() {
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-      const int v = tid + 256 * i;
-      *reinterpret_cast<f32x4_t*>(&Ks[v / (4 * NC) * LDK + v % (4 * NC) * 4]) = rk[i];
-    }
-  };
-  auto stash_values = [&]() {
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-      const int v = tid + 256 * i;
-      *reinterpret_cast<f32x4_t*>(&Vt[(v >> 4) * LDV + (v & 15) * 4]) = rv[i];
-    }
-  };
-
-  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};     // l: of this lane's keys
-  // whether the wave has met a key that the row sees: until then what is in acc is no weight times values
-  // of other rows' keys, zeros, or, where such a value is infinite or undefined, to be thrown away
-  bool seen[2] = {false, false};
-  f32x4_t acc[2][NC];
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-    for (int c = 0; c < NC; ++c) acc[rt][c] = zero;
-
-  int tile0 = next_tile(kept_end > range_lo ? range_lo : tile_first);
-  if (AHEAD && tile0 <= range_hi) {
-    fetch_keys(tile0);
-    fetch_values(tile0);
-  }
-  while (tile0 <= range_hi) {
-    __syncthreads();  // the tile before has been read
-    if (!AHEAD) fetch_keys(tile0);
-    stash_keys();
-    if (!AHEAD) fetch_values(tile0);
-    stash_values();
-    __syncthreads();
-    const int key0 = tile0 + wave * 16 + quarter * 4;          // this lane's four keys
-    const int next = next_tile(tile0 + AT_KT);
-    if (AHEAD && next <= range_hi) {
-      fetch_keys(next);
-      fetch_values(next);
-    }
-    if (tile0 + wave * 16 <= range_hi) {
-      f32x4_t s[2] = {zero, zero};
+    // this lane's row: its position and queries (some row's where there is none)
+    const bool busy = first_row + 16 * block < rows;
+    const int own_row = min(first_row + 16 * block + r16, rows - 1), own_token = row0 + own_row / G;
+    const int pos = positions[own_token];
+    const float temper = query_temperature(ex, pos);
+    f32x4_t qf[NC];
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    {
+      const T* from = q + ((size_t)own_token * nh + g * G + own_row % G) * d;
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
-        if (16 * c >= d) break;
-        const f32x4_t k = *reinterpret_cast<const f32x4_t*>(&Ks[(wave * 16 + r16) * LDK + 16 * c + 4 * quarter]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], qf[0][c][e], s[0], 0, 0, 0);
-          if (rows > 16) s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], qf[1][c][e], s[1], 0, 0, 0);
-        }
+        const int at = 16 * c + 4 * quarter;
+        qf[c] = at < d ? at_load4<T>(from + at) : zero;
       }
+    }
+
+    // What 256 threads bring of a tile at a time, a unit: of its keys 16 keys x 64 channels, of the channels
+    // beyond whole 64 all keys x 16 channels; of its values 16 channels x all keys.  Pages first, then what
+    // lies on them, some valid place's where there is nothing: behind conditions each request would wait
+    // for its own page.  Units that nothing is in are left out.  (Pages a tile further ahead gained nothing.)
+    constexpr int FULL = NC / 4 * 4, UNITS = (NC + RB - 1) / RB, PAGES = 4 / RB;
+    int t16 = tid & 15, row = (tid & 255) >> 4;
+    f32x4_t rk[UNITS], rv[UNITS];
+    unsigned lost_keys = 0;               // units on pages that are gone
+    bool lost_values = false;
+    auto page_of = [&](int kp) { return table[page_entry(min(kp, range_hi), page_size, shift)]; };
+    auto key_of = [&](int u) { return u < FULL ? row + 16 * (u & 3) : (tid & 255) >> 2; };
+    auto channel_of = [&](int u) { return u < FULL ? 4 * t16 + 16 * (u & ~3) : 16 * u + 4 * (tid & 3); };
+    auto keys_in = [&](int tile0, int u) {
+      return u < NC && 16 * (u < FULL ? u & ~3 : u) < d && (u >= FULL || tile0 + 16 * (u & 3) <= range_hi);
+    };
+    auto fetch_keys = [&](int tile0) {
+      int page[PAGES + 1];
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
-        if (rt * 16 >= rows) break;
+      for (int p = 0; p < PAGES; ++p) page[p] = page_of(tile0 + row + 16 * (RB * p + block));
+      page[PAGES] = FULL < NC ? page_of(tile0 + ((tid & 255) >> 2)) : 0;
+      lost_keys = 0;
+#pragma unroll
+      for (int j = 0; j < UNITS; ++j) {
+        const int u = RB * j + block;
+        if (!keys_in(tile0, u)) continue;
+        const int p = RB * j < FULL ? page[j % PAGES] : page[PAGES];
+        const unsigned off = (unsigned)((g * page_size + page_offset(tile0 + key_of(u), page_size, shift)) * d +
+                                        min(channel_of(u), d - 4));
+        rk[j] = at_load4<T>(kv + (size_t)max(p, 0) * page_elems + off);
+        lost_keys |= p < 0 ? 1u << j : 0u;
+      }
+    };
+    auto fetch_values = [&](int tile0) {
+      if (!fours) return;
+      const int kp = tile0 + 4 * t16, page = page_of(kp), off = page_offset(kp, page_size, shift);
+      lost_values = page < 0;
+      const T* from = kv + (size_t)max(page, 0) * page_elems + value_base;
+#pragma unroll
+      for (int j = 0; j < UNITS; ++j) {
+        const int u = RB * j + block;
+        if (16 * u < dv) rv[j] = at_load4<T>(from + (unsigned)((g * dv + min(16 * u + row, dv - 1)) * page_size + off));
+      }
+    };
+    // (a key that is not there leaves a score that is not looked at; its value is to be zero, or no weight
+    // times it would be no number.  On a page that is gone both are zeros.)
+    auto stash_keys = [&](int tile0) {
+#pragma unroll
+      for (int j = 0; j < UNITS; ++j) {
+        const int u = RB * j + block;
+        if (!keys_in(tile0, u)) continue;
+        const bool ok = channel_of(u) < d && !(lost_keys >> j & 1);
+        *reinterpret_cast<f32x4_t*>(&Ks[key_of(u) * LDK + channel_of(u)]) = ok ? rk[j] : zero;
+      }
+    };
+    auto stash_values = [&](int tile0) {
+      if (!fours) {        // (odd page sizes: element by element, as they come)
+        const int kp = tile0 + (tid & 63);
+        const int page = there(kp) ? table[kp / page_size] : -1;
+        const T* from = kv + (size_t)max(page, 0) * page_elems + value_base + (size_t)g * dv * page_size + kp % page_size;
+#pragma unroll 8
+        for (int dd = wave; dd < dv; dd += 4 * RB)
+          Vt[dd * LDV + (tid & 63)] = page >= 0 ? to_f32<T>(from[(size_t)dd * page_size]) : 0.f;
+        return;
+      }
+      const int kp = tile0 + 4 * t16;
+      bool ok[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ok[e] = there(kp + e) && !lost_values;
+#pragma unroll
+      for (int j = 0; j < UNITS; ++j) {
+        const int u = RB * j + block;
+        if (16 * u >= dv) continue;
+        f32x4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = ok[e] ? rv[j][e] : 0.f;
+        *reinterpret_cast<f32x4_t*>(&Vt[(16 * u + row) * LDV + 4 * t16]) = v;
+      }
+    };
+
+    float m = -INFINITY, l = 0.f;         // l: of this lane's keys
+    // whether the wave has met a key that the row sees: until then what is in acc is no weight times values
+    // of other rows' keys, zeros, or, where such a value is infinite or undefined, to be thrown away
+    bool seen = false;
+    f32x4_t acc[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] = zero;
+
+    int tile0 = next_tile(kept_end > range_lo ? range_lo : tile_first);
+    if (tile0 <= range_hi) {
+      fetch_keys(tile0);
+      if (!TURNS) fetch_values(tile0);
+    }
+    while (tile0 <= range_hi) {
+      asm volatile("" : "+v"(t16), "+v"(row));      // (places of units: worked out anew, not kept in registers)
+      __syncthreads();  // the tile before has been read
+      stash_keys(tile0);
+      if (TURNS) fetch_values(tile0);
+      else stash_values(tile0);
+      __syncthreads();
+      const int wave_first = tile0 + part * 16, key0 = wave_first + quarter * 4;      // this lane's four keys
+      const int next = next_tile(tile0 + AT_KT);
+      if (!TURNS && next <= range_hi) {
+        fetch_keys(next);
+        fetch_values(next);
+      }
+      const bool mine = busy && wave_first <= range_hi;
+      f32x4_t s = zero;
+      if (mine) {
+        // (whole groups of 64 channels of wide heads: their reads of LDS overlap)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          if ((NC == 4 || c % 4 == 0) && 16 * c >= d) break;
+          const f32x4_t k = *reinterpret_cast<const f32x4_t*>(&Ks[(part * 16 + r16) * LDK + 16 * c + 4 * quarter]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], qf[c][e], s, 0, 0, 0);
+        }
         bool valid[4];
         float top = -INFINITY;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int kp = key0 + e;
           valid[e] = kp >= lo;
-          if (window > 0 && kp <= pos[rt] - window) valid[e] = false;
-          if (kp < chunk_start(ex, pos[rt])) valid[e] = false;
-          valid[e] = (valid[e] || kp < ex.keep) && kp <= pos[rt] && kp <= range_hi;
-          s[rt][e] = valid[e] ? capped_score(ex, s[rt][e] * temper[rt] * scale) : -INFINITY;
-          top = fmaxf(top, s[rt][e]);
+          if (window > 0 && kp <= pos - window) valid[e] = false;
+          if (kp < chunk_start(ex, pos)) valid[e] = false;
+          valid[e] = (valid[e] || kp < ex.keep) && kp <= pos && kp <= range_hi;
+          s[e] = valid[e] ? capped_score(ex, s[e] * temper * scale) : -INFINITY;
+          top = fmaxf(top, s[e]);
         }
-        const float m_new = fmaxf(m[rt], quad_max(top));
+        const float m_new = fmaxf(m, quad_max(top));
         // (no key yet, or scores of minus infinity only: no difference of infinities)
         const float m_use = m_new > -INFINITY ? m_new : 0.f;
-        const float alpha = m_new > -INFINITY ? expf(m[rt] - m_new) : 1.f;
+        const float alpha = m_new > -INFINITY ? expf(m - m_new) : 1.f;
         float own = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          s[rt][e] = valid[e] ? expf(s[rt][e] - m_use) : 0.f;
-          own += s[rt][e];
+          s[e] = valid[e] ? expf(s[e] - m_use) : 0.f;
+          own += s[e];
         }
-        l[rt] = l[rt] * alpha + own;
-        m[rt] = m_new;
-        if (seen[rt]) {
+        l = l * alpha + own;
+        m = m_new;
 #pragma unroll
-          for (int c = 0; c < NC; ++c) acc[rt][c] *= alpha;
-        } else {
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
-          for (int c = 0; c < NC; ++c) acc[rt][c] = zero;
-        }
-        const int wave_first = tile0 + wave * 16, last = min(pos[rt], range_hi);
-        int first = max(lo, chunk_start(ex, pos[rt]));
-        if (window > 0) first = max(first, pos[rt] - window + 1);
-        seen[rt] |= max(first, wave_first) <= min(last, wave_first + 15) || wave_first <= min(last, ex.keep - 1);
+          for (int e = 0; e < 4; ++e) acc[c][e] = seen ? acc[c][e] * alpha : 0.f;
+        const int last = min(pos, range_hi);
+        int first = max(lo, chunk_start(ex, pos));
+        if (window > 0) first = max(first, pos - window + 1);
+        seen |= max(first, wave_first) <= min(last, wave_first + 15) || wave_first <= min(last, ex.keep - 1);
       }
+      if (TURNS) {
+        __syncthreads();                // the keys have been read
+        stash_values(tile0);
+        if (next <= range_hi) fetch_keys(next);
+        __syncthreads();
+      }
+      if (mine) {
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        if (16 * c >= dv) break;
-        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&Vt[(16 * c + r16) * LDV + wave * 16 + 4 * quarter]);
+        for (int c = 0; c < NC; ++c) {
+          if ((NC == 4 || c % 4 == 0) && 16 * c >= dv) break;
+          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&Vt[(16 * c + r16) * LDV + part * 16 + 4 * quarter]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          acc[0][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], s[0][e], acc[0][c], 0, 0, 0);
-          if (rows > 16) acc[1][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], s[1][e], acc[1][c], 0, 0, 0);
+          for (int e = 0; e < 4; ++e) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], s[e], acc[c], 0, 0, 0);
         }
       }
+      tile0 = next;
     }
-    tile0 = next;
-  }
 
-  // ---- the waves' parts together
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const float sum = quad_sum(l[rt]);
-    if (quarter == 0) {
-      wave_m[wave][rt * 16 + r16] = m[rt];
-      wave_l[wave][rt * 16 + r16] = sum;
-    }
-  }
-  __syncthreads();      // (and the last tile has been read)
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    if (rt * 16 >= rows) break;
-    const int r = rt * 16 + r16;
-    const float top = fmaxf(fmaxf(wave_m[0][r], wave_m[1][r]), fmaxf(wave_m[2][r], wave_m[3][r]));
-    const float f = m[rt] > -INFINITY ? expf(m[rt] - top) : 0.f;
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-      if (16 * c < dv)
-        *reinterpret_cast<f32x4_t*>(&smem[(wave * AT_MAX_ROWS + r) * LDK + 16 * c + 4 * quarter]) =
-            seen[rt] ? acc[rt][c] * f : zero;
-  }
-  __syncthreads();
-  for (int idx = tid; idx < rows * dv; idx += 256) {
-    const int r = idx / dv, dd = idx - r * dv;
-    const int tok = row0 + r / G, h = g * G + r % G;
-    float top = wave_m[0][r];
-#pragma unroll
-    for (int w = 1; w < 4; ++w) top = fmaxf(top, wave_m[w][r]);
-    float total = 0.f, sum = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      total += wave_m[w][r] > -INFINITY ? wave_l[w][r] * expf(wave_m[w][r] - top) : 0.f;
-      sum += smem[(w * AT_MAX_ROWS + r) * LDK + dd];
-    }
-    if (nsplit == 1) {
-      if (ex.sink) total += expf(ex.sink[h] - top);
-      sum *= total > 0.f ? 1.0f / total : 0.f;
-      if (gate) {
-        const size_t col = gate_elem ? (size_t)h * dv + dd : (size_t)h;
-        const float gl = to_f32<T>(gate[(size_t)tok * gate_stride + gate_col + col]);
-        sum *= out_scale / (1.0f + expf(-gl));
+    // ---- the waves' parts together
+    {
+      const float sum = quad_sum(l);
+      if (quarter == 0) {
+        wave_m[wave][r16] = m;
+        wave_l[wave][r16] = sum;
       }
-      out[((size_t)tok * nh + h) * dv + dd] = from_f32<T>(sum);
-    } else {
-      const size_t pidx = ((size_t)tok * nh + h) * nsplit + z;
-      part_acc[pidx * dv + dd] = sum;
-      if (dd == 0) {
-        part_ml[pidx * 2] = top;
-        part_ml[pidx * 2 + 1] = total;
+    }
+    __syncthreads();      // (and the last tile has been read)
+    if (busy) {
+      const float(*peers)[16] = wave_m + 4 * block;
+      const float top = fmaxf(fmaxf(peers[0][r16], peers[1][r16]), fmaxf(peers[2][r16], peers[3][r16]));
+      const float f = m > -INFINITY ? expf(m - top) : 0.f;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        if (16 * c < dv)
+          *reinterpret_cast<f32x4_t*>(&smem[(wave * 16 + r16) * LDK + 16 * c + 4 * quarter]) = seen ? acc[c] * f : zero;
+    }
+    __syncthreads();
+    const int here = min(rows - first_row, 16 * RB);
+    for (int idx = tid; idx < here * dv; idx += 256 * RB) {
+      const int r = idx / dv, dd = idx - r * dv, first_wave = r >> 4 << 2, in_block = r & 15;
+      const int tok = row0 + (first_row + r) / G, h = g * G + (first_row + r) % G;
+      float top = wave_m[first_wave][in_block];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) top = fmaxf(top, wave_m[first_wave + w][in_block]);
+      float total = 0.f, sum = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float mw = wave_m[first_wave + w][in_block];
+        total += mw > -INFINITY ? wave_l[first_wave + w][in_block] * expf(mw - top) : 0.f;
+        sum += smem[((first_wave + w) * 16 + in_block) * LDK + dd];
+      }
+      if (nsplit == 1) {
+        if (ex.sink) total += expf(ex.sink[h] - top);
+        sum *= total > 0.f ? 1.0f / total : 0.f;
+        if (gate) {
+          const size_t col = gate_elem ? (size_t)h * dv + dd : (size_t)h;
+          const float gl = to_f32<T>(gate[(size_t)tok * gate_stride + gate_col + col]);
+          sum *= out_scale / (1.0f + expf(-gl));
+        }
+        out[((size_t)tok * nh + h) * dv + dd] = from_f32<T>(sum);
+      } else {
+        const size_t pidx = ((size_t)tok * nh + h) * nsplit + z;
+        part_acc[pidx * dv + dd] = sum;
+        if (dd == 0) {
+          part_ml[pidx * 2] = top;
+          part_ml[pidx * 2 + 1] = total;
+        }
       }
     }
   }
@@ -1182,7 +1204,7 @@ paged_attention_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restr
   }
 }
 
-template <typename T, int NC>
+template <typename T, int NC, int RB>
 static int launch_attention(const void* q, void* out, const void* kv, const int* block_table,
                             int bt_stride, const int* positions, const int* wi_seq,
                             const int* wi_row0, const int* wi_count, int n_items, float* part_acc,
@@ -1190,12 +1212,12 @@ static int launch_attention(const void* q, void* out, const void* kv, const int*
                             int window, int keys_per_split, int nsplit, int dv, const void* gate,
                             int gate_stride, int gate_col, float out_scale, ScoreExtras ex,
                             int gate_elem, hipStream_t stream) {
-  constexpr size_t shmem = at_lds<NC>() * sizeof(float);
-  auto kernel = paged_attention_kernel<T, NC>;
+  constexpr size_t shmem = at_lds<NC, RB>() * sizeof(float);
+  auto kernel = paged_attention_kernel<T, NC, RB>;
   static const hipError_t allowed = hipFuncSetAttribute(
       (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
   if (allowed != hipSuccess) return (int)allowed;
-  dim3 grid(n_items, nkv, nsplit), block(256);
+  dim3 grid(n_items, nkv, nsplit), block(256 * RB);
   hipLaunchKernelGGL(kernel, grid, block, shmem, stream, (const T*)q, (T*)out, (const T*)kv,
                      block_table, bt_stride, positions, wi_seq, wi_row0, wi_count, part_acc,
                      part_ml, nh, nkv, d, page_size, scale, window, keys_per_split, nsplit, dv,
@@ -1341,15 +1363,25 @@ static int paged_attention_any(const void* q, void* out, const void* kv, const i
       part_ml, nh, nkv, d, page_size, scale, window, keys_per_split, nsplit, dv, gate,         \
       gate_stride, gate_col, out_scale, ex, gate_elem, stream
   const int wide = d > dv ? d : dv;
+  // single tokens (an item with more rows than 16 takes them in turn all the same): four waves, three or two
+  // workgroups a compute unit; heads beyond 128 have no registers for a tile in four waves
+  const bool few = n_items >= n_tokens && nh / nkv <= 16 && wide <= 128;
+#define ZA_AT_WIDE(T)                                                                            \
+  rc = few ? wide <= 64 ? launch_attention<T, 4, 1>(ZA_AT_ARGS)                                  \
+             : wide <= 80 ? launch_attention<T, 5, 1>(ZA_AT_ARGS)                                \
+             : launch_attention<T, 8, 1>(ZA_AT_ARGS)                                             \
+       : wide <= 64 ? launch_attention<T, 4, 2>(ZA_AT_ARGS)                                      \
+       : wide <= 80 ? launch_attention<T, 5, 2>(ZA_AT_ARGS)                                      \
+       : wide <= 128 ? launch_attention<T, 8, 2>(ZA_AT_ARGS)                                     \
+       : wide <= 192 ? launch_attention<T, 12, 2>(ZA_AT_ARGS) : launch_attention<T, 16, 2>(ZA_AT_ARGS)
   if (dtype == 0) {
-    rc = wide <= 64 ? launch_attention<float, 4>(ZA_AT_ARGS)
-         : wide <= 128 ? launch_attention<float, 8>(ZA_AT_ARGS) : launch_attention<float, 16>(ZA_AT_ARGS);
+    ZA_AT_WIDE(float);
   } else if (dtype == 1) {
-    rc = wide <= 64 ? launch_attention<bf16_t, 4>(ZA_AT_ARGS)
-         : wide <= 128 ? launch_attention<bf16_t, 8>(ZA_AT_ARGS) : launch_attention<bf16_t, 16>(ZA_AT_ARGS);
+    ZA_AT_WIDE(bf16_t);
   } else {
     return ZA_ERR_UNSUPPORTED;
   }
+#undef ZA_AT_WIDE
 #undef ZA_AT_ARGS
   if (rc != 0 || nsplit == 1) return rc;
   const size_t merged = (size_t)n_tokens * nh;

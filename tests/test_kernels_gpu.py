@@ -1809,12 +1809,13 @@ def test_grouped_products_at_the_edges_of_their_tiles(dtype, E, top, N, K, T):
     assert torch.equal(alone, whole[:top])
 
 
-@pytest.mark.parametrize("K", [64, 128, 192, 256, 320])
-@pytest.mark.parametrize("columns,top", [(1700, 1), (3300, 1), (3304, 2)])
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 512, 576, 640])
+@pytest.mark.parametrize("columns,top", [(1700, 1), (2500, 1), (3300, 1), (3304, 2)])
 def test_grouped_products_in_wide_tiles(K, columns, top):
-    """Steps of many rows, in tiles of 256 or (few outputs) 128 assignments: counts around the tiles'
-    edges and an empty expert, one to five steps of K, outputs off multiples of a tile; the same bits
-    as a token on its own has, which takes the low tiles."""
+    """Steps of many rows, from 512 elements of K on in tiles of 256 or (2,500 outputs) 128 assignments,
+    below in the low tiles: counts around the tiles' edges and an empty expert, whole steps of K even and
+    odd, outputs off multiples of a tile; the same bits as a token on its own has, which takes the low
+    tiles."""
     o = ops()
     want = [1, 127, 128, 129, 255, 256, 257, 0, 384, 385, 513]
     E = len(want) + 1

@@ -29,6 +29,7 @@
 //    does not depend on which other tokens share its expert or its tile.
 //      bfloat16: matrix cores (v_mfma_f32_16x16x32_bf16), tiles through LDS.
 //      32-bit: tiles of 32 x 64 on the matrix cores' 32-bit instruction (gemm_f32.h).
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -482,10 +483,23 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     // token, 1,900 tokens: up 99 -> 64 (128 high 85), down, 128 high for want of tiles, 92 -> 75 (256
     // high 95); 500 tokens: up, 128 high, 56 -> 43, down stays (54 against 66).  The sums are the same
     // to the last bit.
+    // And only where the rounds that the tiles make, 256 of them at a time or 512 of the low ones, take no
+    // longer (few steps of K, outputs that fill little of a wide tile, a wide round that is nearly empty
+    // where the low tiles make whole ones): a round of 128 x 128, two to a compute unit, as K, of 128 x 256 as
+    // 0.9 K + 400, of 256 x 256 as 1.2 K + 400, an expert's last tile of those half as long; fitted to 420
+    // products of 300 to 64,000 rows, 64 to 8,192 outputs and 128 to 4,096 elements of K (us, low and wide):
+    // 32 experts, 4 a token, gated, 8,000 tokens, 64 x 2,048 38 and 67; 4,000 tokens, 192 x 2,048 41 and 70;
+    // 8 experts, 2 a token, gated, 12,000 tokens, 320 x 2,048 79 and 112, 448 x 2,048 115 and 117, 640 x
+    // 2,048 157 and 131; not gated, 640 x 2,048 76 and 96, 512 x 2,048 72 and 56.
     if (K % GG_BK == 0 && A >= 80LL * experts) {
       const long long columns = (N + (gate ? 127 : 255)) / (gate ? 128 : 256);
-      const int high = (A / 256 + experts / 2) * columns >= 176 ? 256
-                       : (A / 128 + experts / 2) * columns >= 150 ? 128 : 0;
+      int high = (A / 256 + experts / 2) * columns >= 176 ? 256
+                 : (A / 128 + experts / 2) * columns >= 150 ? 128 : 0;
+      const double tiles128 = A / 128.0 + experts / 2.0, low_columns = (N + (gate ? 63 : 127)) / (gate ? 64 : 128);
+      const double low = ceil(tiles128 * low_columns / 512 + 0.06) * K;
+      const double wide = high == 256 ? ceil((A / 256.0 + experts / 4.0) * columns / 128) / 2 * (1.2 * K + 400)
+                                      : ceil(tiles128 * columns / 256) * (0.9 * K + 400);
+      if (wide > low) high = 0;
       // (an expert's full tiles and its last one, each kind an eighth a die)
       const long long tiles = (A + high - 1) / max(high, 1) + experts;
       const long long blocks = (tiles * columns + 7) / 8 * 8 + 8;

@@ -142,10 +142,10 @@ def test_gemm_f32_order_of_sums(N, K):
     assert torch.equal(ops().linear(x[:33].contiguous(), w, bias), whole[:33] + bias)
 
 
-@pytest.mark.parametrize("K", [32, 96, 128, 160, 512, 544, 672])
+@pytest.mark.parametrize("K", [32, 96, 128, 160, 512, 544, 672, 736, 768, 800, 1056])
 @pytest.mark.parametrize("M,N", [(130, 2100), (200, 4001), (130, 6000), (65, 16385)])
 def test_gemm_f32_steps_through_lds(M, N, K):
-    """K of whole steps of 32, below, at and off whole chains of 128 and what two and four groups take
+    """K of whole steps of 32, below, at and off whole chains of 128 and what one, two and four groups take
     together: right, and the bits of rows on their own, which another kernel takes."""
     x, w = rand((M, K), torch.float32, 63).to(dev()), rand((N, K), torch.float32, 64).to(dev())
     whole = ops().linear(x, w)

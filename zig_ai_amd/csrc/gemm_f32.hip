@@ -61,9 +61,13 @@ static int launch_f32(const TA* A, const float* W, const float* bias, TC* C, int
     // several layers in turn, before and now: 448 x 9216 x 1024 101 and 91, 448 x 3072 x 1024 40 and
     // 38, 448 x 2048 x 1024 27 and 25, 448 x 1024 x 4608 61 and 59, 100 x 9216 x 1024 42 and 38,
     // 512 x 16384 x 2048 333 and 305 (113 TFLOP/s), 500 x 2048 x 8192 199 and 179.
+    // Tiles of 32 x 64 with a second group of waves from six chains of K on: with fewer it waits for the
+    // first (one chain: it has none of its own).  Registers, two groups, one: 65 x 16384 x 96 6, 8, 6,
+    // 130 x 16384 x 384 26, 29, 28, 130 x 65536 x 384 86, 97, 84, x 768 169, 170, 170.
     if (K % F32_BK == 0 && n32 > 256) {
       if (n3264 <= 256) ZA_F32_ASYNC(32, 64, 4, 2)
       if (n64 <= 256 || ((n64 + 255) / 256) * 200 <= ((n3264 + 255) / 256) * 115) ZA_F32_ASYNC(64, 64, 1, 3)
+      if (K < 768) ZA_F32_ASYNC(32, 64, 1, 3)
       ZA_F32_ASYNC(32, 64, 2, 3)
     }
 #undef ZA_F32_ASYNC

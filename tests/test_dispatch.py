@@ -142,3 +142,16 @@ def test_where_a_router_runs_in_one_kernel():
     # steps beyond 64 tokens, where a launch costs more
     assert pays(65, 80, 1024) and pays(1777, 48, 2048) and pays(8192, 16, 4096)
     assert not pays(65, 64, 2048) and not pays(1777, 32, 2560) and not pays(4096, 16, 5120)
+
+
+def test_how_far_portions_over_planes_are_cut():
+    """Beyond one workgroup a compute unit where walks differ in length and two workgroups share a
+    compute unit; not where ranges only add a merge."""
+    from zig_ai_amd.parts.attention import planes_target
+    most, least = planes_target(128, 64, 1200, True, True), planes_target(128, 128, 1200, True, True)
+    assert (most, least) == (400, 256)
+    assert planes_target(64, 64, 1200, True, True) == planes_target(96, 96, 5000, True, False) == most
+    assert planes_target(128, 64, 3000, False, False) == planes_target(72, 8, 800, False, False) == most
+    assert planes_target(128, 64, 1028, False, True) == planes_target(64, 64, 3000, False, False) == least
+    assert planes_target(128, 64, 700, True, False) == planes_target(192, 96, 3000, True, False) == least
+    assert planes_target(136, 64, 3000, False, False) == planes_target(128, 104, 3000, True, False) == least

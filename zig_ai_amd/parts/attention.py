@@ -109,6 +109,27 @@ def plan_split(n_items: int, num_kv_heads: int, max_keys: int, target: int = SPL
     return (keys, nsplit) if nsplit > 1 else (0, 1)
 
 
+def planes_target(head_dim: int, value_dim: int, keys: int, mixed: bool, limited: bool) -> int:
+    """The workgroups up to which ``planes_attention`` cuts the contexts of prompt portions into ranges.
+    An item's walk over its tiles is a chain, and the longest decides where items differ: single tokens of
+    long contexts beside portions (``mixed``), or contexts that grow along a prompt (not ``limited`` by a
+    window or chunk, behind which all walks are the same).  There three workgroups for two compute units
+    pay, where two of the kernel's share one (heads up to 128 with values up to 96); elsewhere, and below
+    some 800 keys, the ranges' merge costs more than it gives.  Measured (us, cut for 256 and for 400;
+    16 heads on 4 key heads, keys of 128 and values of 64 unless stated):
+      5 single tokens at 1,200 keys, portions of 512 and 512      35, 28   (values of 128 38, 30)
+      20 at 900, a portion of 512 at 1,500                         38, 31
+      a portion of 1,100 at 3,000 keys                            105, 75  (behind a window of 1,024 38, 39)
+      a portion of 1,400 at 3,000 keys, window                     38, 42  (values of 128 44, 61)
+      prompts of 700 and 400                                       23, 25  (32 on 8 of 64: 700 18, 26)
+      a portion of 900 at 2,000, values of 128                     59, 76
+      32 heads on 8 of 64, a portion of 800 at 1,000 keys          25, 33"""
+    shared = head_dim <= 128 and value_dim <= 96
+    if shared and keys > 768 and (mixed or (not limited and head_dim > 64)):
+        return PLANES_PORTION_TARGET
+    return SPLIT_TARGET
+
+
 def _round_up8(n: int) -> int:
     return -(-int(n) // 8) * 8
 
@@ -521,8 +542,11 @@ class GroupedQueryAttention(Mixer):
             if step.n_tokens > step.n_seqs or self.group > ops.PLANES_DECODE_GROUP:
                 items = step.attention_items(self.planes_rows_per_item)
             # (an item's list of tiles is cut, not the context: behind a window it stays short)
-            tiles, nsplit = self._plan_tiles(items[3] if items else step.n_seqs,
-                                             self._reach(step.max_keys), items is not None)
+            reach = self._reach(step.max_keys)
+            target = SPLIT_TARGET if items is None else planes_target(
+                d, dv, reach, step.portions_below(2).requests > 0, reach < step.max_keys)
+            keys, nsplit = plan_split(items[3] if items else step.n_seqs, nkv, reach, target=target)
+            tiles = -(-keys // ops.PLANES_TILE_KEYS)
             o = ops.planes_attention(q, key_plane, value_plane, table, step.positions, items,
                                      self.scale, self.window, tiles, nsplit, shape=self.shape)
         else:
@@ -544,17 +568,6 @@ class GroupedQueryAttention(Mixer):
             if limit:
                 max_keys = min(max_keys, limit + self.keep_first)
         return max_keys
-
-    def _plan_tiles(self, n_items: int, keys: int, portions: bool):
-        """``plan_split`` in tiles of the kernel.  (Prompt portions are cut while that stays within
-        400 workgroups, three for two compute units: an item's walk over its tiles is a chain, and two
-        of them on a compute unit hide each other's waits, but the ranges have to be merged.  Steps of 862 to
-        1,029 tokens of 16 heads on 4 key heads behind a window of 1,024, 132 to 148 workgroups whole:
-        a step's time whole 4,239 us, cut for 320 workgroups 4,150, for 400 4,084, for 511 4,097.
-        2,048 tokens, 256 workgroups: 36.7 us whole, 45.1 in two ranges.)"""
-        per_range, nsplit = plan_split(n_items, self.num_kv_heads, keys,
-                                       **({"target": PLANES_PORTION_TARGET} if portions else {}))
-        return -(-per_range // ops.PLANES_TILE_KEYS), nsplit
 
     def _leave_taps(self, step, cache, q: torch.Tensor, o: torch.Tensor) -> None:
         """Diagnostics: the queries, the keys and values of the step's tokens as they lie in

@@ -1313,6 +1313,73 @@ def test_ranges_merged(d, nsplit):
     assert ((got - want).abs() <= want.abs() * 2.0 ** -8 + sums).all()     # and one rounding to bfloat16
 
 
+def _empty_ranges(n, *shape):
+    acc, ml = torch.full(shape[:-1] + (n, shape[-1]), math.nan), torch.zeros(shape[:-1] + (n, 2))
+    ml[..., 0] = -math.inf
+    return acc, ml
+
+
+@pytest.mark.parametrize("nsplit", [9, 16, 17, 40, 64])
+@pytest.mark.parametrize("d", [8, 72, 128, 256])
+def test_many_ranges_merged_to_the_bits_of_few(d, nsplit):
+    """The kernel for 9 to 64 ranges against the one for any number, which merges the same ranges with empty
+    ones up to 65 behind them."""
+    gen = torch.Generator().manual_seed(d * nsplit)
+    acc = torch.randn((7, 3, nsplit, d), generator=gen)
+    ml = torch.stack([torch.randint(-30, 9, (7, 3, nsplit), generator=gen).float(),
+                      torch.rand((7, 3, nsplit), generator=gen) * 40], dim=-1)
+    ml[2, 1, nsplit // 3] = torch.tensor([-math.inf, 0.0])
+    more_acc, more_ml = _empty_ranges(65 - nsplit, 7, 3, d)
+    many = ops().MergedRows(acc.to(dev()), ml.to(dev())).materialise()
+    few = ops().MergedRows(torch.cat([acc, more_acc], 2).to(dev()), torch.cat([ml, more_ml], 2).to(dev())).materialise()
+    assert torch.equal(many, few)
+
+
+@pytest.mark.parametrize("nsplit", [9, 16, 33, 64])
+@pytest.mark.parametrize("kernel", ["general", "general bfloat16", "decode", "portions", "planes"])
+def test_sinks_in_merges_of_many_ranges(kernel, nsplit):
+    """The same through the attention kernels that merge with a sink, on either base: contexts of up to
+    ``nsplit`` ranges, cut into that many and into 65."""
+    dtype = torch.float32 if kernel == "general" else torch.bfloat16
+    nh, nkv, d, ps = 4, 2, 64, 16
+    ctx = [64 * nsplit - 3, 64 * (nsplit - 2) + 5, 130, 0]
+    new = [1, 1, 1, 1] if kernel != "portions" else [3, 1, 5, 2]
+    ks, vs, q, pos = [], [], [], []
+    for s, (c, n) in enumerate(zip(ctx, new)):
+        ks.append(rand((c + n, nkv, d), dtype, 700 + s))
+        vs.append(rand((c + n, nkv, d), dtype, 710 + s))
+        q.append(rand((n, nh, d), dtype, 720 + s))
+        pos += list(range(c, c + n))
+    cache, table = paged_from_dense(ks, vs, ps, dtype)
+    cache, table, pos = cache.to(dev()), table.to(dev()), torch.tensor(pos, dtype=torch.int32, device=dev())
+    q, sink = torch.cat(q).to(dev()), torch.tensor([1.5, -2.0, 0.0, 4.0], device=dev())
+    shape = ops().ScoreShape(sink=sink)
+
+    def run(n):
+        if kernel.startswith("general"):
+            return ops().paged_attention(q, cache, table, pos, *items_for(new, 16), d ** -0.5, 0, 64, n, shape=shape)
+        if kernel == "decode":
+            return ops().paged_attention_decode_mfma(q, cache, table, pos, None, None, None, len(new), d ** -0.5, 0,
+                                                     64, n, shape=shape)
+        if kernel == "portions":
+            return ops().paged_attention_mfma(q, cache, table, pos, *items_for(new, 64), d ** -0.5, 0, 64, n, shape=shape)
+        flat = cache.view(-1)
+        per = 2 * nkv * ps * d
+        planes = [flat.as_strided((cache.shape[0], nkv, ps, d), (per, ps * d, d, 1), o) for o in (0, nkv * ps * d)]
+        return ops().planes_attention(q, *planes, table, pos, None, d ** -0.5, 0, 1, n, shape=shape)
+
+    many, few = run(nsplit), run(65)
+    assert torch.equal(many, few)
+    row = 0
+    for k, v, c, n in zip(ks, vs, ctx, new):
+        for i in range(n):
+            s = torch.einsum("hd,jhd->hj", q[row].double().cpu(), k[:c + i + 1].double().repeat_interleave(2, 1)) * d ** -0.5
+            e = torch.exp(torch.cat([s, sink.double().cpu()[:, None]], 1))
+            want = torch.einsum("hj,jhd->hd", e[:, :-1] / e.sum(1, keepdim=True), v[:c + i + 1].double().repeat_interleave(2, 1))
+            assert rel_err(many[row], want) < (F32_TOL if dtype == torch.float32 else 2e-2)
+            row += 1
+
+
 def decode_step_case(nh, nkv, d, page_size, positions, seed):
     """A decode step: request i holds positions[i] cached tokens and brings one more.
     Returns qkv [T, (nh + 2 nkv) d], the cache with random contents in the requests' pages
@@ -1801,6 +1868,10 @@ def test_grouped_products_at_the_edges_of_their_tiles(dtype, E, top, N, K, T):
                            gate="gelu_tanh", rounded=True)
     both = o.grouped_linear(x.to(dev()), gate_up.to(dev()), lists, counts, T, per_token=True, out_dtype=dtype)
     assert torch.equal(got, o.gated_unit(both, "gelu_tanh"))
+    row_weight = torch.rand((T, top), generator=torch.Generator().manual_seed(T)).to(dev())
+    got = o.grouped_linear(x.to(dev()), gate_up.to(dev()), lists, counts, T, per_token=True, out_dtype=dtype,
+                           bounded=(0.7, 1.702, 1.0), row_weight=row_weight, rounded=True)
+    assert torch.equal(got, o.clamped_glu(both, 0.7, 1.702, 1.0, row_weight.view(-1)))
     # (a row's bits do not depend on the other tokens of its step)
     l1, c1 = o.expert_lists(None, chosen[:1].contiguous().to(dev()), 1, E)
     alone = o.grouped_linear(x[:1].contiguous().to(dev()), w.to(dev()), l1, c1, 1, per_token=True,
@@ -1843,6 +1914,12 @@ def test_grouped_products_in_wide_tiles(K, columns, top):
     unit = torch.nn.functional.silu(full[:, :columns // 2]) * full[:, columns // 2:]
     gated = o.grouped_linear(xd, wd, lists, counts, T, per_token=True, out_dtype=torch.bfloat16, gate="silu")
     assert rel_err(gated, unit) < tol_of(torch.bfloat16)
+    both = o.grouped_linear(xd, wd, lists, counts, T, per_token=True, out_dtype=torch.bfloat16)
+    assert torch.equal(o.gated_unit(both, "silu"), o.grouped_linear(
+        xd, wd, lists, counts, T, per_token=True, out_dtype=torch.bfloat16, gate="silu", rounded=True))
+    bounds, shares = (0.7, 1.702, 1.0), weight.abs().to(dev())
+    assert torch.equal(o.clamped_glu(both, *bounds, shares.view(-1)), o.grouped_linear(
+        xd, wd, lists, counts, T, per_token=True, out_dtype=torch.bfloat16, bounded=bounds, row_weight=shares, rounded=True))
     for t in (0, T // 2, T - 1):
         l1, c1 = o.expert_lists(None, chosen[t:t + 1].contiguous().to(dev()), 1, E)
         one = dict(lists=l1, counts=c1, n_tokens=1, per_token=True)

@@ -486,6 +486,47 @@ def test_matrix_core_paths(dim, heads, kv):
         assert_bfloat16_same(torch.cat(got), torch.cat(base), name)
 
 
+@pytest.mark.parametrize("reproducible", [False, True])
+@pytest.mark.parametrize("B", [8, 20])
+def test_feed_forwards_beside_the_mixer_at_real_width(B, reproducible):
+    """Decode steps whose dense feed-forward opens in ranges of K (beyond 16 requests) and leaves a stack of
+    partial sums pending where it may not add to the stream itself, and whose experts leave one plane a
+    choice: read by the next norm, by the loop's mix and by the last norm for some of the rows only."""
+    from zig_ai_amd.engine import DecoderModel, StepEntry
+    from zig_ai_amd.kernels import ops
+    cfg = nu.config([
+        nu.layer("attention", nu.attention(heads=8, kv_heads=2, dim=64, scale=0.125, chunk=100, rot_dims=32, base=1e4),
+                 nu.dense(3072)),
+        nu.layer("lightning", nu.lightning(heads=3, dim=64, vdim=32), nu.moe(ff=256, experts=4, top=2)),
+        nu.layer("attention_2", nu.attention_2(heads=8, kv_heads=2, dim=64, vdim=64, scale=0.125, conv=4, rot_dims=64),
+                 nu.dense(3072)),
+    ], width=1024, vocab=211, loop=(0, 2, 2))
+    d, tensors = nu.folder(cfg, 21)
+    model = DecoderModel.from_folder(d, "bfloat16", reproducible=reproducible)
+    runner = runner_for(model, page_size=16, tokens=16 * B, slots=B, graphs=False)
+    steps, prompts = 3, [nu.tokens(4 + i % 6, cfg["vocab"], 90 + i) for i in range(B)]
+    want = [w[-steps:] for w in plain_logits(cfg, tensors, prompts)]
+    for i in range(B):
+        runner.admit(i)
+    runner.step([StepEntry(i, p[:-steps], []) for i, p in enumerate(prompts)])
+    asked, got, expected = [i for i in range(B) if i % 3], [], []
+    for j in range(steps):
+        ops.form_log = []
+        try:
+            got.append(runner.step([StepEntry(i, [p[j - steps]], [0] if i in asked else [])
+                                    for i, p in enumerate(prompts)]).cpu())
+        finally:
+            log, ops.form_log = ops.form_log, None
+        expected += [want[i][j] for i in asked]
+        linear = [r for r in log if r["op"] == "linear" and r["M"] == B]
+        up = [r for r in linear if (r["N"], r["K"]) == (3072, 1024)]
+        down = [r for r in linear if (r["N"], r["K"]) == (1024, 3072)]
+        assert len(up) == len(down) == 3                          # two passes and the last layer
+        assert all((r["partial_sums"] > 1) == (B > 16) for r in up)
+        assert all(r["added_to_stream"] != reproducible and (r["partial_sums"] > 1) == reproducible for r in down)
+    assert_bfloat16_close(torch.cat(got), torch.stack(expected))
+
+
 # ------------------------------------------- generation through engine and scheduler
 def test_greedy_generation():
     from zig_ai_amd.engine import Engine

@@ -481,48 +481,40 @@ extern "C" int za_decay_chunked(const float* vec, int width, int q_col, int k_co
   if (dtype != 0 && dtype != 1) return ZA_ERR_UNSUPPORTED;
   const long long elems = (long long)H * dk * dv;
   if (dk > 128 || elems > 0x7fffffffLL || H > 65535) return ZA_ERR_UNSUPPORTED;
+  if ((reinterpret_cast<uintptr_t>(scores) & 15) != 0) return ZA_ERR_ARG;
   const DecayArgs a{vec, width, q_col, k_col, x_col, proj, proj_stride, gate_col, dtype, dt_bias, A_log, D,
                     fixed, item_row0, item_count, sums, chunk_state, total, out, H, G, dk, dv, scores};
   dim3 grid(n_items, H, (dv + 63) / 64);
   const dim3 block(256);
   const bool full = dv % 64 == 0 && width % 4 == 0 && q_col % 4 == 0 && k_col % 4 == 0 &&
                     ((reinterpret_cast<uintptr_t>(vec) | reinterpret_cast<uintptr_t>(chunk_state)) & 15) == 0;
-#define ZA_DECAY(KERNEL)                                                                       \
+#define ZA_DECAY(KERNEL, ...)                                                                  \
   {                                                                                            \
-    if (full && dk == 64) hipLaunchKernelGGL((KERNEL<4, true>), grid, block, 0, stream, a);    \
-    else if (full && dk == 128) hipLaunchKernelGGL((KERNEL<8, true>), grid, block, 0, stream, a); \
-    else if (dk <= 32) hipLaunchKernelGGL((KERNEL<2, false>), grid, block, 0, stream, a);      \
-    else if (dk <= 64) hipLaunchKernelGGL((KERNEL<4, false>), grid, block, 0, stream, a);      \
-    else hipLaunchKernelGGL((KERNEL<8, false>), grid, block, 0, stream, a);                    \
+    if (full && dk == 64) hipLaunchKernelGGL((KERNEL<4, true __VA_ARGS__>), grid, block, 0, stream, a);    \
+    else if (full && dk == 128) hipLaunchKernelGGL((KERNEL<8, true __VA_ARGS__>), grid, block, 0, stream, a); \
+    else if (dk <= 32) hipLaunchKernelGGL((KERNEL<2, false __VA_ARGS__>), grid, block, 0, stream, a);      \
+    else if (dk <= 64) hipLaunchKernelGGL((KERNEL<4, false __VA_ARGS__>), grid, block, 0, stream, a);      \
+    else hipLaunchKernelGGL((KERNEL<8, false __VA_ARGS__>), grid, block, 0, stream, a);                    \
     const int rc = za_launch_status();                                                         \
     if (rc != 0) return rc;                                                                    \
   }
+#define ZA_COMMA ,
   ZA_DECAY(decay_chunk_state_kernel)
   hipLaunchKernelGGL(decay_prefix_kernel, dim3(n_seqs, (unsigned)((elems + 255) / 256)), dim3(256), 0, stream,
                      chunk_state, state, slot_stride, slot_id, item_seq, n_items, total, (int)elems, H, dk * dv);
   const int rc = za_launch_status();
   if (rc != 0) return rc;
   if (scores) {
-    if ((reinterpret_cast<uintptr_t>(scores) & 15) != 0 || G > 65535) return ZA_ERR_ARG;
     const dim3 by_heads = grid;
     grid = dim3(n_items, G, DC_CHUNK / 16);
     ZA_DECAY(decay_chunk_scores_kernel)
     grid = by_heads;
-#define ZA_SHARED(NT, FULL) decay_chunk_out_kernel<NT, FULL, true>
-    if (full && dk == 64) hipLaunchKernelGGL((ZA_SHARED(4, true)), grid, block, 0, stream, a);
-    else if (full && dk == 128) hipLaunchKernelGGL((ZA_SHARED(8, true)), grid, block, 0, stream, a);
-    else if (dk <= 32) hipLaunchKernelGGL((ZA_SHARED(2, false)), grid, block, 0, stream, a);
-    else if (dk <= 64) hipLaunchKernelGGL((ZA_SHARED(4, false)), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((ZA_SHARED(8, false)), grid, block, 0, stream, a);
-#undef ZA_SHARED
-    return za_launch_status();
+    ZA_DECAY(decay_chunk_out_kernel, ZA_COMMA true)
+  } else {
+    ZA_DECAY(decay_chunk_out_kernel, ZA_COMMA false)
   }
-  if (full && dk == 64) hipLaunchKernelGGL((decay_chunk_out_kernel<4, true, false>), grid, block, 0, stream, a);
-  else if (full && dk == 128) hipLaunchKernelGGL((decay_chunk_out_kernel<8, true, false>), grid, block, 0, stream, a);
-  else if (dk <= 32) hipLaunchKernelGGL((decay_chunk_out_kernel<2, false, false>), grid, block, 0, stream, a);
-  else if (dk <= 64) hipLaunchKernelGGL((decay_chunk_out_kernel<4, false, false>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((decay_chunk_out_kernel<8, false, false>), grid, block, 0, stream, a);
-  return za_launch_status();
+  return 0;
+#undef ZA_COMMA
 #undef ZA_DECAY
 }
 

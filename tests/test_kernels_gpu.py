@@ -1242,6 +1242,21 @@ def test_paged_attention_widths(dtype, nh, nkv, d, page_size):
         assert rel_err(out, expect) < tol_of(dtype), (new, window, nsplit)
 
 
+@pytest.mark.parametrize("nsplit", [1, 2])
+@pytest.mark.parametrize("nh,nkv", [(2, 2), (4, 2)])
+def test_paged_attention_items_without_rows(nh, nkv, nsplit):
+    """A work item of no rows, the first among them, is none: nothing is read or written for it."""
+    d, T, c = 64, 6, 70
+    k, v, q = (rand(s, torch.float32, 420 + i) for i, s in enumerate(((c + T, nkv, d), (c + T, nkv, d), (T, nh, d))))
+    cache, table = paged_from_dense([k], [v], 16, torch.float32)
+    pos = torch.arange(c, c + T, dtype=torch.int32, device=dev())
+    mk = lambda x: torch.tensor(x, dtype=torch.int32, device=dev())
+    args = (q.to(dev()), cache.to(dev()), table.to(dev()), pos)
+    got = ops().paged_attention(*args, mk([0] * 4), mk([0, 0, 3, 3]), mk([0, 3, 0, 3]), 4, d ** -0.5, 0, 64, nsplit)
+    want = ops().paged_attention(*args, mk([0, 0]), mk([0, 3]), mk([3, 3]), 2, d ** -0.5, 0, 64, nsplit)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("d", [64, 80, 104])
 def test_paged_attention_items_that_overlap(d):
     """As many work items as tokens, which a step of single tokens has, but each of several tokens and
@@ -1833,7 +1848,8 @@ def test_repetition_penalty():
 # ------------------------------------------------------------------- experts
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("E,top,N,K,T", [(8, 2, 72, 64, 1), (8, 3, 130, 200, 40), (3, 1, 256, 192, 200),
-                                         (6, 2, 66, 136, 330), (70, 4, 64, 40, 600), (1, 1, 20, 8, 5)])
+                                         (6, 2, 66, 136, 330), (70, 4, 64, 40, 600), (1, 1, 20, 8, 5),
+                                         (90, 4, 330, 72, 200), (64, 2, 300, 64, 900), (64, 2, 700, 64, 900)])
 def test_grouped_products_at_the_edges_of_their_tiles(dtype, E, top, N, K, T):
     """Every height of tile (32, 64 and 128 assignments, by the rows an expert has on average), K
     below, at and off multiples of a step of 64, outputs off multiples of a tile and of four,

@@ -130,6 +130,7 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
   const int seq = wi_seq[item];
   const int row0 = wi_row0[item];
   int count = wi_count[item];
+  if (count <= 0) return;
   if (count * G > AT_MAX_ROWS) count = AT_MAX_ROWS / G;  // the host never asks for more
   const int rows = count * G;
   const int* table = block_table + (size_t)seq * bt_stride;

@@ -1945,6 +1945,48 @@ def test_grouped_products_in_wide_tiles(K, columns, top):
                                             **one), gated[mine])
 
 
+@pytest.mark.parametrize("E,top,K,columns", [(12, 3, 1024, 2304), (12, 1, 1088, 2311), (70, 7, 512, 640), (70, 2, 576, 1288)])
+def test_grouped_products_whose_experts_end_in_each_height_of_tile(E, top, K, columns):
+    """Wide tiles of 256, 192 and 128: an expert's rest of 0, 1, 128, 129, 192, 193 and 255 assignments behind
+    none, one and two full tiles, experts beyond the first 64, tokens of which several assignments fall
+    to one place of the lists; against 64-bit sums, and the bits that tokens on their own have."""
+    o = ops()
+    rests = [0, 1, 128, 129, 192, 193, 255]
+    want = [256 * ((e // 3) % 3) + rests[e % 7] for e in range(E)]
+    want[-1] += -sum(want) % top
+    A = sum(want)
+    chosen = torch.cat([torch.full((n,), e) for e, n in enumerate(want)])
+    chosen = chosen[torch.randperm(A, generator=torch.Generator().manual_seed(E + K))].int().view(-1, top).contiguous()
+    T = chosen.shape[0]
+    lists, counts = o.expert_lists(None, chosen.to(dev()), T, E)
+    assert counts.tolist() == want
+    x, w = rand((T, K), torch.bfloat16, 83).to(dev()), rand((E, columns, K), torch.bfloat16, 84, K ** -0.5).to(dev())
+    which = chosen.view(-1).long().to(dev())
+    rows = x.double().repeat_interleave(top, 0)
+    full = torch.empty((A, columns), dtype=torch.double, device=dev())
+    for e in range(E):
+        full[which == e] = rows[which == e] @ w[e].double().T
+    got = o.grouped_linear(x, w, lists, counts, T, per_token=True, out_dtype=torch.float32)
+    assert rel_err(got, full.cpu()) < F32_TOL
+    planes = o.grouped_linear(rows.bfloat16(), w, lists, counts, T, per_token=False, stacked=True)
+    assert torch.equal(planes, got.view(T, top, columns).transpose(0, 1))
+    short = o.grouped_linear(x, w, lists, counts, T, per_token=True, out_dtype=torch.bfloat16)
+    assert torch.equal(short, got.bfloat16())
+    if columns % 2 == 0:
+        for gate in ("silu", "gelu_tanh"):
+            unit = o.grouped_linear(x, w, lists, counts, T, per_token=True, out_dtype=torch.bfloat16, gate=gate, rounded=True)
+            assert torch.equal(unit, o.gated_unit(short, gate))
+            exact = o.grouped_linear(x, w, lists, counts, T, per_token=True, out_dtype=torch.float32, gate=gate)
+            v, u = full[:, :columns // 2], full[:, columns // 2:]
+            v = torch.nn.functional.silu(v) if gate == "silu" else torch.nn.functional.gelu(v, approximate="tanh")
+            assert rel_err(exact, (v * u).cpu()) < 4 * F32_TOL
+    for t in (0, T - 1):
+        l1, c1 = o.expert_lists(None, chosen[t:t + 1].contiguous().to(dev()), 1, E)
+        alone = o.grouped_linear(x[t:t + 1].contiguous(), w, l1, c1, 1, per_token=True, out_dtype=torch.float32)
+        assert torch.equal(alone, got[t * top:(t + 1) * top])
+
+
+
 @pytest.mark.parametrize("T", [1, 7, 16, 17, 32, 33, 100])
 @pytest.mark.parametrize("n,extra,top,groups,keep,K,scores", [(8, 0, 2, 0, 0, 2048, "softmax"), (32, 1, 4, 4, 2, 1024, "softmax"),
                                                               (16, 0, 3, 0, 0, 200, "sigmoid"), (48, 0, 5, 0, 0, 520, "sigmoid"),

@@ -3,7 +3,9 @@
 // computed in 32-bit (/root/reference/src/transformer/ffn.zig:24-30,
 // /root/reference/src/cuda/layer_kernels.cu:62-70).
 // Also the element-wise cast between storage types.
+// (gate_unit.h: for bfloat16 the unit in the hardware's exponential, as the products that apply it themselves)
 #include "common.h"
+#include "gate_unit.h"
 
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -14,8 +16,7 @@ swiglu_kernel(const T* __restrict__ gu, T* __restrict__ out, int n_tokens, int i
   const size_t t = idx / inter, i = idx % inter;
   const float g = to_f32<T>(gu[t * 2 * inter + i]);
   const float u = to_f32<T>(gu[t * 2 * inter + inter + i]);
-  const float sig = 1.0f / (1.0f + expf(-g));
-  out[idx] = from_f32<T>(g * sig * u);
+  out[idx] = from_f32<T>(gated_value<1, sizeof(T) == 4>(g, u, 0.f, 1.f, 0.f));
 }
 
 template <typename T>
@@ -29,7 +30,7 @@ swiglu_vec8_kernel(const T* __restrict__ gu, T* __restrict__ out, int n_tokens, 
   load8<T>(gu + t * 2 * inter + i, g);
   load8<T>(gu + t * 2 * inter + inter + i, u);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) o[k] = g[k] * (1.0f / (1.0f + expf(-g[k]))) * u[k];
+  for (int k = 0; k < 8; ++k) o[k] = gated_value<1, sizeof(T) == 4>(g[k], u[k], 0.f, 1.f, 0.f);
   store8<T>(out + idx, o);
 }
 
@@ -141,11 +142,7 @@ clamped_glu_kernel(const T* __restrict__ gu, T* __restrict__ out,
     g *= row_scale[t];
     u *= row_scale[t];
   }
-  if (limit > 0.f) {
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-  }
-  out[idx] = from_f32<T>(g * (1.0f / (1.0f + expf(-alpha * g))) * (u + up_offset));
+  out[idx] = from_f32<T>(gated_value<3, sizeof(T) == 4>(g, u, limit, alpha, up_offset));
 }
 
 template <typename T>
@@ -162,14 +159,8 @@ clamped_glu_vec8_kernel(const T* __restrict__ gu, T* __restrict__ out,
   load8<T>(gu + t * 2 * inter + inter + i, u);
   const float rs = row_scale ? row_scale[t] : 1.f;
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    float gk = g[k] * rs, uk = u[k] * rs;
-    if (limit > 0.f) {
-      gk = fminf(gk, limit);
-      uk = fminf(fmaxf(uk, -limit), limit);
-    }
-    o[k] = gk * (1.0f / (1.0f + expf(-alpha * gk))) * (uk + up_offset);
-  }
+  for (int k = 0; k < 8; ++k)
+    o[k] = gated_value<3, sizeof(T) == 4>(g[k] * rs, u[k] * rs, limit, alpha, up_offset);
   store8<T>(out + idx, o);
 }
 
@@ -201,12 +192,9 @@ extern "C" int za_clamped_glu(const void* gu, void* out, int dtype, const float*
 //   act 0: silu(g) = g / (1 + exp(-g))
 //   act 1: gelu in its tanh form, 0.5 g (1 + tanh(sqrt(2/pi) (g + 0.044715 g^3)))
 // in 32-bit.
-__device__ __forceinline__ float gate_act(float g, int act) {
-  if (act == 1) {
-    const float z = 0.7978845608028654f * (g + 0.044715f * g * g * g);
-    return 0.5f * g * (1.0f + tanhf(z));
-  }
-  return g * (1.0f / (1.0f + expf(-g)));
+template <typename T>
+__device__ __forceinline__ float gate_act(float g, float u, int act) {
+  return act == 1 ? gated_value<2, sizeof(T) == 4>(g, u, 0.f, 1.f, 0.f) : gated_value<1, sizeof(T) == 4>(g, u, 0.f, 1.f, 0.f);
 }
 
 template <typename T, int VEC>
@@ -221,12 +209,12 @@ gated_unit_kernel(const T* __restrict__ gu, T* __restrict__ out, int n_tokens, i
     load8<T>(gu + t * 2 * inter + i, g);
     load8<T>(gu + t * 2 * inter + inter + i, u);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) o[k] = gate_act(g[k], act) * u[k];
+    for (int k = 0; k < 8; ++k) o[k] = gate_act<T>(g[k], u[k], act);
     store8<T>(out + idx, o);
   } else {
     const float g = to_f32<T>(gu[t * 2 * inter + i]);
     const float u = to_f32<T>(gu[t * 2 * inter + inter + i]);
-    out[idx] = from_f32<T>(gate_act(g, act) * u);
+    out[idx] = from_f32<T>(gate_act<T>(g, u, act));
   }
 }
 
@@ -395,7 +383,7 @@ table_gate_kernel(const T* __restrict__ g, const int* __restrict__ ids,
   const size_t t = idx / dim;
   const int j = (int)(idx % dim), id = ids[t];
   const float e = (id >= 0 && id < rows) ? to_f32<TT>(table[(size_t)id * ld + col0 + j]) : 0.f;
-  out[idx] = from_f32<T>(gate_act(to_f32<T>(g[idx]), act) * e);
+  out[idx] = from_f32<T>(gate_act<T>(to_f32<T>(g[idx]), e, act));
 }
 
 // dtype codes: 0 = float32, 1 = bfloat16 (of g and out; the table has its own)

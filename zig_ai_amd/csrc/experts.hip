@@ -33,6 +33,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gate_unit.h"
 #include "gemm_f32.h"
 #include "tiles_bf16.h"
 #include "tiles_wide.h"
@@ -115,7 +116,15 @@ struct GroupedArgs {
   int gate;                  // 0: none, 1: silu, 2: the tanh form of gelu, 3: bounded
   float bound, slope, offset;
   int rounded;               // with a gate: the sums are rounded to the result's type ahead of it
+  unsigned per_magic;        // a / top, a < 2^31, as the upper half of a * per_magic, shifted (top > 1)
+  int per_shift;
 };
+
+// The division of an assignment by `top`: a 32-bit division takes some 30 instructions, and a wide tile's rows
+// have sixteen of them ahead of its first request.
+__device__ __forceinline__ int token_of(const GroupedArgs& g, int a) {
+  return g.top == 1 ? a : (int)(__umulhi((unsigned)a, g.per_magic) >> g.per_shift);
+}
 
 // The expert and the tile within it that workgroup `b` serves; false when there is none.  A wave
 // looks at 64 experts at a time (every wave of the workgroup for itself; the answer is the same
@@ -166,29 +175,29 @@ __device__ __forceinline__ float expert_act(float v, int act) {
 }
 
 // The gated unit (gate > 0) of one assignment's sums `v` (gate) and `u` (up).
-template <typename TO>
+template <typename TO, int KIND>
 __device__ __forceinline__ float expert_unit(const GroupedArgs& g, float v, float u, float w) {
-  if (g.rounded) {
-    v = to_f32<TO>(from_f32<TO>(v));
-    u = to_f32<TO>(from_f32<TO>(u));
+  constexpr bool EXACT = sizeof(TO) == 4;
+  if constexpr (!EXACT) {
+    const float rv = to_f32<TO>(from_f32<TO>(v)), ru = to_f32<TO>(from_f32<TO>(u));
+    v = g.rounded ? rv : v;
+    u = g.rounded ? ru : u;
   }
-  v *= w;
-  u *= w;
-  if (g.gate == 3) {
-    if (g.bound > 0.f) {
-      v = fminf(v, g.bound);
-      u = fminf(fmaxf(u, -g.bound), g.bound);
-    }
-    return v * (1.0f / (1.0f + expf(-g.slope * v))) * (u + g.offset);
-  }
-  const float a = g.gate == 2
-                      ? 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)))
-                      : v * (1.0f / (1.0f + expf(-v)));
-  return a * u;
+  return gated_value<KIND, EXACT>(v * w, u * w, g.bound, g.slope, g.offset);
+}
+
+// `what(kind)` with the unit's kind as a constant.
+template <typename What>
+__device__ __forceinline__ void with_unit(const GroupedArgs& g, What what) {
+  if (g.gate == 1) what(std::integral_constant<int, 1>{});
+  else if (g.gate == 2) what(std::integral_constant<int, 2>{});
+  else what(std::integral_constant<int, 3>{});
 }
 
 __device__ __forceinline__ size_t dst_row(const GroupedArgs& g, int a) {
-  return g.stacked ? (size_t)(a % g.top) * g.T + a / g.top : (size_t)a;
+  if (!g.stacked) return (size_t)a;
+  const int t = token_of(g, a);
+  return (size_t)(a - t * g.top) * g.T + t;
 }
 
 // A wave's sums, acc[i][j][r] of assignment m + 16 i + lane % 16 of the expert's list and weight row
@@ -222,13 +231,16 @@ __device__ __forceinline__ void grouped_store(const GroupedArgs& g, const int* _
     TO* to = out + dst_row(g, mine[row]) * N;
     const float w = g.row_weight ? g.row_weight[mine[row]] : 1.0f;
     if constexpr (GATED) {
+      with_unit(g, [&](auto kind) {
 #pragma unroll
-      for (int j = 0; j < TN; j += 2) {
-        f32x4_t v;
+        for (int j = 0; j < TN; j += 2) {
+          f32x4_t v;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = expert_unit<TO>(g, acc[i][j][r], acc[i][j + 1][r], w);
-        put(to, n0 + (wn >> 1) + (j / 2) * 16 + kq * 4, v);
-      }
+          for (int r = 0; r < 4; ++r)
+            v[r] = expert_unit<TO, decltype(kind)::value>(g, acc[i][j][r], acc[i][j + 1][r], w);
+          put(to, n0 + (wn >> 1) + (j / 2) * 16 + kq * 4, v);
+        }
+      });
     } else {
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
@@ -301,108 +313,159 @@ grouped_gemm_bf16_tiled_kernel(GroupedArgs g) {
   grouped_store<TO, GATED>(g, mine, count, tile * BM + wm, n0, wn, lane, acc);
 }
 
-// The tile that workgroup `b` of a list of tiles serves, which holds an expert's full tiles (of more than
-// 128 assignments) or, LAST, the one of what is left of at most 128; HIGH 128: all tiles are such.
-// Returns the number of tiles.
-template <int HIGH, bool LAST>
+// How many tiles of class CLASS (their rows) an expert of `c` assignments makes.  HIGH 256: full tiles of 256,
+// and what is left at its end in one as low as holds it, 128, 192 or 256; HIGH 128: tiles of 128 only.
+template <int HIGH, int CLASS>
 __device__ __forceinline__ int wide_tiles(int c) {
-  if (HIGH == 128) return LAST ? (c + 127) / 128 : 0;
-  const int full = (c + 127) / 256;
-  return LAST ? (c > full * 256 ? 1 : 0) : full;
+  if (HIGH == 128) return CLASS == 128 ? (c + 127) / 128 : 0;
+  const int rest = c & 255;
+  return CLASS == 256 ? (c >> 8) + (rest > 192) : CLASS == 192 ? rest > 128 && rest <= 192 : rest > 0 && rest <= 128;
 }
 
-template <int HIGH, bool LAST>
-__device__ __forceinline__ int wide_count(const int* __restrict__ counts, int E) {
-  int tiles = 0;
-  for (int e = threadIdx.x & 63; e < E; e += 64) tiles += wide_tiles<HIGH, LAST>(counts[e]);
-#pragma unroll
-  for (int o = ZA_WAVE / 2; o > 0; o >>= 1) tiles += __shfl_xor(tiles, o, ZA_WAVE);
-  return __builtin_amdgcn_readfirstlane(tiles);
+// Sums over a wave's lanes up to and including each, without LDS (six shuffles take some 600 clocks of waiting).
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);      // from 1, 2, 4, 8 lanes below in sixteen
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);      // the second and fourth sixteen: the one before
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);      // the upper half: the lower
+  return v;
 }
 
-// Tile `b` of those: its expert, the first of its assignments and the expert's count.
-template <int HIGH, bool LAST>
-__device__ __forceinline__ void wide_find(const int* __restrict__ counts, int E, int b, int* e_out, int* m0_out,
-                                          int* count_out) {
+// Tile `b` of a class: its expert, the first of its assignments and the expert's count.  `own` is the count
+// of the lane's expert among the first 64.
+template <int HIGH, int CLASS>
+__device__ __forceinline__ void wide_find(const int* __restrict__ counts, int E, int own, int b, int* e_out,
+                                          int* m0_out, int* count_out) {
   const int lane = threadIdx.x & 63;
   int first = 0;
   for (int e0 = 0; e0 < E; e0 += 64) {
-    const int c = e0 + lane < E ? counts[e0 + lane] : 0;
-    const int tiles = wide_tiles<HIGH, LAST>(c);
-    int end = tiles;
-#pragma unroll
-    for (int o = 1; o < ZA_WAVE; o <<= 1) {
-      const int v = __shfl_up(end, o, ZA_WAVE);
-      if (lane >= o) end += v;
-    }
+    const int c = e0 == 0 ? own : e0 + lane < E ? counts[e0 + lane] : 0;
+    const int tiles = wide_tiles<HIGH, CLASS>(c), end = wave_scan(tiles);
     const unsigned long long past = __ballot(b < first + end);
     if (past) {
       const int at = __ffsll(past) - 1, n = __builtin_amdgcn_readlane(c, at);
       const int tile = b - first - (__builtin_amdgcn_readlane(end, at) - __builtin_amdgcn_readlane(tiles, at));
       *e_out = __builtin_amdgcn_readfirstlane(e0 + at);
       *count_out = n;
-      *m0_out = HIGH == 256 && LAST ? (n + 127) / 256 * 256 : tile * HIGH;
+      *m0_out = HIGH == 256 && CLASS != 256 ? n & ~255 : tile * HIGH;
       return;
     }
     first += __builtin_amdgcn_readlane(end, 63);
   }
 }
 
-// Tiles of 256 x 256 or, for what is left of an expert's rows at its end, 128 x 256 (tiles_wide.h);
-// HIGH 128: of 128 x 256 only.  GATED as above.
-template <typename TO, bool GATED, int HIGH>
-__global__ void __launch_bounds__(512, 2)
+// Tiles of 256, 192 or 128 x 256 (tiles_wide.h); HIGH as above.  UNIT: 0 without, else GATED as above with the
+// unit's kind as a constant, 4: any (for 32-bit results; the three kinds' stores side by side cost registers).
+template <typename TO, int UNIT, int HIGH>
+__global__ void __launch_bounds__(256, 1)
 grouped_gemm_bf16_wide_kernel(GroupedArgs g) {
-  __shared__ __attribute__((aligned(16))) bf16_t lds[GW_LDS];
-  // Workgroups are dealt to the eight dies in turn: a die takes an eighth of the full tiles, an expert's
-  // stretches of outputs side by side, and then an eighth of the others, which take half as long and
+  constexpr bool GATED = UNIT > 0;
+  __shared__ __attribute__((aligned(16))) char lds[GW_LDS];
+  // Workgroups are dealt to the eight dies in turn: a die takes an eighth of the highest tiles, an expert's
+  // stretches of outputs side by side, and then an eighth of each lower kind, which take less long and
   // fill the ends.
   const int columns = (g.N + (GATED ? 127 : 255)) / (GATED ? 128 : 256), die = blockIdx.x & 7;
-  const int full = HIGH == 256 ? wide_count<HIGH, false>(g.counts, g.E) * columns : 0;
-  const int rest = wide_count<HIGH, true>(g.counts, g.E) * columns;
-  const int full_each = (full + 7) >> 3, rest_each = (rest + 7) >> 3;
-  int at = blockIdx.x >> 3, index;
-  const bool last = at >= full_each;
-  if (last) {
-    at -= full_each;
-    index = die * rest_each + at;
-    if (at >= rest_each || index >= rest) return;
-  } else {
-    index = die * full_each + at;
-    if (index >= full) return;
+  int n256 = 0, n192 = 0, n128 = 0;
+  const int lane64 = threadIdx.x & 63, first64 = lane64 < g.E ? g.counts[lane64] : 0;
+  for (int e0 = 0; e0 < g.E; e0 += 64) {
+    const int c = e0 == 0 ? first64 : e0 + lane64 < g.E ? g.counts[e0 + lane64] : 0;
+    n256 += wide_tiles<HIGH, 256>(c);
+    n192 += wide_tiles<HIGH, 192>(c);
+    n128 += wide_tiles<HIGH, 128>(c);
   }
+  int at = blockIdx.x >> 3, index = -1;
+  auto mine_of = [&](int tiles) {      // whether this workgroup's tile is one of a kind
+    const int total = __builtin_amdgcn_readlane(wave_scan(tiles), 63) * columns, each = (total + 7) >> 3;
+    if (at >= each) {
+      at -= each;
+      return false;
+    }
+    index = die * each + at < total ? die * each + at : -1;
+    return true;
+  };
   int e, m0, count;
-  if (last) wide_find<HIGH, true>(g.counts, g.E, index / columns, &e, &m0, &count);
-  else wide_find<HIGH, false>(g.counts, g.E, index / columns, &e, &m0, &count);
-  const int n0 = (index % columns) * (GATED ? 128 : 256);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int* mine = g.lists + (size_t)e * g.A;
-  const int K = g.K, N = g.N;
-  const bf16_t* wbase = (const bf16_t*)g.W + (size_t)e * (GATED ? 2 * N : N) * K;
   auto serve = [&](auto tm) {
     constexpr int TM = decltype(tm)::value;
     using Tiles = TilesWide<TM>;
-    const int lrow = wave * 8 + (lane >> 3), piece = ((lane & 7) ^ (lane >> 3)) * 8;
-    const bf16_t* arow[Tiles::LA];
-    const bf16_t* wrow[Tiles::LW];
+    const int n0 = (index % columns) * (GATED ? 128 : 256);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int* mine = g.lists + (size_t)e * g.A;
+    const int K = g.K, N = g.N;
+    const int lrow = wave * 8 + (lane >> 3), piece = ((lane & 7) ^ (lane >> 3)) * 16;
+    unsigned offa[Tiles::LA], offw[Tiles::LW];
 #pragma unroll
     for (int i = 0; i < Tiles::LA; ++i) {
-      const int r = min(m0 + lrow + 64 * i, count - 1);      // (rows beyond are not stored)
-      arow[i] = (const bf16_t*)g.src + (size_t)(mine[r] / g.src_div) * K + piece;
+      const int r = min(m0 + lrow + 32 * i, count - 1);      // (rows beyond are not stored)
+      const int a = mine[r];
+      offa[i] = (unsigned)(g.src_div == 1 ? a : token_of(g, a)) * (unsigned)(K * 2) + piece;
     }
 #pragma unroll
     for (int i = 0; i < Tiles::LW; ++i) {
-      const int tr = lrow + 64 * i;
+      const int tr = lrow + 32 * i;
       const int n = min(n0 + (GATED ? (tr >> 5) * 16 + (tr & 15) : tr), N - 1);
-      wrow[i] = wbase + (size_t)(n + (GATED && (tr & 16) ? N : 0)) * K + piece;
+      offw[i] = (unsigned)(n + (GATED && (tr & 16) ? N : 0)) * (unsigned)(K * 2) + piece;
     }
+    // this lane's rows of the sums: where they go, and their weights
+    const int wm = m0 + (wave >> 1) * 16 * TM, r16 = lane & 15;
+    int to[TM];
+    float weight[TM];
     f32x4_t acc[TM][Tiles::TN];
-    Tiles::run(lds, wave, lane, K, arow, wrow, acc);
-    grouped_store<TO, GATED>(g, mine, count, m0 + (wave >> 2) * 16 * TM, n0, (wave & 3) * 64, lane, acc);
+    Tiles::run(lds, wave, lane, K, (const char*)g.src, (const char*)g.W + (size_t)e * (GATED ? 2 * N : N) * K * 2, offa,
+               offw, acc, [&]() {
+#pragma unroll
+                 for (int i = 0; i < TM; ++i) {
+                   const int row = wm + 16 * i + r16, a = row < count ? mine[row] : -1;
+                   to[i] = a < 0 ? -1 : (int)dst_row(g, a);
+                   weight[i] = g.row_weight && a >= 0 ? g.row_weight[a] : 1.0f;
+                 }
+               });
+    if (sizeof(TO) == 2) __syncthreads();
+    auto put = [&](auto value) {
+      wide_store<TO, GATED ? 64 : 128, TM>(
+          lds, wave, lane, (TO*)g.out, n0 + (wave & 1) * (GATED ? 64 : 128), N,
+          [&](int i, int j) {
+            f32x4_t v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = value(i, j, r);
+            return v;
+          },
+          [&](int i, int r) { return sizeof(TO) == 4 ? to[i] : __shfl(to[i], r, ZA_WAVE); });
+    };
+    if constexpr (UNIT == 4)
+      with_unit(g, [&](auto kind) {
+        put([&](int i, int j, int r) {
+          return expert_unit<TO, decltype(kind)::value>(g, acc[i][2 * j][r], acc[i][2 * j + 1][r], weight[i]);
+        });
+      });
+    else if constexpr (GATED)
+      put([&](int i, int j, int r) {
+        return expert_unit<TO, UNIT>(g, acc[i][2 * j][r], acc[i][2 * j + 1][r], weight[i]);
+      });
+    else
+      put([&](int i, int j, int r) { return expert_act(acc[i][j][r], g.act) * g.out_scale * weight[i]; });
   };
-  if (last) serve(std::integral_constant<int, 4>{});
-  else if constexpr (HIGH == 256) serve(std::integral_constant<int, 8>{});
+  if constexpr (HIGH == 256) {
+    if (mine_of(n256)) {
+      if (index < 0) return;
+      wide_find<HIGH, 256>(g.counts, g.E, first64, index / columns, &e, &m0, &count);
+      serve(std::integral_constant<int, 8>{});
+      return;
+    }
+    if (mine_of(n192)) {
+      if (index < 0) return;
+      wide_find<HIGH, 192>(g.counts, g.E, first64, index / columns, &e, &m0, &count);
+      serve(std::integral_constant<int, 6>{});
+      return;
+    }
+  }
+  if (mine_of(n128)) {
+    if (index < 0) return;
+    wide_find<HIGH, 128>(g.counts, g.E, first64, index / columns, &e, &m0, &count);
+    serve(std::integral_constant<int, 4>{});
+  }
 }
 
 // 32-bit weights (src of either type): tiles of 32 assignments x 64 weight rows, the sums in the
@@ -436,7 +499,9 @@ grouped_gemm_f32_kernel(GroupedArgs g) {
       const int first = n0 + (n >> 5) * 16 + (n & 15);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (first + i < N) at[first + i] = from_f32<TO>(expert_unit<TO>(g, v[0][i], v[1][i], w));
+        if (first + i < N) with_unit(g, [&](auto kind) {
+          at[first + i] = from_f32<TO>(expert_unit<TO, decltype(kind)::value>(g, v[0][i], v[1][i], w));
+        });
     } else {
 #pragma unroll
       for (int j = 0; j < GF_BN / 32; ++j)
@@ -469,7 +534,13 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
   if (experts > EX_MAX_EXPERTS) return ZA_ERR_UNSUPPORTED;
   if (stacked && out_dtype != 0) return ZA_ERR_UNSUPPORTED;
   GroupedArgs g{src, W, lists, counts, out, (int)A, n_tokens, top, experts, N, K,
-                src_div, stacked, act, out_scale, row_weight, gate, bound, slope, offset, rounded};
+                src_div, stacked, act, out_scale, row_weight, gate, bound, slope, offset, rounded, 0, 0};
+  if (top > 1) {      // 2^(31 + bits) / top, rounded up, fits 32 bits and is exact for a below 2^31
+    int bits = 1;
+    while ((1LL << bits) < top) ++bits;
+    g.per_magic = (unsigned)(((1ULL << (31 + bits)) + top - 1) / top);
+    g.per_shift = bits - 1;
+  }
   if (w_dtype == 1) {
     if (src_dtype != 1 || K % 8 != 0 || ((uintptr_t)src | (uintptr_t)W) % 16 != 0) return ZA_ERR_UNSUPPORTED;
     if (out_dtype != 0 && out_dtype != 1) return ZA_ERR_UNSUPPORTED;
@@ -496,16 +567,22 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     // -> 182 | 107; at 517 tokens (65 rows an expert) 73 | 36 against 84 | 38.  8 experts of 4,096, 2 a
     // token, 1,900 tokens: up 99 -> 64 (128 high 85), down, 128 high for want of tiles, 92 -> 75 (256
     // high 95); 500 tokens: up, 128 high, 56 -> 43, down stays (54 against 66).  The sums are the same
-    // to the last bit.
+    // to the last bit.  With four waves of 128 x 128 in place of eight of 128 x 64, ends of 192, the unit in
+    // the hardware's exponential and bfloat16 stored in whole lines, before and after (us): 32 experts, gated,
+    // 1,777 tokens 90 and 79, unevenly taken 105 and 92, 4,096 tokens unevenly 186 and 154; 8 experts of 4,096,
+    // gated, 1,777 tokens 168 and 123; their down product at 4,096 tokens 153 and 145.  32-bit results of few
+    // steps of K are bound by the 58 MB and more that they write: 2,048 x 1,024, 1,777 tokens unevenly 58 to 64
+    // and 58 to 62, 4,096 tokens 103 and 106.
     // And only where the rounds that the tiles make, 256 of them at a time or 512 of the low ones, take no
     // longer (few steps of K, outputs that fill little of a wide tile, a wide round that is nearly empty
     // where the low tiles make whole ones): a round of 128 x 128, two to a compute unit, as K, of 128 x 256 as
     // 0.9 K + 400, of 256 x 256 as 1.2 K + 400, an expert's last tile of those half as long; fitted to 420
-    // products of 300 to 64,000 rows, 64 to 8,192 outputs and 128 to 4,096 elements of K (us, low and wide):
+    // products of 300 to 64,000 rows, 64 to 8,192 outputs and 128 to 4,096 elements of K with eight waves (us, low
+    // and wide; with four, over 450 products, the choice is 1.5 percent from the best of the three on average):
     // 32 experts, 4 a token, gated, 8,000 tokens, 64 x 2,048 38 and 67; 4,000 tokens, 192 x 2,048 41 and 70;
     // 8 experts, 2 a token, gated, 12,000 tokens, 320 x 2,048 79 and 112, 448 x 2,048 115 and 117, 640 x
     // 2,048 157 and 131; not gated, 640 x 2,048 76 and 96, 512 x 2,048 72 and 56.
-    if (K % GG_BK == 0 && A >= 80LL * experts) {
+    if (K % GG_BK == 0 && A >= 80LL * experts && src_rows * K <= 0x7fffffffLL && (gate ? 2LL : 1LL) * N * K <= 0x7fffffffLL) {
       const long long columns = (N + (gate ? 127 : 255)) / (gate ? 128 : 256);
       int high = (A / 256 + experts / 2) * columns >= 176 ? 256
                  : (A / 128 + experts / 2) * columns >= 150 ? 128 : 0;
@@ -516,19 +593,22 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
       if (wide > low) high = 0;
       // (an expert's full tiles and its last one, each kind an eighth a die)
       const long long tiles = (A + high - 1) / max(high, 1) + experts;
-      const long long blocks = (tiles * columns + 7) / 8 * 8 + 8;
+      const long long blocks = (tiles * columns + 7) / 8 * 8 + 16;
       if (high && blocks > 0x7fffffffLL) return ZA_ERR_ARG;
-#define ZA_GW(TO, GATED)                                                                                   \
+#define ZA_GW(TO, UNIT)                                                                                    \
   {                                                                                                        \
     if (high == 256)                                                                                       \
-      hipLaunchKernelGGL((grouped_gemm_bf16_wide_kernel<TO, GATED, 256>), dim3((unsigned)blocks), dim3(512), 0, stream, g); \
+      hipLaunchKernelGGL((grouped_gemm_bf16_wide_kernel<TO, UNIT, 256>), dim3((unsigned)blocks), dim3(256), 0, stream, g); \
     else                                                                                                   \
-      hipLaunchKernelGGL((grouped_gemm_bf16_wide_kernel<TO, GATED, 128>), dim3((unsigned)blocks), dim3(512), 0, stream, g); \
+      hipLaunchKernelGGL((grouped_gemm_bf16_wide_kernel<TO, UNIT, 128>), dim3((unsigned)blocks), dim3(256), 0, stream, g); \
     return za_launch_status();                                                                             \
   }
       if (high) {
-        if (out_dtype == 0) { if (gate) ZA_GW(float, true) else ZA_GW(float, false) }
-        else { if (gate) ZA_GW(bf16_t, true) else ZA_GW(bf16_t, false) }
+        if (out_dtype == 0) { if (gate) ZA_GW(float, 4) else ZA_GW(float, 0) }
+        else if (gate == 0) ZA_GW(bf16_t, 0)
+        else if (gate == 1) ZA_GW(bf16_t, 1)
+        else if (gate == 2) ZA_GW(bf16_t, 2)
+        else ZA_GW(bf16_t, 3)
       }
 #undef ZA_GW
     }

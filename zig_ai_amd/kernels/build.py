@@ -42,8 +42,8 @@ EXTRA_FLAGS = {"blaslt": ["-lhipblaslt"]}   # host code around the GEMM library,
 # headers a source includes beside common.h
 EXTRA_HEADERS = {"sampling": ["no_alloc.h"], "rope_kv": ["rope_math.h"], "attention": ["attention_common.h", "rope_math.h"],
                  "attention_planes": ["attention_common.h"], "recurrent": ["rope_math.h"], "gemm_f32": ["gemm_f32.h"],
-                 "experts": ["gemm_f32.h", "tiles_bf16.h", "tiles_wide.h"], "latent": ["tiles_bf16.h"],
-                 "gemm_tiles": ["tiles_bf16.h"]}
+                 "experts": ["gate_unit.h", "gemm_f32.h", "tiles_bf16.h", "tiles_wide.h"], "latent": ["tiles_bf16.h"],
+                 "gemm_tiles": ["tiles_bf16.h"], "activation": ["gate_unit.h"]}
 
 _loaded: Dict[str, ctypes.CDLL] = {}
 _lock = threading.Lock()

@@ -1945,6 +1945,47 @@ def test_grouped_products_in_wide_tiles(K, columns, top):
                                             **one), gated[mine])
 
 
+@pytest.mark.parametrize("M", [65, 128, 129, 192, 193, 256, 257, 450, 520])
+@pytest.mark.parametrize("I,K", [(8, 64), (72, 128), (130, 192), (301, 256), (1100, 448)])
+def test_gated_products_of_many_rows(M, I, K):
+    """The wide tiles with the unit applied: every height of the last tile, one to seven steps of K, outputs off
+    multiples of a tile, of 16 and of 8; each unit, bounded and not, against 64-bit arithmetic."""
+    o = ops()
+    assert o.wide_takes_gated(M, I, K)
+    x, w = rand((M, K), torch.bfloat16, M), rand((2 * I, K), torch.bfloat16, I, K ** -0.5)
+    both = x.double() @ w.double().T
+    g, u = both[:, :I], both[:, I:]
+    act = torch.nn.functional
+    for activation, want in (("silu", act.silu(g) * u), ("gelu_tanh", act.gelu(g, approximate="tanh") * u)):
+        assert rel_err(o.linear_gated_wide(x.to(dev()), w.to(dev()), activation), want) < tol_of(torch.bfloat16)
+    for limit in (0.0, 0.7):
+        gl, ul = (g.clamp(max=limit), u.clamp(-limit, limit)) if limit else (g, u)
+        got = o.linear_gated_wide(x.to(dev()), w.to(dev()), bounded=(limit, 1.702, 1.0))
+        assert rel_err(got, gl * torch.sigmoid(1.702 * gl) * (ul + 1.0)) < tol_of(torch.bfloat16)
+        got = o.linear_gated_wide(x.to(dev()), w.to(dev()), bounded=(limit, 1.702, 1.0), rounded=True)
+        gl, ul = both[:, :I].bfloat16().double(), both[:, I:].bfloat16().double()
+        gl, ul = (gl.clamp(max=limit), ul.clamp(-limit, limit)) if limit else (gl, ul)
+        assert rel_err(got, gl * torch.sigmoid(1.702 * gl) * (ul + 1.0)) < tol_of(torch.bfloat16)
+
+
+def test_gated_products_of_many_rows_leave_other_rows_alone():
+    """Infinite and undefined inputs reach their own row's outputs only, and products the rule or the kernel
+    does not take are refused."""
+    o = ops()
+    x, w = rand((300, 128), torch.bfloat16, 1).to(dev()), rand((512, 128), torch.bfloat16, 2, 0.1).to(dev())
+    want = o.linear_gated_wide(x, w)
+    x2 = x.clone()
+    x2[7], x2[140, 3], x2[299] = float("nan"), float("inf"), -float("inf")
+    got = o.linear_gated_wide(x2, w)
+    rows = [r for r in range(300) if r not in (7, 140, 299)]
+    assert torch.equal(got[rows], want[rows]) and bool(got[7].isnan().all())
+    assert o.linear_gated_wide(x[:64], w) is None                      # (few rows have kernels of their own)
+    assert o.linear_gated_wide(x[:, :72].contiguous(), w[:, :72].contiguous()) is None      # K off whole steps
+    assert o.linear_gated_wide(x.float(), w) is None
+    flat = torch.zeros(300 * 128 + 1, dtype=torch.bfloat16, device=dev())
+    assert o.linear_gated_wide(flat[1:].view(300, 128), w) is None     # an operand off 16 bytes
+
+
 @pytest.mark.parametrize("E,top,K,columns", [(12, 3, 1024, 2304), (12, 1, 1088, 2311), (70, 7, 512, 640), (70, 2, 576, 1288)])
 def test_grouped_products_whose_experts_end_in_each_height_of_tile(E, top, K, columns):
     """Wide tiles of 256, 192 and 128: an expert's rest of 0, 1, 128, 129, 192, 193 and 255 assignments behind

@@ -66,6 +66,8 @@ _SIGNATURES = {
                                         c_int, c_int, c_void_p],
     ("sampling", "za_argmax"): [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int,
                                 c_void_p],
+    ("gemm_wide", "za_gemm_bf16_wide_gated"): [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                               c_float, c_float, c_float, c_int, c_void_p],
     ("gemm", "za_gemm_bf16_rows16"): [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                                       c_int, c_int, c_int, c_void_p],
     ("gemm", "za_gemm_bf16_rows16_stream"): [c_void_p, c_void_p, c_void_p, c_void_p, c_float,
@@ -900,6 +902,65 @@ def linear_gated_tiles(x: torch.Tensor, gate_up_weight: torch.Tensor,
     if not _tiles_product(x, gate_up_weight, out, gated=True, activation=GATE_ACTIVATIONS[activation]):
         return None
     _note("linear_swiglu", M=M, N=2 * I, K=K, norm_in_product=False, kernel="tiles")
+    return out
+
+
+# The gated product of a step of many rows on csrc/gemm_wide.hip: where the rounds of its tiles, 256 at a
+# time, a step of 64 elements of K 1.1 us of a round, end before the library's product and the unit's kernel
+# after it would, 1.28 PFLOP/s and 12 us together.  Measured (us; weights from memory, the library's
+# product with the unit's kernel and this one): 2 x 8192 x 2048 at 400, 600, 1,037, 1,300, 2,048 and 4,096
+# rows 37, 46, 79, 91, 119, 226 and 40, 43, 70, 86, 102, 200; 2 x 7168 x 2048 at 600, 1,037, 1,300, 2,048
+# rows 42, 73, 84, 107 and 39, 56, 85, 93; 2 x 4608 x 1024 at 512, 700, 1,037, 1,777, 4,096 rows 22, 24, 30,
+# 41, 95 and 23, 24, 25, 30, 77; 2 x 1024 x 2048 at 2,048 and 4,096 rows 25, 38 and 37, 40.
+WIDE_ROUND_US = 4.0
+WIDE_STEP_US = 1.1
+WIDE_LIBRARY_US = 12.0
+WIDE_LIBRARY_FLOPS = 1.28e9       # a microsecond
+WIDE_MAX_ELEMENTS = 0x7fffffff    # of either operand: offsets of 32 bits in bytes
+
+
+def wide_rounds(M: int, columns: int) -> float:
+    """The rounds that ``columns`` stretches of outputs make of M rows' tiles: the full tiles, and the lower
+    ones at the rows' end, which take some two thirds as long, where the last round has no room."""
+    rest = M % 256
+    full, low = (M // 256 + (rest > 192)) * columns, columns if 0 < rest <= 192 else 0
+    rounds = -(-full // 256)
+    return rounds + (0.0 if low <= (1.0 if rest > 128 else 2.0) * (rounds * 256 - full)
+                     else 0.67 * -(-low // 256))
+
+
+def wide_takes_gated(M: int, I: int, K: int) -> bool:
+    """Whether ``linear_gated_wide`` takes a gated product of ``M`` rows and ``I`` outputs."""
+    if M <= TILES_MAX_ROWS or K % 64 or M * K > WIDE_MAX_ELEMENTS or 2 * I * K > WIDE_MAX_ELEMENTS:
+        return False
+    own = wide_rounds(M, -(-I // 128)) * (WIDE_ROUND_US + K / 64 * WIDE_STEP_US)
+    return own <= WIDE_LIBRARY_US + 4.0 * M * I * K / WIDE_LIBRARY_FLOPS
+
+
+def linear_gated_wide(x, gate_up_weight: torch.Tensor, activation: str = "silu",
+                      bounded: Optional[Tuple[float, float, float]] = None,
+                      rounded: bool = False) -> Optional[torch.Tensor]:
+    """``act(x Wg^T) * (x Wu^T)`` of a step of many rows of bfloat16 ``x`` in one kernel, the unit on the
+    product's 32-bit sums (``rounded``: on them rounded to bfloat16, as the unit's own kernel reads them);
+    ``bounded``: ``(limit, alpha, up_offset)`` of ``clamped_glu`` in place of ``activation``.  ``None``: not a product that ``wide_takes_gated`` names, or operands that the kernel does not
+    take."""
+    if not isinstance(x, torch.Tensor) or x.dtype != torch.bfloat16 or gate_up_weight.dtype != torch.bfloat16 \
+            or x.dim() != 2 or gate_up_weight.dim() != 2 or gate_up_weight.shape[0] % 2:
+        return None
+    M, K = x.shape
+    I = gate_up_weight.shape[0] // 2
+    if not wide_takes_gated(M, I, K) or (x.data_ptr() | gate_up_weight.data_ptr()) % 16:
+        return None
+    _need(x, "x", torch.bfloat16)
+    _need(gate_up_weight, "gate_up_weight", torch.bfloat16, (2 * I, K))
+    limit, alpha, up_offset = bounded if bounded is not None else (0.0, 1.0, 0.0)
+    kind = 3 if bounded is not None else 1 + GATE_ACTIVATIONS[activation]
+    out = torch.empty((M, I), dtype=torch.bfloat16, device=x.device)
+    rc = _fn("gemm_wide", "za_gemm_bf16_wide_gated")(
+        _ptr(x), _ptr(gate_up_weight), _ptr(out), M, I, K, kind, float(limit), float(alpha),
+        float(up_offset), 1 if rounded else 0, _stream())
+    _check(rc, "gemm_bf16_wide_gated", f"M={M} N={I} K={K} kind={kind}")
+    _note("linear_swiglu", M=M, N=2 * I, K=K, norm_in_product=False, kernel="wide")
     return out
 
 

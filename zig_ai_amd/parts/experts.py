@@ -113,7 +113,7 @@ class RoutedExperts(FeedForward):
 
     kind = "routed_experts"
     graph_safe = True
-    kernel_sources = ("experts", "gemm", "gemm_rows64", "activation")
+    kernel_sources = ("experts", "gemm", "gemm_rows64", "gemm_wide", "activation")
 
     @staticmethod
     def _sizes(params):
@@ -253,8 +253,10 @@ class RoutedExperts(FeedForward):
             # a decode batch: the gate is applied to the projection's accumulators
             s = ops.linear_swiglu(x, self.shared_gate_up, self.activation)
         else:
-            s = ops.gated_unit(ops.linear(x, self.shared_gate_up, tune=self.runtime.tune),
-                               self.activation)
+            s = ops.linear_gated_wide(x, self.shared_gate_up, self.activation)
+            if s is None:
+                s = ops.gated_unit(ops.linear(x, self.shared_gate_up, tune=self.runtime.tune),
+                                   self.activation)
         return ops.linear(s, self.shared_down, out_dtype=torch.float32, tune=self.runtime.tune,
                           into=into)
 

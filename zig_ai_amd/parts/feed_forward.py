@@ -44,7 +44,7 @@ class SwiGLU(FeedForward):
     graph_safe = True
     takes_stream = True
     opens_with_swiglu = True
-    kernel_sources = ("gemm", "gemm_rows64", "activation")
+    kernel_sources = ("gemm", "gemm_rows64", "gemm_wide", "activation")
 
     @classmethod
     def tensor_rules(cls, params: Mapping[str, Any]) -> Dict[str, TensorRule]:
@@ -71,8 +71,10 @@ class SwiGLU(FeedForward):
         ops.check_projection_weight(self.down, "feed_forward down")
 
     def gated_by_tiles(self, x: torch.Tensor) -> Optional[torch.Tensor]:
-        """The gated product of a step of 17 to 64 normalised rows in one kernel; ``None``: not
+        """The gated product of a step of more than 16 normalised rows in one kernel; ``None``: not
         taken."""
+        if x.shape[0] > ops.TILES_MAX_ROWS:
+            return ops.linear_gated_wide(x, self.gate_up, self.activation)
         if x.dtype == torch.bfloat16 and self.gate_up.dtype == torch.bfloat16 \
                 and ops.tiles_take_gated(x.shape[0], self.gate_up.shape[0] // 2, x.shape[1]):
             return ops.linear_gated_tiles(x, self.gate_up, self.activation)
@@ -116,13 +118,13 @@ class ClampedGLU(FeedForward):
         y = (g * sigmoid(alpha * g) * (u + up_offset)) Wd^T
 
     ``limit`` (none if 0), ``alpha`` and ``up_offset`` come from ``params``.  Gate and up
-    weights are one matrix, as in ``SwiGLU``; the unit is a kernel of its own, or with
-    ``unit_in_product`` applied by a decode batch's product to its own 32-bit sums (which the
-    kernel of its own reads rounded to the run's type)."""
+    weights are one matrix, as in ``SwiGLU``; the unit is a kernel of its own, which reads them rounded to
+    the run's type, or applied by the product: with many rows by the wide one, and with ``unit_in_product``
+    by a decode batch's, then in 32-bit."""
 
     kind = "clamped_glu"
     graph_safe = True
-    kernel_sources = ("gemm", "activation")
+    kernel_sources = ("gemm", "gemm_wide", "activation")
 
     @classmethod
     def tensor_rules(cls, params: Mapping[str, Any]) -> Dict[str, TensorRule]:
@@ -144,8 +146,11 @@ class ClampedGLU(FeedForward):
                 and self.gate_up.dtype == torch.bfloat16 and x.shape[0] <= 16 and x.shape[1] <= 8192:
             a = ops.linear_swiglu(x, self.gate_up, bounded=(self.limit, self.alpha, self.up_offset))
         else:
-            a = ops.clamped_glu(ops.linear(x, self.gate_up, tune=self.runtime.tune), self.limit,
-                                self.alpha, self.up_offset)
+            a = ops.linear_gated_wide(x, self.gate_up, bounded=(self.limit, self.alpha, self.up_offset),
+                                      rounded=not self.unit_in_product)
+            if a is None:
+                a = ops.clamped_glu(ops.linear(x, self.gate_up, tune=self.runtime.tune), self.limit,
+                                    self.alpha, self.up_offset)
         return ops.linear(a, self.down, partial_ok=self.partial_ok, tune=self.runtime.tune)
 
 

@@ -1986,6 +1986,55 @@ def test_gated_products_of_many_rows_leave_other_rows_alone():
     assert o.linear_gated_wide(flat[1:].view(300, 128), w) is None     # an operand off 16 bytes
 
 
+@pytest.mark.parametrize("height", [128, 192, 256])
+@pytest.mark.parametrize("M,N", [(65, 8), (127, 127), (128, 128), (129, 130), (192, 300), (193, 640), (257, 68), (520, 1032)])
+def test_products_of_one_round_of_tiles(height, M, N):
+    """Every height of tile, rows and outputs below, at and off multiples of a tile, of eight and of four, K of as
+    few steps as a place in LDS each and of more, whole and in equal and unequal ranges; against 64-bit sums, and
+    the ranges' sum to 32-bit rounding."""
+    o = ops()
+    for K, ranges in ((320, 1), (384, 1), (448, 1), (1088, 1), (640, 2), (1088, 3), (1536, 4)):
+        x, w = rand((M, K), torch.bfloat16, M + K), rand((N, K), torch.bfloat16, N, K ** -0.5)
+        want = x.double() @ w.double().T
+        got = o._half_product(x.to(dev()), w.to(dev()), height, ranges)
+        if ranges == 1:
+            assert got.dtype == torch.bfloat16 and rel_err(got, want) < BF16_TOL, K
+        else:
+            assert got.shape == (ranges, M, N) and rel_err(got.double().sum(0), want) < F32_TOL, (K, ranges)
+            step = -(-(K // 64) // ranges) * 64
+            for r in range(ranges):
+                k = slice(r * step, min(K, (r + 1) * step))
+                assert rel_err(got[r], x[:, k].double() @ w[:, k].double().T) < F32_TOL, (K, r)
+
+
+@pytest.mark.parametrize("M,N,K", [(1037, 2048, 7168), (1100, 256, 4096), (2048, 384, 8192), (987, 3070, 1024), (1037, 2050, 2048)])
+def test_products_that_the_estimates_give_to_one_round(M, N, K):
+    """Where ``half_plan`` names a plan: ``linear_closing``'s product comes back in ranges and leaves the stream
+    alone, ``linear``'s plain one in the type asked for or into a given tensor; an operand off 16 bytes takes the other
+    way."""
+    o = ops()
+    x, w = rand((M, K), torch.bfloat16, 5).to(dev()), rand((N, K), torch.bfloat16, 6, K ** -0.5).to(dev())
+    want = (x.double() @ w.double().T).cpu()
+    if K >= 4096:
+        assert o.half_plan(M, N, K, True)[1] > 1
+        stream = rand((M, N), torch.float32, 7).to(dev())
+        kept = stream.clone()
+        stack = o.linear_closing(x, w, stream)
+        assert stack.dim() == 3 and torch.equal(stream, kept)
+        assert rel_err(stack.sum(0), want) < F32_TOL
+        assert o.linear(x, w, partial_ok=True, accumulate=stream) is None      # (``linear`` adds as before)
+        assert rel_err(stream - kept, want) < 4 * F32_TOL
+        return
+    assert o.half_plan(M, N, K, False)[0] > 0
+    got = o.linear(x, w)
+    assert got.dtype == torch.bfloat16 and rel_err(got, want) < BF16_TOL
+    into = torch.zeros((M, N), dtype=torch.bfloat16, device=dev())
+    assert torch.equal(o.linear(x, w, into=into), got) and torch.equal(into, got)
+    assert rel_err(o.linear(x, w, out_dtype=torch.float32), want) < F32_TOL
+    off = torch.empty(M * K + 1, dtype=torch.bfloat16, device=dev())[1:].view(M, K).copy_(x)
+    assert rel_err(o.linear(off, w), want) < BF16_TOL
+
+
 @pytest.mark.parametrize("E,top,K,columns", [(12, 3, 1024, 2304), (12, 1, 1088, 2311), (70, 7, 512, 640), (70, 2, 576, 1288)])
 def test_grouped_products_whose_experts_end_in_each_height_of_tile(E, top, K, columns):
     """Wide tiles of 256, 192 and 128: an expert's rest of 0, 1, 128, 129, 192, 193 and 255 assignments behind

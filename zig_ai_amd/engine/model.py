@@ -168,7 +168,7 @@ class DecoderModel:
             if "gemm" in self.kernel_sources:
                 wanted.append("gemm_f32")                    # matrices kept in 32-bit, also in a bfloat16 run
                 if runtime.dtype == torch.bfloat16:
-                    wanted += ["blaslt", "gemm_tiles"]       # the products of more than 16 rows
+                    wanted += ["blaslt", "gemm_half", "gemm_tiles"]       # the products of more than 16 rows
             kernel_build.build_all(wanted, jobs=len(wanted))
 
     # ------------------------------------------------------------- construction

@@ -10,6 +10,7 @@ operands other than the ones its indexing assumes.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional, Tuple
 
@@ -66,6 +67,8 @@ _SIGNATURES = {
                                         c_int, c_int, c_void_p],
     ("sampling", "za_argmax"): [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int,
                                 c_void_p],
+    ("gemm_half", "za_gemm_bf16_half"): [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
+                                         c_void_p],
     ("gemm_wide", "za_gemm_bf16_wide_gated"): [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                                c_float, c_float, c_float, c_int, c_void_p],
     ("gemm", "za_gemm_bf16_rows16"): [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
@@ -964,6 +967,97 @@ def linear_gated_wide(x, gate_up_weight: torch.Tensor, activation: str = "silu",
     return out
 
 
+# Products of many rows on csrc/gemm_half.hip: where its tiles, of a height and over ranges of K to choose, make one
+# round (256 at most) that ends before the library's product would.  Both times are estimated (us), by fits to 292
+# products of 120 to 4,500 rows, 1,024 to 8,192 outputs and elements of K, weights from memory: a tile's step of 64
+# elements of K by its height, slower the fuller the round is (the card's power), and what is written and, of
+# ranges, read again by the kernel that adds them up; the library's as the best of its usual tiles.  Over those
+# products, the library's time and with this choice (us): 2,048 x 2,048 at 1,037 rows 16.3 and 15.3, 3,072 x 2,048
+# 20.2 and 16.3, 3,072 x 1,024 13.6 and 10.7; a closing product with the sum that its reader takes: 2,048 x 7,168 at
+# 1,037 rows 50.2 and 39.5, at 2,048 67 and 58, 2,048 x 8,192 at 2,048 69 and 64, 1,024 x 4,608 at 1,777 32 and 24.
+# On average 4 percent (products), 10 (closing ones), the worst 5 and 3 slower.  Beyond 3,072 rows few tiles'
+# outputs are left and the estimates are worth less: not taken.
+HALF_STEP_US = {128: 0.331, 192: 0.456, 256: 0.593}
+HALF_FULLER = {128: 0.67, 192: 0.58, 256: 0.41}      # of a step's time, for a full round, from half a round on 0
+HALF_START_US = 4.6
+HALF_WRITE_US = 0.224                               # a megabyte of 32-bit sums
+HALF_MAX_ROWS = 3072
+HALF_MIN_RANGE = 512
+READ_BYTES_PER_US = 7.5e6                           # of ranges that the norm adds up, and of the stream it then writes
+LIBRARY_TILES = ((256, 256), (256, 192), (192, 256), (256, 128), (128, 256), (128, 128), (128, 96), (96, 128),
+                 (128, 64), (64, 128), (64, 64))
+
+
+def library_us(M: int, N: int, K: int, area: float, sides: float, start: float) -> float:
+    """An estimate of the library's product: the best over its tiles, whose step of 64 elements of K takes
+    ``area`` for a full tile of 256 x 256 and ``sides`` for its rows and columns."""
+    best = float("inf")
+    for a, b in LIBRARY_TILES:
+        tiles = -(-M // a) * -(-N // b)
+        rounds = -(-tiles // 256)
+        step = area * a * b / 65536 + sides * (a + b) / 512
+        best = min(best, start + rounds * (K / 64 * step * (0.9 + 0.2 * max(0.5, tiles / 256 / rounds)) + 2.0))
+    return best
+
+
+@functools.lru_cache(maxsize=16384)
+def half_plan(M: int, N: int, K: int, closing: bool) -> Tuple[int, int]:
+    """``(height of a tile, ranges of K)`` for a product of ``M`` rows on csrc/gemm_half.hip, or ``(0, 0)``.
+    ``closing``: its ranges are added up by the next norm, and the library would add it to the stream."""
+    if not TILES_MAX_ROWS < M <= HALF_MAX_ROWS or K % 64 or K < HALF_MIN_RANGE or N * K > WIDE_MAX_ELEMENTS:
+        return 0, 0
+    best = library_us(M, N, K, 0.162, 0.86, 0.55) if closing else library_us(M, N, K, 0.881, 0.343, 4.86)
+    plan = 0, 0
+    for height, step in HALF_STEP_US.items():
+        for ranges in (2, 3, 4) if closing else (1,):
+            tiles = -(-M // height) * -(-N // 128) * ranges
+            steps = -(-(K // 64) // ranges)
+            if tiles > 256 or K - (ranges - 1) * steps * 64 < HALF_MIN_RANGE:
+                continue
+            us = HALF_START_US + steps * step * (1 + HALF_FULLER[height] * max(0.0, tiles / 256 - 0.5)) \
+                + HALF_WRITE_US * M * N * 4e-6 * (ranges if closing else 0.5) \
+                + ((ranges + 1) * M * N * 4 / READ_BYTES_PER_US if closing else 0.0)
+            if us < best:
+                best, plan = us, (height, ranges)
+    return plan
+
+
+def _half_product(x: torch.Tensor, weight: torch.Tensor, height: int, ranges: int,
+                  into: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """The product with ``half_plan``'s answer: bfloat16 ``[M, N]``, or with ranges 32-bit ``[ranges, M, N]``;
+    ``None``: operands that do not start on 16 bytes."""
+    if not height or (x.data_ptr() | weight.data_ptr()) % 16:
+        return None
+    M, K = x.shape
+    N = weight.shape[0]
+    out = into if into is not None else \
+        torch.empty((ranges, M, N) if ranges > 1 else (M, N),
+                    dtype=torch.float32 if ranges > 1 else torch.bfloat16, device=x.device)
+    rc = _fn("gemm_half", "za_gemm_bf16_half")(_ptr(x), _ptr(weight), _ptr(out), _code(out.dtype), M, N, K, height,
+                                               ranges, _stream())
+    _check(rc, "gemm_bf16_half", f"M={M} N={N} K={K} height={height} ranges={ranges}")
+    _note("linear", M=M, N=N, K=K, norm_in_product=False, added_to_stream=False, partial_sums=ranges,
+          out=out.dtype, kernel="half")
+    return out
+
+
+def linear_closing(x, weight: torch.Tensor, accumulate: Optional[torch.Tensor] = None,
+                   tune: Optional[bool] = None) -> Optional[torch.Tensor]:
+    """``linear`` of a product that the next norm may add up (``partial_ok``) or that may add itself to
+    ``accumulate``, with a third way: where the library would add many rows to the stream, ranges of K on
+    csrc/gemm_half.hip if ``half_plan`` expects them, and the norm that adds them up, to end sooner."""
+    if accumulate is not None and isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 \
+            and weight.dtype == torch.bfloat16 and x.dim() == 2 and weight.dim() == 2 \
+            and x.shape[0] > LIBRARY_SPLIT_ROWS and library_adds(x.shape[0], weight.shape[0], x.shape[1]):
+        M, K = x.shape
+        _need(x, "x", torch.bfloat16)
+        _need(weight, "weight", torch.bfloat16, (weight.shape[0], K))
+        out = _half_product(x, weight, *half_plan(M, weight.shape[0], K, True))
+        if out is not None:
+            return out
+    return linear(x, weight, partial_ok=True, accumulate=accumulate, tune=tune)
+
+
 def linear(x, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out_dtype: Optional[torch.dtype] = None, force_tiled: bool = False,
            partial_ok: bool = False,
@@ -1137,6 +1231,10 @@ def linear(x, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
         if _tiles_product(x, weight, out, splits):
             _note("linear", M=M, N=N, K=K, norm_in_product=False, added_to_stream=False,
                   partial_sums=splits, out=out.dtype, kernel="tiles")
+            return out
+    if library and splits == 1 and bias is None and out_dtype == torch.bfloat16:
+        out = _half_product(x, weight, *half_plan(M, N, K, False), into=into)
+        if out is not None:
             return out
     if library:
         # (with ranges of K: one batched product, [P, M, K/P] x [P, K/P, N])

@@ -93,8 +93,7 @@ class SwiGLU(FeedForward):
                 if a is None:
                     a = ops.gated_unit(ops.linear(x, self.gate_up, tune=self.runtime.tune),
                                        self.activation)
-            return ops.linear(a, self.down, partial_ok=True, accumulate=stream,
-                              tune=self.runtime.tune)
+            return ops.linear_closing(a, self.down, stream, tune=self.runtime.tune)
         bf16 = x.dtype == torch.bfloat16 and self.gate_up.dtype == torch.bfloat16
         if bf16 and x.shape[0] <= 16 and x.shape[1] <= 8192:
             # a decode batch: the gate is applied to the projection's accumulators
@@ -108,7 +107,7 @@ class SwiGLU(FeedForward):
             a = self.gated_by_tiles(x)
             if a is None:
                 a = ops.swiglu(ops.linear(x, self.gate_up, tune=self.runtime.tune))
-        return ops.linear(a, self.down, partial_ok=True, accumulate=stream, tune=self.runtime.tune)
+        return ops.linear_closing(a, self.down, stream, tune=self.runtime.tune)
 
 
 class ClampedGLU(FeedForward):

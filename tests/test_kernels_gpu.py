@@ -2037,7 +2037,7 @@ def test_products_that_the_estimates_give_to_one_round(M, N, K):
 
 @pytest.mark.parametrize("E,top,K,columns", [(12, 3, 1024, 2304), (12, 1, 1088, 2311), (70, 7, 512, 640), (70, 2, 576, 1288)])
 def test_grouped_products_whose_experts_end_in_each_height_of_tile(E, top, K, columns):
-    """Wide tiles of 256, 192 and 128: an expert's rest of 0, 1, 128, 129, 192, 193 and 255 assignments behind
+    """Wide tiles of 256 and 128: an expert's rest of 0, 1, 128, 129, 192, 193 and 255 assignments behind
     none, one and two full tiles, experts beyond the first 64, tokens of which several assignments fall
     to one place of the lists; against 64-bit sums, and the bits that tokens on their own have."""
     o = ops()

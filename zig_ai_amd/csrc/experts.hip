@@ -314,12 +314,14 @@ grouped_gemm_bf16_tiled_kernel(GroupedArgs g) {
 }
 
 // How many tiles of class CLASS (their rows) an expert of `c` assignments makes.  HIGH 256: full tiles of 256,
-// and what is left at its end in one as low as holds it, 128, 192 or 256; HIGH 128: tiles of 128 only.
+// and what is left at its end in one of 128 where that holds it; HIGH 128: tiles of 128 only.  (Ends of 192 as a
+// third kind take the experts' tiles apart: 32 experts, 1,029 tokens unevenly, 4 each, 71 us instead of 70, down
+// 40 instead of 38.)
 template <int HIGH, int CLASS>
 __device__ __forceinline__ int wide_tiles(int c) {
   if (HIGH == 128) return CLASS == 128 ? (c + 127) / 128 : 0;
-  const int rest = c & 255;
-  return CLASS == 256 ? (c >> 8) + (rest > 192) : CLASS == 192 ? rest > 128 && rest <= 192 : rest > 0 && rest <= 128;
+  const int full = (c + 127) >> 8;
+  return CLASS == 256 ? full : c > full * 256;
 }
 
 // Sums over a wave's lanes up to and including each, without LDS (six shuffles take some 600 clocks of waiting).
@@ -349,30 +351,29 @@ __device__ __forceinline__ void wide_find(const int* __restrict__ counts, int E,
       const int tile = b - first - (__builtin_amdgcn_readlane(end, at) - __builtin_amdgcn_readlane(tiles, at));
       *e_out = __builtin_amdgcn_readfirstlane(e0 + at);
       *count_out = n;
-      *m0_out = HIGH == 256 && CLASS != 256 ? n & ~255 : tile * HIGH;
+      *m0_out = HIGH != CLASS ? n & ~255 : tile * HIGH;
       return;
     }
     first += __builtin_amdgcn_readlane(end, 63);
   }
 }
 
-// Tiles of 256, 192 or 128 x 256 (tiles_wide.h); HIGH as above.  UNIT: 0 without, else GATED as above with the
+// Tiles of 256 or 128 x 256 (tiles_wide.h); HIGH as above.  UNIT: 0 without, else GATED as above with the
 // unit's kind as a constant, 4: any (for 32-bit results; the three kinds' stores side by side cost registers).
 template <typename TO, int UNIT, int HIGH>
 __global__ void __launch_bounds__(256, 1)
 grouped_gemm_bf16_wide_kernel(GroupedArgs g) {
   constexpr bool GATED = UNIT > 0;
   __shared__ __attribute__((aligned(16))) char lds[GW_LDS];
-  // Workgroups are dealt to the eight dies in turn: a die takes an eighth of the highest tiles, an expert's
-  // stretches of outputs side by side, and then an eighth of each lower kind, which take less long and
+  // Workgroups are dealt to the eight dies in turn: a die takes an eighth of the high tiles, an expert's
+  // stretches of outputs side by side, and then an eighth of the low ones, which take half as long and
   // fill the ends.
   const int columns = (g.N + (GATED ? 127 : 255)) / (GATED ? 128 : 256), die = blockIdx.x & 7;
-  int n256 = 0, n192 = 0, n128 = 0;
+  int n256 = 0, n128 = 0;
   const int lane64 = threadIdx.x & 63, first64 = lane64 < g.E ? g.counts[lane64] : 0;
   for (int e0 = 0; e0 < g.E; e0 += 64) {
     const int c = e0 == 0 ? first64 : e0 + lane64 < g.E ? g.counts[e0 + lane64] : 0;
     n256 += wide_tiles<HIGH, 256>(c);
-    n192 += wide_tiles<HIGH, 192>(c);
     n128 += wide_tiles<HIGH, 128>(c);
   }
   int at = blockIdx.x >> 3, index = -1;
@@ -452,12 +453,6 @@ grouped_gemm_bf16_wide_kernel(GroupedArgs g) {
       if (index < 0) return;
       wide_find<HIGH, 256>(g.counts, g.E, first64, index / columns, &e, &m0, &count);
       serve(std::integral_constant<int, 8>{});
-      return;
-    }
-    if (mine_of(n192)) {
-      if (index < 0) return;
-      wide_find<HIGH, 192>(g.counts, g.E, first64, index / columns, &e, &m0, &count);
-      serve(std::integral_constant<int, 6>{});
       return;
     }
   }
@@ -567,7 +562,7 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     // -> 182 | 107; at 517 tokens (65 rows an expert) 73 | 36 against 84 | 38.  8 experts of 4,096, 2 a
     // token, 1,900 tokens: up 99 -> 64 (128 high 85), down, 128 high for want of tiles, 92 -> 75 (256
     // high 95); 500 tokens: up, 128 high, 56 -> 43, down stays (54 against 66).  The sums are the same
-    // to the last bit.  With four waves of 128 x 128 in place of eight of 128 x 64, ends of 192, the unit in
+    // to the last bit.  With four waves of 128 x 128 in place of eight of 128 x 64, the unit in
     // the hardware's exponential and bfloat16 stored in whole lines, before and after (us): 32 experts, gated,
     // 1,777 tokens 90 and 79, unevenly taken 105 and 92, 4,096 tokens unevenly 186 and 154; 8 experts of 4,096,
     // gated, 1,777 tokens 168 and 123; their down product at 4,096 tokens 153 and 145.  32-bit results of few
@@ -593,7 +588,7 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
       if (wide > low) high = 0;
       // (an expert's full tiles and its last one, each kind an eighth a die)
       const long long tiles = (A + high - 1) / max(high, 1) + experts;
-      const long long blocks = (tiles * columns + 7) / 8 * 8 + 16;
+      const long long blocks = (tiles * columns + 7) / 8 * 8 + 8;
       if (high && blocks > 0x7fffffffLL) return ZA_ERR_ARG;
 #define ZA_GW(TO, UNIT)                                                                                    \
   {                                                                                                        \

@@ -471,7 +471,7 @@ grouped_gemm_bf16_wide_kernel(GroupedArgs g) {
 
 // VEC: 0 an element at a time, 1 four, 2 (32-bit rows, K a multiple of 32) through LDS without registers.
 template <typename TA, typename TO, bool GATED, int VEC>
-__global__ void __launch_bounds__(512)
+__global__ void __launch_bounds__(VEC == 2 ? 256 : 512)
 grouped_gemm_f32_kernel(GroupedArgs g) {
   int e, tile, count;
   if (!find_tile<GF_BM>(g.counts, g.E, blockIdx.x, &e, &tile, &count)) return;
@@ -480,10 +480,13 @@ grouped_gemm_f32_kernel(GroupedArgs g) {
   const int K = g.K, N = g.N;
   const float* W = (const float*)g.W + (size_t)e * (GATED ? 2 * N : N) * K;
   TO* out = (TO*)g.out;
-  auto a_at = [&](int r) { return (const TA*)g.src + (size_t)(mine[min(m0 + r, count - 1)] / g.src_div) * K; };
-  auto w_at = [&](int r) {
+  auto a_row = [&](int r) {
+    const int a = mine[min(m0 + r, count - 1)];
+    return g.src_div == 1 ? a : token_of(g, a);
+  };
+  auto w_row = [&](int r) {
     const int n = min(n0 + (GATED ? (r >> 5) * 16 + (r & 15) : r), N - 1);
-    return W + (size_t)(n + (GATED && (r & 16) ? N : 0)) * K;
+    return n + (GATED && (r & 16) ? N : 0);
   };
   auto store = [&](int r, int n, const f32x4_t(&v)[GF_BN / 32]) {
     if (m0 + r >= count) return;
@@ -506,8 +509,12 @@ grouped_gemm_f32_kernel(GroupedArgs g) {
             at[n0 + n + j * 16 + i] = from_f32<TO>(expert_act(v[j][i], g.act) * g.out_scale * w);
     }
   };
-  if constexpr (VEC == 2) f32_tile_async<GF_BM, GF_BN, 2, 3>(K, a_at, w_at, store);
-  else f32_tile<TA, GF_BM, GF_BN, 2, VEC == 1>(K, a_at, w_at, store);
+  if constexpr (VEC == 2)
+    f32_tile_async<GF_BM, GF_BN, 4>(K, (const float*)g.src, W, [&](int r) { return (unsigned)a_row(r) * (unsigned)(K * 4); },
+                                    [&](int r) { return (unsigned)w_row(r) * (unsigned)(K * 4); }, store);
+  else
+    f32_tile<TA, GF_BM, GF_BN, 2, VEC == 1>(K, [&](int r) { return (const TA*)g.src + (size_t)a_row(r) * K; },
+                                            [&](int r) { return W + (size_t)w_row(r) * K; }, store);
 }
 
 // dtype codes: 0 = float32, 1 = bfloat16.  `src` has `src_rows` rows of K elements; the
@@ -631,12 +638,13 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
   const int columns = gate ? GF_BN / 2 : GF_BN;
   dim3 grid((unsigned)((A + GF_BM - 1) / GF_BM + experts), (unsigned)((N + columns - 1) / columns)), block(512);
   const bool vec = K % 4 == 0 && (uintptr_t)src % (src_dtype == 1 ? 8 : 16) == 0 && (uintptr_t)W % 16 == 0;
-  const bool whole = vec && src_dtype == 0 && K % F32_BK == 0;
+  const bool whole = vec && src_dtype == 0 && K % F32_BK == 0 && src_rows * K < (1LL << 30) &&
+                     (gate ? 2LL : 1LL) * N * K < (1LL << 30);
 #define ZA_GFV(TA, TO, GATED)                                                                              \
   {                                                                                                        \
     if constexpr (std::is_same<TA, float>::value) {                                                        \
       if (whole) {                                                                                         \
-        hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, GATED, 2>), grid, block, 0, stream, g);        \
+        hipLaunchKernelGGL((grouped_gemm_f32_kernel<TA, TO, GATED, 2>), grid, dim3(256), 0, stream, g);    \
         return za_launch_status();                                                                         \
       }                                                                                                    \
     }                                                                                                      \

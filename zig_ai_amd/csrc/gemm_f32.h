@@ -13,6 +13,8 @@
 // weights are the first operand: a lane ends with four consecutive outputs of one row.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 #define F32_CHAIN 128
@@ -168,167 +170,190 @@ __device__ __forceinline__ void f32_tile(int K, AAt a_at, WAt w_at, Store store)
   for (int i = 0; i < TM; ++i) store(wm + i * 16 + frow, wn + fk, total[i]);
 }
 
-// The same tile, groups and order of sums for 32-bit rows on 16 bytes and K in whole steps of 32: the
-// steps go from memory into NS places of LDS without passing registers, NS - 1 of them under way (the
-// tile above has one, in registers, and waits for memory where the weights come from there).  A row's
-// eight pieces of four elements lie in the order piece ^ (row % 8), so that the sixteen rows that a
-// fragment is read from fall into different banks.  Reads of LDS and their wait stand in one block: the
-// compiler would have each wait for every request under way to LDS.
-template <int BM, int BN, int KG, int NS, typename AAt, typename WAt, typename Store>
-__device__ __forceinline__ void f32_tile_async(int K, AAt a_at, WAt w_at, Store store) {
+// The same order of sums for 32-bit rows on 16 bytes and K in whole steps of 32, by four waves without groups: the
+// steps go from memory into NS places of LDS without passing registers.  A phase is 16 elements of k, four
+// products for each of TM x TN sums, one asm statement: the reads of the next phase's fragments and, in a step's
+// second phase, the requests for step s + NS stand between the products, in their shadow, and the wait for the
+// reads ends the statement, as their results may only be known to the compiler when they are there.  One
+// barrier a step, between its phases: it ends the reads of the step's place and says that the next step has
+// arrived.
+// Nothing may touch the sums between these statements: another instruction that reads a product's sums has to wait
+// some clocks for them, which the compiler does not see to here.  So a chain's steps stand in a row without a
+// branch (with one, the compiler copies sums where the ways meet: wrong, and half a step's time); what lies
+// beyond K is requested for no lane.
+// 64 x 64 takes 1,150 clocks a step of 1,024 of products, 32 x 64 615 of 512.  A row's eight pieces of four elements
+// lie in the order piece ^ (row % 8), so that the sixteen rows that a fragment is read from fall into
+// different banks.
+#define GF_MF(i, j, e) "v_mfma_f32_16x16x4_f32 %[c" #i #j "], %[w" #j #e "], %[a" #i #e "], %[c" #i #j "]\n"
+#define GF_RD(k, p, o) "ds_read_b128 %[n" #k "], %[" #p "] offset:" #o "\n"
+// (m0 is set one instruction ahead of the request, which needs that distance; nothing else here keeps a value in it)
+#define GF_TO(k) "s_mov_b32 m0, %[m" #k "]\n"
+#define GF_RQ(k, b)                                                                                     \
+  "s_mov_b32 exec_lo, %[go]\n" "s_mov_b32 exec_hi, %[go]\n" "global_load_lds_dwordx4 %[v" #k "], %[" #b "]\n" \
+  "s_mov_b64 exec, -1\n"
+#define GF_FOUR(n, v) [n##0] "v"(v[0]), [n##1] "v"(v[1]), [n##2] "v"(v[2]), [n##3] "v"(v[3])
+#define GF_WAIT "s_waitcnt lgkmcnt(0)\n"
+#define GF_ALL12(e) GF_MF(0, 0, e) GF_MF(0, 1, e)
+#define GF_ALL22(e) GF_ALL12(e) GF_MF(1, 0, e) GF_MF(1, 1, e)
+#define GF_START12 GF_MF(0, 0, 0) GF_RD(0, pw, 0) GF_MF(0, 1, 0) GF_RD(1, pw, 2048) GF_RD(2, pa, 0)
+#define GF_START22 \
+  GF_MF(0, 0, 0) GF_RD(0, pw, 0) GF_MF(0, 1, 0) GF_RD(1, pw, 2048) GF_MF(1, 0, 0) GF_RD(2, pa, 0) GF_MF(1, 1, 0) GF_RD(3, pa, 2048)
+#define GF_WITH12                                                                                     \
+  GF_MF(0, 0, 1) GF_TO(0) GF_MF(0, 1, 1) GF_RQ(0, bw) GF_MF(0, 0, 2) GF_TO(1) GF_MF(0, 1, 2) GF_RQ(1, bw) \
+  GF_MF(0, 0, 3) GF_TO(2) GF_MF(0, 1, 3) GF_RQ(2, ba)
+#define GF_WITH22                                                                                         \
+  GF_MF(0, 0, 1) GF_TO(0) GF_MF(0, 1, 1) GF_RQ(0, bw) GF_MF(1, 0, 1) GF_TO(1) GF_MF(1, 1, 1) GF_RQ(1, bw)     \
+  GF_MF(0, 0, 2) GF_MF(0, 1, 2) GF_TO(2) GF_MF(1, 0, 2) GF_RQ(2, ba) GF_MF(1, 1, 2) GF_TO(3) GF_MF(0, 0, 3) \
+  GF_RQ(3, ba) GF_MF(0, 1, 3) GF_MF(1, 0, 3) GF_MF(1, 1, 3)
+#define GF_C12 [c00] "+v"(c[0][0]), [c01] "+v"(c[0][1])
+#define GF_C22 GF_C12, [c10] "+v"(c[1][0]), [c11] "+v"(c[1][1])
+#define GF_N12 [n0] "=&v"(nw[0]), [n1] "=&v"(nw[1]), [n2] "=&v"(na[0])
+#define GF_N22 GF_N12, [n3] "=&v"(na[1])
+#define GF_IN12 GF_FOUR(w0, w[0]), GF_FOUR(w1, w[1]), GF_FOUR(a0, a[0]), [pw] "v"(pw), [pa] "v"(pa)
+#define GF_IN22 GF_IN12, GF_FOUR(a1, a[1])
+#define GF_Q12                                                                                              \
+  [v0] "v"(q.offw[0]), [m0] "s"(q.tow), [v1] "v"(q.offw[1]), [m1] "s"(q.tow + 4096), [v2] "v"(q.offa[0]),         \
+  [m2] "s"(q.toa), [bw] "s"(q.w), [ba] "s"(q.a), [go] "s"(q.go)
+#define GF_Q22 GF_Q12, [v3] "v"(q.offa[1]), [m3] "s"(q.toa + 4096)
+
+struct F32Requests {      // W's and A's offsets of a lane, where its first piece goes, W's and A's base, all lanes or none
+  const unsigned *offw, *offa;
+  unsigned tow, toa;
+  const char *w, *a;
+  int go;
+};
+
+template <int TM, int TN, bool REQUEST>
+__device__ __forceinline__ void f32_phase(f32x4_t (&c)[TM][TN], const f32x4_t (&w)[TN], const f32x4_t (&a)[TM],
+                                          f32x4_t (&nw)[TN], f32x4_t (&na)[TM], unsigned pw, unsigned pa,
+                                          const F32Requests& q) {
+  static_assert(TN == 2 && (TM == 2 || TM == 1), "one of these");
+  if constexpr (TM == 1 && REQUEST)
+    asm volatile(GF_START12 GF_WITH12 GF_WAIT : GF_C12, GF_N12 : GF_IN12, GF_Q12 : "memory");
+  else if constexpr (TM == 1)
+    asm volatile(GF_START12 GF_ALL12(1) GF_ALL12(2) GF_ALL12(3) GF_WAIT : GF_C12, GF_N12 : GF_IN12 : "memory");
+  else if constexpr (REQUEST)
+    asm volatile(GF_START22 GF_WITH22 GF_WAIT : GF_C22, GF_N22 : GF_IN22, GF_Q22 : "memory");
+  else
+    asm volatile(GF_START22 GF_ALL22(1) GF_ALL22(2) GF_ALL22(3) GF_WAIT : GF_C22, GF_N22 : GF_IN22 : "memory");
+}
+
+// `a_at(r)` and `w_at(r)`: bytes from A and W to the tile's row r (to some readable row where there is none), below
+// 4 GB; `store` as above.
+template <int BM, int BN, int NS, typename AAt, typename WAt, typename Store>
+__device__ __forceinline__ void f32_tile_async(int K, const float* A, const float* W, AAt a_at, WAt w_at, Store store) {
   constexpr int TM = BM / 32, TN = BN / 32, LA = BM / 32, LW = BN / 32, STEPS = F32_CHAIN / F32_BK;
-  static_assert((TM == 2 && TN == 2) || (TM == 1 && TN == 2) || (TM == 1 && TN == 1), "see take");
-  __shared__ __attribute__((aligned(16))) float As[KG][NS][BM * F32_BK];
-  __shared__ __attribute__((aligned(16))) float Ws[KG][NS][BN * F32_BK];
-  __shared__ __attribute__((aligned(16))) f32x4_t sums[KG > 1 ? KG - 1 : 1][KG > 1 ? TM * TN * 256 : 1];
-  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-  const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int PLACE = (BM + BN) * F32_BK * 4;      // bytes; A's rows behind W's
+  __shared__ __attribute__((aligned(16))) char lds[NS * PLACE];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
-  const int lrow = wave * 8 + (lane >> 3), piece = ((lane & 7) ^ (lane >> 3)) * 4;
-  const float *a_row[LA], *w_row[LW];
+  const int lrow = wave * 8 + (lane >> 3), piece = ((lane & 7) ^ (lane >> 3)) * 16;
+  unsigned offa[LA], offw[LW];
 #pragma unroll
-  for (int i = 0; i < LA; ++i) a_row[i] = a_at(lrow + 32 * i) + piece;
+  for (int i = 0; i < LA; ++i) offa[i] = a_at(lrow + 32 * i) + piece;
 #pragma unroll
-  for (int i = 0; i < LW; ++i) w_row[i] = w_at(lrow + 32 * i) + piece;
-  // step s of the group: a chain's steps, then those of the chain KG on
-  auto k_of = [&](int s) { return ((s / STEPS) * KG + group) * F32_CHAIN + (s % STEPS) * F32_BK; };
-  auto request = [&](int s, int p) {
-    const int k0 = k_of(s) < K ? k_of(s) : 0;      // (a step beyond K: not multiplied)
-#pragma unroll
-    for (int i = 0; i < LA; ++i) lds_request(a_row[i] + k0, &As[group][p][(32 * i + wave * 8) * F32_BK]);
-#pragma unroll
-    for (int i = 0; i < LW; ++i) lds_request(w_row[i] + k0, &Ws[group][p][(32 * i + wave * 8) * F32_BK]);
+  for (int i = 0; i < LW; ++i) offw[i] = w_at(lrow + 32 * i) + piece;
+  const int steps = K / F32_BK;
+  const unsigned base = lds_address(lds);
+  F32Requests q{offw, offa, base + wave * 1024, base + BN * F32_BK * 4 + wave * 1024, (const char*)W, (const char*)A, 0};
+  auto all_if_negative = [](int n) {      // (in a scalar register, whatever the compiler prefers)
+    int v = n >> 31;
+    asm volatile("" : "+v"(v));
+    return __builtin_amdgcn_readfirstlane(v);
   };
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4_t acc[TM][TN], total[TM][TN];
+  auto behind = [&](bool last) {      // a step's requests, which went to the last place
+    const unsigned by = last ? (unsigned)(-(NS - 1) * PLACE) : (unsigned)PLACE;
+    q.w += F32_BK * 4;
+    q.a += F32_BK * 4;
+    q.tow += by;
+    q.toa += by;
+  };
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const int go = all_if_negative(s - steps);
+    auto request = [&](const char* from, unsigned offset, unsigned to) {
+      asm volatile("s_mov_b32 m0, %0\n" "s_mov_b32 exec_lo, %3\n" "s_mov_b32 exec_hi, %3\n" "global_load_lds_dwordx4 %1, %2\n"
+                   "s_mov_b64 exec, -1\n" :: "s"(to), "v"(offset), "s"(from), "s"(go) : "memory");
+    };
+#pragma unroll
+    for (int i = 0; i < LW; ++i) request(q.w, offw[i], q.tow + i * 4096);
+#pragma unroll
+    for (int i = 0; i < LA; ++i) request(q.a, offa[i], q.toa + i * 4096);
+    behind(s == NS - 1);
+  }
+  f32x4_t total[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = total[i][j] = zero;
+    for (int j = 0; j < TN; ++j) total[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   const int frow = lane & 15, fk = lane >> 4;
-  const unsigned slot[2] = {(unsigned)((fk ^ (frow & 7)) * 16), (unsigned)(((4 + fk) ^ (frow & 7)) * 16)};
-  f32x4_t fa[2][TM], fw[2][TN];
-  auto take = [&](int p) {
-    const unsigned w = lds_address(&Ws[group][p][(wn + frow) * F32_BK]), a = lds_address(&As[group][p][(wm + frow) * F32_BK]);
-    const unsigned w0 = w + slot[0], w1 = w + slot[1], a0 = a + slot[0], a1 = a + slot[1];
-    if constexpr (TM == 2) {
-      asm volatile(
-          "ds_read_b128 %0, %8 offset:0\n" "ds_read_b128 %1, %8 offset:2048\n"
-          "ds_read_b128 %2, %10 offset:0\n" "ds_read_b128 %3, %10 offset:2048\n"
-          "ds_read_b128 %4, %9 offset:0\n" "ds_read_b128 %5, %9 offset:2048\n"
-          "ds_read_b128 %6, %11 offset:0\n" "ds_read_b128 %7, %11 offset:2048\n"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(fw[0][0]), "=&v"(fw[0][1]), "=&v"(fa[0][0]), "=&v"(fa[0][1]),
-            "=&v"(fw[1][0]), "=&v"(fw[1][1]), "=&v"(fa[1][0]), "=&v"(fa[1][1])
-          : "v"(w0), "v"(w1), "v"(a0), "v"(a1)
-          : "memory");
-    } else if constexpr (TN == 2) {
-      asm volatile(
-          "ds_read_b128 %0, %6 offset:0\n" "ds_read_b128 %1, %6 offset:2048\n"
-          "ds_read_b128 %2, %8 offset:0\n" "ds_read_b128 %3, %7 offset:0\n"
-          "ds_read_b128 %4, %7 offset:2048\n" "ds_read_b128 %5, %9 offset:0\n"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(fw[0][0]), "=&v"(fw[0][1]), "=&v"(fa[0][0]), "=&v"(fw[1][0]),
-            "=&v"(fw[1][1]), "=&v"(fa[1][0])
-          : "v"(w0), "v"(w1), "v"(a0), "v"(a1)
-          : "memory");
-    } else {
-      asm volatile(
-          "ds_read_b128 %0, %4 offset:0\n" "ds_read_b128 %1, %6 offset:0\n"
-          "ds_read_b128 %2, %5 offset:0\n" "ds_read_b128 %3, %7 offset:0\n"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(fw[0][0]), "=&v"(fa[0][0]), "=&v"(fw[1][0]), "=&v"(fa[1][0])
-          : "v"(w0), "v"(w1), "v"(a0), "v"(a1)
-          : "memory");
-    }
+  const unsigned half[2] = {(unsigned)((fk ^ (frow & 7)) * 16), (unsigned)(((4 + fk) ^ (frow & 7)) * 16)};
+  const unsigned rw = base + (wn + frow) * F32_BK * 4, ra = base + (BN + wm + frow) * F32_BK * 4;
+  auto meet = [&]() {      // nothing moves over it
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
   };
-  // the other groups' sums of the chain that has ended, behind a barrier
-  auto add_sums = [&]() {
+  __builtin_amdgcn_s_waitcnt(ZA_VMCNT((NS - 1) * (LA + LW)));
+  meet();
+  f32x4_t a0[TM], w0[TN], a1[TM], w1[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+    asm volatile("ds_read_b128 %0, %1\n" "s_waitcnt lgkmcnt(0)" : "=&v"(w0[j]) : "v"(rw + half[0] + j * 2048) : "memory");
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+    asm volatile("ds_read_b128 %0, %1\n" "s_waitcnt lgkmcnt(0)" : "=&v"(a0[i]) : "v"(ra + half[0] + i * 2048) : "memory");
+  unsigned at = 0;
+  int left = steps - NS;      // steps that are still to be requested
+  auto chain = [&](auto count) {
+    f32x4_t acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int g = 1; g < KG; ++g) {
-          f32x4_t v;
-          asm volatile("ds_read_b128 %0, %1\ns_waitcnt lgkmcnt(0)"
-                       : "=&v"(v) : "v"(lds_address(&sums[g - 1][(i * TN + j) * 256 + tid])) : "memory");
-          total[i][j] += v;
-        }
-  };
-  // all groups walk the same number of steps
-  const int steps = K <= KG * F32_CHAIN ? (min(K, F32_CHAIN) + F32_BK - 1) / F32_BK
-                                        : (K + KG * F32_CHAIN - 1) / (KG * F32_CHAIN) * STEPS;
-#pragma unroll
-  for (int i = 0; i < NS - 1; ++i)
-    if (i < steps) request(i, i);
-  int p = 0, q = NS - 1;
-  bool pending = false;
-  for (int s = 0; s < steps; ++s) {
-    // this step's tiles have arrived when only those requested after them are on their way
-    if (s + NS - 2 < steps) __builtin_amdgcn_s_waitcnt(ZA_VMCNT((NS - 2) * (LA + LW)));
-    else __builtin_amdgcn_s_waitcnt(ZA_VMCNT(0));
-    __builtin_amdgcn_s_barrier();
-    take(p);
-    if (s + NS - 1 < steps) request(s + NS - 1, q);
-    if (KG > 1 && pending && group == 0) add_sums();
-    pending = false;
-    if (k_of(s) < K) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[h][j][e], fa[h][i][e], acc[i][j], 0, 0, 0);
+    for (int u = 0; u < decltype(count)::value; ++u) {
+      const bool last = at == (NS - 1) * PLACE;
+      const unsigned to = last ? 0 : at + PLACE;
+      f32_phase<TM, TN, false>(acc, w0, a0, w1, a1, rw + at + half[1], ra + at + half[1], q);
+      __builtin_amdgcn_s_waitcnt(ZA_VMCNT((NS - 2) * (LA + LW)));      // (the next step has arrived)
+      meet();
+      q.go = all_if_negative(-left);
+      --left;
+      // (the last step's reads find an older step's tiles: not used)
+      f32_phase<TM, TN, true>(acc, w1, a1, w0, a0, rw + to + half[0], ra + to + half[0], q);
+      behind(last);
+      at = to;
     }
-    if (s + 1 == steps || (s + 1) % STEPS == 0) {
-      if (KG == 1 || group == 0) {
+    asm volatile("s_nop 15" : "+v"(acc[0][0]));
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) total[i][j] += acc[i][j];
-      } else {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            asm volatile("ds_write_b128 %0, %1" :: "v"(lds_address(&sums[group - 1][(i * TN + j) * 256 + tid])),
-                         "v"(acc[i][j]) : "memory");
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      for (int j = 0; j < TN; ++j) {
+        if (i + j > 0) asm volatile("" : "+v"(acc[i][j]));
+        total[i][j] += acc[i][j];
       }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = zero;
-      pending = true;
-    }
-    __builtin_amdgcn_sched_barrier(0);     // (or the products move behind the next wait)
-    p = p + 1 == NS ? 0 : p + 1;
-    q = q + 1 == NS ? 0 : q + 1;
-  }
-  if constexpr (KG > 1) {
-    __builtin_amdgcn_s_barrier();
-    if (group > 0) return;
-    add_sums();
-  }
+  };
+  for (int c = steps / STEPS; c > 0; --c) chain(std::integral_constant<int, STEPS>{});
+  const int rest = steps % STEPS;
+  if (rest == 1) chain(std::integral_constant<int, 1>{});
+  else if (rest == 2) chain(std::integral_constant<int, 2>{});
+  else if (rest == 3) chain(std::integral_constant<int, 3>{});
 #pragma unroll
   for (int i = 0; i < TM; ++i) store(wm + i * 16 + frow, wn + fk * 4, total[i]);
 }
 
-template <typename TC, int BM, int BN, int KG, int NS>
-__global__ void __launch_bounds__(256 * KG)
+template <typename TC, int BM, int BN, int NS>
+__global__ void __launch_bounds__(256)
 gemm_f32_async_kernel(const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
                       TC* __restrict__ C, int M, int N, int K, int m_tiles, int n_tiles, int wide) {
   const int at = blockIdx.x >> 3;                  // (dies and tiles as below)
   const int n_tile = (at / m_tiles) * 8 + (blockIdx.x & 7);
   if (n_tile >= n_tiles) return;
   const int m0 = (at % m_tiles) * BM, n0 = n_tile * BN;
-  f32_tile_async<BM, BN, KG, NS>(
-      K, [&](int r) { return A + (size_t)min(m0 + r, M - 1) * K; },
-      [&](int r) { return W + (size_t)min(n0 + r, N - 1) * K; },
+  f32_tile_async<BM, BN, NS>(
+      K, A, W, [&](int r) { return (unsigned)min(m0 + r, M - 1) * (unsigned)(K * 4); },
+      [&](int r) { return (unsigned)min(n0 + r, N - 1) * (unsigned)(K * 4); },
       [&](int r, int n, const f32x4_t(&v)[BN / 32]) {
         if (m0 + r >= M) return;
 #pragma unroll

@@ -50,25 +50,23 @@ static int launch_f32(const TA* A, const float* W, const float* bias, TC* C, int
     if (M <= 16) ZA_F32_TILE(32, 64, 2)
     const long long n32 = (long long)tiles(M, 32) * tiles(N, 32), n3264 = (long long)tiles(M, 32) * tiles(N, 64),
                     n64 = (long long)tiles(M, 64) * tiles(N, 64);
-#define ZA_F32_ASYNC(BM, BN, KG, NS)                                                                      \
+#define ZA_F32_ASYNC(BM, BN, NS)                                                                          \
   {                                                                                                       \
     ZA_F32_GRID(BM, BN)                                                                                   \
-    hipLaunchKernelGGL((gemm_f32_async_kernel<TC, BM, BN, KG, NS>), grid, dim3(256 * KG), 0, stream,      \
-                       A, W, bias, C, M, N, K, mt, nt, wide);                                             \
+    hipLaunchKernelGGL((gemm_f32_async_kernel<TC, BM, BN, NS>), grid, dim3(256), 0, stream, A, W, bias,   \
+                       C, M, N, K, mt, nt, wide);                                                         \
     return za_launch_status();                                                                            \
   }
-    // K in whole steps: tiles through LDS without registers, the same sums.  Measured, weights of
-    // several layers in turn, before and now: 448 x 9216 x 1024 101 and 91, 448 x 3072 x 1024 40 and
-    // 38, 448 x 2048 x 1024 27 and 25, 448 x 1024 x 4608 61 and 59, 100 x 9216 x 1024 42 and 38,
-    // 512 x 16384 x 2048 333 and 305 (113 TFLOP/s), 500 x 2048 x 8192 199 and 179.
-    // Tiles of 32 x 64 with a second group of waves from six chains of K on: with fewer it waits for the
-    // first (one chain: it has none of its own).  Registers, two groups, one: 65 x 16384 x 96 6, 8, 6,
-    // 130 x 16384 x 384 26, 29, 28, 130 x 65536 x 384 86, 97, 84, x 768 169, 170, 170.
-    if (K % F32_BK == 0 && n32 > 256) {
-      if (n3264 <= 256) ZA_F32_ASYNC(32, 64, 4, 2)
-      if (n64 <= 256 || ((n64 + 255) / 256) * 200 <= ((n3264 + 255) / 256) * 115) ZA_F32_ASYNC(64, 64, 1, 3)
-      if (K < 768) ZA_F32_ASYNC(32, 64, 1, 3)
-      ZA_F32_ASYNC(32, 64, 2, 3)
+    // K in whole steps: tiles through LDS without registers, the same sums, reads and requests between the
+    // products.  Measured, weights of several layers in turn, the kernels before it (with groups of waves that
+    // took a step's reads, its products and its barrier one after the other) and now: 448 x 9216 x 1024 84 and
+    // 65 (130 TFLOP/s), 350 x 9216 x 1024 84 and 61, 448 x 3072 x 1024 39 and 28, 448 x 2048 x 1024 26 and
+    // 20, 448 x 1024 x 1024 15 and 11.5, 448 x 1024 x 4608 54 and 42.
+    // 64 x 64 where the compute units take a tile half as often (0.93 of two of 32 x 64: 448 x 9216 65 and 68,
+    // 448 x 3072 34 and 28).
+    if (K % F32_BK == 0 && n32 > 256 && (long long)M * K < (1LL << 30) && (long long)N * K < (1LL << 30)) {
+      if (((n64 + 255) / 256) * 186 <= ((n3264 + 255) / 256) * 100) ZA_F32_ASYNC(64, 64, 4)
+      ZA_F32_ASYNC(32, 64, 4)
     }
 #undef ZA_F32_ASYNC
     if (n32 <= 256) ZA_F32_TILE(32, 32, 4)

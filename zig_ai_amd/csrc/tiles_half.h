@@ -179,8 +179,8 @@ struct TilesHalf {
     if constexpr (NS > 4) step(no, no, std::integral_constant<int, (NS > 4 ? NS - 5 : 0)>{});
     step(no, no, std::integral_constant<int, 0>{});
     // the last products' sums may be read by other instructions only so many clocks later
+    asm volatile("s_nop 15\n" "s_nop 15" : "+a"(acc[TM - 1][0]), "+a"(acc[TM - 1][1]), "+a"(acc[TM - 1][2]), "+a"(acc[TM - 1][3]));
 #pragma unroll
-    for (int i = TM - ROWS; i < TM; ++i)
-      asm volatile("s_nop 15\n" "s_nop 15" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]));
+    for (int i = 0; i < TM - 1; ++i) asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]));
   }
 };

@@ -208,10 +208,12 @@ struct TilesWide {
     for (; s < steps; ++s) step(std::false_type{});      // (the last one's second reads find older tiles: not used)
     // the last products' sums may be read by other instructions only so many clocks later
     asm volatile("s_nop 15\n" "s_nop 15"
-                 : "+a"(acc[TM - 2][0]), "+a"(acc[TM - 2][1]), "+a"(acc[TM - 2][2]), "+a"(acc[TM - 2][3]), "+a"(acc[TM - 2][4]),
-                   "+a"(acc[TM - 2][5]), "+a"(acc[TM - 2][6]), "+a"(acc[TM - 2][7]), "+a"(acc[TM - 1][0]), "+a"(acc[TM - 1][1]),
-                   "+a"(acc[TM - 1][2]), "+a"(acc[TM - 1][3]), "+a"(acc[TM - 1][4]), "+a"(acc[TM - 1][5]), "+a"(acc[TM - 1][6]),
-                   "+a"(acc[TM - 1][7]));
+                 : "+a"(acc[TM - 1][0]), "+a"(acc[TM - 1][1]), "+a"(acc[TM - 1][2]), "+a"(acc[TM - 1][3]), "+a"(acc[TM - 1][4]),
+                   "+a"(acc[TM - 1][5]), "+a"(acc[TM - 1][6]), "+a"(acc[TM - 1][7]));
+#pragma unroll
+    for (int i = 0; i < TM - 1; ++i)
+      asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]),
+                   "+a"(acc[i][6]), "+a"(acc[i][7]));
   }
 };
 

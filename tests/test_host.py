@@ -205,3 +205,24 @@ def test_context_split_plan():
     assert plan_split(20, 8, 8192) == (0, 1) and plan_split(7, 8, 3072)[1] == 4
     assert plan_split(1, 8, 1024) == (256, 4)             # short contexts are cut finer
     assert plan_split(1, 8, 3072) == (512, 6) and plan_split(1, 8, 512) == (0, 1)
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(32, 8, 64), (16, 2, 128), (5, 1, 64), (24, 24, 128)])
+@pytest.mark.parametrize("max_keys", [1, 63, 256, 511, 1000, 1536, 5000, 16385, 131072])
+def test_ranges_of_prompt_portions(heads, kv_heads, head_dim, max_keys):
+    """The ranges cover the longest context, none is empty, tiles do not cross them, and a launch
+    that already fills the chip, or whose rows see a short window only, is not cut."""
+    from zig_ai_amd.parts.attention import BUSY_WORKGROUPS, plan_portions
+    for rows in (2, 64, 512, 1024, 8192):
+        items = -(-rows * (heads // kv_heads) // 128)
+        for window in (0, 100):
+            keys, nsplit = plan_portions(items, kv_heads, rows, heads, head_dim, max_keys, window)
+            if nsplit == 1:
+                assert keys == 0
+                continue
+            assert not window
+            assert keys % (128 if head_dim == 64 else 64) == 0
+            assert keys * (nsplit - 1) < max_keys <= keys * nsplit
+            assert items * kv_heads * nsplit <= BUSY_WORKGROUPS
+    assert plan_portions(1024, 8, 32768, 32, 64, 32768) == (0, 1)
+    assert plan_portions(2, 8, 64, 32, 64, 8192)[1] > 8          # few rows, a long context

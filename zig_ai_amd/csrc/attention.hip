@@ -424,6 +424,17 @@ paged_attention_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __
 // The tiles go through two LDS buffers: while a tile is being computed the next one is
 // on its way from memory into registers, and the page numbers of the one after that
 // are being read.  Every tile issues the same loads, unconditionally.
+// What bounds it: the vector instructions of the softmax and the reads of LDS (32 of 1 KB a
+// wave and tile of 128 keys), which the barrier of every tile keeps from overlapping fully
+// with the products; in one prompt of some 2,000 tokens the chain of tiles of its last rows.
+// So what is not the softmax is kept scalar or out of the loop: the wave's number and with
+// it all bounds of its rows, one branch on the page size for all of a tile's pieces, two
+// instructions a masked score.  32 query heads on 8 key heads of 64, us, with a branch a
+// piece and the bounds a lane, and so: prompts of 512, 2,048, 8,192 tokens 13.9, 44, 399 ->
+// 12.7, 39.5, 383; 64 prompts of 128 40.7 -> 35; heads of 128, 2,048 tokens 75 -> 65.  (Two
+// teams of eight waves in a workgroup that share out the tiles of two items, or of one, even
+// the chains out and lose the rest to their common barrier: 35.3 for 37.2 at 2,048, but 413
+// for 360 at 8,192 and 42 for 32 at 64 prompts of 128.)
 // Operand layout of v_mfma_f32_16x16x32_bf16: lane l supplies row (l % 16), k-slots
 // (l / 16) * 8 .. + 7 of either operand and receives rows (l / 16) * 4 .. + 3, column
 // (l % 16) of the product.
@@ -463,7 +474,9 @@ paged_attention_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ o
   bf16_t* Vt = Ks + 2 * KT * LDK;                 // [2][dim][key slot]
 
   const int gkv = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // (`wave` is the same for all its lanes and known to be: what its rows can see stays in
+  // scalar registers, and the branches on it are scalar branches)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, grp = lane >> 4;
   const int G = nh / nkv;
   const bf16x8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -557,29 +570,47 @@ paged_attention_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ o
   int kpg[KVEC], vpg;
   bf16x8_t kreg[KVEC];
   bf16x4_t vreg[VVEC];
+  // (one branch on the kind of page size for all of a tile's pieces: one a piece were nine
+  // branches a tile)
   auto load_pages = [&](int tile0) {
+    int e[KVEC + 1];
 #pragma unroll
-    for (int v = 0; v < KVEC; ++v) {
-      const int e = page_entry(tile0 + krow0 + v * KROWS, page_size, ps_shift);
-      kpg[v] = table[e < last_entry ? e : last_entry];
+    for (int v = 0; v < KVEC; ++v) e[v] = tile0 + krow0 + v * KROWS;
+    e[KVEC] = tile0 + vkr * 4;
+    if (ps_shift >= 0) {
+#pragma unroll
+      for (int v = 0; v <= KVEC; ++v) e[v] >>= ps_shift;
+    } else {
+#pragma unroll
+      for (int v = 0; v <= KVEC; ++v) e[v] /= page_size;
     }
-    const int e = page_entry(tile0 + vkr * 4, page_size, ps_shift);
-    vpg = table[e < last_entry ? e : last_entry];
+#pragma unroll
+    for (int v = 0; v < KVEC; ++v) kpg[v] = table[e[v] < last_entry ? e[v] : last_entry];
+    vpg = table[e[KVEC] < last_entry ? e[KVEC] : last_entry];
   };
   // Loads never leave the pool: an unused table entry (-1) reads page 0 instead, and
   // tiles beyond the last one are fetched like any other.  A key that must not count is
   // masked in the scores, whatever its row holds; its values are cleared on their way
   // into LDS, since 0 * (not a number) would not be 0.
   auto load_data = [&](int tile0) {
+    int off[KVEC + 1];
+#pragma unroll
+    for (int v = 0; v < KVEC; ++v) off[v] = tile0 + krow0 + v * KROWS;
+    off[KVEC] = tile0 + vkr * 4;
+    if (ps_shift >= 0) {
+#pragma unroll
+      for (int v = 0; v <= KVEC; ++v) off[v] &= page_size - 1;
+    } else {
+#pragma unroll
+      for (int v = 0; v <= KVEC; ++v) off[v] %= page_size;
+    }
 #pragma unroll
     for (int v = 0; v < KVEC; ++v) {
-      const int off = page_offset(tile0 + krow0 + v * KROWS, page_size, ps_shift);
       const unsigned page = kpg[v] < 0 ? 0u : (unsigned)kpg[v];
-      kreg[v] = *reinterpret_cast<const bf16x8_t*>(kbase + ((size_t)page * page_stride + (unsigned)(off * D)));
+      kreg[v] = *reinterpret_cast<const bf16x8_t*>(kbase + ((size_t)page * page_stride + (unsigned)(off[v] * D)));
     }
-    const int off = page_offset(tile0 + vkr * 4, page_size, ps_shift);
     const unsigned page = vpg < 0 ? 0u : (unsigned)vpg;
-    const bf16_t* src = vbase + ((size_t)page * page_stride + (unsigned)off);
+    const bf16_t* src = vbase + ((size_t)page * page_stride + (unsigned)off[KVEC]);
 #pragma unroll
     for (int v = 0; v < VVEC; ++v)
       vreg[v] = *reinterpret_cast<const bf16x4_t*>(src + v * vstep);
@@ -594,19 +625,18 @@ paged_attention_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ o
     for (int v = 0; v < KVEC; ++v)
       *reinterpret_cast<bf16x8_t*>(ks + (krow0 + v * KROWS) * LDK + (tid % VEC_PER_ROW) * 8) =
           kreg[v];
-    const int kp = tile0 + vkr * 4;
-    const bool edge_tile = tile0 < lo || tile0 + KT - 1 > hi;   // the same for all threads
+    if (tile0 < lo || tile0 + KT - 1 > hi) {   // the same for all threads
+      // keys outside [lo, hi] (pages that are not there lie outside it too)
+      const int kp = tile0 + vkr * 4;
 #pragma unroll
-    for (int v = 0; v < VVEC; ++v) {
-      bf16x4_t x = vreg[v];
-      if (edge_tile) {
-        // keys outside [lo, hi] (pages that are not there lie outside it too)
+      for (int v = 0; v < VVEC; ++v)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (kp + e < lo || kp + e > hi) x[e] = (bf16_t)0.f;
-      }
-      *reinterpret_cast<bf16x4_t*>(vt + (vdd0 + v * (NT / VRUNS)) * LDV + vslot) = x;
+          if (kp + e < lo || kp + e > hi) vreg[v][e] = (bf16_t)0.f;
     }
+#pragma unroll
+    for (int v = 0; v < VVEC; ++v)
+      *reinterpret_cast<bf16x4_t*>(vt + (vdd0 + v * (NT / VRUNS)) * LDV + vslot) = vreg[v];
   };
 
   int tile_first = (lo / KT) * KT;
@@ -660,24 +690,20 @@ paged_attention_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ o
               s[c][jb][i] = shaped_score_log2(ex, s[c][jb][i], row_mul[c]);
         }
         if (needs_mask) {
-          // key jb * 16 + grp * 4 + i of the tile counts for this lane's row if it lies in
-          // [first, last]; both bounds are taken relative to the lane's own keys once, so
-          // that an element costs two comparisons with constants
-          int last = pos_row[c] < hi ? pos_row[c] : hi;
+          // key jb * 16 + grp * 4 + i of the tile counts for this lane's row if it is one of
+          // `counted` keys from `first` on, and `first` is taken relative to the lane's own
+          // keys once: a subtraction and one comparison an element, whatever bounds there are
+          const int last = pos_row[c] < hi ? pos_row[c] : hi;
           int first = lo;
           if (window > 0 && pos_row[c] - window + 1 > first) first = pos_row[c] - window + 1;
           if (SHAPED && chunk_lo[c] > first) first = chunk_lo[c];
-          last -= tile0 + grp * 4;
+          const unsigned counted = last >= first ? (unsigned)(last - first) + 1u : 0u;
           first -= tile0 + grp * 4;
-          const bool below = __any(first > 0);   // does any lane have keys before its first?
 #pragma unroll
           for (int jb = 0; jb < JB; ++jb)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              bool valid = jb * 16 + i <= last;
-              if (below) valid = valid && jb * 16 + i >= first;
-              if (!valid) s[c][jb][i] = -INFINITY;
-            }
+            for (int i = 0; i < 4; ++i)
+              if ((unsigned)(jb * 16 + i - first) >= counted) s[c][jb][i] = -INFINITY;
         }
         float tmax = -INFINITY;
 #pragma unroll

@@ -63,6 +63,7 @@ there several times: the rows of the k and v projections are repeated until a gr
 
 from __future__ import annotations
 
+import functools
 import math
 from typing import Any, Dict, Mapping, Optional
 
@@ -107,6 +108,42 @@ def plan_split(n_items: int, num_kv_heads: int, max_keys: int, target: int = SPL
     keys = ((max_keys + nsplit - 1) // nsplit + 63) // 64 * 64   # a multiple of the key tile
     nsplit = (max_keys + keys - 1) // keys
     return (keys, nsplit) if nsplit > 1 else (0, 1)
+
+
+# What a tile of keys takes a workgroup of the kernel for prompt portions (us; 128 keys of heads of 64
+# or 64 keys of heads of 128), alone on its compute unit and with another beside it; and what cutting
+# costs: the launch of the merge, and each MB of 32-bit partial results, written and read again.
+PORTION_TILE_US, PORTION_TILE_SHARED_US = 1.7, 2.4
+PORTION_MERGE_US, PORTION_MB_US = 2.0, 1.0
+
+
+@functools.lru_cache(maxsize=4096)
+def plan_portions(n_items: int, num_kv_heads: int, rows: int, heads: int, head_dim: int, max_keys: int,
+                  window: int = 0):
+    """(keys per range, number of ranges) for a launch of the kernel for prompt portions, which runs two
+    workgroups per compute unit: of the numbers of ranges that stay within 512 workgroups the one
+    whose longest chain of tiles and merge take least by the figures above.  Cutting whatever left
+    compute units idle lost time at portions that bring many rows to a short context.  Measured (us,
+    32 heads on 8 key heads of 64; cut as far as 512 workgroups go, and by this rule):
+      a prompt of 1,024                                34, 20
+      a portion of 512 up to 1,500, 4,096, 8,192       30, 26;  44, 44;  65, 65
+      a portion of 256 up to 2,048                     27, 26
+      5 single tokens at 1,200, a portion of 512       27, 20
+    A function of the batch's shape and of the longest context only."""
+    groups = n_items * num_kv_heads
+    tile = 128 if head_dim == 64 else 64
+    best, plan = None, (0, 1)
+    for n in range(1, max(1, min(BUSY_WORKGROUPS // groups, SPLIT_MAX, max_keys // 256)) + 1):
+        keys = ((max_keys + n - 1) // n + tile - 1) // tile * tile
+        if (max_keys + keys - 1) // keys != n:
+            continue
+        chain = (min(keys, window) if window else keys) / tile
+        us = chain * (PORTION_TILE_US if groups * n <= SPLIT_TARGET else PORTION_TILE_SHARED_US)
+        if n > 1:
+            us += PORTION_MERGE_US + PORTION_MB_US * 4e-6 * rows * heads * head_dim * n
+        if best is None or us < best:
+            best, plan = us, (keys, n) if n > 1 else (0, 1)
+    return plan
 
 
 def planes_target(head_dim: int, value_dim: int, keys: int, mixed: bool, limited: bool) -> int:
@@ -464,7 +501,7 @@ class GroupedQueryAttention(Mixer):
             # prompt portions in the step: both products on the matrix cores
             items = step.attention_items(self.mfma_rows_per_item)
             # a portion far into a long request yields few work items: cut its context
-            keys, nsplit = plan_split(items[3], nkv, step.max_keys, target=BUSY_WORKGROUPS)
+            keys, nsplit = plan_portions(items[3], nkv, step.n_tokens, nh, d, step.max_keys, self.window)
             # tiles of 128 keys spread a tile's fixed work over twice the scores (measured
             # faster from 512 tokens to 32,768); head size 128 keeps tiles of 64 (LDS)
             o = ops.paged_attention_mfma(q, cache.kv, step.block_tables[cache.group],
@@ -519,14 +556,14 @@ class GroupedQueryAttention(Mixer):
         table = step.block_tables[cache.group]
         # (ranges are cut at absolute key positions: behind a window nearly all of them
         # would be empty, so a windowed layer's contexts are never cut)
-        def split(n_items, **kw):
+        def split(n_items):
             # (nor are a chunked layer's, for the same reason)
-            return (0, 1) if self.window or self.chunk \
-                else plan_split(n_items, nkv, step.max_keys, **kw)
+            return (0, 1) if self.window or self.chunk else plan_split(n_items, nkv, step.max_keys)
         if self.mfma and cache.kv is not None and cache.kv.shape[3] % 4 == 0:
             if step.n_tokens > step.n_seqs:
                 items = step.attention_items(self.mfma_rows_per_item)
-                keys, nsplit = split(items[3], target=BUSY_WORKGROUPS)
+                keys, nsplit = (0, 1) if self.window or self.chunk else plan_portions(
+                    items[3], nkv, step.n_tokens, nh, d, step.max_keys)
                 o = ops.paged_attention_mfma(q, cache.kv, table, step.positions, *items,
                                              self.scale, self.window, keys, nsplit,
                                              tile_keys=128 if d == 64 else 64, shape=self.shape)

@@ -871,6 +871,44 @@ def test_qk_norm_rope_kv_write_many_tokens(dtype, nh, nkv, d, rot, pairing, page
     assert (untouched_v == 0).all()
 
 
+@pytest.mark.parametrize("shift", [0, 1, 5, 7, 8])
+@pytest.mark.parametrize("page_size", [8, 12, 64])
+@pytest.mark.parametrize("whole_rows", [False, True])
+def test_values_of_many_tokens_wherever_their_runs_start(shift, page_size, whole_rows):
+    """Runs of eight neighbouring slots may start at any token: behind single ones, after stretches of
+    every length around eight, at slots that are and are not multiples of eight, with tokens that are
+    not stored and descending slots between.  Every value lands at its place, and nothing else."""
+    nh, nkv, d = 4, 2, 64
+    slots, base = [], 0
+    for n, first in [(1, 3)] * shift + [(16, 0), (7, 0), (8, 8), (9, 8), (23, 5), (6, 2), (40, 7), (8, 1), (65, 0)]:
+        slots += range(base + first, base + first + n)
+        base += 120                                     # (a multiple of every page size but 64)
+    slots += [-1, base + 9, base + 8, -1, -1] + list(range(base + 16, base + 23))
+    T, pages = len(slots), (base + 64) // page_size + 1
+    assert T >= 128
+    qkv = rand((T, (nh + 2 * nkv) * d), torch.bfloat16, 40 + shift).to(dev())
+    at = torch.tensor(slots, dtype=torch.int32)
+    pos = torch.arange(T, dtype=torch.int32).to(dev())
+    if whole_rows:
+        per_page = nkv * page_size * d
+        mem = torch.zeros((pages, 2 * per_page), dtype=torch.bfloat16, device=dev())
+        planes = [mem[:, :per_page].unflatten(1, (nkv, page_size, d)), mem[:, per_page:].unflatten(1, (nkv, page_size, d))]
+        ones = torch.ones(nh * d, device=dev())
+        ops().qk_norm_rope_kv_write_wide(qkv, pos, at.to(dev()), ones, ones[:nkv * d], None, *planes, nh, nkv,
+                                         d, d, 0, False, 1e-5, row_norm=(nh * d, nkv * d))
+        cv = mem[:, per_page:].cpu().view(pages, nkv, d, page_size)
+    else:
+        cache = torch.zeros((pages, 2, nkv, page_size, d), dtype=torch.bfloat16, device=dev())
+        ops().qk_norm_rope_kv_write(qkv, pos, at.to(dev()), None, None, None, cache, nh, nkv, d, 0, False, 1e-5)
+        cv = cache[:, 1].cpu().reshape(pages, nkv, d, page_size)
+    want = torch.zeros_like(cv)
+    v = qkv[:, (nh + nkv) * d:].cpu().view(T, nkv, d)
+    for t, slot in enumerate(slots):
+        if slot >= 0:
+            want[slot // page_size, :, :, slot % page_size] = v[t]
+    assert torch.equal(cv, want)
+
+
 def test_rope_position_zero_is_identity_and_norm_is_kept():
     """rope.zig:226-253 holds the rotation to preserving the norm; position 0 rotates
     by nothing."""

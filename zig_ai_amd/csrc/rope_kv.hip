@@ -20,6 +20,39 @@
 
 #define RK_MAX_D 256
 
+// Which of a step's values a wave stores that looks at the eight tokens from t0 on.  Eight
+// tokens whose slots are neighbours from a multiple of eight on (in a page of a size that is
+// one too) are a run, and go to the cache with one access of eight values per head-dim element;
+// a run is stored by the wave in whose window it starts, wherever that is (a portion of a
+// prompt behind a few single tokens starts anywhere: with runs from a multiple of eight tokens
+// on only, all of its values went one by one, 2 bytes a page row apart).  Tokens of no run
+// (a request's edges, single tokens) are stored element by element by their own window's wave.
+// Every lane of the wave calls.
+struct ValueShare {
+  int run, slot;        // the run's first token in the window (-1: none), and its slot
+  unsigned singles;     // bit j: token t0 + j, by itself
+};
+
+__device__ __forceinline__ ValueShare value_share(const int* slots, int t0, int n_tokens, int page_size) {
+  const int lane = threadIdx.x & 63, t = t0 - 7 + lane;    // lanes 7 .. 14: the window
+  const int slot = lane < 22 && t >= 0 && t < n_tokens ? slots[t] : -1;
+  const int next = __shfl_down(slot, 1, 64);
+  const unsigned here = (unsigned)__ballot(slot >= 0);
+  const unsigned goes_on = (unsigned)__ballot(slot >= 0 && next == slot + 1);
+  unsigned starts = (unsigned)__ballot(slot >= 0 && slot % 8 == 0 && page_size % 8 == 0);
+#pragma unroll
+  for (int j = 0; j < 7; ++j) starts &= goes_on >> j;
+  unsigned in_run = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) in_run |= starts << j;
+  const unsigned mine = starts >> 7 & 0xffu;               // (one bit at most)
+  ValueShare share;
+  share.run = mine ? __builtin_ctz(mine) : -1;
+  share.slot = __builtin_amdgcn_readlane(slot, 7 + (mine ? share.run : 0));
+  share.singles = (here & ~in_run) >> 7 & 0xffu;
+  return share;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256)
 qk_norm_rope_kv_write_kernel(const T* __restrict__ qkv, const int* __restrict__ positions,
@@ -116,32 +149,27 @@ qk_norm_rope_kv_write_pow2_kernel(const T* __restrict__ qkv, const int* __restri
   constexpr int LPH = D / 8;   // lanes per head
   __shared__ float cs_tab[D / 2], sn_tab[D / 2];
   if ((int)blockIdx.x < value_blocks) {
-    // ---- values only, for steps of many tokens: a wave takes eight consecutive tokens
-    // and stores, where these lie at eight neighbouring offsets of one page from a
-    // multiple of eight on (a stretch of a prompt), each head-dim element's eight
-    // values with one 16-byte access (32 bytes in 32-bit) instead of eight 2-byte
-    // ones a page row apart.  Other groups (a request's edge, single tokens between
-    // prompts) store element by element.
+    // ---- values only, for steps of many tokens: see ValueShare.  32 heads on 8 of 64 in
+    // bfloat16, us, with runs from a multiple of eight tokens on only and so: 2,048 tokens of a
+    // prompt 10.7 -> 9.5, behind 13 single ones 18.7 -> 11.5; 512 behind 5 14.0 -> 6.8; four
+    // prompts of 300 14.6 -> 7.6; 128 single ones 13.2 -> 12.7.
     const int lane = threadIdx.x & 63;
     const int t0 = ((int)blockIdx.x * 4 + ((int)threadIdx.x >> 6)) * 8;   // a wave's 8 tokens
     if (t0 >= n_tokens) return;
     const int total = nh + 2 * nkv;
-    int slot[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) slot[j] = t0 + j < n_tokens ? slots[t0 + j] : -1;
-    bool side_by_side = page_size % 8 == 0 && slot[0] >= 0 && slot[0] % 8 == 0;
-#pragma unroll
-    for (int j = 1; j < 8; ++j) side_by_side = side_by_side && slot[j] == slot[0] + j;
+    const ValueShare share = value_share(slots, t0, n_tokens, page_size);
     for (int pair = lane; pair < nkv * LPH; pair += 64) {
       const int hv = pair / LPH, e0 = (pair % LPH) * 8;
-      float x[8][8];
+      const T* src = qkv + ((size_t)t0 * total + nh + nkv + hv) * D + e0;
+      auto place = [&](int slot) {
+        return kv_cache + (((size_t)(slot / page_size) * 2 + 1) * nkv + hv) * page_size * D +
+               (size_t)e0 * page_size + slot % page_size;
+      };
+      if (share.run >= 0) {
+        float x[8][8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (t0 + j < n_tokens)
-          load8<T>(qkv + ((size_t)(t0 + j) * total + nh + nkv + hv) * D + e0, x[j]);
-      if (side_by_side) {
-        T* dst = kv_cache + (((size_t)(slot[0] / page_size) * 2 + 1) * nkv + hv) * page_size * D +
-                 (size_t)e0 * page_size + slot[0] % page_size;
+        for (int j = 0; j < 8; ++j) load8<T>(src + (size_t)(share.run + j) * total * D, x[j]);
+        T* dst = place(share.slot);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           float run[8];
@@ -149,16 +177,14 @@ qk_norm_rope_kv_write_pow2_kernel(const T* __restrict__ qkv, const int* __restri
           for (int j = 0; j < 8; ++j) run[j] = x[j][i];
           store8<T>(dst + (size_t)i * page_size, run);
         }
-      } else {
+      }
+      for (unsigned left = share.singles; left; left &= left - 1) {
+        const int j = __builtin_ctz(left);
+        float x[8];
+        load8<T>(src + (size_t)j * total * D, x);
+        T* dst = place(slots[t0 + j]);
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (slot[j] >= 0) {
-            T* dst = kv_cache +
-                     (((size_t)(slot[j] / page_size) * 2 + 1) * nkv + hv) * page_size * D +
-                     (size_t)e0 * page_size + slot[j] % page_size;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) dst[(size_t)i * page_size] = from_f32<T>(x[j][i]);
-          }
+        for (int i = 0; i < 8; ++i) dst[(size_t)i * page_size] = from_f32<T>(x[i]);
       }
     }
     return;
@@ -380,26 +406,20 @@ qk_row_norm_rope_kv_write_kernel(const T* __restrict__ qkv, const int* __restric
   if ((int)blockIdx.x < value_blocks) {
     const int t0 = ((int)blockIdx.x * n_waves + wave) * 8;   // a wave's 8 tokens
     if (t0 >= n_tokens) return;
-    int slot[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) slot[j] = t0 + j < n_tokens ? slots[t0 + j] : -1;
-    bool side_by_side = page_size % 8 == 0 && slot[0] >= 0 && slot[0] % 8 == 0;
-#pragma unroll
-    for (int j = 1; j < 8; ++j) side_by_side = side_by_side && slot[j] == slot[0] + j;
+    const ValueShare share = value_share(slots, t0, n_tokens, page_size);
     constexpr int E = 16 / (int)sizeof(T);             // elements of a 16-byte piece
     typedef T piece_t __attribute__((ext_vector_type(E)));
     typedef T run_t __attribute__((ext_vector_type(8)));
     const int pieces = nkv * dv / E;
     const T* src = qkv + (size_t)t0 * row_stride + (size_t)(nh + nkv) * d;
     for (int piece = lane; piece < pieces; piece += 64) {
-      piece_t x[8];
+      if (share.run >= 0) {
+        piece_t x[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j)      // (a token beyond the last reads the last one again)
-        x[j] = *reinterpret_cast<const piece_t*>(
-            src + (size_t)(min(t0 + j, n_tokens - 1) - t0) * row_stride + piece * E);
-      if (side_by_side) {
-        T* dst = kv_cache + (size_t)(slot[0] / page_size) * page_elems + value_base +
-                 (size_t)piece * E * page_size + slot[0] % page_size;
+        for (int j = 0; j < 8; ++j)
+          x[j] = *reinterpret_cast<const piece_t*>(src + (size_t)(share.run + j) * row_stride + piece * E);
+        T* dst = kv_cache + (size_t)(share.slot / page_size) * page_elems + value_base +
+                 (size_t)piece * E * page_size + share.slot % page_size;
 #pragma unroll
         for (int i = 0; i < E; ++i) {
           run_t run;
@@ -407,17 +427,15 @@ qk_row_norm_rope_kv_write_kernel(const T* __restrict__ qkv, const int* __restric
           for (int j = 0; j < 8; ++j) run[j] = x[j][i];
           *reinterpret_cast<run_t*>(dst + (size_t)i * page_size) = run;
         }
-      } else {
+      }
 #pragma unroll 1
-        for (int j = 0; j < 8 && t0 + j < n_tokens; ++j) {   // (a rare group: tokens one by one)
-          const int place = slots[t0 + j];
-          if (place < 0) continue;
-          const piece_t one = *reinterpret_cast<const piece_t*>(src + (size_t)j * row_stride + piece * E);
-          T* dst = kv_cache + (size_t)(place / page_size) * page_elems + value_base +
-                   (size_t)piece * E * page_size + place % page_size;
+      for (unsigned left = share.singles; left; left &= left - 1) {
+        const int j = __builtin_ctz(left), slot = slots[t0 + j];
+        const piece_t one = *reinterpret_cast<const piece_t*>(src + (size_t)j * row_stride + piece * E);
+        T* dst = kv_cache + (size_t)(slot / page_size) * page_elems + value_base +
+                 (size_t)piece * E * page_size + slot % page_size;
 #pragma unroll
-          for (int i = 0; i < E; ++i) dst[(size_t)i * page_size] = one[i];
-        }
+        for (int i = 0; i < E; ++i) dst[(size_t)i * page_size] = one[i];
       }
     }
     return;

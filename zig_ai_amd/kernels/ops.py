@@ -1046,9 +1046,10 @@ def linear_closing(x, weight: torch.Tensor, accumulate: Optional[torch.Tensor] =
     """``linear`` of a product that the next norm may add up (``partial_ok``) or that may add itself to
     ``accumulate``, with a third way: where the library would add many rows to the stream, ranges of K on
     csrc/gemm_half.hip if ``half_plan`` expects them, and the norm that adds them up, to end sooner."""
-    if accumulate is not None and isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 \
-            and weight.dtype == torch.bfloat16 and x.dim() == 2 and weight.dim() == 2 \
-            and x.shape[0] > LIBRARY_SPLIT_ROWS and library_adds(x.shape[0], weight.shape[0], x.shape[1]):
+    if accumulate is not None and isinstance(x, torch.Tensor) and x.dim() == 2 \
+            and x.shape[0] > LIBRARY_SPLIT_ROWS and x.dtype == torch.bfloat16 \
+            and weight.dtype == torch.bfloat16 and weight.dim() == 2 \
+            and library_adds(x.shape[0], weight.shape[0], x.shape[1]):
         M, K = x.shape
         _need(x, "x", torch.bfloat16)
         _need(weight, "weight", torch.bfloat16, (weight.shape[0], K))
@@ -1232,7 +1233,7 @@ def linear(x, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
             _note("linear", M=M, N=N, K=K, norm_in_product=False, added_to_stream=False,
                   partial_sums=splits, out=out.dtype, kernel="tiles")
             return out
-    if library and splits == 1 and bias is None and out_dtype == torch.bfloat16:
+    if library and splits == 1 and bias is None and out_dtype == torch.bfloat16 and M > TILES_MAX_ROWS:
         out = _half_product(x, weight, *half_plan(M, N, K, False), into=into)
         if out is not None:
             return out

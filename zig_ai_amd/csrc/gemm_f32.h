@@ -180,7 +180,8 @@ __device__ __forceinline__ void f32_tile(int K, AAt a_at, WAt w_at, Store store)
 // Nothing may touch the sums between these statements: another instruction that reads a product's sums has to wait
 // some clocks for them, which the compiler does not see to here.  So a chain's steps stand in a row without a
 // branch (with one, the compiler copies sums where the ways meet: wrong, and half a step's time); what lies
-// beyond K is requested for no lane.
+// beyond K is requested for no lane.  Nor does it see that a chain's first product reads sums that it has just
+// cleared, which takes two wait states: the first statement of a chain begins with them.
 // 64 x 64 takes 1,150 clocks a step of 1,024 of products, 32 x 64 615 of 512.  A row's eight pieces of four elements
 // lie in the order piece ^ (row % 8), so that the sixteen rows that a fragment is read from fall into
 // different banks.
@@ -193,6 +194,7 @@ __device__ __forceinline__ void f32_tile(int K, AAt a_at, WAt w_at, Store store)
   "s_mov_b64 exec, -1\n"
 #define GF_FOUR(n, v) [n##0] "v"(v[0]), [n##1] "v"(v[1]), [n##2] "v"(v[2]), [n##3] "v"(v[3])
 #define GF_WAIT "s_waitcnt lgkmcnt(0)\n"
+#define GF_CLEARED "s_nop 1\n"
 #define GF_ALL12(e) GF_MF(0, 0, e) GF_MF(0, 1, e)
 #define GF_ALL22(e) GF_ALL12(e) GF_MF(1, 0, e) GF_MF(1, 1, e)
 #define GF_START12 GF_MF(0, 0, 0) GF_RD(0, pw, 0) GF_MF(0, 1, 0) GF_RD(1, pw, 2048) GF_RD(2, pa, 0)
@@ -223,17 +225,22 @@ struct F32Requests {      // W's and A's offsets of a lane, where its first piec
   int go;
 };
 
-template <int TM, int TN, bool REQUEST>
+// FIRST: of a chain, whose sums have just been cleared (then without requests)
+template <int TM, int TN, bool REQUEST, bool FIRST>
 __device__ __forceinline__ void f32_phase(f32x4_t (&c)[TM][TN], const f32x4_t (&w)[TN], const f32x4_t (&a)[TM],
                                           f32x4_t (&nw)[TN], f32x4_t (&na)[TM], unsigned pw, unsigned pa,
                                           const F32Requests& q) {
-  static_assert(TN == 2 && (TM == 2 || TM == 1), "one of these");
+  static_assert(TN == 2 && (TM == 2 || TM == 1) && !(REQUEST && FIRST), "one of these");
   if constexpr (TM == 1 && REQUEST)
     asm volatile(GF_START12 GF_WITH12 GF_WAIT : GF_C12, GF_N12 : GF_IN12, GF_Q12 : "memory");
+  else if constexpr (TM == 1 && FIRST)
+    asm volatile(GF_CLEARED GF_START12 GF_ALL12(1) GF_ALL12(2) GF_ALL12(3) GF_WAIT : GF_C12, GF_N12 : GF_IN12 : "memory");
   else if constexpr (TM == 1)
     asm volatile(GF_START12 GF_ALL12(1) GF_ALL12(2) GF_ALL12(3) GF_WAIT : GF_C12, GF_N12 : GF_IN12 : "memory");
   else if constexpr (REQUEST)
     asm volatile(GF_START22 GF_WITH22 GF_WAIT : GF_C22, GF_N22 : GF_IN22, GF_Q22 : "memory");
+  else if constexpr (FIRST)
+    asm volatile(GF_CLEARED GF_START22 GF_ALL22(1) GF_ALL22(2) GF_ALL22(3) GF_WAIT : GF_C22, GF_N22 : GF_IN22 : "memory");
   else
     asm volatile(GF_START22 GF_ALL22(1) GF_ALL22(2) GF_ALL22(3) GF_WAIT : GF_C22, GF_N22 : GF_IN22 : "memory");
 }
@@ -315,13 +322,15 @@ __device__ __forceinline__ void f32_tile_async(int K, const float* A, const floa
     for (int u = 0; u < decltype(count)::value; ++u) {
       const bool last = at == (NS - 1) * PLACE;
       const unsigned to = last ? 0 : at + PLACE;
-      f32_phase<TM, TN, false>(acc, w0, a0, w1, a1, rw + at + half[1], ra + at + half[1], q);
+      const unsigned pw = rw + at + half[1], pa = ra + at + half[1];
+      if (u == 0) f32_phase<TM, TN, false, true>(acc, w0, a0, w1, a1, pw, pa, q);
+      else f32_phase<TM, TN, false, false>(acc, w0, a0, w1, a1, pw, pa, q);
       __builtin_amdgcn_s_waitcnt(ZA_VMCNT((NS - 2) * (LA + LW)));      // (the next step has arrived)
       meet();
       q.go = all_if_negative(-left);
       --left;
       // (the last step's reads find an older step's tiles: not used)
-      f32_phase<TM, TN, true>(acc, w1, a1, w0, a0, rw + to + half[0], ra + to + half[0], q);
+      f32_phase<TM, TN, true, false>(acc, w1, a1, w0, a0, rw + to + half[0], ra + to + half[0], q);
       behind(last);
       at = to;
     }

@@ -226,3 +226,17 @@ def test_ranges_of_prompt_portions(heads, kv_heads, head_dim, max_keys):
             assert items * kv_heads * nsplit <= BUSY_WORKGROUPS
     assert plan_portions(1024, 8, 32768, 32, 64, 32768) == (0, 1)
     assert plan_portions(2, 8, 64, 32, 64, 8192)[1] > 8          # few rows, a long context
+
+
+def test_plans_of_products_within_what_their_kernels_address():
+    """Products of many rows whose operands hold more than 2^31 - 1 elements stay with the library, by either
+    operand; the largest ones below are planned as any other."""
+    from zig_ai_amd.kernels import ops
+    assert ops.half_plan(2048, 128, 65536, True) != (0, 0)
+    for M, N, K in ((3000, 128, 716800), (3072, 64, 1 << 20), (128, 3000, 716800)):
+        assert ops.half_plan(M, N, K, True) == ops.half_plan(M, N, K, False) == (0, 0)
+        assert not ops.wide_takes_gated(M, N, K)
+    most = ops.WIDE_MAX_ELEMENTS // 3000 // 64 * 64
+    for closing in (True, False):
+        assert ops.half_plan(3000, 128, most + 64, closing) == (0, 0)
+    assert ops.half_plan(3000, 128, most, True) != (0, 0)

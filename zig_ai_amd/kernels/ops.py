@@ -1004,7 +1004,7 @@ def library_us(M: int, N: int, K: int, area: float, sides: float, start: float) 
 def half_plan(M: int, N: int, K: int, closing: bool) -> Tuple[int, int]:
     """``(height of a tile, ranges of K)`` for a product of ``M`` rows on csrc/gemm_half.hip, or ``(0, 0)``.
     ``closing``: its ranges are added up by the next norm, and the library would add it to the stream."""
-    if not TILES_MAX_ROWS < M <= HALF_MAX_ROWS or K % 64 or K < HALF_MIN_RANGE or N * K > WIDE_MAX_ELEMENTS:
+    if not TILES_MAX_ROWS < M <= HALF_MAX_ROWS or K % 64 or K < HALF_MIN_RANGE or max(M, N) * K > WIDE_MAX_ELEMENTS:
         return 0, 0
     best = library_us(M, N, K, 0.162, 0.86, 0.55) if closing else library_us(M, N, K, 0.881, 0.343, 4.86)
     plan = 0, 0

@@ -2073,6 +2073,21 @@ def test_products_that_the_estimates_give_to_one_round(M, N, K):
     assert rel_err(o.linear(off, w), want) < BF16_TOL
 
 
+def test_closing_products_refuse_a_stream_of_another_kind():
+    """A stream of another shape, type or layout is refused whichever way the product takes."""
+    o = ops()
+    M, N, K = 1100, 256, 4096
+    x, w = rand((M, K), torch.bfloat16, 5).to(dev()), rand((N, K), torch.bfloat16, 6, K ** -0.5).to(dev())
+    assert o.half_plan(M, N, K, True)[1] > 1
+    for stream in (torch.zeros((M + 1, N)), torch.zeros((M, N + 4)), torch.zeros((M, N), dtype=torch.bfloat16),
+                   torch.zeros((N, M)).t()):
+        for product in (o.linear_closing, lambda a, b, s: o.linear(a, b, partial_ok=True, accumulate=s)):
+            with pytest.raises(o.KernelError, match="accumulate"):
+                product(x, w, stream.to(dev()))
+    with pytest.raises(o.KernelError, match="accumulate"):
+        o.linear_closing(x, w, torch.zeros((M, N)))
+
+
 @pytest.mark.parametrize("E,top,K,columns", [(12, 3, 1024, 2304), (12, 1, 1088, 2311), (70, 7, 512, 640), (70, 2, 576, 1288)])
 def test_grouped_products_whose_experts_end_in_each_height_of_tile(E, top, K, columns):
     """Wide tiles of 256 and 128: an expert's rest of 0, 1, 128, 129, 192, 193 and 255 assignments behind

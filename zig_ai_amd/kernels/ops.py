@@ -1053,6 +1053,7 @@ def linear_closing(x, weight: torch.Tensor, accumulate: Optional[torch.Tensor] =
         M, K = x.shape
         _need(x, "x", torch.bfloat16)
         _need(weight, "weight", torch.bfloat16, (weight.shape[0], K))
+        _need(accumulate, "accumulate", torch.float32, (M, weight.shape[0]))      # (whether it is added to or not)
         out = _half_product(x, weight, *half_plan(M, weight.shape[0], K, True))
         if out is not None:
             return out

@@ -2073,6 +2073,44 @@ def test_products_that_the_estimates_give_to_one_round(M, N, K):
     assert rel_err(o.linear(off, w), want) < BF16_TOL
 
 
+@pytest.mark.parametrize("form", ["swiglu", "gated", "clamped", "table"])
+def test_gated_units_are_worked_out_in_32_bit(form):
+    """A unit's result in bfloat16 is its value in 64 bits, rounded, but for what 32-bit sums leave: a few units of
+    2^-24 beside the half unit of 2^-8 of the rounding, for every gate value, large negative ones among them,
+    whose sigmoid is below the normal range and their result, times a large up value, is not; infinities
+    and NaN as the formula in 64 bits has them."""
+    o = ops()
+    g = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).to(dev())
+    g = g[(g.abs() < 2.0 ** 40) & ((g.abs() > 2.0 ** -40) | (g == 0)) & (g > -88.5)]
+    u = (torch.rand(512, generator=torch.Generator().manual_seed(1)) + 1.0).bfloat16().to(dev()) * 2.0 ** 60
+    u[::2] *= -1
+
+    def unit(g, u):
+        if form == "table":
+            table = u.view(1, -1).contiguous()
+            rows = g.view(-1, 1).expand(-1, u.numel()).contiguous()
+            return o.table_gate(rows, torch.zeros(len(g), dtype=torch.int32, device=dev()), table, 0, "silu")
+        both = torch.cat([g.view(-1, 1).expand(-1, u.numel()), u.view(1, -1).expand(g.numel(), -1)], 1).contiguous()
+        return {"swiglu": o.swiglu, "gated": lambda x: o.gated_unit(x, "silu"),
+                "clamped": lambda x: o.clamped_glu(x, 0.0, 1.0, 0.0)}[form](both)
+
+    for first in range(0, len(g), 8192):
+        v = g[first:first + 8192]
+        got = unit(v, u).double()
+        want = v.double().view(-1, 1) / (1 + torch.exp(-v.double().view(-1, 1))) * u.double()
+        half = torch.exp2(torch.floor(torch.log2(want.abs().clamp_min(1e-30))) - 8)
+        # exponential, sum, reciprocal and two products round to 2^-24 each, and the exponential's own error is a
+        # unit: 4e-7; a sigmoid below 2^-126 is a multiple of 2^-149, at -88.5 of 2^-128 2^-21 of itself
+        bound = torch.where(v.view(-1, 1) < -87.0, 1e-6, 4e-7)
+        over = ((got - want).abs() - half) / want.abs().clamp_min(1e-30) - bound
+        assert float(over.max()) <= 0, (float(over.max()), float(v[int(over.max(1).values.argmax())]))
+    ends = torch.tensor([float("inf"), -float("inf"), float("nan"), -1000.0, -120.0, 3e38]).bfloat16().to(dev())
+    ones = torch.ones(8, dtype=torch.bfloat16, device=dev())
+    got = unit(ends, ones).float().cpu()
+    assert bool(got[0].isinf().all()) and bool(got[1:3].isnan().all()) and bool((got[3:5] == 0).all())
+    assert torch.equal(got[5], ends[5].float().cpu().expand(8))
+
+
 def test_closing_products_refuse_a_stream_of_another_kind():
     """A stream of another shape, type or layout is refused whichever way the product takes."""
     o = ops()

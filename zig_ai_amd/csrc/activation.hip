@@ -3,7 +3,7 @@
 // computed in 32-bit (/root/reference/src/transformer/ffn.zig:24-30,
 // /root/reference/src/cuda/layer_kernels.cu:62-70).
 // Also the element-wise cast between storage types.
-// (gate_unit.h: for bfloat16 the unit in the hardware's exponential, as the products that apply it themselves)
+// (gate_unit.h: the units as the wide and grouped products that apply them themselves have them)
 #include "common.h"
 #include "gate_unit.h"
 

@@ -569,12 +569,13 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     // -> 182 | 107; at 517 tokens (65 rows an expert) 73 | 36 against 84 | 38.  8 experts of 4,096, 2 a
     // token, 1,900 tokens: up 99 -> 64 (128 high 85), down, 128 high for want of tiles, 92 -> 75 (256
     // high 95); 500 tokens: up, 128 high, 56 -> 43, down stays (54 against 66).  The sums are the same
-    // to the last bit.  With four waves of 128 x 128 in place of eight of 128 x 64, the unit in
-    // the hardware's exponential and bfloat16 stored in whole lines, before and after (us): 32 experts, gated,
-    // 1,777 tokens 90 and 79, unevenly taken 105 and 92, 4,096 tokens unevenly 186 and 154; 8 experts of 4,096,
-    // gated, 1,777 tokens 168 and 123; their down product at 4,096 tokens 153 and 145.  32-bit results of few
-    // steps of K are bound by the 58 MB and more that they write: 2,048 x 1,024, 1,777 tokens unevenly 58 to 64
-    // and 58 to 62, 4,096 tokens 103 and 106.
+    // to the last bit.  With four waves of 128 x 128 in place of eight of 128 x 64, the unit of
+    // gate_unit.h and bfloat16 stored in whole lines, before and after (us): 32 experts, gated, 1,777 tokens 93
+    // and 87, unevenly taken 105 and 95, 4,096 tokens 169 and 158, unevenly 163 and 149; 8 experts of 4,096,
+    // gated, 1,777 tokens 173 and 159; their down product at 4,096 tokens 153 and 145.  32-bit results of few
+    // steps of K are bound by the 58 MB and more that they write: 2,048 x 1,024, 1,777 tokens unevenly 58 and
+    // 57, 1,024 tokens 38.4 and 39.3, unevenly 36.3 and 36.2, 1,277 45 and 42, 4,096 104 and 104; 64 experts of 2,048 x
+    // 1,408, 6 a token, 1,093 tokens 96.4 and 95.5, unevenly 77.1 and 77.4.  Low tiles take longer at all of these.
     // And only where the rounds that the tiles make, 256 of them at a time or 512 of the low ones, take no
     // longer (few steps of K, outputs that fill little of a wide tile, a wide round that is nearly empty
     // where the low tiles make whole ones): a round of 128 x 128, two to a compute unit, as K, of 128 x 256 as

@@ -7,8 +7,8 @@
 // write and read them).  Full tiles of 256 rows and, at the end, one as low as holds what is left, 128, 192
 // or 256: 1,037 rows make 4.5 rows of tiles.  Which products take it is the caller's rule.
 // Measured (us; weights from memory, the library's product and the unit's kernel in brackets): 2 x 8192 x 2048
-// at 2,048 rows 102 (119), 1.35 PFLOP/s; 2 x 7168 x 2048 at 1,037 56 (73), at 917 47 (57); 2 x 4608 x 1024 at
-// 1,777 30 (41).  Without a unit the same tiles gain nothing: 6144 x 2048 at 2,048 rows 44 (42).
+// at 2,048 rows 110 (123), 1.25 PFLOP/s; 2 x 7168 x 2048 at 1,037 61 (77), at 917 51 (59); 2 x 4608 x 1024 at
+// 1,777 34 (42).  Without a unit the same tiles gain nothing: 6144 x 2048 at 2,048 rows 44 (42).
 #include <type_traits>
 
 #include "gate_unit.h"

@@ -912,9 +912,10 @@ def linear_gated_tiles(x: torch.Tensor, gate_up_weight: torch.Tensor,
 # time, a step of 64 elements of K 1.1 us of a round, end before the library's product and the unit's kernel
 # after it would, 1.28 PFLOP/s and 12 us together.  Measured (us; weights from memory, the library's
 # product with the unit's kernel and this one): 2 x 8192 x 2048 at 400, 600, 1,037, 1,300, 2,048 and 4,096
-# rows 37, 46, 79, 91, 119, 226 and 40, 43, 70, 86, 102, 200; 2 x 7168 x 2048 at 600, 1,037, 1,300, 2,048
-# rows 42, 73, 84, 107 and 39, 56, 85, 93; 2 x 4608 x 1024 at 512, 700, 1,037, 1,777, 4,096 rows 22, 24, 30,
-# 41, 95 and 23, 24, 25, 30, 77; 2 x 1024 x 2048 at 2,048 and 4,096 rows 25, 38 and 37, 40.
+# rows 39, 47, 85, 96, 123, 235 and 46, 48, 78, 97, 110, 215; 2 x 7168 x 2048 at 600, 1,037, 1,300, 2,048
+# rows 43, 77, 85, 111 and 44, 61, 95, 103; 2 x 4608 x 1024 at 512, 700, 1,037, 1,777, 4,096 rows 22, 24, 30,
+# 42, 95 and 27, 28, 29, 34, 90; 2 x 1024 x 2048 at 2,048 and 4,096 rows 25, 39 and 41, 45.  Over 171 products of
+# 100 to 5,000 rows the choice is 0.9 percent from the better of the two on average.
 WIDE_ROUND_US = 4.0
 WIDE_STEP_US = 1.1
 WIDE_LIBRARY_US = 12.0

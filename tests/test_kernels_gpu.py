@@ -155,6 +155,22 @@ def test_gemm_f32_steps_through_lds(M, N, K):
     assert torch.equal(ops().linear(x, w, bias), whole + bias)
 
 
+@pytest.mark.parametrize("M,N,K", [(40, (1 << 20) + 70, 1056), (33, 262144 + 5, 4096)])
+def test_gemm_f32_of_more_than_4_gigabytes(M, N, K):
+    """Weights of more than 2^30 elements: the outputs at their end, and at both sides of 4 GB, have the
+    bits of those weight rows by themselves."""
+    assert N * K > 1 << 30
+    g = torch.Generator(device=dev()).manual_seed(66)
+    x, w = torch.randn((M, K), device=dev(), generator=g), torch.randn((N, K), device=dev(), generator=g)
+    whole = ops().linear(x, w)
+    middle = (1 << 30) // K
+    for first in (0, middle - 2100, N - 4100):
+        part = w[first:first + 4100]
+        got = whole[:, first:first + 4100]
+        assert torch.equal(got, ops().linear(x, part)), first
+        assert rel_err(got, x.double() @ part.double().T) < 1e-6      # (as above)
+
+
 def test_gemm_f32_weight_with_bf16_activations():
     """A weight stored in 32-bit stays 32-bit in a bfloat16 run."""
     x, w = rand((9, 40), torch.bfloat16, 11), rand((23, 40), torch.float32, 12)

@@ -360,9 +360,10 @@ gemm_f32_async_kernel(const float* __restrict__ A, const float* __restrict__ W, 
   const int n_tile = (at / m_tiles) * 8 + (blockIdx.x & 7);
   if (n_tile >= n_tiles) return;
   const int m0 = (at % m_tiles) * BM, n0 = n_tile * BN;
+  // (offsets from the tile's own first rows: operands may hold more than 4 GB)
   f32_tile_async<BM, BN, NS>(
-      K, A, W, [&](int r) { return (unsigned)min(m0 + r, M - 1) * (unsigned)(K * 4); },
-      [&](int r) { return (unsigned)min(n0 + r, N - 1) * (unsigned)(K * 4); },
+      K, A + (size_t)m0 * K, W + (size_t)n0 * K, [&](int r) { return (unsigned)min(r, M - 1 - m0) * (unsigned)(K * 4); },
+      [&](int r) { return (unsigned)min(r, N - 1 - n0) * (unsigned)(K * 4); },
       [&](int r, int n, const f32x4_t(&v)[BN / 32]) {
         if (m0 + r >= M) return;
 #pragma unroll

@@ -63,8 +63,8 @@ static int launch_f32(const TA* A, const float* W, const float* bias, TC* C, int
     // 65 (130 TFLOP/s), 350 x 9216 x 1024 84 and 61, 448 x 3072 x 1024 39 and 28, 448 x 2048 x 1024 26 and
     // 20, 448 x 1024 x 1024 15 and 11.5, 448 x 1024 x 4608 54 and 42.
     // 64 x 64 where the compute units take a tile half as often (0.93 of two of 32 x 64: 448 x 9216 65 and 68,
-    // 448 x 3072 34 and 28).
-    if (K % F32_BK == 0 && n32 > 256 && (long long)M * K < (1LL << 30) && (long long)N * K < (1LL << 30)) {
+    // 448 x 3072 34 and 28).  A tile's rows are reached by 32-bit offsets in bytes: 64 K x 4 of them.
+    if (K % F32_BK == 0 && n32 > 256 && K < (1 << 24)) {
       if (((n64 + 255) / 256) * 186 <= ((n3264 + 255) / 256) * 100) ZA_F32_ASYNC(64, 64, 4)
       ZA_F32_ASYNC(32, 64, 4)
     }

@@ -128,3 +128,15 @@ def test_the_reading_of_listings():
     assert of(product, "s_nop 8", "v_add_f32_e32 v9, v9, v4") and not of(product, "s_nop 9", "v_add_f32_e32 v9, v9, v4")
     assert of(product, "s_nop 3", "ds_write_b128 v9, v[4:7]")
     assert not of(product, "v_mfma_f32_16x16x4_f32 v[4:7], v2, v3, v[4:7]", "s_endpgm", "v_mov_b32_e32 v8, v4")
+
+
+@pytest.mark.skipif(OBJDUMP is None or build.find_hipcc() is None, reason="the compiler's tools are not here")
+@pytest.mark.parametrize("name", ["gemm_f32", "gemm_half", "gemm_wide", "experts"])
+def test_requests_are_made_for_all_lanes(name, tmp_path):
+    """A wait that lets so many requests stay under way counts requests: none is made under a mask of no lanes,
+    of which it is not said whether it counts."""
+    code = re.findall(r"^\t(.*?)\s*//", listing_of(name, str(tmp_path)), re.M)
+    requests = [i for i, op in enumerate(code) if op.startswith("global_load_lds")]
+    assert requests
+    for i in requests:
+        assert not any("exec" in op.split(",")[0] for op in code[i - 2:i]), code[i - 3:i + 1]

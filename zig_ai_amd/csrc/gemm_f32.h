@@ -179,8 +179,9 @@ __device__ __forceinline__ void f32_tile(int K, AAt a_at, WAt w_at, Store store)
 // arrived.
 // Nothing may touch the sums between these statements: another instruction that reads a product's sums has to wait
 // some clocks for them, which the compiler does not see to here.  So a chain's steps stand in a row without a
-// branch (with one, the compiler copies sums where the ways meet: wrong, and half a step's time); what lies
-// beyond K is requested for no lane.  Nor does it see that a chain's first product reads sums that it has just
+// branch (with one, the compiler copies sums where the ways meet: wrong, and half a step's time), and the last
+// whole chain is there once for each number of steps behind it: how many steps are still to be requested and
+// are under way at each wait is known where the code is written.  Nor does it see that a chain's first product reads sums that it has just
 // cleared, which takes two wait states: the first statement of a chain begins with them.
 // 64 x 64 takes 1,150 clocks a step of 1,024 of products, 32 x 64 615 of 512.  A row's eight pieces of four elements
 // lie in the order piece ^ (row % 8), so that the sixteen rows that a fragment is read from fall into
@@ -189,9 +190,7 @@ __device__ __forceinline__ void f32_tile(int K, AAt a_at, WAt w_at, Store store)
 #define GF_RD(k, p, o) "ds_read_b128 %[n" #k "], %[" #p "] offset:" #o "\n"
 // (m0 is set one instruction ahead of the request, which needs that distance; nothing else here keeps a value in it)
 #define GF_TO(k) "s_mov_b32 m0, %[m" #k "]\n"
-#define GF_RQ(k, b)                                                                                     \
-  "s_mov_b32 exec_lo, %[go]\n" "s_mov_b32 exec_hi, %[go]\n" "global_load_lds_dwordx4 %[v" #k "], %[" #b "]\n" \
-  "s_mov_b64 exec, -1\n"
+#define GF_RQ(k, b) "global_load_lds_dwordx4 %[v" #k "], %[" #b "]\n"
 #define GF_FOUR(n, v) [n##0] "v"(v[0]), [n##1] "v"(v[1]), [n##2] "v"(v[2]), [n##3] "v"(v[3])
 #define GF_WAIT "s_waitcnt lgkmcnt(0)\n"
 #define GF_CLEARED "s_nop 1\n"
@@ -215,14 +214,13 @@ __device__ __forceinline__ void f32_tile(int K, AAt a_at, WAt w_at, Store store)
 #define GF_IN22 GF_IN12, GF_FOUR(a1, a[1])
 #define GF_Q12                                                                                              \
   [v0] "v"(q.offw[0]), [m0] "s"(q.tow), [v1] "v"(q.offw[1]), [m1] "s"(q.tow + 4096), [v2] "v"(q.offa[0]),         \
-  [m2] "s"(q.toa), [bw] "s"(q.w), [ba] "s"(q.a), [go] "s"(q.go)
+  [m2] "s"(q.toa), [bw] "s"(q.w), [ba] "s"(q.a)
 #define GF_Q22 GF_Q12, [v3] "v"(q.offa[1]), [m3] "s"(q.toa + 4096)
 
-struct F32Requests {      // W's and A's offsets of a lane, where its first piece goes, W's and A's base, all lanes or none
+struct F32Requests {      // W's and A's offsets of a lane, where its first piece goes, W's and A's base
   const unsigned *offw, *offa;
   unsigned tow, toa;
   const char *w, *a;
-  int go;
 };
 
 // FIRST: of a chain, whose sums have just been cleared (then without requests)
@@ -262,12 +260,7 @@ __device__ __forceinline__ void f32_tile_async(int K, const float* A, const floa
   for (int i = 0; i < LW; ++i) offw[i] = w_at(lrow + 32 * i) + piece;
   const int steps = K / F32_BK;
   const unsigned base = lds_address(lds);
-  F32Requests q{offw, offa, base + wave * 1024, base + BN * F32_BK * 4 + wave * 1024, (const char*)W, (const char*)A, 0};
-  auto all_if_negative = [](int n) {      // (in a scalar register, whatever the compiler prefers)
-    int v = n >> 31;
-    asm volatile("" : "+v"(v));
-    return __builtin_amdgcn_readfirstlane(v);
-  };
+  F32Requests q{offw, offa, base + wave * 1024, base + BN * F32_BK * 4 + wave * 1024, (const char*)W, (const char*)A};
   auto behind = [&](bool last) {      // a step's requests, which went to the last place
     const unsigned by = last ? (unsigned)(-(NS - 1) * PLACE) : (unsigned)PLACE;
     q.w += F32_BK * 4;
@@ -277,10 +270,10 @@ __device__ __forceinline__ void f32_tile_async(int K, const float* A, const floa
   };
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const int go = all_if_negative(s - steps);
+    if (s >= steps) continue;
     auto request = [&](const char* from, unsigned offset, unsigned to) {
-      asm volatile("s_mov_b32 m0, %0\n" "s_mov_b32 exec_lo, %3\n" "s_mov_b32 exec_hi, %3\n" "global_load_lds_dwordx4 %1, %2\n"
-                   "s_mov_b64 exec, -1\n" :: "s"(to), "v"(offset), "s"(from), "s"(go) : "memory");
+      asm volatile("s_mov_b32 m0, %0\n" "s_nop 0\n" "global_load_lds_dwordx4 %1, %2\n"
+                   :: "s"(to), "v"(offset), "s"(from) : "memory");
     };
 #pragma unroll
     for (int i = 0; i < LW; ++i) request(q.w, offw[i], q.tow + i * 4096);
@@ -301,7 +294,8 @@ __device__ __forceinline__ void f32_tile_async(int K, const float* A, const floa
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
-  __builtin_amdgcn_s_waitcnt(ZA_VMCNT((NS - 1) * (LA + LW)));
+  if (steps >= NS) __builtin_amdgcn_s_waitcnt(ZA_VMCNT((NS - 1) * (LA + LW)));
+  else __builtin_amdgcn_s_waitcnt(ZA_VMCNT(0));
   meet();
   f32x4_t a0[TM], w0[TN], a1[TM], w1[TN];
 #pragma unroll
@@ -311,26 +305,30 @@ __device__ __forceinline__ void f32_tile_async(int K, const float* A, const floa
   for (int i = 0; i < TM; ++i)
     asm volatile("ds_read_b128 %0, %1\n" "s_waitcnt lgkmcnt(0)" : "=&v"(a0[i]) : "v"(ra + half[0] + i * 2048) : "memory");
   unsigned at = 0;
-  int left = steps - NS;      // steps that are still to be requested
-  auto chain = [&](auto count) {
+  auto chain = [&](auto count, auto behind_it) {      // its steps, and how many (or NS, if more) are behind them
+    constexpr int COUNT = decltype(count)::value, BEHIND = decltype(behind_it)::value;
     f32x4_t acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < decltype(count)::value; ++u) {
+    for (int u = 0; u < COUNT; ++u) {
+      const int follow = COUNT - 1 - u + BEHIND;
       const bool last = at == (NS - 1) * PLACE;
       const unsigned to = last ? 0 : at + PLACE;
       const unsigned pw = rw + at + half[1], pa = ra + at + half[1];
       if (u == 0) f32_phase<TM, TN, false, true>(acc, w0, a0, w1, a1, pw, pa, q);
       else f32_phase<TM, TN, false, false>(acc, w0, a0, w1, a1, pw, pa, q);
-      __builtin_amdgcn_s_waitcnt(ZA_VMCNT((NS - 2) * (LA + LW)));      // (the next step has arrived)
+      // (the next step has arrived: of what follows it the NS - 2 steps are under way that are left)
+      if (follow >= NS - 1) __builtin_amdgcn_s_waitcnt(ZA_VMCNT((NS - 2) * (LA + LW)));
+      else if (follow == NS - 2) __builtin_amdgcn_s_waitcnt(ZA_VMCNT((NS - 3) * (LA + LW)));
+      else __builtin_amdgcn_s_waitcnt(ZA_VMCNT(0));
       meet();
-      q.go = all_if_negative(-left);
-      --left;
       // (the last step's reads find an older step's tiles: not used)
-      f32_phase<TM, TN, true, false>(acc, w1, a1, w0, a0, rw + to + half[0], ra + to + half[0], q);
+      const unsigned qw = rw + to + half[0], qa = ra + to + half[0];
+      if (follow >= NS) f32_phase<TM, TN, true, false>(acc, w1, a1, w0, a0, qw, qa, q);
+      else f32_phase<TM, TN, false, false>(acc, w1, a1, w0, a0, qw, qa, q);
       behind(last);
       at = to;
     }
@@ -343,11 +341,26 @@ __device__ __forceinline__ void f32_tile_async(int K, const float* A, const floa
         total[i][j] += acc[i][j];
       }
   };
-  for (int c = steps / STEPS; c > 0; --c) chain(std::integral_constant<int, STEPS>{});
-  const int rest = steps % STEPS;
-  if (rest == 1) chain(std::integral_constant<int, 1>{});
-  else if (rest == 2) chain(std::integral_constant<int, 2>{});
-  else if (rest == 3) chain(std::integral_constant<int, 3>{});
+  static_assert(NS == 4 && STEPS == 4, "see the waits, and the ends");
+  constexpr std::integral_constant<int, 0> none;
+  constexpr std::integral_constant<int, 1> one;
+  constexpr std::integral_constant<int, 2> two;
+  constexpr std::integral_constant<int, 3> three;
+  constexpr std::integral_constant<int, 4> four;
+  const int whole = steps / STEPS, rest = steps % STEPS;
+  for (int c = 1; c < whole; ++c) chain(four, four);
+  if (rest == 0) {
+    chain(four, none);
+  } else if (rest == 1) {
+    if (whole > 0) chain(four, one);
+    chain(one, none);
+  } else if (rest == 2) {
+    if (whole > 0) chain(four, two);
+    chain(two, none);
+  } else {
+    if (whole > 0) chain(four, three);
+    chain(three, none);
+  }
 #pragma unroll
   for (int i = 0; i < TM; ++i) store(wm + i * 16 + frow, wn + fk * 4, total[i]);
 }

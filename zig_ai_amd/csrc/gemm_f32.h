@@ -188,7 +188,7 @@ __device__ __forceinline__ void f32_tile(int K, AAt a_at, WAt w_at, Store store)
 // different banks.
 #define GF_MF(i, j, e) "v_mfma_f32_16x16x4_f32 %[c" #i #j "], %[w" #j #e "], %[a" #i #e "], %[c" #i #j "]\n"
 #define GF_RD(k, p, o) "ds_read_b128 %[n" #k "], %[" #p "] offset:" #o "\n"
-// (m0 is set one instruction ahead of the request, which needs that distance; nothing else here keeps a value in it)
+// (m0 is set one instruction ahead of the request, which needs that distance)
 #define GF_TO(k) "s_mov_b32 m0, %[m" #k "]\n"
 #define GF_RQ(k, b) "global_load_lds_dwordx4 %[v" #k "], %[" #b "]\n"
 #define GF_FOUR(n, v) [n##0] "v"(v[0]), [n##1] "v"(v[1]), [n##2] "v"(v[2]), [n##3] "v"(v[3])
@@ -230,13 +230,13 @@ __device__ __forceinline__ void f32_phase(f32x4_t (&c)[TM][TN], const f32x4_t (&
                                           const F32Requests& q) {
   static_assert(TN == 2 && (TM == 2 || TM == 1) && !(REQUEST && FIRST), "one of these");
   if constexpr (TM == 1 && REQUEST)
-    asm volatile(GF_START12 GF_WITH12 GF_WAIT : GF_C12, GF_N12 : GF_IN12, GF_Q12 : "memory");
+    asm volatile(GF_START12 GF_WITH12 GF_WAIT : GF_C12, GF_N12 : GF_IN12, GF_Q12 : "memory", "m0");
   else if constexpr (TM == 1 && FIRST)
     asm volatile(GF_CLEARED GF_START12 GF_ALL12(1) GF_ALL12(2) GF_ALL12(3) GF_WAIT : GF_C12, GF_N12 : GF_IN12 : "memory");
   else if constexpr (TM == 1)
     asm volatile(GF_START12 GF_ALL12(1) GF_ALL12(2) GF_ALL12(3) GF_WAIT : GF_C12, GF_N12 : GF_IN12 : "memory");
   else if constexpr (REQUEST)
-    asm volatile(GF_START22 GF_WITH22 GF_WAIT : GF_C22, GF_N22 : GF_IN22, GF_Q22 : "memory");
+    asm volatile(GF_START22 GF_WITH22 GF_WAIT : GF_C22, GF_N22 : GF_IN22, GF_Q22 : "memory", "m0");
   else if constexpr (FIRST)
     asm volatile(GF_CLEARED GF_START22 GF_ALL22(1) GF_ALL22(2) GF_ALL22(3) GF_WAIT : GF_C22, GF_N22 : GF_IN22 : "memory");
   else
@@ -273,7 +273,7 @@ __device__ __forceinline__ void f32_tile_async(int K, const float* A, const floa
     if (s >= steps) continue;
     auto request = [&](const char* from, unsigned offset, unsigned to) {
       asm volatile("s_mov_b32 m0, %0\n" "s_nop 0\n" "global_load_lds_dwordx4 %1, %2\n"
-                   :: "s"(to), "v"(offset), "s"(from) : "memory");
+                   :: "s"(to), "v"(offset), "s"(from) : "memory", "m0");
     };
 #pragma unroll
     for (int i = 0; i < LW; ++i) request(q.w, offw[i], q.tow + i * 4096);

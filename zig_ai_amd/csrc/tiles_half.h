@@ -29,7 +29,7 @@
 #define GH_IN3 GH_W, [a0] "v"(a[0]), [a1] "v"(a[1]), [a2] "v"(a[2])
 #define GH_IN4 GH_IN3, [a3] "v"(a[3])
 #define GH_BLOCK(TEXT, R, READS, ...) \
-  asm volatile(TEXT GH_WAIT : GH_SUMS##R, READS : GH_IN##R, __VA_ARGS__ : "memory")
+  asm volatile(TEXT GH_WAIT : GH_SUMS##R, READS : GH_IN##R, __VA_ARGS__ : "memory", "m0")
 #define GH_RQ2 GW_REQUEST(0), GW_REQUEST(1), [from] "s"(from)
 #define GH_RQ3 GW_REQUEST(0), GW_REQUEST(1), GW_REQUEST(2), [from] "s"(from)
 #define GH_RQ4 GW_REQUEST(0), GW_REQUEST(1), GW_REQUEST(2), GW_REQUEST(3), [from] "s"(from)
@@ -117,7 +117,7 @@ struct TilesHalf {
     const unsigned base = lds_address(lds), own = wave * 1024;
     auto request = [&](const char* from, unsigned offset, unsigned to) {
       asm volatile("s_mov_b32 m0, %0\n" "s_nop 0\n" "global_load_lds_dwordx4 %1, %2\n"
-                   :: "s"(to), "v"(offset), "s"(from) : "memory");
+                   :: "s"(to), "v"(offset), "s"(from) : "memory", "m0");
     };
 #pragma unroll
     for (int s = 0; s < NS; ++s)

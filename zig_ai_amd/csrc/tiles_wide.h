@@ -35,7 +35,7 @@
 #define GW_MF0(j) "v_mfma_f32_16x16x32_bf16 %[c" #j "], %[w" #j "], %[a0], %[c" #j "]\n"
 #define GW_MF1(j) "v_mfma_f32_16x16x32_bf16 %[d" #j "], %[w" #j "], %[a1], %[d" #j "]\n"
 #define GW_RD(k) "ds_read_b128 %[n" #k "], %[p" #k "] offset:%[o" #k "]\n"
-// (one instruction ahead of the request, which needs that distance; nothing else here keeps a value in m0)
+// (one instruction ahead of the request, which needs that distance)
 #define GW_TO(k) "s_mov_b32 m0, %[m" #k "]\n"
 #define GW_RQ(k) "global_load_lds_dwordx4 %[v" #k "], %[from]\n"
 // what stands behind the first to the fifteenth product
@@ -71,7 +71,7 @@
 #define GW_REQUEST4 , GW_REQUEST(0), GW_REQUEST(1), GW_REQUEST(2), GW_REQUEST(3), [from] "s"(from)
 #define GW_BLOCK(R, READS, REQUESTS, INPUTS)                                                          \
   asm volatile(GW_CALL(GW_TEXT, READS, REQUESTS) : GW_SUMS, GW_OUT##R : GW_OPERANDS, GW_PLACED##R INPUTS \
-               : "memory")
+               : "memory", "m0")
 
 template <int TM>      // a wave's rows of A in sixteens; the tile has 32 TM
 struct TilesWide {
@@ -140,7 +140,7 @@ struct TilesWide {
     const unsigned As = lds_address(lds), Ws = As + 2 * GW_PLACE, own = wave * 1024;
     auto request = [&](const char* from, unsigned offset, unsigned to) {
       asm volatile("s_mov_b32 m0, %0\n" "s_nop 0\n" "global_load_lds_dwordx4 %1, %2\n"
-                   :: "s"(to), "v"(offset), "s"(from) : "memory");
+                   :: "s"(to), "v"(offset), "s"(from) : "memory", "m0");
     };
     auto request_step = [&](int s) {
 #pragma unroll

@@ -176,12 +176,12 @@ __device__ __forceinline__ float expert_act(float v, int act) {
 
 // The gated unit (gate > 0) of one assignment's sums `v` (gate) and `u` (up).
 template <typename TO, int KIND>
-__device__ __forceinline__ float expert_unit(const GroupedArgs& g, float v, float u, float w) {
+__device__ __forceinline__ float expert_unit(const GroupedArgs& g, bool rounded, float v, float u, float w) {
   constexpr bool EXACT = sizeof(TO) == 4;
   if constexpr (!EXACT) {
     const float rv = to_f32<TO>(from_f32<TO>(v)), ru = to_f32<TO>(from_f32<TO>(u));
-    v = g.rounded ? rv : v;
-    u = g.rounded ? ru : u;
+    v = rounded ? rv : v;
+    u = rounded ? ru : u;
   }
   return gated_value<KIND, EXACT>(v * w, u * w, g.bound, g.slope, g.offset);
 }
@@ -237,7 +237,7 @@ __device__ __forceinline__ void grouped_store(const GroupedArgs& g, const int* _
           f32x4_t v;
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            v[r] = expert_unit<TO, decltype(kind)::value>(g, acc[i][j][r], acc[i][j + 1][r], w);
+            v[r] = expert_unit<TO, decltype(kind)::value>(g, g.rounded, acc[i][j][r], acc[i][j + 1][r], w);
           put(to, n0 + (wn >> 1) + (j / 2) * 16 + kq * 4, v);
         }
       });
@@ -360,7 +360,8 @@ __device__ __forceinline__ void wide_find(const int* __restrict__ counts, int E,
 
 // Tiles of 256 or 128 x 256 (tiles_wide.h); HIGH as above.  UNIT: 0 without, else GATED as above with the
 // unit's kind as a constant, 4: any (for 32-bit results; the three kinds' stores side by side cost registers).
-template <typename TO, int UNIT, int HIGH>
+// ROUNDED: as g.rounded says (a choice an element takes six instructions).
+template <typename TO, int UNIT, int HIGH, bool ROUNDED>
 __global__ void __launch_bounds__(256, 1)
 grouped_gemm_bf16_wide_kernel(GroupedArgs g) {
   constexpr bool GATED = UNIT > 0;
@@ -438,12 +439,12 @@ grouped_gemm_bf16_wide_kernel(GroupedArgs g) {
     if constexpr (UNIT == 4)
       with_unit(g, [&](auto kind) {
         put([&](int i, int j, int r) {
-          return expert_unit<TO, decltype(kind)::value>(g, acc[i][2 * j][r], acc[i][2 * j + 1][r], weight[i]);
+          return expert_unit<TO, decltype(kind)::value>(g, false, acc[i][2 * j][r], acc[i][2 * j + 1][r], weight[i]);
         });
       });
     else if constexpr (GATED)
       put([&](int i, int j, int r) {
-        return expert_unit<TO, UNIT>(g, acc[i][2 * j][r], acc[i][2 * j + 1][r], weight[i]);
+        return expert_unit<TO, UNIT>(g, ROUNDED, acc[i][2 * j][r], acc[i][2 * j + 1][r], weight[i]);
       });
     else
       put([&](int i, int j, int r) { return expert_act(acc[i][j][r], g.act) * g.out_scale * weight[i]; });
@@ -498,7 +499,7 @@ grouped_gemm_f32_kernel(GroupedArgs g) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (first + i < N) with_unit(g, [&](auto kind) {
-          at[first + i] = from_f32<TO>(expert_unit<TO, decltype(kind)::value>(g, v[0][i], v[1][i], w));
+          at[first + i] = from_f32<TO>(expert_unit<TO, decltype(kind)::value>(g, g.rounded, v[0][i], v[1][i], w));
         });
     } else {
 #pragma unroll
@@ -571,8 +572,8 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     // high 95); 500 tokens: up, 128 high, 56 -> 43, down stays (54 against 66).  The sums are the same
     // to the last bit.  With four waves of 128 x 128 in place of eight of 128 x 64, the unit of
     // gate_unit.h and bfloat16 stored in whole lines, before and after (us): 32 experts, gated, 1,777 tokens 93
-    // and 87, unevenly taken 105 and 95, 4,096 tokens 169 and 158, unevenly 163 and 149; 8 experts of 4,096,
-    // gated, 1,777 tokens 173 and 159; their down product at 4,096 tokens 153 and 145.  32-bit results of few
+    // and 84, unevenly taken 105 and 94, 4,096 tokens 169 and 156, unevenly 163 and 148; 8 experts of 4,096,
+    // gated, 1,777 tokens 173 and 158; their down product at 4,096 tokens 153 and 145.  32-bit results of few
     // steps of K are bound by the 58 MB and more that they write: 2,048 x 1,024, 1,777 tokens unevenly 58 and
     // 57, 1,024 tokens 38.4 and 39.3, unevenly 36.3 and 36.2, 1,277 45 and 42, 4,096 104 and 104; 64 experts of 2,048 x
     // 1,408, 6 a token, 1,093 tokens 96.4 and 95.5, unevenly 77.1 and 77.4.  Low tiles take longer at all of these.
@@ -598,12 +599,16 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
       const long long tiles = (A + high - 1) / max(high, 1) + experts;
       const long long blocks = (tiles * columns + 7) / 8 * 8 + 8;
       if (high && blocks > 0x7fffffffLL) return ZA_ERR_ARG;
+#define ZA_GWH(TO, UNIT, HIGH, ROUNDED)                                                                    \
+  hipLaunchKernelGGL((grouped_gemm_bf16_wide_kernel<TO, UNIT, HIGH, ROUNDED>), dim3((unsigned)blocks),     \
+                     dim3(256), 0, stream, g)
 #define ZA_GW(TO, UNIT)                                                                                    \
   {                                                                                                        \
-    if (high == 256)                                                                                       \
-      hipLaunchKernelGGL((grouped_gemm_bf16_wide_kernel<TO, UNIT, 256>), dim3((unsigned)blocks), dim3(256), 0, stream, g); \
-    else                                                                                                   \
-      hipLaunchKernelGGL((grouped_gemm_bf16_wide_kernel<TO, UNIT, 128>), dim3((unsigned)blocks), dim3(256), 0, stream, g); \
+    constexpr bool CHOICE = UNIT > 0 && UNIT < 4;                                                          \
+    if (high == 256 && CHOICE && rounded) ZA_GWH(TO, UNIT, 256, CHOICE);                                   \
+    else if (high == 256) ZA_GWH(TO, UNIT, 256, false);                                                    \
+    else if (CHOICE && rounded) ZA_GWH(TO, UNIT, 128, CHOICE);                                             \
+    else ZA_GWH(TO, UNIT, 128, false);                                                                     \
     return za_launch_status();                                                                             \
   }
       if (high) {
@@ -613,6 +618,7 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
         else if (gate == 2) ZA_GW(bf16_t, 2)
         else ZA_GW(bf16_t, 3)
       }
+#undef ZA_GWH
 #undef ZA_GW
     }
     const int BM = A >= 40LL * experts ? 128 : A >= 24LL * experts ? 64 : 32, BN = BM == 32 ? 64 : 128;

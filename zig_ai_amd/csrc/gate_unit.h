@@ -25,9 +25,9 @@ __device__ __forceinline__ float unit_sigmoid(float x) {
 
 // KIND 1: silu, 2: the tanh form of gelu, 3: v * sigmoid(slope * v) * (u + offset) with v and u bounded
 // (bound > 0).  For results in bfloat16 EXACT is left out.  (us, with EXACT and without: gated products of the wide
-// tiles 2 x 8192 x 2048 at 2,048 rows 116 and 111, 2 x 4608 x 1024 at 1,037 rows 32 and 29.4; the unit by itself on 8,192
+// tiles 2 x 8192 x 2048 at 2,048 rows 114 and 109, 2 x 4608 x 1024 at 1,037 rows 31 and 28; the unit by itself on 8,192
 // outputs of 1,037 rows 11.0 and 9.9.  The hardware's exponential of a rounded product and its reciprocal as they are,
-// 108, 27.6 and 9.1, were off by up to 1e-6 at |x| of 20 and 4e-6 at 87.)
+// 106, 26 and 9.1, were off by up to 1e-6 at |x| of 20 and 4e-6 at 87.)
 template <int KIND, bool EXACT>
 __device__ __forceinline__ float gated_value(float v, float u, float bound, float slope, float offset) {
   if constexpr (KIND == 3) {

@@ -7,8 +7,8 @@
 // write and read them).  Full tiles of 256 rows and, at the end, one as low as holds what is left, 128, 192
 // or 256: 1,037 rows make 4.5 rows of tiles.  Which products take it is the caller's rule.
 // Measured (us; weights from memory, the library's product and the unit's kernel in brackets): 2 x 8192 x 2048
-// at 2,048 rows 110 (123), 1.25 PFLOP/s; 2 x 7168 x 2048 at 1,037 61 (77), at 917 51 (59); 2 x 4608 x 1024 at
-// 1,777 34 (42).  Without a unit the same tiles gain nothing: 6144 x 2048 at 2,048 rows 44 (42).
+// at 2,048 rows 109 (123), 1.26 PFLOP/s; 2 x 7168 x 2048 at 1,037 60 (78), at 917 52 (60); 2 x 4608 x 1024 at
+// 1,777 32 (42).  Without a unit the same tiles gain nothing: 6144 x 2048 at 2,048 rows 44 (42).
 #include <type_traits>
 
 #include "gate_unit.h"
@@ -20,10 +20,10 @@ struct WideArgs {
   bf16_t* out;
   int M, N, K;
   float bound, slope, offset;
-  int rounded;      // the unit reads the sums rounded to bfloat16, as a kernel of its own would
 };
 
-template <int UNIT>      // the unit's kind (gate_unit.h)
+// UNIT: the unit's kind (gate_unit.h); ROUNDED: it reads the sums rounded to bfloat16, as a kernel of its own would
+template <int UNIT, bool ROUNDED>
 __global__ void __launch_bounds__(256, 1)
 gemm_bf16_wide_gated_kernel(WideArgs g) {
   __shared__ __attribute__((aligned(16))) char lds[GW_LDS];
@@ -61,8 +61,8 @@ gemm_bf16_wide_gated_kernel(WideArgs g) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float a = acc[i][2 * j][r], b = acc[i][2 * j + 1][r];
-            v[r] = gated_value<UNIT, false>(g.rounded ? (float)(bf16_t)a : a, g.rounded ? (float)(bf16_t)b : b, g.bound,
-                                            g.slope, g.offset);
+            v[r] = gated_value<UNIT, false>(ROUNDED ? (float)(bf16_t)a : a, ROUNDED ? (float)(bf16_t)b : b, g.bound, g.slope,
+                                            g.offset);
           }
           return v;
         },
@@ -91,12 +91,17 @@ extern "C" int za_gemm_bf16_wide_gated(const void* x, const void* W, void* out, 
   const long long columns = (N + 127LL) / 128, rows = (M + 255LL) / 256;
   const long long blocks = (rows * columns + 7) / 8 * 8 + 8;      // (two kinds, each an eighth a die)
   if (blocks > 0x7fffffffLL) return ZA_ERR_ARG;
-  const WideArgs g{(const bf16_t*)x, (const bf16_t*)W, (bf16_t*)out, M, N, K, bound, slope, offset, rounded};
-#define ZA_GW(UNIT) \
-  hipLaunchKernelGGL((gemm_bf16_wide_gated_kernel<UNIT>), dim3((unsigned)blocks), dim3(256), 0, stream, g)
-  if (kind == 1) ZA_GW(1);
-  else if (kind == 2) ZA_GW(2);
-  else ZA_GW(3);
+  const WideArgs g{(const bf16_t*)x, (const bf16_t*)W, (bf16_t*)out, M, N, K, bound, slope, offset};
+#define ZA_GW(UNIT)                                                                                                     \
+  {                                                                                                                     \
+    if (rounded)                                                                                                        \
+      hipLaunchKernelGGL((gemm_bf16_wide_gated_kernel<UNIT, true>), dim3((unsigned)blocks), dim3(256), 0, stream, g);   \
+    else                                                                                                                \
+      hipLaunchKernelGGL((gemm_bf16_wide_gated_kernel<UNIT, false>), dim3((unsigned)blocks), dim3(256), 0, stream, g);  \
+  }
+  if (kind == 1) ZA_GW(1)
+  else if (kind == 2) ZA_GW(2)
+  else ZA_GW(3)
 #undef ZA_GW
   return za_launch_status();
 }

@@ -912,10 +912,10 @@ def linear_gated_tiles(x: torch.Tensor, gate_up_weight: torch.Tensor,
 # time, a step of 64 elements of K 1.1 us of a round, end before the library's product and the unit's kernel
 # after it would, 1.28 PFLOP/s and 12 us together.  Measured (us; weights from memory, the library's
 # product with the unit's kernel and this one): 2 x 8192 x 2048 at 400, 600, 1,037, 1,300, 2,048 and 4,096
-# rows 39, 47, 85, 96, 123, 235 and 46, 48, 78, 97, 110, 215; 2 x 7168 x 2048 at 600, 1,037, 1,300, 2,048
-# rows 43, 77, 85, 111 and 44, 61, 95, 103; 2 x 4608 x 1024 at 512, 700, 1,037, 1,777, 4,096 rows 22, 24, 30,
-# 42, 95 and 27, 28, 29, 34, 90; 2 x 1024 x 2048 at 2,048 and 4,096 rows 25, 39 and 41, 45.  Over 171 products of
-# 100 to 5,000 rows the choice is 0.9 percent from the better of the two on average.
+# rows 38, 47, 85, 94, 123, 234 and 45, 45, 74, 93, 110, 211; 2 x 7168 x 2048 at 600, 1,037, 1,300, 2,048
+# rows 43, 78, 86, 112 and 45, 61, 91, 101; 2 x 4608 x 1024 at 512, 700, 1,037, 1,777, 4,096 rows 22, 24, 30,
+# 42, 96 and 26, 26, 27, 32, 86; 2 x 1024 x 2048 at 2,048 and 4,096 rows 25, 39 and 40, 43.  Over 171 products of
+# 100 to 5,000 rows the choice is 0.7 percent from the better of the two on average.
 WIDE_ROUND_US = 4.0
 WIDE_STEP_US = 1.1
 WIDE_LIBRARY_US = 12.0

@@ -145,14 +145,34 @@ def test_gemm_f32_order_of_sums(N, K):
 @pytest.mark.parametrize("K", [32, 96, 128, 160, 512, 544, 672, 736, 768, 800, 1056])
 @pytest.mark.parametrize("M,N", [(130, 2100), (200, 4001), (130, 6000), (65, 16385)])
 def test_gemm_f32_steps_through_lds(M, N, K):
-    """K of whole steps of 32, below, at and off whole chains of 128 and what one, two and four groups take
-    together: right, and the bits of rows on their own, which another kernel takes."""
+    """K of whole steps of 32, below, at and off whole chains of 128 and several of them: right, and the bits of
+    rows on their own, which another kernel takes."""
     x, w = rand((M, K), torch.float32, 63).to(dev()), rand((N, K), torch.float32, 64).to(dev())
     whole = ops().linear(x, w)
     assert rel_err(whole, x.double() @ w.double().T) < 1e-6      # (as above)
     assert torch.equal(ops().linear(x[M - 1:].contiguous(), w), whole[M - 1:])
     bias = rand((N,), torch.float32, 65).to(dev())
     assert torch.equal(ops().linear(x, w, bias), whole + bias)
+
+
+@pytest.mark.parametrize("K", [64, 192, 224, 256, 288, 320, 352, 384, 416, 448, 480])
+@pytest.mark.parametrize("M,N", [(200, 4001), (130, 2100)])
+def test_gemm_f32_each_number_of_last_steps(M, N, K):
+    """Tiles of 64 x 64 and 32 x 64 through LDS: no, one, two and three steps of 32 behind no, one, two and three whole
+    chains of four, each of which ends its requests and waits in its own code: right, and the bits of rows on
+    their own, also of the grouped products, which share that code."""
+    o = ops()
+    x, w = rand((M, K), torch.float32, 67).to(dev()), rand((N, K), torch.float32, 68).to(dev())
+    whole = o.linear(x, w)
+    assert rel_err(whole, x.double() @ w.double().T) < 1e-6      # (as above)
+    for row in (0, M - 1):
+        assert torch.equal(o.linear(x[row:row + 1].contiguous(), w), whole[row:row + 1])
+    chosen = (torch.arange(M, dtype=torch.int32) % 2).view(M, 1).to(dev())
+    lists, counts = o.expert_lists(None, chosen, M, 2)
+    both = w[:N // 2 * 2].view(2, N // 2, K).contiguous()
+    got = o.grouped_linear(x, both, lists, counts, M, per_token=True)
+    for e in (0, 1):
+        assert torch.equal(got[e::2], o.linear(x[e::2].contiguous(), both[e]))
 
 
 @pytest.mark.parametrize("M,N,K", [(40, (1 << 20) + 70, 1056), (33, 262144 + 5, 4096)])

@@ -836,10 +836,11 @@ paged_attention_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restr
   [[maybe_unused]] __shared__ float rope_cs[ROPE ? D / 2 : 1], rope_sn[ROPE ? D / 2 : 1];
 
   const int item = blockIdx.x, gkv = blockIdx.y, z = blockIdx.z;
-  // (heads of 64: known to be the same for all lanes, and its branches and bounds scalar: one request at sixty keys
-  // 11.2 -> 10.8 us a layer, eight at 2,048 14.6 -> 14.4; heads of 128 spill up to 11 registers by it)
+  // (eight waves: known to be the same for all lanes, and its branches and bounds scalar: one request at sixty keys
+  // 11.2 -> 10.8 us a layer, eight at 2,048 14.6 -> 14.4; with four waves nothing is gained, and heads of 128 spill
+  // up to 11 registers by it)
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = D == 64 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+  const int wave = NWV == 8 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int r16 = lane & 15, grp = lane >> 4;
   const int G = nh / nkv;
   // without work-item arrays item i is request i's single token (a pure decode step)

@@ -837,7 +837,7 @@ paged_attention_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restr
 
   const int item = blockIdx.x, gkv = blockIdx.y, z = blockIdx.z;
   // (eight waves: known to be the same for all lanes, and its branches and bounds scalar: one request at sixty keys
-  // 11.2 -> 10.8 us a layer, eight at 2,048 14.6 -> 14.4; with four waves nothing is gained, and heads of 128 spill
+  // 11.2 -> 11.0 us a layer, eight at 2,048 14.6 -> 14.35; with four waves nothing is gained, and heads of 128 spill
   // up to 11 registers by it)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = NWV == 8 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;

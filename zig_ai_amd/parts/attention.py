@@ -89,8 +89,8 @@ SPLIT_MAX = 64
 
 def plan_split(n_items: int, num_kv_heads: int, max_keys: int, target: int = SPLIT_TARGET):
     """(keys per range, number of ranges) for one launch; a function of the batch
-    shape and of the longest context only.  ``target``: workgroups to reach (the
-    kernel for prompt portions runs two workgroups per compute unit and wants 512)."""
+    shape and of the longest context only.  ``target``: workgroups to reach (attention over planes
+    has a rule of its own, ``planes_target``; prompt portions over whole rows go by ``plan_portions``)."""
     groups = n_items * num_kv_heads
     # (a range of 512 keys is one tile for each of the decode kernel's eight waves; short
     # contexts are cut finer: decoding one request at 512 keys, 4 ranges 0.692 ms a step,

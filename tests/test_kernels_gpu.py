@@ -2042,6 +2042,22 @@ def test_gated_products_of_many_rows(M, I, K):
         assert rel_err(got, gl * torch.sigmoid(1.702 * gl) * (ul + 1.0)) < tol_of(torch.bfloat16)
 
 
+@pytest.mark.parametrize("M", [65, 200, 257])
+def test_gated_products_of_many_rows_from_rounded_sums(M):
+    """Each unit on sums rounded ahead of it: where the sums are whole numbers, and so the same in any order, the
+    bits of the unit's own kernel on a product in bfloat16, bounded and not."""
+    o = ops()
+    g = torch.Generator().manual_seed(M)
+    x = torch.randint(-3, 4, (M, 128), generator=g).bfloat16().to(dev())
+    w = torch.randint(-1, 2, (2 * 136, 128), generator=g).bfloat16().to(dev()) * 0.125
+    both = (x.double() @ w.double().T).bfloat16()
+    assert o.wide_takes_gated(M, 136, 128)
+    for activation in ("silu", "gelu_tanh"):
+        assert torch.equal(o.linear_gated_wide(x, w, activation, rounded=True), o.gated_unit(both, activation))
+    for bounds in ((0.0, 1.702, 1.0), (2.0, 1.702, 1.0)):
+        assert torch.equal(o.linear_gated_wide(x, w, bounded=bounds, rounded=True), o.clamped_glu(both, *bounds))
+
+
 def test_gated_products_of_many_rows_leave_other_rows_alone():
     """Infinite and undefined inputs reach their own row's outputs only, and products the rule or the kernel
     does not take are refused."""

@@ -886,3 +886,70 @@ def test_latent_prepare_kernels(dtype, Rq, R, Dr, rot, adjacent):
             assert float(((got[s] - rows[t]) / (1 + rows[t].abs())).abs().max()) < tol
     untouched = [s for s in range(12) if s not in slots]
     assert bool((got[untouched] == 9).all())
+
+
+@pytest.mark.parametrize("H,rotated,mode,lens,ctxs", [
+    (16, 64, None, [33, 64, 65], [0, 0, 0]), (3, 64, "element", [2, 129, 200], [0, 77, 5]),
+    (5, 0, "head", [63, 300], [1, 640]), (1, 64, "head", [2], [0]), (40, 0, None, [900], [0])])
+def test_latent_attention_over_formed_keys(H, rotated, mode, lens, ctxs):
+    """Portions at the edges of items of 64 rows and of tiles of 64 keys, with and without cached rows, from one
+    workgroup to several rounds of them: rows laid out, queries turned, keys and values formed, attention,
+    sink and gate."""
+    from zig_ai_amd.engine.batch import _make_items
+    from zig_ai_amd.kernels import ops
+    dev, R, d, page = torch.device("cuda"), 256, 128, 12
+    g = torch.Generator().manual_seed(H + sum(lens))
+    S, T, W = len(lens), sum(lens), R + rotated
+    pages = [-(-(n + c) // page) for n, c in zip(lens, ctxs)]
+    table = torch.full((S, max(pages) + 1), -1, dtype=torch.int32)
+    order, at = torch.randperm(sum(pages), generator=g), 0
+    for s, n in enumerate(pages):
+        table[s, :n] = order[at:at + n]
+        at += n
+    plane = torch.randn(sum(pages), 1, page, W, generator=g).bfloat16()
+    q = torch.randn(T, H, d + rotated, generator=g).bfloat16()
+    up = (torch.randn(2 * H * d, R, generator=g) * R ** -0.5).bfloat16()
+    rot_dims = rotated // 2
+    inv = torch.rand(max(rot_dims // 2, 1), generator=g) if rot_dims else None
+    sink = torch.randn(H, generator=g)
+    gate = torch.randn(T, 8 + (H * d if mode == "element" else -(-H // 8) * 8), generator=g).bfloat16()
+    positions = [c + j for n, c in zip(lens, ctxs) for j in range(n)]
+    mk = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
+    seq, row0, cnt = _make_items(lens, ops.LATENT_EXPANDED_ROWS, 2)
+    start = [sum(lens[:s]) for s in range(S + 1)]
+    turned = q.to(dev)
+    latent, rot = ops.latent_open_rows(turned, d, rotated, mk(positions), inv.to(dev) if rot_dims else None, rot_dims,
+                                       True, 1.25, plane.to(dev), R, table.to(dev), mk(start), mk(ctxs),
+                                       T + sum(ctxs))
+    kv = ops.linear(latent, up.to(dev))
+    got = ops.latent_expanded(turned, kv, rot, mk(positions), (mk(seq), mk(row0), mk(cnt), len(seq)), mk(start),
+                              mk(ctxs), 0.09, sink.to(dev), gate.to(dev) if mode else None, 8, mode).cpu().double()
+    qd = q.double()
+    if rot_dims:
+        angle = torch.tensor(positions).double()[:, None, None] * inv.double()
+        c, s = 1.25 * angle.cos(), 1.25 * angle.sin()
+        u, v = qd[..., d:d + rot_dims:2].clone(), qd[..., d + 1:d + rot_dims:2].clone()
+        qd[..., d:d + rot_dims:2], qd[..., d + 1:d + rot_dims:2] = u * c - v * s, v * c + u * s
+    for s in range(S):
+        n = lens[s] + ctxs[s]
+        rows = plane[table[s, :pages[s]].long()].view(-1, W)[:n]
+        at = start[s] + sum(ctxs[:s])
+        assert torch.equal(latent[at:at + n].cpu(), rows[:, :R])
+        assert not rotated or torch.equal(rot[at:at + n].cpu(), rows[:, R:])
+        formed = (rows[:, :R].double() @ up.double().T).view(n, 2, H, d)
+        keys = torch.cat([formed[:, 0], rows[:, None, R:].double().expand(n, H, rotated)], dim=2)
+        mine = slice(start[s], start[s + 1])
+        scores = torch.einsum("thd,nhd->htn", qd[mine], keys) * 0.09
+        scores = scores.masked_fill(torch.arange(n)[None, :] > torch.tensor(positions[mine])[:, None], -math.inf)
+        weights = torch.softmax(torch.cat([scores, sink.double()[:, None, None].expand(H, lens[s], 1)], dim=2), dim=2)
+        want = torch.einsum("htn,nhd->thd", weights[..., :n], formed[:, 1])
+        if mode:
+            z = torch.sigmoid(gate[mine, 8:].double())
+            want = want * (z[:, :H, None] if mode == "head" else z.view(-1, H, d))
+        # (roundings to bfloat16, 2^-9 at most and a third of its square on average, of queries' turned parts, keys,
+        # values, weights and the result: sqrt(5 / 3) 2^-9 = 2.5e-3 of the norm; scores of deviation 1.2)
+        assert rel_norm(got[mine], want) < 5e-3, s
+
+
+def rel_norm(got, want):
+    return float((got - want).norm() / want.norm())

@@ -78,6 +78,9 @@ class StepContext:
     host: Optional[np.ndarray] = None
     offsets: Dict[str, Tuple[int, int]] = field(default_factory=dict)
     table_width: int = 0
+    # the step's arrays lie in a buffer that is filled again before every replay of a recording: sizes that
+    # follow from the contexts' lengths on the host would be those of the recorded step
+    replayed: bool = False
     # diagnostics: when a dict, the part that is running may leave copies of its
     # intermediate tensors in it by name (token rows first); see DecoderModel.forward
     taps: Optional[Dict[str, torch.Tensor]] = None
@@ -308,7 +311,7 @@ def build_step(entries: Sequence[StepEntry], cache: CacheManager, device: torch.
         seq_start=view("seq_start"), ctx_len=view("ctx_len"), slot_id=view("slot_id"),
         logit_rows=view("logit_rows"),
         seq_lens_host=seq_lens, ctx_lens_host=ctx_lens, slots_host=slots,
-        host=host, offsets=offsets, table_width=max_pages)
+        host=host, offsets=offsets, table_width=max_pages, replayed=into is not None)
     for g in groups:
         ctx.slot_mapping[g.index] = view(f"slots{g.index}")
         ctx.block_tables[g.index] = view(f"table{g.index}").view(S, max_pages)

@@ -28,7 +28,7 @@ PACKAGE_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC_DIR = os.path.join(PACKAGE_DIR, "csrc")
 ARCH = "gfx950"
 SOURCES = ("norm", "gemm", "gemm_f32", "gemm_rows64", "gemm_tiles", "gemm_wide", "gemm_half", "rope_kv", "attention", "attention_planes", "shortconv", "recurrent",
-           "recurrent_chunks", "activation", "experts", "latent", "sampling", "blaslt", "calibrate")
+           "recurrent_chunks", "activation", "experts", "latent", "latent_expanded", "sampling", "blaslt", "calibrate")
 HOST_SOURCES = ("host", "plain")    # plain C++, no device code: usable without a GPU or ROCm
 ALL_SOURCES = SOURCES + HOST_SOURCES
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden"]
@@ -41,7 +41,7 @@ HIPCC_FLAGS = [
 EXTRA_FLAGS = {"blaslt": ["-lhipblaslt"]}   # host code around the GEMM library, no kernels
 # headers a source includes beside common.h
 EXTRA_HEADERS = {"sampling": ["no_alloc.h"], "rope_kv": ["rope_math.h"], "attention": ["attention_common.h", "rope_math.h"],
-                 "attention_planes": ["attention_common.h"], "recurrent": ["rope_math.h"], "gemm_f32": ["gemm_f32.h"],
+                 "attention_planes": ["attention_common.h"], "latent_expanded": ["attention_common.h"], "recurrent": ["rope_math.h"], "gemm_f32": ["gemm_f32.h"],
                  "experts": ["gate_unit.h", "gemm_f32.h", "tiles_bf16.h", "tiles_wide.h"], "latent": ["tiles_bf16.h"],
                  "gemm_tiles": ["tiles_bf16.h"], "gemm_wide": ["gate_unit.h", "tiles_bf16.h", "tiles_wide.h"],
                  "gemm_half": ["tiles_bf16.h", "tiles_wide.h", "tiles_half.h"], "activation": ["gate_unit.h"]}

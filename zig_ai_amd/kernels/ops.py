@@ -223,6 +223,12 @@ _SIGNATURES = {
                                       c_int, c_void_p],
     ("latent", "za_rotate_part"): [c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int,
                                    c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
+    ("latent_expanded", "za_latent_open_rows"): [
+        c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p,
+        c_longlong, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
+    ("latent_expanded", "za_latent_expanded"): [
+        c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+        c_int, c_int, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     ("latent", "za_head_linear"): [c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int,
                                    c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int,
                                    c_int, c_void_p],
@@ -3349,6 +3355,105 @@ def latent_attention(q: torch.Tensor, plane: torch.Tensor, kv_rank: int, block_t
     _check(rc, "latent_attention")
     _note("attention", kernel="latent_mfma" if waves else "latent", rows=T, dtype=q.dtype,
           nsplit=int(nsplit), waves=int(waves))
+    return out
+
+
+LATENT_EXPANDED_HEAD = 128     # channels of a head's values and of its keys' unrotated part
+LATENT_EXPANDED_ROWS = 64     # tokens of a work item
+
+
+def latent_expanded_fits(dtype, head_dim: int, rot_dim: int, value_dim: int, kv_rank: int) -> bool:
+    """Whether keys and values of these sizes can be formed and attended to."""
+    return dtype == torch.bfloat16 and head_dim == value_dim == LATENT_EXPANDED_HEAD and rot_dim in (0, 64) \
+        and kv_rank % 8 == 0
+
+
+def latent_open_rows(q: torch.Tensor, q_col: int, rot_dim: int, positions: torch.Tensor,
+                     inv_freq: Optional[torch.Tensor], rot_dims: int, adjacent_pairs: bool, magnitude: float,
+                     plane: torch.Tensor, kv_rank: int, block_table: torch.Tensor, seq_start: torch.Tensor,
+                     ctx_len: torch.Tensor, n_rows: int):
+    """``(latents [n_rows, kv_rank], rotated key parts [n_rows, rot_dim] or None)``: every request's
+    cached rows, its ``ctx_len`` earlier ones and this step's (already written), one request's behind
+    the other's; ``n_rows`` is their number.  ``q[t, h, q_col : q_col + rot_dim]`` is rotated in place
+    (its first ``rot_dims`` elements, as ``rotate_part_`` does)."""
+    _need(q, "q", torch.bfloat16)
+    if q.dim() != 3 or q_col < 0 or q_col + rot_dim > q.shape[2]:
+        raise KernelError(f"q must be [T, heads, width], got {tuple(q.shape)}")
+    T, H = q.shape[:2]
+    page_size, stride = _latent_plane(plane, q.dtype, kv_rank + rot_dim)
+    S = ctx_len.numel()
+    _need(positions, "positions", torch.int32, (T,))
+    _need(seq_start, "seq_start", torch.int32, (S + 1,))
+    _need(ctx_len, "ctx_len", torch.int32, (S,))
+    _need(block_table, "block_table", torch.int32)
+    if block_table.dim() != 2 or block_table.shape[0] != S:
+        raise KernelError("block_table must be [requests, max_pages]")
+    if rot_dims % 2 or not 0 <= rot_dims <= rot_dim:
+        raise KernelError(f"rot_dims {rot_dims} must be even and at most {rot_dim}")
+    if rot_dims:
+        _need(inv_freq, "inv_freq", torch.float32, (rot_dims // 2,))
+    if n_rows < T:
+        raise KernelError(f"{n_rows} rows cannot hold the step's {T} tokens")
+    latent = torch.empty((n_rows, kv_rank), dtype=q.dtype, device=q.device)
+    rot = torch.empty((n_rows, rot_dim), dtype=q.dtype, device=q.device) if rot_dim else None
+    rc = _fn("latent_expanded", "za_latent_open_rows")(
+        _ptr(q), q.shape[2], int(q_col), T, H, int(rot_dim), _ptr(positions),
+        _ptr(inv_freq) if rot_dims else None, int(rot_dims), 1 if adjacent_pairs else 0, float(magnitude),
+        _ptr(plane), stride, _ptr(block_table), block_table.shape[1], page_size, _ptr(seq_start),
+        _ptr(ctx_len), S, int(n_rows), int(kv_rank), _ptr(latent), _ptr(rot), _stream())
+    _check(rc, "latent_open_rows")
+    return latent, rot
+
+
+def latent_expanded(q: torch.Tensor, kv: torch.Tensor, rot: Optional[torch.Tensor], positions: torch.Tensor,
+                    items, seq_start: torch.Tensor, ctx_len: torch.Tensor, scale: float,
+                    sink: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None, gate_col: int = 0,
+                    gate_mode: Optional[str] = None) -> torch.Tensor:
+    """Causal attention of ``q [T, heads, 128 + rot_dim]`` (rotated) over formed keys and values
+    ``kv [rows, 2 * heads * 128]`` (all heads' keys, then all heads' values) and the keys' rotated parts
+    ``rot [rows, rot_dim]``, rows as ``latent_open_rows`` lays them out; ``[T, heads, 128]``, times the
+    gate as in ``head_linear``.  ``items``: (request, first row, rows, number) of work items of at most
+    ``LATENT_EXPANDED_ROWS`` tokens that cover the step."""
+    _need(q, "q", torch.bfloat16)
+    if q.dim() != 3:
+        raise KernelError(f"q must be [T, heads, width], got {tuple(q.shape)}")
+    T, H, W = q.shape
+    rot_dim = W - LATENT_EXPANDED_HEAD
+    if rot_dim not in (0, 64) or (rot_dim > 0) != (rot is not None):
+        raise KernelError(f"heads of {W}: keys of {LATENT_EXPANDED_HEAD} with 0 or 64 rotated elements")
+    rows = kv.shape[0]
+    _need(kv, "kv", torch.bfloat16, (rows, 2 * H * LATENT_EXPANDED_HEAD))
+    if rot is not None:
+        _need(rot, "rot", torch.bfloat16, (rows, rot_dim))
+    S = ctx_len.numel()
+    _need(positions, "positions", torch.int32, (T,))
+    _need(seq_start, "seq_start", torch.int32, (S + 1,))
+    _need(ctx_len, "ctx_len", torch.int32, (S,))
+    item_seq, item_row0, item_count, n_items = items
+    for name, t in (("item_seq", item_seq), ("item_row0", item_row0), ("item_count", item_count)):
+        _need(t, name, torch.int32)
+        if t.numel() < n_items:
+            raise KernelError(f"{name} holds {t.numel()} entries, fewer than {n_items} items")
+    if sink is not None:
+        _need(sink, "sink", torch.float32, (H,))
+    gate_ld = 0
+    if gate_mode not in HEAD_GATES:
+        raise KernelError(f"gate_mode must be None, head or element, got {gate_mode!r}")
+    if gate_mode is not None:
+        _need(gate, "gate", torch.bfloat16)
+        need = H if gate_mode == "head" else H * LATENT_EXPANDED_HEAD
+        if gate.dim() != 2 or gate.shape[0] != T or gate_col < 0 or gate_col + need > gate.shape[1]:
+            raise KernelError(f"gate has shape {tuple(gate.shape)}; columns {gate_col}..{gate_col + need} of {T} "
+                              f"rows are needed")
+        gate_ld = gate.shape[1]
+    out = torch.empty((T, H, LATENT_EXPANDED_HEAD), dtype=q.dtype, device=q.device)
+    rc = _fn("latent_expanded", "za_latent_expanded")(
+        _ptr(q), _ptr(kv), _ptr(rot), rows, _ptr(out), _ptr(positions), _ptr(item_seq), _ptr(item_row0),
+        _ptr(item_count), _ptr(seq_start), _ptr(ctx_len), n_items, H, rot_dim, float(scale), _ptr(sink),
+        _ptr(gate) if gate_mode is not None else None, gate_ld, int(gate_col), HEAD_GATES[gate_mode],
+        _stream())
+    _check(rc, "latent_expanded")
+    _note("attention", kernel="latent_expanded", rows=T, dtype=q.dtype)
     return out
 
 

@@ -12,8 +12,10 @@ Per token, with ``h`` the mixer's input:
   y   = Wo (o * sigmoid(Wg h))                      ``gate="element"``: a number an element of
                                                     o; ``"head"``: a number a head; None: none
 
-Only ``[c | rot(k_r)]`` is cached, one plane of ``kv_rank + rotated_dim`` elements a token, and
-keys and values are never formed: ``Wuk_i^T q_i,n`` is taken instead (the score against ``c``
+Only ``[c | rot(k_r)]`` is cached, one plane of ``kv_rank + rotated_dim`` elements a token.  Where
+many new tokens see the same rows (``forming_pays``) every head's keys and values are formed from the
+visible rows and attended to (``csrc/latent_expanded.hip``).  Elsewhere
+they are not: ``Wuk_i^T q_i,n`` is taken instead (the score against ``c``
 is the same number) and ``Wuv_i`` is applied to ``sum_j p_j c_j``, so the attention kernel sees
 one key/value head whose value is a prefix of its key (``csrc/latent.hip``).  bfloat16 rows of
 16-byte pieces run on the matrix cores (work items of 64 rows; a step that only decodes takes the
@@ -63,10 +65,24 @@ def plan_latent_split(groups: int, max_keys: int):
     return (keys, nsplit) if nsplit > 1 else (0, 1)
 
 
+FORMING_ROWS_A_TOKEN = 16      # visible rows a new token, at most
+FORMING_BYTES = 256 << 20      # the most that formed keys and values may take
+
+
+def forming_pays(seq_lens, ctx_lens, bytes_a_row: int) -> bool:
+    """Whether a step's keys and values are formed: every request brings a portion, and a visible row is
+    seen by enough new tokens.  Us a layer folded and formed (16 heads, R = 512 with 64 rotated): 4
+    tokens of 8 requests each 31 and 13, one prompt of 64 32 and 15, 512 61 and 26, 1,777 147 and 60, 4,096 523 and 145;
+    128 tokens behind 900 cached ones 51 and 39, behind 2,000 135 and 65, 64 of 8 requests each behind 400 62 and 42, 512 behind
+    6,000 348 and 158.  Single tokens share their rows with nobody, and a row costs 7 ns to form."""
+    rows = sum(seq_lens) + sum(ctx_lens)
+    return min(seq_lens) > 1 and rows <= FORMING_ROWS_A_TOKEN * sum(seq_lens) and rows * bytes_a_row <= FORMING_BYTES
+
+
 class LatentAttention(Mixer):
     kind = "latent_attention"
     graph_safe = True
-    kernel_sources = ("gemm", "gemm_rows64", "latent", "norm", "activation")
+    kernel_sources = ("gemm", "gemm_rows64", "latent", "latent_expanded", "norm", "activation")
 
     @staticmethod
     def _sizes(params):
@@ -148,6 +164,11 @@ class LatentAttention(Mixer):
         # per head: Wuk^T as [R, d] (folds into the query), Wuv as [dv, R] (expands the result)
         k_up = tensors["k_up.weight"].view(nh, d, R).transpose(1, 2).contiguous()
         v_up = tensors["v_up.weight"].view(nh, dv, R).contiguous()
+        # all heads' Wuk, then all heads' Wuv, where keys and values may be formed
+        self.w_form = None
+        if ops.latent_expanded_fits(runtime.dtype, d, dr, dv, R) and k_up.dtype == v_up.dtype == torch.bfloat16:
+            self.w_form = fuse_rows(tensors["k_up.weight"], tensors["v_up.weight"])
+            v_up = self.w_form[nh * d:].view(nh, dv, R)
         # (the matrix-core form reads 16-byte pieces of its rows)
         if k_up.dtype == torch.bfloat16 and (d % 8 or (d + dr) % 8):
             k_up = k_up.float()
@@ -159,6 +180,9 @@ class LatentAttention(Mixer):
         most = ops.LATENT_MFMA_ROWS if self.mfma else ops.LATENT_MAX_ROWS
         self.rows_per_item = max(1, most // min(nh, most))
         self.item_granularities = [self.rows_per_item]
+        if self.w_form is not None:
+            self.item_granularities.append((ops.LATENT_EXPANDED_ROWS, 2))
+            ops.check_projection_weight(self.w_form, "latent attention w_form")
         for w, what in ((self.w_open, "w_open"), (self.w_q_up, "w_q_up"), (self.w_out, "w_out")):
             ops.check_projection_weight(w, "latent attention " + what)
 
@@ -176,6 +200,10 @@ class LatentAttention(Mixer):
                                 self.inv_freq, self.rot_dims, self.adjacent,
                                 plane if cache.writes else None, self.magnitude)
         q = ops.linear(cq, self.w_q_up, tune=tune).view(T, nh, d + dr)
+        if self.w_form is not None and not step.replayed \
+                and forming_pays(step.seq_lens_host, step.ctx_lens_host, 2 * nh * (d + dv)):
+            a = self._formed(q, down, plane, step, cache)
+            return ops.linear(a.view(T, nh * dv), self.w_out, partial_ok=self.partial_ok, tune=tune)
         # the folded query [Wuk^T q_n | rot(q_r)]
         qf = torch.empty((T, nh, self.width), dtype=q.dtype, device=q.device)
         ops.head_linear(q, 0, self.k_fold, out=qf, out_col=0)
@@ -204,6 +232,21 @@ class LatentAttention(Mixer):
             step.taps["q"] = qf.clone()
             step.taps["o"] = a.clone()
         return ops.linear(a.view(T, nh * dv), self.w_out, partial_ok=self.partial_ok, tune=tune)
+
+    def _formed(self, q, down, plane, step, cache):
+        """The heads' gated results over formed keys and values."""
+        latent, rot = ops.latent_open_rows(
+            q, self.head_dim, self.rotated_dim, step.positions, self.inv_freq, self.rot_dims, self.adjacent,
+            self.magnitude, plane, self.kv_rank, step.block_tables[cache.group], step.seq_start, step.ctx_len,
+            step.n_tokens + sum(step.ctx_lens_host))
+        kv = ops.linear(latent, self.w_form, tune=self.runtime.tune)
+        a = ops.latent_expanded(q, kv, rot, step.positions, step.attention_items(ops.LATENT_EXPANDED_ROWS, 2),
+                                step.seq_start, step.ctx_len, self.scale, self.sink, down if self.gate else None,
+                                self.gate_col, self.gate)
+        if getattr(step, "taps", None) is not None:
+            step.taps["q"] = q.clone()      # (not folded)
+            step.taps["o"] = a.clone()
+        return a
 
 
 register_mixer(LatentAttention.kind, LatentAttention)

@@ -627,6 +627,32 @@ def test_ssd_recurrence_in_chunks(dtype, H, G, N, P, strong):
     assert float(mem[:, H * N * P:].abs().max()) == 0.0 and float(state[1].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("H,G,N,P", [(8, 1, 128, 64), (3, 3, 64, 128), (2, 2, 128, 192), (64, 1, 64, 64)])
+def test_ssd_chunks_off_their_boundaries(H, G, N, P):
+    """Whole tiles, whose rows are read 16 bytes at a time, against the same rows a float further on, which
+    are read one element at a time: the same bits, in chunks of one to a hundred and twenty-eight tokens."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator(device=dev).manual_seed(H + N + P)
+    C = ops.RETENTION_CHUNK
+    lengths, slots = [C + 1, 1, 2 * C + 16, C - 1, 17], [2, 3, 0, 4, 1]
+    T, width = sum(lengths), H * P + 2 * G * N
+    rand = lambda *shape: torch.randn(*shape, device=dev, generator=gen)
+    x, proj, bias, A_log, D, first = rand(T, width), rand(T, H), rand(H), rand(H) - 1.0, rand(H), rand(6, H * N * P)
+    x[C + 40, 3], x[5, H * P - 1] = math.inf, math.nan
+    slot_id = torch.tensor(slots, dtype=torch.int32, device=dev)
+    got = []
+    for off in (0, 1):
+        conv = torch.cat([rand(T, off), x, rand(T, 4 - off)], dim=1).contiguous()
+        state = first.clone()
+        out = ops.ssd_recurrence_chunked(conv, off + H * P + G * N, off + H * P, off, proj, 0, bias, A_log, D, state, 0,
+                                         slot_id, _chunk_items(lengths, C, dev), H, G, N, P)
+        got.append((out, state))
+    for a, b in zip(*got):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+    assert bool(torch.isfinite(got[0][0][C + 1:C + 2]).all()) and bool(torch.isnan(got[0][0]).any())
+
+
 @pytest.mark.parametrize("H,G,N,P", [(8, 1, 128, 64), (8, 2, 64, 128), (12, 3, 24, 16), (4, 1, 33, 130), (5, 1, 128, 70)])
 def test_ssd_chunks_with_scores_worked_out_once(H, G, N, P, monkeypatch):
     """Heads that share keys and queries take their scores from one place: the bits of the same heads with

@@ -77,11 +77,13 @@ __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + lo
 //   3. decay_chunk_out:     o_i = 2^c_i B^T q_i + sum_(j <= i) 2^(c_i - c_j) dt_j (q_i . k_j) v_j
 // Every factor is a power of at most zero while decays are at most one.  All products are matrix
 // products of 16 x 16 x dk and 16 x 16 x dv blocks; the walk is a chain of tokens instead, 0.34 us
-// each.  2,048 tokens, 64 heads of 128 x 64: 698 us walked; 42 + 16 + 98 us here, 64 + 7 in place of the
-// 98 where the heads share their scores (a head's own take 15 of the products' 37 us and most of the
-// registers), where the products
-// time is 14 + 37 us and the rest waits for operands that pass registers; 16 heads of 128 x 128:
-// 624 us walked, 78 here (92 as chunks of 256 walked side by side and corrected).
+// each.  2,048 tokens, 64 heads of 128 x 64: 698 us walked; 33 + 16 + 51 + 7 us here, where the heads share
+// their scores (a head's own take 15 us and most of the registers); 16 heads of 128 x 128:
+// 624 us walked, 70 here (92 as chunks of 256 walked side by side and corrected).  The products' time is 14 + 21 us;
+// all workgroups are on the chip at once and load, multiply and store at the same time, 67 + 67 + 100 MB in
+// all.  Where the sizes are whole, tiles take neighbouring channels and columns a lane, so that rows are read
+// and written 16 bytes at a time, and the state before a chunk goes into LDS once (element by element, a wave all
+// key channels, and the state a wave: 44 and 64 in place of the 33 and 51).
 #define DC_CHUNK 128
 
 // The least log2 of a decay that is told apart from zero.  Any power this small is zero in 32-bit
@@ -126,19 +128,35 @@ decay_chunk_state_kernel(DecayArgs a) {
   const int row0 = a.item_row0[item], n = a.item_count[item];
   const int dk = a.dk, dv = a.dv;
 
-  const int col = blockIdx.z * 64 + wave * 16 + r16;
-  const bool col_ok = col < dv;
-  const float* krow = a.vec + (size_t)row0 * a.width + a.k_col + (h / (a.H / a.G)) * dk + r16;
-  const float* vrow = a.vec + (size_t)row0 * a.width + a.x_col + h * dv + (col_ok ? col : 0);
-  f32x4_t kk[NT], v;
+  // FULL: a wave takes half of the key channels and 32 columns, neighbouring ones a lane, so that a key's are read 16
+  // bytes at a time (8 at states of 64 rows) and a value's 8: tile t's row r is channel r * CT + t, tile c's column
+  // 2 r + c.  Otherwise all key channels and 16 columns, an element at a time.
+  constexpr int CT = FULL ? NT / 2 : NT, VT = FULL ? 2 : 1;      // tiles of channels, and of columns
+  typedef __attribute__((ext_vector_type(CT))) float keys_t;
+  typedef __attribute__((ext_vector_type(VT))) float values_t;
+  const int chan0 = FULL ? (wave & 1) * CT * 16 : 0, col0 = blockIdx.z * 64 + (FULL ? (wave >> 1) * 32 : wave * 16);
+  const int col = col0 + r16;
+  const bool col_ok = FULL || col < dv;
+  const float* krow = a.vec + (size_t)row0 * a.width + a.k_col + (h / (a.H / a.G)) * dk + chan0 + (FULL ? r16 * CT : r16);
+  const float* vrow = a.vec + (size_t)row0 * a.width + a.x_col + h * dv + (FULL ? col0 + r16 * VT : col_ok ? col : 0);
+  f32x4_t kk[CT], v[VT];
   auto request = [&](int t0) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       // (tokens beyond the chunk have weight zero)
       const size_t at = (size_t)min(t0 + 4 * g + j, n - 1) * a.width;
-      v[j] = FULL || col_ok ? vrow[at] : 0.f;
+      if constexpr (FULL) {
+        const keys_t x = *reinterpret_cast<const keys_t*>(krow + at);
+        const values_t y = *reinterpret_cast<const values_t*>(vrow + at);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) kk[t][j] = FULL || t * 16 + r16 < dk ? krow[at + t * 16] : 0.f;
+        for (int t = 0; t < CT; ++t) kk[t][j] = x[t];
+#pragma unroll
+        for (int c = 0; c < VT; ++c) v[c][j] = y[c];
+      } else {
+        v[0][j] = col_ok ? vrow[at] : 0.f;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) kk[t][j] = t * 16 + r16 < dk ? krow[at + t * 16] : 0.f;
+      }
     }
   };
   request(0);
@@ -186,29 +204,53 @@ decay_chunk_state_kernel(DecayArgs a) {
   }
   __syncthreads();
 
-  f32x4_t S[NT];
+  f32x4_t S[VT][CT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) S[t] = zero4();
+  for (int c = 0; c < VT; ++c)
+#pragma unroll
+    for (int t = 0; t < CT; ++t) S[c][t] = zero4();
   for (int t0 = 0; t0 < n; t0 += 16) {
-    f32x4_t k0[NT];
-    const f32x4_t v0 = v * *reinterpret_cast<const f32x4_t*>(&weight[t0 + 4 * g]);
+    f32x4_t k0[CT], v0[VT];
+    const f32x4_t w = *reinterpret_cast<const f32x4_t*>(&weight[t0 + 4 * g]);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) k0[t] = kk[t];
+    for (int c = 0; c < VT; ++c) v0[c] = v[c] * w;
+#pragma unroll
+    for (int t = 0; t < CT; ++t) k0[t] = kk[t];
     if (t0 + 16 < n) request(t0 + 16);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) S[t] = mfma4(k0[t], v0, S[t]);
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int c = 0; c < VT; ++c)
+#pragma unroll
+        for (int t = 0; t < CT; ++t)
+          S[c][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k0[t][j], v0[c][j], S[c][t], 0, 0, 0);
   }
   if (!col_ok) return;
+  if constexpr (FULL) {
+    // row 4 g + i of all tiles: channels (4 g + i) * CT .. + CT - 1
+#pragma unroll
+    for (int c = 0; c < VT; ++c) {
+      float* st = a.chunk_state + (((size_t)item * a.H + h) * dv + col0 + r16 * VT + c) * dk + chan0 + 4 * g * CT;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        keys_t x;
+#pragma unroll
+        for (int t = 0; t < CT; ++t) x[t] = S[c][t][i];
+        *reinterpret_cast<keys_t*>(st + i * CT) = x;
+      }
+    }
+    return;
+  }
   float* st = a.chunk_state + (((size_t)item * a.H + h) * dv + col) * dk;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
+  for (int t = 0; t < CT; ++t) {
     const int c4 = t * 16 + 4 * g;
-    if (FULL || dk % 4 == 0) {
-      if (FULL || c4 < dk) *reinterpret_cast<f32x4_t*>(st + c4) = S[t];
+    if (dk % 4 == 0) {
+      if (c4 < dk) *reinterpret_cast<f32x4_t*>(st + c4) = S[0][t];
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (c4 + i < dk) st[c4 + i] = S[t][i];
+        if (c4 + i < dk) st[c4 + i] = S[0][t][i];
     }
   }
 }
@@ -291,10 +333,24 @@ template <int NT, bool FULL, bool SHARED>
 __global__ void __launch_bounds__(256, 2)
 decay_chunk_out_kernel(DecayArgs a) {
   __shared__ float hi[DC_CHUNK], lo[DC_CHUNK], step[DC_CHUNK];
+  // FULL: the 64 columns of the state before the chunk, a column's 16-byte pieces in the order piece ^ (column / 4 % 8)
+  // (the eight columns read together fall into different banks)
+  __shared__ __attribute__((aligned(16))) float Bs[FULL ? 64 * NT * 16 : 4];
   const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
   const int row0 = a.item_row0[item], n = a.item_count[item];
   const int dk = a.dk, dv = a.dv, grp = h / (a.H / a.G);
+  const float* B = a.chunk_state + ((size_t)item * a.H + h) * dv * dk;
+  if constexpr (FULL) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int piece = (wave * NT + i) * 64 + lane, col = piece / (NT * 4);
+      lds_request(B + (size_t)(blockIdx.z * 64 + col) * dk + ((piece % (NT * 4)) ^ (col >> 2 & 7)) * 4,
+                  Bs + (wave * NT + i) * 256);
+    }
+  }
+  const int blocks = (n + 15) / 16;
+  const int tile[2] = {wave, 7 - wave};
   if (tid < DC_CHUNK) {
     const bool in = tid < n;
     const float* s = a.sums + ((size_t)(row0 + (in ? tid : 0)) * a.H + h) * 3;
@@ -302,12 +358,13 @@ decay_chunk_out_kernel(DecayArgs a) {
     lo[tid] = in ? s[1] : 0.f;
     step[tid] = in ? s[2] : 0.f;
   }
+  if constexpr (FULL) __builtin_amdgcn_s_waitcnt(ZA_VMCNT(0));      // (the state's pieces)
   __syncthreads();
-  const int blocks = (n + 15) / 16;
-  const int tile[2] = {wave, 7 - wave};
   if (tile[0] >= blocks) return;
   const bool second = tile[1] < blocks;
   const int n0 = blockIdx.z * 64;
+  // a lane's column of tile j: FULL: a lane's four are neighbours, read and written 16 bytes at a time
+  auto col_of = [&](int j) { return n0 + (FULL ? 4 * r16 + j : j * 16 + r16); };
   const float* rows = a.vec + (size_t)row0 * a.width;
   const bool aligned = dk % 4 == 0 && a.width % 4 == 0 && ((a.q_col | a.k_col) % 4) == 0 &&
                        (reinterpret_cast<uintptr_t>(a.vec) & 15) == 0;
@@ -326,15 +383,16 @@ decay_chunk_out_kernel(DecayArgs a) {
     for (int j = 0; j < 4; ++j) acc[i][j] = zero4();
 
   // ---- what the state before the chunk gives
-  const float* B = a.chunk_state + ((size_t)item * a.H + h) * dv * dk;
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     f32x4_t fb[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int col = n0 + j * 16 + r16;
-      fb[j] = FULL || col < dv ? load4<FULL>(B + (size_t)col * dk + t * 16 + 4 * g, dk - (t * 16 + 4 * g), dk % 4 == 0)
-                       : zero4();
+      const int col = col_of(j);
+      if constexpr (FULL)
+        fb[j] = *reinterpret_cast<const f32x4_t*>(&Bs[(4 * r16 + j) * (NT * 16) + ((t * 4 + g) ^ (r16 & 7)) * 4]);
+      else
+        fb[j] = col < dv ? load4_below(B + (size_t)col * dk + t * 16 + 4 * g, dk - (t * 16 + 4 * g), dk % 4 == 0) : zero4();
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -377,10 +435,12 @@ decay_chunk_out_kernel(DecayArgs a) {
     for (int r = 0; r < 4; ++r) {
       // (no token sees one beyond the chunk)
       const float* x = rows + (size_t)min(J * 16 + 4 * g + r, n - 1) * a.width + a.x_col + h * dv;
+      [[maybe_unused]] f32x4_t four;
+      if constexpr (FULL) four = *reinterpret_cast<const f32x4_t*>(x + col_of(0));
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int col = n0 + j * 16 + r16;
-        v[j][r] = FULL || col < dv ? x[col] : 0.f;
+        if constexpr (FULL) v[j][r] = four[j];
+        else v[j][r] = col_of(j) < dv ? x[col_of(j)] : 0.f;
       }
     }
   };
@@ -436,7 +496,7 @@ decay_chunk_out_kernel(DecayArgs a) {
           f32x4_t x;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int col = n0 + j * 16 + r16;
+            const int col = col_of(j);
             x[r] = FULL || col < dv
                        ? rows[(size_t)min(tile[i] * 16 + 4 * g + r, n - 1) * a.width + a.x_col + h * dv + col] : 0.f;
           }
@@ -452,10 +512,20 @@ decay_chunk_out_kernel(DecayArgs a) {
       if (tok >= n) continue;
       float* o = a.out + (size_t)(row0 + tok) * a.H * dv + h * dv;
       const float* x = rows + (size_t)tok * a.width + a.x_col + h * dv;
+      if constexpr (FULL) {
+        f32x4_t y = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
+        if (a.D) {
+          const f32x4_t four = *reinterpret_cast<const f32x4_t*>(x + col_of(0));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = n0 + j * 16 + r16;
-        if (FULL || col < dv) o[col] = a.D ? fmaf(D, x[col], acc[i][j][r]) : acc[i][j][r];
+          for (int j = 0; j < 4; ++j) y[j] = fmaf(D, four[j], y[j]);
+        }
+        *reinterpret_cast<f32x4_t*>(o + col_of(0)) = y;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int col = col_of(j);
+          if (col < dv) o[col] = a.D ? fmaf(D, x[col], acc[i][j][r]) : acc[i][j][r];
+        }
       }
     }
   }
@@ -486,8 +556,9 @@ extern "C" int za_decay_chunked(const float* vec, int width, int q_col, int k_co
                     fixed, item_row0, item_count, sums, chunk_state, total, out, H, G, dk, dv, scores};
   dim3 grid(n_items, H, (dv + 63) / 64);
   const dim3 block(256);
-  const bool full = dv % 64 == 0 && width % 4 == 0 && q_col % 4 == 0 && k_col % 4 == 0 &&
-                    ((reinterpret_cast<uintptr_t>(vec) | reinterpret_cast<uintptr_t>(chunk_state)) & 15) == 0;
+  const bool full = dv % 64 == 0 && width % 4 == 0 && q_col % 4 == 0 && k_col % 4 == 0 && x_col % 4 == 0 &&
+                    ((reinterpret_cast<uintptr_t>(vec) | reinterpret_cast<uintptr_t>(chunk_state) |
+                      reinterpret_cast<uintptr_t>(out)) & 15) == 0;
 #define ZA_DECAY(KERNEL, ...)                                                                  \
   {                                                                                            \
     if (full && dk == 64) hipLaunchKernelGGL((KERNEL<4, true __VA_ARGS__>), grid, block, 0, stream, a);    \

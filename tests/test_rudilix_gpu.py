@@ -951,3 +951,29 @@ def test_causal_conv_at_the_edges_of_its_blocks(taps):
         want = plain.silu(plain.causal_conv(torch.cat([rows, rows]), w.double(), b.double()))
         assert float((torch.cat([y[at:at + n] for y in got]) - want).abs().max()) < 1e-5
         at += n
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,width,group,weights", [
+    (1, 32, 32, 32), (3, 96, 32, 96), (67, 320, 64, 1), (5, 512, 256, 256), (9, 768, 96, 768), (130, 260, 260, 260),
+    (2, 3072, 1024, 3072), (7, 1028, 1028, 1028), (3, 4096, 2048, 2048), (2, 4096, 4096, 4096), (2, 4100, 4100, 4100),
+    (4, 600, 300, 1)])
+def test_gated_group_norm_forms(dtype, T, width, group, weights):
+    """Groups within a wave, a workgroup's, and those that go column by column (widths that are no power of two,
+    one weight for wide groups), each with the gate before and behind the norm, on and off its boundaries."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator().manual_seed(width + group)
+    y, w = torch.randn(T, width, generator=gen), torch.randn(weights, generator=gen)
+    for off in (8, 3):
+        gate = torch.randn(T, width + off, generator=gen).to(dtype)
+        g, wide = gate[:, off:].double(), w.double().repeat(width // weights)
+        for first, act in ((True, "silu"), (False, "sigmoid")):
+            a = plain.silu(g) if act == "silu" else torch.sigmoid(g)
+            v = y.double() * a if first else y.double()
+            want = plain.rms(v.view(T, -1, group), 1e-5).reshape(T, width) * wide * (1.0 if first else a) * 0.75
+            got = ops.gated_group_norm(y.to(dev), gate.to(dev), off, w.to(dev), group, 1e-5, act, first, 0.75)
+            assert got.dtype == dtype
+            # (32-bit sums of up to 4,100 squares; the one rounding to bfloat16 is 2^-9 of a value)
+            tol = 1e-5 if dtype == torch.float32 else 2.0 ** -8
+            assert float(((got.cpu().double() - want).abs() / want.abs().clamp(min=1.0)).max()) < tol, (off, first)

@@ -1105,6 +1105,9 @@ __device__ __forceinline__ f32x4_t four_or_fewer(const float* p, int n, bool ali
 // either operand and receives rows (l / 16) * 4 .. + 3, column (l % 16).  The order in which k
 // runs is free as long as both operands agree: slot g of step j is channel 4 g + j of a
 // block of 16, so that a lane's four steps are four neighbouring floats.
+// FULL: dk fills its tiles and dv its 64 columns; a lane's four columns are neighbours then, read and written 16
+// bytes at a time.
+template <bool FULL>
 __global__ void __launch_bounds__(256)
 channel_readout_kernel(const float* __restrict__ scaled_q,
                        const float* __restrict__ chunk_state, const int* __restrict__ item_row0,
@@ -1121,18 +1124,28 @@ channel_readout_kernel(const float* __restrict__ scaled_q,
   const float* q = scaled_q + ((size_t)(row0 + (row_ok ? t0 + r16 : 0)) * H + h) * dk;
   const float* B = chunk_state + ((size_t)item * H + h) * dv * dk;
   const bool aligned = dk % 4 == 0;
+  auto col_of = [&](int j) { return n0 + (FULL ? 4 * r16 + j : j * 16 + r16); };
+  // (the results that are added to, requested first)
+  [[maybe_unused]] f32x4_t before[4];
+  if constexpr (FULL)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      before[i] = *reinterpret_cast<const f32x4_t*>(out + ((size_t)(row0 + min(t0 + g * 4 + i, cnt - 1)) * H + h) * dv +
+                                                    col_of(0));
   f32x4_t acc[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
   for (int k0 = 0; k0 < dk; k0 += 16) {
     const int k = k0 + 4 * g, left = dk - k;
-    const f32x4_t fq = row_ok ? four_or_fewer(q + k, left, aligned) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-    f32x4_t fb[4];
+    f32x4_t fq, fb[4];
+    if constexpr (FULL) fq = *reinterpret_cast<const f32x4_t*>(q + k);      // (a row beyond the chunk: not stored)
+    else fq = row_ok ? four_or_fewer(q + k, left, aligned) : f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int n = n0 + j * 16 + r16;
-      fb[j] = n < dv ? four_or_fewer(B + (size_t)n * dk + k, left, aligned)
-                     : f32x4_t{0.f, 0.f, 0.f, 0.f};
+      const int n = col_of(j);
+      if constexpr (FULL) fb[j] = *reinterpret_cast<const f32x4_t*>(B + (size_t)n * dk + k);
+      else fb[j] = n < dv ? four_or_fewer(B + (size_t)n * dk + k, left, aligned) : f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int step = 0; step < 4; ++step)
@@ -1145,10 +1158,12 @@ channel_readout_kernel(const float* __restrict__ scaled_q,
     const int t = t0 + g * 4 + i;
     if (t >= cnt) continue;
     float* o = out + (size_t)(row0 + t) * H * dv + h * dv;
+    if constexpr (FULL) {
+      *reinterpret_cast<f32x4_t*>(o + col_of(0)) = before[i] + f32x4_t{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
+    } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + j * 16 + r16;
-      if (n < dv) o[n] += acc[j][i];
+      for (int j = 0; j < 4; ++j)
+        if (col_of(j) < dv) o[col_of(j)] += acc[j][i];
     }
   }
 }
@@ -1180,10 +1195,16 @@ extern "C" int za_channel_recurrence_chunked(const float* vectors, int width, fl
   rc = za_launch_status();
   if (rc != 0) return rc;
   const int column_blocks = (dv + 63) / 64;
-  hipLaunchKernelGGL(channel_readout_kernel,
-                     dim3(n_items, H, (unsigned)((chunk + 63) / 64 * column_blocks)), dim3(256), 0,
-                     stream, scaled_q, chunk_state, item_row0, item_count, out, H, dk, dv,
-                     column_blocks);
+  const dim3 grid(n_items, H, (unsigned)((chunk + 63) / 64 * column_blocks));
+  const bool full = dk % 16 == 0 && dv % 64 == 0 &&
+                    ((reinterpret_cast<uintptr_t>(scaled_q) | reinterpret_cast<uintptr_t>(chunk_state) |
+                      reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+  if (full)
+    hipLaunchKernelGGL((channel_readout_kernel<true>), grid, dim3(256), 0, stream, scaled_q, chunk_state, item_row0,
+                       item_count, out, H, dk, dv, column_blocks);
+  else
+    hipLaunchKernelGGL((channel_readout_kernel<false>), grid, dim3(256), 0, stream, scaled_q, chunk_state, item_row0,
+                       item_count, out, H, dk, dv, column_blocks);
   return za_launch_status();
 }
 

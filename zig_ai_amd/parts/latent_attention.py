@@ -82,6 +82,7 @@ def forming_pays(seq_lens, ctx_lens, bytes_a_row: int) -> bool:
 class LatentAttention(Mixer):
     kind = "latent_attention"
     graph_safe = True
+    takes_normed_rows = True      # ``x`` is only ever handed to ``ops.linear``
     kernel_sources = ("gemm", "gemm_rows64", "latent", "latent_expanded", "norm", "activation")
 
     @staticmethod

@@ -697,6 +697,31 @@ def test_latent_prefill_on_whole_tiles(H, R, rotated, page_size):
         assert float((got - want).abs().max()) < 2e-2, nsplit
 
 
+@pytest.mark.parametrize("H,R,rotated,page_size", [
+    (16, 512, 64, 16), (3, 512, 32, 64), (40, 512, 0, 4), (17, 256, 64, 8), (1, 128, 32, 16), (16, 128, 0, 32)])
+def test_latent_decoding_on_whole_tiles(H, R, rotated, page_size):
+    """Single tokens, 128 keys at a time: contexts at the edges of a wave's 16 keys, of the 32 that a product takes
+    and of tiles, whole and in ranges of less, one and several tiles, with and without pages."""
+    from zig_ai_amd.kernels import ops
+    assert ops.latent_range_fits(R + rotated, R, page_size)
+    requests = [(c, 1) for c in (0, 1, 15, 16, 30, 31, 32, 47, 95, 96, 126, 127, 128, 159, 255, 256, 300)]
+    W = R + rotated
+    q, plane, table, pos, iseq, irow, icnt, n, scale, sink, want = _latent_attention_case(
+        torch.bfloat16, H, W, R, requests, page_size, 1, seed=H + W)
+    for keys, nsplit in ((0, 1), (64, 5), (128, 3), (256, 2), (384, 1)):
+        got = ops.latent_attention(q, plane, R, table, pos, iseq, irow, icnt, n, scale, sink, keys if nsplit > 1 else 0,
+                                   nsplit, 1).cpu().double()
+        # (the probabilities and the result in bfloat16: 2^-9 of values up to 4 either time)
+        assert float((got - want).abs().max()) < 2e-2, nsplit
+    missing, zeros = table.clone(), table.clone()
+    plane = torch.cat([plane, torch.zeros_like(plane[:1])])      # a page of zeros at the end
+    missing[:, ::3], zeros[:, ::3] = -1, plane.shape[0] - 1
+    for keys, nsplit in ((0, 1), (128, 3)):
+        got, want = (ops.latent_attention(q, plane, R, t, pos, iseq, irow, icnt, n, scale, sink, keys, nsplit, 1)
+                     for t in (missing, zeros))
+        assert torch.equal(got, want), nsplit
+
+
 @pytest.mark.parametrize("R,rotated,page_size", [(512, 64, 16), (256, 32, 4), (128, 0, 64), (512, 64, 12)])
 def test_latent_prefill_without_a_page(R, rotated, page_size):
     """A table entry below zero stands for rows of zeros, never for another request's page."""

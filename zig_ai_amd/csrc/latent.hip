@@ -28,6 +28,8 @@
 // elements, angle = position * inv_freq[i] in 32-bit, cosine and sine times `magnitude`.
 #include <math.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "tiles_bf16.h"
 
@@ -211,6 +213,7 @@ extern "C" int za_latent_prepare(const void* down, int dtype, int ld, int q_col,
   if (dtype == 0) ZA_LP(float);
   else if (dtype == 1) ZA_LP(bf16_t);
 #undef ZA_LP
+#undef ZA_LD
   else
     return ZA_ERR_UNSUPPORTED;
   return za_launch_status();
@@ -1524,6 +1527,225 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out
   }
 }
 
+// Single tokens, rows of whole tiles: a workgroup takes LD_KT keys at a time, 16 of them a wave, for up to 16 rows
+// (token, head).  All of a range's rows are requested into LDS at once, without registers, a key's 16-byte pieces in the
+// order piece ^ (key % 8); a wave has the scores of its keys, over the whole of a row; the waves' maxima meet in
+// LDS, then their weights, and a wave takes every eighth of the latent over all keys, turned round on the way to
+// registers (ds_read_b64_tr_b16).  What bounds it is the way to memory (item, position, page, rows) once a range:
+// 8 requests of 16 heads at 2,051 keys, R = 512 with 64 rotated, ranges of 128, with the merge: 18.7 us, tiles of 32 through
+// registers with three meetings each 23.5; 64 at 1,200 in ranges of 512 32, before in ranges of 128 58; 8 at 8,000 29 and 50.
+#define LD_KT 128
+#define LD_NW (LD_KT / 16)
+template <int RT, int DT>
+struct LdShape {
+  static constexpr int R = RT * 16, W = R + DT * 32, WS = W / 32;
+  static constexpr int NP = (WS * 4 + 7) / 8 * 8;            // pieces of a key in LDS
+  static constexpr size_t LDS = (size_t)LD_KT * NP * 16 + 16 * LD_KT * 2 + 16 * LD_NW * 4;
+};
+
+template <int RT, int DT>
+__global__ void __launch_bounds__(LD_NW * 64)
+latent_decode_range_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ plane,
+                           long long page_stride, const int* __restrict__ block_table, int bt_stride,
+                           const int* __restrict__ positions, const int* __restrict__ wi_seq,
+                           const int* __restrict__ wi_row0, const int* __restrict__ wi_count,
+                           float* __restrict__ part_acc, float* __restrict__ part_ml, int H, int HC, int page_shift,
+                           float scale_log2, int keys_per_split, int nsplit, const float* __restrict__ sink) {
+  using S = LdShape<RT, DT>;
+  constexpr int R = S::R, W = S::W, WS = S::WS, NP = S::NP, OT = RT / LD_NW > 0 ? RT / LD_NW : 1;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lm_lds[];
+  unsigned char* Ks = lm_lds;                                                   // [LD_KT][NP * 16 bytes]
+  unsigned char* Ps = Ks + (size_t)LD_KT * NP * 16;                             // [16 rows][LD_KT]
+  float* Xs = reinterpret_cast<float*>(Ps + 16 * LD_KT * 2);                    // [16 rows][LD_NW]
+
+  const int item = blockIdx.x, z = blockIdx.z, h0 = blockIdx.y * HC;
+  const int G = min(HC, H - h0);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int seq = wi_seq[item], row0 = wi_row0[item];
+  const int count = min(wi_count[item], max(16 / G, 1));      // (the host never asks for more)
+  const int rows = count * G;
+  const int hi = positions[row0 + count - 1];                 // inclusive
+  int range_lo = z * keys_per_split, range_hi = range_lo + keys_per_split - 1;
+  if (nsplit == 1) { range_lo = 0; range_hi = hi; }
+  range_hi = min(range_hi, hi);
+  const bool row_ok = r16 < rows;
+  const int tok = row0 + (row_ok ? r16 / G : 0), h = h0 + (row_ok ? r16 % G : 0);
+  if (nsplit > 1 && range_lo > hi) {
+    // (a range behind the context, as in the kernel above)
+    if (row_ok && wave == 0 && kq == 0) {
+      const size_t pidx = ((size_t)tok * H + h) * nsplit + z;
+      part_ml[pidx * 2] = -INFINITY;
+      part_ml[pidx * 2 + 1] = -1.f;
+    }
+    return;
+  }
+  const int* table = block_table + (size_t)seq * bt_stride;
+
+  // the wave's sixteen keys: a lane knows where one lies (beyond the range its last key, whose score is masked)
+  // (what two waves bring is left out where none of it is in the range: nobody reads it)
+  auto request = [&](int tile0) {
+    if (tile0 + (wave & ~1) * 16 > range_hi) return;
+    const int kp = min(tile0 + wave * 16 + r16, range_hi), page = table[kp >> page_shift];
+    const bf16_t* row = page >= 0 ? plane + (long long)page * page_stride + (long long)(kp & ((1 << page_shift) - 1)) * W
+                                  : (const bf16_t*)lp_no_row;
+    const int low = (int)(uintptr_t)row, high = (int)((uintptr_t)row >> 32);
+    unsigned char* to = Ks + wave * 16 * NP * 16;
+#pragma unroll
+    for (int i = 0; i < NP / 4; ++i) {
+      const int at = i * 64 + lane, key = at / NP;
+      int piece = (at - key * NP) ^ (key & 7);
+      if (NP > WS * 4 && piece >= WS * 4) piece = 0;          // (room that no fragment reads)
+      const uintptr_t from = (unsigned)__shfl(low, key, ZA_WAVE) | (uintptr_t)(unsigned)__shfl(high, key, ZA_WAVE) << 32;
+      lds_request((const bf16_t*)from + piece * 8, to + i * 1024);
+    }
+  };
+  request(range_lo);
+
+  const int pos_q = row_ok ? positions[tok] : -1;
+  bf16x8_t qf[WS];
+  {
+    const bf16_t* qrow = q + ((size_t)tok * H + h) * W + kq * 8;      // (a row that is not there: masked)
+#pragma unroll
+    for (int ks = 0; ks < WS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8_t*>(qrow + ks * 32);
+  }
+  float m = -INFINITY, l = 0.f;
+  f32x4_t o[OT];
+#pragma unroll
+  for (int t = 0; t < OT; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int k_at = (wave * 16 + r16) * NP * 16 + ((kq ^ (r16 & 7)) << 4);
+  const int v_key = kq * 8 + (r16 >> 2);                      // of the first four of a lane group's eight keys
+  const bool has_tiles = wave * OT < RT;
+
+  for (int tile0 = range_lo; tile0 <= range_hi; tile0 += LD_KT) {
+    __builtin_amdgcn_s_waitcnt(ZA_VMCNT(0));
+    __syncthreads();
+    // ---- scores: fragments four ahead of their products, which go to two accumulators
+    f32x4_t s = {0.f, 0.f, 0.f, 0.f}, u = s;
+    bf16x8_t kf[2][4];
+    auto read_keys = [&](int g, bf16x8_t (&f)[4]) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (g * 4 + i < WS)
+          f[i] = *reinterpret_cast<const bf16x8_t*>(Ks + (k_at ^ (((g * 4 + i) & 1) << 6)) + (g * 4 + i) / 2 * 128);
+    };
+    read_keys(0, kf[0]);
+#pragma unroll
+    for (int g = 0; g < (WS + 3) / 4; ++g) {
+      if (g * 4 + 4 < WS) read_keys(g + 1, kf[(g + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int ks = g * 4 + i;
+        if (ks >= WS) continue;
+        if (ks & 1) u = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[g & 1][i], qf[ks], u, 0, 0, 0);
+        else s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[g & 1][i], qf[ks], s, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    s += u;
+    const int kp0 = tile0 + wave * 16 + kq * 4, last = min(pos_q, range_hi);
+    float top = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s[i] = kp0 + i <= last ? s[i] * scale_log2 : -INFINITY;
+      top = fmaxf(top, s[i]);
+    }
+    top = fmaxf(top, __shfl_xor(top, 16, ZA_WAVE));
+    top = fmaxf(top, __shfl_xor(top, 32, ZA_WAVE));
+    if (kq == 0) Xs[r16 * LD_NW + wave] = top;
+    __syncthreads();
+    float m_new = m;
+#pragma unroll
+    for (int w = 0; w < LD_NW; w += 4) {
+      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(&Xs[r16 * LD_NW + w]);
+      m_new = fmaxf(m_new, fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
+    }
+    const float m_use = m_new > -INFINITY ? m_new : 0.f;
+    const float alpha = m == m_new ? 1.0f : exp2f(m - m_use);
+    m = m_new;
+    bf16x4_t p;
+    float psum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[i] = (bf16_t)exp2f(s[i] - m_use);
+      psum += (float)p[i];
+    }
+    l = l * alpha + psum;
+    // (weights of a row in pieces of eight keys, piece ^ (row % 8))
+    *reinterpret_cast<bf16x4_t*>(Ps + r16 * (LD_KT * 2) + (((wave * 2 + (kq >> 1)) ^ (r16 & 7)) << 4) + (kq & 1) * 8) = p;
+    __syncthreads();
+    // ---- values
+    auto values = [&](auto whole) {      // (of blocks of 32 keys, those in the range)
+#pragma unroll
+      for (int t = 0; t < OT; ++t) {
+        o[t] *= alpha;
+        bf16x8_t pf[LD_KT / 32], vf[LD_KT / 32];
+#pragma unroll
+        for (int kk = 0; kk < LD_KT / 32; ++kk) {
+          if (!decltype(whole)::value && tile0 + kk * 32 > range_hi) continue;
+          pf[kk] = *reinterpret_cast<const bf16x8_t*>(Ps + r16 * (LD_KT * 2) + (((kk * 4 + kq) ^ (r16 & 7)) << 4));
+          bf16x4_t half[2];
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {
+            const int key = kk * 32 + v_key + hf * 4, piece = (wave * OT + t) * 2 + ((r16 >> 1) & 1);
+            half[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4_t*)(
+                Ks + key * NP * 16 + ((piece ^ (key & 7)) << 4) + (r16 & 1) * 8));
+          }
+          vf[kk] = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+#pragma unroll
+        for (int kk = 0; kk < LD_KT / 32; ++kk)
+          if (decltype(whole)::value || tile0 + kk * 32 <= range_hi)
+            o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[kk], pf[kk], o[t], 0, 0, 0);
+      }
+    };
+    if (has_tiles) {
+      if (tile0 + LD_KT - 32 <= range_hi) values(std::true_type{});
+      else values(std::false_type{});
+    }
+    if (tile0 + LD_KT <= range_hi) {
+      __syncthreads();                                        // the tile has been read
+      request(tile0 + LD_KT);
+    }
+  }
+
+  // the rows' sums meet like their maxima
+  l += __shfl_xor(l, 16, ZA_WAVE);
+  l += __shfl_xor(l, 32, ZA_WAVE);
+  __syncthreads();
+  if (kq == 0) Xs[r16 * LD_NW + wave] = l;
+  __syncthreads();
+  if (!row_ok) return;
+  float lt = 0.f;
+#pragma unroll
+  for (int w = 0; w < LD_NW; ++w) lt += Xs[r16 * LD_NW + w];
+  if (nsplit == 1) {
+    if (sink) lt += exp2f(sink[h] * LM_LOG2E - m);
+    const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+    if (!has_tiles) return;
+    bf16_t* orow = out + ((size_t)tok * H + h) * R + wave * OT * 16 + kq * 4;
+#pragma unroll
+    for (int t = 0; t < OT; ++t) {
+      bf16x4_t v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (bf16_t)(o[t][i] * inv);
+      *reinterpret_cast<bf16x4_t*>(orow + t * 16) = v;
+    }
+  } else {
+    const size_t pidx = ((size_t)tok * H + h) * nsplit + z;
+    if (has_tiles) {
+      float* pa = part_acc + pidx * R + wave * OT * 16 + kq * 4;
+#pragma unroll
+      for (int t = 0; t < OT; ++t) *reinterpret_cast<f32x4_t*>(pa + t * 16) = o[t];
+    }
+    if (wave == 0 && kq == 0) {
+      part_ml[pidx * 2] = m * LM_LN2;
+      part_ml[pidx * 2 + 1] = lt;
+    }
+  }
+}
+
 // The partial results of a row's ranges -> the row.  `base2`: the partial maxima are whole
 // numbers on the base-2 scale (what the matrix-core kernel keeps), so a partial result's
 // weight 2^(m_z - m) is an exact power of two.
@@ -1689,6 +1911,29 @@ static int launch_latent_prefill(const void* q, void* out, const void* plane, lo
   return za_launch_status();
 }
 
+template <int RT, int DT>
+static int launch_latent_range(const void* q, void* out, const void* plane, long long page_stride,
+                               const int* block_table, int bt_stride, const int* positions, const int* wi_seq,
+                               const int* wi_row0, const int* wi_count, int n_items, float* part_acc, float* part_ml,
+                               int H, int W, int R, int page_size, float scale, int keys_per_split, int nsplit,
+                               const float* sink, hipStream_t stream) {
+  auto kernel = latent_decode_range_kernel<RT, DT>;
+  constexpr size_t LDS = LdShape<RT, DT>::LDS;
+  static bool allowed = false;
+  if (!allowed) {
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS);
+    if (e != hipSuccess) return (int)e;
+    allowed = true;
+  }
+  int shift = 0;
+  while ((1 << shift) < page_size) ++shift;
+  const int HC = H < 16 ? H : 16;
+  hipLaunchKernelGGL(kernel, dim3(n_items, (H + HC - 1) / HC, nsplit), dim3(LD_NW * 64), LDS, stream, (const bf16_t*)q,
+                     (bf16_t*)out, (const bf16_t*)plane, page_stride, block_table, bt_stride, positions, wi_seq, wi_row0,
+                     wi_count, part_acc, part_ml, H, HC, shift, scale * LM_LOG2E, keys_per_split, nsplit, sink);
+  return za_launch_status();
+}
+
 // The matrix-core form: bfloat16, `width` and `kv_rank` multiples of 8.  `waves`: 4 (work
 // items of at most 64 / min(heads, 64) tokens, 16 rows a wave) or 1 (single tokens, as a
 // step that only decodes has: heads in chunks of 16 whose rows the four waves share).
@@ -1724,7 +1969,15 @@ extern "C" int za_latent_attention_mfma(const void* q, void* out, const void* pl
   rc = rotated == 0    ? launch_latent_prefill<RT, 0>(ZA_LM_ARGS)                               \
        : rotated == 32 ? launch_latent_prefill<RT, 1>(ZA_LM_ARGS)                               \
                        : launch_latent_prefill<RT, 2>(ZA_LM_ARGS)
-  if (waves == 4 && whole) {
+#define ZA_LD(RT)                                                                               \
+  rc = rotated == 0    ? launch_latent_range<RT, 0>(ZA_LM_ARGS)                                 \
+       : rotated == 32 ? launch_latent_range<RT, 1>(ZA_LM_ARGS)                                 \
+                       : launch_latent_range<RT, 2>(ZA_LM_ARGS)
+  if (waves == 1 && whole) {
+    if (kv_rank == 128) ZA_LD(8);
+    else if (kv_rank == 256) ZA_LD(16);
+    else ZA_LD(32);
+  } else if (waves == 4 && whole) {
     if (kv_rank == 128) ZA_LP(8);
     else if (kv_rank == 256) ZA_LP(16);
     else ZA_LP(32);
@@ -1738,6 +1991,7 @@ extern "C" int za_latent_attention_mfma(const void* q, void* out, const void* pl
     rc = waves == 4 ? launch_latent_mfma<18, 32, false>(ZA_LM_ARGS)
                     : launch_latent_mfma<18, 32, true>(ZA_LM_ARGS);
 #undef ZA_LP
+#undef ZA_LD
 #undef ZA_LM_ARGS
   if (rc != 0 || nsplit == 1) return rc;
   dim3 grid((unsigned)((size_t)n_tokens * heads));

@@ -3358,6 +3358,12 @@ def latent_attention(q: torch.Tensor, plane: torch.Tensor, kv_rank: int, block_t
     return out
 
 
+def latent_range_fits(width: int, kv_rank: int, page_size: int) -> bool:
+    """Whether single tokens over rows of these sizes take the kernel of 128 keys at a time (the others tiles of
+    32 through registers)."""
+    return kv_rank in (128, 256, 512) and width - kv_rank in (0, 32, 64) and page_size & (page_size - 1) == 0
+
+
 LATENT_EXPANDED_HEAD = 128     # channels of a head's values and of its keys' unrotated part
 LATENT_EXPANDED_ROWS = 64     # tokens of a work item
 

@@ -50,19 +50,26 @@ LATENT_SPLIT_KEYS = 128       # keys of a range at least
 LATENT_SPLIT_BYTES = 32 << 20  # the most that the ranges' partial results may take
 
 
-def plan_latent_split(groups: int, max_keys: int):
-    """(keys per range, number of ranges) for one launch of the matrix-core kernel: a function
+def plan_latent_split(groups: int, max_keys: int, target: int = LATENT_SPLIT_TARGET, tile: int = 64):
+    """(keys per range, number of ranges) for one launch of the matrix-core kernels: a function
     of the batch shape and of the longest context only.  A workgroup holds one or four waves
-    and takes 32 keys a tile, so short ranges pay: as many as reach ``LATENT_SPLIT_TARGET``
-    workgroups, of at least ``LATENT_SPLIT_KEYS`` keys each."""
-    if groups >= LATENT_SPLIT_TARGET or max_keys <= 2 * LATENT_SPLIT_KEYS:
+    and takes 32 keys a tile, so short ranges pay: as many as reach ``target``
+    workgroups, of at least ``LATENT_SPLIT_KEYS`` keys each, in whole tiles of ``tile``."""
+    if groups >= target or max_keys <= 2 * LATENT_SPLIT_KEYS:
         return 0, 1
-    nsplit = min(LATENT_SPLIT_TARGET // groups, max_keys // LATENT_SPLIT_KEYS, 64)
+    nsplit = min(target // groups, max_keys // LATENT_SPLIT_KEYS, 64)
     if nsplit <= 1:
         return 0, 1
-    keys = ((max_keys + nsplit - 1) // nsplit + 63) // 64 * 64
+    keys = ((max_keys + nsplit - 1) // nsplit + tile - 1) // tile * tile
     nsplit = (max_keys + keys - 1) // keys
     return (keys, nsplit) if nsplit > 1 else (0, 1)
+
+
+# The kernel that takes single tokens' keys 128 at a time (``ops.latent_range_fits``) has one workgroup a compute
+# unit at latents of 512 (three at 128), and a second round of them costs more than longer ranges.  Us with
+# ranges of 128, 256 and 512 keys, 16 heads, R = 512 with 64 rotated: 8 requests at 2,050 keys 18.5, 19.8, 25.5, at
+# 8,000 42, 29, 30; 32 at 2,000 36, 26, 29; 64 at 1,200 46, 39, 32; R = 128 with 32: 64 at 2,000 19.0, 15.7, 17.1.
+LATENT_RANGE_TARGET, LATENT_RANGE_TARGET_SMALL, LATENT_RANGE_TILE = 256, 512, 128
 
 
 FORMING_ROWS_A_TOKEN = 16      # visible rows a new token, at most
@@ -216,7 +223,12 @@ class LatentAttention(Mixer):
         if self.mfma:
             # a step that only decodes: a wave a workgroup, heads in chunks of 16
             waves = 1 if step.n_tokens == step.n_seqs else 4
-            keys, nsplit = plan_latent_split(n_items * (-(-nh // (16 * waves))), step.max_keys)
+            groups = n_items * (-(-nh // (16 * waves)))
+            if waves == 1 and ops.latent_range_fits(self.width, R, plane.shape[2]):
+                keys, nsplit = plan_latent_split(groups, step.max_keys, LATENT_RANGE_TARGET if R > 256 else
+                                                 LATENT_RANGE_TARGET_SMALL, LATENT_RANGE_TILE)
+            else:
+                keys, nsplit = plan_latent_split(groups, step.max_keys)
             # (the ranges' partial results are 32-bit rows of the latent's width: no cut where
             # they would be larger than the step is worth)
             if T * nh * nsplit * R * 4 > LATENT_SPLIT_BYTES:

@@ -976,5 +976,25 @@ def test_latent_attention_over_formed_keys(H, rotated, mode, lens, ctxs):
         assert rel_norm(got[mine], want) < 5e-3, s
 
 
+@pytest.mark.parametrize("T", [1, 7, 16, 17])
+@pytest.mark.parametrize("H,R,d,rotated,rot_dims,adjacent", [(16, 512, 128, 64, 64, True), (3, 40, 24, 16, 8, False),
+                                                             (5, 72, 128, 32, 0, True), (2, 128, 264, 64, 64, False)])
+def test_latent_fold_in_one_launch(T, H, R, d, rotated, rot_dims, adjacent):
+    """A decode batch's folded queries against the product and the rotation one after the other: the same bits
+    (17 rows, and heads whose K is shared out, take the two)."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(T + H + d)
+    q = torch.randn(T, H, d + rotated, generator=g).bfloat16().to(dev)
+    fold = (torch.randn(H, R, d, generator=g) * d ** -0.5).bfloat16().to(dev)
+    positions = torch.randint(0, 100000, (T,), generator=g, dtype=torch.int32).to(dev)
+    inv = torch.rand(max(rot_dims // 2, 1), generator=g).to(dev) if rot_dims else None
+    got = ops.latent_fold(q, fold, rotated, positions, inv, rot_dims, adjacent, 1.25)
+    want = torch.full((T, H, R + rotated), float("nan"), dtype=torch.bfloat16, device=dev)
+    ops.head_linear(q, 0, fold, out=want, out_col=0)
+    ops.rotate_part_(q, d, want, R, rotated, positions, inv, rot_dims, adjacent, 1.25)
+    assert torch.equal(got, want)
+
+
 def rel_norm(got, want):
     return float((got - want).norm() / want.norm())

@@ -223,23 +223,13 @@ extern "C" int za_latent_prepare(const void* down, int dtype, int ld, int q_col,
 // dst[t][h][dst_col + i] = rotation of src[t][h][src_col + i], i < Dr (elements beyond
 // rot_dims are copied).  One thread a pair.
 template <typename T>
-__global__ void __launch_bounds__(256)
-rotate_part_kernel(const T* __restrict__ src, int src_ld, int src_col, T* __restrict__ dst,
-                   int dst_ld, int dst_col, int H, int Dr, const int* __restrict__ positions,
-                   const float* __restrict__ inv_freq, int rot_dims, int adjacent, float magnitude,
-                   size_t total) {
-  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= total) return;
-  const int per = Dr - rot_dims / 2;         // pairs, then the elements that pass unchanged
-  const size_t th = idx / per;               // token * H + head
-  const int i = (int)(idx % per);
-  const T* s = src + th * src_ld + src_col;
-  T* d = dst + th * dst_ld + dst_col;
+__device__ __forceinline__ void rotate_pair(const T* s, T* d, int i, int position, const float* __restrict__ inv_freq,
+                                            int rot_dims, int adjacent, float magnitude) {
   const int half = rot_dims / 2;
   if (i < half) {
     const int a = adjacent ? 2 * i : i, b = adjacent ? 2 * i + 1 : i + half;
     float sn, cs;
-    sincosf((float)positions[th / H] * inv_freq[i], &sn, &cs);
+    sincosf((float)position * inv_freq[i], &sn, &cs);
     sn *= magnitude;
     cs *= magnitude;
     const float u = to_f32<T>(s[a]), v = to_f32<T>(s[b]);
@@ -249,6 +239,20 @@ rotate_part_kernel(const T* __restrict__ src, int src_ld, int src_col, T* __rest
     const int e = rot_dims + (i - half);
     d[e] = s[e];
   }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+rotate_part_kernel(const T* __restrict__ src, int src_ld, int src_col, T* __restrict__ dst,
+                   int dst_ld, int dst_col, int H, int Dr, const int* __restrict__ positions,
+                   const float* __restrict__ inv_freq, int rot_dims, int adjacent, float magnitude,
+                   size_t total) {
+  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= total) return;
+  const int per = Dr - rot_dims / 2;         // pairs, then the elements that pass unchanged
+  const size_t th = idx / per;               // token * H + head
+  rotate_pair<T>(src + th * src_ld + src_col, dst + th * dst_ld + dst_col, (int)(idx % per), positions[th / H], inv_freq,
+                 rot_dims, adjacent, magnitude);
 }
 
 extern "C" int za_rotate_part(const void* src, int dtype, int src_ld, int src_col, void* dst,
@@ -289,6 +293,11 @@ struct HeadLinearArgs {
   int T, H, N, K;
   int x_ld, x_col, o_ld, o_col;
   int gate_ld, gate_col, gate_mode;
+  // Dr > 0: a further workgroup a head rotates x's columns rot_src .. into out's columns rot_dst .. (rotate_pair)
+  int Dr, rot_src, rot_dst, rot_dims, adjacent;
+  float magnitude;
+  const int* positions;
+  const float* inv_freq;
 };
 
 template <typename TG>
@@ -314,6 +323,17 @@ head_linear_rows16_kernel(HeadLinearArgs a) {
   const int h = blockIdx.z, n0 = SPLIT ? blockIdx.y * 16 : blockIdx.y * 64 + wave * 16;
   const int r16 = lane & 15, kq = lane >> 4;
   const int K = a.K, N = a.N;
+  if constexpr (!SPLIT && std::is_same<TO, bf16_t>::value)
+    if (a.Dr > 0 && blockIdx.y == gridDim.y - 1) {
+      const int per = a.Dr - a.rot_dims / 2;
+      for (int idx = tid; idx < a.T * per; idx += 256) {
+        const int t = idx / per;
+        const size_t th = (size_t)t * a.H + h;
+        rotate_pair<bf16_t>((const bf16_t*)a.x + th * a.x_ld + a.rot_src, (bf16_t*)a.out + th * a.o_ld + a.rot_dst,
+                            idx - t * per, a.positions[t], a.inv_freq, a.rot_dims, a.adjacent, a.magnitude);
+      }
+      return;
+    }
   const int range = SPLIT ? (K + 127) / 128 * 32 : K, k_lo = SPLIT ? wave * range : 0;
   const int k_end = min(K, k_lo + range);
   const bf16_t* arow = (const bf16_t*)a.x + ((size_t)min(r16, a.T - 1) * a.H + h) * a.x_ld + a.x_col;
@@ -505,7 +525,7 @@ extern "C" int za_head_linear(const void* x, int x_dtype, int x_ld, int x_col, c
       (gate_mode == 2 && (long long)gate_col + (long long)heads * N > gate_ld))
     return ZA_ERR_ARG;
   HeadLinearArgs a{x, W, out, gate, n_tokens, heads, N, K, x_ld, x_col, o_ld, o_col,
-                   gate_ld, gate_col, gate_mode};
+                   gate_ld, gate_col, gate_mode, 0, 0, 0, 0, 0, 0.f, nullptr, nullptr};
   if (w_dtype == 1) {
     if (x_dtype != 1 || K % 8 != 0 || x_ld % 8 != 0 || x_col % 8 != 0 || ((uintptr_t)x | (uintptr_t)W) % 16 != 0)
       return ZA_ERR_UNSUPPORTED;
@@ -536,6 +556,26 @@ extern "C" int za_head_linear(const void* x, int x_dtype, int x_ld, int x_col, c
   else if (x_dtype == 0 && out_dtype == 1) ZA_HF(float, bf16_t);
   else return ZA_ERR_UNSUPPORTED;
 #undef ZA_HF
+  return za_launch_status();
+}
+
+// A decode batch's folded queries in one launch: every head's product of x's columns [0, K) into out's [0, N), and x's
+// columns [K, K + Dr) rotated into out's [N, N + Dr), to the bits of za_head_linear and za_rotate_part, whose second
+// launch took 4 us of a layer (8 rows of 16 heads).  At most 16 tokens, bfloat16, K below HL_SPLIT_MIN_K.
+extern "C" int za_latent_fold(const void* x, int x_ld, const void* W, void* out, int o_ld, int n_tokens, int heads, int N,
+                              int K, int Dr, const int* positions, const float* inv_freq, int rot_dims, int adjacent,
+                              float magnitude, hipStream_t stream) {
+  if (n_tokens == 0) return 0;
+  if (n_tokens < 0 || heads <= 0 || heads > 65535 || N <= 0 || K <= 0 || Dr <= 0 || rot_dims < 0 || rot_dims > Dr ||
+      rot_dims % 2 || !x || !W || !out || K + Dr > x_ld || N + Dr > o_ld || (rot_dims > 0 && (!positions || !inv_freq)))
+    return ZA_ERR_ARG;
+  if (n_tokens > 16 || K >= HL_SPLIT_MIN_K || K % 8 || x_ld % 8 || !positions ||
+      (((uintptr_t)x | (uintptr_t)W) & 15) != 0)
+    return ZA_ERR_UNSUPPORTED;
+  const HeadLinearArgs a{x, W, out, nullptr, n_tokens, heads, N, K, x_ld, 0, o_ld, 0, 0, 0, 0,
+                         Dr, K, N, rot_dims, adjacent, magnitude, positions, inv_freq};
+  hipLaunchKernelGGL((head_linear_rows16_kernel<bf16_t, false>), dim3(1, (unsigned)((N + 63) / 64) + 1, heads), dim3(256),
+                     0, stream, a);
   return za_launch_status();
 }
 

@@ -223,6 +223,8 @@ _SIGNATURES = {
                                       c_int, c_void_p],
     ("latent", "za_rotate_part"): [c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int,
                                    c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
+    ("latent", "za_latent_fold"): [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
+                                   c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
     ("latent_expanded", "za_latent_open_rows"): [
         c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p,
         c_longlong, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
@@ -3246,6 +3248,7 @@ def rotate_part_(src: torch.Tensor, src_col: int, dst: torch.Tensor, dst_col: in
     return dst
 
 
+HEAD_SPLIT_MIN_K = 256     # from here on a decode batch's head products share K out to a workgroup's waves
 HEAD_GATES = {None: 0, "head": 1, "element": 2}
 
 
@@ -3296,6 +3299,38 @@ def head_linear(x: torch.Tensor, x_col: int, weight: torch.Tensor, out: Optional
         _ptr(gate) if gate_mode is not None else None, gate_ld, int(gate_col),
         HEAD_GATES[gate_mode], _stream())
     _check(rc, "head_linear", f"T={T} H={H} N={N} K={K}")
+    return out
+
+
+def latent_fold(q: torch.Tensor, fold: torch.Tensor, rot_dim: int, positions: torch.Tensor,
+                inv_freq: Optional[torch.Tensor], rot_dims: int, adjacent_pairs: bool,
+                magnitude: float = 1.0) -> torch.Tensor:
+    """The folded queries ``[T, heads, rank + rot_dim]`` of ``q [T, heads, d + rot_dim]``: ``fold [heads, rank, d]``
+    times the unrotated part, then the rotated part as ``rotate_part_`` gives it.  A decode batch in bfloat16
+    takes one launch, anything else the two."""
+    _need(q, "q", (torch.float32, torch.bfloat16))
+    if q.dim() != 3 or fold.dim() != 3 or fold.shape[0] != q.shape[1] or fold.shape[2] + rot_dim != q.shape[2]:
+        raise KernelError(f"latent_fold takes q [T, heads, d + {rot_dim}] and fold [heads, rank, d], got "
+                          f"{tuple(q.shape)} and {tuple(fold.shape)}")
+    T, H, ld = q.shape
+    rank, d = fold.shape[1:]
+    out = torch.empty((T, H, rank + rot_dim), dtype=q.dtype, device=q.device)
+    if rot_dim and T <= 16 and q.dtype == fold.dtype == torch.bfloat16 and d < HEAD_SPLIT_MIN_K and d % 8 == 0 \
+            and ld % 8 == 0 and q.data_ptr() % 16 == 0 and fold.data_ptr() % 16 == 0:
+        _need(fold, "fold", torch.bfloat16)
+        _need(positions, "positions", torch.int32, (T,))
+        if rot_dims % 2 or not 0 <= rot_dims <= rot_dim:
+            raise KernelError(f"rot_dims {rot_dims} must be even and at most {rot_dim}")
+        if rot_dims:
+            _need(inv_freq, "inv_freq", torch.float32, (rot_dims // 2,))
+        rc = _fn("latent", "za_latent_fold")(
+            _ptr(q), ld, _ptr(fold), _ptr(out), rank + rot_dim, T, H, rank, d, int(rot_dim), _ptr(positions),
+            _ptr(inv_freq) if rot_dims else None, int(rot_dims), 1 if adjacent_pairs else 0, float(magnitude), _stream())
+        _check(rc, "latent_fold", f"T={T} H={H} N={rank} K={d}")
+        return out
+    head_linear(q, 0, fold, out=out, out_col=0)
+    if rot_dim:
+        rotate_part_(q, d, out, rank, rot_dim, positions, inv_freq, rot_dims, adjacent_pairs, magnitude)
     return out
 
 

@@ -213,11 +213,8 @@ class LatentAttention(Mixer):
             a = self._formed(q, down, plane, step, cache)
             return ops.linear(a.view(T, nh * dv), self.w_out, partial_ok=self.partial_ok, tune=tune)
         # the folded query [Wuk^T q_n | rot(q_r)]
-        qf = torch.empty((T, nh, self.width), dtype=q.dtype, device=q.device)
-        ops.head_linear(q, 0, self.k_fold, out=qf, out_col=0)
-        if dr:
-            ops.rotate_part_(q, d, qf, R, dr, step.positions, self.inv_freq, self.rot_dims,
-                             self.adjacent, self.magnitude)
+        qf = ops.latent_fold(q, self.k_fold, dr, step.positions, self.inv_freq, self.rot_dims, self.adjacent,
+                             self.magnitude)
         item_seq, item_row0, item_count, n_items = step.attention_items(self.rows_per_item)
         waves = 0
         if self.mfma:

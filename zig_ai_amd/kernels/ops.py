@@ -223,6 +223,8 @@ _SIGNATURES = {
                                       c_int, c_void_p],
     ("latent", "za_rotate_part"): [c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int,
                                    c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
+    ("activation", "za_table_gate_linear"): [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p,
+                                             c_int, c_int, c_int, c_int, c_void_p],
     ("latent", "za_latent_fold"): [c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                                    c_void_p, c_void_p, c_int, c_int, c_float, c_void_p],
     ("latent_expanded", "za_latent_open_rows"): [
@@ -3138,6 +3140,30 @@ def table_gate(g: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, col0: in
         _ptr(g), _code(g.dtype), _ptr(ids), _ptr(table), _code(table.dtype), table.shape[0],
         table.shape[1], int(col0), _ptr(out), T, dim, GATE_ACTIVATIONS[activation], _stream())
     _check(rc, "table_gate")
+    return out
+
+
+def table_gate_linear(x: torch.Tensor, weight: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, col0: int,
+                      activation: str, tune: Optional[bool] = None) -> torch.Tensor:
+    """``table_gate`` of ``x weight^T``: a decode batch in bfloat16 takes one kernel, anything else two."""
+    T, K = x.shape
+    dim = weight.shape[0]
+    if T > 16 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or K % 8 or x.data_ptr() % 16 \
+            or weight.data_ptr() % 16:
+        return table_gate(linear(x, weight, tune=tune), ids, table, col0, activation)
+    if activation not in GATE_ACTIVATIONS:
+        raise KernelError(f"activation must be one of {sorted(GATE_ACTIVATIONS)}, got {activation!r}")
+    _need(x, "x", torch.bfloat16, (T, K))
+    _need(weight, "weight", torch.bfloat16, (dim, K))
+    _need(ids, "ids", torch.int32, (T,))
+    _need(table, "table", (torch.float32, torch.bfloat16))
+    if table.dim() != 2 or col0 < 0 or col0 + dim > table.shape[1]:
+        raise KernelError(f"columns [{col0}, {col0 + dim}) of a table {tuple(table.shape)}")
+    out = torch.empty((T, dim), dtype=x.dtype, device=x.device)
+    rc = _fn("activation", "za_table_gate_linear")(
+        _ptr(x), _ptr(weight), _ptr(ids), _ptr(table), _code(table.dtype), table.shape[0], table.shape[1], int(col0),
+        _ptr(out), T, dim, K, GATE_ACTIVATIONS[activation], _stream())
+    _check(rc, "table_gate_linear")
     return out
 
 

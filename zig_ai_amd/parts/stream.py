@@ -141,8 +141,8 @@ class TokenSide(Part):
         x, step.rounded = step.rounded, None
         if x is None:
             x = ops.cast(residual, self.runtime.dtype)
-        g = ops.table_gate(ops.linear(x, self.gate[i], tune=self.runtime.tune), step.token_ids,
-                           self.table, i * self.dim, self.activation)
+        g = ops.table_gate_linear(x, self.gate[i], step.token_ids, self.table, i * self.dim, self.activation,
+                                  tune=self.runtime.tune)
         y = ops.linear(g, self.proj[i], out_dtype=torch.float32, tune=self.runtime.tune)
         ops.normed_add_(residual, y, self.norm[i], self.eps, self.scale)
         return residual, None

@@ -673,16 +673,30 @@ delta_chunk_prepare_kernel(DeltaArgs a) {
   // ---- what the tokens bring (those beyond the chunk change nothing: no decay, nothing written
   // or read): unit q, times dk^(-1/2), and k; decays; write strengths
   const float neg_A = -expf(a.A_log[h]);
-  for (int i = tid; i < DL_CHUNK * DK; i += 256) {
-    const int t = i / DK, c = i % DK;
-    const bool in = t < n && c < dk;
-    const size_t row = row0 + (in ? t : 0);
-    const int ch = in ? c : 0;
-    const float* x = a.conv + row * a.conv_width + grp * dk + ch;
-    qs[t][c] = in ? x[a.q_col] : 0.f;
-    ks[t][c] = in ? x[a.k_col] : 0.f;
-    const float raw = to_f32<T>(((const T*)a.decay)[row * a.decay_stride + h * dk + ch]);
-    gs[t][c] = in ? expf(neg_A * softplus_f(raw + a.dt_bias[h * dk + ch])) : 1.f;
+  {
+    // (All requested before any is waited for, from rows and channels that are there: with a row
+    // asked for once the one before had come, 2,048 tokens of 16 heads of 128 took 77.0 us instead
+    // of 69.6, of 8 heads 40.2 instead of 36.7.)
+    constexpr int PER = DL_CHUNK * DK / 256, ROWS = 256 / DK;
+    const int c = tid % DK, ch = c < dk ? c : 0;
+    float q[PER], k[PER], raw[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const size_t row = row0 + min(tid / DK + i * ROWS, n - 1);
+      const float* x = a.conv + row * a.conv_width + grp * dk + ch;
+      q[i] = x[a.q_col];
+      k[i] = x[a.k_col];
+      raw[i] = to_f32<T>(((const T*)a.decay)[row * a.decay_stride + h * dk + ch]);
+    }
+    const float bias = a.dt_bias[h * dk + ch];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int t = tid / DK + i * ROWS;
+      const bool in = t < n && c < dk;
+      qs[t][c] = in ? q[i] : 0.f;
+      ks[t][c] = in ? k[i] : 0.f;
+      gs[t][c] = in ? expf(neg_A * softplus_f(raw[i] + bias)) : 1.f;
+    }
   }
   if (tid < DL_CHUNK) {
     const float raw = to_f32<T>(((const T*)a.proj)[(size_t)(row0 + min(tid, n - 1)) * a.proj_stride + a.gate_col + h]);

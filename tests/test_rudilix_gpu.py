@@ -744,6 +744,38 @@ def test_ssd_chunks_keep_a_bad_value_from_earlier_tokens(bad, at):
     assert float((got - want)[~after].abs().max()) < 2e-5 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("d,dv", [(128, 128), (40, 24), (16, 16)])
+@pytest.mark.parametrize("last", [1, 17, 32])
+@pytest.mark.parametrize("chunks", [3, 4, 5, 6, 7])
+def test_delta_chunks_far_ahead(chunks, last, d, dv):
+    """A portion of several chunks, walked with the next ones' operands on their way, leaves the bits
+    that its chunks leave one call after the other (the state between them is 32-bit either way)."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator().manual_seed(chunks)
+    H, C = 2, ops.DELTA_CHUNK
+    T = (chunks - 1) * C + last
+    conv = torch.randn(T, 2 * H * d + H * dv, generator=gen).to(dev)
+    proj, raw = torch.randn(T, H, generator=gen).to(dev), torch.randn(T, H * d, generator=gen).to(dev)
+    A_log, bias = torch.full((H,), -2.0, device=dev), torch.zeros(H * d, device=dev)
+    start = torch.randn(H * d * dv, generator=gen).to(dev)
+
+    def run(portions):
+        _, state = _slots(2, H * d * dv, dev)
+        state[1] = start
+        out, at = [], 0
+        for n in portions:
+            rows = slice(at, at + n)
+            out.append(ops.delta_recurrence_chunked(
+                conv[rows], 0, H * d, 2 * H * d, proj[rows], 0, raw[rows], bias, A_log, state, 0,
+                torch.tensor([1], dtype=torch.int32, device=dev), _chunk_items([n], C, dev), H, H, d, dv))
+            at += n
+        return torch.cat(out), state
+
+    (whole, state), (parts, want) = run([T]), run([C] * (chunks - 1) + [last])
+    assert torch.equal(whole, parts) and torch.equal(state, want)
+
+
 @pytest.mark.parametrize("bad", [math.nan, math.inf])
 @pytest.mark.parametrize("at", [5, 16, 20, 31, 40, 69])
 def test_delta_chunks_keep_a_bad_value_from_earlier_tokens(bad, at):

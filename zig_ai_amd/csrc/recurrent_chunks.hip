@@ -878,7 +878,7 @@ delta_chunk_prepare_kernel(DeltaArgs a) {
 // (or one) tiles of 16 rows each, and its image in LDS, where all eight read it as an operand (a
 // lane's four rows side by side, as the products leave them); a chunk is two products with the
 // state, W B for u and (P q) B for o, each over two blocks of tokens and, in halves, over the
-// rows, then the products with u.  Two barriers a chunk, the next two chunks' operands on their way.
+// rows, then the products with u.  Two barriers a chunk, the next three chunks' operands on their way.
 // FULL: dk fills its tiles and dv its 16 columns.
 template <int NT, bool FULL>
 __global__ void __launch_bounds__(512)
@@ -921,8 +921,9 @@ delta_chunk_walk_kernel(DeltaArgs a) {
   }
 
   const int begin = a.item_row0[first], end = a.item_row0[last - 1] + a.item_count[last - 1];
-  // A chunk's operands are requested two chunks ahead: with one the way from memory outlasts a
-  // chunk.  A use of some waits for a known number of later requests, so every chunk of a role makes
+  // A chunk's operands are requested three chunks ahead: with one the way from memory outlasts a
+  // chunk, and two leave 2,048 tokens of 16 heads of 128 at 126 us where three take 119 (8 heads 123
+  // and 117; without any loads 84: the chain of products and barriers).  A use of some waits for a known number of later requests, so every chunk of a role makes
   // the same ones (beyond the last chunk for that one again).  A lane's places within a chunk; where
   // a chunk lies is the same for all lanes.  (The rows of a last chunk that has fewer than 32 are
   // there, but hold nothing: no use of them reaches a result.)
@@ -990,19 +991,22 @@ delta_chunk_walk_kernel(DeltaArgs a) {
 #pragma unroll
         for (int o = 0; o < OWN; ++o) Bs[wave * OWN + o][lane] = S[o];
       }
-      request(min(item + 2, last - 1), x);
+      request(min(item + 3, last - 1), x);
       lds_barrier();
     };
-    Operands x, y;
+    Operands x, y, z;
     request(first, x);
     request(min(first + 1, last - 1), y);
+    request(min(first + 2, last - 1), z);
     lds_barrier();
     int item = first;
-    for (; item + 1 < last; item += 2) {
+    for (; item + 2 < last; item += 3) {
       chunk(item, x);
       chunk(item + 1, y);
+      chunk(item + 2, z);
     }
     if (item < last) chunk(item, x);
+    if (item + 1 < last) chunk(item + 1, y);
   } else {
     struct Operands {
       f32x4_t left[HT], q;
@@ -1022,7 +1026,7 @@ delta_chunk_walk_kernel(DeltaArgs a) {
       }
       p = mfma4(x.q, u, p);
       if (half == 1) late[block][lane] = p;
-      request(min(item + 2, last - 1), x);
+      request(min(item + 3, last - 1), x);
       lds_barrier();
       if (half == 0 && col_ok) {
         p += late[block][lane];
@@ -1033,16 +1037,19 @@ delta_chunk_walk_kernel(DeltaArgs a) {
           if (t + i < end) o[(size_t)i * a.H * dv] = p[i];
       }
     };
-    Operands x, y;
+    Operands x, y, z;
     request(first, x);
     request(min(first + 1, last - 1), y);
+    request(min(first + 2, last - 1), z);
     lds_barrier();
     int item = first;
-    for (; item + 1 < last; item += 2) {
+    for (; item + 2 < last; item += 3) {
       chunk(item, x);
       chunk(item + 1, y);
+      chunk(item + 2, z);
     }
     if (item < last) chunk(item, x);
+    if (item + 1 < last) chunk(item + 1, y);
   }
   if (!has_rows || !col_ok) return;
 #pragma unroll

@@ -1919,6 +1919,52 @@ def test_repetition_penalty():
     assert torch.allclose(work.cpu(), torch.tensor([[1.0, -4.0, 0.0, 4.0], [1.0 / 1.5, 1.0, -1.0, -4.0]]))
 
 
+@pytest.mark.parametrize("E,top,T", [(4, 2, 1), (4, 2, 20), (4, 2, 60), (4, 4, 79), (7, 3, 40)])
+@pytest.mark.parametrize("N,K", [(4104, 1032), (8200, 576)])
+def test_large_expert_weights_read_past_the_caches(E, top, T, N, K):
+    """Experts' weights of 32 MB and more, each height of tile: the bits that their rows give in parts
+    small enough to stay in the caches."""
+    o = ops()
+    assert E * N * K * 2 >= 32 << 20 > E * N // 4 * K * 2
+    gen = torch.Generator().manual_seed(E * T)
+    chosen = torch.stack([torch.randperm(E, generator=gen)[:top] for _ in range(T)]).int()
+    lists, counts = o.expert_lists(None, chosen.to(dev()), T, E)
+    x, w = rand((T, K), torch.bfloat16, 70).to(dev()), rand((E, N, K), torch.bfloat16, 71, K ** -0.5).to(dev())
+    for out in (torch.float32, torch.bfloat16):
+        whole = o.grouped_linear(x, w, lists, counts, T, per_token=True, out_dtype=out)
+        parts = [o.grouped_linear(x, part.contiguous(), lists, counts, T, per_token=True, out_dtype=out)
+                 for part in w.split(N // 8, 1)]
+        assert torch.equal(whole, torch.cat(parts, 1))
+        whole = o.grouped_linear(x, w, lists, counts, T, per_token=True, out_dtype=out, gate="silu")
+        parts = [o.grouped_linear(x, torch.cat(part, 1), lists, counts, T, per_token=True, out_dtype=out, gate="silu")
+                 for part in zip(w[:, :N // 2].split(N // 8, 1), w[:, N // 2:].split(N // 8, 1))]
+        assert torch.equal(whole, torch.cat(parts, 1))
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(8200, 2056), (4104, 8192)])
+def test_large_weights_read_past_the_caches(M, N, K):
+    """The same for a decode batch's product with one weight, in ranges of K and gated."""
+    o = ops()
+    x, w = rand((M, K), torch.bfloat16, 70).to(dev()), rand((N, K), torch.bfloat16, 71, K ** -0.5).to(dev())
+
+    def product(weight, ranges, gated):
+        n = weight.shape[0] // (2 if gated else 1)
+        out = torch.empty((ranges, M, n) if not gated else (M, n),
+                          dtype=torch.bfloat16 if gated else torch.float32, device=dev())
+        assert o._fn("gemm_tiles", "za_gemm_bf16_tiles")(
+            o._ptr(x), o._ptr(weight), o._ptr(out), o._code(out.dtype), M, n, K, ranges, 1 if gated else 0, 0,
+            o._stream()) == 0
+        return out
+
+    for ranges in (1, 3):
+        assert torch.equal(product(w, ranges, False),
+                           torch.cat([product(part, ranges, False) for part in w.split(N // 4)], 2))
+    assert torch.equal(product(w, 1, True), torch.cat(
+        [product(torch.cat(part), 1, True)
+         for part in zip(w[:N // 2].split(N // 8), w[N // 2:].split(N // 8))], 1))
+
+
 # ------------------------------------------------------------------- experts
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("E,top,N,K,T", [(8, 2, 72, 64, 1), (8, 3, 130, 200, 40), (3, 1, 256, 192, 200),

@@ -103,10 +103,12 @@ __device__ __forceinline__ unsigned lds_address(const void* p) {
 // The wait for all but the last n requests to memory.
 #define ZA_VMCNT(n) (((n) & 15) | (7 << 4) | (15 << 8) | (((n) >> 4) << 14))
 
-// 16 bytes a lane: from each lane's `from` to `to`, one lane's behind the other's.
+// 16 bytes a lane: from each lane's `from` to `to`, one lane's behind the other's.  ONCE: whole lines that nothing
+// reads again (non-temporal).
+template <bool ONCE = false>
 __device__ __forceinline__ void lds_request(const void* from, void* to) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
-                                   (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+                                   (__attribute__((address_space(3))) void*)to, 16, 0, ONCE ? 2 : 0);
 }
 
 static inline int za_launch_status() { return (int)hipGetLastError(); }

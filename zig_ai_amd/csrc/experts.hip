@@ -255,10 +255,10 @@ __device__ __forceinline__ void grouped_store(const GroupedArgs& g, const int* _
 
 // Tiles of BM assignments x BN weight rows (tiles_bf16.h).
 // GATED: a tile is BN / 2 outputs; its weight rows are gate and up rows in turn, 16 each.
-template <typename TO, bool GATED, int BM, int BN, int NS>
+template <typename TO, bool GATED, int BM, int BN, int NS, bool ONCE>
 __global__ void __launch_bounds__(256, 2)
 grouped_gemm_bf16_tiled_kernel(GroupedArgs g) {
-  using Tiles = TilesBf16<BM, BN, NS>;
+  using Tiles = TilesBf16<BM, BN, NS, ONCE>;
   constexpr int WM = Tiles::WM, WN = Tiles::WN, TM = Tiles::TM, TN = Tiles::TN, LA = Tiles::LA, LW = Tiles::LW;
   __shared__ __attribute__((aligned(16))) bf16_t As[NS][BM * GG_BK];
   __shared__ __attribute__((aligned(16))) bf16_t Ws[NS][BN * GG_BK];
@@ -626,14 +626,29 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     const long long rows = (A + BM - 1) / BM + experts, blocks = (rows + 7) / 8 * 8 * ((N + columns - 1) / columns);
     if (blocks > 0x7fffffffLL) return ZA_ERR_ARG;
     const dim3 grid((unsigned)blocks);
-#define ZA_GT(TO, GATED, BM, BN, NS) \
-  hipLaunchKernelGGL((grouped_gemm_bf16_tiled_kernel<TO, GATED, BM, BN, NS>), grid, dim3(256), 0, stream, g)
+    // Weights that few rows read: past the caches' other contents, where the experts have more than a
+    // model that stays in the last level's cache (256 MB) would give one product.  Weights of four
+    // layers or more in turn, gate|up and down, before and after (us): 8 experts of 4,096 over 2,048, 2 a
+    // token, 20 tokens 70.2 + 31.6 and 62.9 + 27.6, 150 tokens 65.7 + 42.7 and 60.0 + 39.4; 32 experts of
+    // 1,024, 4 a token, 64 tokens 56.1 + 29.8 and 49.9 + 26.5, 400 tokens 73.3 + 33.3 and 67.4 + 30.6,
+    // one token 13.6 + 8.6 and 13.6 + 8.3 (only where 200 MB of its experts were still cached 11.0 +
+    // 7.2 became 13.1 + 8.3: smaller sets than 32 MB, which may stay there, are left in).
+    const bool once = A < 80LL * experts && (gate ? 2LL : 1LL) * experts * N * K * 2 >= ZA_ONCE_BYTES;
+#define ZA_GT(TO, GATED, BM, BN, NS)                                                                                \
+  {                                                                                                                 \
+    if (once)                                                                                                       \
+      hipLaunchKernelGGL((grouped_gemm_bf16_tiled_kernel<TO, GATED, BM, BN, NS, true>), grid, dim3(256), 0, stream, \
+                         g);                                                                                        \
+    else                                                                                                            \
+      hipLaunchKernelGGL((grouped_gemm_bf16_tiled_kernel<TO, GATED, BM, BN, NS, false>), grid, dim3(256), 0,        \
+                         stream, g);                                                                                \
+  }
 #define ZA_GT_ROWS(TO, GATED)                                      \
   {                                                                \
-    if (BM == 128 && blocks <= 256) ZA_GT(TO, GATED, 128, 128, 3); \
-    else if (BM == 128) ZA_GT(TO, GATED, 128, 128, 2);             \
-    else if (BM == 64) ZA_GT(TO, GATED, 64, 128, 3);               \
-    else ZA_GT(TO, GATED, 32, 64, 4);                              \
+    if (BM == 128 && blocks <= 256) ZA_GT(TO, GATED, 128, 128, 3)  \
+    else if (BM == 128) ZA_GT(TO, GATED, 128, 128, 2)              \
+    else if (BM == 64) ZA_GT(TO, GATED, 64, 128, 3)                \
+    else ZA_GT(TO, GATED, 32, 64, 4)                               \
   }
     if (out_dtype == 0) { if (gate) ZA_GT_ROWS(float, true) else ZA_GT_ROWS(float, false) }
     else { if (gate) ZA_GT_ROWS(bf16_t, true) else ZA_GT_ROWS(bf16_t, false) }

@@ -29,11 +29,11 @@ __device__ __forceinline__ float gt_unit(int act, float g, float u) {
   return 0.5f * g * (1.0f + tanhf(z)) * u;
 }
 
-template <typename TO, bool GATED, int BM, int NS>
+template <typename TO, bool GATED, int BM, int NS, bool ONCE>
 __global__ void __launch_bounds__(256)
 gemm_bf16_tiles_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, TO* __restrict__ out,
                        int M, int N, int K, int range, int act) {
-  using Tiles = TilesBf16<BM, GT_BN, NS>;
+  using Tiles = TilesBf16<BM, GT_BN, NS, ONCE>;
   __shared__ __attribute__((aligned(16))) bf16_t As[NS][BM * GG_BK];
   __shared__ __attribute__((aligned(16))) bf16_t Ws[NS][GT_BN * GG_BK];
   const int n0 = blockIdx.x * (GATED ? GT_BN / 2 : GT_BN), k0 = blockIdx.y * range;
@@ -98,20 +98,30 @@ extern "C" int za_gemm_bf16_tiles(const void* x, const void* W, void* out, int o
     return ZA_ERR_UNSUPPORTED;
   const int per = gated ? GT_BN / 2 : GT_BN;
   dim3 grid((unsigned)((N + per - 1) / per), (unsigned)ranges);
+  // Large weights past the caches' other contents (us, before and after, in a decode step of 64 tokens of the
+  // 2,048-wide hybrid: gate|up 67 MB 18.6 and 17.0, down 33 MB 10.2 and 9.7, head 268 MB 63.1 and
+  // 60.6; of 20 tokens 8,192 x 2,048 8.9 and 8.4, head 53.4 and 48.8; 12 MB 9.5 and 9.7, 8 MB 5.6 and 5.8).
+  const bool once = (gated ? 2LL : 1LL) * N * K * 2 >= ZA_ONCE_BYTES;
 #define ZA_GT(TO, GATED, BM, NS)                                                                      \
-  hipLaunchKernelGGL((gemm_bf16_tiles_kernel<TO, GATED, BM, NS>), grid, dim3(256), 0, stream,         \
-                     (const bf16_t*)x, (const bf16_t*)W, (TO*)out, M, N, K, range, act)
+  {                                                                                                   \
+    if (once)                                                                                         \
+      hipLaunchKernelGGL((gemm_bf16_tiles_kernel<TO, GATED, BM, NS, true>), grid, dim3(256), 0,       \
+                         stream, (const bf16_t*)x, (const bf16_t*)W, (TO*)out, M, N, K, range, act);  \
+    else                                                                                              \
+      hipLaunchKernelGGL((gemm_bf16_tiles_kernel<TO, GATED, BM, NS, false>), grid, dim3(256), 0,      \
+                         stream, (const bf16_t*)x, (const bf16_t*)W, (TO*)out, M, N, K, range, act);  \
+  }
   // (65536 x 2048, 64 rows: 63.8 us with five places in LDS, 67.6 with four; in ranges four
   // are as good or better: 9.8 against 10.0)
   if (M <= 32) {
-    if (gated) ZA_GT(bf16_t, true, 32, 6);
-    else if (out_dtype == 0) ZA_GT(float, false, 32, 6);
-    else ZA_GT(bf16_t, false, 32, 6);
+    if (gated) ZA_GT(bf16_t, true, 32, 6)
+    else if (out_dtype == 0) ZA_GT(float, false, 32, 6)
+    else ZA_GT(bf16_t, false, 32, 6)
   } else {
-    if (gated) ZA_GT(bf16_t, true, 64, 4);
-    else if (ranges > 1) ZA_GT(float, false, 64, 4);
-    else if (out_dtype == 0) ZA_GT(float, false, 64, 5);
-    else ZA_GT(bf16_t, false, 64, 5);
+    if (gated) ZA_GT(bf16_t, true, 64, 4)
+    else if (ranges > 1) ZA_GT(float, false, 64, 4)
+    else if (out_dtype == 0) ZA_GT(float, false, 64, 5)
+    else ZA_GT(bf16_t, false, 64, 5)
   }
 #undef ZA_GT
   return za_launch_status();

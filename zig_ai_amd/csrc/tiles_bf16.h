@@ -13,7 +13,7 @@
 // waves, takes its fragments, requests the tiles NS - 1 steps on, into the place the step before it
 // has left, and multiplies meanwhile: one barrier a step, NS - 1 steps' tiles under way.  With few
 // rows the weights' way from memory bounds it, with many the reads of LDS, which take as long as
-// the products (tiles of 64 x 64 a wave).  The rows of W are the first operand, so a lane ends with
+// the products (tiles of 64 x 64 a wave).  ONCE: the weights are read past the caches' other contents.  The rows of W are the first operand, so a lane ends with
 // four consecutive outputs of one row of A.
 #pragma once
 
@@ -21,7 +21,11 @@
 
 #define GG_BK 64
 
-template <int BM, int BN, int NS>
+// A product whose weights take this many bytes or more is not one of a model that the last level's cache
+// (256 MB) could hold from one step to the next.
+#define ZA_ONCE_BYTES (32LL << 20)
+
+template <int BM, int BN, int NS, bool ONCE = false>
 struct TilesBf16 {
   static constexpr int WM = BM >= 64 || BN == 64 ? 2 : 1, WN = 4 / WM;   // waves along the rows of A and of W
   static constexpr int TM = BM / (16 * WM), TN = BN / (16 * WN);
@@ -41,7 +45,7 @@ struct TilesBf16 {
 #pragma unroll
       for (int i = 0; i < LA; ++i) lds_request(arow[i] + k0, &As[p][(32 * i + wave * 8) * GG_BK]);
 #pragma unroll
-      for (int i = 0; i < LW; ++i) lds_request(wrow[i] + k0, &Ws[p][(32 * i + wave * 8) * GG_BK]);
+      for (int i = 0; i < LW; ++i) lds_request<ONCE>(wrow[i] + k0, &Ws[p][(32 * i + wave * 8) * GG_BK]);
     };
 #pragma unroll
     for (int i = 0; i < TM; ++i)

@@ -210,6 +210,19 @@ class Forms:
             probabilities=bool(self.kernels - {"plain"}))
 
 
+class FormedKeys:
+    """Collects, as ``forms`` of ``run_schedule``, which steps attended to keys and values formed from the latent
+    rows in every latent layer (``True``), in none (``False``)."""
+
+    def __init__(self, layers):
+        self.layers, self.steps = layers, []
+
+    def note_step(self, entries, wanted_rows, log):
+        formed = sum(r.get("kernel") == "latent_expanded" for r in log)
+        assert formed in (0, self.layers), (entries, formed)
+        self.steps.append((entries, formed > 0))
+
+
 def run_schedule(runner, prompts, schedule, wants=None, forms=None, streams=None):
     """Drive ``runner`` through ``schedule`` asking for the logits of every token (or, with
     ``wants``, of the positions ``wants[i]`` of request ``i``); returns one ``[wanted,

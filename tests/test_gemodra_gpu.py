@@ -382,6 +382,45 @@ def test_sinks_that_take_most_of_the_weight(kind):
             assert worst(g, w) < F32_BOUND
 
 
+# ------------------------------------------- keys and values formed from the latent rows
+# heads of 128, rotated and not, gates of either kind
+FORMED = gu.config([
+    gu.layer("latent_attention", gu.latent(heads=2, dim=128, vdim=128, kv_rank=64, q_rank=24, rot_dim=64,
+                                           rot_dims=32, base=1e4), None),
+    gu.layer("latent_attention_2", gu.plain_latent(heads=3, dim=128, vdim=128, kv_rank=40, q_rank=16), None)])
+
+
+def test_recorded_portions_take_one_form(monkeypatch):
+    """Where portions are recorded, a shape's first step, the recorded one with other contexts behind it, and a step
+    of that shape with taps all take the kernels that do not hang on the contexts' lengths; larger steps, which
+    are never recorded, form keys and values."""
+    from zig_ai_amd.engine import ModelRunner, graphs
+    model, tensors = build(FORMED, seed=8, dtype="bfloat16")
+    prompts = [gu.tokens(120, FORMED["vocab"], 1), gu.tokens(200, FORMED["vocab"], 2)]
+    want = plain_logits(FORMED, tensors, prompts)
+    monkeypatch.setattr(graphs, "PORTION_GRAPH_MAX_TOKENS", 64)
+    make = lambda on: ModelRunner(model, page_size=16, num_pages=32, num_slots=2, portion_graphs=on)
+    recorded, plain_run = make(True), make(False)
+    schedule = [([(0, a, a + 40)], [0] if a == 80 else []) for a in (0, 40, 80)] + \
+        [([(1, a, a + 100)], [1] if a else []) for a in (0, 100)]
+    small = lambda forms: {formed for entries, formed in forms.steps if entries[0][0] == 0}
+    large = lambda forms: {formed for entries, formed in forms.steps if entries[0][0] == 1}
+    first = None
+    for _ in range(3):
+        forms = eu.FormedKeys(2)
+        got = eu.run_schedule(recorded, prompts, schedule, forms=forms)
+        assert small(forms) == {False} and large(forms) == {True}
+        assert_bfloat16_close(torch.cat(got), torch.cat(want))
+        first = first or got
+        # (every sum of the two runs is the same but for the cut of the contexts into ranges)
+        assert worst(torch.cat(got), torch.cat(first)) < 0.02
+    assert recorded.graphs.portion_captures == 1 and recorded.graphs.portion_replays == 8
+    for runner, formed in ((recorded, False), (plain_run, True)):
+        forms = eu.FormedKeys(2)
+        eu.run_schedule(runner, prompts, schedule[:3], forms=forms, streams={})
+        assert small(forms) == {formed}
+
+
 # -------------------------- a long context: ranges of keys, merged, with the sink once
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_long_context_in_ranges(dtype):

@@ -78,9 +78,10 @@ class StepContext:
     host: Optional[np.ndarray] = None
     offsets: Dict[str, Tuple[int, int]] = field(default_factory=dict)
     table_width: int = 0
-    # the step's arrays lie in a buffer that is filled again before every replay of a recording: sizes that
-    # follow from the contexts' lengths on the host would be those of the recorded step
-    replayed: bool = False
+    # steps of this shape may be recorded and replayed (this one, or a later one: a shape's first step runs as it
+    # is): sizes that follow from the contexts' lengths on the host would be those of the recorded step, so nothing
+    # may hang on them, and the steps that are not replayed do as the replayed ones
+    recordable: bool = False
     # diagnostics: when a dict, the part that is running may leave copies of its
     # intermediate tensors in it by name (token rows first); see DecoderModel.forward
     taps: Optional[Dict[str, torch.Tensor]] = None
@@ -235,7 +236,8 @@ def build_step(entries: Sequence[StepEntry], cache: CacheManager, device: torch.
                max_position: int = 0, min_pages: int = 0, max_keys: int = 0,
                into: Optional[torch.Tensor] = None,
                staging=None,
-               prepared: Optional[PreparedEntries] = None) -> StepContext:
+               prepared: Optional[PreparedEntries] = None,
+               recordable: bool = False) -> StepContext:
     """Lay out the step.  Every request must be admitted and its pages for this
     step reserved beforehand; nothing is committed here.
 
@@ -248,7 +250,7 @@ def build_step(entries: Sequence[StepEntry], cache: CacheManager, device: torch.
     that does not block; the caller waits for that copy before it lays out the
     next step there; a ``StagingRing`` in its place hands out such buffers in turn and a new
     device buffer is filled from them.  ``prepared``: the same entries, already turned
-    into arrays."""
+    into arrays.  ``recordable``: see ``StepContext`` (a step laid out in ``into`` is)."""
     prep = prepared if prepared is not None else PreparedEntries(entries, cache, vocab_size)
     S = len(entries)
     counts, meta = prep.counts, prep.meta
@@ -311,7 +313,7 @@ def build_step(entries: Sequence[StepEntry], cache: CacheManager, device: torch.
         seq_start=view("seq_start"), ctx_len=view("ctx_len"), slot_id=view("slot_id"),
         logit_rows=view("logit_rows"),
         seq_lens_host=seq_lens, ctx_lens_host=ctx_lens, slots_host=slots,
-        host=host, offsets=offsets, table_width=max_pages, replayed=into is not None)
+        host=host, offsets=offsets, table_width=max_pages, recordable=recordable or into is not None)
     for g in groups:
         ctx.slot_mapping[g.index] = view(f"slots{g.index}")
         ctx.block_tables[g.index] = view(f"table{g.index}").view(S, max_pages)

@@ -303,7 +303,8 @@ class DecodeGraphs:
                     self.portion_entries.pop(old)
             self.portion_entries[key] = {"graph": None, "seen": 1, "bytes": 0}
             ctx = build_step(entries, cache, runner.device, self._vocab, self._granularities,
-                             self._max_position, prepared=prepared, staging=runner.staging)
+                             self._max_position, prepared=prepared, staging=runner.staging,
+                             recordable=True)
             return model.forward(ctx, runner.views)
         self.portion_entries[key] = self.portion_entries.pop(key)      # now the most recently used
         if slot["graph"] is None:

@@ -19,6 +19,7 @@ from typing import Callable, Hashable, List, Optional, Sequence
 import torch
 
 from ..cache.pages import OutOfPages, OutOfSlots
+from . import graphs
 from .batch import StagingRing, StepContext, StepEntry, StepError, build_step
 from .graphs import DecodeGraphs
 from .model import DecoderModel
@@ -123,9 +124,12 @@ class ModelRunner:
     def prepare(self, entries: Sequence[StepEntry]) -> StepContext:
         """Reserve pages for the entries and lay out the step."""
         self.reserve(entries)
+        # (a step of a shape that is recorded may come here as well, for its taps)
+        recordable = self.graphs is not None and self.portion_graphs \
+            and sum(len(e.tokens) for e in entries) <= graphs.PORTION_GRAPH_MAX_TOKENS
         return build_step(entries, self.cache, self.device, self.model.spec.vocab_size,
                           self.model.item_granularities, self.model.spec.max_position,
-                          staging=self.staging)
+                          staging=self.staging, recordable=recordable)
 
     def step(self, entries: Sequence[StepEntry],
              taps: Optional[list] = None) -> torch.Tensor:

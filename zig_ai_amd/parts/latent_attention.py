@@ -208,7 +208,7 @@ class LatentAttention(Mixer):
                                 self.inv_freq, self.rot_dims, self.adjacent,
                                 plane if cache.writes else None, self.magnitude)
         q = ops.linear(cq, self.w_q_up, tune=tune).view(T, nh, d + dr)
-        if self.w_form is not None and not step.replayed \
+        if self.w_form is not None and not step.recordable \
                 and forming_pays(step.seq_lens_host, step.ctx_lens_host, 2 * nh * (d + dv)):
             a = self._formed(q, down, plane, step, cache)
             return ops.linear(a.view(T, nh * dv), self.w_out, partial_ok=self.partial_ok, tune=tune)

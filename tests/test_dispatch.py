@@ -155,3 +155,17 @@ def test_how_far_portions_over_planes_are_cut():
     assert planes_target(128, 64, 1028, False, True) == planes_target(64, 64, 3000, False, False) == least
     assert planes_target(128, 64, 700, True, False) == planes_target(192, 96, 3000, True, False) == least
     assert planes_target(136, 64, 3000, False, False) == planes_target(128, 104, 3000, True, False) == least
+
+
+@pytest.mark.parametrize("outputs,rank", [(4096, 512), (4096, 128), (32768, 512), (2560, 1024)])
+def test_how_many_rows_keys_and_values_are_formed_for(outputs, rank):
+    """Any sum of contexts leaves the library few numbers of rows, none of them far more than there are."""
+    from zig_ai_amd.parts.latent_attention import FORMING_BLOCK, forming_rows
+    asked = set()
+    for rows in range(1, 33000):
+        room = forming_rows(rows, outputs, rank)
+        assert rows <= room < rows + max(FORMING_BLOCK, rows / 4)
+        assert forming_rows(room, outputs, rank) == room
+        if room > FORMING_BLOCK and not ops.half_plan(room, outputs, rank, False)[0]:
+            asked.add(room)
+    assert len(asked) <= 25

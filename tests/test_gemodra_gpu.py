@@ -421,6 +421,55 @@ def test_recorded_portions_take_one_form(monkeypatch):
         assert small(forms) == {formed}
 
 
+def test_forming_with_rows_to_spare(monkeypatch):
+    """Keys and values formed for more rows than there are, whatever memory holds there: the logits of just as many."""
+    from zig_ai_amd.parts import latent_attention
+    model, tensors = build(FORMED, seed=8, dtype="bfloat16")
+    lengths = [190, 33]
+    prompts = [gu.tokens(n, FORMED["vocab"], 1 + i) for i, n in enumerate(lengths)]
+    want = plain_logits(FORMED, tensors, prompts)
+    schedule = [([(0, 0, 64)], []), ([(0, 64, 96), (1, 0, 33)], [1]), ([(0, 96, 129)], []), ([(0, 129, 190)], [0])]
+    got = []
+    for block in (256, 16, 100):
+        monkeypatch.setattr(latent_attention, "FORMING_BLOCK", block)
+        for size in (1 << 16, 1 << 14):      # (memory that the next tensors are likely to get)
+            torch.full((size,), float("nan"), dtype=torch.bfloat16, device="cuda")
+        forms = eu.FormedKeys(2)
+        got.append(torch.cat(eu.run_schedule(runner_for(model, page_size=16, tokens=256), prompts, schedule,
+                                             forms=forms)))
+        assert all(formed for _, formed in forms.steps)
+        assert_bfloat16_close(got[-1], torch.cat(want), block)
+        assert_bfloat16_same_run(got[-1], got[0], block)
+
+
+def test_forming_meets_no_row_count_that_warm_up_has_not(monkeypatch):
+    """A long prompt in portions behind an engine's warm-up: the GEMM library is asked to form keys and values for no
+    number of rows that it has not planned, however long the contexts get."""
+    from zig_ai_amd.engine import Engine
+    from zig_ai_amd.engine.model import walk_parts
+    from zig_ai_amd.kernels import ops
+    cfg = gu.config([gu.layer("latent_attention", gu.latent(heads=16, dim=128, vdim=128, kv_rank=128, q_rank=24,
+                                                            rot_dim=64, base=1e4), None)])
+    model, _ = build(cfg, seed=8, dtype="bfloat16")
+    weight_of = [p.w_form for b in model.blocks for part in b.parts.values() for p in walk_parts(part)
+                 if hasattr(p, "w_form")]
+    assert len(weight_of) == 1
+    met, library = set(), ops._library_matmul
+
+    def counted(x, weight, *more, **named):
+        if weight is weight_of[0]:
+            met.add(x.shape[0])
+        return library(x, weight, *more, **named)
+
+    monkeypatch.setattr(ops, "_library_matmul", counted)
+    engine = Engine(model, page_size=16, num_pages=256, max_num_seqs=2, max_num_batched_tokens=512)
+    planned = set(met)
+    assert {256 * k for k in range(1, 9)} | {2560, 3072, 3584, 4096, 5120, 8192} <= planned
+    met.clear()
+    engine.generate([gu.tokens(3100, cfg["vocab"], 1)], max_new_tokens=2, temperature=0.0, eos_token_id=-1)
+    assert len(met) >= 4 and met <= planned, (met, planned)
+
+
 # -------------------------- a long context: ranges of keys, merged, with the sink once
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_long_context_in_ranges(dtype):

@@ -87,7 +87,7 @@ latent_open_rows_kernel(OpenRowsArgs a) {
   }
 }
 
-// n_rows: the sum of ctx_len and the step's tokens; rot_dims may be smaller than Dr.
+// n_rows: the sum of ctx_len and the step's tokens, or more; rot_dims may be smaller than Dr.
 extern "C" int za_latent_open_rows(void* q, int q_ld, int q_col, int n_tokens, int H, int Dr, const int* positions,
                                    const float* inv_freq, int rot_dims, int adjacent, float magnitude,
                                    const void* plane, long long page_stride, const int* block_table, int bt_stride,
@@ -368,7 +368,7 @@ static int launch_latent_expanded(const LxArgs& a, hipStream_t stream) {
 }
 
 // Work items of at most LX_ROWS consecutive tokens of one request; `kv` and `rot` hold every request's visible rows, one
-// request's behind the other's (ctx_len of them, then its tokens), n_rows in all.
+// request's behind the other's (ctx_len of them, then its tokens), n_rows in all or fewer.
 extern "C" int za_latent_expanded(const void* q, const void* kv, const void* rot, int n_rows, void* out,
                                   const int* positions, const int* wi_seq, const int* wi_row0, const int* wi_count,
                                   const int* seq_start, const int* ctx_len, int n_items, int H, int Dr, float scale,

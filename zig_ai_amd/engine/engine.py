@@ -153,6 +153,9 @@ class Engine:
                 steps += 1
             finally:
                 runner.release(name)
+        for part in top:
+            for p in walk_parts(part):
+                p.warm_up(self.max_num_batched_tokens)
         torch.cuda.synchronize(rt.device)
         return steps
 

@@ -3441,7 +3441,7 @@ def latent_open_rows(q: torch.Tensor, q_col: int, rot_dim: int, positions: torch
                      ctx_len: torch.Tensor, n_rows: int):
     """``(latents [n_rows, kv_rank], rotated key parts [n_rows, rot_dim] or None)``: every request's
     cached rows, its ``ctx_len`` earlier ones and this step's (already written), one request's behind
-    the other's; ``n_rows`` is their number.  ``q[t, h, q_col : q_col + rot_dim]`` is rotated in place
+    the other's; ``n_rows`` is their number or more (what lies behind them is not written).  ``q[t, h, q_col : q_col + rot_dim]`` is rotated in place
     (its first ``rot_dims`` elements, as ``rotate_part_`` does)."""
     _need(q, "q", torch.bfloat16)
     if q.dim() != 3 or q_col < 0 or q_col + rot_dim > q.shape[2]:

@@ -142,6 +142,10 @@ class Part:
 
     kind: str = ""
 
+    def warm_up(self, step_tokens: int) -> None:
+        """Run the part's products at the row counts that steps of up to ``step_tokens`` tokens meet only behind
+        cached ones, so that no request waits while the GEMM library plans and times them (``Engine.warm_up``)."""
+
     @classmethod
     def tensor_rules(cls, params: Mapping[str, Any]) -> Dict[str, TensorRule]:
         return {}

@@ -86,6 +86,27 @@ def forming_pays(seq_lens, ctx_lens, bytes_a_row: int) -> bool:
     return min(seq_lens) > 1 and rows <= FORMING_ROWS_A_TOKEN * sum(seq_lens) and rows * bytes_a_row <= FORMING_BYTES
 
 
+FORMING_BLOCK = 256      # rows
+
+
+def forming_block(rows: int) -> int:
+    """What ``rows`` are rounded up to a multiple of: an eighth of the power of two at or above them."""
+    return max(FORMING_BLOCK, 1 << max((rows - 1).bit_length() - 3, 0))
+
+
+def forming_rows(rows: int, outputs: int, kv_rank: int) -> int:
+    """The rows that the forming product is asked for: ``rows``, which is any sum of contexts, or more.  The GEMM
+    library plans every row count that it meets, and times its candidates for every block of them (10 to 60 ms), so
+    it meets few: beyond ``FORMING_BLOCK`` its multiples, from eight of them on four to an octave
+    (``LatentAttention.warm_up`` runs them ahead).  Pieces of 2,048 rows each would be fewer still, but take 49 us for
+    6,512 rows of 16 heads where one product takes 33 (K = 512), for 32,768 225 and 129.  A count that this package's
+    kernel takes is left as it is."""
+    if rows <= FORMING_BLOCK or ops.half_plan(rows, outputs, kv_rank, False)[0]:
+        return rows
+    block = forming_block(rows)
+    return -(-rows // block) * block
+
+
 class LatentAttention(Mixer):
     kind = "latent_attention"
     graph_safe = True
@@ -243,12 +264,27 @@ class LatentAttention(Mixer):
             step.taps["o"] = a.clone()
         return ops.linear(a.view(T, nh * dv), self.w_out, partial_ok=self.partial_ok, tune=tune)
 
+    def warm_up(self, step_tokens):
+        if self.w_form is None:
+            return
+        outputs, counts = self.w_form.shape[0], [FORMING_BLOCK]
+        most = min(FORMING_ROWS_A_TOKEN * step_tokens, FORMING_BYTES // (2 * outputs))
+        while counts[-1] < most:
+            counts.append(counts[-1] + forming_block(counts[-1] + 1))
+        # (values as steps have them: on zeros other candidates win)
+        latent = self.w_form.new_empty((counts[-1], self.kv_rank))
+        latent.normal_(generator=torch.Generator(device=latent.device))
+        for rows in counts:
+            if not ops.half_plan(rows, outputs, self.kv_rank, False)[0]:
+                ops.linear(latent[:rows], self.w_form, tune=self.runtime.tune)
+
     def _formed(self, q, down, plane, step, cache):
         """The heads' gated results over formed keys and values."""
+        rows = forming_rows(step.n_tokens + sum(step.ctx_lens_host), self.w_form.shape[0], self.kv_rank)
         latent, rot = ops.latent_open_rows(
             q, self.head_dim, self.rotated_dim, step.positions, self.inv_freq, self.rot_dims, self.adjacent,
             self.magnitude, plane, self.kv_rank, step.block_tables[cache.group], step.seq_start, step.ctx_len,
-            step.n_tokens + sum(step.ctx_lens_host))
+            rows)
         kv = ops.linear(latent, self.w_form, tune=self.runtime.tune)
         a = ops.latent_expanded(q, kv, rot, step.positions, step.attention_items(ops.LATENT_EXPANDED_ROWS, 2),
                                 step.seq_start, step.ctx_len, self.scale, self.sink, down if self.gate else None,

@@ -421,6 +421,25 @@ def test_recorded_portions_take_one_form(monkeypatch):
         assert small(forms) == {formed}
 
 
+def test_taps_of_formed_steps(monkeypatch):
+    """The queries that a step leaves in its taps are the folded ones, whichever form it takes."""
+    from zig_ai_amd.parts import latent_attention
+    model, _ = build(FORMED, seed=8, dtype="bfloat16")
+    prompts = [gu.tokens(61, FORMED["vocab"], 1)]
+    schedule = [([(0, 0, 40)], []), ([(0, 40, 41)], []), ([(0, 41, 61)], [0])]
+    left = []
+    for most in (256 << 20, 0):
+        monkeypatch.setattr(latent_attention, "FORMING_BYTES", most)
+        forms, streams = eu.FormedKeys(2), {}
+        eu.run_schedule(runner_for(model, page_size=16), prompts, schedule, forms=forms, streams=streams)
+        assert [formed for _, formed in forms.steps] == [most > 0, False, most > 0]
+        left.append(streams[0])
+    for layer, (heads, width) in enumerate(((2, 64 + 64), (3, 40))):
+        assert all(run[layer + 1]["q"].shape == (61, heads, width) for run in left)
+    # (the first layer's queries hang on nothing that the form changes)
+    assert torch.equal(left[0][1]["q"], left[1][1]["q"])
+
+
 def test_forming_with_rows_to_spare(monkeypatch):
     """Keys and values formed for more rows than there are, whatever memory holds there: the logits of just as many."""
     from zig_ai_amd.parts import latent_attention

@@ -233,9 +233,7 @@ class LatentAttention(Mixer):
                 and forming_pays(step.seq_lens_host, step.ctx_lens_host, 2 * nh * (d + dv)):
             a = self._formed(q, down, plane, step, cache)
             return ops.linear(a.view(T, nh * dv), self.w_out, partial_ok=self.partial_ok, tune=tune)
-        # the folded query [Wuk^T q_n | rot(q_r)]
-        qf = ops.latent_fold(q, self.k_fold, dr, step.positions, self.inv_freq, self.rot_dims, self.adjacent,
-                             self.magnitude)
+        qf = self._folded(q, step)
         item_seq, item_row0, item_count, n_items = step.attention_items(self.rows_per_item)
         waves = 0
         if self.mfma:
@@ -278,8 +276,15 @@ class LatentAttention(Mixer):
             if not ops.half_plan(rows, outputs, self.kv_rank, False)[0]:
                 ops.linear(latent[:rows], self.w_form, tune=self.runtime.tune)
 
+    def _folded(self, q, step):
+        """The folded queries [Wuk^T q_n | rot(q_r)]."""
+        return ops.latent_fold(q, self.k_fold, self.rotated_dim, step.positions, self.inv_freq, self.rot_dims,
+                               self.adjacent, self.magnitude)
+
     def _formed(self, q, down, plane, step, cache):
         """The heads' gated results over formed keys and values."""
+        if getattr(step, "taps", None) is not None:
+            step.taps["q"] = self._folded(q, step)      # (what the other steps leave)
         rows = forming_rows(step.n_tokens + sum(step.ctx_lens_host), self.w_form.shape[0], self.kv_rank)
         latent, rot = ops.latent_open_rows(
             q, self.head_dim, self.rotated_dim, step.positions, self.inv_freq, self.rot_dims, self.adjacent,
@@ -290,7 +295,6 @@ class LatentAttention(Mixer):
                                 step.seq_start, step.ctx_len, self.scale, self.sink, down if self.gate else None,
                                 self.gate_col, self.gate)
         if getattr(step, "taps", None) is not None:
-            step.taps["q"] = q.clone()      # (not folded)
             step.taps["o"] = a.clone()
         return a
 

@@ -169,3 +169,21 @@ def test_how_many_rows_keys_and_values_are_formed_for(outputs, rank):
         if room > FORMING_BLOCK and not ops.half_plan(room, outputs, rank, False)[0]:
             asked.add(room)
     assert len(asked) <= 25
+
+
+@pytest.mark.parametrize("tokens,top,experts,outputs,inner,once", [
+    (1, 4, 32, 1024, 2048, False),       # a token's four experts of 32
+    (1, 4, 32, 512, 1024, False),
+    (1, 2, 8, 2048, 1024, False),
+    (1, 2, 8, 4096, 2048, True),
+    (2, 4, 32, 1024, 2048, True),
+    (8, 4, 32, 512, 1024, True),
+    (8, 2, 8, 1024, 1024, False),        # all of them together are no more
+    (20, 2, 8, 4096, 2048, True),
+    (400, 4, 32, 1024, 2048, True),
+    (640, 4, 32, 1024, 2048, False),     # many rows an expert
+])
+def test_which_experts_are_read_past_the_caches(tokens, top, experts, outputs, inner, once):
+    """By the bytes that a launch can read, not by those of experts that no token of the step goes to."""
+    rule = ops.build.load("experts").za_grouped_reads_once
+    assert bool(rule(tokens * top, experts, outputs, inner)) == once

@@ -525,6 +525,25 @@ grouped_gemm_f32_kernel(GroupedArgs g) {
                                             [&](int r) { return W + (size_t)w_row(r) * K; }, store);
 }
 
+// Whether a grouped product reads its weights past the caches' other contents: few rows an expert, and
+// more bytes than layers of which some could stay in the last level's cache (256 MB) from one step to the
+// next would read, counted for the experts that A assignments can name and for the down product (gate|up
+// reads twice that, so that two such layers and a half fill the cache).  What a step reads again loses by
+// it, what comes from memory gains.  Us, gate|up and down of a layer, first with the layers' weights left
+// in the cache where they fit, then from memory, each as usual and past the caches; MB of the down product:
+//   32 experts of 1,024 over 2,048, 4 a token, one token, 17 MB       19.4 23.5    22.4 23.4
+//      2 tokens, 34 MB                                                24.5 28.2    27.9 25.4
+//      4 tokens, 67 MB; 8 tokens                                      35.2 40.4    42.5 38.4;  65.3 59.9
+//      64 tokens; 400 tokens                                                       85.9 76.4;  106.6 98.0
+//   32 of 512 over 1,024, one token, 4 MB; 8 tokens, 34 MB            12.6 13.7    14.0 13.6;  22.1 19.7
+//   8 of 2,048 over 1,024, 2 a token, one token, 8 MB; 8, 34 MB       17.9 20.3    20.8 19.5;  26.4 24.0
+//   8 of 4,096 over 2,048, 2 a token, one token, 34 MB; 20 tokens     34.7 39.4    40.3 37.6;  101.8 90.5
+//   8 of 1,024 over 1,024, 2 a token, 8 tokens, 17 MB                 17.0 19.2    18.2 16.8
+// So the smaller sets, which a small model keeps (and a loop over layers reads twice a step), are left in.
+extern "C" int za_grouped_reads_once(long long A, int experts, int N, int K) {
+  return A < 80LL * experts && (A < experts ? A : experts) * N * K * 2 >= ZA_ONCE_BYTES;
+}
+
 // dtype codes: 0 = float32, 1 = bfloat16.  `src` has `src_rows` rows of K elements; the
 // lists name assignments below n_tokens * top, so src_rows >= n_tokens (src_div == top) or
 // >= n_tokens * top (src_div == 1).  With `gate` (see GroupedArgs) W is [experts][2N][K].
@@ -633,14 +652,7 @@ extern "C" int za_grouped_gemm(const void* src, int src_dtype, long long src_row
     const long long rows = (A + BM - 1) / BM + experts, blocks = (rows + 7) / 8 * 8 * ((N + columns - 1) / columns);
     if (blocks > 0x7fffffffLL) return ZA_ERR_ARG;
     const dim3 grid((unsigned)blocks);
-    // Weights that few rows read: past the caches' other contents, where the experts have more than a
-    // model that stays in the last level's cache (256 MB) would give one product.  Weights of four
-    // layers or more in turn, gate|up and down, before and after (us): 8 experts of 4,096 over 2,048, 2 a
-    // token, 20 tokens 70.2 + 31.6 and 62.9 + 27.6, 150 tokens 65.7 + 42.7 and 60.0 + 39.4; 32 experts of
-    // 1,024, 4 a token, 64 tokens 56.1 + 29.8 and 49.9 + 26.5, 400 tokens 73.3 + 33.3 and 67.4 + 30.6,
-    // one token 13.6 + 8.6 and 13.6 + 8.3 (only where 200 MB of its experts were still cached 11.0 +
-    // 7.2 became 13.1 + 8.3: smaller sets than 32 MB, which may stay there, are left in).
-    const bool once = A < 80LL * experts && (gate ? 2LL : 1LL) * experts * N * K * 2 >= ZA_ONCE_BYTES;
+    const bool once = za_grouped_reads_once(A, experts, N, K) != 0;
 #define ZA_GT(TO, GATED, BM, BN, NS)                                                                                \
   {                                                                                                                 \
     if (once)                                                                                                       \

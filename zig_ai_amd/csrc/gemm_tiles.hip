@@ -98,9 +98,13 @@ extern "C" int za_gemm_bf16_tiles(const void* x, const void* W, void* out, int o
     return ZA_ERR_UNSUPPORTED;
   const int per = gated ? GT_BN / 2 : GT_BN;
   dim3 grid((unsigned)((N + per - 1) / per), (unsigned)ranges);
-  // Large weights past the caches' other contents (us, before and after, in a decode step of 64 tokens of the
-  // 2,048-wide hybrid: gate|up 67 MB 18.6 and 17.0, down 33 MB 10.2 and 9.7, head 268 MB 63.1 and
-  // 60.6; of 20 tokens 8,192 x 2,048 8.9 and 8.4, head 53.4 and 48.8; 12 MB 9.5 and 9.7, 8 MB 5.6 and 5.8).
+  // Large weights past the caches' other contents, by size: what comes from memory gains, what is left of the step
+  // before in the last level's cache (256 MB) loses, and of weights of 32 MB and more a model of more than two or
+  // three layers does not stay there.  Us as usual and past the caches, from memory and from the cache, 32 rows:
+  // 8 MB 6.6 6.2 and 5.7 6.4, 17 MB 6.8 6.6 and 6.1 7.6, 25 MB 10.6 10.3 and 9.7 11.4, 34 MB 11.7 10.9 and
+  // 10.1 12.9, 50 MB 14.1 12.3 and 11.3 14.3, 67 MB 17.4 15.3 and 14.3 17.5, 134 MB 30.1 27.8; 64 rows, 34 MB 13.2 12.9 and
+  // 12.1 14.7, 67 MB 18.5 16.2 and 14.9 18.9.  In a decode step of 64 tokens of the 2,048-wide hybrid gate|up 18.6 and
+  // 17.0, down 10.2 and 9.7, head 63.1 and 60.6, but 12 MB 9.5 and 9.7, 8 MB 5.6 and 5.8.
   const bool once = (gated ? 2LL : 1LL) * N * K * 2 >= ZA_ONCE_BYTES;
 #define ZA_GT(TO, GATED, BM, NS)                                                                      \
   {                                                                                                   \

@@ -21,8 +21,8 @@
 
 #define GG_BK 64
 
-// A product whose weights take this many bytes or more is not one of a model that the last level's cache
-// (256 MB) could hold from one step to the next.
+// From this many bytes of weights on a product reads them past the caches' other contents: a guess from one product's
+// size that its model is larger than the last level's cache (256 MB) holds from one step to the next.
 #define ZA_ONCE_BYTES (32LL << 20)
 
 template <int BM, int BN, int NS, bool ONCE = false>

@@ -187,3 +187,11 @@ def test_which_experts_are_read_past_the_caches(tokens, top, experts, outputs, i
     """By the bytes that a launch can read, not by those of experts that no token of the step goes to."""
     rule = ops.build.load("experts").za_grouped_reads_once
     assert bool(rule(tokens * top, experts, outputs, inner)) == once
+
+
+def test_where_a_token_gate_runs_in_its_product():
+    """Up to a round of loads, or whole ones and few rows: part of a round costs as much as a whole one."""
+    assert all(ops.table_gate_fuses(T, K) for T in (1, 8, 16) for K in (8, 1024, 1544, 2048))
+    assert all(ops.table_gate_fuses(T, K) for T in (1, 8) for K in (4096, 8192))
+    assert not any(ops.table_gate_fuses(T, K) for T in (1, 8, 16) for K in (2056, 2560, 3072, 5120))
+    assert not any(ops.table_gate_fuses(T, K) for T, K in ((9, 4096), (16, 8192), (17, 1024), (4, 1028)))

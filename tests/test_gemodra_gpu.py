@@ -1103,7 +1103,8 @@ def test_latent_fold_in_one_launch(T, H, R, d, rotated, rot_dims, adjacent):
     assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("T,K,dim", [(1, 8, 5), (3, 250 * 8, 40), (16, 2048, 256), (8, 4104, 17), (17, 64, 32)])
+@pytest.mark.parametrize("T,K,dim", [(1, 8, 5), (3, 250 * 8, 40), (16, 2048, 256), (8, 4104, 17), (17, 64, 32),
+                                     (8, 4096, 17), (1, 6144, 24), (9, 4096, 32), (2, 2560, 32)])
 @pytest.mark.parametrize("table_dtype", [torch.float32, torch.bfloat16])
 def test_table_gate_on_its_own_product(T, K, dim, table_dtype):
     """Steps of K below, at and beyond what eight waves have under way; outputs that fill no tile; ids that are not in
@@ -1116,7 +1117,14 @@ def test_table_gate_on_its_own_product(T, K, dim, table_dtype):
     table = torch.randn(50, dim + 9, generator=g).to(table_dtype)
     ids = torch.randint(0, 50, (T,), generator=g, dtype=torch.int32)
     ids[0] = 50 if T > 1 else 3
-    got = ops.table_gate_linear(x.to(dev), w.to(dev), ids.to(dev), table.to(dev), 9, "gelu_tanh").cpu().double()
+    ops.form_log = []
+    try:
+        got = ops.table_gate_linear(x.to(dev), w.to(dev), ids.to(dev), table.to(dev), 9, "gelu_tanh").cpu().double()
+        product, = [r for r in ops.form_log if r["op"] == "linear"]
+    finally:
+        ops.form_log = None
+    assert (product["M"], product["N"], product["K"]) == (T, dim, K)
+    assert (product.get("kernel") == "table_gate") == ops.table_gate_fuses(T, K)
     rows = torch.where((ids < 50)[:, None], table[ids.clamp(max=49).long(), 9:].double(), torch.zeros(()).double())
     want = torch.nn.functional.gelu(x.double() @ w.double().T, approximate="tanh") * rows
     # (product and result are rounded to bfloat16: 2^-9 each of values that the gate carries on with slopes up to 1.13)

@@ -410,8 +410,8 @@ extern "C" int za_table_gate(const void* g, int dtype, const int* ids, const voi
 // The same on a product that is taken here, for a decode batch (at most 16 rows, bfloat16): act(round(x W^T)) times the
 // table's slice.  A workgroup takes 16 outputs and its eight waves the steps of K in turn, fragments straight from
 // memory and eight under way a wave; their sums meet in LDS.  What bounds it is one way to memory; a kernel of its
-// own for the gate takes another: 8 rows, 256 outputs of 2,048, 2 us
-// less a layer than the two.
+// own for the gate takes another: 8 rows, 256 outputs of 2,048, 4.9 us for the two's 6.5.  Which K
+// and rows gain is ops.table_gate_fuses.
 #define TL_WAVES 8
 template <typename TT>
 __global__ void __launch_bounds__(TL_WAVES * 64)

@@ -3143,13 +3143,25 @@ def table_gate(g: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, col0: in
     return out
 
 
+TABLE_GATE_ROUND = 2048        # elements of K that the workgroup's waves have under way at once
+
+
+def table_gate_fuses(T: int, K: int) -> bool:
+    """Whether ``table_gate_linear`` takes one kernel: every round of its loads is another way to memory, and costs as
+    much where K fills a part of it.  Us in two kernels and in one, 256 outputs, 1, 8 and 16 rows: K = 1,024 5.2 5.6
+    5.6 and 4.2 4.9 5.6, 2,048 6.2 6.5 6.7 and 4.2 4.9 5.5, 2,560 6.6 7.1 7.8 and 6.5 7.9 9.4, 3,072 7.4 7.7 8.7 and 6.9
+    8.2 10.1, 4,096 8.5 8.9 9.8 and 7.0 8.5 10.4, 8,192 14.0 16.3 18.8 and 11.8 15.1 18.6; 1,024 and 2,048 outputs alike."""
+    return T <= 16 and K % 8 == 0 and (K <= TABLE_GATE_ROUND or K % TABLE_GATE_ROUND == 0 and T <= 8)
+
+
 def table_gate_linear(x: torch.Tensor, weight: torch.Tensor, ids: torch.Tensor, table: torch.Tensor, col0: int,
                       activation: str, tune: Optional[bool] = None) -> torch.Tensor:
-    """``table_gate`` of ``x weight^T``: a decode batch in bfloat16 takes one kernel, anything else two."""
+    """``table_gate`` of ``x weight^T``: a decode batch in bfloat16 takes one kernel (``table_gate_fuses``),
+    anything else two."""
     T, K = x.shape
     dim = weight.shape[0]
-    if T > 16 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or K % 8 or x.data_ptr() % 16 \
-            or weight.data_ptr() % 16:
+    if not table_gate_fuses(T, K) or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 \
+            or x.data_ptr() % 16 or weight.data_ptr() % 16:
         return table_gate(linear(x, weight, tune=tune), ids, table, col0, activation)
     if activation not in GATE_ACTIVATIONS:
         raise KernelError(f"activation must be one of {sorted(GATE_ACTIVATIONS)}, got {activation!r}")
@@ -3164,6 +3176,8 @@ def table_gate_linear(x: torch.Tensor, weight: torch.Tensor, ids: torch.Tensor, 
         _ptr(x), _ptr(weight), _ptr(ids), _ptr(table), _code(table.dtype), table.shape[0], table.shape[1], int(col0),
         _ptr(out), T, dim, K, GATE_ACTIVATIONS[activation], _stream())
     _check(rc, "table_gate_linear")
+    _note("linear", M=T, N=dim, K=K, norm_in_product=False, added_to_stream=False, partial_sums=1, out=out.dtype,
+          kernel="table_gate")
     return out
 
 

@@ -653,6 +653,30 @@ def test_ssd_chunks_off_their_boundaries(H, G, N, P):
     assert bool(torch.isfinite(got[0][0][C + 1:C + 2]).all()) and bool(torch.isnan(got[0][0]).any())
 
 
+@pytest.mark.parametrize("H,G,N,P", [(8, 1, 128, 64), (3, 3, 64, 128), (2, 2, 128, 192)])
+def test_ssd_chunks_with_values_off_their_boundaries(H, G, N, P):
+    """Values that start one, two and three floats off a multiple of four, keys and queries on it: the bits of the
+    same values on it, which take the kernels of whole tiles as well."""
+    from zig_ai_amd.kernels import ops
+    dev = torch.device("cuda")
+    gen = torch.Generator(device=dev).manual_seed(H + N + P)
+    C = ops.RETENTION_CHUNK
+    lengths, slots = [C + 1, 1, 2 * C + 16, C - 1, 17], [2, 3, 0, 4, 1]
+    T, keys = sum(lengths), G * N
+    rand = lambda *shape: torch.randn(*shape, device=dev, generator=gen)
+    values, k, q = rand(T, H * P), rand(T, keys), rand(T, keys)
+    proj, bias, A_log, D, first = rand(T, H), rand(H), rand(H) - 1.0, rand(H), rand(6, H * N * P)
+    slot_id = torch.tensor(slots, dtype=torch.int32, device=dev)
+    base = None
+    for off in (0, 1, 2, 3):
+        conv = torch.cat([k, q, rand(T, off), values, rand(T, 4 - off)], dim=1).contiguous()
+        state = first.clone()
+        out = ops.ssd_recurrence_chunked(conv, keys, 0, 2 * keys + off, proj, 0, bias, A_log, D, state, 0, slot_id,
+                                         _chunk_items(lengths, C, dev), H, G, N, P)
+        base = base or (out, state)
+        assert torch.equal(out, base[0]) and torch.equal(state, base[1]), off
+
+
 @pytest.mark.parametrize("H,G,N,P", [(8, 1, 128, 64), (8, 2, 64, 128), (12, 3, 24, 16), (4, 1, 33, 130), (5, 1, 128, 70)])
 def test_ssd_chunks_with_scores_worked_out_once(H, G, N, P, monkeypatch):
     """Heads that share keys and queries take their scores from one place: the bits of the same heads with

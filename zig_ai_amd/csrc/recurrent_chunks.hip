@@ -86,6 +86,9 @@ __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + lo
 // key channels, and the state a wave: 44 and 64 in place of the 33 and 51).
 #define DC_CHUNK 128
 
+// Four neighbouring floats from any place on (memory takes 16 bytes a lane from any multiple of 4).
+typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_any_t;
+
 // The least log2 of a decay that is told apart from zero.  Any power this small is zero in 32-bit
 // (2^-149 is the last that is not), and a chunk's sum of such numbers still has 37 binary places in
 // double, so the decays behind a token that forgets everything keep theirs.
@@ -133,7 +136,7 @@ decay_chunk_state_kernel(DecayArgs a) {
   // 2 r + c.  Otherwise all key channels and 16 columns, an element at a time.
   constexpr int CT = FULL ? NT / 2 : NT, VT = FULL ? 2 : 1;      // tiles of channels, and of columns
   typedef __attribute__((ext_vector_type(CT))) float keys_t;
-  typedef __attribute__((ext_vector_type(VT))) float values_t;
+  typedef __attribute__((ext_vector_type(VT), aligned(4))) float values_t;      // (x_col may be any)
   const int chan0 = FULL ? (wave & 1) * CT * 16 : 0, col0 = blockIdx.z * 64 + (FULL ? (wave >> 1) * 32 : wave * 16);
   const int col = col0 + r16;
   const bool col_ok = FULL || col < dv;
@@ -436,7 +439,7 @@ decay_chunk_out_kernel(DecayArgs a) {
       // (no token sees one beyond the chunk)
       const float* x = rows + (size_t)min(J * 16 + 4 * g + r, n - 1) * a.width + a.x_col + h * dv;
       [[maybe_unused]] f32x4_t four;
-      if constexpr (FULL) four = *reinterpret_cast<const f32x4_t*>(x + col_of(0));
+      if constexpr (FULL) four = *reinterpret_cast<const f32x4_any_t*>(x + col_of(0));
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if constexpr (FULL) v[j][r] = four[j];
@@ -515,11 +518,11 @@ decay_chunk_out_kernel(DecayArgs a) {
       if constexpr (FULL) {
         f32x4_t y = {acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]};
         if (a.D) {
-          const f32x4_t four = *reinterpret_cast<const f32x4_t*>(x + col_of(0));
+          const f32x4_t four = *reinterpret_cast<const f32x4_any_t*>(x + col_of(0));
 #pragma unroll
           for (int j = 0; j < 4; ++j) y[j] = fmaf(D, four[j], y[j]);
         }
-        *reinterpret_cast<f32x4_t*>(o + col_of(0)) = y;
+        *reinterpret_cast<f32x4_any_t*>(o + col_of(0)) = y;
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -556,9 +559,8 @@ extern "C" int za_decay_chunked(const float* vec, int width, int q_col, int k_co
                     fixed, item_row0, item_count, sums, chunk_state, total, out, H, G, dk, dv, scores};
   dim3 grid(n_items, H, (dv + 63) / 64);
   const dim3 block(256);
-  const bool full = dv % 64 == 0 && width % 4 == 0 && q_col % 4 == 0 && k_col % 4 == 0 && x_col % 4 == 0 &&
-                    ((reinterpret_cast<uintptr_t>(vec) | reinterpret_cast<uintptr_t>(chunk_state) |
-                      reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+  const bool full = dv % 64 == 0 && width % 4 == 0 && q_col % 4 == 0 && k_col % 4 == 0 &&
+                    ((reinterpret_cast<uintptr_t>(vec) | reinterpret_cast<uintptr_t>(chunk_state)) & 15) == 0;
 #define ZA_DECAY(KERNEL, ...)                                                                  \
   {                                                                                            \
     if (full && dk == 64) hipLaunchKernelGGL((KERNEL<4, true __VA_ARGS__>), grid, block, 0, stream, a);    \

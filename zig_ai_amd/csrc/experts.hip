@@ -529,16 +529,16 @@ grouped_gemm_f32_kernel(GroupedArgs g) {
 // more bytes than layers of which some could stay in the last level's cache (256 MB) from one step to the
 // next would read, counted for the experts that A assignments can name and for the down product (gate|up
 // reads twice that, so that two such layers and a half fill the cache).  What a step reads again loses by
-// it, what comes from memory gains.  Us, gate|up and down of a layer, first with the layers' weights left
-// in the cache where they fit, then from memory, each as usual and past the caches; MB of the down product:
-//   32 experts of 1,024 over 2,048, 4 a token, one token, 17 MB       19.4 23.5    22.4 23.4
-//      2 tokens, 34 MB                                                24.5 28.2    27.9 25.4
-//      4 tokens, 67 MB; 8 tokens                                      35.2 40.4    42.5 38.4;  65.3 59.9
-//      64 tokens; 400 tokens                                                       85.9 76.4;  106.6 98.0
-//   32 of 512 over 1,024, one token, 4 MB; 8 tokens, 34 MB            12.6 13.7    14.0 13.6;  22.1 19.7
-//   8 of 2,048 over 1,024, 2 a token, one token, 8 MB; 8, 34 MB       17.9 20.3    20.8 19.5;  26.4 24.0
-//   8 of 4,096 over 2,048, 2 a token, one token, 34 MB; 20 tokens     34.7 39.4    40.3 37.6;  101.8 90.5
-//   8 of 1,024 over 1,024, 2 a token, 8 tokens, 17 MB                 17.0 19.2    18.2 16.8
+// it, what comes from memory gains less.  Us, gate|up and down of a layer, as usual and past the caches, first
+// with 180 MB of layers' weights that stay in the cache, then from memory; MB of the down product:
+//   32 experts of 1,024 over 2,048, 4 a token, one token, 17 MB       19.4 23.6    24.2 23.1
+//      2 tokens, 34 MB; 4, 67 MB                                      24.1 26.8    27.6 25.2;  40.0 36.8
+//      8 tokens, 134 MB; 64; 400                                      58.7 54.1;  85.9 76.4;  106.6 98.0
+//   32 of 512 over 1,024, one token, 4 MB; 8 tokens, 34 MB            12.6 13.8    14.5 13.7;  21.4 20.0
+//   60 of 704 over 2,048, 4 a token, one token, 12 MB; 3, 35 MB       17.3 19.9    20.3 19.5;  28.1 26.0
+//   8 of 2,048 over 1,024, 2 a token, one token, 8 MB; 8, 34 MB       17.8 20.4    21.1 20.3;  30.6 28.7
+//   8 of 4,096 over 2,048, 2 a token, one token, 34 MB; 20, 134 MB    35.3 39.8    39.9 37.4;  95.7 86.0
+//   8 of 1,024 over 1,024, 2 a token, 8 tokens, 17 MB                 17.4 19.4    19.4 18.6
 // So the smaller sets, which a small model keeps (and a loop over layers reads twice a step), are left in.
 extern "C" int za_grouped_reads_once(long long A, int experts, int N, int K) {
   return A < 80LL * experts && (A < experts ? A : experts) * N * K * 2 >= ZA_ONCE_BYTES;

@@ -222,6 +222,12 @@ class FormedKeys:
         assert formed in (0, self.layers), (entries, formed)
         self.steps.append((entries, formed > 0))
 
+    def as_the_rule_says(self, rows_a_token):
+        """Steps of portions alone, none of which sees many rows a token, form; no others."""
+        return all(formed == (min(b - a for _, a, b in entries) > 1
+                              and sum(b for _, _, b in entries) <= rows_a_token * sum(b - a for _, a, b in entries))
+                   for entries, formed in self.steps)
+
 
 def run_schedule(runner, prompts, schedule, wants=None, forms=None, streams=None):
     """Drive ``runner`` through ``schedule`` asking for the logits of every token (or, with

@@ -390,6 +390,34 @@ FORMED = gu.config([
     gu.layer("latent_attention_2", gu.plain_latent(heads=3, dim=128, vdim=128, kv_rank=40, q_rank=16), None)])
 
 
+def test_schedules_over_formed_keys(monkeypatch):
+    """Whole prompts, portions behind cached tokens, portions beside single tokens and decoding, from pages of 4
+    and 16 tokens: the plain logits whichever form a step takes, and those of the same steps all folded."""
+    from zig_ai_amd.parts import latent_attention
+    model, tensors = build(FORMED, seed=8, dtype="bfloat16")
+    lengths = [150, 37, 70, 2, 1]
+    prompts = [gu.tokens(n, FORMED["vocab"], 20 + i) for i, n in enumerate(lengths)]
+    want = torch.cat(plain_logits(FORMED, tensors, prompts))
+    both = set()
+    for name, schedule in dict(schedules(lengths), together=[([(0, 0, 60), (1, 0, 37), (2, 0, 66), (3, 0, 2)], [1, 3]),
+                                                             ([(0, 60, 148), (2, 66, 68)], []),
+                                                             ([(0, 148, 150), (2, 68, 70)], [0, 2]),
+                                                             ([(4, 0, 1)], [4])]).items():
+        page_size = 4 if len(name) % 2 else 16
+        got = []
+        for most in (256 << 20, 0):
+            monkeypatch.setattr(latent_attention, "FORMING_BYTES", most)
+            forms = eu.FormedKeys(2)
+            peak = eu.peak_tokens(lengths, schedule, round_to=16)
+            runner = runner_for(model, page_size=page_size, tokens=peak, slots=4, graphs=False)
+            got.append(torch.cat(eu.run_schedule(runner, prompts, schedule, forms=forms)))
+            assert forms.as_the_rule_says(16 if most else 0), name
+            both |= {formed for _, formed in forms.steps if most}
+            assert_bfloat16_close(got[-1], want, name)
+        assert_bfloat16_same_run(got[0], got[1], name)
+    assert both == {False, True}
+
+
 def test_recorded_portions_take_one_form(monkeypatch):
     """Where portions are recorded, a shape's first step, the recorded one with other contexts behind it, and a step
     of that shape with taps all take the kernels that do not hang on the contexts' lengths; larger steps, which

@@ -109,6 +109,38 @@ def test_mechanism_alone(name):
             assert worst(g, w) < F32_BOUND
 
 
+# heads of 128: a layer whose rows two others read, in either pairing of the rotated elements
+FORMED = vu.config([
+    vu.layer("latent_attention_2", vu.latent(heads=2, dim=128, vdim=128, kv_rank=64, q_rank=24, rot_dim=64, base=1e4)),
+    vu.layer("latent_attention_2", vu.latent(heads=5, dim=128, vdim=128, kv_rank=64, q_rank=40, rot_dim=64, base=1e4,
+                                             kv_from=0)),
+    vu.layer("latent_attention", vu.latent(heads=1, dim=128, vdim=128, kv_rank=24, q_rank=16, rot_dim=64,
+                                           scaling=vu.yarn())),
+    vu.layer("latent_attention_2", vu.latent(heads=3, dim=128, vdim=128, kv_rank=64, q_rank=16, rot_dim=64, base=1e4,
+                                             scale=0.05, kv_from=0))])
+
+
+def test_schedules_over_formed_keys(monkeypatch):
+    """Layers that form keys and values from their own rows and from another layer's: the plain logits, and those
+    of the same steps all folded."""
+    from zig_ai_amd.parts import latent_attention
+    model, tensors = build(FORMED, seed=8, dtype="bfloat16")
+    lengths = [130, 37, 2]
+    prompts = [vu.tokens(n, FORMED["vocab"], 20 + i) for i, n in enumerate(lengths)]
+    want = torch.cat(plain_logits(FORMED, tensors, prompts))
+    for name, schedule in (("whole", eu.whole(lengths)), ("portions", eu.changing_portions(lengths, seed=1)),
+                           ("mixed", eu.mixed(lengths, seed=2, max_live=3, decode_tail=20))):
+        got = []
+        for most in (256 << 20, 0):
+            monkeypatch.setattr(latent_attention, "FORMING_BYTES", most)
+            forms = eu.FormedKeys(4)
+            runner = runner_for(model, tokens=256, graphs=False)
+            got.append(torch.cat(eu.run_schedule(runner, prompts, schedule, forms=forms)))
+            assert forms.as_the_rule_says(16 if most else 0), name
+            assert_bfloat16_close(got[-1], want, name)
+        assert_bfloat16_same_run(got[0], got[1], name)
+
+
 def test_streams_after_every_layer():
     cfg = vu.TINY_ALL
     model, tensors = build(cfg, seed=3)

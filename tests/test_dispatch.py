@@ -195,3 +195,12 @@ def test_where_a_token_gate_runs_in_its_product():
     assert all(ops.table_gate_fuses(T, K) for T in (1, 8) for K in (4096, 8192))
     assert not any(ops.table_gate_fuses(T, K) for T in (1, 8, 16) for K in (2056, 2560, 3072, 5120))
     assert not any(ops.table_gate_fuses(T, K) for T, K in ((9, 4096), (16, 8192), (17, 1024), (4, 1028)))
+
+
+def test_where_a_decode_batch_shares_k_out_to_waves():
+    """What the host takes for the kernels' own line between their two forms is that line."""
+    import os
+    import re
+    with open(os.path.join(ops.build.CSRC_DIR, "latent.hip")) as f:
+        line, = re.findall(r"#define HL_SPLIT_MIN_K (\d+)", f.read())
+    assert int(line) == ops.HEAD_SPLIT_MIN_K

@@ -213,7 +213,6 @@ extern "C" int za_latent_prepare(const void* down, int dtype, int ld, int q_col,
   if (dtype == 0) ZA_LP(float);
   else if (dtype == 1) ZA_LP(bf16_t);
 #undef ZA_LP
-#undef ZA_LD
   else
     return ZA_ERR_UNSUPPORTED;
   return za_launch_status();
@@ -1592,7 +1591,8 @@ latent_decode_range_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
                            float* __restrict__ part_acc, float* __restrict__ part_ml, int H, int HC, int page_shift,
                            float scale_log2, int keys_per_split, int nsplit, const float* __restrict__ sink) {
   using S = LdShape<RT, DT>;
-  constexpr int R = S::R, W = S::W, WS = S::WS, NP = S::NP, OT = RT / LD_NW > 0 ? RT / LD_NW : 1;
+  static_assert(RT % LD_NW == 0, "a wave takes as much of the latent as any other");
+  constexpr int R = S::R, W = S::W, WS = S::WS, NP = S::NP, OT = RT / LD_NW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lm_lds[];
   unsigned char* Ks = lm_lds;                                                   // [LD_KT][NP * 16 bytes]
   unsigned char* Ps = Ks + (size_t)LD_KT * NP * 16;                             // [16 rows][LD_KT]
@@ -1655,7 +1655,6 @@ latent_decode_range_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
   for (int t = 0; t < OT; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int k_at = (wave * 16 + r16) * NP * 16 + ((kq ^ (r16 & 7)) << 4);
   const int v_key = kq * 8 + (r16 >> 2);                      // of the first four of a lane group's eight keys
-  const bool has_tiles = wave * OT < RT;
 
   for (int tile0 = range_lo; tile0 <= range_hi; tile0 += LD_KT) {
     __builtin_amdgcn_s_waitcnt(ZA_VMCNT(0));
@@ -1740,10 +1739,8 @@ latent_decode_range_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
             o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[kk], pf[kk], o[t], 0, 0, 0);
       }
     };
-    if (has_tiles) {
-      if (tile0 + LD_KT - 32 <= range_hi) values(std::true_type{});
-      else values(std::false_type{});
-    }
+    if (tile0 + LD_KT - 32 <= range_hi) values(std::true_type{});
+    else values(std::false_type{});
     if (tile0 + LD_KT <= range_hi) {
       __syncthreads();                                        // the tile has been read
       request(tile0 + LD_KT);
@@ -1763,7 +1760,6 @@ latent_decode_range_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
   if (nsplit == 1) {
     if (sink) lt += exp2f(sink[h] * LM_LOG2E - m);
     const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-    if (!has_tiles) return;
     bf16_t* orow = out + ((size_t)tok * H + h) * R + wave * OT * 16 + kq * 4;
 #pragma unroll
     for (int t = 0; t < OT; ++t) {
@@ -1774,11 +1770,9 @@ latent_decode_range_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
     }
   } else {
     const size_t pidx = ((size_t)tok * H + h) * nsplit + z;
-    if (has_tiles) {
-      float* pa = part_acc + pidx * R + wave * OT * 16 + kq * 4;
+    float* pa = part_acc + pidx * R + wave * OT * 16 + kq * 4;
 #pragma unroll
-      for (int t = 0; t < OT; ++t) *reinterpret_cast<f32x4_t*>(pa + t * 16) = o[t];
-    }
+    for (int t = 0; t < OT; ++t) *reinterpret_cast<f32x4_t*>(pa + t * 16) = o[t];
     if (wave == 0 && kq == 0) {
       part_ml[pidx * 2] = m * LM_LN2;
       part_ml[pidx * 2 + 1] = lt;

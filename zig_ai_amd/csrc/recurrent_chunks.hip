@@ -607,9 +607,9 @@ extern "C" int za_decay_chunked(const float* vec, int width, int q_col, int k_co
 // most one when they are, and a decay of zero is nothing special.  Pairs of tokens within 16 take
 // their product token by token; those of two neighbouring blocks of 16 as (product up to the
 // first block's end) times (product from the second one's start on).
-// 2,048 tokens, 16 heads of 128 x 128: 840 us walked token by token beside 38 us of preparation; 76 +
-// 131 us here.  The walk over chunks is a chain of 2.0 us a chunk, of which the products with the
-// state take 0.7 and its operands' way through the compute unit's cache 0.4 (2.8 us when every wave
+// 2,048 tokens, 16 heads of 128 x 128: 840 us walked token by token beside 38 us of preparation; 70 +
+// 119 us here.  The walk over chunks is a chain of 1.9 us a chunk, 1.3 without any loads; of the
+// rest some is its operands' way through the compute unit's cache (0.8 us more when every wave
 // requested every operand).
 #define DL_CHUNK 32
 

@@ -3288,7 +3288,7 @@ def rotate_part_(src: torch.Tensor, src_col: int, dst: torch.Tensor, dst_col: in
     return dst
 
 
-HEAD_SPLIT_MIN_K = 256     # from here on a decode batch's head products share K out to a workgroup's waves
+HEAD_SPLIT_MIN_K = 256     # from here on a decode batch's head products share K out to a workgroup's waves (csrc/latent.hip)
 HEAD_GATES = {None: 0, "head": 1, "element": 2}
 
 

@@ -52,9 +52,9 @@ LATENT_SPLIT_BYTES = 32 << 20  # the most that the ranges' partial results may t
 
 def plan_latent_split(groups: int, max_keys: int, target: int = LATENT_SPLIT_TARGET, tile: int = 64):
     """(keys per range, number of ranges) for one launch of the matrix-core kernels: a function
-    of the batch shape and of the longest context only.  A workgroup holds one or four waves
-    and takes 32 keys a tile, so short ranges pay: as many as reach ``target``
-    workgroups, of at least ``LATENT_SPLIT_KEYS`` keys each, in whole tiles of ``tile``."""
+    of the batch shape and of the longest context only.  As many ranges as reach ``target``
+    workgroups, of at least ``LATENT_SPLIT_KEYS`` keys each, in whole multiples of ``tile``: the kernels of one
+    and four waves take 32 keys at a time, so short ranges pay; the one of eight waves takes 128."""
     if groups >= target or max_keys <= 2 * LATENT_SPLIT_KEYS:
         return 0, 1
     nsplit = min(target // groups, max_keys // LATENT_SPLIT_KEYS, 64)
@@ -69,6 +69,9 @@ def plan_latent_split(groups: int, max_keys: int, target: int = LATENT_SPLIT_TAR
 # unit at latents of 512 (three at 128), and a second round of them costs more than longer ranges.  Us with
 # ranges of 128, 256 and 512 keys, 16 heads, R = 512 with 64 rotated: 8 requests at 2,050 keys 18.5, 19.8, 25.5, at
 # 8,000 42, 29, 30; 32 at 2,000 36, 26, 29; 64 at 1,200 46, 39, 32; R = 128 with 32: 64 at 2,000 19.0, 15.7, 17.1.
+# 129 to 255 groups get a range each, which leaves compute units idle, but cuts them only gain where contexts are long
+# and three ranges fill two rounds well: in one, two and three ranges 130 requests at 1,000 keys 42, 59, 53, at 2,000
+# 88, 105, 91, at 4,000 171, 193, 151, 200 at 4,000 191, 215, 223; 20 requests of 128 heads at 4,000 118, 132, 102.
 LATENT_RANGE_TARGET, LATENT_RANGE_TARGET_SMALL, LATENT_RANGE_TILE = 256, 512, 128
 
 
@@ -78,10 +81,13 @@ FORMING_BYTES = 256 << 20      # the most that formed keys and values may take
 
 def forming_pays(seq_lens, ctx_lens, bytes_a_row: int) -> bool:
     """Whether a step's keys and values are formed: every request brings a portion, and a visible row is
-    seen by enough new tokens.  Us a layer folded and formed (16 heads, R = 512 with 64 rotated): 4
-    tokens of 8 requests each 31 and 13, one prompt of 64 32 and 15, 512 61 and 26, 1,777 147 and 60, 4,096 523 and 145;
-    128 tokens behind 900 cached ones 51 and 39, behind 2,000 135 and 65, 64 of 8 requests each behind 400 62 and 42, 512 behind
-    6,000 348 and 158.  Single tokens share their rows with nobody, and a row costs 7 ns to form."""
+    seen by enough new tokens.  Us a layer folded and formed (16 heads, R = 512 with 64 rotated), by visible rows a new
+    token.  1: one prompt of 64 32 and 15, 512 61 and 26, 1,777 145 and 61, 4,096 523 and 145; 4 tokens of 8 requests each 31 and
+    13.  8 to 9: 128 tokens behind 900 cached ones 51 and 39, 64 of 8 requests each behind 512 65 and 54.  13: 512 behind
+    6,000 348 and 158.  17: 128 behind 2,048 135 and 64, 64 behind 1,024 50 and 40, 64 of 8 each behind 1,024 91 and 81, 2 of 32
+    each behind 32 27 and 23.  25: 128 behind 3,072 185 and 81, but 64 behind 1,536 50 and 55, 2 of 32 each behind 48 28 and
+    31.  33: 512 behind 16,384 836 and 390, 64 of 8 each behind 2,048 140 and 144.  The line lies where all gain: beyond it
+    few tokens lose, whose folded kernel cuts contexts into ranges.  Single tokens share their rows with nobody."""
     rows = sum(seq_lens) + sum(ctx_lens)
     return min(seq_lens) > 1 and rows <= FORMING_ROWS_A_TOKEN * sum(seq_lens) and rows * bytes_a_row <= FORMING_BYTES
 

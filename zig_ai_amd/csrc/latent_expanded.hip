@@ -115,7 +115,8 @@ extern "C" int za_latent_open_rows(void* q, int q_ld, int q_col, int n_tokens, i
 // ------------------------------------------------------------------------ attention
 // A workgroup of four waves takes up to 64 tokens of one head, 16 rows a wave.  As in paged_attention_mfma_kernel:
 //   S^T = K Q^T        queries in registers, keys from LDS; a lane has the scores of one row
-//   p = 2^(S^T scale log2(e) - m), rounded to bfloat16; m the running maximum rounded up to a whole number
+//   p = 2^(S^T scale log2(e) - m), rounded to bfloat16; m the running maximum, not rounded: the largest
+//                      weight is one, and rounding it to bfloat16 costs nothing
 //   O^T += V^T P^T     P from the accumulator straight into the second operand; V^T from LDS, where values lie as
 //                      they come, turned round on the way to registers (ds_read_b64_tr_b16)
 // The next tile goes from memory into the other of two places in LDS without registers while one is computed.  A
@@ -292,9 +293,9 @@ latent_expanded_kernel(LxArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[jb][i]);
       tmax = quad_max(tmax);
-      const float m_new = fmaxf(m, ceilf(tmax * a.scale_log2e));      // (the factor is positive)
+      const float m_new = fmaxf(m, tmax * a.scale_log2e);      // (the factor is positive)
       const float m_use = m_new > -INFINITY ? m_new : 0.f;
-      const float alpha = m > -INFINITY ? ldexpf(1.0f, (int)(m - m_use)) : 1.0f;
+      const float alpha = m == m_new || m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - m_use);
 #pragma unroll
       for (int jb = 0; jb < JB; ++jb)
 #pragma unroll

@@ -857,6 +857,20 @@ def test_latent_decoding_on_whole_tiles(H, R, rotated, page_size):
         assert torch.equal(got, want), nsplit
 
 
+@pytest.mark.parametrize("H,R,rotated", [(16, 512, 64), (40, 512, 0), (16, 256, 64), (3, 128, 32)])
+def test_latent_decoding_is_off_by_its_results_rounding(H, R, rotated):
+    """Single tokens, whole and in ranges: no further from 64 bits than the result's own rounding to bfloat16, but
+    for 3 in 100 (scores and weights are rounded far below that)."""
+    from zig_ai_amd.kernels import ops
+    q, plane, table, pos, iseq, irow, icnt, n, scale, sink, want = _latent_attention_case(
+        torch.bfloat16, H, R + rotated, R, [(c, 1) for c in (40, 100, 129, 300, 517, 1000)], 16, 1, seed=H)
+    bound = 1.03 * rel_norm(want.bfloat16().double(), want)
+    for keys, nsplit in ((0, 1), (128, 8), (512, 2)):
+        got = ops.latent_attention(q, plane, R, table, pos, iseq, irow, icnt, n, scale, sink, keys, nsplit, 1).cpu().double()
+        off = rel_norm(got, want)
+        assert off < bound, nsplit
+
+
 @pytest.mark.parametrize("R,rotated,page_size", [(512, 64, 16), (256, 32, 4), (128, 0, 64), (512, 64, 12)])
 def test_latent_prefill_without_a_page(R, rotated, page_size):
     """A table entry below zero stands for rows of zeros, never for another request's page."""

@@ -1570,16 +1570,20 @@ latent_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out
 // (token, head).  All of a range's rows are requested into LDS at once, without registers, a key's 16-byte pieces in the
 // order piece ^ (key % 8); a wave has the scores of its keys, over the whole of a row; the waves' maxima meet in
 // LDS, then their weights, and a wave takes every eighth of the latent over all keys, turned round on the way to
-// registers (ds_read_b64_tr_b16).  What bounds it is the way to memory (item, position, page, rows) once a range:
-// 8 requests of 16 heads at 2,051 keys, R = 512 with 64 rotated, ranges of 128, with the merge: 18.7 us, tiles of 32 through
-// registers with three meetings each 23.5; 64 at 1,200 in ranges of 512 32, before in ranges of 128 58; 8 at 8,000 29 and 50.
+// registers (ds_read_b64_tr_b16).  A weight goes into the products as two bfloat16 numbers, it and what its rounding
+// leaves: in tiles of 32 keys the running maximum has more weights of exactly one, so the same weights rounded
+// once here were 1 to 3 percent further from 64 bits (8 requests at 2,050 keys 1.89e-3 and 1.86e-3; so 1.66e-3, the
+// rounding of the result).  What bounds it is the way to memory (item, position, page, rows) once a range: 8 requests of
+// 16 heads at 2,051 keys, R = 512 with 64 rotated, ranges of 128, with the merge: 19.1 us (weights rounded once 18.9),
+// tiles of 32 through registers with three meetings each 23.5; 64 at 1,200 in ranges of 512 33.3 (32.6), before in ranges
+// of 128 58; 8 at 8,000 30 (29.5) and 50.
 #define LD_KT 128
 #define LD_NW (LD_KT / 16)
 template <int RT, int DT>
 struct LdShape {
   static constexpr int R = RT * 16, W = R + DT * 32, WS = W / 32;
   static constexpr int NP = (WS * 4 + 7) / 8 * 8;            // pieces of a key in LDS
-  static constexpr size_t LDS = (size_t)LD_KT * NP * 16 + 16 * LD_KT * 2 + 16 * LD_NW * 4;
+  static constexpr size_t LDS = (size_t)LD_KT * NP * 16 + 2 * 16 * LD_KT * 2 + 16 * LD_NW * 4;
 };
 
 template <int RT, int DT>
@@ -1596,7 +1600,8 @@ latent_decode_range_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
   extern __shared__ __attribute__((aligned(16))) unsigned char lm_lds[];
   unsigned char* Ks = lm_lds;                                                   // [LD_KT][NP * 16 bytes]
   unsigned char* Ps = Ks + (size_t)LD_KT * NP * 16;                             // [16 rows][LD_KT]
-  float* Xs = reinterpret_cast<float*>(Ps + 16 * LD_KT * 2);                    // [16 rows][LD_NW]
+  unsigned char* Rs = Ps + 16 * LD_KT * 2;                                      // what rounding took from them
+  float* Xs = reinterpret_cast<float*>(Rs + 16 * LD_KT * 2);                    // [16 rows][LD_NW]
 
   const int item = blockIdx.x, z = blockIdx.z, h0 = blockIdx.y * HC;
   const int G = min(HC, H - h0);
@@ -1703,27 +1708,33 @@ latent_decode_range_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
     const float m_use = m_new > -INFINITY ? m_new : 0.f;
     const float alpha = m == m_new ? 1.0f : exp2f(m - m_use);
     m = m_new;
-    bf16x4_t p;
+    bf16x4_t p, rest;
     float psum = 0.f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      p[i] = (bf16_t)exp2f(s[i] - m_use);
-      psum += (float)p[i];
+      const float e = exp2f(s[i] - m_use);
+      p[i] = (bf16_t)e;
+      rest[i] = (bf16_t)(e - (float)p[i]);
+      psum += (float)p[i] + (float)rest[i];
     }
     l = l * alpha + psum;
     // (weights of a row in pieces of eight keys, piece ^ (row % 8))
-    *reinterpret_cast<bf16x4_t*>(Ps + r16 * (LD_KT * 2) + (((wave * 2 + (kq >> 1)) ^ (r16 & 7)) << 4) + (kq & 1) * 8) = p;
+    const int p_at = r16 * (LD_KT * 2) + (((wave * 2 + (kq >> 1)) ^ (r16 & 7)) << 4) + (kq & 1) * 8;
+    *reinterpret_cast<bf16x4_t*>(Ps + p_at) = p;
+    *reinterpret_cast<bf16x4_t*>(Rs + p_at) = rest;
     __syncthreads();
     // ---- values
     auto values = [&](auto whole) {      // (of blocks of 32 keys, those in the range)
 #pragma unroll
-      for (int t = 0; t < OT; ++t) {
-        o[t] *= alpha;
-        bf16x8_t pf[LD_KT / 32], vf[LD_KT / 32];
+      for (int t = 0; t < OT; ++t) o[t] *= alpha;
 #pragma unroll
-        for (int kk = 0; kk < LD_KT / 32; ++kk) {
-          if (!decltype(whole)::value && tile0 + kk * 32 > range_hi) continue;
-          pf[kk] = *reinterpret_cast<const bf16x8_t*>(Ps + r16 * (LD_KT * 2) + (((kk * 4 + kq) ^ (r16 & 7)) << 4));
+      for (int kk = 0; kk < LD_KT / 32; ++kk) {
+        if (!decltype(whole)::value && tile0 + kk * 32 > range_hi) continue;
+        const int at = r16 * (LD_KT * 2) + (((kk * 4 + kq) ^ (r16 & 7)) << 4);
+        const bf16x8_t pf = *reinterpret_cast<const bf16x8_t*>(Ps + at), rf = *reinterpret_cast<const bf16x8_t*>(Rs + at);
+        bf16x8_t vf[OT];
+#pragma unroll
+        for (int t = 0; t < OT; ++t) {
           bf16x4_t half[2];
 #pragma unroll
           for (int hf = 0; hf < 2; ++hf) {
@@ -1731,12 +1742,12 @@ latent_decode_range_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ ou
             half[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4_t*)(
                 Ks + key * NP * 16 + ((piece ^ (key & 7)) << 4) + (r16 & 1) * 8));
           }
-          vf[kk] = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
+          vf[t] = __builtin_shufflevector(half[0], half[1], 0, 1, 2, 3, 4, 5, 6, 7);
         }
 #pragma unroll
-        for (int kk = 0; kk < LD_KT / 32; ++kk)
-          if (decltype(whole)::value || tile0 + kk * 32 <= range_hi)
-            o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[kk], pf[kk], o[t], 0, 0, 0);
+        for (int t = 0; t < OT; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], rf, o[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < OT; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[t], pf, o[t], 0, 0, 0);
       }
     };
     if (tile0 + LD_KT - 32 <= range_hi) values(std::true_type{});

@@ -11,6 +11,7 @@ device in one transfer.
 
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass, field
 from typing import Dict, Hashable, List, NamedTuple, Optional, Sequence, Tuple
 
@@ -88,6 +89,16 @@ class StepContext:
     # the residual stream rounded to the run's type, when the kernel that wrote the stream last
     # left such a copy; the model drops it as soon as anything else touches the stream
     rounded: Optional[torch.Tensor] = None
+
+    @functools.cached_property
+    def visible_rows(self) -> int:
+        """Tokens that the step's requests have in all, cached and new."""
+        return self.n_tokens + sum(self.ctx_lens_host)
+
+    @functools.cached_property
+    def fewest_tokens(self) -> int:
+        """The new tokens of the request that brings fewest."""
+        return min(self.seq_lens_host, default=0)
 
     def attention_items(self, rows_per_item: int, from_tokens: int = 1):
         """Work items of at most ``rows_per_item`` consecutive query rows of one request that

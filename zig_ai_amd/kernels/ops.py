@@ -3348,7 +3348,6 @@ def latent_fold(q: torch.Tensor, fold: torch.Tensor, rot_dim: int, positions: to
     """The folded queries ``[T, heads, rank + rot_dim]`` of ``q [T, heads, d + rot_dim]``: ``fold [heads, rank, d]``
     times the unrotated part, then the rotated part as ``rotate_part_`` gives it.  A decode batch in bfloat16
     takes one launch, anything else the two."""
-    _need(q, "q", (torch.float32, torch.bfloat16))
     if q.dim() != 3 or fold.dim() != 3 or fold.shape[0] != q.shape[1] or fold.shape[2] + rot_dim != q.shape[2]:
         raise KernelError(f"latent_fold takes q [T, heads, d + {rot_dim}] and fold [heads, rank, d], got "
                           f"{tuple(q.shape)} and {tuple(fold.shape)}")
@@ -3357,6 +3356,7 @@ def latent_fold(q: torch.Tensor, fold: torch.Tensor, rot_dim: int, positions: to
     out = torch.empty((T, H, rank + rot_dim), dtype=q.dtype, device=q.device)
     if rot_dim and T <= 16 and q.dtype == fold.dtype == torch.bfloat16 and d < HEAD_SPLIT_MIN_K and d % 8 == 0 \
             and ld % 8 == 0 and q.data_ptr() % 16 == 0 and fold.data_ptr() % 16 == 0:
+        _need(q, "q", torch.bfloat16)
         _need(fold, "fold", torch.bfloat16)
         _need(positions, "positions", torch.int32, (T,))
         if rot_dims % 2 or not 0 <= rot_dims <= rot_dim:

@@ -66,7 +66,7 @@ def plan_latent_split(groups: int, max_keys: int, target: int = LATENT_SPLIT_TAR
 
 
 # The kernel that takes single tokens' keys 128 at a time (``ops.latent_range_fits``) has one workgroup a compute
-# unit at latents of 512 (three at 128), and a second round of them costs more than longer ranges.  Us with
+# unit at latents of 512 (two at 128), and a second round of them costs more than longer ranges.  Us with
 # ranges of 128, 256 and 512 keys, 16 heads, R = 512 with 64 rotated: 8 requests at 2,050 keys 18.5, 19.8, 25.5, at
 # 8,000 42, 29, 30; 32 at 2,000 36, 26, 29; 64 at 1,200 46, 39, 32; R = 128 with 32: 64 at 2,000 19.0, 15.7, 17.1.
 # 129 to 255 groups get a range each, which leaves compute units idle, but cuts them only gain where contexts are long
@@ -79,7 +79,7 @@ FORMING_ROWS_A_TOKEN = 16      # visible rows a new token, at most
 FORMING_BYTES = 256 << 20      # the most that formed keys and values may take
 
 
-def forming_pays(seq_lens, ctx_lens, bytes_a_row: int) -> bool:
+def forming_pays(step, bytes_a_row: int) -> bool:
     """Whether a step's keys and values are formed: every request brings a portion, and a visible row is
     seen by enough new tokens.  Us a layer folded and formed (16 heads, R = 512 with 64 rotated), by visible rows a new
     token.  1: one prompt of 64 32 and 15, 512 61 and 26, 1,777 145 and 61, 4,096 523 and 145; 4 tokens of 8 requests each 31 and
@@ -88,8 +88,8 @@ def forming_pays(seq_lens, ctx_lens, bytes_a_row: int) -> bool:
     each behind 32 27 and 23.  25: 128 behind 3,072 185 and 81, but 64 behind 1,536 50 and 55, 2 of 32 each behind 48 28 and
     31.  33: 512 behind 16,384 836 and 390, 64 of 8 each behind 2,048 140 and 144.  The line lies where all gain: beyond it
     few tokens lose, whose folded kernel cuts contexts into ranges.  Single tokens share their rows with nobody."""
-    rows = sum(seq_lens) + sum(ctx_lens)
-    return min(seq_lens) > 1 and rows <= FORMING_ROWS_A_TOKEN * sum(seq_lens) and rows * bytes_a_row <= FORMING_BYTES
+    return step.fewest_tokens > 1 and step.visible_rows <= FORMING_ROWS_A_TOKEN * step.n_tokens \
+        and step.visible_rows * bytes_a_row <= FORMING_BYTES
 
 
 FORMING_BLOCK = 256      # rows
@@ -235,8 +235,7 @@ class LatentAttention(Mixer):
                                 self.inv_freq, self.rot_dims, self.adjacent,
                                 plane if cache.writes else None, self.magnitude)
         q = ops.linear(cq, self.w_q_up, tune=tune).view(T, nh, d + dr)
-        if self.w_form is not None and not step.recordable \
-                and forming_pays(step.seq_lens_host, step.ctx_lens_host, 2 * nh * (d + dv)):
+        if self.w_form is not None and not step.recordable and forming_pays(step, 2 * nh * (d + dv)):
             a = self._formed(q, down, plane, step, cache)
             return ops.linear(a.view(T, nh * dv), self.w_out, partial_ok=self.partial_ok, tune=tune)
         qf = self._folded(q, step)
@@ -291,7 +290,7 @@ class LatentAttention(Mixer):
         """The heads' gated results over formed keys and values."""
         if getattr(step, "taps", None) is not None:
             step.taps["q"] = self._folded(q, step)      # (what the other steps leave)
-        rows = forming_rows(step.n_tokens + sum(step.ctx_lens_host), self.w_form.shape[0], self.kv_rank)
+        rows = forming_rows(step.visible_rows, self.w_form.shape[0], self.kv_rank)
         latent, rot = ops.latent_open_rows(
             q, self.head_dim, self.rotated_dim, step.positions, self.inv_freq, self.rot_dims, self.adjacent,
             self.magnitude, plane, self.kv_rank, step.block_tables[cache.group], step.seq_start, step.ctx_len,
